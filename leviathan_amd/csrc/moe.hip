@@ -1493,12 +1493,15 @@ int check_pools(lev_ctx *ctx, const lev_moe_experts *p, uint32_t top_k, uint32_t
     return LEV_OK;
 }
 
-bool experts_fast(const moe_args &a, const float *x) {
+// rows of whole block pairs on 4-byte boundaries, x on a 16-byte one
+bool experts_aligned(const moe_args &a, const float *x) {
     auto al4 = [&](uint64_t v) { return ((reinterpret_cast<uintptr_t>(a.base) + v) & 3u) == 0; };
-    return a.hidden % 64u == 0 && a.inter % 64u == 0 && a.hidden <= 4096u && a.inter <= 4096u &&
-           al4(a.gate_off) && al4(a.up_off) && al4(a.down_off) && a.gate_stride % 4u == 0 &&
-           a.up_stride % 4u == 0 && a.down_stride % 4u == 0 &&
+    return a.hidden % 64u == 0 && a.inter % 64u == 0 && al4(a.gate_off) && al4(a.up_off) && al4(a.down_off) &&
+           a.gate_stride % 4u == 0 && a.up_stride % 4u == 0 && a.down_stride % 4u == 0 &&
            (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
+}
+bool experts_fast(const moe_args &a, const float *x) {
+    return experts_aligned(a, x) && a.hidden <= 4096u && a.inter <= 4096u;
 }
 
 // rt.ids == NULL (selection inside the gate/up kernel) is only valid on the
@@ -1578,7 +1581,7 @@ bool use_grouped(const lev_ctx *ctx, const moe_args &a, const float *x, uint32_t
         const char *e = getenv("LEV_MOE_GROUPED");   // LEV_MOE_GROUPED=0: per-pair kernels, for comparison
         return !(e && e[0] == '0');
     }();
-    return enabled && tokens >= kGroupedMinTokens && experts_fast(a, x) &&
+    return enabled && tokens >= kGroupedMinTokens && experts_aligned(a, x) &&
            lev_moe_grouped_usable(ctx, grouped_args(a, tokens));
 }
 
@@ -1682,7 +1685,7 @@ extern "C" int lev_hip_moe_experts_q4_0(lev_ctx *ctx, const lev_moe_experts *poo
     moe_scratch s{nullptr, nullptr, nullptr};
     if (!act || grouped) {
         st = get_scratch(ctx, tokens, a.experts, top_k, a.inter, &s,
-                         grouped ? lev_moe_grouped_scratch_bytes(grouped_args(a, tokens)) : 0);
+                         grouped ? lev_moe_grouped_scratch_bytes(ctx, grouped_args(a, tokens)) : 0);
         if (st != LEV_OK) return st;
         if (!act) act = s.act;
     }
@@ -1731,7 +1734,7 @@ int moe_layer_impl(lev_ctx *ctx, const lev_moe_experts *pools, const float *d_ro
         s.grouped = nullptr;
     } else {
         st = get_scratch(ctx, tokens, a.experts, top_k, a.inter, &s,
-                         grouped ? lev_moe_grouped_scratch_bytes(grouped_args(a, tokens)) : 0);
+                         grouped ? lev_moe_grouped_scratch_bytes(ctx, grouped_args(a, tokens)) : 0);
         if (st != LEV_OK) return st;
     }
     const bool fast = experts_fast(a, d_x);

@@ -28,10 +28,13 @@ struct alignas(32) lev_grp_start {
     uint32_t pad[3];
 };
 
-size_t lev_moe_grouped_scratch_bytes(const lev_moe_grouped_args &a);
-// Geometry the grouped path serves (the caller also checks 4-byte aligned pools).
+// Whether the many-token path takes the call (the caller also checks 4-byte aligned pools and x).
 bool lev_moe_grouped_usable(const lev_ctx *ctx, const lev_moe_grouped_args &a);
+size_t lev_moe_grouped_scratch_bytes(const lev_ctx *ctx, const lev_moe_grouped_args &a);
 // act: f32 [tokens*top_k][inter] (written here, read by the down stage).
 hipError_t lev_moe_grouped_launch(lev_ctx *ctx, const lev_moe_grouped_args &a, const float *x,
                                   const int32_t *ids, const float *weights, float *y, float *act,
                                   void *scratch);
+// y[t] = sum over slots, in slot order, of weights * dn (f32 [pair][hidden]); pairs that are not valid add zero.
+hipError_t lev_moe_merge_launch(lev_ctx *ctx, const lev_moe_grouped_args &a, const float *dn, const float *weights,
+                                const uint8_t *valid, float *y);

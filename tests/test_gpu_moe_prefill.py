@@ -1,0 +1,34 @@
+"""GPU parity of the grouped matrix product that serves prompts and large batches of the MoE layer, at the
+edges of its tiles: column tiles of 32 in items of 64 pairs, rows in tiles of 128 (gate/up) and 256 (down)
+cut into waves, K in steps of two blocks and weight groups of four.  FP64 chain at the reference's 1e-4."""
+import numpy as np
+import pytest
+
+import oracle as O
+from tests import helpers as H
+from tests.test_gpu_moe_gemm import TOL, ctx, run_experts  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("hidden,inter,counts", [
+    (64, 64, (1, 32)),            # one K-step, one weight group of two blocks
+    (192, 320, (33, 31, 0)),      # rows past the last whole wave tile; a last group of two blocks
+    (320, 192, (64, 65)),         # a full item; a second item of one pair
+    (2816, 704, (97, 7, 128)),
+    (4160, 128, (40, 24)),        # rows wider than the few-token kernels take
+])
+def test_moe_grouped_product_tiles(ctx, hidden, inter, counts):
+    """One slot a token: expert e takes exactly counts[e] pairs."""
+    experts, tokens = len(counts), sum(counts)
+    wr, pool, offs, x = H.config5(hidden, inter, experts, tokens, seed=hidden + inter)
+    rng = np.random.default_rng(tokens)
+    ids = rng.permutation(np.repeat(np.arange(experts), counts)).astype(np.int32)[:, None]
+    wts = rng.random((tokens, 1)).astype(np.float32)
+    y, act = run_experts(ctx, pool, offs, hidden, inter, experts, x, ids, wts)
+    g, u, d = (pool[offs["gate_off"]:], pool[offs["up_off"]:], pool[offs["down_off"]:])
+    for t in range(0, tokens, 1 if hidden < 1000 else 9):
+        ref = O.moe_experts_f64(g, u, d, hidden, inter, ids[t], wts[t], x[t])
+        assert O.max_rel_err(act[t], ref["act"]) < TOL, t
+        y32, _ = O.moe_experts_f32(g, u, d, hidden, inter, ids[t], wts[t], x[t])
+        assert O.max_rel_err(y[t], ref["y"]) < max(TOL, 1.5 * O.max_rel_err(y32, ref["y"])), t
