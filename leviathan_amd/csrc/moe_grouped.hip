@@ -14,13 +14,14 @@
 // [pair][inter]), down -> dn (f32, [pair][hidden]), merge: y[t] = sum over slots, IN SLOT ORDER,
 // fmaf(w_slot, dn_slot, acc).
 //
-// Batches of at most five and a half pairs per expert on average, with rows of up to 2048
+// Batches of at most eight pairs per expert on average, with rows of up to 4096
 // activations, take these kernels (the digit planes of the few-token kernels, four tokens of an expert
 // per product, operands in registers): they cost less per product than the grouped matrix product of
 // moe_prefill.hip and more per token, and win while most experts hold no more than a handful of pairs.
 #include "moe_prefill.hpp"
 
 #include <array>
+#include <cmath>
 #include <cstdio>
 #include "q4_0_mfma.hpp"
 
@@ -234,16 +235,17 @@ moe_group_kernel(const int32_t *__restrict__ ids, uint32_t pairs, uint32_t exper
 // and stores.
 // ---------------------------------------------------------------------------
 constexpr uint32_t kG8MaxGrid = 512;                      // workgroups of an expert kernel (one per CU)
-constexpr int kG8MaxWpr = 8;                              // waves that share a row group: one task each
-constexpr int kG8WavesGateUp = 8;                         // 2048 activations: eight column tasks, one slot
+constexpr int kG8WavesGateUp = 8;                         // up to 2048 activations: eight column tasks, one slot
 constexpr int kG8WavesDown = 12;                          // 768 activations: three column tasks, four slots (three
                                                           // waves a SIMD; eight waves leave two SIMDs with one)
+constexpr int kG8WavesWide = 12, kG8WavesMax = 16;        // wider rows: one wave per column task still, up to 3072 and 4096
 constexpr int kG8TilesDown = 1;                          // row groups a wave of the down kernel takes per round (2: rounds twice
                                                           // as long, the stretches a workgroup gets then differ by more: 106.8
                                                           // against 104.4 us a layer at 64 tokens)
-constexpr uint32_t kG8Batch = 4;                          // rounds between two barriers of a workgroup (2: 55.4
-                                                          // against 53.6 us for gate/up, 1: 64.9)
-constexpr uint32_t kG8MaxInLen = 256u * kG8MaxWpr;
+constexpr uint32_t g8_batch(int nw) { return nw > 12 ? 2u : 4u; }   // rounds between two barriers of a workgroup (2: 55.4
+                                                          // against 53.6 us for gate/up, 1: 64.9; the sums of four rounds of
+                                                          // sixteen waves do not fit the LDS)
+constexpr uint32_t kG8MaxInLen = 256u * kG8WavesMax;
 constexpr uint32_t kG8Plane = 272u;                       // a digit plane of a staged task: 256 bytes + 16, so that
 constexpr uint32_t kG8TokArea = 4u * kG8Plane;            // the 64 lanes of an operand read hit 64 different banks
 constexpr uint32_t kG8WaveLds = 4u * kG8TokArea;           // four tokens are staged at a time
@@ -252,7 +254,7 @@ constexpr uint32_t kG8WaveLds = 4u * kG8TokArea;           // four tokens are st
 // wave four staged tasks
 template <int NTILE, int NW>
 constexpr size_t g8_lds() {
-    return (size_t)2 * kG8Batch * NTILE * (kG8NT / 4) * (NW * 256u) + (size_t)NW * kG8WaveLds;
+    return (size_t)2 * g8_batch(NW) * NTILE * (kG8NT / 4) * (NW * 256u) + (size_t)NW * kG8WaveLds;
 }
 
 // Digit planes of one token's task into `tok` (kG8TokArea bytes, this wave's own): lane i holds
@@ -372,6 +374,7 @@ moe_grouped_i8_kernel(lev_moe_grouped_args a, const float *__restrict__ src, con
     constexpr uint32_t NT = kG8NT, NJ = NT / 4u;
     constexpr uint32_t TO = PAIRED ? 1u : (uint32_t)NTILE;       // row groups a slot finishes per round
     constexpr uint32_t kG8Unit = NW * 256u;                       // bytes of part[wave][row][token % 4]: one tile's sums of four tokens
+    constexpr uint32_t kG8Batch = g8_batch(NW);
     constexpr uint32_t kHalf = kG8Batch * NTILE * NJ * kG8Unit;   // one parity of `part`: a batch of rounds (with one
                                                                   // token group an item: twice as many rounds)
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
@@ -383,6 +386,10 @@ moe_grouped_i8_kernel(lev_moe_grouped_args a, const float *__restrict__ src, con
     const uint32_t ngroups = (out_rows + 15u) >> 4;
     const uint64_t row_bytes = (uint64_t)(in_len >> 6) * 36u;
     const uint32_t r = lane & 15u, g = lane >> 4, lrow = lane >> 2;
+    // the last task of a row may be a part of one: the pairs and activations past the row's end repeat
+    // the row's last ones, and the activations count as zero
+    const uint32_t npairs = in_len >> 6, wpair = 4u * tw + (lane & 3u), wpoff = (wpair < npairs ? wpair : npairs - 1u) * 36u;
+    const uint32_t a4 = 64u * tw + lane, a4c = a4 < (in_len >> 2) ? a4 : (in_len >> 2) - 1u;
 
     // this workgroup's stretch of the line of rounds
     const uint32_t G = gridDim.x;
@@ -414,7 +421,7 @@ moe_grouped_i8_kernel(lev_moe_grouped_args a, const float *__restrict__ src, con
         for (uint32_t k = 0; k < NT; ++k) {
             pk[k] = item->pair[k];
             const uint32_t srow = (uint32_t)(PAIRED ? item->src[k] : item->pair[k]);
-            v[k] = reinterpret_cast<const lev_f32x4 *>(src + (uint64_t)srow * in_len)[64u * tw + lane];
+            v[k] = reinterpret_cast<const lev_f32x4 *>(src + (uint64_t)srow * in_len)[a4c];
         }
         const uint8_t *m0 = a.base + (PAIRED ? a.gate_off + e * a.gate_stride : a.down_off + e * a.down_stride);
         const uint8_t *m1 = PAIRED ? a.base + a.up_off + e * a.up_stride : m0;
@@ -425,7 +432,7 @@ moe_grouped_i8_kernel(lev_moe_grouped_args a, const float *__restrict__ src, con
                 rg = rg < ngroups ? rg : ngroups - 1u;
                 uint32_t row = rg * 16u + lrow;
                 row = row < out_rows ? row : out_rows - 1u;
-                q4m_load_task((PAIRED && t == 1 ? m1 : m0) + (uint64_t)row * row_bytes, 4u * tw, D[t]);
+                lev_q4_load_pair((PAIRED && t == 1 ? m1 : m0) + ((uint64_t)row * row_bytes + wpoff), D[t]);
             }
         };
         __builtin_amdgcn_sched_barrier(0);
@@ -437,7 +444,10 @@ moe_grouped_i8_kernel(lev_moe_grouped_args a, const float *__restrict__ src, con
         // the count repeat the last pair), in front of the weights: a request inside the branch
         // below would queue behind them
 #pragma unroll
-        for (uint32_t k = 0; k < NT; ++k) lev_pin(v[k]);
+        for (uint32_t k = 0; k < NT; ++k) {
+            lev_pin(v[k]);
+            if (a4 != a4c) v[k] = lev_f32x4{0.f, 0.f, 0.f, 0.f};
+        }
         long A[NJ][8];
         float unscale[NJ];
 #pragma unroll
@@ -503,11 +513,18 @@ moe_grouped_i8_kernel(lev_moe_grouped_args a, const float *__restrict__ src, con
                 const float *pp = reinterpret_cast<const float *>(
                     smem + half + b * round_bytes + (t * ng + j) * kG8Unit + ((s * wpr * 16u + r) * 4u + g) * 4u);
                 auto slot_sum = [&](const float *q) {
-                    float p[kG8MaxWpr];
+                    float p[8];
 #pragma unroll
-                    for (uint32_t w = 0; w < (uint32_t)kG8MaxWpr; ++w) p[w] = q[(w < wpr ? w : 0u) * 64u];   // eight reads in flight
+                    for (uint32_t w = 0; w < 8u; ++w) p[w] = q[(w < wpr ? w : 0u) * 64u];   // eight reads in flight
 #pragma unroll
-                    for (uint32_t w = 0; w < (uint32_t)kG8MaxWpr; ++w) p[w] = w < wpr ? p[w] : 0.f;
+                    for (uint32_t w = 0; w < 8u; ++w) p[w] = w < wpr ? p[w] : 0.f;
+                    if (NW > 8 && wpr > 8u) {
+                        float hi[8];
+#pragma unroll
+                        for (uint32_t w = 0; w < 8u; ++w) hi[w] = q[(w + 8u < wpr ? w + 8u : 0u) * 64u];
+#pragma unroll
+                        for (uint32_t w = 0; w < 8u; ++w) p[w] += w + 8u < wpr ? hi[w] : 0.f;
+                    }
                     return ((p[0] + p[4]) + (p[2] + p[6])) + ((p[1] + p[5]) + (p[3] + p[7]));
                 };
                 float res = slot_sum(pp);
@@ -591,8 +608,8 @@ grouped_layout layout_of(const lev_moe_grouped_args &a) {
     return L;
 }
 
-// Where the integer matrix-core kernels serve: rows of whole 256-value tasks, one task per wave, and
-// at most five and a half pairs per expert on average -- they multiply four tokens at a time and are
+// Where the integer matrix-core kernels serve: rows of up to 4096 values, one 256-value task per wave, and
+// at most eight pairs per expert on average -- they multiply four tokens at a time and are
 // the faster ones while most experts hold no more than four or eight pairs; the grouped matrix product
 // (moe_prefill.hip) takes 32 at one price.  LEV_MOE_GROUPED_I8=0 never takes them, =1 for any token
 // count (for comparison and for the tests).
@@ -602,36 +619,40 @@ bool g8_usable(const lev_ctx *ctx, const lev_moe_grouped_args &a) {
         return v && v[0] == '0' ? 0 : v && v[0] == '1' ? 1 : 2;
     }();
     if (mode == 0) return false;
-    const bool shape = a.hidden % 256u == 0u && a.hidden <= kG8MaxInLen && a.inter % 256u == 0u && a.inter <= kG8MaxInLen;
+    const bool shape = a.hidden % 64u == 0u && a.hidden <= kG8MaxInLen && a.inter % 64u == 0u && a.inter <= kG8MaxInLen;
     const size_t limit = ctx->props.sharedMemPerBlockOptin > ctx->props.sharedMemPerBlock
                              ? ctx->props.sharedMemPerBlockOptin
                              : ctx->props.sharedMemPerBlock;
     const size_t lds_group = (size_t)5 * a.experts * 4;
-    const bool fits = g8_lds<2, kG8WavesGateUp>() <= limit && g8_lds<kG8TilesDown, kG8WavesDown>() <= limit && lds_group <= limit;
-    // (hidden 2048, intermediate 768, top-8 of 128 experts, us a layer: 64 tokens 100 against 143 for the grouped
-    // product, 96 tokens 147 for the product; 1024 / 512, top-4 of 32: 32 tokens 36 against 44, 48 tokens 44 for it)
-    return shape && fits && (mode == 1 || 2u * (uint64_t)a.tokens * a.top_k <= 11u * (uint64_t)a.experts);
+    const bool fits = g8_lds<2, kG8WavesWide>() <= limit && g8_lds<2, kG8WavesMax>() <= limit && g8_lds<kG8TilesDown, kG8WavesMax>() <= limit &&
+                      lds_group <= limit;
+    // (us a layer, these kernels against the grouped product: 2048 / 768, top-8 of 128: 64 tokens 101, 145; 128 tokens
+    // 129, 150; 2816 / 704, top-8 of 128: 128 tokens 164, 200; 1408 / 320, top-4 of 64: 128 tokens 58, 58; 3072 / 1024,
+    // top-6 of 60: 64 tokens 116, 145; 96 tokens 142, 145; 128 tokens 166, 148.  Measured with 32 experts and more: fewer
+    // keep the earlier line of five and a half pairs)
+    return shape && fits && (mode == 1 || 2u * (uint64_t)a.tokens * a.top_k <= (a.experts >= 32u ? 16u : 11u) * (uint64_t)a.experts);
 }
 
 struct g8_geometry {
+    int nw;                     // waves of the kernel's instantiation
     uint32_t wpr, slots, rpi;   // waves a row, row-group slots a workgroup, rounds an item
 };
-template <int NTILE, bool PAIRED, int NW>
-g8_geometry g8_geometry_of(const lev_moe_grouped_args &a) {
-    const uint32_t in_len = PAIRED ? a.hidden : a.inter, out_rows = PAIRED ? a.inter : a.hidden;
+g8_geometry g8_geometry_of(const lev_moe_grouped_args &a, bool paired) {
+    const uint32_t in_len = paired ? a.hidden : a.inter, out_rows = paired ? a.inter : a.hidden;
     g8_geometry q;
-    q.wpr = in_len >> 8;
-    q.slots = (uint32_t)NW / q.wpr;
+    q.wpr = (in_len + 255u) >> 8;
+    q.nw = paired && q.wpr <= (uint32_t)kG8WavesGateUp ? kG8WavesGateUp : q.wpr <= (uint32_t)kG8WavesWide ? kG8WavesWide : kG8WavesMax;
+    q.slots = (uint32_t)q.nw / q.wpr;
     const uint32_t ngroups = (out_rows + 15u) / 16u;
-    const uint32_t per_round = q.slots * (PAIRED ? 1u : (uint32_t)NTILE);   // row groups a round finishes
+    const uint32_t per_round = q.slots * (paired ? 1u : (uint32_t)kG8TilesDown);   // row groups a round finishes
     q.rpi = (ngroups + per_round - 1u) / per_round;
     return q;
 }
+static_assert(kG8WavesDown == kG8WavesWide, "one instantiation serves both");
 
 template <int NTILE, bool PAIRED, int NW>
-hipError_t g8_launch(lev_ctx *ctx, const lev_moe_grouped_args &a, const float *src, const lev_grp_item *items,
-                     const lev_grp_start *starts, uint32_t grid, float *out) {
-    const g8_geometry q = g8_geometry_of<NTILE, PAIRED, NW>(a);
+hipError_t g8_launch_as(lev_ctx *ctx, const lev_moe_grouped_args &a, const g8_geometry &q, const float *src,
+                        const lev_grp_item *items, const lev_grp_start *starts, uint32_t grid, float *out) {
     uint64_t slot_of_wave, pos_of_wave;
     lev_wave_tables(q.wpr, &slot_of_wave, &pos_of_wave);
     constexpr size_t lds = g8_lds<NTILE, NW>();
@@ -646,6 +667,14 @@ hipError_t g8_launch(lev_ctx *ctx, const lev_moe_grouped_args &a, const float *s
                        ctx->stream, a, src, items, starts, out, q.wpr, q.slots, q.rpi, slot_of_wave, pos_of_wave);
     return hipGetLastError();
 }
+template <int NTILE, bool PAIRED>
+hipError_t g8_launch(lev_ctx *ctx, const lev_moe_grouped_args &a, const g8_geometry &q, const float *src,
+                     const lev_grp_item *items, const lev_grp_start *starts, uint32_t grid, float *out) {
+    if (PAIRED && q.nw == kG8WavesGateUp)
+        return g8_launch_as<NTILE, PAIRED, PAIRED ? kG8WavesGateUp : kG8WavesDown>(ctx, a, q, src, items, starts, grid, out);
+    if (q.nw == kG8WavesWide) return g8_launch_as<NTILE, PAIRED, kG8WavesWide>(ctx, a, q, src, items, starts, grid, out);
+    return g8_launch_as<NTILE, PAIRED, kG8WavesMax>(ctx, a, q, src, items, starts, grid, out);
+}
 
 }  // namespace
 
@@ -656,11 +685,19 @@ hipError_t lev_moe_merge_launch(lev_ctx *ctx, const lev_moe_grouped_args &a, con
     return hipGetLastError();
 }
 
-// The grouped product streams an expert once whatever it holds, behind 45 us of launches: it wins over
-// the kernels that stream an expert per pair from about two pairs per expert on (2816 / 704, top-8 of 128, us
-// a layer: 16 tokens 148 against 109, 32 tokens 173 against 189, 64 tokens 193 against 352).
+// Grouping costs some 13 us of launches over the kernels that stream an expert for every pair, and saves the
+// bytes of the experts that several tokens share (top_k of `experts` each: expected number of distinct
+// ones). Those kernels also stream large experts less well: ten experts' worth of bytes.  65 MB is where the
+// two meet (us a layer, grouped against per pair: 2816 / 704, top-8 of 128: 5 tokens 62, 66; 16 tokens 89, 109;
+// 1408 / 320, top-4 of 64: 16 tokens 39, 31; 64 tokens 50, 57; 1024 / 576, top-2 of 32: 32 tokens 34, 31;
+// 64 tokens 36, 45; 3072 / 1024, top-6 of 60: 5 tokens 69, 79).  Rows of whole 256-value tasks up to
+// 2048 wide are always grouped, so that a token's bits do not depend on how many travel with it.
 bool lev_moe_grouped_usable(const lev_ctx *ctx, const lev_moe_grouped_args &a) {
-    return lev_moe_prefill_usable(a) && (g8_usable(ctx, a) || (uint64_t)a.tokens * a.top_k >= 2u * (uint64_t)a.experts);
+    if (!lev_moe_prefill_usable(a)) return false;
+    if (a.hidden % 256u == 0u && a.inter % 256u == 0u && a.hidden <= 2048u && a.inter <= 2048u) return true;
+    const double expert_bytes = 3.0 * a.hidden * a.inter * 18.0 / 32.0;
+    const double distinct = a.experts * (1.0 - std::pow(1.0 - (double)a.top_k / a.experts, (double)a.tokens));
+    return ((double)a.tokens * a.top_k - distinct + 10.0) * expert_bytes >= 65e6;
 }
 
 size_t lev_moe_grouped_scratch_bytes(const lev_ctx *ctx, const lev_moe_grouped_args &a) {
@@ -682,7 +719,7 @@ hipError_t lev_moe_grouped_launch(lev_ctx *ctx, const lev_moe_grouped_args &a, c
     lev_grp_item *items = reinterpret_cast<lev_grp_item *>(s + L.items);
     lev_grp_start *starts = reinterpret_cast<lev_grp_start *>(s + L.starts);
     const uint32_t grid = (uint32_t)ctx->num_cus < kG8MaxGrid ? (uint32_t)ctx->num_cus : kG8MaxGrid;
-    const g8_geometry q_gu = g8_geometry_of<2, true, kG8WavesGateUp>(a), q_dn = g8_geometry_of<kG8TilesDown, false, kG8WavesDown>(a);
+    const g8_geometry q_gu = g8_geometry_of(a, true), q_dn = g8_geometry_of(a, false);
     // what a round of an item of up to four pairs and of a larger one cost, relative to each other
     // (gate/up 52 against 62 us, down 33 against 38 with every item of the one or the other kind;
     // equal weights: 62 + 39 us at 64 tokens, these: 58 + 36.5)
@@ -716,8 +753,8 @@ hipError_t lev_moe_grouped_launch(lev_ctx *ctx, const lev_moe_grouped_args &a, c
                        a.experts, a.top_k, valid, ctx->d_flag, items, starts, grid, q_gu.rpi, q_dn.rpi, w1, w2, w1_dn, w2_dn,
                        s0_gu, s0_dn);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    if ((e = g8_launch<2, true, kG8WavesGateUp>(ctx, a, x, items, starts, grid, act)) != hipSuccess) return e;
+    if ((e = g8_launch<2, true>(ctx, a, q_gu, x, items, starts, grid, act)) != hipSuccess) return e;
     // rows of act that belong to dropped pairs are never written and never read
-    if ((e = g8_launch<kG8TilesDown, false, kG8WavesDown>(ctx, a, act, items, starts + grid, grid, dn)) != hipSuccess) return e;
+    if ((e = g8_launch<kG8TilesDown, false>(ctx, a, q_dn, act, items, starts + grid, grid, dn)) != hipSuccess) return e;
     return lev_moe_merge_launch(ctx, a, dn, weights, valid, y);
 }

@@ -32,3 +32,24 @@ def test_moe_grouped_product_tiles(ctx, hidden, inter, counts):
         assert O.max_rel_err(act[t], ref["act"]) < TOL, t
         y32, _ = O.moe_experts_f32(g, u, d, hidden, inter, ids[t], wts[t], x[t])
         assert O.max_rel_err(y[t], ref["y"]) < max(TOL, 1.5 * O.max_rel_err(y32, ref["y"])), t
+
+
+@pytest.mark.parametrize("hidden,inter,experts,top_k,tokens", [
+    (2816, 704, 14, 8, 9),        # eleven column tasks a row (twelve waves); a last task of three pairs
+    (4096, 4096, 4, 2, 6),        # sixteen tasks both ways
+    (3136, 1088, 9, 4, 12),       # thirteen, the last of one pair; five, the last of one
+])
+def test_moe_grouped_integer_kernels_ragged_rows(ctx, hidden, inter, experts, top_k, tokens):
+    """The integer grouped kernels on rows that end inside a 256-value task and rows wider than eight tasks."""
+    wr, pool, offs, x = H.config5(hidden, inter, experts, tokens, seed=hidden + inter)
+    rng = np.random.default_rng(tokens)
+    ids = np.stack([rng.permutation(experts)[:top_k] for _ in range(tokens)]).astype(np.int32)
+    wts = rng.random((tokens, top_k)).astype(np.float32)
+    assert 2 * tokens * top_k <= 11 * experts
+    y, act = run_experts(ctx, pool, offs, hidden, inter, experts, x, ids, wts)
+    g, u, d = (pool[offs["gate_off"]:], pool[offs["up_off"]:], pool[offs["down_off"]:])
+    for t in range(tokens):
+        ref = O.moe_experts_f64(g, u, d, hidden, inter, ids[t], wts[t], x[t])
+        assert O.max_rel_err(act[t], ref["act"]) < TOL
+        y32, _ = O.moe_experts_f32(g, u, d, hidden, inter, ids[t], wts[t], x[t])
+        assert O.max_rel_err(y[t], ref["y"]) < max(TOL, 1.5 * O.max_rel_err(y32, ref["y"]))
