@@ -183,6 +183,23 @@ __device__ __forceinline__ void lev_barrier_lds() {
     asm volatile("s_barrier" ::: "memory");
 }
 
+// s_waitcnt vmcnt(n) leaves at most n vector memory operations of the wave outstanding; they complete
+// in issue order, so everything older than the n newest has landed.  Encoding: vmcnt in bits 3:0 and
+// 15:14, expcnt (6:4) and lgkmcnt (11:8) left at "any".
+#define LEV_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | (((n) >> 4) << 14) | (7 << 4) | (15 << 8))
+
+// Direct global -> LDS load: 16 bytes a lane from `src` to the 1 KB at LDS offset `dst` (uniform).
+// Spelled as assembly because the compiler makes every later LDS read wait for all such loads in
+// flight (it cannot tell the buffers apart), which would undo a prefetch; the waits are counted by
+// hand (LEV_WAIT_VMCNT before the barrier that publishes the buffer).  m0 is the compiler's scratch: it
+// sets the register right in front of each use of its own and keeps nothing in it.
+__device__ __forceinline__ void lev_load_lds16(const void *src, uint32_t dst) {
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(dst) : "memory");
+}
+__device__ __forceinline__ uint32_t lev_lds_offset(const void *lds) {
+    return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const uint8_t *)lds;
+}
+
 // ---- shared by the kernels in which a wave owns one column block of the matrix (a Q4_0 task,
 // a Q4_K or Q6_K superblock column) and `wpr` waves of a workgroup of 16 cover a row ----
 

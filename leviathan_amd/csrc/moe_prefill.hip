@@ -205,17 +205,6 @@ struct pf_lds_map {
     static constexpr uint32_t kBytes = kW + 2u * kWBuf;
 };
 
-// Direct global -> LDS load: 16 bytes a lane from `src` to the 1 KB at LDS offset `dst` (uniform).
-// Spelled as assembly because the compiler makes every later LDS read wait for all such loads in
-// flight (it cannot tell the buffers apart), which would undo the prefetch; the waits are counted by
-// hand (LEV_WAIT_VM before the barrier that publishes the buffer).  m0 is the compiler's scratch: it
-// sets the register right in front of each use of its own and keeps nothing in it.
-__device__ __forceinline__ void pf_load_lds(const void *src, uint32_t dst) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(dst) : "memory");
-}
-// at most n of the wave's vector memory operations left in flight (they complete in order)
-#define LEV_WAIT_VM(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | (((n) >> 4) << 14) | (7 << 4) | (15 << 8))
-
 // the four code bytes of one dword -> half a B operand (fp16 integers n - 8): bytes (0, 2), (1, 3) of
 // the nibble that `shift` (0 or 4) selects
 __device__ __forceinline__ void pf_decode(uint32_t codes, uint32_t mask, uint32_t magic, uint32_t out[2]) {
@@ -244,7 +233,7 @@ __device__ __forceinline__ void pf_tile(const lev_moe_grouped_args &a, const lev
     // group of a row may hold two blocks (36 bytes): then its third piece is bytes 20 .. 35, the second block's codes ----
     const uint32_t row0 = PAIRED ? rt * 128u + wave * 16u : rt * 256u + wave * 32u;
     const bool live = row0 < out_rows;   // a wave past the last row only brings activations
-    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
+    const uint32_t lds0 = lev_lds_offset(lds);
     const uint8_t *wsrc[kPfFetch];
     uint32_t wpos = 0u;                  // three bytes: the pieces' positions in a whole group
 #pragma unroll
@@ -263,7 +252,7 @@ __device__ __forceinline__ void pf_tile(const lev_moe_grouped_args &a, const lev
 #pragma unroll
         for (int j = 0; j < kPfFetch; ++j) {
             const uint32_t at = (wpos >> (8 * j)) & 0xFFu;
-            if (j < 2 || lane < 32u) pf_load_lds(wsrc[j] + (gc * 72u + (at < last ? at : last)), dst + j * 1024u);
+            if (j < 2 || lane < 32u) lev_load_lds16(wsrc[j] + (gc * 72u + (at < last ? at : last)), dst + j * 1024u);
         }
     };
     w_request(0);
@@ -293,7 +282,7 @@ __device__ __forceinline__ void pf_tile(const lev_moe_grouped_args &a, const lev
 #pragma unroll
         for (int j = 0; j < T; ++j) {
             const uint32_t k = wave * T + j;
-            pf_load_lds(asrc[j] + s * kPfStep, dst + (k & 1u) * 8192u + (k >> 1) * 1024u);
+            lev_load_lds16(asrc[j] + s * kPfStep, dst + (k & 1u) * 8192u + (k >> 1) * 1024u);
         }
     };
     a_request(0);
@@ -318,8 +307,8 @@ __device__ __forceinline__ void pf_tile(const lev_moe_grouped_args &a, const lev
         constexpr uint32_t st = decltype(odd)::value;   // second step of a group
         // This step's activations have landed: they are the newest loads but for the next group's
         // weights, which are requested behind them in the first step of a group.
-        if (st == 1u) LEV_WAIT_VM(kPfFetch);
-        else LEV_WAIT_VM(0);
+        if (st == 1u) LEV_WAIT_VMCNT(kPfFetch);
+        else LEV_WAIT_VMCNT(0);
         lev_barrier_lds();   // everybody's have, and everybody is done with the other buffer
         a_request(step + 1u);
         if (st == 0u) w_request((step >> 1) + 1u);
@@ -379,7 +368,7 @@ __device__ __forceinline__ void pf_tile(const lev_moe_grouped_args &a, const lev
         if (step + 1u < nsteps) step_of(step + 1u, std::integral_constant<uint32_t, 1>());
     }
 
-    LEV_WAIT_VM(0);   // the request past the end lands before the LDS is given back
+    LEV_WAIT_VMCNT(0);   // the request past the end lands before the LDS is given back
     if (!live) return;
     // lane (lr, g), register i of a tile: weight row lr, column 8 (i / 4) + 4 g + i % 4
     const uint32_t row = row0 + (PAIRED ? lr & 15u : lr);

@@ -33,12 +33,9 @@
 // MFMA q (0..3) of chunk c takes, for lane half h, elements
 //   q<2 : 64c + 16h + 8q .. +7        (low nibbles of code bytes 8q..8q+7)
 //   q>=2: 64c + 32 + 16h + 8(q-2) ..  (high nibbles of the same bytes)
-#include "lev_common.hpp"
+#include "prefill_decode.hpp"
 
 namespace {
-
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kBM = 256;          // tokens per workgroup
 constexpr int kSBN = 96;          // rows per workgroup
@@ -51,64 +48,6 @@ constexpr int kXBufs = 4;         // X buffers in LDS: the step in use, the next
 constexpr int kBFrag = 64 * 16;                 // one B fragment: 16 bytes per lane
 constexpr int kBBuf = 4 * kSRT * kBFrag;        // [q][row tile][lane], one K-step; two of them
 constexpr int kSThreads = 512;                  // four multiplying waves and four that load X
-
-// (d*sc, dmin*m) of the 8 sub-blocks of a superblock (lev-cpu/src/lib.rs:64-74,
-// 117-124).
-__device__ __forceinline__ void q4k_all_factors(const lev_u32x4 hdr, float d1[8], float mm[8]) {
-    const float d = lev_f16_bits_to_f32(hdr.x & 0xFFFFu);
-    const float dmin = lev_f16_bits_to_f32(hdr.x >> 16);
-    const uint32_t s03 = hdr.y, s47 = hdr.z, s811 = hdr.w;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        uint32_t sc = (s03 >> (8 * j)) & 63u, mn = (s47 >> (8 * j)) & 63u;
-        d1[j] = d * (float)sc;
-        mm[j] = dmin * (float)mn;
-        uint32_t a = (s811 >> (8 * j)) & 0xFFu;
-        uint32_t sc2 = (a & 0x0Fu) | (((s03 >> (8 * j + 6)) & 3u) << 4);
-        uint32_t mn2 = (a >> 4) | (((s47 >> (8 * j + 6)) & 3u) << 4);
-        d1[4 + j] = d * (float)sc2;
-        mm[4 + j] = dmin * (float)mn2;
-    }
-}
-
-// One weight exactly as the reference rounds it: f32(d1*q - mm) first, THEN
-// round-to-nearest-even to fp16 (dequant_block_f32 followed by f32_to_f16_bits,
-// lev-cli/src/main.rs:1201-1217).  The empty asm pins the f32 value in a
-// register so that the compiler cannot merge the multiply-add with the
-// conversion into a single-rounding mixed-precision FMA, which differs from
-// the two-step rounding in about one weight in ten thousand.
-__device__ __forceinline__ _Float16 q4k_weight_f16(float d1, float code, float mm) {
-    float w32 = fmaf(d1, code, -mm);   // d1*code is exact (17 + 4 bits): one rounding, as in the reference
-    asm("" : "+v"(w32));
-    return (_Float16)w32;
-}
-
-// 8 weights (one per code byte of the two dwords, nibble selected by `hi`)
-// -> fp16 B fragment, bit-exact with fp16(f32(d1*q - mm)).
-__device__ __forceinline__ f16x8 q4k_frag(uint32_t q0, uint32_t q1, bool hi, float d1, float mm) {
-    uint32_t a = hi ? (q0 >> 4) : q0, b = hi ? (q1 >> 4) : q1;
-    a &= 0x0F0F0F0Fu;
-    b &= 0x0F0F0F0Fu;
-    // opaque from here: the compiler would otherwise fold the mask into four
-    // bit-field extracts per dword instead of using v_cvt_f32_ubyte0..3 directly
-    asm("" : "+v"(a));
-    asm("" : "+v"(b));
-    f16x8 f;
-    f[0] = q4k_weight_f16(d1, (float)(a & 0xFFu), mm);
-    f[1] = q4k_weight_f16(d1, (float)((a >> 8) & 0xFFu), mm);
-    f[2] = q4k_weight_f16(d1, (float)((a >> 16) & 0xFFu), mm);
-    f[3] = q4k_weight_f16(d1, (float)(a >> 24), mm);
-    f[4] = q4k_weight_f16(d1, (float)(b & 0xFFu), mm);
-    f[5] = q4k_weight_f16(d1, (float)((b >> 8) & 0xFFu), mm);
-    f[6] = q4k_weight_f16(d1, (float)((b >> 16) & 0xFFu), mm);
-    f[7] = q4k_weight_f16(d1, (float)(b >> 24), mm);
-    return f;
-}
-
-// s_waitcnt vmcnt(n) leaves at most n loads outstanding; loads complete in
-// issue order, so everything older than the n newest has landed.  Encoding:
-// vmcnt in bits 3:0 and 15:14, expcnt (6:4) and lgkmcnt (11:8) left at "any".
-#define LEV_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | (((n) >> 4) << 14) | (7 << 4) | (15 << 8))
 
 // grid (ceil(rows/96), ceil(tokens/256)); LDS kXBufs*kXBuf + 2*kBBuf bytes.
 __global__ void __launch_bounds__(kSThreads)
@@ -337,6 +276,8 @@ q4_k_gemm_kernel(const uint8_t *__restrict__ w, const uint16_t *__restrict__ x,
 
 hipError_t lev_q4_k_gemm_launch(lev_ctx *ctx, const uint8_t *w, const uint16_t *x, float *y,
                                 uint32_t in_dim, uint32_t rows, uint32_t tokens) {
+    const lev_gemm_split_plan plan = lev_gemm_split_choose(ctx, false, in_dim, rows, tokens, kSBN);
+    if (plan.kw) return lev_gemm_split_launch(ctx, false, w, x, y, in_dim, rows, tokens, plan);
     static bool attr_set = false;
     const size_t lds = (size_t)kXBufs * kXBuf + 2 * kBBuf;
     if (!attr_set) {

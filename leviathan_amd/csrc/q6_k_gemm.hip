@@ -23,35 +23,13 @@
 // a half are its elements 0..63, the high nibbles 64..127).  K order inside a
 // step, on both operands: MFMA q (0..3), lane half h takes elements
 // 32h + 8q .. +7.  One barrier per step, a bare s_barrier behind counted waits.
-#include "lev_common.hpp"
+#include "prefill_decode.hpp"
 
 namespace {
-
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kTR = 128;                 // rows per workgroup
 constexpr int kTT = 256;                 // tokens per workgroup (128 measured 6 % slower at 512 tokens)
 constexpr int kTK = 64;                  // K-step: one nibble plane of a half superblock
-
-struct __attribute__((packed, aligned(2))) u32x4_a2 { uint32_t v[4]; };
-
-// Four codes packed in `c` -> fp16 weights out[at..at+3], one instruction per weight
-// (Q6.swift:4-62 for the layout).  ds = d * sc has at most 18
-// significant bits and q - 32 six, so ds * (q - 32) is exact in f32 and the reference's
-// two roundings (f32, then fp16) are one rounding of the exact product.  A code byte
-// under the exponent byte 0x64 is the fp16 number 1024 + q; fma(1024 + q, ds, -1056 ds)
-// is that exact product, and the mixed-precision FMA rounds it to fp16 once.
-__device__ __forceinline__ void q6g_put4_mix(uint32_t c, float ds, float nbm, f16x8 &out, int at) {
-    const uint32_t ma = __builtin_amdgcn_perm(0x64646464u, c, 0x04020400u);   // bytes (c0, 0x64, c2, 0x64)
-    const uint32_t mb = __builtin_amdgcn_perm(0x64646464u, c, 0x04030401u);   // bytes (c1, 0x64, c3, 0x64)
-    const f16x2 a = __builtin_bit_cast(f16x2, ma), b = __builtin_bit_cast(f16x2, mb);
-    out[at + 0] = (_Float16)fmaf((float)a.x, ds, nbm);
-    out[at + 1] = (_Float16)fmaf((float)b.x, ds, nbm);
-    out[at + 2] = (_Float16)fmaf((float)a.y, ds, nbm);
-    out[at + 3] = (_Float16)fmaf((float)b.y, ds, nbm);
-}
 
 constexpr int kRXRow = 128;                    // bytes per token row in LDS
 constexpr int kRXBuf = kTT * kRXRow;           // 32 KB
@@ -60,8 +38,6 @@ constexpr int kRBFrag = 64 * 16;               // one B fragment: 16 bytes per l
 constexpr int kRRT = kTR / 32;                 // row tiles
 constexpr int kRBBuf = 4 * kRRT * kRBFrag;     // [q][row tile][lane], one K-step; two of them
 constexpr int kRThreads = 512;
-
-#define LEV_Q6G_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | (((n) >> 4) << 14) | (7 << 4) | (15 << 8))
 
 __global__ void __launch_bounds__(kRThreads)
 q6_k_gemm_kernel(const uint8_t *__restrict__ w, const uint16_t *__restrict__ x, float *__restrict__ y,
@@ -174,9 +150,9 @@ q6_k_gemm_kernel(const uint8_t *__restrict__ w, const uint16_t *__restrict__ x, 
             for (int c = 0; c < 4; ++c) {
                 const uint32_t ks = sb * 4u + c;
                 if (c == 1)
-                    LEV_Q6G_WAIT_VMCNT(18);
+                    LEV_WAIT_VMCNT(18);
                 else
-                    LEV_Q6G_WAIT_VMCNT(8);
+                    LEV_WAIT_VMCNT(8);
                 __builtin_amdgcn_s_waitcnt(0xC07F);   // this wave's B fragments of step ks are in LDS
                 asm volatile("s_barrier" ::: "memory");
                 __builtin_amdgcn_sched_barrier(0);   // a step's decode stays inside the step
@@ -197,7 +173,7 @@ q6_k_gemm_kernel(const uint8_t *__restrict__ w, const uint16_t *__restrict__ x, 
             }
         }
         }
-        LEV_Q6G_WAIT_VMCNT(0);
+        LEV_WAIT_VMCNT(0);
         return;
     }
 
@@ -284,6 +260,8 @@ q6_k_gemm_kernel(const uint8_t *__restrict__ w, const uint16_t *__restrict__ x, 
 
 hipError_t lev_q6_k_gemm_launch(lev_ctx *ctx, const uint8_t *w, const uint16_t *x, float *y,
                                 uint32_t in_dim, uint32_t rows, uint32_t tokens) {
+    const lev_gemm_split_plan plan = lev_gemm_split_choose(ctx, true, in_dim, rows, tokens, kTR);
+    if (plan.kw) return lev_gemm_split_launch(ctx, true, w, x, y, in_dim, rows, tokens, plan);
     static bool attr_set = false;
     const size_t lds = (size_t)kRXBufs * kRXBuf + 2 * kRBBuf;   // 160 KB: one workgroup per CU
     if (!attr_set) {
