@@ -990,35 +990,40 @@ moe_down_kernel(moe_args a, const float *__restrict__ act, const int32_t *__rest
 // its own (no workgroup barrier in front of the products) and keeps the operands in registers.
 // ---------------------------------------------------------------------------
 
-constexpr int kMmWaves = 8;
+constexpr int kMmWaves = 8;                       // of a down workgroup
 constexpr int kMmThreads = kMmWaves * LEV_WAVE;
-constexpr uint32_t kGumPartBytes = 2u * 2u * kMmWaves * 16u * 4u;   // [round parity][gate, up][wave][row] f32
+// bytes of [gate, up][wave][row] f32 of a round of gate/up: a power of two, so that the parity is one XOR away
+__host__ __device__ constexpr uint32_t gum_part_bytes(int nw) { return 2u * (nw <= 8 ? 8u : 16u) * 16u * 4u; }
 
-__host__ __device__ constexpr size_t mm_areas_bytes(uint32_t tpw) {
-    return (size_t)kMmWaves * (tpw * kQ4mTaskArea + kQ4mZeroBytes);
+__host__ __device__ constexpr size_t mm_areas_bytes(uint32_t waves, uint32_t tpw) {
+    return (size_t)waves * (tpw * kQ4mTaskArea + kQ4mZeroBytes);
 }
 
-// grid (chunks, top_k, tokens), 8 waves.  Wave w multiplies the column tasks w*TPW.. of gate row
-// group i AND of up row group i (the same operands); the eight partial sums of a row meet in LDS
-// and wave 0 writes act = gelu_tanh(g) * u.  A workgroup takes rows_per_block rows in groups of 16
-// with the next group's weights in flight.
+// grid (chunks, top_k, tokens), NW waves (at least one per 256-value column task).  Wave w multiplies the
+// column task w of gate row group i AND of up row group i (the same operands); the partial sums of a
+// row meet in LDS and wave 0 writes act = gelu_tanh(g) * u.  A workgroup takes rows_per_block rows in groups of
+// 16 with the next group's weights in flight; SINGLE: one group, nothing to prefetch.  Registers for two
+// workgroups a CU.  A wave per task up to 4096 wide: at hidden 2816 eight waves of two tasks took 11.7 us a layer
+// (five of them idle for half of the time), twelve take 8.4.
 // ROUTE > 0 (experts <= 64*ROUTE): the expert comes from this token's router scores, ranked by
 // wave 0 alone while the other waves' activation requests are on their way (every workgroup of a
 // token repeats the selection, which costs less than a kernel boundary; one wave ranking costs an
 // eighth of the vector instructions of eight); the first workgroup of a token publishes ids and
 // weights.  Otherwise the ids are read from `ids`.
-// LDS: part | expert word | task areas | router area (ROUTE > 0)
-template <int TPW, int ROUTE>
-__global__ void __launch_bounds__(kMmThreads)
+// LDS: part [2] | expert word | task areas | router area (ROUTE > 0)
+template <int NW, bool SINGLE, int ROUTE>
+__global__ void __launch_bounds__(NW * LEV_WAVE, SINGLE || NW < 16 ? NW / 2 : NW / 4)
 moe_gate_up_mfma(moe_args a, const float *__restrict__ x, const int32_t *ids, const float *__restrict__ scores,
                  const float *__restrict__ expert_scale, int32_t *ids_out, float *weights_out,
                  float *__restrict__ act, int *__restrict__ flag, uint32_t rows_per_block) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    constexpr uint32_t kPart = gum_part_bytes(NW), kUp = kPart / 2u;
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
     const uint32_t slot = blockIdx.y, t = blockIdx.z;
-    const uint32_t ntask = a.hidden >> 8;
-    const uint32_t t_first = wave * TPW;
+    const uint32_t npairs = a.hidden >> 6, ntask = (npairs + 3u) >> 2;
+    const bool active = wave < ntask;
+    const uint32_t T = active ? wave : ntask - 1u;
     const float *xt = x + (uint64_t)t * a.hidden;
 
     // request order = return order: the scores (the expert, and with it every weight address,
@@ -1027,17 +1032,13 @@ moe_gate_up_mfma(moe_args a, const float *__restrict__ x, const int32_t *ids, co
     if constexpr (ROUTE > 0) {
         if (wave == 0u) router_load_scores<ROUTE>(scores + (uint64_t)t * a.experts, a.experts, sc);
     }
-    lev_f32x4 v[TPW];
-#pragma unroll
-    for (int k = 0; k < TPW; ++k) {
-        const uint32_t T = t_first + k < ntask ? t_first + k : ntask - 1u;
-        v[k] = reinterpret_cast<const lev_f32x4 *>(xt)[64u * T + lane];
-    }
+    bool v_live;
+    lev_f32x4 v = q4m_load_activations(xt, T, a.hidden >> 2, v_live);
 
-    uint32_t *s_e = reinterpret_cast<uint32_t *>(smem + kGumPartBytes);
-    uint8_t *area = smem + kGumPartBytes + 16u + (size_t)wave * (TPW * kQ4mTaskArea + kQ4mZeroBytes);
-    uint8_t *zero = area + TPW * kQ4mTaskArea;
-    void *rl = smem + kGumPartBytes + 16u + mm_areas_bytes(TPW);
+    uint32_t *s_e = reinterpret_cast<uint32_t *>(smem + 2u * kPart);
+    uint8_t *area = smem + 2u * kPart + 16u + (size_t)wave * (kQ4mTaskArea + kQ4mZeroBytes);
+    uint8_t *zero = area + kQ4mTaskArea;
+    void *rl = smem + 2u * kPart + 16u + mm_areas_bytes(NW, 1u);
     uint32_t e;
     bool ok = true;
     const bool publisher = ROUTE > 0 && blockIdx.x == 0 && slot == 0;
@@ -1071,18 +1072,14 @@ moe_gate_up_mfma(moe_args a, const float *__restrict__ x, const int32_t *ids, co
     const uint32_t i_begin = blockIdx.x * rows_per_block;
     const uint32_t i_end = min(i_begin + rows_per_block, a.inter);
     const uint32_t lrow = lane >> 2;                              // fetch order: lane = 4 * row + pair
-    auto issue = [&](uint32_t i0, uint32_t (&Dg)[TPW][9], uint32_t (&Du)[TPW][9]) {
+    auto issue = [&](uint32_t i0, uint32_t (&Dg)[9], uint32_t (&Du)[9]) {
         uint32_t row = i0 + lrow;
         row = row < i_end ? row : i_end - 1u;
         const uint64_t off = (uint64_t)row * row_bytes;
-#pragma unroll
-        for (int k = 0; k < TPW; ++k) {
-            const uint32_t T = t_first + k < ntask ? t_first + k : ntask - 1u;
-            q4m_load_task(gbase + off, 4u * T, Dg[k]);
-            q4m_load_task(ubase + off, 4u * T, Du[k]);
-        }
+        q4m_load_task_part(gbase + off, 4u * T, npairs, Dg);
+        q4m_load_task_part(ubase + off, 4u * T, npairs, Du);
     };
-    uint32_t Ga[TPW][9], Ua[TPW][9];
+    uint32_t Ga[9], Ua[9];
     uint32_t i0 = i_begin;
     issue(i0, Ga, Ua);
 
@@ -1103,49 +1100,53 @@ moe_gate_up_mfma(moe_args a, const float *__restrict__ x, const int32_t *ids, co
     }
     const uint32_t r16 = lane & 15u, q = lane >> 4;
     uint32_t pw = (wave * 16u + lane) * 4u;                       // byte offsets into `part`: gate, then up at + 512
-    uint32_t pr = (q * 16u + r16) * 4u;                           // wave 0: lane (r, q) adds waves q and q + 4
+    uint32_t pr = (q * 16u + r16) * 4u;                           // wave 0: lane (r, q) adds waves q, q + 4, ..
     float *arow = act + ((uint64_t)t * a.top_k + slot) * a.inter;
     lev_pin(pw);
     lev_pin(pr);
     if (lane < kQ4mZeroBytes / 4u) reinterpret_cast<uint32_t *>(zero)[lane] = 0u;
-    q4m_operand op[TPW];
-#pragma unroll
-    for (int k = 0; k < TPW; ++k) q4m_stage_task(v[k], area + k * kQ4mTaskArea, zero, t_first + k < ntask, op[k]);
+    q4m_operand op;
+    q4m_stage_task(q4m_mask_activations(v, v_live), area, zero, active, op);
     __builtin_amdgcn_sched_barrier(0);
 
-    auto finish = [&](uint32_t i_here, const uint32_t (&Dg)[TPW][9], const uint32_t (&Du)[TPW][9]) {
-        float vg = 0.f, vu = 0.f;
-#pragma unroll
-        for (int k = 0; k < TPW; ++k) {
-            uint32_t W[9];
-            q4m_turn_task(Dg[k], W);
-            vg += q4m_task_dot(W, op[k]);
-            q4m_turn_task(Du[k], W);
-            vu += q4m_task_dot(W, op[k]);
-        }
+    auto finish = [&](uint32_t i_here, const uint32_t (&Dg)[9], const uint32_t (&Du)[9]) {
+        uint32_t W[9];
+        q4m_turn_task(Dg, W);
+        float vg = q4m_task_dot(W, op);
+        q4m_turn_task(Du, W);
+        float vu = q4m_task_dot(W, op);
         vg = q4m_row_sum(vg);
         vu = q4m_row_sum(vu);
         if (lane < 16u) {
             *reinterpret_cast<float *>(smem + pw) = vg;
-            *reinterpret_cast<float *>(smem + pw + kMmWaves * 16u * 4u) = vu;
+            *reinterpret_cast<float *>(smem + pw + kUp) = vu;
         }
         lev_barrier_lds();
         if (wave == 0u) {
-            const float *pp = reinterpret_cast<const float *>(smem + pr);
-            const float g0 = pp[0], g1 = pp[64], u0 = pp[128], u1 = pp[192];
-            const float g = q4m_row_sum(g0 + g1), u = q4m_row_sum(u0 + u1);
+            const float *pg = reinterpret_cast<const float *>(smem + pr), *pu = reinterpret_cast<const float *>(smem + pr + kUp);
+            float g = pg[0] + pg[64], u = pu[0] + pu[64];
+            if (NW > 8) {
+                g += pg[128];
+                u += pu[128];
+            }
+            if (NW > 12) {
+                g += pg[192];
+                u += pu[192];
+            }
+            g = q4m_row_sum(g);
+            u = q4m_row_sum(u);
             if (q == 0u && i_here + r16 < i_end) arow[i_here + r16] = lev_gelu_up_value(g, u);
         }
-        pw ^= kGumPartBytes / 2u;                                 // the other half of `part` next round
-        pr ^= kGumPartBytes / 2u;
+        pw ^= kPart;                                              // the other half of `part` next round
+        pr ^= kPart;
     };
-    if (rows_per_block <= 16u) {   // one group per workgroup: nothing to prefetch
+    if (SINGLE) {
         finish(i0, Ga, Ua);
         return;
     }
     // unconditional (clamped) prefetch: a branch around the loads would make the compiler wait
     // for them before the current group is multiplied
-    uint32_t Gb[TPW][9], Ub[TPW][9];
+    uint32_t Gb[9], Ub[9];
     while (true) {
         uint32_t next = i0 + 16u;
         issue(next < i_end ? next : i0, Gb, Ub);
@@ -1173,7 +1174,7 @@ moe_down_mfma(moe_args a, const float *__restrict__ act, const int32_t *__restri
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
     const uint32_t t = blockIdx.y;
-    const uint32_t ntask = a.inter >> 8;
+    const uint32_t npairs = a.inter >> 6, ntask = (npairs + 3u) >> 2;
     const uint32_t row_begin = blockIdx.x * tile;
     const uint32_t row_end = min(row_begin + tile, a.hidden);
     float *partial = reinterpret_cast<float *>(smem);                       // [top_k][16]
@@ -1195,10 +1196,11 @@ moe_down_mfma(moe_args a, const float *__restrict__ act, const int32_t *__restri
         const int32_t ids_mine = expert_ids_request(tids, a.top_k);
         const float *av = act + ((uint64_t)t * a.top_k + slot) * a.inter;
         lev_f32x4 v[TPW];
+        bool v_live[TPW];
 #pragma unroll
         for (int k = 0; k < TPW; ++k) {
             const uint32_t T = (uint32_t)k < ntask ? (uint32_t)k : ntask - 1u;
-            v[k] = reinterpret_cast<const lev_f32x4 *>(av)[64u * T + lane];
+            v[k] = q4m_load_activations(av, T, a.inter >> 2, v_live[k]);
         }
         uint32_t e;
         if (!expert_ids_verdict(ids_mine, a.top_k, slot, a.experts, &e)) {
@@ -1212,12 +1214,13 @@ moe_down_mfma(moe_args a, const float *__restrict__ act, const int32_t *__restri
 #pragma unroll
         for (int k = 0; k < TPW; ++k) {
             const uint32_t T = (uint32_t)k < ntask ? (uint32_t)k : ntask - 1u;
-            q4m_load_task(rowp, 4u * T, D[k]);
+            q4m_load_task_part(rowp, 4u * T, npairs, D[k]);
         }
         // the slot's activations become operands while its weights are on their way
         q4m_operand op[TPW];
 #pragma unroll
-        for (int k = 0; k < TPW; ++k) q4m_stage_task(v[k], area + k * kQ4mTaskArea, zero, (uint32_t)k < ntask, op[k]);
+        for (int k = 0; k < TPW; ++k)
+            q4m_stage_task(q4m_mask_activations(v[k], v_live[k]), area + k * kQ4mTaskArea, zero, (uint32_t)k < ntask, op[k]);
         __builtin_amdgcn_sched_barrier(0);
         float val = 0.f;
 #pragma unroll
@@ -1398,35 +1401,50 @@ hipError_t launch_down(lev_ctx *ctx, const moe_args &a, const float *act, const 
     return hipGetLastError();
 }
 
-// Shapes the matrix-core expert kernels take: rows of whole 256-value tasks, at most two tasks a
-// wave for gate/up (the hidden dimension is split over the eight waves), at most four for down
-// (a wave reduces over the whole intermediate dimension).
-bool gate_up_mfma_ok(const moe_args &a) { return a.hidden % 256u == 0u && a.hidden <= 4096u; }
-bool down_mfma_ok(const moe_args &a) { return a.inter % 256u == 0u && a.inter <= 1024u; }
+// Shapes the matrix-core expert kernels take (block pairs: hidden and inter are multiples of 64): a wave per
+// column task for gate/up, sixteen at most; for down a wave reduces over the whole intermediate dimension,
+// four tasks at most.
+bool gate_up_mfma_ok(const moe_args &a) { return a.hidden % 64u == 0u && a.hidden <= 4096u; }
+bool down_mfma_ok(const moe_args &a) { return a.inter % 64u == 0u && a.inter <= 1024u; }
+
+template <int NW, int ROUTE>
+void launch_gate_up_as(lev_ctx *ctx, const moe_args &a, const float *x, const gu_route &rt, float *act, const dim3 &grid,
+                       uint32_t rows_per_block) {
+    const size_t lds = 2u * gum_part_bytes(NW) + 16u + mm_areas_bytes(NW, 1u) + (ROUTE ? router_lds_bytes(ROUTE) + 8u : 0u);
+#define LEV_GUM(SINGLE)                                                                                            \
+    hipLaunchKernelGGL((moe_gate_up_mfma<NW, SINGLE, ROUTE>), grid, dim3(NW * LEV_WAVE), lds, ctx->stream, a, x, rt.ids, \
+                       rt.scores, rt.expert_scale, rt.ids_out, rt.weights_out, act, ctx->d_flag, rows_per_block)
+    if (rows_per_block <= 16u) LEV_GUM(true);
+    else LEV_GUM(false);
+#undef LEV_GUM
+}
 
 hipError_t launch_gate_up_mfma(lev_ctx *ctx, const moe_args &a, const float *x, const gu_route &rt,
                                float *act, uint32_t tokens, uint32_t per_cu) {
-    const uint64_t slots = (uint64_t)a.top_k * tokens;
-    uint32_t want = (uint32_t)(((uint64_t)ctx->num_cus * per_cu + slots - 1) / slots);
-    if (want < 1) want = 1;
-    const uint32_t rows_per_block = (a.inter + want - 1) / want;
+    // A group is 16 rows.  `most` workgroups of one group fit a CU at once: while three rounds of them hold all rows, a
+    // workgroup takes one group, as small as the same number of workgroups a CU allows (3968 / 1472, top-6, one token:
+    // 18 rows a workgroup are two groups, the second of two rows); beyond, several whole groups with the next one's
+    // weights in flight.  per_cu: at least that many workgroups a CU (a schedule's field; built in: 2).
+    const uint64_t rows = (uint64_t)a.inter * a.top_k * tokens, cus = (uint64_t)ctx->num_cus;
+    const uint64_t most = a.hidden <= 2048u ? 4u : 2u;
+    uint64_t per = (rows + 16u * cus - 1) / (16u * cus);                          // groups a CU
+    if (per > most) per = (per + most - 1) / most * most;                         // whole rounds
+    if (per < per_cu) per = per_cu;
+    const uint64_t want = per <= 3u * most && (most == 2u || per <= most) ? (rows + per * cus - 1) / (per * cus)
+                                                                          : 16u * ((rows + 32u * cus - 1) / (32u * cus));
+    const uint32_t rows_per_block = want < a.inter ? (uint32_t)want : a.inter;
     const uint32_t chunks = (a.inter + rows_per_block - 1) / rows_per_block;
-    const uint32_t tpw = a.hidden > 2048u ? 2u : 1u;
     const uint32_t route = rt.ids ? 0u : a.experts <= 128u ? 2u : 4u;      // callers keep experts <= kRouteInKernelMax
-    const size_t lds = kGumPartBytes + 16u + mm_areas_bytes(tpw) + (route ? router_lds_bytes(route) + 8u : 0u);
     const dim3 grid(chunks, a.top_k, tokens);
-#define LEV_GUM(TPW, ROUTE)                                                                          \
-    hipLaunchKernelGGL((moe_gate_up_mfma<TPW, ROUTE>), grid, dim3(kMmThreads), lds, ctx->stream, a, x, rt.ids,   \
-                       rt.scores, rt.expert_scale, rt.ids_out, rt.weights_out, act, ctx->d_flag, rows_per_block)
-    if (tpw == 1u) {
-        if (route == 0u) LEV_GUM(1, 0);
-        else if (route == 2u) LEV_GUM(1, 2);
-        else LEV_GUM(1, 4);
-    } else {
-        if (route == 0u) LEV_GUM(2, 0);
-        else if (route == 2u) LEV_GUM(2, 2);
-        else LEV_GUM(2, 4);
+#define LEV_GUM(NW)                                                                             \
+    {                                                                                           \
+        if (route == 0u) launch_gate_up_as<NW, 0>(ctx, a, x, rt, act, grid, rows_per_block);    \
+        else if (route == 2u) launch_gate_up_as<NW, 2>(ctx, a, x, rt, act, grid, rows_per_block); \
+        else launch_gate_up_as<NW, 4>(ctx, a, x, rt, act, grid, rows_per_block);                \
     }
+    if (a.hidden <= 2048u) LEV_GUM(8)
+    else if (a.hidden <= 3072u) LEV_GUM(12)
+    else LEV_GUM(16)
 #undef LEV_GUM
     return hipGetLastError();
 }
@@ -1440,7 +1458,7 @@ hipError_t launch_down_mfma(lev_ctx *ctx, const moe_args &a, const float *act, c
     tile = tile < 4u ? 4u : tile > 16u ? 16u : tile;
     const uint32_t tiles = (a.hidden + tile - 1) / tile;
     const uint32_t tpw = (a.inter + 255u) / 256u;
-    const size_t lds = (size_t)a.top_k * 64u + 256u + mm_areas_bytes(tpw);
+    const size_t lds = (size_t)a.top_k * 64u + 256u + mm_areas_bytes(kMmWaves, tpw);
     const dim3 grid(tiles, tokens);
 #define LEV_DNM(TPW)                                                                                 \
     hipLaunchKernelGGL((moe_down_mfma<TPW>), grid, dim3(kMmThreads), lds, ctx->stream, a, act, ids, weights, y, \

@@ -99,6 +99,24 @@ __device__ __forceinline__ void q4m_load_task(const uint8_t *rowp, uint32_t task
     lev_q4_load_pair(rowp + (uint64_t)(task_pair0 + (lane & 3u)) * 36u, D);
 }
 
+// The same where the row's last task may be a part of one (npairs pairs a row): lanes past the row's end
+// repeat its last pair.  Their activations count as zero (q4m_load_activations).
+__device__ __forceinline__ void q4m_load_task_part(const uint8_t *rowp, uint32_t task_pair0, uint32_t npairs, uint32_t D[9]) {
+    const uint32_t pair = task_pair0 + (threadIdx.x & 3u);
+    lev_q4_load_pair(rowp + (uint64_t)((pair < npairs ? pair : npairs - 1u) * 36u), D);
+}
+
+// The 256 activations of task T of a vector of n4 float4: lane i requests elements 4i..4i+3; past the end the
+// vector's last ones are requested, and `live` (what to pass to q4m_mask_activations behind the wait) is false.
+__device__ __forceinline__ lev_f32x4 q4m_load_activations(const float *x, uint32_t T, uint32_t n4, bool &live) {
+    const uint32_t i = 64u * T + (threadIdx.x & 63u);
+    live = i < n4;
+    return reinterpret_cast<const lev_f32x4 *>(x)[live ? i : n4 - 1u];
+}
+__device__ __forceinline__ lev_f32x4 q4m_mask_activations(lev_f32x4 v, bool live) {
+    return live ? v : lev_f32x4{0.f, 0.f, 0.f, 0.f};
+}
+
 // Lane (r, g) <- lane 4*r + g, for every dword of a fetched task.
 __device__ __forceinline__ void q4m_turn_task(const uint32_t D[9], uint32_t W[9]) {
     const uint32_t lane = threadIdx.x & 63u;

@@ -53,3 +53,22 @@ def test_moe_grouped_integer_kernels_ragged_rows(ctx, hidden, inter, experts, to
         assert O.max_rel_err(act[t], ref["act"]) < TOL
         y32, _ = O.moe_experts_f32(g, u, d, hidden, inter, ids[t], wts[t], x[t])
         assert O.max_rel_err(y[t], ref["y"]) < max(TOL, 1.5 * O.max_rel_err(y32, ref["y"]))
+
+
+@pytest.mark.parametrize("hidden,inter,experts,top_k,tokens", [
+    (3136, 960, 6, 4, 1),         # thirteen column tasks a row, the last of one pair; four, the last of three
+    (2112, 64, 4, 2, 3), (4032, 448, 5, 3, 4), (192, 704, 9, 8, 2),
+])
+def test_moe_few_tokens_ragged_rows(ctx, hidden, inter, experts, top_k, tokens):
+    """The few-token matrix-core kernels on rows that end inside a 256-value task."""
+    wr, pool, offs, x = H.config5(hidden, inter, experts, tokens, seed=hidden + inter)
+    rng = np.random.default_rng(tokens)
+    ids = np.stack([rng.permutation(experts)[:top_k] for _ in range(tokens)]).astype(np.int32)
+    wts = rng.random((tokens, top_k)).astype(np.float32)
+    y, act = run_experts(ctx, pool, offs, hidden, inter, experts, x, ids, wts)
+    g, u, d = (pool[offs["gate_off"]:], pool[offs["up_off"]:], pool[offs["down_off"]:])
+    for t in range(tokens):
+        ref = O.moe_experts_f64(g, u, d, hidden, inter, ids[t], wts[t], x[t])
+        assert O.max_rel_err(act[t], ref["act"]) < TOL
+        y32, _ = O.moe_experts_f32(g, u, d, hidden, inter, ids[t], wts[t], x[t])
+        assert O.max_rel_err(y[t], ref["y"]) < max(TOL, 1.5 * O.max_rel_err(y32, ref["y"]))
