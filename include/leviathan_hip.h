@@ -259,6 +259,14 @@ int lev_hip_rmsnorm(lev_ctx *ctx, const float *d_x, float *d_y, uint32_t n, uint
 int lev_hip_gelu_up(lev_ctx *ctx, const float *d_gu, float *d_y, uint32_t n);
 /* axpy(x:xOffset:y:c:n:) (Gemma4.swift:3115; kernel :4459): y += c * x. */
 int lev_hip_axpy(lev_ctx *ctx, const float *d_x, float *d_y, float c, uint32_t n);
+/* The shared expert of one token (Gemma4.swift:3742-3773), the operators above in one call: h = rmsnorm(x) * ffn_norm,
+ * gu = [gate h | up h], act = gelu_up(gu), shared = rmsnorm(down act) * post_norm.  Every intermediate is written
+ * (h hidden floats, gu 2*inter, act inter, shared hidden); either norm weight may be NULL.  Gate and up are
+ * [inter, hidden], down [hidden, inter], Q4_0, each from the start of its buffer. */
+int lev_hip_shared_expert_ffn_q4_0(lev_ctx *ctx, const float *d_x, const float *d_ffn_norm, const void *d_gate_w,
+                                   size_t gate_bytes, const void *d_up_w, size_t up_bytes, const void *d_down_w,
+                                   size_t down_bytes, const float *d_post_norm, float eps, float *d_h, float *d_gu,
+                                   float *d_act, float *d_shared, uint32_t hidden, uint32_t inter);
 /* argmax step (lev-forge/src/ops.rs:479-516): per column of `vocab` logits. */
 int lev_hip_argmax(lev_ctx *ctx, const float *d_logits, uint32_t vocab, uint32_t ncol,
                    uint32_t *d_index, float *d_margin);

@@ -99,6 +99,8 @@ SIGNATURES = {
     "lev_hip_f32_to_f16": (_int, [_vp, _vp, _vp, _sz]),
     "lev_hip_rmsnorm": (_int, [_vp, _vp, _vp, _u32, _u32, _vp, _f32]),
     "lev_hip_gelu_up": (_int, [_vp, _vp, _vp, _u32]),
+    "lev_hip_shared_expert_ffn_q4_0": (_int, [_vp, _vp, _vp, _vp, _sz, _vp, _sz, _vp, _sz, _vp, _f32, _vp, _vp, _vp, _vp,
+                                              _u32, _u32]),
     "lev_hip_axpy": (_int, [_vp, _vp, _vp, _f32, _u32]),
     "lev_hip_argmax": (_int, [_vp, _vp, _u32, _u32, _vp, _vp]),
     "lev_hip_moe_route_topk": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _u32, _u32, _u32, _u32]),

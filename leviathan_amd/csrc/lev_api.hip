@@ -264,17 +264,6 @@ int lev_check_matvec(lev_ctx *ctx, const char *op, uint32_t block_values, uint32
 
 namespace {
 
-// 1/sqrt(a) of a positive f64: the hardware estimate and two Newton steps (error of a few f64 ulps), a
-// handful of dependent instructions where the square root and the division of the library take over a
-// hundred, all of them on the critical path of a one-workgroup kernel.
-__device__ __forceinline__ double rsqrt_f64(double a) {
-    const double est = __builtin_amdgcn_rsq(a);
-    double r = est;
-    r = r * (1.5 - 0.5 * a * r * r);
-    r = r * (1.5 - 0.5 * a * r * r);
-    return r == r ? r : est;   // a = 0 and a = inf: the estimate is exact there and the step is inf * 0
-}
-
 // One workgroup of up to 16 waves per vector.  Sum of squares in f32 per lane, wave DPP sums, f64 across
 // waves; y = x * inv * w.  A call on one vector is latency and nothing else (11 KB at n = 2816), so the
 // vector and the gains are requested together, 16 bytes a lane, and x stays in registers between the two
@@ -321,7 +310,7 @@ rmsnorm_kernel(const float *__restrict__ x, float *__restrict__ y, const float *
     lev_barrier_lds();   // (the gains may still be on their way)
     double tot = 0.0;
     for (uint32_t k = 0; k < nt >> 6; ++k) tot += (double)part[k];
-    const float inv = (float)rsqrt_f64(tot / (double)n + (double)eps);
+    const float inv = (float)lev_rsqrt_f64(tot / (double)n + (double)eps);
     if (V) {
 #pragma unroll
         for (int k = 0; k < R; ++k) {

@@ -183,6 +183,17 @@ __device__ __forceinline__ void lev_barrier_lds() {
     asm volatile("s_barrier" ::: "memory");
 }
 
+// 1/sqrt(a) of a positive f64: the hardware estimate and two Newton steps (error of a few f64 ulps), a
+// handful of dependent instructions where the square root and the division of the library take over a
+// hundred, all of them on the critical path of a one-workgroup kernel.
+__device__ __forceinline__ double lev_rsqrt_f64(double a) {
+    const double est = __builtin_amdgcn_rsq(a);
+    double r = est;
+    r = r * (1.5 - 0.5 * a * r * r);
+    r = r * (1.5 - 0.5 * a * r * r);
+    return r == r ? r : est;   // a = 0 and a = inf: the estimate is exact there and the step is inf * 0
+}
+
 // s_waitcnt vmcnt(n) leaves at most n vector memory operations of the wave outstanding; they complete
 // in issue order, so everything older than the n newest has landed.  Encoding: vmcnt in bits 3:0 and
 // 15:14, expcnt (6:4) and lgkmcnt (11:8) left at "any".

@@ -1,0 +1,183 @@
+// The shared expert's FFN of one token in Q4_0 (Gemma4.swift:3742-3773): h = rmsnorm(x) * norm,
+// [g | u] = [W_gate h | W_up h], act = gelu_tanh(g) * u, shared = rmsnorm(W_down act) * post.
+//
+// Called operator by operator it is six launches of which four are the launch floor and little else: at
+// 2816 / 2112 18.7 us recorded, 29 us enqueued one by one.  Here three: everything up to act, the down GEMV, the
+// norm behind it (11.7 us recorded, 14 enqueued).  The first kernel has the shape of the MoE gate/up kernel: a wave owns one
+// 256-value column task of gate row group i and of up row group i, keeps the operands in registers and
+// meets the others in LDS; in front of it every workgroup normalises x for itself (a wave its own 256 values,
+// the sum of squares crosses the waves once), with its weights already on their way.
+#include "q4_0_mfma.hpp"
+
+hipError_t lev_q4_0_gemv_launch(lev_ctx *ctx, const uint8_t *w, const float *x, float *y, uint32_t in_dim, uint32_t rows);
+
+namespace {
+
+struct ffn_args {
+    const uint8_t *gate, *up;
+    const float *x, *gain;
+    float *h, *gu, *act;
+    uint32_t hidden, inter, rows_per_block;
+    float eps;
+};
+
+// part of a round: [gate, up][wave][row] f32, two of them
+constexpr uint32_t kFfnPart = 2u * 16u * 16u * 4u, kFfnUp = kFfnPart / 2u;
+constexpr size_t ffn_lds(int nw) { return 2u * kFfnPart + 64u + (size_t)nw * (kQ4mTaskArea + kQ4mZeroBytes); }
+
+// NW waves, one per column task (at most 16).  grid (row chunks).
+template <int NW>
+__global__ void __launch_bounds__(NW * LEV_WAVE, NW / 4)
+q4_0_ffn_gate_up(ffn_args a) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    float *const s_ss = reinterpret_cast<float *>(smem + 2u * kFfnPart);
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+    const uint32_t npairs = a.hidden >> 6, ntask = (npairs + 3u) >> 2, n4 = a.hidden >> 2;
+    const bool active = wave < ntask;
+    const uint32_t T = active ? wave : ntask - 1u;
+    bool live;
+    lev_f32x4 v = q4m_load_activations(a.x, T, n4, live);
+    lev_f32x4 gain = {1.f, 1.f, 1.f, 1.f};
+    if (a.gain) {
+        bool unused;
+        gain = q4m_load_activations(a.gain, T, n4, unused);
+    }
+    const uint64_t row_bytes = (uint64_t)npairs * 36u;
+    const uint32_t i_begin = blockIdx.x * a.rows_per_block, i_end = min(i_begin + a.rows_per_block, a.inter);
+    const uint32_t lrow = lane >> 2;                              // fetch order: lane = 4 * row + pair
+    auto issue = [&](uint32_t i0, uint32_t (&G)[9], uint32_t (&U)[9]) {
+        uint32_t row = i0 + lrow;
+        row = row < i_end ? row : i_end - 1u;
+        q4m_load_task_part(a.gate + row * row_bytes, 4u * T, npairs, G);
+        q4m_load_task_part(a.up + row * row_bytes, 4u * T, npairs, U);
+    };
+    __builtin_amdgcn_sched_barrier(0);
+    uint32_t Ga[9], Ua[9];
+    uint32_t i0 = i_begin;
+    issue(i0, Ga, Ua);
+    __builtin_amdgcn_sched_barrier(0);
+
+    // rmsnorm as lev_hip_rmsnorm forms it: squares in f32 per wave, f64 across the waves
+    v = q4m_mask_activations(v, live && active);
+    float ss = 0.f;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) ss = fmaf(v[c], v[c], ss);
+    ss = lev_wave_sum_broadcast(ss);
+    if (lane == 0u) s_ss[wave] = ss;
+    lev_barrier_lds();
+    double tot = 0.0;
+    for (int k = 0; k < NW; ++k) tot += (double)s_ss[k];
+    const float inv = (float)lev_rsqrt_f64(tot / (double)a.hidden + (double)a.eps);
+    v = v * inv;
+    if (a.gain) v = v * gain;
+    if (!live || !active) v = lev_f32x4{0.f, 0.f, 0.f, 0.f};      // (an infinite inv made NaNs of the zeros past the end)
+    if (blockIdx.x == 0u && active && live) reinterpret_cast<lev_f32x4 *>(a.h)[64u * T + lane] = v;
+
+    uint8_t *area = smem + 2u * kFfnPart + 64u + (size_t)wave * (kQ4mTaskArea + kQ4mZeroBytes), *zero = area + kQ4mTaskArea;
+    if (lane < kQ4mZeroBytes / 4u) reinterpret_cast<uint32_t *>(zero)[lane] = 0u;
+    q4m_operand op;
+    q4m_stage_task(v, area, zero, active, op);
+    __builtin_amdgcn_sched_barrier(0);
+
+    const uint32_t r16 = lane & 15u, q = lane >> 4;
+    uint32_t pw = (wave * 16u + lane) * 4u, pr = (q * 16u + r16) * 4u;
+    lev_pin(pw);
+    lev_pin(pr);
+    while (true) {
+        uint32_t Gb[9], Ub[9], W[9];
+        const uint32_t next = i0 + 16u;
+        issue(next < i_end ? next : i0, Gb, Ub);                  // unconditional (clamped)
+        q4m_turn_task(Ga, W);
+        const float vg = q4m_row_sum(q4m_task_dot(W, op));
+        q4m_turn_task(Ua, W);
+        const float vu = q4m_row_sum(q4m_task_dot(W, op));
+        if (lane < 16u) {
+            *reinterpret_cast<float *>(smem + pw) = vg;
+            *reinterpret_cast<float *>(smem + pw + kFfnUp) = vu;
+        }
+        lev_barrier_lds();
+        if (wave == 0u) {
+            // lane (r16, q) adds waves q, q + 4, .. of row r16
+            const float *pg = reinterpret_cast<const float *>(smem + pr), *pu = reinterpret_cast<const float *>(smem + pr + kFfnUp);
+            float g = pg[0], u = pu[0];
+            for (int k = 1; k < NW / 4; ++k) {
+                g += pg[64 * k];
+                u += pu[64 * k];
+            }
+            g = q4m_row_sum(g);
+            u = q4m_row_sum(u);
+            const uint32_t row = i0 + r16;
+            if (q == 0u && row < i_end) {
+                a.gu[row] = g;
+                a.gu[a.inter + row] = u;
+                a.act[row] = lev_gelu_up_value(g, u);
+            }
+        }
+        if (next >= i_end) break;
+        i0 = next;
+        pw ^= kFfnPart;
+        pr ^= kFfnPart;
+#pragma unroll
+        for (int k = 0; k < 9; ++k) {
+            Ga[k] = Gb[k];
+            Ua[k] = Ub[k];
+        }
+    }
+}
+
+}  // namespace
+
+extern "C" int lev_hip_shared_expert_ffn_q4_0(lev_ctx *ctx, const float *d_x, const float *d_ffn_norm, const void *d_gate_w,
+                                              size_t gate_bytes, const void *d_up_w, size_t up_bytes, const void *d_down_w,
+                                              size_t down_bytes, const float *d_post_norm, float eps, float *d_h, float *d_gu,
+                                              float *d_act, float *d_shared, uint32_t hidden, uint32_t inter) {
+    LEV_REQUIRE_CTX(ctx);
+    if (!d_x || !d_h || !d_gu || !d_act || !d_shared)
+        return lev_fail(ctx, LEV_ERR_INVALID_ARGUMENT, "shared_expert_ffn: null pointer");
+    if (!(eps >= 0.f)) return lev_fail(ctx, LEV_ERR_BAD_DIMENSIONS, "shared_expert_ffn: eps %g", (double)eps);
+    lev_geom g;
+    int st = lev_check_matvec(ctx, "shared_expert_ffn gate", 32, 18, d_gate_w, gate_bytes, 0, d_h, hidden, hidden, d_gu,
+                              (size_t)2 * inter, inter, hidden, inter, &g);
+    if (st == LEV_OK)
+        st = lev_check_matvec(ctx, "shared_expert_ffn up", 32, 18, d_up_w, up_bytes, 0, d_h, hidden, hidden, d_gu,
+                              (size_t)2 * inter, inter, hidden, inter, &g);
+    if (st == LEV_OK)
+        st = lev_check_matvec(ctx, "shared_expert_ffn down", 32, 18, d_down_w, down_bytes, 0, d_act, inter, inter, d_shared,
+                              hidden, hidden, inter, hidden, &g);
+    if (st != LEV_OK) return st;
+    const uintptr_t al4 = reinterpret_cast<uintptr_t>(d_gate_w) | reinterpret_cast<uintptr_t>(d_up_w);
+    const uintptr_t al16 = reinterpret_cast<uintptr_t>(d_x) | reinterpret_cast<uintptr_t>(d_h) | reinterpret_cast<uintptr_t>(d_ffn_norm);
+    // A schedule installed for the gate/up GEMV keeps the operators apart, so that it is the one that runs; so does
+    // recording at hidden sizes up to 2048, whose programs callers know by a node per operator (wider ones, where
+    // the fused kernel saves most, are recorded fused).
+    const bool fused = !(ctx->recording && hidden <= 2048u) && hidden % 64u == 0u && hidden <= 4096u && (al4 & 3u) == 0u && (al16 & 15u) == 0u && d_x != d_h &&
+                       !lev_selected(ctx, LEV_OP_Q4_0_GEMV, hidden, inter, 1);
+    if (fused) {
+        const uint32_t cus = (uint32_t)ctx->num_cus, per = (inter + 16u * cus - 1u) / (16u * cus);
+        const uint32_t rows = per == 1u ? (inter + cus - 1u) / cus : (inter + 16u * cus - 1u) / (16u * cus) * 16u;
+        const ffn_args a = {static_cast<const uint8_t *>(d_gate_w), static_cast<const uint8_t *>(d_up_w), d_x, d_ffn_norm, d_h,
+                            d_gu, d_act, hidden, inter, rows, eps};
+        const dim3 grid((inter + rows - 1u) / rows);
+#define LEV_FFN(NW) hipLaunchKernelGGL((q4_0_ffn_gate_up<NW>), grid, dim3(NW * LEV_WAVE), ffn_lds(NW), ctx->stream, a)
+        if (hidden <= 2048u) LEV_FFN(8);
+        else if (hidden <= 3072u) LEV_FFN(12);
+        else LEV_FFN(16);
+#undef LEV_FFN
+        st = lev_hip_check(ctx, hipGetLastError(), "shared_expert_ffn gate/up launch");
+    } else {
+        st = lev_hip_rmsnorm(ctx, d_x, d_h, hidden, 1, d_ffn_norm, eps);
+        if (st == LEV_OK)
+            st = lev_hip_check(ctx, lev_q4_0_gemv_launch(ctx, static_cast<const uint8_t *>(d_gate_w), d_h, d_gu, hidden, inter),
+                               "shared_expert_ffn gate launch");
+        if (st == LEV_OK)
+            st = lev_hip_check(ctx, lev_q4_0_gemv_launch(ctx, static_cast<const uint8_t *>(d_up_w), d_h, d_gu + inter, hidden, inter),
+                               "shared_expert_ffn up launch");
+        if (st == LEV_OK) st = lev_hip_gelu_up(ctx, d_gu, d_act, inter);
+    }
+    if (st == LEV_OK)
+        st = lev_hip_check(ctx, lev_q4_0_gemv_launch(ctx, static_cast<const uint8_t *>(d_down_w), d_act, d_shared, inter, hidden),
+                           "shared_expert_ffn down launch");
+    if (st == LEV_OK) st = lev_hip_rmsnorm(ctx, d_shared, d_shared, hidden, 1, d_post_norm, eps);
+    return st;
+}

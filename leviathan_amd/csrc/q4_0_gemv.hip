@@ -343,10 +343,10 @@ uint32_t lev_q4_0_gemv_candidates(const lev_ctx *ctx, uint32_t in_dim, uint32_t 
             if (all[i].family == 0u && all[i].rows_in_flight == r && all[i].persistent == p) return;
         all[n++] = lev_schedule{LEV_OP_Q4_0_GEMV, 0u, r, p};
     };
-    // rows of whole 256-value tasks: the matrix-core kernel (family 1), the built-in choice, with
-    // one workgroup per round of row groups or a resident grid
-    if (in_dim % 256u == 0u && in_dim <= kLevQ4MfmaMaxInDim) {
-        const uint32_t ntask = in_dim >> 8, slots = ntask <= 16u ? 16u / ntask : 1u;
+    // where it serves, the matrix-core kernel (family 1) is the built-in choice, with one workgroup per
+    // round of row groups or a resident grid
+    if (lev_q4_0_mfma_in_dim(in_dim)) {
+        const uint32_t ntask = (in_dim + 255u) >> 8, slots = ntask <= 16u ? 16u / ntask : 1u;
         const uint32_t nrounds = ((rows + 15u) / 16u + slots - 1u) / slots;
         const uint32_t builtin = nrounds <= (uint32_t)ctx->num_cus ? 0u : 1u;
         all[n++] = lev_schedule{LEV_OP_Q4_0_GEMV, 1u, 0u, builtin};

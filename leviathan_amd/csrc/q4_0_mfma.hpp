@@ -32,6 +32,11 @@
 typedef int lev_i32x4 __attribute__((ext_vector_type(4)));
 
 constexpr uint32_t kLevQ4MfmaMaxInDim = 8192u;   // widest row the matrix-core GEMV takes
+// Rows it takes: whole 256-value tasks, and from five tasks on rows that end inside one (narrower ones of
+// those are the launch floor with either kernel, 3 us at 1088 x 5000, and stay with the vector-ALU kernels).
+__host__ inline bool lev_q4_0_mfma_in_dim(uint32_t in_dim) {
+    return in_dim != 0u && in_dim <= kLevQ4MfmaMaxInDim && (in_dim % 256u == 0u || (in_dim % 64u == 0u && in_dim > 1280u));
+}
 constexpr uint32_t kQ4mTaskArea = 1024u;   // LDS bytes of one staged task: [pair 4][plane 4][half 4][16 B]
 constexpr uint32_t kQ4mZeroBytes = 16u;    // what the lanes outside a row's own lane group read as their A operand
 

@@ -1,9 +1,10 @@
 // Q4_0 decode GEMV  y = W x  on the integer matrix cores (gfx950).
 //
 // Stands in for g4_q4_matvec and its tiled / generated variants
-// (Sources/LeviathanCore/Gemma4.swift:3931, 4031; Q4Lowering.swift:541-664) wherever a row is a
-// whole number of 256-value tasks; q4_0_gemv.hip keeps the vector-ALU kernels for every other
-// shape and as forge candidates.
+// (Sources/LeviathanCore/Gemma4.swift:3931, 4031; Q4Lowering.swift:541-664) for rows of whole block
+// pairs up to 8192 wide (lev_q4_0_mfma_in_dim); q4_0_gemv.hip keeps the vector-ALU kernels for every other shape and as forge
+// candidates.  The last 256-value task of a row may be a part of one: 2112 columns, 20000 rows 6.8 us a call
+// against 8.0 with the vector-ALU kernel, 8000 x 9000 9.9 against 12.9.
 //
 // Workgroup = 16 waves.  A row group is 16 rows; its in_dim / 256 column tasks are split over
 // WPR waves, TPW adjacent tasks each (WPR * TPW >= tasks).  Rows narrower than 16 tasks leave
@@ -38,15 +39,16 @@ q4_0_mfma_gemv(const uint8_t *__restrict__ w, const float *__restrict__ x, float
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
     const uint32_t slot = (uint32_t)(slot_of_wave >> (4u * wave)) & 15u;   // idle waves: slot >= slots
     const uint32_t tw = (uint32_t)(pos_of_wave >> (4u * wave)) & 15u;
-    const uint32_t ntask = in_dim >> 8;
+    const uint32_t npairs = in_dim >> 6, ntask = (npairs + 3u) >> 2;   // the last task may be a part of one
     const uint32_t t_first = tw * TPW;
 
     // the activations of the wave's tasks first (short, mostly L2 hits) ...
     lev_f32x4 v[TPW];
+    bool v_live[TPW];
 #pragma unroll
     for (int t = 0; t < TPW; ++t) {
         const uint32_t T = t_first + t < ntask ? t_first + t : ntask - 1u;
-        v[t] = reinterpret_cast<const lev_f32x4 *>(x)[64u * T + lane];
+        v[t] = q4m_load_activations(x, T, in_dim >> 2, v_live[t]);
     }
     // ... the first row group's weights right behind them
     const bool active = slot < slots;
@@ -62,7 +64,7 @@ q4_0_mfma_gemv(const uint8_t *__restrict__ w, const float *__restrict__ x, float
 #pragma unroll
         for (int t = 0; t < TPW; ++t) {
             const uint32_t T = t_first + t < ntask ? t_first + t : ntask - 1u;
-            q4m_load_task(rowp, 4u * T, D[t]);
+            q4m_load_task_part(rowp, 4u * T, npairs, D[t]);
         }
     };
     uint32_t Da[TPW][9];
@@ -100,7 +102,7 @@ q4_0_mfma_gemv(const uint8_t *__restrict__ w, const float *__restrict__ x, float
     q4m_operand op[TPW];
 #pragma unroll
     for (int t = 0; t < TPW; ++t)
-        q4m_stage_task(v[t], area + t * kQ4mTaskArea, zero, active && t_first + t < ntask, op[t]);
+        q4m_stage_task(q4m_mask_activations(v[t], v_live[t]), area + t * kQ4mTaskArea, zero, active && t_first + t < ntask, op[t]);
     // the operands are read back before the wait for the weights, not behind it
     __builtin_amdgcn_sched_barrier(0);
 
@@ -187,17 +189,16 @@ hipError_t launch(lev_ctx *ctx, const uint8_t *w, const float *x, float *y, uint
 
 }  // namespace
 
-// Shapes the matrix-core GEMV takes: rows of whole 256-value tasks, at most two tasks a wave
-// (the operands of more do not fit the 128 registers a wave of a 16-wave workgroup has).
+// At most two tasks a wave: the operands of more do not fit the 128 registers a wave of a 16-wave workgroup has.
 bool lev_q4_0_mfma_gemv_usable(const uint8_t *w, const float *x, uint32_t in_dim) {
-    return in_dim % 256u == 0u && in_dim != 0u && in_dim <= kLevQ4MfmaMaxInDim &&
-           (reinterpret_cast<uintptr_t>(w) & 3u) == 0u && (reinterpret_cast<uintptr_t>(x) & 15u) == 0u;
+    return lev_q4_0_mfma_in_dim(in_dim) && (reinterpret_cast<uintptr_t>(w) & 3u) == 0u &&
+           (reinterpret_cast<uintptr_t>(x) & 15u) == 0u;
 }
 
 // persistent: 0 = one workgroup per round of row groups, 1 = resident grid, < 0 = built-in choice.
 hipError_t lev_q4_0_mfma_gemv_launch(lev_ctx *ctx, const uint8_t *w, const float *x, float *y, uint32_t in_dim,
                                      uint32_t rows, int persistent) {
-    const uint32_t ntask = in_dim >> 8;
+    const uint32_t ntask = (in_dim + 255u) >> 8;
     if (ntask <= (uint32_t)kQ4mWaves) {
         // one task per wave; 16 / ntask row groups share a round
         const uint32_t slots = (uint32_t)kQ4mWaves / ntask;

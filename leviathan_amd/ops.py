@@ -288,12 +288,17 @@ class Context:
                     torch.empty(inter, dtype=torch.float32, device=dev),
                     torch.empty(hidden, dtype=torch.float32, device=dev))
         h, gu, act, shared = bufs
-        self.rmsnorm(x, hidden, 1, weight=ffn_norm, eps=eps, y=h)
-        self.q4_0_gemv(gate_w, h, hidden, inter, y=gu)
-        self.q4_0_gemv(up_w, h, hidden, inter, y=gu[inter:])
-        self.gelu_up(gu, inter, y=act)
-        self.q4_0_gemv(down_w, act, inter, hidden, y=shared)
-        self.rmsnorm(shared, hidden, 1, weight=post_norm, eps=eps, y=shared)
+        for t, what in ((x, "x"), (h, "h"), (gu, "gu"), (act, "act"), (shared, "shared")):
+            _dev(t, torch.float32, what)
+        for t, what in ((gate_w, "gate_w"), (up_w, "up_w"), (down_w, "down_w")):
+            _dev(t, torch.uint8, what)
+        if h.numel() != hidden or act.numel() != inter:
+            raise LevError(capi.WRONG_INPUT_COUNT, f"shared expert: h {h.numel()}, act {act.numel()} values")
+        if gu.numel() < 2 * inter or shared.numel() < hidden:
+            raise LevError(capi.BAD_DIMENSIONS, f"shared expert: gu {gu.numel()}, shared {shared.numel()} values")
+        self._check(self.lib.lev_hip_shared_expert_ffn_q4_0(
+            self.ctx, _ptr(x), _ptr(ffn_norm), _ptr(gate_w), gate_w.numel(), _ptr(up_w), up_w.numel(), _ptr(down_w),
+            down_w.numel(), _ptr(post_norm), eps, _ptr(h), _ptr(gu), _ptr(act), _ptr(shared), hidden, inter))
         return h, shared
 
     def argmax(self, logits, vocab: int, ncol: int = 1):
