@@ -1,4 +1,5 @@
-"""Builds ``libleviathan_hip.so`` (gfx950 only) from ``csrc/*.hip`` with hipcc.
+"""Builds ``libleviathan_hip.so`` (gfx950 only) from ``csrc/*.hip`` with hipcc, and with the host compiler
+``_lev_ops.so``, the argument handling of ``ops.py``, from ``csrc/py_ops.cpp``.
 
 Run ``python -m leviathan_amd.build``.  hipcc cross-compiles without a GPU.
 Objects are compiled in parallel and linked into ``leviathan_amd/lib``.
@@ -16,6 +17,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIB_DIR = os.path.join(HERE, "lib")
 OBJ_DIR = os.path.join(HERE, "build")
 LIB_PATH = os.path.join(LIB_DIR, "libleviathan_hip.so")
+OPS_PATH = os.path.join(LIB_DIR, "_lev_ops.so")
 
 ARCH = "gfx950"
 HIPCC_FLAGS = [
@@ -59,6 +61,26 @@ def _compile(src: str, force: bool, extra: list[str]) -> str:
     return obj
 
 
+def _build_ops(force: bool) -> None:
+    """The CPython extension. It names torch's libraries without a path: they are loaded when it is."""
+    import sysconfig
+    from torch.utils import cpp_extension
+    src = os.path.join(CSRC, "py_ops.cpp")
+    if (not force and os.path.exists(OPS_PATH)
+            and os.path.getmtime(OPS_PATH) >= max(os.path.getmtime(src), _headers_mtime())):
+        return
+    cxx = os.environ.get("CXX") or shutil.which("g++") or "g++"
+    tmp = OPS_PATH + ".tmp"
+    cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-fvisibility=hidden",
+           *(a for p in (*cpp_extension.include_paths(), sysconfig.get_paths()["include"]) for a in ("-isystem", p)),
+           src, "-o", tmp, f"-L{LIB_DIR}", *(f"-L{p}" for p in cpp_extension.library_paths()),
+           "-lleviathan_hip", "-ltorch_python", "-ltorch_cpu", "-lc10", "-Wl,-rpath,$ORIGIN"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed for {src}:\n{res.stderr}")
+    os.replace(tmp, OPS_PATH)
+
+
 def build(force: bool = True, jobs: int = 8, extra_flags: list[str] | None = None) -> str:
     os.makedirs(LIB_DIR, exist_ok=True)
     os.makedirs(OBJ_DIR, exist_ok=True)
@@ -71,6 +93,7 @@ def build(force: bool = True, jobs: int = 8, extra_flags: list[str] | None = Non
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stderr}")
     os.replace(tmp, LIB_PATH)
+    _build_ops(force)
     return LIB_PATH
 
 

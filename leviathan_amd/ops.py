@@ -1,7 +1,9 @@
 """Thin Python view of the C ABI for callers that hold torch tensors.
 
 torch is used here only as a device-memory and stream provider: every method
-passes ``tensor.data_ptr()`` and sizes straight to ``libleviathan_hip.so``.
+passes pointers and sizes straight to ``libleviathan_hip.so``, the operators of
+a decode step through ``_lev_ops`` (``csrc/py_ops.cpp``: argument checks and
+outputs in native code), the rest through ctypes.
 Method names follow the reference's operator vocabulary
 (``Gemma4Runner.matvec`` / ``rmsnorm`` / ``geluUp`` / ``axpy`` /
 ``runMoeBatchedRouted``; ``Builder::matvec`` / ``norm_quant`` / argmax step).
@@ -25,6 +27,25 @@ class LevError(RuntimeError):
         self.status = status
         self.name = name
         self.message = message
+
+
+def _load_native():
+    """The extension beside the library; the library first, which says what to do where nothing is built."""
+    import importlib.machinery
+    import importlib.util
+    import os
+    capi.load()
+    path = os.path.join(os.path.dirname(capi.LIB_PATH), "_lev_ops.so")
+    if not os.path.exists(path):
+        raise capi.LibraryMissing(f"{path} not found: build it with `python -m leviathan_amd.build`")
+    loader = importlib.machinery.ExtensionFileLoader("_lev_ops", path)
+    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_lev_ops", loader))
+    loader.exec_module(module)
+    module.set_error(LevError)
+    return module
+
+
+_native = None
 
 
 def _ptr(t):
@@ -54,13 +75,17 @@ class Context:
         st = self.lib.lev_hip_ctx_create(device, handle, C.byref(ctx))
         if st != capi.OK:
             raise LevError(st, "ctx_create")
+        global _native
+        if _native is None:
+            _native = _load_native()
         self.ctx = ctx
+        self._h = ctx.value
         self.device = device
 
     def close(self):
         if getattr(self, "ctx", None):
             self.lib.lev_hip_ctx_destroy(self.ctx)
-            self.ctx = None
+            self.ctx = self._h = None
 
     def __del__(self):
         try:
@@ -101,104 +126,34 @@ class Context:
 
     # -- GEMV -------------------------------------------------------------
     def q4_0_gemv(self, w, x, in_dim: int, out_rows: int, y=None, w_off: int = 0, x_count=None):
-        _dev(w, torch.uint8, "w")
-        _dev(x, torch.float32, "x")
-        if y is None:
-            y = torch.empty(max(out_rows, 1), dtype=torch.float32, device=w.device)
-        xc = x.numel() if x_count is None else x_count
-        self._check(self.lib.lev_hip_q4_0_gemv(self.ctx, _ptr(w), w.numel(), w_off, _ptr(x), xc,
-                                               _ptr(y), y.numel(), in_dim, out_rows))
-        return y
+        return _native.q4_0_gemv(self._h, w, x, in_dim, out_rows, y, w_off, x_count)
 
     def q6_k_gemv(self, w, x, in_dim: int, out_rows: int, y=None, w_off: int = 0, argmax=False):
-        _dev(w, torch.uint8, "w")
-        _dev(x, torch.float32, "x")
-        if y is None:
-            y = torch.empty(max(out_rows, 1), dtype=torch.float32, device=w.device)
-        idx = mg = None
-        if argmax:
-            idx = torch.empty(1, dtype=torch.int32, device=w.device)
-            mg = torch.empty(1, dtype=torch.float32, device=w.device)
-        self._check(self.lib.lev_hip_q6_k_gemv(self.ctx, _ptr(w), w.numel(), w_off, _ptr(x),
-                                               x.numel(), _ptr(y), y.numel(), in_dim, out_rows,
-                                               _ptr(idx), _ptr(mg)))
-        return (y, idx, mg) if argmax else y
+        return _native.q6_k_gemv(self._h, w, x, in_dim, out_rows, y, w_off, argmax)
 
     def q4_k_gemv_ncol(self, w, x, in_dim: int, rows: int, ncol: int, gain=None, eps: float = 1e-6,
                        y=None, w_off: int = 0):
-        _dev(w, torch.uint8, "w")
-        _dev(x, torch.float32, "x")
-        if gain is not None:
-            _dev(gain, torch.float32, "gain")
-        if y is None:
-            y = torch.empty((max(ncol, 1), max(rows, 1)), dtype=torch.float32, device=w.device)
-        self._check(self.lib.lev_hip_q4_k_gemv_ncol(self.ctx, _ptr(w), w.numel(), w_off, _ptr(x),
-                                                    x.numel(), _ptr(gain), eps, _ptr(y), y.numel(),
-                                                    in_dim, rows, ncol))
-        return y
+        return _native.q4_k_gemv_ncol(self._h, w, x, in_dim, rows, ncol, gain, eps, y, w_off)
 
     def q6_k_gemv_ncol(self, w, x, in_dim: int, rows: int, ncol: int, gain=None, eps: float = 1e-6,
                        y=None, w_off: int = 0):
         """Q6_K GEMV of ``ncol`` f32 columns per weight read (optional RMSNorm in front)."""
-        _dev(w, torch.uint8, "w")
-        _dev(x, torch.float32, "x")
-        if gain is not None:
-            _dev(gain, torch.float32, "gain")
-        if y is None:
-            y = torch.empty((max(ncol, 1), max(rows, 1)), dtype=torch.float32, device=w.device)
-        self._check(self.lib.lev_hip_q6_k_gemv_ncol(self.ctx, _ptr(w), w.numel(), w_off, _ptr(x),
-                                                    x.numel(), _ptr(gain), eps, _ptr(y), y.numel(),
-                                                    in_dim, rows, ncol))
-        return y
+        return _native.q6_k_gemv_ncol(self._h, w, x, in_dim, rows, ncol, gain, eps, y, w_off)
 
     def norm_quant_q8(self, x, n: int, ncol: int, gain=None, eps: float = 1e-6, add=None,
                       want_y: bool = False):
         """Int8 activations of ``x`` [ncol][n]: returns (xq int8, xs (d, s) pairs[, y f32])."""
-        _dev(x, torch.float32, "x")
-        if gain is not None:
-            _dev(gain, torch.float32, "gain")
-        if add is not None:
-            _dev(add, torch.float32, "add")
-        xq = torch.empty((max(ncol, 1), max(n, 1)), dtype=torch.int8, device=x.device)
-        xs = torch.empty((max(ncol, 1), max(n // 32, 1), 2), dtype=torch.float32, device=x.device)
-        y = torch.empty_like(x) if want_y else None
-        self._check(self.lib.lev_hip_norm_quant_q8(self.ctx, _ptr(x), x.numel(), _ptr(add), _ptr(gain),
-                                                   eps, _ptr(xq), _ptr(xs), _ptr(y), n, ncol))
-        return (xq, xs, y) if want_y else (xq, xs)
+        return _native.norm_quant_q8(self._h, x, n, ncol, gain, eps, add, want_y)
 
     def q4_k_gemv_q8(self, w, xq, xs, in_dim: int, rows: int, ncol: int, y=None, w_off: int = 0):
-        _dev(w, torch.uint8, "w")
-        _dev(xq, torch.int8, "xq")
-        _dev(xs, torch.float32, "xs")
-        if y is None:
-            y = torch.empty((max(ncol, 1), max(rows, 1)), dtype=torch.float32, device=w.device)
-        self._check(self.lib.lev_hip_q4_k_gemv_q8(self.ctx, _ptr(w), w.numel(), w_off, _ptr(xq),
-                                                  _ptr(xs), xq.numel(), _ptr(y), y.numel(), in_dim,
-                                                  rows, ncol))
-        return y
+        return _native.q4_k_gemv_q8(self._h, w, xq, xs, in_dim, rows, ncol, y, w_off)
 
     def q6_k_gemv_q8(self, w, xq, xs, in_dim: int, rows: int, ncol: int, y=None, w_off: int = 0):
-        _dev(w, torch.uint8, "w")
-        _dev(xq, torch.int8, "xq")
-        _dev(xs, torch.float32, "xs")
-        if y is None:
-            y = torch.empty((max(ncol, 1), max(rows, 1)), dtype=torch.float32, device=w.device)
-        self._check(self.lib.lev_hip_q6_k_gemv_q8(self.ctx, _ptr(w), w.numel(), w_off, _ptr(xq),
-                                                  _ptr(xs), xq.numel(), _ptr(y), y.numel(), in_dim,
-                                                  rows, ncol))
-        return y
+        return _native.q6_k_gemv_q8(self._h, w, xq, xs, in_dim, rows, ncol, y, w_off)
 
     def swiglu_quant_q8(self, gate, up, want_act: bool = False):
         """Int8 activations of silu(gate) * up: returns (xq, xs (d, s) pairs[, act f32])."""
-        _dev(gate, torch.float32, "gate")
-        _dev(up, torch.float32, "up")
-        n = gate.numel()
-        xq = torch.empty(max(n, 1), dtype=torch.int8, device=gate.device)
-        xs = torch.empty((max(n // 32, 1), 2), dtype=torch.float32, device=gate.device)
-        act = torch.empty_like(gate) if want_act else None
-        self._check(self.lib.lev_hip_swiglu_quant_q8(self.ctx, _ptr(gate), _ptr(up), n, _ptr(xq),
-                                                     _ptr(xs), _ptr(act)))
-        return (xq, xs, act) if want_act else (xq, xs)
+        return _native.swiglu_quant_q8(self._h, gate, up, want_act)
 
     def embed_q4_k(self, w, tokens, dim: int, vocab: int, out=None, w_off: int = 0):
         _dev(w, torch.uint8, "w")
@@ -224,24 +179,10 @@ class Context:
         self._check(self.lib.lev_hip_forge_clear(self.ctx, op, in_dim, rows, ncol))
 
     def q4_k_gemm_prefill(self, w, x_f16, in_dim: int, rows: int, tokens: int, y=None, w_off: int = 0):
-        _dev(w, torch.uint8, "w")
-        _dev(x_f16, torch.float16, "x")
-        if y is None:
-            y = torch.empty((max(tokens, 1), max(rows, 1)), dtype=torch.float32, device=w.device)
-        self._check(self.lib.lev_hip_q4_k_gemm_prefill(self.ctx, _ptr(w), w.numel(), w_off,
-                                                       _ptr(x_f16), x_f16.numel(), _ptr(y),
-                                                       y.numel(), in_dim, rows, tokens))
-        return y
+        return _native.q4_k_gemm_prefill(self._h, w, x_f16, in_dim, rows, tokens, y, w_off)
 
     def q6_k_gemm_prefill(self, w, x_f16, in_dim: int, rows: int, tokens: int, y=None, w_off: int = 0):
-        _dev(w, torch.uint8, "w")
-        _dev(x_f16, torch.float16, "x")
-        if y is None:
-            y = torch.empty((max(tokens, 1), max(rows, 1)), dtype=torch.float32, device=w.device)
-        self._check(self.lib.lev_hip_q6_k_gemm_prefill(self.ctx, _ptr(w), w.numel(), w_off,
-                                                       _ptr(x_f16), x_f16.numel(), _ptr(y),
-                                                       y.numel(), in_dim, rows, tokens))
-        return y
+        return _native.q6_k_gemm_prefill(self._h, w, x_f16, in_dim, rows, tokens, y, w_off)
 
     def f32_to_f16(self, x):
         _dev(x, torch.float32, "x")
@@ -251,25 +192,13 @@ class Context:
 
     # -- elementwise operators -------------------------------------------
     def rmsnorm(self, x, n: int, vectors: int, weight=None, eps: float = 1e-6, y=None):
-        _dev(x, torch.float32, "x")
-        if y is None:
-            y = torch.empty_like(x)
-        self._check(self.lib.lev_hip_rmsnorm(self.ctx, _ptr(x), _ptr(y), n, vectors, _ptr(weight),
-                                             eps))
-        return y
+        return _native.rmsnorm(self._h, x, n, vectors, weight, eps, y)
 
     def gelu_up(self, gu, n: int, y=None):
-        _dev(gu, torch.float32, "gu")
-        if y is None:
-            y = torch.empty(max(n, 1), dtype=torch.float32, device=gu.device)
-        self._check(self.lib.lev_hip_gelu_up(self.ctx, _ptr(gu), _ptr(y), n))
-        return y
+        return _native.gelu_up(self._h, gu, n, y)
 
     def axpy(self, x, y, c: float, n: int):
-        _dev(x, torch.float32, "x")
-        _dev(y, torch.float32, "y")
-        self._check(self.lib.lev_hip_axpy(self.ctx, _ptr(x), _ptr(y), c, n))
-        return y
+        return _native.axpy(self._h, x, y, c, n)
 
     def shared_expert_ffn(self, x, ffn_norm, gate_w, up_w, down_w, post_norm, hidden: int, inter: int,
                           eps: float = 1e-6, bufs=None):
@@ -288,25 +217,12 @@ class Context:
                     torch.empty(inter, dtype=torch.float32, device=dev),
                     torch.empty(hidden, dtype=torch.float32, device=dev))
         h, gu, act, shared = bufs
-        for t, what in ((x, "x"), (h, "h"), (gu, "gu"), (act, "act"), (shared, "shared")):
-            _dev(t, torch.float32, what)
-        for t, what in ((gate_w, "gate_w"), (up_w, "up_w"), (down_w, "down_w")):
-            _dev(t, torch.uint8, what)
-        if h.numel() != hidden or act.numel() != inter:
-            raise LevError(capi.WRONG_INPUT_COUNT, f"shared expert: h {h.numel()}, act {act.numel()} values")
-        if gu.numel() < 2 * inter or shared.numel() < hidden:
-            raise LevError(capi.BAD_DIMENSIONS, f"shared expert: gu {gu.numel()}, shared {shared.numel()} values")
-        self._check(self.lib.lev_hip_shared_expert_ffn_q4_0(
-            self.ctx, _ptr(x), _ptr(ffn_norm), _ptr(gate_w), gate_w.numel(), _ptr(up_w), up_w.numel(), _ptr(down_w),
-            down_w.numel(), _ptr(post_norm), eps, _ptr(h), _ptr(gu), _ptr(act), _ptr(shared), hidden, inter))
+        _native.shared_expert_ffn(self._h, x, ffn_norm, gate_w, up_w, down_w, post_norm, eps, h, gu, act, shared,
+                                  hidden, inter)
         return h, shared
 
     def argmax(self, logits, vocab: int, ncol: int = 1):
-        _dev(logits, torch.float32, "logits")
-        idx = torch.empty(max(ncol, 1), dtype=torch.int32, device=logits.device)
-        mg = torch.empty(max(ncol, 1), dtype=torch.float32, device=logits.device)
-        self._check(self.lib.lev_hip_argmax(self.ctx, _ptr(logits), vocab, ncol, _ptr(idx), _ptr(mg)))
-        return idx, mg
+        return _native.argmax(self._h, logits, vocab, ncol)
 
     # -- MoE ---------------------------------------------------------------
     @staticmethod
@@ -350,18 +266,7 @@ class Context:
         """``noalloc``: the entry point that allocates nothing inside the call (static
         device scratch; pass ``y``, ``ids`` and ``weights`` so that this wrapper
         allocates nothing either)."""
-        _dev(x, torch.float32, "x")
-        if y is None:
-            y = torch.empty((max(tokens, 1), pools.hidden), dtype=torch.float32, device=x.device)
-        if ids is None:
-            ids = torch.empty((max(tokens, 1), max(top_k, 1)), dtype=torch.int32, device=x.device)
-        if weights is None:
-            weights = torch.empty((max(tokens, 1), max(top_k, 1)), dtype=torch.float32,
-                                  device=x.device)
-        fn = self.lib.lev_hip_moe_layer_q4_0_noalloc if noalloc else self.lib.lev_hip_moe_layer_q4_0
-        self._check(fn(self.ctx, C.byref(pools), _ptr(router_w), _ptr(expert_scale), _ptr(x), _ptr(y),
-                       _ptr(ids), _ptr(weights), top_k, tokens))
-        return y, ids, weights
+        return _native.moe_layer_q4_0(self._h, pools, router_w, x, top_k, tokens, expert_scale, y, ids, weights, noalloc)
 
 
 class Program:
@@ -371,7 +276,7 @@ class Program:
         self.ctx, self.handle = ctx, handle
 
     def run(self):
-        self.ctx._check(self.ctx.lib.lev_hip_program_run(self.ctx.ctx, self.handle))
+        _native.program_run(self.ctx._h, self.handle.value if self.handle else None)
 
     def node_count(self) -> int:
         n = C.c_size_t()
