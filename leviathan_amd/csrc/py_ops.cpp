@@ -11,7 +11,6 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <ATen/ops/empty.h>
-#include <ATen/ops/empty_like.h>
 
 #include <algorithm>
 

@@ -80,19 +80,28 @@ struct q6m_regs {
 // are [16p, +16) for p < 13.  Piece 13 is bytes [194, 210) for both, so that d is its last
 // two bytes and nothing behind the block is read (for an even superblock that one piece is
 // off the dword boundary).  Lanes 14 and 15 of a row repeat piece 1: never used.
+// Even and odd count from the matrix's start, row * SB + sb: where SB is odd every other row
+// is an odd one (q6m_odd).  Measured with rows of 11 superblocks, 262144 of them: 154 us with
+// the parity of sb alone, 127 with this.
 __device__ __forceinline__ int32_t q6m_piece_offset(uint32_t lane, uint32_t odd) {
     const uint32_t p = ((lane & 15u) - 4u * (lane >> 4)) & 15u;
     if (p == 13u) return 194;
     return (int32_t)(16u * (p < 13u ? p : 1u)) - (odd ? 14 : 0);
 }
 
+// `alt`: 1 where the parity alternates from row to row (a one-row matrix keeps to its row).  row: its
+// index modulo two is enough; tasks start at multiples of 16.
+__device__ __forceinline__ uint32_t q6m_alt(uint32_t SB, uint32_t rows) { return rows > 1u ? SB & 1u : 0u; }
+__device__ __forceinline__ uint32_t q6m_odd(uint32_t sb, uint32_t row, uint32_t alt) { return (sb + row * alt) & 1u; }
+
+// (A row past the end reads row 0 or, where its parity matters, the row of its parity.)
 __device__ __forceinline__ void q6m_issue(const uint8_t *__restrict__ w, uint64_t row_bytes, uint32_t row0,
-                                          uint32_t rows, uint32_t sb, uint32_t lane, int32_t poff,
+                                          uint32_t rows, uint32_t alt, uint32_t sb, uint32_t lane, int32_t poff,
                                           q6m_regs &R) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         uint32_t row = row0 + 4u * (uint32_t)i + (lane >> 4);
-        row = row < rows ? row : rows - 1u;
+        row = row < rows ? row : row & alt;
         const q6m_u4 v = *reinterpret_cast<const q6m_u4 *>(
             w + (uint64_t)row * row_bytes + (uint64_t)(int64_t)((int32_t)(sb * 210u) + poff));
         R.p[i] = q6m_i4{(int)v.v[0], (int)v.v[1], (int)v.v[2], (int)v.v[3]};
@@ -101,7 +110,7 @@ __device__ __forceinline__ void q6m_issue(const uint8_t *__restrict__ w, uint64_
 
 // What a lane needs to turn a task's pieces into its matrix-core operands.
 // lane (r, g): weight row r of the task's 16, chunk g of the superblock (half hf = g/2,
-// j in {jb, jb + 2} with jb = g%2).  `odd`: the wave's superblocks are the odd ones.
+// j in {jb, jb + 2} with jb = g%2).  `odd`: the lane's row r has its superblock at an odd place.
 struct q6m_lane {
     uint8_t *area;                // the wave's turn-round area
     uint32_t lane, sel, maskq;
@@ -342,15 +351,16 @@ q6_k_mfma_gemv(const uint8_t *__restrict__ w, const float *__restrict__ x, const
             ++c.rd;
         }
     };
-    const uint32_t odd = kpart & 1u;
-    const int32_t poff = q6m_piece_offset(lane, odd), poff_even = q6m_piece_offset(lane, 0u);
+    const uint32_t alt = q6m_alt(SB, rows);
+    const int32_t poff = q6m_piece_offset(lane, q6m_odd(kpart, g, alt));
+    const int32_t poff_first = q6m_piece_offset(lane, q6m_odd(0u, g, alt));
     auto group_of = [&](uint32_t rd, uint32_t sl) { return (rd * gridDim.x + blockIdx.x) * slots + sl; };
     auto issue = [&](cursor &c, q6m_regs &W) {
         const uint32_t sbw = kpart + S * c.t;
         const bool real = c.k < ntasks && sbw < SB;
-        // (past the end: the first superblock of the matrix, pieces as for an even one)
-        q6m_issue(w, row_bytes, real ? group_of(c.rd, slot) * 16u : 0u, rows, real ? sbw : 0u, lane,
-                  real ? poff : poff_even, W);
+        // (past the end: the first superblocks of the matrix's first rows)
+        q6m_issue(w, row_bytes, real ? group_of(c.rd, slot) * 16u : 0u, rows, alt, real ? sbw : 0u, lane,
+                  real ? poff : poff_first, W);
         advance(c);
     };
     cursor ci{0u, 0u, 0u}, cc{0u, 0u, 0u};
@@ -476,7 +486,7 @@ q6_k_mfma_gemv(const uint8_t *__restrict__ w, const float *__restrict__ x, const
     // ---- stream the weights ----
     const uint32_t hf = g >> 1, jb = g & 1u;
     const bool feeds = (r >> 2) == g;                      // this lane's A row belongs to its own lane group
-    const q6m_lane L6(area_all, wave, lane, odd);
+    const q6m_lane L6(area_all, wave, lane, q6m_odd(kpart, r, alt));
     double yacc[NC];
 #pragma unroll
     for (int q = 0; q < NC; ++q) yacc[q] = 0.0;
@@ -599,6 +609,7 @@ q6_k_mfma_gemv(const uint8_t *__restrict__ w, const float *__restrict__ x, const
 // LDS: part [2][16 waves][16 rows][NC] f64 | sums of squares [NC][16] f64 | per wave: turn-round
 // area, digit planes [NC][16 groups][4 planes][16 B], a zero strip.
 // ---------------------------------------------------------------------------
+constexpr int kQ1FewWaves = 12;
 constexpr uint32_t kQ1DigBytes = 1024u, kQ1ZeroBytes = 16u;
 __host__ __device__ constexpr uint32_t q6m_one_part_bytes(uint32_t nc) { return 2u * kQWaves * 16u * 8u * nc; }
 __host__ __device__ constexpr uint32_t q6m_one_norm_bytes(uint32_t nc) { return kQWaves * 8u * nc; }
@@ -611,8 +622,8 @@ __host__ __device__ constexpr size_t q6m_one_lds(uint32_t nc) {
 // front of the first load).  NC: columns staged (1 or 2; >= ncol); one column keeps its A
 // operands in registers, several read them from the wave's planes at every product.
 // NORM: RMSNorm (gain != nullptr) in front.  partials (optional, ncol == 1): the greedy token.
-template <int NC, bool NORM>
-__global__ void __launch_bounds__(kQThreads)
+template <int NC, bool NORM, int MAXW>
+__global__ void __launch_bounds__(MAXW * LEV_WAVE)
 q6_k_mfma_gemv_one(const uint8_t *__restrict__ w, const float *__restrict__ x, const float *__restrict__ gain,
                    float eps, float *__restrict__ y, uint32_t cols, uint32_t rows, uint32_t ncol, uint32_t wpr,
                    uint32_t slots, uint64_t slot_of_wave, uint64_t pos_of_wave, double rcols,
@@ -639,14 +650,15 @@ q6_k_mfma_gemv_one(const uint8_t *__restrict__ w, const float *__restrict__ x, c
     const uint64_t row_bytes = (uint64_t)SB * 210u;
     const uint32_t ngroups = (rows + 15u) >> 4;
     const uint32_t nrounds = (ngroups + slots - 1u) / slots;     // rounds of `slots` row groups
-    const uint32_t odd = sb & 1u;
-    const int32_t poff = q6m_piece_offset(lane, odd);
+    const uint32_t alt = q6m_alt(SB, rows);
+    const int32_t poff = q6m_piece_offset(lane, q6m_odd(sb, lane >> 4, alt));
     auto issue = [&](uint32_t round_block, q6m_regs &W) {
         uint32_t rg = round_block * slots + (active ? slot : 0u);
         rg = rg < ngroups ? rg : ngroups - 1u;
-        q6m_issue(w, row_bytes, rg * 16u, rows, sb, lane, poff, W);
+        q6m_issue(w, row_bytes, rg * 16u, rows, alt, sb, lane, poff, W);
     };
-    q6m_regs Wa, Wb;
+    constexpr uint32_t DEPTH = MAXW <= kQ1FewWaves ? 3u : 2u;    // row groups a wave has in flight
+    q6m_regs Wa, Wb, Wc;
     uint32_t rb = blockIdx.x;
     // ... and the first row group's weights; with RMSNorm in front only once every wave's request
     // for its activations is in the CU's memory queue (a short load queued behind other waves'
@@ -759,7 +771,7 @@ q6_k_mfma_gemv_one(const uint8_t *__restrict__ w, const float *__restrict__ x, c
 #pragma unroll
             for (int lh = 0; lh < 2; ++lh) A1[nb][lh] = *reinterpret_cast<const q6m_i4 *>(ab + (4 * nb + lh) * hs);
     }
-    const q6m_lane L6(smem + kPart + kNorm, wave, lane, odd, kWave);
+    const q6m_lane L6(smem + kPart + kNorm, wave, lane, q6m_odd(sb, r, alt), kWave);
     // the operands are read back before the wait for the weights, not behind it
     __builtin_amdgcn_sched_barrier(0);
 
@@ -829,25 +841,26 @@ q6_k_mfma_gemv_one(const uint8_t *__restrict__ w, const float *__restrict__ x, c
         yp += (uint64_t)orow_step * 4u;
         stores = writer && orow < rows ? 1u : 0u;
     };
-    // Unconditional (clamped) prefetch, one round ahead (a branch around the loads would make the
-    // compiler wait for them before the current group is multiplied).
+    // Unconditional (clamped) prefetch, DEPTH - 1 rounds ahead (a branch around the loads would make
+    // the compiler wait for them before the current group is multiplied).
     // (The scheduling barriers keep the requests where they are written: sunk below the products
     // of the round in hand they would no longer run ahead of anything.)
-    while (true) {
-        uint32_t next = rb + gridDim.x;
+    auto step = [&](const q6m_regs &current, q6m_regs &ahead) {
+        const uint32_t next = rb + (DEPTH - 1u) * gridDim.x;
         __builtin_amdgcn_sched_barrier(0);
-        issue(next < nrounds ? next : rb, Wb);
+        issue(next < nrounds ? next : rb, ahead);
         __builtin_amdgcn_sched_barrier(0);
-        finish(Wa);
-        if (next >= nrounds) break;
-        rb = next;
-        next = rb + gridDim.x;
-        __builtin_amdgcn_sched_barrier(0);
-        issue(next < nrounds ? next : rb, Wa);
-        __builtin_amdgcn_sched_barrier(0);
-        finish(Wb);
-        if (next >= nrounds) break;
-        rb = next;
+        finish(current);
+        rb += gridDim.x;
+        return rb < nrounds;
+    };
+    if constexpr (DEPTH == 3u) {
+        issue(rb + gridDim.x < nrounds ? rb + gridDim.x : rb, Wb);
+        while (step(Wa, Wc) && step(Wb, Wa) && step(Wc, Wb)) {
+        }
+    } else {
+        while (step(Wa, Wb) && step(Wb, Wa)) {
+        }
     }
     if (NC == 1 && partials) q6m_greedy_token(best, slots, partials, tickets, out_idx, out_margin);
 }
@@ -910,14 +923,15 @@ q6_k_mfma_gemv_q8(const uint8_t *__restrict__ w, const uint32_t *__restrict__ xq
             ++c.rd;
         }
     };
-    const uint32_t odd = kpart & 1u;
-    const int32_t poff = q6m_piece_offset(lane, odd), poff_even = q6m_piece_offset(lane, 0u);
+    const uint32_t alt = q6m_alt(SB, rows);
+    const int32_t poff = q6m_piece_offset(lane, q6m_odd(kpart, g, alt));
+    const int32_t poff_first = q6m_piece_offset(lane, q6m_odd(0u, g, alt));
     auto group_of = [&](uint32_t rd, uint32_t sl) { return (rd * gridDim.x + blockIdx.x) * slots + sl; };
     auto issue = [&](cursor &c, q6m_regs &W) {
         const uint32_t sbw = kpart + S * c.t;
         const bool real = c.k < ntasks && sbw < SB;
-        q6m_issue(w, row_bytes, real ? group_of(c.rd, slot) * 16u : 0u, rows, real ? sbw : 0u, lane,
-                  real ? poff : poff_even, W);
+        q6m_issue(w, row_bytes, real ? group_of(c.rd, slot) * 16u : 0u, rows, alt, real ? sbw : 0u, lane,
+                  real ? poff : poff_first, W);
         advance(c);
     };
     cursor ci{0u, 0u, 0u}, cc{0u, 0u, 0u};
@@ -944,7 +958,7 @@ q6_k_mfma_gemv_q8(const uint8_t *__restrict__ w, const uint32_t *__restrict__ xq
     // ---- stream the weights ----
     const uint32_t hf = g >> 1, jb = g & 1u;
     const bool feeds = (r >> 2) == g;
-    const q6m_lane L6(area_all, wave, lane, odd);
+    const q6m_lane L6(area_all, wave, lane, q6m_odd(kpart, r, alt));
     float yacc[NCH][4];
 #pragma unroll
     for (int ch = 0; ch < NCH; ++ch)
@@ -1100,12 +1114,12 @@ q6_k_mfma_gemv_q8_one(const uint8_t *__restrict__ w, const uint32_t *__restrict_
     const uint64_t row_bytes = (uint64_t)SB * 210u;
     const uint32_t ngroups = (rows + 15u) >> 4;
     const uint32_t nrounds = (ngroups + slots - 1u) / slots;     // rounds of `slots` row groups
-    const uint32_t odd = sb & 1u;
-    const int32_t poff = q6m_piece_offset(lane, odd);
+    const uint32_t alt = q6m_alt(SB, rows);
+    const int32_t poff = q6m_piece_offset(lane, q6m_odd(sb, lane >> 4, alt));
     auto issue = [&](uint32_t round_block, q6m_regs &W) {
         uint32_t rg = round_block * slots + (active ? slot : 0u);
         rg = rg < ngroups ? rg : ngroups - 1u;
-        q6m_issue(w, row_bytes, rg * 16u, rows, sb, lane, poff, W);
+        q6m_issue(w, row_bytes, rg * 16u, rows, alt, sb, lane, poff, W);
     };
     q6m_regs Wa, Wb;
     uint32_t rb = blockIdx.x;
@@ -1133,7 +1147,7 @@ q6_k_mfma_gemv_q8_one(const uint8_t *__restrict__ w, const uint32_t *__restrict_
 #pragma unroll
             for (int i = 0; i < 4; ++i) dx[ch][nb][i] *= active ? 0.25f : 0.f;
         }
-    const q6m_lane L6(smem + kPart, wave, lane, odd);
+    const q6m_lane L6(smem + kPart, wave, lane, q6m_odd(sb, r, alt));
     __builtin_amdgcn_sched_barrier(0);
 
     auto finish = [&](const q6m_regs &W) {
@@ -1261,8 +1275,8 @@ hipError_t q6m_launch(lev_ctx *ctx, const uint8_t *w, const float *x, const floa
     return hipGetLastError();
 }
 
-template <int NC, bool NORM>
-hipError_t q6m_one_launch(lev_ctx *ctx, const uint8_t *w, const float *x, const float *gain, float eps, float *y,
+template <int NC, bool NORM, int MAXW>
+hipError_t q6m_one_launch_waves(lev_ctx *ctx, const uint8_t *w, const float *x, const float *gain, float eps, float *y,
                           uint32_t cols, uint32_t rows, uint32_t ncol, lev_f32x4 *partials, uint32_t *d_argmax,
                           float *d_margin) {
     const uint32_t wpr = cols >> 8, slots = (uint32_t)kQWaves / wpr;
@@ -1273,7 +1287,7 @@ hipError_t q6m_one_launch(lev_ctx *ctx, const uint8_t *w, const float *x, const 
     constexpr size_t lds = q6m_one_lds(NC);
     static bool configured = false;   // per instantiation: raise the dynamic LDS limit once
     if (!configured) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&q6_k_mfma_gemv_one<NC, NORM>),
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&q6_k_mfma_gemv_one<NC, NORM, MAXW>),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
         configured = true;
@@ -1282,10 +1296,23 @@ hipError_t q6m_one_launch(lev_ctx *ctx, const uint8_t *w, const float *x, const 
     uint32_t blocks = nrounds < (uint32_t)ctx->num_cus ? nrounds : (uint32_t)ctx->num_cus;
     if (partials && blocks > lev_ctx::kArgmaxPartials) blocks = lev_ctx::kArgmaxPartials;
     uint32_t *tickets = partials ? reinterpret_cast<uint32_t *>(ctx->d_flag) + lev_ctx::kArgmaxTicketWord : nullptr;
-    hipLaunchKernelGGL((q6_k_mfma_gemv_one<NC, NORM>), dim3(blocks), dim3(kQThreads), lds, ctx->stream, w, x, gain,
-                       eps, y, cols, rows, ncol, wpr, slots, slot_of_wave, pos_of_wave, 1.0 / (double)cols, partials,
-                       tickets, d_argmax, d_margin);
+    hipLaunchKernelGGL((q6_k_mfma_gemv_one<NC, NORM, MAXW>), dim3(blocks), dim3(slots * wpr * LEV_WAVE), lds, ctx->stream,
+                       w, x, gain, eps, y, cols, rows, ncol, wpr, slots, slot_of_wave, pos_of_wave, 1.0 / (double)cols,
+                       partials, tickets, d_argmax, d_margin);
     return hipGetLastError();
+}
+
+// Rows of six, nine, ten, eleven or twelve superblocks fill no more than twelve of the sixteen waves: the registers of
+// the other four hold a third row group in flight, without which such a row streams at its share of waves (2816 columns
+// x 262144: 127 us with two in flight, 101 with three).
+template <int NC, bool NORM>
+hipError_t q6m_one_launch(lev_ctx *ctx, const uint8_t *w, const float *x, const float *gain, float eps, float *y,
+                          uint32_t cols, uint32_t rows, uint32_t ncol, lev_f32x4 *partials, uint32_t *d_argmax,
+                          float *d_margin) {
+    const uint32_t wpr = cols >> 8;
+    if ((uint32_t)kQWaves / wpr * wpr <= kQ1FewWaves)
+        return q6m_one_launch_waves<NC, NORM, kQ1FewWaves>(ctx, w, x, gain, eps, y, cols, rows, ncol, partials, d_argmax, d_margin);
+    return q6m_one_launch_waves<NC, NORM, kQWaves>(ctx, w, x, gain, eps, y, cols, rows, ncol, partials, d_argmax, d_margin);
 }
 
 template <int NC>
@@ -1395,7 +1422,7 @@ hipError_t q6m_q8_one_launch(lev_ctx *ctx, const uint8_t *w, const uint32_t *xq,
         configured = true;
     }
     const uint32_t blocks = nrounds < (uint32_t)ctx->num_cus ? nrounds : (uint32_t)ctx->num_cus;
-    hipLaunchKernelGGL((q6_k_mfma_gemv_q8_one<NC>), dim3(blocks), dim3(kQThreads), lds, ctx->stream, w, xq, xs, y,
+    hipLaunchKernelGGL((q6_k_mfma_gemv_q8_one<NC>), dim3(blocks), dim3(slots * wpr * LEV_WAVE), lds, ctx->stream, w, xq, xs, y,
                        cols, rows, ncol, wpr, slots, slot_of_wave, pos_of_wave);
     return hipGetLastError();
 }
