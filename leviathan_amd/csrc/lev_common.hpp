@@ -46,7 +46,8 @@ struct lev_ctx {
     // zero between launches (the last workgroup to arrive resets its counter)
     int *d_flag = nullptr;
     // words kArgmaxTicketWord + 1024*k, k = 0..8: arrival counters of the greedy-token merge
-    // (4 KB apart: counters that share a cache line serialise in one L2 channel), zero between launches
+    // (4 KB apart: counters that share a cache line serialise in one L2 channel), zero between launches;
+    // words kArgmaxTicketWord + 512 + 16*c: those of the columns of the argmax operator
     static constexpr uint32_t kFlagWords = 10 * 1024, kTicketWord = 16, kArgmaxTicketWord = 1024;
     int *h_flag = nullptr;   // pinned
     // True between lev_hip_program_begin and lev_hip_program_end: the stream

@@ -467,43 +467,78 @@ q6_k_gemv_generic(const uint8_t *__restrict__ w, const float *__restrict__ x,
     if (lane == LEV_WAVE - 1) y[row] = (float)acc;
 }
 
-__global__ void __launch_bounds__(1024)
-argmax_kernel(const float *__restrict__ logits, uint32_t vocab, uint32_t *__restrict__ out_idx,
-              float *__restrict__ out_margin) {
+// Greedy token of each column: gridDim.x workgroups a column (blockIdx.y) take a share of the logits each, the last of
+// a column to finish merges their records (one workgroup a column instead is a chain of round trips: 47 us for 130000
+// logits, 5 with 32).  tickets: a zero counter per column, left at zero; unused with one workgroup a column.
+constexpr uint32_t kArgmaxThreads = 1024, kArgmaxLoads = 4, kArgmaxMaxParts = 64, kArgmaxTicketStep = 16;
+
+__global__ void __launch_bounds__(kArgmaxThreads)
+argmax_kernel(const float *__restrict__ logits, uint32_t vocab, lev_f32x4 *__restrict__ partials,
+              uint32_t *__restrict__ tickets, uint32_t *__restrict__ out_idx, float *__restrict__ out_margin) {
     __shared__ float s_best[16], s_second[16];
     __shared__ uint32_t s_idx[16];
-    const float *l = logits + (uint64_t)blockIdx.x * vocab;
-    const uint32_t t = threadIdx.x;
+    const uint32_t col = blockIdx.y, parts = gridDim.x, t = threadIdx.x, lane = t & 63u;
+    const float *l = logits + (uint64_t)col * vocab;
     top2 m{kTop2Floor, kTop2Floor, 0xFFFFFFFFu};
-    for (uint32_t i = t; i < vocab; i += 1024) {
-        float v = l[i];
-        if (v > m.best) {
-            m.second = m.best;
-            m.best = v;
-            m.idx = i;
-        } else if (v > m.second) {
-            m.second = v;
+    for (uint32_t i0 = blockIdx.x * (kArgmaxThreads * kArgmaxLoads) + t; i0 < vocab;
+         i0 += parts * (kArgmaxThreads * kArgmaxLoads)) {
+        float v[kArgmaxLoads];
+#pragma unroll
+        for (uint32_t u = 0; u < kArgmaxLoads; ++u) {
+            const uint32_t i = i0 + u * kArgmaxThreads;
+            v[u] = l[i < vocab ? i : i0];
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < kArgmaxLoads; ++u) {
+            const uint32_t i = i0 + u * kArgmaxThreads;
+            if (i >= vocab) break;
+            if (v[u] > m.best) {
+                m.second = m.best;
+                m.best = v[u];
+                m.idx = i;
+            } else if (v[u] > m.second) {
+                m.second = v[u];
+            }
         }
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        top2 o;
-        o.best = __shfl_xor(m.best, off);
-        o.second = __shfl_xor(m.second, off);
-        o.idx = __shfl_xor(m.idx, off);
-        m = top2_merge(m, o);
-    }
-    if ((t & 63u) == 0) {
+    m = top2_wave(m);
+    if (lane == 0u) {
         s_best[t >> 6] = m.best;
         s_second[t >> 6] = m.second;
         s_idx[t >> 6] = m.idx;
     }
     __syncthreads();
-    if (t == 0) {
-        top2 r{s_best[0], s_second[0], s_idx[0]};
-        for (int k = 1; k < 16; ++k) r = top2_merge(r, top2{s_best[k], s_second[k], s_idx[k]});
-        if (out_idx) out_idx[blockIdx.x] = r.idx == 0xFFFFFFFFu ? 0u : r.idx;
-        if (out_margin) out_margin[blockIdx.x] = r.best - r.second;
+    if (t >= LEV_WAVE) return;
+    m = top2{kTop2Floor, kTop2Floor, 0xFFFFFFFFu};
+    if (lane < 16u) m = top2{s_best[lane], s_second[lane], s_idx[lane]};
+    m = top2_wave(m);
+    if (parts > 1u) {
+        uint32_t last = 0u;
+        float *rec = reinterpret_cast<float *>(partials + (uint64_t)col * parts);
+        if (lane == 0u) {
+            float *pf = rec + 4u * blockIdx.x;
+            __hip_atomic_store(pf, m.best, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(pf + 1, m.second, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(pf + 2, __builtin_bit_cast(float, m.idx), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            lev_publish_wait();
+            uint32_t *ticket = tickets + kArgmaxTicketStep * col;
+            if (__hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == parts - 1u) {
+                __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                last = 1u;
+            }
+        }
+        if (!__builtin_amdgcn_readfirstlane((int)last)) return;
+        m = top2{kTop2Floor, kTop2Floor, 0xFFFFFFFFu};
+        if (lane < parts) {
+            m.best = __hip_atomic_load(rec + 4u * lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            m.second = __hip_atomic_load(rec + 4u * lane + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            m.idx = __float_as_uint(__hip_atomic_load(rec + 4u * lane + 2u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        }
+        m = top2_wave(m);
+    }
+    if (lane == 0u) {
+        if (out_idx) out_idx[col] = m.idx == 0xFFFFFFFFu ? 0u : m.idx;
+        if (out_margin) out_margin[col] = m.best - m.second;
     }
 }
 
@@ -537,6 +572,8 @@ hipError_t launch_units(lev_ctx *ctx, const uint8_t *w, const float *x, float *y
 }
 
 }  // namespace
+
+hipError_t lev_argmax_launch(lev_ctx *ctx, const float *logits, uint32_t vocab, uint32_t ncol, uint32_t *idx, float *margin);
 
 uint32_t lev_q6_k_mfma_cols(const lev_ctx *ctx, uint32_t in_dim);
 uint32_t lev_q6_k_mfma_waves(const lev_ctx *ctx, uint32_t in_dim, uint32_t rows);
@@ -610,9 +647,7 @@ hipError_t lev_q6_k_gemv_argmax_launch(lev_ctx *ctx, const uint8_t *w, const flo
                            units, rows);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess || (!d_argmax && !d_margin)) return e;
-        hipLaunchKernelGGL(argmax_kernel, dim3(1), dim3(1024), 0, ctx->stream, y, rows, d_argmax,
-                           d_margin);
-        return hipGetLastError();
+        return lev_argmax_launch(ctx, y, rows, 1u, d_argmax, d_margin);
     }
     if (units > 128) return launch_units<64, 4, false>(ctx, w, x, y, units, rows, d_argmax, d_margin);
     if (units > 64) {
@@ -631,10 +666,18 @@ hipError_t lev_q6_k_gemv_launch(lev_ctx *ctx, const uint8_t *w, const float *x, 
     return lev_q6_k_gemv_argmax_launch(ctx, w, x, y, in_dim, rows, nullptr, nullptr);
 }
 
+// Workgroups a column: one per 4096 logits (all of them requested at once), at most a lane each of the wave that
+// merges; one alone beyond sixteen columns, which fill the chip's memory queues by themselves and have no counters.
 hipError_t lev_argmax_launch(lev_ctx *ctx, const float *logits, uint32_t vocab, uint32_t ncol,
                              uint32_t *idx, float *margin) {
-    hipLaunchKernelGGL(argmax_kernel, dim3(ncol), dim3(1024), 0, ctx->stream, logits, vocab, idx,
-                       margin);
+    constexpr uint32_t per = kArgmaxThreads * kArgmaxLoads;
+    uint32_t parts = ncol <= 16u ? (uint32_t)(((uint64_t)vocab + per - 1u) / per) : 1u;
+    if (parts > kArgmaxMaxParts) parts = kArgmaxMaxParts;
+    static_assert(16u * kArgmaxMaxParts <= lev_ctx::kArgmaxPartials, "records of sixteen columns");
+    static_assert(16u * kArgmaxTicketStep <= 512u, "counters of sixteen columns, in the page of counter 0");
+    uint32_t *tickets = reinterpret_cast<uint32_t *>(ctx->d_flag) + lev_ctx::kArgmaxTicketWord + 512u;
+    hipLaunchKernelGGL(argmax_kernel, dim3(parts, ncol), dim3(kArgmaxThreads), 0, ctx->stream, logits, vocab,
+                       static_cast<lev_f32x4 *>(ctx->argmax_partials), tickets, idx, margin);
     return hipGetLastError();
 }
 
