@@ -200,10 +200,9 @@ q4_0_gemv_pairs(const uint8_t *__restrict__ w, const float *__restrict__ x, floa
     }
 }
 
-// Any geometry (odd block counts, rows that are only 2-byte aligned, rows too
-// long for LDS): one wave per row, 16-bit loads, activations from global
-// memory.  Correct everywhere, fast nowhere; the pair kernel covers every
-// shape the models on this path use.
+// Any geometry (matrices that are only 2-byte aligned, rows too long for LDS):
+// one wave per row, 16-bit loads, activations from global memory.  Correct
+// everywhere, fast nowhere.
 __global__ void __launch_bounds__(256)
 q4_0_gemv_generic(const uint8_t *__restrict__ w, const float *__restrict__ x,
                   float *__restrict__ y, uint32_t blocks_per_row, uint32_t rows) {
@@ -272,6 +271,7 @@ hipError_t launch_pairs(lev_ctx *ctx, const uint8_t *w, const float *x, float *y
 bool lev_q4_0_mfma_gemv_usable(const uint8_t *w, const float *x, uint32_t in_dim);
 hipError_t lev_q4_0_mfma_gemv_launch(lev_ctx *ctx, const uint8_t *w, const float *x, float *y, uint32_t in_dim,
                                      uint32_t rows, int persistent);
+void lev_q4_0_mfma_gemv_choice(const lev_ctx *ctx, uint32_t in_dim, uint32_t rows, uint32_t *persistent, bool *other);
 
 // Enqueue without argument checks (callers validated the geometry).
 hipError_t lev_q4_0_gemv_launch(lev_ctx *ctx, const uint8_t *w, const float *x, float *y,
@@ -346,11 +346,11 @@ uint32_t lev_q4_0_gemv_candidates(const lev_ctx *ctx, uint32_t in_dim, uint32_t 
     // where it serves, the matrix-core kernel (family 1) is the built-in choice, with one workgroup per
     // round of row groups or a resident grid
     if (lev_q4_0_mfma_in_dim(in_dim)) {
-        const uint32_t ntask = (in_dim + 255u) >> 8, slots = ntask <= 16u ? 16u / ntask : 1u;
-        const uint32_t nrounds = ((rows + 15u) / 16u + slots - 1u) / slots;
-        const uint32_t builtin = nrounds <= (uint32_t)ctx->num_cus ? 0u : 1u;
+        uint32_t builtin;
+        bool other;
+        lev_q4_0_mfma_gemv_choice(ctx, in_dim, rows, &builtin, &other);
         all[n++] = lev_schedule{LEV_OP_Q4_0_GEMV, 1u, 0u, builtin};
-        all[n++] = lev_schedule{LEV_OP_Q4_0_GEMV, 1u, 0u, 1u - builtin};
+        if (other) all[n++] = lev_schedule{LEV_OP_Q4_0_GEMV, 1u, 0u, 1u - builtin};
     }
     if (!family) {
         push(0u, 0u);   // the vector-ALU kernel of the shape, which has no parameters here

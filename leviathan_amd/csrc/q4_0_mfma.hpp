@@ -31,11 +31,14 @@
 
 typedef int lev_i32x4 __attribute__((ext_vector_type(4)));
 
-constexpr uint32_t kLevQ4MfmaMaxInDim = 8192u;   // widest row the matrix-core GEMV takes
-// Rows it takes: whole 256-value tasks, and from five tasks on rows that end inside one (narrower ones of
-// those are the launch floor with either kernel, 3 us at 1088 x 5000, and stay with the vector-ALU kernels).
+// Rows the matrix-core GEMV takes, up to 8192 values: whole 256-value tasks, and from five tasks on rows that end
+// inside one (narrower ones of those are the launch floor with either kernel, 3 us at 1088 x 5000, and stay with the
+// vector-ALU kernels).  From a task on and up to 16384 values: rows of an odd number of blocks, which only a kernel of
+// 2-byte loads takes beside it (narrower ones keep that: the experts' kernels form such rows' sums in its order).
 __host__ inline bool lev_q4_0_mfma_in_dim(uint32_t in_dim) {
-    return in_dim != 0u && in_dim <= kLevQ4MfmaMaxInDim && (in_dim % 256u == 0u || (in_dim % 64u == 0u && in_dim > 1280u));
+    if (in_dim == 0u || in_dim % 32u != 0u) return false;
+    if (in_dim % 64u != 0u) return in_dim > 256u && in_dim <= 16384u;
+    return in_dim <= 8192u && (in_dim % 256u == 0u || in_dim > 1280u);
 }
 constexpr uint32_t kQ4mTaskArea = 1024u;   // LDS bytes of one staged task: [pair 4][plane 4][half 4][16 B]
 constexpr uint32_t kQ4mZeroBytes = 16u;    // what the lanes outside a row's own lane group read as their A operand
@@ -48,12 +51,10 @@ struct q4m_operand {
 };
 
 // Stages the task whose activations are v (lane i holds elements 4i..4i+3 of the task's 256)
-// into `area` (kQ4mTaskArea bytes, this wave's own) and reads the lane's A operands back.
-// `zero` points at kQ4mZeroBytes of zeros.  live == false: the task lies beyond the row (its
-// operands are zero, it adds nothing).  A NaN or an infinity among the 64 activations of a pair
+// into `area` (kQ4mTaskArea bytes, this wave's own); returns the lane's `unscale`.  live == false: the
+// task lies beyond the row (it adds nothing).  A NaN or an infinity among the 64 activations of a pair
 // makes the pair's factor NaN, and with it every row's sum.
-__device__ __forceinline__ void q4m_stage_task(const lev_f32x4 v, uint8_t *area, const uint8_t *zero,
-                                               bool live, q4m_operand &op) {
+__device__ __forceinline__ float q4m_stage_planes(const lev_f32x4 v, uint8_t *area, bool live) {
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t r = lane & 15u, g = lane >> 4;
     uint32_t mb = 0u;
@@ -67,7 +68,7 @@ __device__ __forceinline__ void q4m_stage_task(const lev_f32x4 v, uint8_t *area,
     const bool bad = ex == 255u;
     ex = ex < 34u ? 34u : (ex > 254u ? 254u : ex);             // keeps both powers of two normal numbers
     const float scale = __uint_as_float((283u - ex) << 23);    // 2^(156 - ex): |x * scale| < 2^30
-    op.unscale = !live ? 0.f : bad ? __builtin_nanf("") : __uint_as_float((ex - 33u) << 23);   // 2^(ex - 160)
+    const float unscale = !live ? 0.f : bad ? __builtin_nanf("") : __uint_as_float((ex - 33u) << 23);   // 2^(ex - 160)
     uint32_t Y[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) Y[k] = ((uint32_t)(int)rintf(v[k] * scale) + 0x00808080u) ^ 0x00808080u;
@@ -90,11 +91,25 @@ __device__ __forceinline__ void q4m_stage_task(const lev_f32x4 v, uint8_t *area,
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    return unscale;
+}
+
+// The lane's A operands of a staged task.  `zero` points at kQ4mZeroBytes of zeros: what a lane outside the
+// row's own lane group reads, and every lane of a task that is not live.
+__device__ __forceinline__ void q4m_read_operands(const uint8_t *area, const uint8_t *zero, bool live, q4m_operand &op) {
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t r = lane & 15u, g = lane >> 4;
     const bool feeds = live && (r >> 2) == g;                  // A row r belongs to lane group r / 4
     const uint8_t *ab = feeds ? area + g * 256u + (r & 3u) * 64u : zero;
     const uint32_t hs = feeds ? 16u : 0u;
 #pragma unroll
     for (int h = 0; h < 4; ++h) op.a[h] = *reinterpret_cast<const lev_i32x4 *>(ab + h * hs);
+}
+
+__device__ __forceinline__ void q4m_stage_task(const lev_f32x4 v, uint8_t *area, const uint8_t *zero,
+                                               bool live, q4m_operand &op) {
+    op.unscale = q4m_stage_planes(v, area, live);
+    q4m_read_operands(area, zero, live, op);
 }
 
 // The weights of one task as they are fetched: lane 4*row + pair holds pair `pair` of row `row`.
@@ -111,11 +126,27 @@ __device__ __forceinline__ void q4m_load_task_part(const uint8_t *rowp, uint32_t
     lev_q4_load_pair(rowp + (uint64_t)((pair < npairs ? pair : npairs - 1u) * 36u), D);
 }
 
-// The 256 activations of task T of a vector of n4 float4: lane i requests elements 4i..4i+3; past the end the
-// vector's last ones are requested, and `live` (what to pass to q4m_mask_activations behind the wait) is false.
-__device__ __forceinline__ lev_f32x4 q4m_load_activations(const float *x, uint32_t T, uint32_t n4, bool &live) {
-    const uint32_t i = 64u * T + (threadIdx.x & 63u);
-    live = i < n4;
+// The same for rows of an odd number of blocks, whose half of a pair may end the matrix, at w_end: nothing behind it is
+// requested.  Of such a pair block A is right, its last two bytes moved to where they belong, and block B arbitrary.
+__device__ __forceinline__ void q4m_load_task_odd(const uint8_t *rowp, uint32_t task_pair0, uint32_t npairs, const uint8_t *w_end, uint32_t D[9]) {
+    struct __attribute__((packed, aligned(2))) u4 { uint32_t v[4]; };
+    struct __attribute__((packed, aligned(2))) u1 { uint32_t v; };
+    const uint32_t pair = task_pair0 + (threadIdx.x & 3u);
+    const uint8_t *p = rowp + (uint64_t)((pair < npairs ? pair : npairs - 1u) * 36u);
+    const bool half = w_end - p < 36;
+    const u4 a = *reinterpret_cast<const u4 *>(p);
+    const u1 m = *reinterpret_cast<const u1 *>(half ? p + 14 : p + 16);
+    const u4 b = *reinterpret_cast<const u4 *>(half ? p : p + 20);
+    D[0] = a.v[0], D[1] = a.v[1], D[2] = a.v[2], D[3] = a.v[3];
+    D[4] = half ? m.v >> 16 : m.v;
+    D[5] = b.v[0], D[6] = b.v[1], D[7] = b.v[2], D[8] = b.v[3];
+}
+
+// The 256 activations of task T of a vector of n4 float4: lane i requests elements 4i..4i+3 (`late` float4 earlier); past
+// either end one of the vector's is requested, and `live` (what to pass to q4m_mask_activations behind the wait) is false.
+__device__ __forceinline__ lev_f32x4 q4m_load_activations(const float *x, uint32_t T, uint32_t n4, bool &live, uint32_t late = 0u) {
+    const uint32_t i = 64u * T + (threadIdx.x & 63u) - late;
+    live = i < n4;                                             // (a lane before the first element wraps round)
     return reinterpret_cast<const lev_f32x4 *>(x)[live ? i : n4 - 1u];
 }
 __device__ __forceinline__ lev_f32x4 q4m_mask_activations(lev_f32x4 v, bool live) {

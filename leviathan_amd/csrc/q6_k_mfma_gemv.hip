@@ -938,22 +938,52 @@ q6_k_mfma_gemv_q8(const uint8_t *__restrict__ w, const uint32_t *__restrict__ xq
     q6m_regs W0, W1, W2;
 
     // ---- stage the activations: the codes as they come, the block scales transposed ----
-    if (tid < kQZeroBytes / 4u) reinterpret_cast<uint32_t *>(zero)[tid] = 0u;
-    {
-        const lev_u32x4 *src = reinterpret_cast<const lev_u32x4 *>(xq);
-        lev_u32x4 *dst = reinterpret_cast<lev_u32x4 *>(dig);
-        const uint32_t n16 = ncol * (cols >> 4);
-        for (uint32_t i = tid; i < n16; i += kQThreads) dst[i] = src[i];
-        // columns of the layout beyond ncol: zero codes and scales (their outputs are never stored)
-        for (uint32_t i = n16 + tid; i < (uint32_t)NC * (cols >> 4); i += kQThreads) dst[i] = lev_u32x4{0u, 0u, 0u, 0u};
-        for (uint32_t i = tid; i < nblk * NC; i += kQThreads) {
-            const uint32_t c = i & (NC - 1u), b = i >> kLogNC;
-            // a quarter of the activation scale: the codes in the operand are 4*(q - 32)
-            dxs[i] = c < ncol ? 0.25f * xs[((uint64_t)c * nblk + b) * 2u] : 0.f;
-        }
+    // Every wave requests its share, and once all have (a CU's memory pipeline is one queue) the first
+    // tasks' weights behind it: they are on their way while the activations go into LDS.  (Requested
+    // behind that barrier, and so a round trip later, they cost 4096 x 12288 2 of 14 us.)
+    constexpr int CH = 4, CS = 3;                            // pieces requested ahead of the weights
+    const lev_u32x4 *src = reinterpret_cast<const lev_u32x4 *>(xq);
+    lev_u32x4 *dst = reinterpret_cast<lev_u32x4 *>(dig);
+    const uint32_t n16 = ncol * (cols >> 4), all16 = (uint32_t)NC * (cols >> 4), nsc = nblk * NC;
+    auto scale_of = [&](uint32_t i) {
+        const uint32_t c = i & (NC - 1u), b = i >> kLogNC;
+        // (columns of the layout beyond ncol: zero codes and scales, their outputs are never stored)
+        return xs[((uint64_t)(c < ncol ? c : 0u) * nblk + b) * 2u];
+    };
+    lev_u32x4 xv[CH];
+    float sv[CS];
+#pragma unroll
+    for (int k = 0; k < CH; ++k) {
+        const uint32_t i = tid + (uint32_t)k * kQThreads;
+        xv[k] = src[i < n16 ? i : 0u];
     }
-    lev_barrier_lds();
+#pragma unroll
+    for (int k = 0; k < CS; ++k) {
+        const uint32_t i = tid + (uint32_t)k * kQThreads;
+        sv[k] = scale_of(i < nsc ? i : 0u);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_barrier" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
     issue(ci, W0);
+    issue(ci, W1);
+    if (DEPTH > 2) issue(ci, W2);
+    __builtin_amdgcn_sched_barrier(0);
+    if (tid < kQZeroBytes / 4u) reinterpret_cast<uint32_t *>(zero)[tid] = 0u;
+#pragma unroll
+    for (int k = 0; k < CH; ++k) {
+        const uint32_t i = tid + (uint32_t)k * kQThreads;
+        if (i < all16) dst[i] = i < n16 ? xv[k] : lev_u32x4{0u, 0u, 0u, 0u};
+    }
+#pragma unroll
+    for (int k = 0; k < CS; ++k) {
+        const uint32_t i = tid + (uint32_t)k * kQThreads;
+        // a quarter of the activation scale: the codes in the operand are 4*(q - 32)
+        if (i < nsc) dxs[i] = (i & (NC - 1u)) < ncol ? 0.25f * sv[k] : 0.f;
+    }
+    for (uint32_t i = tid + CH * kQThreads; i < all16; i += kQThreads) dst[i] = i < n16 ? src[i] : lev_u32x4{0u, 0u, 0u, 0u};
+    for (uint32_t i = tid + CS * kQThreads; i < nsc; i += kQThreads) dxs[i] = (i & (NC - 1u)) < ncol ? 0.25f * scale_of(i) : 0.f;
+    lev_barrier_lds();
 
     // ---- stream the weights ----
     const uint32_t hf = g >> 1, jb = g & 1u;
@@ -1033,8 +1063,6 @@ q6_k_mfma_gemv_q8(const uint8_t *__restrict__ w, const uint32_t *__restrict__ xq
         advance(c);
     };
 
-    issue(ci, W1);
-    if (DEPTH > 2) issue(ci, W2);
     while (true) {
         compute(cc, W0);
         __builtin_amdgcn_sched_barrier(0);
