@@ -340,16 +340,18 @@ hipError_t lev_q4_k_mfma_gemv_launch(lev_ctx *ctx, const uint8_t *w, const float
 // wherever its activation staging fits; the vector-ALU kernel (f32 FMA chains)
 // takes the other shapes and stays a candidate for lev_hip_forge_select.
 uint32_t lev_q4_k_mfma_narrow_cols(const lev_ctx *ctx, uint32_t in_dim);
+bool lev_q4_k_mfma_planes(const lev_ctx *ctx, uint32_t in_dim, uint32_t rows, uint32_t ncol);
 
 // Whether the matrix-core family takes this shape: its four-columns-per-product kernel up to
-// in_dim 8192, its one- and two-column kernel up to in_dim 32768 / ncol.
-static bool q4k_mfma_serves(const lev_ctx *ctx, uint32_t in_dim, uint32_t ncol) {
-    return lev_q4_k_mfma_cols(ctx, in_dim) != 0u || ncol <= lev_q4_k_mfma_narrow_cols(ctx, in_dim);
+// in_dim 8192, up to in_dim 16384 from three columns on with the planes made in front, its one-
+// and two-column kernel up to in_dim 32768 / ncol.
+static bool q4k_mfma_serves(const lev_ctx *ctx, uint32_t in_dim, uint32_t rows, uint32_t ncol) {
+    return lev_q4_k_mfma_cols(ctx, in_dim) != 0u || ncol <= lev_q4_k_mfma_narrow_cols(ctx, in_dim) ||
+           lev_q4_k_mfma_planes(ctx, in_dim, rows, ncol);
 }
 
 static uint32_t q4k_builtin_family(const lev_ctx *ctx, uint32_t in_dim, uint32_t rows, uint32_t ncol) {
-    (void)rows;
-    return q4k_mfma_serves(ctx, in_dim, ncol) ? 1u : 0u;
+    return q4k_mfma_serves(ctx, in_dim, rows, ncol) ? 1u : 0u;
 }
 
 hipError_t lev_q4_k_gemv_launch(lev_ctx *ctx, const uint8_t *w, const float *x, const float *gain,
@@ -363,6 +365,15 @@ hipError_t lev_q4_k_gemv_launch(lev_ctx *ctx, const uint8_t *w, const float *x, 
     // one column, or two of a row too wide for the four-column kernel: the narrow kernel
     if (mfma && ncol <= lev_q4_k_mfma_narrow_cols(ctx, in_dim) && (ncol == 1u || lev_q4_k_mfma_cols(ctx, in_dim) < ncol))
         return lev_q4_k_mfma_gemv_launch(ctx, w, x, gain, eps, y, in_dim, rows, ncol);
+    while (mfma && done < ncol) {
+        const uint32_t nc = ncol - done < 8u ? ncol - done : 8u;
+        if (!lev_q4_k_mfma_planes(ctx, in_dim, rows, nc)) break;
+        hipError_t e = lev_q4_k_mfma_gemv_launch(ctx, w, x + (uint64_t)done * in_dim, gain, eps,
+                                                 y + (uint64_t)done * rows, in_dim, rows, nc);
+        if (e == hipErrorOutOfMemory) break;
+        if (e != hipSuccess) return e;
+        done += nc;
+    }
     const uint32_t mfma_cols = mfma ? lev_q4_k_mfma_cols(ctx, in_dim) : 0u;
     while (mfma_cols && done < ncol) {
         uint32_t nc = ncol - done < mfma_cols ? ncol - done : mfma_cols;
@@ -400,7 +411,7 @@ uint32_t lev_q4_k_gemv_candidates(const lev_ctx *ctx, uint32_t in_dim, uint32_t 
     uint32_t n = 0;
     if (n < capacity) out[n] = lev_schedule{LEV_OP_Q4_K_GEMV, first, 0u, 0u};
     ++n;
-    if (q4k_mfma_serves(ctx, in_dim, ncol)) {
+    if (q4k_mfma_serves(ctx, in_dim, rows, ncol)) {
         if (n < capacity) out[n] = lev_schedule{LEV_OP_Q4_K_GEMV, 1u - first, 0u, 0u};
         ++n;
     }

@@ -37,8 +37,8 @@
 // activations take 64 KB of LDS).  The waves of a workgroup share 16 weight rows,
 // one superblock column each; their partial sums meet in LDS.
 //
-// Five to eight columns of at most sixteen superblocks: the planes are made once per launch
-// by a small kernel in front (q4k_planes_kernel, below) instead of by every workgroup.
+// Five to eight columns, or three and more of a row of more than sixteen superblocks: the planes are made
+// once per launch by a small kernel in front (q4k_planes_kernel, below) instead of by every workgroup.
 //
 // A NaN or infinity in a column of x makes every output of that column NaN.
 #include "lev_common.hpp"
@@ -119,57 +119,85 @@ struct q4k_lds {
 //
 // Turning a column of activations into digit planes costs a compute unit about a
 // microsecond whoever does it, and in q4_k_mfma_gemv every workgroup does it for every
-// column: at eight columns that is more than half of the kernel's instructions.  For five
-// to eight columns of at most sixteen superblocks q4k_planes_kernel (one workgroup per
-// column) writes the planes to device scratch in the order the matrix cores read them, and
+// column: at eight columns that is more than half of the kernel's instructions, and from 16384
+// values on they do not fit its LDS.  So q4k_planes_kernel (one workgroup per column) writes the planes to device scratch in the order the matrix cores read them, and
 // the workgroups of q4_k_mfma_gemv<NC, SHORT, true> load the planes of their wave's
 // superblock column straight into registers: no staging, no digit area in LDS, no LDS read
 // per product.  The numbers are the same integers, so the outputs are the same bits.
 //
+// A row of more than sixteen superblocks is cut into slices of at most sixteen (gridDim.y), a workgroup
+// taking one: the sums of a row group's slices meet in scratch, in f64, and the last workgroup to get there
+// adds them in order (hand-over as in lev_common.hpp; every row group has a counter, cleared with the
+// planes).  Six columns of 6095 x 4608 25.5 us with four columns a launch, 14.0 like this; seven of
+// 1052 x 8448 40.1 us on the vector ALU, 11.4; eight of 16000 x 12288 199 and 43.
+//
 // Scratch, for NX groups of four layout columns and SB superblocks:
 //   planes [SB][4 sub-block pairs][NX][64 lanes][16 B]   lane (r, g): A row r (4 * (column % 4) + plane,
 //          plane 0 the highest digit), k-group g, of sub-blocks 2jp (low 8 bytes) and 2jp + 1 (high)
-//   psb    [SB][4 * NX] f64                               2^(e-151) per superblock and column
-//   bad    [4 * NX] u32                                   a NaN or infinity in the column
+//   psb    [SB][4 * NX] f64                               2^(e-151) per superblock and column; NaN where one of
+//          its activations is NaN or infinite, and with it every output of the column
+//   count  [row groups] u32 and sums [slices][row groups][4 * NX][16] f64, where the row is cut
 // The sum of X per sub-block (for the mins) is not stored: the matrix cores form
 // sum_j m_j * sum_k digit directly, with the min of a sub-block in all of its B bytes.
 // ---------------------------------------------------------------------------
-constexpr int kPThreads = 512;   // one run of 8 activations per thread: in_dim <= 4096
+constexpr uint32_t kPThreads = 512;   // a run of 8 activations per thread
+constexpr uint32_t kPMaxParts = 4u, kPMaxCols = kPMaxParts * 8u * kPThreads;
 __host__ __device__ constexpr size_t q4k_planes_bytes(uint32_t sb, uint32_t nx) { return (size_t)sb * nx * 4096u; }
-__host__ __device__ constexpr size_t q4k_planes_total(uint32_t sb, uint32_t nx) {
-    return q4k_planes_bytes(sb, nx) + (size_t)sb * 4u * nx * 8u + 4u * nx * 4u;
+__host__ __device__ constexpr size_t q4k_count_at(uint32_t sb, uint32_t nx) {
+    return q4k_planes_bytes(sb, nx) + (size_t)sb * 4u * nx * 8u;
+}
+__host__ __device__ constexpr size_t q4k_sums_at(uint32_t sb, uint32_t nx, uint32_t groups) {
+    return q4k_count_at(sb, nx) + ((size_t)groups + 1u) / 2u * 8u;
+}
+__host__ __device__ constexpr size_t q4k_planes_total(uint32_t sb, uint32_t nx, uint32_t groups, uint32_t slices) {
+    return slices > 1u ? q4k_sums_at(sb, nx, groups) + (size_t)slices * groups * nx * 512u : q4k_count_at(sb, nx);
 }
 
-// grid (ncol), kPThreads threads; cols % 256 == 0, cols <= 8 * kPThreads; x and gain 16-byte aligned.
+// grid (ncol, PARTS), PARTS parts of the column of 8 * kPThreads values, the last one shorter: a part is one
+// workgroup's to convert (four columns of 12288 by one workgroup each: 6.7 us, 4.1 in three parts), the sum of
+// squares every part forms for itself.  cols % 256 == 0; x and gain 16-byte aligned.  nclear: counters to clear.
+template <int PARTS>
 __global__ void __launch_bounds__(kPThreads)
 q4k_planes_kernel(const float *__restrict__ x, const float *__restrict__ gain, float eps, uint8_t *__restrict__ scratch,
-                  uint32_t cols, uint32_t nx, double rcols) {
-    __shared__ double run[kPThreads / 4];
+                  uint32_t cols, uint32_t nx, double rcols, uint32_t nclear) {
+    __shared__ double run[PARTS * kPThreads / 4];
     __shared__ double s_inv;
-    __shared__ uint32_t s_bad;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const uint32_t c = blockIdx.x, SB = cols >> 8, subs = cols >> 5, NL = 4u * nx;
     uint8_t *planes = scratch;
     double *psb = reinterpret_cast<double *>(scratch + q4k_planes_bytes(SB, nx));
-    uint32_t *bad = reinterpret_cast<uint32_t *>(psb + (size_t)SB * NL);
-    const bool real = tid < (cols >> 3);
-    const uint32_t k8 = real ? tid : 0u;
-    const lev_f32x4 *xp = reinterpret_cast<const lev_f32x4 *>(x + (uint64_t)c * cols) + 2u * k8;
-    lev_f32x4 va = xp[0], vb = xp[1];
-    if (tid == 0u) s_bad = 0u;
+    if (c == 0u && blockIdx.y == 0u)
+        for (uint32_t i = tid; i < nclear; i += kPThreads)
+            reinterpret_cast<uint32_t *>(scratch + q4k_count_at(SB, nx))[i] = 0u;
+    const uint32_t part0 = blockIdx.y * kPThreads, runs = cols >> 3;
+    auto load = [&](uint32_t k, lev_f32x4 &a, lev_f32x4 &b) {
+        const lev_f32x4 *xp = reinterpret_cast<const lev_f32x4 *>(x + (uint64_t)c * cols) + 2u * (k < runs ? k : 0u);
+        a = xp[0], b = xp[1];
+    };
+    const bool real = part0 + tid < runs;
+    const uint32_t k8 = real ? part0 + tid : 0u;
+    lev_f32x4 va, vb;
+    load(part0 + tid, va, vb);
     if (gain) {
         const lev_f32x4 *gp = reinterpret_cast<const lev_f32x4 *>(gain) + 2u * k8;
         const lev_f32x4 ga = gp[0], gb = gp[1];
         // RMSNorm as the reference computes it (rmsnorm, rust/crates/lev-model/src/lib.rs:110-114):
         // mean square and 1/sqrt in f64, then (f32)(x * inv) * gain; the additions in the order of
         // q4_k_mfma_gemv (a sub-block's four runs, the sub-blocks lane by lane, the lanes)
-        double ss = (double)va.x * (double)va.x;
-        ss = fma((double)va.y, (double)va.y, ss); ss = fma((double)va.z, (double)va.z, ss);
-        ss = fma((double)va.w, (double)va.w, ss); ss = fma((double)vb.x, (double)vb.x, ss);
-        ss = fma((double)vb.y, (double)vb.y, ss); ss = fma((double)vb.z, (double)vb.z, ss);
-        ss = fma((double)vb.w, (double)vb.w, ss);
-        ss = lev_group_sum_f64<4>(ss);
-        if (real && (k8 & 3u) == 3u) run[k8 >> 2] = ss;
+        lev_f32x4 wa[PARTS], wb[PARTS];
+#pragma unroll
+        for (int i = 0; i < PARTS; ++i) load((uint32_t)i * kPThreads + tid, wa[i], wb[i]);
+#pragma unroll
+        for (int i = 0; i < PARTS; ++i) {
+            const uint32_t k = (uint32_t)i * kPThreads + tid;
+            double ss = (double)wa[i].x * (double)wa[i].x;
+            ss = fma((double)wa[i].y, (double)wa[i].y, ss); ss = fma((double)wa[i].z, (double)wa[i].z, ss);
+            ss = fma((double)wa[i].w, (double)wa[i].w, ss); ss = fma((double)wb[i].x, (double)wb[i].x, ss);
+            ss = fma((double)wb[i].y, (double)wb[i].y, ss); ss = fma((double)wb[i].z, (double)wb[i].z, ss);
+            ss = fma((double)wb[i].w, (double)wb[i].w, ss);
+            ss = lev_group_sum_f64<4>(ss);
+            if (k < runs && (k & 3u) == 3u) run[k >> 2] = ss;
+        }
         lev_barrier_lds();
         if (wave == 0u) {
             double tot = 0.0;
@@ -188,8 +216,6 @@ q4k_planes_kernel(const float *__restrict__ x, const float *__restrict__ gain, f
             va[k] = (float)((double)va[k] * inv) * ga[k];
             vb[k] = (float)((double)vb[k] * inv) * gb[k];
         }
-    } else {
-        lev_barrier_lds();   // s_bad is zero before anybody raises it
     }
     const float v[8] = {va.x, va.y, va.z, va.w, vb.x, vb.y, vb.z, vb.w};
     uint32_t mb = 0u;
@@ -204,7 +230,7 @@ q4k_planes_kernel(const float *__restrict__ x, const float *__restrict__ gain, f
         mb = o > mb ? o : mb;
     }
     uint32_t ex = mb >> 23;
-    if (real && ex == 255u) atomicOr(&s_bad, 1u);
+    const bool bad = ex == 255u;
     ex = ex < 25u ? 25u : (ex > 254u ? 254u : ex);
     const float scale = __uint_as_float((278u - ex) << 23);   // 2^(151-ex): |x*scale| < 2^25
     uint32_t dw[4][2];                                        // dw[3] = highest digit
@@ -228,10 +254,8 @@ q4k_planes_kernel(const float *__restrict__ x, const float *__restrict__ gain, f
         uint8_t *at = planes + ((((size_t)sb * 4u + jp) * nx + q) * 64u + 16u * kg + 4u * (c & 3u)) * 16u + 8u * half;
 #pragma unroll
         for (int p = 0; p < 4; ++p) *reinterpret_cast<lev_u2 *>(at + 16 * p) = lev_u2{dw[3 - p][0], dw[3 - p][1]};
-        if ((k8 & 31u) == 31u) psb[sb * NL + c] = __hiloint2double((int)((ex + 872u) << 20), 0);   // 2^(ex-151)
+        if ((k8 & 31u) == 31u) psb[sb * NL + c] = bad ? (double)__builtin_nanf("") : __hiloint2double((int)((ex + 872u) << 20), 0);   // 2^(ex-151)
     }
-    lev_barrier_lds();
-    if (tid == 0u) bad[c] = s_bad;
 }
 
 // NC: columns staged (1, 2, 4 or 8; >= ncol).  SHORT: no wave has more than
@@ -239,8 +263,9 @@ q4k_planes_kernel(const float *__restrict__ x, const float *__restrict__ gain, f
 // code, so the wait before each task covers exactly that task's loads and each
 // task is multiplied while the next streams in.
 // PLANES: the digit planes come from q4k_planes_kernel (`x` then points at its scratch; gain
-// and eps are not used): SB <= 16, so a wave has one superblock column and keeps its A
-// operands in registers; LDS holds the partial sums only.
+// and eps are not used): the workgroup's slice of the row (blockIdx.y) has at most sixteen
+// superblocks, so a wave has one superblock column and keeps its A operands in registers; LDS
+// holds the partial sums only.
 template <int NC, bool SHORT, bool PLANES = false>
 __global__ void __launch_bounds__(kMThreads)
 q4_k_mfma_gemv(const uint8_t *__restrict__ w, const float *__restrict__ x,
@@ -265,7 +290,10 @@ q4_k_mfma_gemv(const uint8_t *__restrict__ w, const float *__restrict__ x,
     const uint32_t r = lane & 15u, g = lane >> 4;
     const uint64_t row_bytes = (uint64_t)SB * 144u;
     const uint32_t ngroups = (rows + 15u) >> 4;
-    const uint32_t tpr = (SB + kMWaves - 1u) / kMWaves;    // tasks per row group and wave
+    const uint32_t slices = PLANES ? gridDim.y : 1u, per_slice = (SB + slices - 1u) / slices;
+    const uint32_t sb0 = PLANES ? blockIdx.y * per_slice : 0u;            // the slice's superblocks
+    const uint32_t nsb = PLANES ? (SB - sb0 < per_slice ? SB - sb0 : per_slice) : SB;
+    const uint32_t tpr = PLANES ? 1u : (SB + kMWaves - 1u) / kMWaves;    // tasks per row group and wave
     const uint32_t ntasks = ((ngroups - blockIdx.x + gridDim.x - 1u) / gridDim.x) * tpr;
     // A cursor walks the wave's tasks in order: row group rg (stride gridDim.x),
     // within it superblock wave + 16*t for t < tpr.  A task past the end (or
@@ -282,10 +310,10 @@ q4_k_mfma_gemv(const uint8_t *__restrict__ w, const float *__restrict__ x,
     };
     auto issue = [&](cursor &c, q4k_regs &W) {
         const uint32_t sbw = wave + kMWaves * c.t;
-        const bool real = c.k < ntasks && sbw < SB;
+        const bool real = c.k < ntasks && sbw < nsb;
         uint32_t row = c.rg * 16u + r;
         row = row < rows ? row : rows - 1u;
-        q4k_issue(w, row_bytes, real ? row : 0u, real ? sbw : 0u, real ? g : 0u, W);
+        q4k_issue(w, row_bytes, real ? row : 0u, real ? sb0 + sbw : 0u, real ? g : 0u, W);
         advance(c);
     };
     cursor ci{0u, blockIdx.x, 0u}, cc{0u, blockIdx.x, 0u};
@@ -296,7 +324,7 @@ q4_k_mfma_gemv(const uint8_t *__restrict__ w, const float *__restrict__ x,
     double pwreg[NX];        // 2^(e-151) of column 4q + g
     if constexpr (PLANES) {
         const uint8_t *scratch = reinterpret_cast<const uint8_t *>(x);
-        const uint32_t sbw = wave < SB ? wave : SB - 1u;
+        const uint32_t sbw = sb0 + (wave < nsb ? wave : nsb - 1u);
         const double *psb_g = reinterpret_cast<const double *>(scratch + q4k_planes_bytes(SB, NX));
 #pragma unroll
         for (int jp = 0; jp < 4; ++jp)
@@ -306,7 +334,7 @@ q4_k_mfma_gemv(const uint8_t *__restrict__ w, const float *__restrict__ x,
                     scratch + ((((size_t)sbw * 4u + (uint32_t)jp) * NX + (uint32_t)q) * 64u + lane) * 16u);
 #pragma unroll
         for (int q = 0; q < NX; ++q) pwreg[q] = psb_g[sbw * NL + 4u * (uint32_t)q + g];
-        if (tid < NL) s_bad[tid] = reinterpret_cast<const uint32_t *>(psb_g + (size_t)SB * NL)[tid];
+        if (tid < NL) s_bad[tid] = 0u;                       // (the powers of two carry it)
         issue(ci, W0);
         if constexpr (!SHORT) {
             issue(ci, W1);
@@ -467,6 +495,8 @@ q4_k_mfma_gemv(const uint8_t *__restrict__ w, const float *__restrict__ x,
 
     }
     // ---- stream the weights ----
+    uint32_t *count = reinterpret_cast<uint32_t *>(reinterpret_cast<uint64_t>(x) + q4k_count_at(SB, NX));
+    double *sums = reinterpret_cast<double *>(reinterpret_cast<uint64_t>(x) + q4k_sums_at(SB, NX, ngroups));
     double yacc[NX];
 #pragma unroll
     for (int q = 0; q < NX; ++q) yacc[q] = 0.0;
@@ -477,8 +507,8 @@ q4_k_mfma_gemv(const uint8_t *__restrict__ w, const float *__restrict__ x,
     auto compute = [&](cursor &c, const q4k_regs &W) {
         const uint32_t rg = c.rg, t = c.t;
         const uint32_t sbw = wave + kMWaves * t;
-        const bool live = sbw < SB;
-        const uint32_t sb = live ? sbw : SB - 1u;
+        const bool live = sbw < nsb;
+        const uint32_t sb = live ? sbw : nsb - 1u;               // (staged planes: the slice is the row)
         // unpack_scale_min, lev-cpu/src/lib.rs:64-74: the eight scales and the eight mins as bytes
         const uint32_t S0 = W.hdr.y, S1 = W.hdr.z, S2 = W.hdr.w;
         const uint32_t sc_w[2] = {S0 & 0x3F3F3F3Fu, (S2 & 0x0F0F0F0Fu) | ((S0 >> 2) & 0x30303030u)};
@@ -580,13 +610,41 @@ q4_k_mfma_gemv(const uint8_t *__restrict__ w, const float *__restrict__ x,
                 const uint32_t col = tid >> 4, rr = tid & 15u, row = rg * 16u + rr;
                 double sum = 0.0;
 #pragma unroll
-                for (int kk = 0; kk < kMWaves; ++kk) sum += pp[((uint32_t)kk * 16u + rr) * NL + col];
-                if (col < ncol && row < rows)
+                for (int kk = 0; kk < kMWaves; ++kk) {
+                    if (PLANES && (uint32_t)kk * LEV_WAVE >= blockDim.x) break;
+                    sum += pp[((uint32_t)kk * 16u + rr) * NL + col];
+                }
+                if (PLANES && slices > 1u)
+                    __hip_atomic_store(sums + (((uint64_t)blockIdx.y * ngroups + rg) * NL + col) * 16u + rr, sum,
+                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                else if (col < ncol && row < rows)
                     y[(uint64_t)col * rows + row] = s_bad[col] ? __builtin_nanf("") : (float)sum;
             }
             if (pb == 1u) lev_barrier_lds();   // the one buffer is written again by the next group
         }
         advance(c);
+    };
+    // The slices' sums of the workgroup's row groups: those it is the last to bring are added up.
+    auto merge = [&]() {
+        if (!PLANES || slices == 1u) return;
+        lev_publish_wait();
+        lev_barrier_lds();                                       // every wave's sums have reached memory
+        uint32_t *last = reinterpret_cast<uint32_t *>(part);     // one flag per row group (kMaxMerged fit)
+        const uint32_t mine = (ngroups - blockIdx.x + gridDim.x - 1u) / gridDim.x;
+        for (uint32_t i = tid; i < mine; i += blockDim.x)
+            last[i] = __hip_atomic_fetch_add(count + blockIdx.x + i * gridDim.x, 1u, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT) == slices - 1u;
+        lev_barrier_lds();
+        for (uint32_t e = tid; e < mine * 16u * NL; e += blockDim.x) {
+            const uint32_t i = e / (16u * NL), col = (e >> 4) % NL, rg = blockIdx.x + i * gridDim.x;
+            const uint32_t row = rg * 16u + (e & 15u);
+            if (!last[i] || col >= ncol || row >= rows) continue;
+            double sum = 0.0;
+            for (uint32_t sl = 0; sl < slices; ++sl)
+                sum += __hip_atomic_load(sums + (((uint64_t)sl * ngroups + rg) * NL + col) * 16u + (e & 15u),
+                                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            y[(uint64_t)col * rows + row] = s_bad[col] ? __builtin_nanf("") : (float)sum;
+        }
     };
 
     if constexpr (SHORT) {
@@ -603,6 +661,7 @@ q4_k_mfma_gemv(const uint8_t *__restrict__ w, const float *__restrict__ x,
         __builtin_amdgcn_sched_barrier(0);
         if (ntasks > 1u) compute(cc, W1);
         if (ntasks > 2u) compute(cc, W2);
+        merge();
         return;
     }
     // Three tasks in flight per wave.
@@ -626,6 +685,7 @@ q4_k_mfma_gemv(const uint8_t *__restrict__ w, const float *__restrict__ x,
         __builtin_amdgcn_sched_barrier(0);
         if (cc.k >= ntasks) break;
     }
+    merge();
 }
 
 // One or two columns: the same sums with half the matrix-core products and half the
@@ -985,6 +1045,10 @@ q4_k_mfma_gemv_narrow(const uint8_t *__restrict__ w, const float *__restrict__ x
     }
 }
 
+}  // namespace
+uint32_t lev_q4_k_mfma_cols(const lev_ctx *ctx, uint32_t in_dim);
+namespace {
+
 size_t q4k_mfma_lds_bytes(uint32_t cols, uint32_t nc, uint32_t pb) {
     return nc > 4u ? q4k_lds<2>::total(cols >> 5, pb) : q4k_lds<1>::total(cols >> 5, pb);
 }
@@ -1024,18 +1088,42 @@ hipError_t launch_mfma(lev_ctx *ctx, const uint8_t *w, const float *x, const flo
     return launch_mfma_variant<NC, false>(ctx, w, x, gain, eps, y, cols, rows, ncol);
 }
 
-// Five to eight columns of at most sixteen superblocks: the planes once per launch (q4k_planes_kernel), then the
-// products.  Returns hipErrorOutOfMemory when the scratch cannot be had (a program is being recorded and the
-// context's scratch is still too small): the caller then takes the kernel that stages for itself (same bits).
+constexpr uint32_t kMaxMerged = 4096u;   // row groups a workgroup can merge: a flag each in the LDS of the partial sums
+
+// Slices of a row, waves of a workgroup (one per superblock of its slice) and workgroups of a slice.  A CU holds sixteen
+// waves of this kernel.  Of the fewest slices possible and up to three more: the number with the shortest busiest
+// workgroup, a round of row groups counted as its waves on a CU and eight more for its latency (4096 x 12288: three
+// slices are 85 workgroups and four rounds of 16 waves, four are 64 and four rounds of 12).
+struct q4k_grid {
+    uint32_t slices, waves, blocks;
+};
+q4k_grid q4k_planes_grid(const lev_ctx *ctx, uint32_t cols, uint32_t rows) {
+    const uint32_t SB = cols >> 8, groups = (rows + 15u) / 16u, W = (uint32_t)kMWaves, cus = (uint32_t)ctx->num_cus;
+    if (SB <= W) return q4k_grid{1u, W, groups < cus ? groups : cus};
+    q4k_grid best{};
+    uint32_t best_cost = 0xFFFFFFFFu;
+    const uint32_t least = (SB + W - 1u) / W;
+    for (uint32_t sl = least; sl <= least + 3u; ++sl) {
+        const uint32_t waves = (SB + sl - 1u) / sl, per_cu = W / waves, room = cus * per_cu / sl;
+        const uint32_t blocks = groups < room ? groups : room > 0u ? room : 1u;
+        const uint32_t cost = (groups + blocks - 1u) / blocks * (waves * per_cu + 8u);
+        if (cost < best_cost) best_cost = cost, best = q4k_grid{sl, waves, blocks};
+    }
+    return best;
+}
+
+// The planes once per launch (q4k_planes_kernel), then the products.  Returns hipErrorOutOfMemory when the scratch
+// cannot be had (a program is being recorded and the context's scratch is still too small): the caller then takes
+// the kernels that stage for themselves.
 template <int NC, bool SHORT>
 hipError_t launch_planes_variant(lev_ctx *ctx, const uint8_t *w, const uint8_t *scratch, float *y, uint32_t cols,
-                                 uint32_t rows, uint32_t ncol) {
+                                 uint32_t rows, uint32_t ncol, const q4k_grid &grid) {
     constexpr uint32_t NL = NC > 4 ? 8u : 4u, pb = 2u;
-    const size_t lds = (size_t)pb * kMWaves * 16u * NL * 8u + (size_t)(cols >> 8) * NL * 8u + (size_t)NL * 12u;   // 34 KB
-    const uint32_t groups = (rows + 15u) / 16u;
-    const uint32_t blocks = groups < (uint32_t)ctx->num_cus ? groups : (uint32_t)ctx->num_cus;
-    hipLaunchKernelGGL((q4_k_mfma_gemv<NC, SHORT, true>), dim3(blocks), dim3(kMThreads), lds, ctx->stream, w,
-                       reinterpret_cast<const float *>(scratch), static_cast<const float *>(nullptr), 0.f, y, cols,
+    constexpr size_t part = (size_t)pb * kMWaves * 16u * NL * 8u;
+    static_assert(part >= kMaxMerged * 4u, "the flags of the merge lie over the partial sums");
+    const size_t lds = part + (size_t)(cols >> 8) * NL * 8u + (size_t)NL * 12u;   // 34 KB at sixteen superblocks
+    hipLaunchKernelGGL((q4_k_mfma_gemv<NC, SHORT, true>), dim3(grid.blocks, grid.slices), dim3(grid.waves * LEV_WAVE), lds,
+                       ctx->stream, w, reinterpret_cast<const float *>(scratch), static_cast<const float *>(nullptr), 0.f, y, cols,
                        rows, ncol, pb, 0.0);
     return hipGetLastError();
 }
@@ -1050,28 +1138,37 @@ uint32_t q4k_planes_min_cols() {
     return v;
 }
 
-bool q4k_planes_serves(uint32_t cols, uint32_t ncol) {
-    return ncol >= q4k_planes_min_cols() && ncol <= 8u && cols % 256u == 0u && cols != 0u && cols <= 8u * kPThreads &&
-           (cols >> 8) <= (uint32_t)kMWaves;
+// Rows of at most sixteen superblocks: from five columns on (four: staged by every workgroup 10.6 us, with the
+// planes in front 11.4, 12288 x 4096).  Wider ones: as soon as the kernel that stages for itself needs a second
+// launch (4352 x 16000, four columns: 19.4 us with it, 21.4 with the planes in front).
+bool q4k_planes_serves(const lev_ctx *ctx, uint32_t cols, uint32_t rows, uint32_t ncol) {
+    const uint32_t from = q4k_planes_min_cols();
+    if (ncol < 3u || ncol > 8u || from > 8u || cols % 256u != 0u || cols == 0u || cols > kPMaxCols) return false;
+    if (cols <= 256u * kMWaves) return ncol >= from;
+    const q4k_grid grid = q4k_planes_grid(ctx, cols, rows);
+    return (ncol >= from || ncol > lev_q4_k_mfma_cols(ctx, cols)) && (rows + 15u) / 16u <= grid.blocks * kMaxMerged;
 }
 
 hipError_t launch_planes(lev_ctx *ctx, const uint8_t *w, const float *x, const float *gain, float eps, float *y,
                          uint32_t cols, uint32_t rows, uint32_t ncol) {
     const uint32_t SB = cols >> 8, nx = ncol > 4u ? 2u : 1u;
-    uint8_t *scratch = static_cast<uint8_t *>(lev_scratch(ctx, q4k_planes_total(SB, nx)));
+    const uint32_t groups = (rows + 15u) / 16u;
+    const q4k_grid grid = q4k_planes_grid(ctx, cols, rows);
+    uint8_t *scratch = static_cast<uint8_t *>(lev_scratch(ctx, q4k_planes_total(SB, nx, groups, grid.slices)));
     if (!scratch) return hipErrorOutOfMemory;
-    hipLaunchKernelGGL(q4k_planes_kernel, dim3(ncol), dim3(kPThreads), 0, ctx->stream, x, gain, eps, scratch, cols, nx,
-                       1.0 / (double)cols);
+    const uint32_t nclear = grid.slices > 1u ? groups : 0u;
+    const uint32_t parts = (cols + 8u * kPThreads - 1u) / (8u * kPThreads);
+    auto planes = parts == 1u ? q4k_planes_kernel<1> : parts == 2u ? q4k_planes_kernel<2> : parts == 3u ? q4k_planes_kernel<3> : q4k_planes_kernel<4>;
+    hipLaunchKernelGGL(planes, dim3(ncol, parts), dim3(kPThreads), 0, ctx->stream, x, gain, eps, scratch, cols, nx,
+                       1.0 / (double)cols, nclear);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    const uint32_t groups = (rows + 15u) / 16u;
-    const uint32_t blocks = groups < (uint32_t)ctx->num_cus ? groups : (uint32_t)ctx->num_cus;
-    const bool few = (groups + blocks - 1u) / blocks <= 3u;
+    const bool few = (groups + grid.blocks - 1u) / grid.blocks <= 3u;
     if (nx == 2u)
-        return few ? launch_planes_variant<8, true>(ctx, w, scratch, y, cols, rows, ncol)
-                   : launch_planes_variant<8, false>(ctx, w, scratch, y, cols, rows, ncol);
-    return few ? launch_planes_variant<4, true>(ctx, w, scratch, y, cols, rows, ncol)
-               : launch_planes_variant<4, false>(ctx, w, scratch, y, cols, rows, ncol);
+        return few ? launch_planes_variant<8, true>(ctx, w, scratch, y, cols, rows, ncol, grid)
+                   : launch_planes_variant<8, false>(ctx, w, scratch, y, cols, rows, ncol, grid);
+    return few ? launch_planes_variant<4, true>(ctx, w, scratch, y, cols, rows, ncol, grid)
+               : launch_planes_variant<4, false>(ctx, w, scratch, y, cols, rows, ncol, grid);
 }
 
 size_t q4k_narrow_lds_bytes(uint32_t cols, uint32_t nc, uint32_t pb) {
@@ -1137,8 +1234,13 @@ bool lev_q4_k_mfma_one_usable(const uint8_t *w, const float *x, const float *gai
 hipError_t lev_q4_k_mfma_one_launch(lev_ctx *ctx, const uint8_t *w, const float *x, const float *gain, float eps,
                                     float *y, uint32_t in_dim, uint32_t rows, uint32_t ncol);
 
-// ncol <= lev_q4_k_mfma_narrow_cols(ctx, in_dim) (the narrow kernel) or
-// ncol <= lev_q4_k_mfma_cols(ctx, in_dim); w 16-byte aligned.
+// Whether up to eight columns go through planes made in front of the products.
+bool lev_q4_k_mfma_planes(const lev_ctx *ctx, uint32_t in_dim, uint32_t rows, uint32_t ncol) {
+    return q4k_planes_serves(ctx, in_dim, rows, ncol);
+}
+
+// ncol <= lev_q4_k_mfma_narrow_cols(ctx, in_dim) (the narrow kernel), ncol <= lev_q4_k_mfma_cols(ctx, in_dim) or
+// lev_q4_k_mfma_planes (which may report hipErrorOutOfMemory while recording: nothing enqueued); w 16-byte aligned.
 hipError_t lev_q4_k_mfma_gemv_launch(lev_ctx *ctx, const uint8_t *w, const float *x, const float *gain,
                                      float eps, float *y, uint32_t in_dim, uint32_t rows,
                                      uint32_t ncol) {
@@ -1155,9 +1257,9 @@ hipError_t lev_q4_k_mfma_gemv_launch(lev_ctx *ctx, const uint8_t *w, const float
         if (ncol > 1) return launch_narrow<2>(ctx, w, x, gain, eps, y, in_dim, rows, ncol);
         return launch_narrow<1>(ctx, w, x, gain, eps, y, in_dim, rows, ncol);
     }
-    if (q4k_planes_serves(in_dim, ncol)) {
+    if (q4k_planes_serves(ctx, in_dim, rows, ncol)) {
         const hipError_t e = launch_planes(ctx, w, x, gain, eps, y, in_dim, rows, ncol);
-        if (e != hipErrorOutOfMemory) return e;
+        if (e != hipErrorOutOfMemory || ncol > lev_q4_k_mfma_cols(ctx, in_dim)) return e;
     }
     if (ncol > 4) return launch_mfma<8>(ctx, w, x, gain, eps, y, in_dim, rows, ncol);
     if (ncol > 2) return launch_mfma<4>(ctx, w, x, gain, eps, y, in_dim, rows, ncol);
