@@ -2,11 +2,12 @@
 // idle:  Y[t][r] = sum_k X[t][k] W[r][k], W rounded to fp16 as the other prefill GEMMs do
 // (lev-forge/src/coopmat.rs:236-425), f32 accumulation.
 //
-// A wave owns 32 rows x up to 128 tokens of a slice of K.  It decodes its rows' weights straight into
+// A wave owns 32 rows x 32 to 128 tokens of a slice of K.  It decodes its rows' weights straight into
 // its own fp16 B fragments (lane = row l%32, half l/32; nothing of W goes through LDS) and multiplies
 // each with T token tiles.  RW waves of a workgroup own different rows of one K slice and share its X
 // steps (64 values of every token, direct global -> LDS loads, four buffers); KW groups of them take
-// different slices, and S workgroups more: the partial tiles of a workgroup meet in LDS, those of
+// different slices (eight waves: four rows of tiles in two slices, or two in four), and S workgroups more: the partial
+// tiles of a workgroup meet in LDS, those of
 // the S workgroups in scratch, and a small kernel adds them in slice order.
 //
 // 4096 rows are 128 row tiles: one wave each would leave seven eighths of the chip idle, so K is cut until the
@@ -15,8 +16,8 @@
 //
 // What bounds it: a step of a wave is some 105 vector instructions of decode and 4 T MFMAs behind LDS reads and a
 // barrier, about twice what the vector unit alone takes; 6 us of a launch are its first weights and its stores.
-// 77 tokens, 4096 rows, 12288 columns of Q6_K: 30 us (218 in 256-token tiles on 32 CUs); 20 tokens, 12288 rows,
-// 4096 columns of Q4_K: 20 us (57).
+// 77 tokens, 4096 rows, 12288 columns of Q6_K: 27 us (218 in 256-token tiles on 32 CUs); 123 tokens, 1617 rows, 4096
+// columns of Q4_K: 13.7 us (49; 17 in tiles of 128 tokens alone).
 #include "prefill_decode.hpp"
 
 #include <cmath>
@@ -27,7 +28,10 @@ typedef lev_u32x4 u32x4_a4 __attribute__((aligned(4)));   // a vector on a dword
 
 constexpr uint32_t kTile = 4096u;        // X step of 32 tokens: 32 rows of 128 bytes
 // X steps in LDS: the one in use and three on their way, or one where 160 KB hold no more
-constexpr uint32_t x_bufs(int t) { return t >= 3 ? 2u : 4u; }
+template <typename W>
+constexpr uint32_t x_bufs(int t, int rw, int kw) {
+    return t >= 3 || kw * (4u * t * kTile + rw * W::kArea) > 160u * 1024u ? 2u : 4u;
+}
 
 // The weights of a wave's 32 rows, a superblock column at a time: request() the column's bytes, touch() (the
 // wait for them), take() them as the current column, frag() its fragments; unit(): the 16-byte unit of the
@@ -172,8 +176,9 @@ struct weights_q6k {
     __device__ __forceinline__ uint32_t unit(int q) const { return 4u * lh + (uint32_t)q; }
 };
 
-// grid: 8 * ceil(row tiles / 8) * token tiles * S workgroups in one line; workgroups go to the XCDs in turn,
-// and the token tiles of a row tile follow each other on one XCD (they read the same weights).
+// grid: row tiles * token tiles * S workgroups in one line, up to a multiple of eight.  Workgroups go to the XCDs in
+// turn: each takes an eighth of the tiles, whose order has the token tiles of a row tile together (they read the same
+// weights).
 template <typename W, int T, int RW, int KW>
 __global__ void __launch_bounds__(RW *KW * 64, 2)
 gemm_split_kernel(const uint8_t *__restrict__ w, const uint16_t *__restrict__ x, float *__restrict__ out, uint32_t in_dim,
@@ -181,10 +186,9 @@ gemm_split_kernel(const uint8_t *__restrict__ w, const uint16_t *__restrict__ x,
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
     const uint32_t lr = lane & 31u, lh = lane >> 5, rw = wave % RW, kw = wave / RW;
-    const uint32_t per_split = ((row_tiles + 7u) >> 3) * tok_tiles * 8u;
-    const uint32_t z = blockIdx.x / per_split, id = blockIdx.x - z * per_split, k8 = id >> 3;
-    const uint32_t rt = (k8 / tok_tiles) * 8u + (id & 7u), tok0 = (k8 % tok_tiles) * (32u * T);
-    if (rt >= row_tiles) return;
+    const uint32_t tile = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3), zr = tile / tok_tiles;
+    const uint32_t z = zr / row_tiles, rt = zr - z * row_tiles, tok0 = (tile - zr * tok_tiles) * (32u * T);
+    if (z >= splits) return;
     const uint32_t row0 = (rt * RW + rw) * 32u, row = row0 + lr;
     const uint32_t nsb = in_dim >> 8, ns = KW * splits;
     const uint32_t sb0 = (z * KW + kw) * nsb / ns, sb1 = (z * KW + kw + 1u) * nsb / ns;
@@ -195,7 +199,7 @@ gemm_split_kernel(const uint8_t *__restrict__ w, const uint16_t *__restrict__ x,
         most = n > most ? n : most;
     }
     // X: load j brings the 128 bytes of eight tokens; 16-byte unit c of token t lies at c ^ (t & 7)
-    constexpr uint32_t kBufs = x_bufs(T);
+    constexpr uint32_t kBufs = x_bufs<W>(T, RW, KW);
     constexpr int kXLoads = 4 * T / RW;
     const uint8_t *xsrc[kXLoads];
 #pragma unroll
@@ -330,7 +334,7 @@ gemm_split_sum_kernel(const float *__restrict__ part, float *__restrict__ y, uin
 template <typename W, int T, int RW, int KW>
 hipError_t launch_as(lev_ctx *ctx, const uint8_t *w, const uint16_t *x, float *out, uint32_t in_dim, uint32_t rows,
                      uint32_t tokens, uint32_t tok_tiles, uint32_t splits) {
-    constexpr size_t lds = (size_t)KW * x_bufs(T) * T * kTile + RW * KW * W::kArea;
+    constexpr size_t lds = (size_t)KW * x_bufs<W>(T, RW, KW) * T * kTile + RW * KW * W::kArea;
     static bool configured = false;
     if (!configured && lds > 48 * 1024) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_split_kernel<W, T, RW, KW>),
@@ -339,7 +343,7 @@ hipError_t launch_as(lev_ctx *ctx, const uint8_t *w, const uint16_t *x, float *o
         configured = true;
     }
     const uint32_t row_tiles = (rows + RW * 32u - 1u) / (RW * 32u);
-    hipLaunchKernelGGL((gemm_split_kernel<W, T, RW, KW>), dim3(((row_tiles + 7u) / 8u) * 8u * tok_tiles * splits),
+    hipLaunchKernelGGL((gemm_split_kernel<W, T, RW, KW>), dim3((row_tiles * tok_tiles * splits + 7u) / 8u * 8u),
                        dim3(RW * KW * 64), lds, ctx->stream, w, x, out, in_dim, rows, tokens, row_tiles, tok_tiles, splits);
     return hipGetLastError();
 }
@@ -357,7 +361,12 @@ hipError_t launch_tiles(lev_ctx *ctx, const uint8_t *w, const uint16_t *x, float
             part = y;
         }
     }
-    hipError_t e = launch_as<W, T, 4, 2>(ctx, w, x, part, in_dim, rows, tokens, tok_tiles, splits);
+    hipError_t e;
+    if constexpr (4u * (x_bufs<W>(T, 2, 4) * T * kTile + 2u * W::kArea) <= 160u * 1024u)
+        e = plan.kw == 4u ? launch_as<W, T, 2, 4>(ctx, w, x, part, in_dim, rows, tokens, tok_tiles, splits)
+                          : launch_as<W, T, 4, 2>(ctx, w, x, part, in_dim, rows, tokens, tok_tiles, splits);
+    else
+        e = launch_as<W, T, 4, 2>(ctx, w, x, part, in_dim, rows, tokens, tok_tiles, splits);
     if (e != hipSuccess || splits == 1u) return e;
     const uint64_t n = (uint64_t)tokens * rows;
     if (n % 4u == 0u && (reinterpret_cast<uintptr_t>(y) & 15u) == 0u)
@@ -369,18 +378,11 @@ hipError_t launch_tiles(lev_ctx *ctx, const uint8_t *w, const uint16_t *x, float
     return hipGetLastError();
 }
 
-// token tiles of equal height, at most four times 32
-uint32_t tok_tiles_of(uint32_t tokens) { return (tokens + 127u) / 128u; }
-uint32_t tile_of(uint32_t tokens) {
-    const uint32_t n = tok_tiles_of(tokens);
-    return ((tokens + n - 1u) / n + 31u) / 32u;
-}
-
 template <typename W>
 hipError_t launch(lev_ctx *ctx, const uint8_t *w, const uint16_t *x, float *y, uint32_t in_dim, uint32_t rows,
                   uint32_t tokens, const lev_gemm_split_plan &plan) {
-    const uint32_t n = tok_tiles_of(tokens);
-    switch (tile_of(tokens)) {
+    const uint32_t n = (tokens + 32u * plan.t - 1u) / (32u * plan.t);
+    switch (plan.t) {
     case 1u: return launch_tiles<W, 1>(ctx, w, x, y, in_dim, rows, tokens, n, plan);
     case 2u: return launch_tiles<W, 2>(ctx, w, x, y, in_dim, rows, tokens, n, plan);
     case 3u: return launch_tiles<W, 3>(ctx, w, x, y, in_dim, rows, tokens, n, plan);
@@ -390,43 +392,62 @@ hipError_t launch(lev_ctx *ctx, const uint8_t *w, const uint16_t *x, float *y, u
 
 }  // namespace
 
-// Which of the GEMMs takes a shape, and in how many K slices: the least of what each would take, from times
-// measured over 1500 to 32000 rows, 1024 to 12288 columns and 17 to 1000 tokens (us; a step is 64 values of K,
-// t = 32-token tiles a wave).
-//   256-token tiles:  a round of workgroups (one per CU) 3 + in_dim / 1024 * (11.3 + 3.5 * share of the CUs it
-//                     fills), Q6_K 17.4 + 4.4 *: 51 to 62 us at 4096 columns of Q4_K, whatever the tokens;
-//   KW = 1:           5 + steps * (0.32 + 0.058 t), Q6_K 0.42 + 0.05 t, twice that (2.2 times) with two workgroups on a CU;
-//   KW = 2, S splits: rounds of one per CU, 5 + steps * (0.45 + 0.14 t), Q6_K 0.62 + 0.11 t, and up to three tenths of that
-//                     more as the chip fills; with S > 1 another 6 for
-//                     the kernel that adds, and the partial sums at 4 TB/s.
+// Which of the GEMMs takes a shape, in how many K slices and token tiles of which height: the least of what each would
+// take, from times measured over 1000 to 32000 rows, 1024 to 12288 columns and 17 to 1000 tokens (us; a step is 64 values
+// of K, t = 32-token tiles a wave; of 60 shapes the choice was within 0.2 % of the best on average, 5 % at worst).
+//   256-token tiles:  a round of workgroups (one per CU) 6.1 + in_dim / 1024 * (9.8 + 3.8 * share of the CUs it
+//                     fills), Q6_K 5.7 + in_dim / 1024 * (19.2 + 3.5 *): 46 to 60 us at 4096 columns of Q4_K;
+//   KW = 1:           a round of up to two workgroups a CU; their steps take 1.6 times those of one alone;
+//   KW = 2, KW = 4:   a round of one a CU, and with S > 1 splits the kernel that adds and its reads and writes.
+// Lower token tiles are more workgroups that decode the same weights: what fills the chip where rows alone do not.
 // Tall matrices (768 row tiles and more) and rows of fewer than six superblocks are never cut along K, so that
 // there every kernel adds in the same order.
 lev_gemm_split_plan lev_gemm_split_choose(const lev_ctx *ctx, bool q6, uint32_t in_dim, uint32_t rows, uint32_t tokens,
                                           uint32_t big_rows) {
-    const double cus = ctx->num_cus, t = tile_of(tokens), nsb = in_dim / 256u;
+    const double cus = ctx->num_cus;
+    const uint32_t nsb = in_dim / 256u, tiles = (tokens + 31u) / 32u;
     const double big_wgs = (double)((rows + big_rows - 1u) / big_rows) * ((tokens + 255u) / 256u);
     const double big_rounds = std::ceil(big_wgs / cus), fill = big_wgs / (big_rounds * cus);
-    lev_gemm_split_plan best{0u, 1u};
-    double least = big_rounds * (3.0 + in_dim / 1024.0 * (q6 ? 17.4 + 4.4 * fill : 11.3 + 3.5 * fill));
-    auto offer = [&](double us, uint32_t kw, uint32_t splits) {
+    lev_gemm_split_plan best{0u, 1u, 1u};
+    double least = big_rounds * (q6 ? 5.7 + in_dim / 1024.0 * (19.2 + 3.5 * fill) : 6.1 + in_dim / 1024.0 * (9.8 + 3.8 * fill));
+    struct cost { double start, step, per_tile, full, sum, sum_mb; };
+    const cost k1 = q6 ? cost{4.9, 0.383, 0.067, 0.60, 0, 0} : cost{4.0, 0.267, 0.076, 0.66, 0, 0};
+    const cost k2 = q6 ? cost{4.3, 0.558, 0.145, 0.16, 3.1, 0.7} : cost{3.9, 0.363, 0.165, 0.08, 2.9, 0.75};
+    const cost k4 = q6 ? cost{4.1, 0.534, 0.248, 0.02, 4.8, 0.0} : cost{4.6, 0.206, 0.287, 0.05, 3.1, 0.56};
+    auto offer = [&](double us, uint32_t kw, uint32_t splits, uint32_t t) {
         if (us < least) {
             least = us;
-            best = lev_gemm_split_plan{kw, splits};
+            best = lev_gemm_split_plan{kw, splits, t};
         }
     };
-    const double wgs = (double)((rows + 127u) / 128u) * tok_tiles_of(tokens);
-    const double c1 = q6 ? 0.42 + 0.05 * t : 0.32 + 0.058 * t, c2 = q6 ? 0.62 + 0.11 * t : 0.45 + 0.14 * t;
-    offer(std::ceil(wgs / (2.0 * cus)) * (5.0 + 4.0 * nsb * c1 * (wgs > cus ? (q6 ? 2.2 : 2.0) : 1.0)), 1u, 1u);
-    if ((rows + 31u) / 32u >= 768u || nsb < 6.0) return best;
-    for (uint32_t s = 1; s <= 8u && s * 2u <= nsb; ++s) {
-        const double rounds = std::ceil(wgs * s / cus), full = wgs * s / (rounds * cus);
-        offer(rounds * (5.0 + 2.0 * nsb / s * c2 * (1.0 + 0.3 * full)) * (rounds > 1.0 ? 1.05 : 1.0) + (s > 1u ? 6.0 + 8e-6 * s * tokens * rows / 4.0 : 0.0), 2u, s);
+    for (uint32_t t = 1; t <= 4u && t <= tiles; ++t) {
+        const double tok_tiles = (tiles + t - 1u) / t;
+        // workgroups, whole eighths of them on an XCD each
+        auto wgs_of = [&](uint32_t rows_wg, uint32_t splits) { return 8.0 * std::ceil((rows + rows_wg - 1u) / rows_wg * tok_tiles * splits / 8.0); };
+        {
+            const double n = wgs_of(128u, 1u), whole = std::floor(n / (2.0 * cus)), rest = n - whole * 2.0 * cus;
+            const double rounds = whole + (rest > 0.0 ? 1.0 : 0.0), pairs = whole + (rest > cus ? 1.0 : 0.0);
+            offer(rounds * k1.start + 4.0 * nsb * (k1.step + k1.per_tile * t) * (rounds + k1.full * pairs), 1u, 1u, t);
+        }
+        if ((rows + 31u) / 32u >= 768u || nsb < 6u) continue;
+        for (uint32_t kw = 2; kw <= 4u; kw += 2u) {
+            if (kw == 4u && q6 && t == 4u) continue;   // (more LDS than there is)
+            const cost &k = kw == 2u ? k2 : k4;
+            for (uint32_t s = 1; s <= 8u && s * kw <= nsb; ++s) {
+                const double n = wgs_of(kw == 2u ? 128u : 64u, s), rounds = std::ceil(n / cus), full = n / (rounds * cus);
+                const double steps = 4.0 * ((nsb + kw * s - 1u) / (kw * s));
+                offer(rounds * (k.start + steps * (k.step + k.per_tile * t) * (1.0 + k.full * full)) +
+                          (s > 1u ? k.sum + k.sum_mb * 1e-6 * (s + 1.0) * tokens * rows : 0.0), kw, s, t);
+            }
+        }
     }
     return best;
 }
 
 hipError_t lev_gemm_split_launch(lev_ctx *ctx, bool q6, const uint8_t *w, const uint16_t *x, float *y, uint32_t in_dim,
                                  uint32_t rows, uint32_t tokens, const lev_gemm_split_plan &plan) {
+    // every slice has a superblock at least: a wave without one would step below its first
+    if (plan.kw == 0u || plan.splits == 0u || plan.kw * plan.splits > in_dim / 256u) return hipErrorInvalidValue;
     return q6 ? launch<weights_q6k>(ctx, w, x, y, in_dim, rows, tokens, plan)
               : launch<weights_q4k>(ctx, w, x, y, in_dim, rows, tokens, plan);
 }

@@ -81,7 +81,7 @@ __device__ __forceinline__ void q6g_put4_mix(uint32_t c, float ds, float nbm, f1
 // The GEMM for short prompts and for shapes whose 256-token tiles leave the chip idle (gemm_split.hip):
 // kw = 0: the 256-token kernel takes the shape (`big_rows` rows a workgroup); else K slices a workgroup, and
 // workgroups that share a tile.
-struct lev_gemm_split_plan { uint32_t kw, splits; };
+struct lev_gemm_split_plan { uint32_t kw, splits, t; };
 lev_gemm_split_plan lev_gemm_split_choose(const lev_ctx *ctx, bool q6, uint32_t in_dim, uint32_t rows, uint32_t tokens,
                                           uint32_t big_rows);
 hipError_t lev_gemm_split_launch(lev_ctx *ctx, bool q6, const uint8_t *w, const uint16_t *x, float *y, uint32_t in_dim,

@@ -19,6 +19,7 @@ pytestmark = pytest.mark.gpu
     (160, 2816, 96), (257, 1536, 97),
     (700, 3328, 128), (96, 4096, 129),
     (400, 2304, 400),       # four token tiles
+    (1130, 4864, 643),      # four slices of tiles of 96 tokens: the most LDS a workgroup of either format takes
 ])
 def test_gemm_split_edges(ctx, kind, rows, cols, tokens):
     if kind == "q4_k":
