@@ -48,7 +48,10 @@ struct lev_ctx {
     // words kArgmaxTicketWord + 1024*k, k = 0..8: arrival counters of the greedy-token merge
     // (4 KB apart: counters that share a cache line serialise in one L2 channel), zero between launches;
     // words kArgmaxTicketWord + 512 + 16*c: those of the columns of the argmax operator
-    static constexpr uint32_t kFlagWords = 10 * 1024, kTicketWord = 16, kArgmaxTicketWord = 1024;
+    // words kSliceTicketWord + kSliceTicketStep*i, i < kSliceTickets: arrival counters of the workgroups that share
+    // the row groups i of a matrix whose rows are cut into slices, zero between launches
+    static constexpr uint32_t kSliceTickets = 256, kSliceTicketStep = 16, kSliceTicketWord = 10 * 1024;
+    static constexpr uint32_t kFlagWords = kSliceTicketWord + kSliceTickets * kSliceTicketStep, kTicketWord = 16, kArgmaxTicketWord = 1024;
     int *h_flag = nullptr;   // pinned
     // True between lev_hip_program_begin and lev_hip_program_end: the stream
     // is being captured, so nothing may allocate or synchronise.

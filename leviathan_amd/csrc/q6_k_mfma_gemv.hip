@@ -1085,36 +1085,45 @@ q6_k_mfma_gemv_q8(const uint8_t *__restrict__ w, const uint32_t *__restrict__ xq
 }
 
 // ---------------------------------------------------------------------------
-// Int8 activations, up to eight columns, rows of at most sixteen superblocks: a wave per
-// superblock COLUMN of the matrix, as q6_k_mfma_gemv_one.  The A operands are the activation
+// Int8 activations, a wave per superblock COLUMN of the matrix, as q6_k_mfma_gemv_one.  The A operands are the activation
 // codes as they lie in memory (16 consecutive codes of one column), so a lane loads the ones of
 // its wave's superblock straight into registers, with the quarter activation scales of its
 // blocks beside them: nothing is staged in LDS but the turn-round of the weights and the
 // partial sums of a round.
-// LDS: part [2][16 waves][16 rows][NC] f32 | per wave: the turn-round area.
+// SLICED: a row of more superblocks than the workgroup has waves is cut into gridDim.y slices of wpr,
+// a workgroup taking one for its row groups.  The slices' sums meet in scratch, and the last of the
+// workgroups that share a blockIdx.x to finish adds them up, in the order of the slices (lev_publish_wait).
+// Staged in LDS as a whole (q6_k_mfma_gemv_q8) such rows leave room for four columns at 12288, and the
+// weights are read again for every four: 4096 x 12288 by one, five and
+// sixteen columns 15.0, 27.5 and 53.8 us with it, 13.5, 15.6 and 28.5 here.
+// LDS: part [2][MAXW waves][16 rows][NC] f32 | per wave: the turn-round area.
 // ---------------------------------------------------------------------------
-__host__ __device__ constexpr uint32_t q6m_q8_one_part_bytes(uint32_t nc) { return 2u * kQWaves * 16u * 4u * nc; }
-__host__ __device__ constexpr size_t q6m_q8_one_lds(uint32_t nc) {
-    return q6m_q8_one_part_bytes(nc) + (size_t)kQWaves * kQAreaBytes;
+__host__ __device__ constexpr uint32_t q6m_q8_one_part_bytes(uint32_t nc, uint32_t waves) { return 2u * waves * 16u * 4u * nc; }
+__host__ __device__ constexpr size_t q6m_q8_one_lds(uint32_t nc, uint32_t waves) {
+    return q6m_q8_one_part_bytes(nc, waves) + (size_t)waves * kQAreaBytes;
 }
+// Waves of a workgroup: the operands of sixteen columns take the registers of sixteen waves.
+constexpr int q6m_q8_one_waves(int nc) { return nc > 8 ? 8 : kQWaves; }
 
-// NC: columns staged (4 or 8; >= ncol).
-template <int NC>
-__global__ void __launch_bounds__(kQThreads)
+// NC: columns held (4, 8 or 16; >= ncol).
+template <int NC, bool SLICED>
+__global__ void __launch_bounds__(q6m_q8_one_waves(NC) * LEV_WAVE)
 q6_k_mfma_gemv_q8_one(const uint8_t *__restrict__ w, const uint32_t *__restrict__ xq, const float *__restrict__ xs,
                       float *__restrict__ y, uint32_t cols, uint32_t rows, uint32_t ncol, uint32_t wpr, uint32_t slots,
-                      uint64_t slot_of_wave, uint64_t pos_of_wave) {
-    constexpr int NCH = NC / 4;
-    constexpr uint32_t kPart = q6m_q8_one_part_bytes(NC);
+                      uint64_t slot_of_wave, uint64_t pos_of_wave, float *__restrict__ sums, uint32_t *__restrict__ tickets) {
+    constexpr int NCH = NC / 4, WAVES = q6m_q8_one_waves(NC);
+    constexpr uint32_t kPart = q6m_q8_one_part_bytes(NC, WAVES);
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
     const uint32_t slot = (uint32_t)(slot_of_wave >> (4u * wave)) & 15u;   // idle waves: slot >= slots
-    const uint32_t sb = (uint32_t)(pos_of_wave >> (4u * wave)) & 15u;      // the wave's superblock column
     const uint32_t SB = cols >> 8, nblk = cols >> 5;
+    const uint32_t pos = (uint32_t)(pos_of_wave >> (4u * wave)) & 15u;
+    const uint32_t sbw = SLICED ? blockIdx.y * wpr + pos : pos;
+    const uint32_t sb = sbw < SB ? sbw : SB - 1u;                          // the wave's superblock column
     const uint32_t r = lane & 15u, q = lane >> 4;
     const uint32_t hf = q >> 1, jb = q & 1u;
-    const bool active = slot < slots;
+    const bool active = slot < slots && sbw < SB;
 
     // the wave's activations first: lane (r, g) feeds A row r = 4*gs + c, i.e. column 4*ch + r%4,
     // the 16 codes of weight group 16*sb + 8*hf + 2*jb (+ 4*nb + lh), when gs == g, zeros
@@ -1145,7 +1154,7 @@ q6_k_mfma_gemv_q8_one(const uint8_t *__restrict__ w, const uint32_t *__restrict_
     const uint32_t alt = q6m_alt(SB, rows);
     const int32_t poff = q6m_piece_offset(lane, q6m_odd(sb, lane >> 4, alt));
     auto issue = [&](uint32_t round_block, q6m_regs &W) {
-        uint32_t rg = round_block * slots + (active ? slot : 0u);
+        uint32_t rg = round_block * slots + (slot < slots ? slot : 0u);
         rg = rg < ngroups ? rg : ngroups - 1u;
         q6m_issue(w, row_bytes, rg * 16u, rows, alt, sb, lane, poff, W);
     };
@@ -1160,7 +1169,8 @@ q6_k_mfma_gemv_q8_one(const uint8_t *__restrict__ w, const uint32_t *__restrict_
     const uint32_t orow_step = gridDim.x * slots * 16u;
     const bool writer = wave < slots;
     uint32_t stores = writer && orow < rows ? 1u : 0u;
-    uint64_t yp = reinterpret_cast<uint64_t>(y + (uint64_t)q * rows + orow);
+    float *out = SLICED ? sums + (uint64_t)blockIdx.y * ncol * rows : y;
+    uint64_t yp = reinterpret_cast<uint64_t>(out + (uint64_t)q * rows + orow);
     lev_pin(pw);
     lev_pin(pr);
     lev_pin(stores);
@@ -1210,17 +1220,22 @@ q6_k_mfma_gemv_q8_one(const uint8_t *__restrict__ w, const uint32_t *__restrict_
                 // the slot's waves in order, four chains added at the end (sixteen reads in flight)
                 float s4[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int k = 0; k < kQWaves; ++k) {
+                for (int k = 0; k < WAVES; ++k) {
                     const float pk = pp[k * 16 * NC + 4 * ch];
                     s4[k & 3] += (uint32_t)k < wpr ? pk : 0.f;
                 }
                 const float s = (s4[0] + s4[1]) + (s4[2] + s4[3]);
-                if (stores && 4u * (uint32_t)ch + q < ncol)
-                    *reinterpret_cast<__attribute__((address_space(1))) float *>(yp + (uint64_t)(4 * ch) * rows * 4u) = s;
+                if (stores && 4u * (uint32_t)ch + q < ncol) {
+                    if (SLICED)
+                        __hip_atomic_store(reinterpret_cast<float *>(yp + (uint64_t)(4 * ch) * rows * 4u), s, __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_AGENT);
+                    else
+                        *reinterpret_cast<__attribute__((address_space(1))) float *>(yp + (uint64_t)(4 * ch) * rows * 4u) = s;
+                }
             }
         }
-        pw ^= kQWaves * 16u * 4u * NC;                         // the other half of `part` next round
-        pr ^= kQWaves * 16u * 4u * NC;
+        pw ^= WAVES * 16u * 4u * NC;                         // the other half of `part` next round
+        pr ^= WAVES * 16u * 4u * NC;
         orow += orow_step;
         yp += (uint64_t)orow_step * 4u;
         stores = writer && orow < rows ? 1u : 0u;
@@ -1242,6 +1257,28 @@ q6_k_mfma_gemv_q8_one(const uint8_t *__restrict__ w, const uint32_t *__restrict_
         finish(Wb);
         if (next >= nrounds) break;
         rb = next;
+    }
+    if (!SLICED) return;
+    lev_publish_wait();
+    lev_barrier_lds();                                           // every wave's sums have reached memory
+    uint32_t *last = reinterpret_cast<uint32_t *>(smem);
+    if (tid == 0u) {
+        uint32_t *ticket = tickets + blockIdx.x * lev_ctx::kSliceTicketStep;
+        *last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.y - 1u;
+        if (*last) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    lev_barrier_lds();
+    if (!*last) return;
+    const uint32_t per_round = slots * 16u, mine = (nrounds - blockIdx.x + gridDim.x - 1u) / gridDim.x;
+    for (uint32_t e = tid; e < mine * per_round * ncol; e += blockDim.x) {
+        const uint32_t rr = e % per_round, c = e / per_round % ncol, i = e / (per_round * ncol);
+        const uint32_t row = (blockIdx.x + i * gridDim.x) * per_round + rr;
+        if (row >= rows) continue;
+        const float *p = sums + (uint64_t)c * rows + row;
+        float sum = 0.f;
+        for (uint32_t sl = 0; sl < gridDim.y; ++sl)
+            sum += __hip_atomic_load(p + (uint64_t)sl * ncol * rows, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        y[(uint64_t)c * rows + row] = sum;
     }
 }
 
@@ -1433,43 +1470,88 @@ uint32_t lev_q6_k_mfma_q8_cols(const lev_ctx *ctx, uint32_t in_dim) {
 }
 
 namespace {
-template <int NC>
-hipError_t q6m_q8_one_launch(lev_ctx *ctx, const uint8_t *w, const uint32_t *xq, const float *xs, float *y,
-                             uint32_t cols, uint32_t rows, uint32_t ncol) {
-    const uint32_t wpr = cols >> 8, slots = (uint32_t)kQWaves / wpr;
-    const uint32_t ngroups = (rows + 15u) / 16u;
-    const uint32_t nrounds = (ngroups + slots - 1u) / slots;
+// Slices of a row and superblocks of one: of the fewest slices whose superblocks a workgroup's waves can take and
+// up to four more, the number whose busiest workgroup is done first, a round of row groups counted as its waves and
+// eight more for its latency (4096 x 12288: three slices of sixteen are 85 workgroups each and four rounds, four of
+// twelve are 64 and four shorter rounds).
+struct q6m_slices {
+    uint32_t slices, wpr, slots, blocks;
+};
+q6m_slices q6m_q8_one_grid(const lev_ctx *ctx, uint32_t cols, uint32_t rows, uint32_t waves) {
+    const uint32_t SB = cols >> 8, ngroups = (rows + 15u) / 16u, cus = (uint32_t)ctx->num_cus;
+    q6m_slices best{};
+    uint32_t best_cost = 0xFFFFFFFFu;
+    const uint32_t least = (SB + waves - 1u) / waves;
+    for (uint32_t sl = least; sl <= (least > 1u ? least + 4u : 1u) && sl <= SB; ++sl) {
+        const uint32_t wpr = (SB + sl - 1u) / sl, slots = waves / wpr, nrounds = (ngroups + slots - 1u) / slots;
+        if ((sl - 1u) * wpr >= SB) continue;      // a slice would be empty
+        uint32_t room = cus / sl;
+        room = room < 1u ? 1u : room > lev_ctx::kSliceTickets ? lev_ctx::kSliceTickets : room;
+        const uint32_t blocks = nrounds < room ? nrounds : room;
+        const uint32_t cost = (nrounds + blocks - 1u) / blocks * (wpr * slots + 8u);
+        if (cost < best_cost) best_cost = cost, best = q6m_slices{sl, wpr, slots, blocks};
+    }
+    return best;
+}
+
+// hipErrorOutOfMemory: the scratch cannot be had (a program is being recorded and the context's is still too small).
+template <int NC, bool SLICED>
+hipError_t q6m_q8_one_launch_grid(lev_ctx *ctx, const uint8_t *w, const uint32_t *xq, const float *xs, float *y,
+                                  uint32_t cols, uint32_t rows, uint32_t ncol, const q6m_slices &g) {
     uint64_t slot_of_wave, pos_of_wave;
-    lev_wave_tables(wpr, &slot_of_wave, &pos_of_wave);
-    constexpr size_t lds = q6m_q8_one_lds(NC);
+    lev_wave_tables(g.wpr, &slot_of_wave, &pos_of_wave);
+    constexpr size_t lds = q6m_q8_one_lds(NC, q6m_q8_one_waves(NC));
     static bool configured = false;   // per instantiation: raise the dynamic LDS limit once
     if (!configured) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&q6_k_mfma_gemv_q8_one<NC>),
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&q6_k_mfma_gemv_q8_one<NC, SLICED>),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
         configured = true;
     }
-    const uint32_t blocks = nrounds < (uint32_t)ctx->num_cus ? nrounds : (uint32_t)ctx->num_cus;
-    hipLaunchKernelGGL((q6_k_mfma_gemv_q8_one<NC>), dim3(blocks), dim3(slots * wpr * LEV_WAVE), lds, ctx->stream, w, xq, xs, y,
-                       cols, rows, ncol, wpr, slots, slot_of_wave, pos_of_wave);
+    float *sums = nullptr;
+    if (SLICED) {
+        sums = static_cast<float *>(lev_scratch(ctx, (size_t)g.slices * ncol * rows * 4u));
+        if (!sums) return hipErrorOutOfMemory;
+    }
+    hipLaunchKernelGGL((q6_k_mfma_gemv_q8_one<NC, SLICED>), dim3(g.blocks, g.slices), dim3(g.slots * g.wpr * LEV_WAVE), lds,
+                       ctx->stream, w, xq, xs, y, cols, rows, ncol, g.wpr, g.slots, slot_of_wave, pos_of_wave, sums,
+                       reinterpret_cast<uint32_t *>(ctx->d_flag) + lev_ctx::kSliceTicketWord);
     return hipGetLastError();
 }
-}  // namespace
 
-// ncol <= lev_q6_k_mfma_q8_cols(ctx, in_dim); w 2-byte, xq 16-byte, xs 8-byte aligned.
-hipError_t lev_q6_k_mfma_gemv_q8_launch(lev_ctx *ctx, const uint8_t *w, const uint32_t *xq, const float *xs,
-                                        float *y, uint32_t in_dim, uint32_t rows, uint32_t ncol, uint32_t waves) {
-    if (waves != 2u && waves != 4u && waves != 8u && waves != 16u) waves = 0u;
-    // up to eight columns of at most sixteen superblocks, no number of waves per row group asked
-    // for: a wave per superblock column
-    static const bool one_off = [] {
+template <int NC>
+hipError_t q6m_q8_one_launch(lev_ctx *ctx, const uint8_t *w, const uint32_t *xq, const float *xs, float *y,
+                             uint32_t cols, uint32_t rows, uint32_t ncol) {
+    const q6m_slices g = q6m_q8_one_grid(ctx, cols, rows, (uint32_t)q6m_q8_one_waves(NC));
+    if (g.slices > 1u) return q6m_q8_one_launch_grid<NC, true>(ctx, w, xq, xs, y, cols, rows, ncol, g);
+    return q6m_q8_one_launch_grid<NC, false>(ctx, w, xq, xs, y, cols, rows, ncol, g);
+}
+
+// LEV_Q6K_ONE=0: the kernel that stages the activations everywhere, for comparison
+bool q6m_q8_one_off() {
+    static const bool off = [] {
         const char *e = getenv("LEV_Q6K_ONE");
         return e && e[0] == '0';
     }();
-    if (ncol <= 8u && waves == 0u && !one_off && in_dim <= 4096u) {
-        if (ncol > 4u) return q6m_q8_one_launch<8>(ctx, w, xq, xs, y, in_dim, rows, ncol);
-        return q6m_q8_one_launch<4>(ctx, w, xq, xs, y, in_dim, rows, ncol);
-    }
+    return off;
+}
+}  // namespace
+
+// All columns (at most sixteen) in one pass over the weights, a wave per superblock column; w 2-byte, xq 16-byte, xs
+// 8-byte aligned.  hipErrorNotSupported: the shape is the staging kernel's (lev_q6_k_mfma_gemv_q8_launch);
+// hipErrorOutOfMemory: the scratch cannot be had.
+hipError_t lev_q6_k_mfma_gemv_q8_one_pass(lev_ctx *ctx, const uint8_t *w, const uint32_t *xq, const float *xs,
+                                          float *y, uint32_t in_dim, uint32_t rows, uint32_t ncol) {
+    if (q6m_q8_one_off()) return hipErrorNotSupported;
+    if (ncol > 8u) return q6m_q8_one_launch<16>(ctx, w, xq, xs, y, in_dim, rows, ncol);
+    if (ncol > 4u) return q6m_q8_one_launch<8>(ctx, w, xq, xs, y, in_dim, rows, ncol);
+    return q6m_q8_one_launch<4>(ctx, w, xq, xs, y, in_dim, rows, ncol);
+}
+
+// The kernel that stages the activations.  ncol <= lev_q6_k_mfma_q8_cols(ctx, in_dim); alignment as above.
+hipError_t lev_q6_k_mfma_gemv_q8_launch(lev_ctx *ctx, const uint8_t *w, const uint32_t *xq, const float *xs,
+                                        float *y, uint32_t in_dim, uint32_t rows, uint32_t ncol, uint32_t waves) {
+    if (waves != 2u && waves != 4u && waves != 8u && waves != 16u) waves = 0u;
     if (ncol > 8) return q6m_q8_launch<16>(ctx, w, xq, xs, y, in_dim, rows, ncol, waves);
     if (ncol > 4) return q6m_q8_launch<8>(ctx, w, xq, xs, y, in_dim, rows, ncol, waves);
     return q6m_q8_launch<4>(ctx, w, xq, xs, y, in_dim, rows, ncol, waves);

@@ -1087,6 +1087,8 @@ static uint32_t q6_q8_cols_per_pass(const lev_ctx *ctx, uint32_t in_dim, uint32_
 }
 
 uint32_t lev_q6_k_mfma_q8_cols(const lev_ctx *ctx, uint32_t in_dim);
+hipError_t lev_q6_k_mfma_gemv_q8_one_pass(lev_ctx *ctx, const uint8_t *w, const uint32_t *xq, const float *xs,
+                                          float *y, uint32_t in_dim, uint32_t rows, uint32_t ncol);
 hipError_t lev_q6_k_mfma_gemv_q8_launch(lev_ctx *ctx, const uint8_t *w, const uint32_t *xq, const float *xs,
                                         float *y, uint32_t in_dim, uint32_t rows, uint32_t ncol, uint32_t waves);
 
@@ -1136,6 +1138,8 @@ extern "C" int lev_hip_q6_k_gemv_q8(lev_ctx *ctx, const void *d_w, size_t w_byte
     const lev_schedule *sel = lev_selected(ctx, LEV_OP_Q6_K_GEMV_Q8, in_dim, rows, ncol);
     const uint32_t mcols = lev_q6_k_mfma_q8_cols(ctx, in_dim);
     if (mcols && (!sel || sel->family == 1u)) {
+        hipError_t one = lev_q6_k_mfma_gemv_q8_one_pass(ctx, w, xq, d_xs, d_y, in_dim, rows, ncol);
+        if (one != hipErrorNotSupported && one != hipErrorOutOfMemory) return lev_hip_check(ctx, one, "q6_k_gemv_q8 launch");
         // the integer matrix-core kernel: up to mcols columns per pass over the weights
         for (uint32_t done = 0; done < ncol; done += mcols) {
             const uint32_t nc = ncol - done < mcols ? ncol - done : mcols;
