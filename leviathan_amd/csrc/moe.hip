@@ -425,56 +425,63 @@ __device__ __forceinline__ float router_weight(const router_sel &r, const float 
     return wgt;
 }
 
-// Router scores, f64 accumulation rounded to f32 once.  Workgroup (e, g) owns
-// router row e.
-//   split = 1 (up to four tokens, gridDim.y = 1): the waves share the row, a
-//     part of the columns each, for every token, and meet in LDS.
-//   split = 0: wave w of group g scores the four tokens 4*(4g+w).. against the
-//     row, which it reads once for the four.
+// Router scores of few tokens, f64 accumulation rounded to f32 once: a workgroup per expert and token, whose waves
+// share the row and meet in LDS.  A launch is one trip to memory, so a thread's four pieces of both operands are
+// requested together (rows of up to 4096 columns; longer ones repeat that).  The router comes from L2 for all tokens
+// but the first: at 2816 columns and 128 experts five tokens take 20 us with a row read once for four tokens by one
+// wave, 4.5 us this way.
+__global__ void __launch_bounds__(256)
+moe_scores_few_kernel(const float *__restrict__ wr, const float *__restrict__ x, float *__restrict__ scores, uint32_t hidden,
+                      uint32_t experts) {
+    __shared__ double partial[4];
+    const uint32_t e = blockIdx.x, t = blockIdx.y, tid = threadIdx.x;
+    const float *row = wr + (uint64_t)e * hidden, *xv = x + (uint64_t)t * hidden;
+    double acc;
+    if ((hidden & 3u) == 0u && ((reinterpret_cast<uintptr_t>(wr) | reinterpret_cast<uintptr_t>(x)) & 15u) == 0u) {
+        const lev_f32x4 *r4 = reinterpret_cast<const lev_f32x4 *>(row), *x4 = reinterpret_cast<const lev_f32x4 *>(xv);
+        const uint32_t n4 = hidden >> 2;
+        double a0 = 0.0, a1 = 0.0;
+        for (uint32_t i0 = tid; i0 < n4; i0 += 1024u) {
+            lev_f32x4 a[4], b[4];
+#pragma unroll
+            for (uint32_t k = 0; k < 4u; ++k) {
+                const uint32_t i = i0 + 256u * k < n4 ? i0 + 256u * k : i0;
+                a[k] = r4[i];
+                b[k] = x4[i];
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < 4u; ++k) {
+                if (i0 + 256u * k >= n4) b[k] = lev_f32x4{0.f, 0.f, 0.f, 0.f}, a[k] = b[k];
+                a0 = fma((double)a[k].x, (double)b[k].x, a0);
+                a1 = fma((double)a[k].y, (double)b[k].y, a1);
+                a0 = fma((double)a[k].z, (double)b[k].z, a0);
+                a1 = fma((double)a[k].w, (double)b[k].w, a1);
+            }
+        }
+        acc = a0 + a1;
+    } else {
+        acc = 0.0;
+        for (uint32_t i = tid; i < hidden; i += 256u) acc = fma((double)row[i], (double)xv[i], acc);
+    }
+    acc = wave_sum_f64(acc);
+    if ((tid & 63u) == 0u) partial[tid >> 6] = acc;
+    lev_barrier_lds();
+    if (tid == 0u) scores[(uint64_t)t * experts + e] = (float)(((partial[0] + partial[1]) + partial[2]) + partial[3]);
+}
+
+// Many tokens where the matrix-core kernel below does not apply (rows of no whole 16 columns, unaligned operands):
+// workgroup (e, g) owns router row e, its wave w scores the four tokens 4*(4g+w).. against the row, which it reads once
+// for the four.
 constexpr uint32_t kScoreTokensPerWave = 4;
 
 __global__ void __launch_bounds__(256)
 moe_scores_kernel(const float *__restrict__ wr, const float *__restrict__ x,
-                  float *__restrict__ scores, uint32_t hidden, uint32_t experts, uint32_t tokens,
-                  int split) {
-    __shared__ double partial[4][4];
+                  float *__restrict__ scores, uint32_t hidden, uint32_t experts, uint32_t tokens) {
     const uint32_t e = blockIdx.x, lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const uint32_t waves = blockDim.x >> 6;
     const float *row = wr + (uint64_t)e * hidden;
     const bool vec = (hidden & 3u) == 0u &&
                      ((reinterpret_cast<uintptr_t>(wr) | reinterpret_cast<uintptr_t>(x)) & 15u) == 0u;
-    if (split) {
-        for (uint32_t t = 0; t < tokens; ++t) {
-            const float *xv = x + (uint64_t)t * hidden;
-            double acc;
-            if (vec) {
-                const lev_f32x4 *r4 = reinterpret_cast<const lev_f32x4 *>(row);
-                const lev_f32x4 *x4 = reinterpret_cast<const lev_f32x4 *>(xv);
-                double a0 = 0.0, a1 = 0.0;
-                for (uint32_t i = threadIdx.x; i < hidden / 4u; i += blockDim.x) {
-                    lev_f32x4 a = r4[i], b = x4[i];
-                    a0 = fma((double)a.x, (double)b.x, a0);
-                    a1 = fma((double)a.y, (double)b.y, a1);
-                    a0 = fma((double)a.z, (double)b.z, a0);
-                    a1 = fma((double)a.w, (double)b.w, a1);
-                }
-                acc = a0 + a1;
-            } else {
-                acc = 0.0;
-                for (uint32_t i = threadIdx.x; i < hidden; i += blockDim.x)
-                    acc = fma((double)row[i], (double)xv[i], acc);
-            }
-            acc = wave_sum_f64(acc);
-            if (lane == 0) partial[t][wave] = acc;
-        }
-        lev_barrier_lds();
-        if (threadIdx.x < tokens) {
-            double acc = partial[threadIdx.x][0];
-            for (uint32_t w = 1; w < waves; ++w) acc += partial[threadIdx.x][w];
-            scores[(uint64_t)threadIdx.x * experts + e] = (float)acc;
-        }
-        return;
-    }
     constexpr uint32_t K = kScoreTokensPerWave;
     const uint32_t t0 = (blockIdx.y * waves + wave) * K;
     if (t0 >= tokens) return;
@@ -510,71 +517,92 @@ moe_scores_kernel(const float *__restrict__ wr, const float *__restrict__ x,
     }
 }
 
-// Many tokens: scores as a small f64 matrix product on the matrix cores
-// (v_mfma_f64_16x16x4_f64: exact products of f32 inputs, f64 sums, rounded to
-// f32 once by the selection kernel).  A 16-token x 16-expert tile is shared by
-// kScoreSplit workgroups of four waves; the sixteen waves split the hidden
-// dimension (the loop is latency-bound: a short share per wave keeps all of its
-// loads in flight at once, and four workgroups a tile put 128 CUs instead of 32
-// to work at 64 tokens x 128 experts).  A workgroup adds its waves' partial
-// tiles in wave order and leaves the f64 sum in partials[split][token][expert];
-// moe_topk_kernel adds the kScoreSplit of them in order.  The router
-// and the activations are each read (tokens/16) resp. (experts/16) times instead
-// of once per (expert, 16 tokens).
-// Lane (i, kq) = (l % 16, l / 16) loads four consecutive floats of token row i
-// and of router row i; MFMA m of a step takes element m of both, i.e. the 16
-// k's of a step are spread as k = 4*kq + m: the same permutation on both
-// operands.  hidden % 256 == 0, rows 16-byte aligned.
+// Many tokens: scores as a small f64 matrix product on the matrix cores (v_mfma_f64_16x16x4_f64: exact products of
+// f32 inputs, f64 sums, rounded to f32 once by the selection kernel).  A tile of 16 * TT tokens x 16 * TE experts is
+// shared by kScoreSplit workgroups of four waves; the sixteen waves split the hidden dimension in shares of whole 16
+// columns (the loop is latency-bound: a short share per wave keeps all of its loads in flight at once, and four
+// workgroups a tile put 128 CUs instead of 32 to work at 64 tokens x 128 experts).  A workgroup adds its waves' partial
+// tiles in wave order and leaves the f64 sum in partials[split][token][expert]; moe_topk_kernel adds the kScoreSplit of
+// them in order.  The router and the activations are each read (tokens / 16 TT) resp. (experts / 16 TE) times.
+// Lane (i, kq) = (l % 16, l / 16) loads four consecutive floats of token row i and of router row i; MFMA m of a step
+// takes element m of both, i.e. the 16 k's of a step are spread as k = 4*kq + m: the same permutation on both operands.
+// hidden % 16 == 0, rows 16-byte aligned.  Tiles of one size or the other: the same sums in the same order.
+// 1000 tokens, 128 experts: 2816 columns 28 us in tiles of 16 x 16, 23 in tiles of 32 x 32 (9 us of f64 products).
 typedef double moe_f64x4 __attribute__((ext_vector_type(4)));
 
 constexpr uint32_t kScoreSplit = 4;
 
+template <int TT, int TE>
 __global__ void __launch_bounds__(256)
 moe_scores_mfma_kernel(const float *__restrict__ wr, const float *__restrict__ x, double *__restrict__ partials,
                        uint32_t hidden, uint32_t experts, uint32_t tokens) {
-    __shared__ double part[16 / kScoreSplit][256];
+    constexpr uint32_t kWaves = 16 / kScoreSplit;
+    __shared__ double part[kWaves][TT * TE * 256];
     const uint32_t lane = threadIdx.x & 63u, lw = threadIdx.x >> 6;
-    const uint32_t wave = blockIdx.z * (16u / kScoreSplit) + lw;   // which sixteenth of the hidden dimension
+    const uint32_t wave = blockIdx.z * kWaves + lw;                    // which sixteenth of the hidden dimension
     const uint32_t i = lane & 15u, kq = lane >> 4;
-    const uint32_t e0 = blockIdx.x * 16u, t0 = blockIdx.y * 16u;
-    const uint32_t tok = t0 + i < tokens ? t0 + i : tokens - 1u;       // rows past the end repeat the last one
-    const uint32_t exp = e0 + i < experts ? e0 + i : experts - 1u;
-    const uint32_t span = hidden >> 4;                                  // this wave's share of the hidden dimension
-    const lev_f32x4 *xa = reinterpret_cast<const lev_f32x4 *>(x + (uint64_t)tok * hidden + wave * span) + kq;
-    const lev_f32x4 *wb = reinterpret_cast<const lev_f32x4 *>(wr + (uint64_t)exp * hidden + wave * span) + kq;
-    moe_f64x4 acc = {0.0, 0.0, 0.0, 0.0};
-    const uint32_t steps = span >> 4;
+    const uint32_t e0 = blockIdx.x * (16u * TE), t0 = blockIdx.y * (16u * TT);
+    const uint32_t all = hidden >> 4, first = all * wave / 16u, last = all * (wave + 1u) / 16u;   // this wave's steps
+    const lev_f32x4 *xa[TT], *wb[TE];
+#pragma unroll
+    for (int t = 0; t < TT; ++t) {
+        const uint32_t tok = t0 + 16u * t + i;                          // rows past the end repeat the last one
+        xa[t] = reinterpret_cast<const lev_f32x4 *>(x + (uint64_t)(tok < tokens ? tok : tokens - 1u) * hidden) + kq;
+    }
+#pragma unroll
+    for (int e = 0; e < TE; ++e) {
+        const uint32_t exp = e0 + 16u * e + i;
+        wb[e] = reinterpret_cast<const lev_f32x4 *>(wr + (uint64_t)(exp < experts ? exp : experts - 1u) * hidden) + kq;
+    }
+    moe_f64x4 acc[TT][TE];
+#pragma unroll
+    for (int t = 0; t < TT; ++t)
+#pragma unroll
+        for (int e = 0; e < TE; ++e) acc[t][e] = moe_f64x4{0.0, 0.0, 0.0, 0.0};
     // four steps' operands are requested together (steps past the end repeat the last one with a zero
     // activation: they add nothing)
-    for (uint32_t s0 = 0; s0 < steps; s0 += 4u) {
-        lev_f32x4 a[4], b[4];
+    for (uint32_t s0 = first; s0 < last; s0 += 4u) {
+        lev_f32x4 a[TT][4], b[TE][4];
 #pragma unroll
         for (uint32_t j = 0; j < 4u; ++j) {
-            const uint32_t s = s0 + j < steps ? s0 + j : steps - 1u;
-            a[j] = xa[4u * s];
-            b[j] = wb[4u * s];
+            const uint32_t s = s0 + j < last ? s0 + j : last - 1u;
+#pragma unroll
+            for (int t = 0; t < TT; ++t) a[t][j] = xa[t][4u * s];
+#pragma unroll
+            for (int e = 0; e < TE; ++e) b[e][j] = wb[e][4u * s];
         }
 #pragma unroll
         for (uint32_t j = 0; j < 4u; ++j) {
-            const bool live = s0 + j < steps;
-            const lev_f32x4 aj = live ? a[j] : lev_f32x4{0.f, 0.f, 0.f, 0.f};
-            const lev_f32x4 bj = live ? b[j] : lev_f32x4{0.f, 0.f, 0.f, 0.f};
-            acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)aj.x, (double)bj.x, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)aj.y, (double)bj.y, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)aj.z, (double)bj.z, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)aj.w, (double)bj.w, acc, 0, 0, 0);
+            const bool live = s0 + j < last;
+#pragma unroll
+            for (int e = 0; e < TE; ++e) b[e][j] = live ? b[e][j] : lev_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+#pragma unroll
+                for (int t = 0; t < TT; ++t) {
+                    const float am = live ? a[t][j][m] : 0.f;
+#pragma unroll
+                    for (int e = 0; e < TE; ++e)
+                        acc[t][e] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)am, (double)b[e][j][m], acc[t][e], 0, 0, 0);
+                }
         }
     }
     // D of the f64 16x16x4 product: register r of lane (i, kq) is row (token) 4*r + kq of column (expert) i
 #pragma unroll
-    for (int r = 0; r < 4; ++r) part[lw][(4u * (uint32_t)r + kq) * 16u + i] = acc[r];
-    lev_barrier_lds();
-    const uint32_t tt = (threadIdx.x >> 4) & 15u, ee = threadIdx.x & 15u;
-    if (t0 + tt < tokens && e0 + ee < experts) {
-        double total = part[0][threadIdx.x];
+    for (int t = 0; t < TT; ++t)
 #pragma unroll
-        for (uint32_t w = 1; w < 16u / kScoreSplit; ++w) total += part[w][threadIdx.x];
-        partials[((uint64_t)blockIdx.z * tokens + t0 + tt) * experts + e0 + ee] = total;
+        for (int e = 0; e < TE; ++e)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) part[lw][(TE * t + e) * 256 + (4u * (uint32_t)r + kq) * 16u + i] = acc[t][e][r];
+    lev_barrier_lds();
+#pragma unroll
+    for (int q = 0; q < TT * TE; ++q) {
+        const uint32_t tt = t0 + 16u * (q / TE) + (threadIdx.x >> 4), ee = e0 + 16u * (q % TE) + (threadIdx.x & 15u);
+        if (tt >= tokens || ee >= experts) continue;
+        double total = part[0][q * 256 + threadIdx.x];
+#pragma unroll
+        for (uint32_t w = 1; w < kWaves; ++w) total += part[w][q * 256 + threadIdx.x];
+        partials[((uint64_t)blockIdx.z * tokens + tt) * experts + ee] = total;
     }
 }
 
@@ -1594,31 +1622,45 @@ lev_moe_grouped_args grouped_args(const moe_args &a, uint32_t tokens) {
                                 a.top_k,       tokens};
 }
 
-bool use_grouped(const lev_ctx *ctx, const moe_args &a, const float *x, uint32_t tokens) {
+// The gate/up kernel selects the experts by itself: fewer tokens than leave their scores as partial sums.
+bool selects_itself(const moe_args &a, const float *x, uint32_t tokens) {
+    return experts_fast(a, x) && tokens < kScoresMfmaMinTokens && a.experts <= kRouteInKernelMax;
+}
+
+// whole_layer: the experts are selected in the same call
+bool use_grouped(const lev_ctx *ctx, const moe_args &a, const float *x, uint32_t tokens, bool whole_layer) {
     static const bool enabled = [] {
         const char *e = getenv("LEV_MOE_GROUPED");   // LEV_MOE_GROUPED=0: per-pair kernels, for comparison
         return !(e && e[0] == '0');
     }();
     return enabled && tokens >= kGroupedMinTokens && experts_aligned(a, x) &&
-           lev_moe_grouped_usable(ctx, grouped_args(a, tokens));
+           lev_moe_grouped_usable(ctx, grouped_args(a, tokens), whole_layer && selects_itself(a, x, tokens));
 }
 
 // *in_partials: the scores were left as f64 partial sums in `partials` (for run_topk), not in `scores`.
 hipError_t run_scores(lev_ctx *ctx, const float *wr, const float *x, float *scores, double *partials,
                       bool *in_partials, uint32_t hidden, uint32_t experts, uint32_t tokens) {
     *in_partials = false;
-    if (partials && tokens >= kScoresMfmaMinTokens && hidden % 256u == 0u &&
-        ((reinterpret_cast<uintptr_t>(wr) | reinterpret_cast<uintptr_t>(x)) & 15u) == 0u) {
-        hipLaunchKernelGGL(moe_scores_mfma_kernel, dim3((experts + 15u) / 16u, (tokens + 15u) / 16u, kScoreSplit),
-                           dim3(256), 0, ctx->stream, wr, x, partials, hidden, experts, tokens);
-        *in_partials = true;
+    if (tokens < kScoresMfmaMinTokens) {
+        hipLaunchKernelGGL(moe_scores_few_kernel, dim3(experts, tokens), dim3(256), 0, ctx->stream, wr, x, scores, hidden,
+                           experts);
         return hipGetLastError();
     }
-    const int split = tokens <= 4u;
+    if (partials && hidden % 16u == 0u && ((reinterpret_cast<uintptr_t>(wr) | reinterpret_cast<uintptr_t>(x)) & 15u) == 0u) {
+        *in_partials = true;
+        // tiles of 32 x 32 as soon as they fill the CUs
+        const uint32_t te = (experts + 31u) / 32u, tt = (tokens + 31u) / 32u;
+        if ((uint64_t)te * tt * kScoreSplit >= (uint64_t)ctx->num_cus)
+            hipLaunchKernelGGL((moe_scores_mfma_kernel<2, 2>), dim3(te, tt, kScoreSplit), dim3(256), 0, ctx->stream, wr, x,
+                               partials, hidden, experts, tokens);
+        else
+            hipLaunchKernelGGL((moe_scores_mfma_kernel<1, 1>), dim3((experts + 15u) / 16u, (tokens + 15u) / 16u, kScoreSplit),
+                               dim3(256), 0, ctx->stream, wr, x, partials, hidden, experts, tokens);
+        return hipGetLastError();
+    }
     const uint32_t per_group = 4u * kScoreTokensPerWave;
-    const uint32_t groups = split ? 1u : (tokens + per_group - 1u) / per_group;
-    hipLaunchKernelGGL(moe_scores_kernel, dim3(experts, groups), dim3(256), 0, ctx->stream, wr, x,
-                       scores, hidden, experts, tokens, split);
+    hipLaunchKernelGGL(moe_scores_kernel, dim3(experts, (tokens + per_group - 1u) / per_group), dim3(256), 0, ctx->stream, wr,
+                       x, scores, hidden, experts, tokens);
     return hipGetLastError();
 }
 
@@ -1698,7 +1740,7 @@ extern "C" int lev_hip_moe_experts_q4_0(lev_ctx *ctx, const lev_moe_experts *poo
     moe_args a;
     int st = check_pools(ctx, pools, top_k, tokens, &a);
     if (st != LEV_OK) return st;
-    const bool grouped = use_grouped(ctx, a, d_x, tokens) && (reinterpret_cast<uintptr_t>(d_act) & 15u) == 0u;
+    const bool grouped = use_grouped(ctx, a, d_x, tokens, false) && (reinterpret_cast<uintptr_t>(d_act) & 15u) == 0u;
     float *act = d_act;
     moe_scratch s{nullptr, nullptr, nullptr};
     if (!act || grouped) {
@@ -1734,7 +1776,7 @@ int moe_layer_impl(lev_ctx *ctx, const lev_moe_experts *pools, const float *d_ro
     int st = check_pools(ctx, pools, top_k, tokens, &a);
     if (st != LEV_OK) return st;
     if (a.experts > 4096u) return lev_fail(ctx, LEV_ERR_BAD_DIMENSIONS, "moe_layer: %u experts", a.experts);
-    const bool grouped = !fixed && use_grouped(ctx, a, d_x, tokens);
+    const bool grouped = !fixed && use_grouped(ctx, a, d_x, tokens, true);
     moe_scratch s;
     if (fixed) {
         if (tokens > LEV_NOALLOC_MOE_MAX_TOKENS)
@@ -1763,7 +1805,7 @@ int moe_layer_impl(lev_ctx *ctx, const lev_moe_experts *pools, const float *d_ro
     const uint32_t family = sel ? sel->family : 1u;
     const uint32_t gu_per_cu = sel && sel->rows_in_flight ? sel->rows_in_flight : 2u;
     const bool matrix_cores = !(sel && sel->persistent);   // schedule field `persistent` = 1: the vector-ALU expert kernels
-    const bool few = fast && tokens <= 4u && a.experts <= kRouteInKernelMax;
+    const bool few = !grouped && selects_itself(a, d_x, tokens);
     if (few && family == 2u) {
         // few tokens: the router kernel's last workgroup selects the experts
         st = lev_hip_check(ctx,

@@ -687,17 +687,19 @@ hipError_t lev_moe_merge_launch(lev_ctx *ctx, const lev_moe_grouped_args &a, con
 
 // Grouping costs some 13 us of launches over the kernels that stream an expert for every pair, and saves the
 // bytes of the experts that several tokens share (top_k of `experts` each: expected number of distinct
-// ones). Those kernels also stream large experts less well: ten experts' worth of bytes.  65 MB is where the
-// two meet (us a layer, grouped against per pair: 2816 / 704, top-8 of 128: 5 tokens 62, 66; 16 tokens 89, 109;
-// 1408 / 320, top-4 of 64: 16 tokens 39, 31; 64 tokens 50, 57; 1024 / 576, top-2 of 32: 32 tokens 34, 31;
-// 64 tokens 36, 45; 3072 / 1024, top-6 of 60: 5 tokens 69, 79).  Rows of whole 256-value tasks up to
+// ones). Those kernels also stream large experts less well: ten experts' worth of bytes.  Where they select the
+// experts themselves (`selects`) they save a launch more, and 125 MB is where the two meet (us a layer, grouped
+// against per pair: 2816 / 704, top-8 of 128: 5 tokens 52, 40; 12 tokens 76, 71; 15 tokens 84, 85; 2176 / 768, top-4 of
+// 60: 15 tokens 50, 45; 3072 / 1408, top-6 of 256: 8 tokens 97, 89; 12 tokens 128, 134); with a selection in front 65 MB
+// (2816 / 704: 16 tokens 89, 109; 1408 / 320, top-4 of 64: 16 tokens 39, 31; 64 tokens 50, 57; 1024 / 576, top-2 of 32:
+// 32 tokens 34, 31; 64 tokens 36, 45).  Rows of whole 256-value tasks up to
 // 2048 wide are always grouped, so that a token's bits do not depend on how many travel with it.
-bool lev_moe_grouped_usable(const lev_ctx *ctx, const lev_moe_grouped_args &a) {
+bool lev_moe_grouped_usable(const lev_ctx *ctx, const lev_moe_grouped_args &a, bool selects) {
     if (!lev_moe_prefill_usable(a)) return false;
     if (a.hidden % 256u == 0u && a.inter % 256u == 0u && a.hidden <= 2048u && a.inter <= 2048u) return true;
     const double expert_bytes = 3.0 * a.hidden * a.inter * 18.0 / 32.0;
     const double distinct = a.experts * (1.0 - std::pow(1.0 - (double)a.top_k / a.experts, (double)a.tokens));
-    return ((double)a.tokens * a.top_k - distinct + 10.0) * expert_bytes >= 65e6;
+    return ((double)a.tokens * a.top_k - distinct + 10.0) * expert_bytes >= (selects ? 125e6 : 65e6);
 }
 
 size_t lev_moe_grouped_scratch_bytes(const lev_ctx *ctx, const lev_moe_grouped_args &a) {

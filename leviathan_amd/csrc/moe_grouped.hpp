@@ -29,7 +29,7 @@ struct alignas(32) lev_grp_start {
 };
 
 // Whether the many-token path takes the call (the caller also checks 4-byte aligned pools and x).
-bool lev_moe_grouped_usable(const lev_ctx *ctx, const lev_moe_grouped_args &a);
+bool lev_moe_grouped_usable(const lev_ctx *ctx, const lev_moe_grouped_args &a, bool selects);
 size_t lev_moe_grouped_scratch_bytes(const lev_ctx *ctx, const lev_moe_grouped_args &a);
 // act: f32 [tokens*top_k][inter] (written here, read by the down stage).
 hipError_t lev_moe_grouped_launch(lev_ctx *ctx, const lev_moe_grouped_args &a, const float *x,

@@ -125,21 +125,35 @@ moe_pf_group_kernel(const int32_t *__restrict__ ids, uint32_t pairs, uint32_t ex
     for (uint32_t e = tid; e < experts; e += 1024u) s_cnt[e] = 0;
     __syncthreads();
     bool bad_seen = false;
-    for (uint32_t p = tid; p < pairs; p += 1024u) {
-        const int32_t e = ids[p];
-        bool ok = e >= 0 && (uint32_t)e < experts;
-        const uint32_t slot = p % top_k, first = p - slot;
-        for (uint32_t k0 = 0; k0 < top_k; k0 += 8u) {           // eight ids per wait
-            int32_t other[8];
+    // a thread takes a token, eight of its ids a wait
+    const uint32_t tokens_all = pairs / top_k;
+    for (uint32_t t = tid; t < tokens_all; t += 1024u) {
+        const int32_t *row = ids + (uint64_t)t * top_k;
+        for (uint32_t k0 = 0; k0 < top_k; k0 += 8u) {
+            int32_t own[8];
+            bool ok[8];
 #pragma unroll
-            for (uint32_t u = 0; u < 8u; ++u) other[u] = ids[first + (k0 + u < top_k ? k0 + u : slot)];
+            for (uint32_t u = 0; u < 8u; ++u) own[u] = row[k0 + u < top_k ? k0 + u : k0];
 #pragma unroll
-            for (uint32_t u = 0; u < 8u; ++u)
-                if (k0 + u < top_k && k0 + u != slot && other[u] == e) ok = false;
+            for (uint32_t u = 0; u < 8u; ++u) ok[u] = own[u] >= 0 && (uint32_t)own[u] < experts;
+            for (uint32_t j0 = 0; j0 < top_k; j0 += 8u) {
+                int32_t other[8];
+#pragma unroll
+                for (uint32_t v = 0; v < 8u; ++v) other[v] = j0 == k0 ? own[v] : row[j0 + v < top_k ? j0 + v : j0];
+#pragma unroll
+                for (uint32_t u = 0; u < 8u; ++u)
+#pragma unroll
+                    for (uint32_t v = 0; v < 8u; ++v)
+                        if (j0 + v < top_k && j0 + v != k0 + u && other[v] == own[u]) ok[u] = false;
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < 8u; ++u) {
+                if (k0 + u >= top_k) continue;
+                valid[(uint64_t)t * top_k + k0 + u] = ok[u] ? 1 : 0;
+                if (ok[u]) atomicAdd(&s_cnt[own[u]], 1);
+                bad_seen = bad_seen || !ok[u];
+            }
         }
-        valid[p] = ok ? 1 : 0;
-        if (ok) atomicAdd(&s_cnt[e], 1);
-        bad_seen = bad_seen || !ok;
     }
     if (bad_seen) atomicOr(flag, kFlagBadExpertId);
     __syncthreads();
@@ -185,8 +199,20 @@ moe_pf_group_kernel(const int32_t *__restrict__ ids, uint32_t pairs, uint32_t ex
     __syncthreads();
     // The order of an expert's pairs depends on the atomics; no result does: every pair is computed
     // by itself and owns its outputs.
-    for (uint32_t p = tid; p < pairs; p += 1024u)
-        if (valid[p]) glist[atomicAdd(&s_cur[ids[p]], 1)] = (int32_t)p;
+    for (uint32_t t = tid; t < tokens_all; t += 1024u)
+        for (uint32_t k0 = 0; k0 < top_k; k0 += 8u) {
+            int32_t own[8];
+            uint8_t ok[8];
+#pragma unroll
+            for (uint32_t u = 0; u < 8u; ++u) {
+                const uint32_t p = t * top_k + (k0 + u < top_k ? k0 + u : k0);
+                own[u] = ids[p];
+                ok[u] = valid[p];
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < 8u; ++u)
+                if (k0 + u < top_k && ok[u]) glist[atomicAdd(&s_cur[own[u]], 1)] = (int32_t)(t * top_k + k0 + u);
+        }
 }
 
 // ---------------------------------------------------------------------------
