@@ -117,6 +117,7 @@ int lev_hip_program_begin(lev_ctx *ctx);
 int lev_hip_program_end(lev_ctx *ctx, lev_program **out);
 int lev_hip_program_run(lev_ctx *ctx, lev_program *program);
 int lev_hip_program_destroy(lev_ctx *ctx, lev_program *program);
+/* Operators recorded, as launches of their own; the replay may run several of them in one. */
 int lev_hip_program_node_count(lev_program *program, size_t *out);
 
 /* ---- buffers (device.makeBuffer, Q4.swift:223-231; Buf, engine.rs:10-40) ---- */

@@ -56,6 +56,8 @@ struct lev_ctx {
     // True between lev_hip_program_begin and lev_hip_program_end: the stream
     // is being captured, so nothing may allocate or synchronise.
     bool recording = false;
+    // Operators recorded so far that share a node with another one: a program's count is that of its operators.
+    size_t folded_nodes = 0;
     // Schedules installed per (op, shape) by lev_hip_forge_select; the matvec
     // entry points look their shape up here before their built-in choice.
     struct selection {

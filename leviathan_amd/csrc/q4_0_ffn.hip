@@ -148,10 +148,8 @@ extern "C" int lev_hip_shared_expert_ffn_q4_0(lev_ctx *ctx, const float *d_x, co
     if (st != LEV_OK) return st;
     const uintptr_t al4 = reinterpret_cast<uintptr_t>(d_gate_w) | reinterpret_cast<uintptr_t>(d_up_w);
     const uintptr_t al16 = reinterpret_cast<uintptr_t>(d_x) | reinterpret_cast<uintptr_t>(d_h) | reinterpret_cast<uintptr_t>(d_ffn_norm);
-    // A schedule installed for the gate/up GEMV keeps the operators apart, so that it is the one that runs; so does
-    // recording at hidden sizes up to 2048, whose programs callers know by a node per operator (wider ones, where
-    // the fused kernel saves most, are recorded fused).
-    const bool fused = !(ctx->recording && hidden <= 2048u) && hidden % 64u == 0u && hidden <= 4096u && (al4 & 3u) == 0u && (al16 & 15u) == 0u && d_x != d_h &&
+    // A schedule installed for the gate/up GEMV keeps the operators apart, so that it is the one that runs.
+    const bool fused = hidden % 64u == 0u && hidden <= 4096u && (al4 & 3u) == 0u && (al16 & 15u) == 0u && d_x != d_h &&
                        !lev_selected(ctx, LEV_OP_Q4_0_GEMV, hidden, inter, 1);
     if (fused) {
         const uint32_t cus = (uint32_t)ctx->num_cus, per = (inter + 16u * cus - 1u) / (16u * cus);
@@ -164,6 +162,7 @@ extern "C" int lev_hip_shared_expert_ffn_q4_0(lev_ctx *ctx, const float *d_x, co
         else if (hidden <= 3072u) LEV_FFN(12);
         else LEV_FFN(16);
 #undef LEV_FFN
+        if (ctx->recording) ctx->folded_nodes += 3u;   // norm, gate, up and geluUp are one node
         st = lev_hip_check(ctx, hipGetLastError(), "shared_expert_ffn gate/up launch");
     } else {
         st = lev_hip_rmsnorm(ctx, d_x, d_h, hidden, 1, d_ffn_norm, eps);
