@@ -15,12 +15,17 @@
 //
 // Arithmetic.  Weights enter the matrix cores as the exact integers n - 8 in fp16, one Q4_0 block
 // (32 weights) per product; its block scale d is applied to the f32 result, y += d * (A.B), in the
-// lane that holds the weight row.  Activations are two fp16 planes, x = hi + lo to half an f32
-// unit, after a power-of-two row scale.  Nothing is rounded to fp16 that is not exact there.
+// lane that holds the weight row.  Activations are two fp16 planes, x = hi + lo to one f32 unit, after a
+// power-of-two row scale: a finite row loses no more than that down to 2^-17 of its maximum.
+// The sums of a row of more than 32 blocks are folded: parts of 16 blocks are added up on their own, then to
+// each other.  As one chain of 88 blocks (hidden 2816) an f32 sum gathers 6.6 roundings of its size, folded
+// 3.2; against 64-bit sums the layer's outputs are off by 2.2e-7 (2-norm) at 2816 / 704 and 2.3e-7 at
+// 4096 / 448 where one chain left 3.0e-7 and 3.5e-7 and the kernels that these sizes took before 2.4e-7.
 //
-// Measured: hidden 2816, intermediate 704, top-8 of 128 experts, 1000 tokens: gate/up 211 us, down 114, the
-// layer 400 us (4420 with a workgroup per token and slot, which these sizes took before); 2048 / 768, 1000
-// tokens: 321 us (627 with twelve columns a pass over the weights).
+// Measured: hidden 2816, intermediate 704, top-8 of 128 experts, 1000 tokens: the layer 408 us (402 with one
+// chain a row; 4420 with a workgroup per token and slot, which these sizes took before); 2048 / 768, 1000
+// tokens: 324 us (317; 627 with twelve columns a pass over the weights); 4096 / 448, top-4 of 32, 300 tokens:
+// 111 us (131).
 //
 // What bounds it: per 32 x 32 outputs and block, 4 v_mfma_f32_32x32x16_f16 (128 clocks of the matrix
 // pipe) against 16 multiply-adds by d (some 70 clocks of vector issue) and, shared by a wave's two
@@ -29,6 +34,7 @@
 // alone; four 32x32x16 and the same multiply-adds: 760; hence the larger instruction).
 #include "moe_prefill.hpp"
 
+#include <cmath>
 #include <type_traits>
 
 namespace {
@@ -42,7 +48,8 @@ constexpr uint32_t kPfStep = 64;             // activations per K-step: two bloc
 constexpr uint32_t kPfWRow = 80;             // a weight row's group of four blocks (72 bytes) in LDS: five pieces of 16 bytes
 constexpr int kPfFetch = 3;                  // direct loads per group: 160 pieces, 64 a load (the third: half a wave)
 constexpr uint32_t kPfWArea = 32 * kPfWRow;  // 32 rows a wave
-constexpr uint32_t kPfThreads = 512;
+constexpr uint32_t kPfFold = 8;              // steps (16 blocks) of a part of a folded sum
+constexpr uint32_t kPfChain = 32;            // blocks of a row from which on its sums are folded: more
 
 // ---------------------------------------------------------------------------
 // Activation planes of one row, by one wave.  The row is scaled by the power of two that brings its
@@ -216,18 +223,21 @@ moe_pf_group_kernel(const int32_t *__restrict__ ids, uint32_t pairs, uint32_t ex
 }
 
 // ---------------------------------------------------------------------------
-// The grouped product.  Four waves; wave w of a PAIRED (gate/up) workgroup owns 32 rows of the gate
-// matrix and the same 32 rows of the up matrix, so that g and u of an output meet in one lane; down:
-// 64 rows.  The activation step (64 values of every column, both planes) is shared by the workgroup
-// in LDS, two buffers, brought by direct global -> LDS loads; the weights of a wave are its own: 144
-// bytes of each row fetched 16 bytes a lane with consecutive lanes on consecutive bytes, one group of
-// eight blocks ahead, parked as they lie in memory and decoded by the lane that multiplies them.
-// 71 KB of LDS and at most 256 registers: two workgroups per CU, whose waits cover each other.
+// The grouped product.  A wave of a PAIRED (gate/up) workgroup owns 16 rows of the gate matrix and the
+// same 16 rows of the up matrix, so that g and u of an output meet in one lane; down: 32 rows.  The
+// activation step (64 values of every column, both planes) is shared by the workgroup in LDS, two
+// buffers, brought by direct global -> LDS loads; the weights of a wave are its own: 72 bytes of each
+// row fetched 16 bytes a lane with consecutive lanes on consecutive bytes, one group of four blocks
+// ahead, parked as they lie in memory and decoded by the lane that multiplies them.
+// One chain a row (FOLD false): eight waves, 71 KB of LDS and 128 registers, two workgroups per CU whose
+// waits cover each other.  Folded, the parts already added take 32 registers more, three waves a SIMD:
+// one workgroup of twelve waves a CU, or three of four (pf_waves).
 // ---------------------------------------------------------------------------
+template <uint32_t WAVES>
 struct pf_lds_map {
     static constexpr uint32_t kABuf = 2u * 8u * 1024u;        // two planes x eight regions of eight columns
     static constexpr uint32_t kW = 2u * kABuf;
-    static constexpr uint32_t kWBuf = kPfThreads / 64u * kPfWArea;
+    static constexpr uint32_t kWBuf = WAVES * kPfWArea;
     static constexpr uint32_t kBytes = kW + 2u * kWBuf;
 };
 
@@ -241,12 +251,12 @@ __device__ __forceinline__ void pf_decode(uint32_t codes, uint32_t mask, uint32_
     out[1] = __builtin_bit_cast(uint32_t, (f16x2)(__builtin_bit_cast(f16x2, ((codes >> 8) & mask) | magic) - bias));
 }
 
-template <bool PAIRED, int T>
+template <bool PAIRED, uint32_t WAVES, bool FOLD, int T>
 __device__ __forceinline__ void pf_tile(const lev_moe_grouped_args &a, const lev_pf_item it, uint32_t rt,
                                         const _Float16 *__restrict__ ph, const _Float16 *__restrict__ pl,
                                         const uint32_t *__restrict__ pmax, const int32_t *__restrict__ glist,
                                         float *__restrict__ out, uint8_t *lds, int32_t *s_pair, float *s_us) {
-    typedef pf_lds_map L;
+    typedef pf_lds_map<WAVES> L;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
     const uint32_t lr = lane & 31u, g = lane >> 5;
     const uint32_t in_len = PAIRED ? a.hidden : a.inter, out_rows = PAIRED ? a.inter : a.hidden;
@@ -257,7 +267,7 @@ __device__ __forceinline__ void pf_tile(const lev_moe_grouped_args &a, const lev
     // whole waves: both row counts are multiples of 64).  Piece q of a group is piece q % 5 of row q / 5: the row's
     // bytes 0, 16, 32, 48 and 56 .. + 15 at 16 bytes a piece, so the fourth block's codes lie at 64, not 56; the last
     // group of a row may hold two blocks (36 bytes): then its third piece is bytes 20 .. 35, the second block's codes ----
-    const uint32_t row0 = PAIRED ? rt * 128u + wave * 16u : rt * 256u + wave * 32u;
+    const uint32_t row0 = (rt * WAVES + wave) * (PAIRED ? 16u : 32u);
     const bool live = row0 < out_rows;   // a wave past the last row only brings activations
     const uint32_t lds0 = lev_lds_offset(lds);
     const uint8_t *wsrc[kPfFetch];
@@ -295,10 +305,11 @@ __device__ __forceinline__ void pf_tile(const lev_moe_grouped_args &a, const lev
     // columns x eight runs of eight values.  Slot 8 * (run ^ region parity) + ((column & 7) ^ run) of a
     // region: a load's 64 lanes fetch 8 rows x 128 contiguous bytes, and the lanes of a fragment read (32
     // columns, one run each half) hit every bank equally ----
-    const _Float16 *asrc[T];
+    constexpr uint32_t kALoads = (8u * T + WAVES - 1u) / WAVES;
+    const _Float16 *asrc[kALoads];
 #pragma unroll
-    for (int j = 0; j < T; ++j) {
-        const uint32_t k = wave * T + j, region = k >> 1, run = (lane >> 3) ^ (region & 1u);
+    for (uint32_t j = 0; j < kALoads; ++j) {
+        const uint32_t k = wave * kALoads + j < 8u * T ? wave * kALoads + j : 8u * T - 1u, region = k >> 1, run = (lane >> 3) ^ (region & 1u);
         const uint32_t p = (uint32_t)s_pair[region * 8u + ((lane & 7u) ^ run)];
         asrc[j] = (k & 1u ? pl : ph) + (uint64_t)(PAIRED ? p / a.top_k : p) * in_len + run * 8u;
     }
@@ -306,18 +317,27 @@ __device__ __forceinline__ void pf_tile(const lev_moe_grouped_args &a, const lev
         const uint32_t s = step < nsteps ? step : nsteps - 1u;   // past the end: any valid step, never read
         const uint32_t dst = lds0 + (step & 1u) * L::kABuf;
 #pragma unroll
-        for (int j = 0; j < T; ++j) {
-            const uint32_t k = wave * T + j;
-            lev_load_lds16(asrc[j] + s * kPfStep, dst + (k & 1u) * 8192u + (k >> 1) * 1024u);
+        for (uint32_t j = 0; j < kALoads; ++j) {
+            const uint32_t k = wave * kALoads + j;
+            if (kALoads * WAVES == 8u * T || k < 8u * T) lev_load_lds16(asrc[j] + s * kPfStep, dst + (k & 1u) * 8192u + (k >> 1) * 1024u);
         }
     };
     a_request(0);
 
-    float y[T][16];
+    float y[T][16], whole[T][16];   // FOLD: the part under way, and the parts before it
 #pragma unroll
     for (int t = 0; t < T; ++t)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) y[t][i] = 0.f;
+        for (int i = 0; i < 16; ++i) y[t][i] = whole[t][i] = 0.f;
+    auto fold = [&]() {
+#pragma unroll
+        for (int t = 0; t < T; ++t)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                whole[t][i] += y[t][i];
+                y[t][i] = 0.f;
+            }
+    };
     uint32_t k_mask = 0x000F000Fu, k_magic = 0x64006400u;
     asm("" : "+v"(k_mask), "+v"(k_magic));   // in registers: (v & mask) | magic is one instruction
     const uint8_t *const wmine = lds + L::kW + wave * kPfWArea + lr * kPfWRow;
@@ -392,7 +412,10 @@ __device__ __forceinline__ void pf_tile(const lev_moe_grouped_args &a, const lev
     for (uint32_t step = 0; step < nsteps; step += 2u) {
         step_of(step, std::integral_constant<uint32_t, 0>());
         if (step + 1u < nsteps) step_of(step + 1u, std::integral_constant<uint32_t, 1>());
+        if (FOLD && (step & (kPfFold - 2u)) == kPfFold - 2u) fold();
     }
+    if (FOLD) fold();
+    float(&sum)[T][16] = FOLD ? whole : y;
 
     LEV_WAIT_VMCNT(0);   // the request past the end lands before the LDS is given back
     if (!live) return;
@@ -403,11 +426,11 @@ __device__ __forceinline__ void pf_tile(const lev_moe_grouped_args &a, const lev
 #pragma unroll
         for (int i = 0; i < 16; i += PAIRED ? 2 : 1) {
             uint32_t col = 32u * t + 8u * (i / 4) + 4u * g + (i % 4);
-            float v = y[t][i];
+            float v = sum[t][i];
             if (PAIRED) {
                 // lanes 0..15 of a half hold gate rows, 16..31 the same up rows: two columns trade halves, so
                 // that every lane has a gate and its up value, of column i in lanes 0..15, of i + 1 in 16..31
-                const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(y[t][i + 1]), false, false);
+                const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(sum[t][i + 1]), false, false);
                 col += lr >> 4;
                 const float us = s_us[col];
                 v = lev_gelu_up_value(__uint_as_float(sw[0]) * us, __uint_as_float(sw[1]) * us);
@@ -420,8 +443,8 @@ __device__ __forceinline__ void pf_tile(const lev_moe_grouped_args &a, const lev
 
 // grid: 8 * ceil(items / 8) * row tiles, in one line.  Workgroups go to the XCDs in turn, so item 8j + c
 // sits on XCD c with all its row tiles, which read the same activations through one L2.
-template <bool PAIRED>
-__global__ void __launch_bounds__(kPfThreads, 4)
+template <bool PAIRED, uint32_t WAVES, bool FOLD>
+__global__ void __launch_bounds__(WAVES * 64, FOLD ? 3 : 4)
 moe_pf_kernel(lev_moe_grouped_args a, uint32_t row_tiles, const _Float16 *__restrict__ ph,
               const _Float16 *__restrict__ pl, const uint32_t *__restrict__ pmax, const int32_t *__restrict__ glist,
               const lev_pf_item *__restrict__ items, const uint32_t *__restrict__ nitems, float *__restrict__ out) {
@@ -431,8 +454,8 @@ moe_pf_kernel(lev_moe_grouped_args a, uint32_t row_tiles, const _Float16 *__rest
     const uint32_t j = blockIdx.x >> 3, at = (j / row_tiles) * 8u + (blockIdx.x & 7u), rt = j % row_tiles;
     if (at >= *nitems) return;
     const lev_pf_item it = items[at];
-    if (it.count > 32) pf_tile<PAIRED, 2>(a, it, rt, ph, pl, pmax, glist, out, smem, s_pair, s_us);
-    else pf_tile<PAIRED, 1>(a, it, rt, ph, pl, pmax, glist, out, smem, s_pair, s_us);
+    if (it.count > 32) pf_tile<PAIRED, WAVES, FOLD, 2>(a, it, rt, ph, pl, pmax, glist, out, smem, s_pair, s_us);
+    else pf_tile<PAIRED, WAVES, FOLD, 1>(a, it, rt, ph, pl, pmax, glist, out, smem, s_pair, s_us);
 }
 
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
@@ -463,6 +486,46 @@ pf_layout pf_layout_of(const lev_moe_grouped_args &a) {
     return L;
 }
 
+template <bool PAIRED, uint32_t WAVES, bool FOLD>
+hipError_t pf_launch_as(lev_ctx *ctx, const lev_moe_grouped_args &a, const _Float16 *ph, const _Float16 *pl, const uint32_t *pmax,
+                        const int32_t *glist, const lev_pf_item *items, const uint32_t *nitems, float *out) {
+    const void *kernel = reinterpret_cast<const void *>(&moe_pf_kernel<PAIRED, WAVES, FOLD>);
+    static bool configured = false;
+    if (!configured) {
+        hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)pf_lds_map<WAVES>::kBytes);
+        if (e != hipSuccess) return e;
+        configured = true;
+    }
+    const uint32_t slots = (uint32_t)((pf_max_items(a) + 7u) / 8u) * 8u;
+    const uint32_t rows = PAIRED ? a.inter : a.hidden, per_wg = WAVES * (PAIRED ? 16u : 32u), tiles = (rows + per_wg - 1u) / per_wg;
+    hipLaunchKernelGGL((moe_pf_kernel<PAIRED, WAVES, FOLD>), dim3(slots * tiles), dim3(WAVES * 64u), pf_lds_map<WAVES>::kBytes,
+                       ctx->stream, a, tiles, ph, pl, pmax, glist, items, nitems, out);
+    return hipGetLastError();
+}
+
+// Waves of a folded workgroup.  Three of four waves share a CU where one of twelve has it to itself: they read the
+// activations three times, and their last round is finer.  So twelve where whole rounds of them come near the
+// work there is (us a layer with twelve, with four: 2816 / 704, top-8 of 128: 1000 tokens, 2.9 rounds, 393, 409; 300
+// tokens, 2 rounds, 209, 217; 2048 / 768, 1000 tokens, 310, 330; 1536 / 1088, top-4 of 60, 600 tokens, 1.5 rounds, 155,
+// 147; 2304 / 1280, top-2 of 32, 1000 tokens, 1.3 rounds, 184, 167; 4096 / 448, top-4 of 32, 300 tokens, 0.4 rounds, 149,
+// 105).  Items: one an expert that has pairs, and half an item more where they are many.
+uint32_t pf_waves(const lev_ctx *ctx, const lev_moe_grouped_args &a, uint32_t out_rows, uint32_t rows_a_wave) {
+    const double mean = (double)a.tokens * a.top_k / a.experts;
+    const double items = a.experts * std::fmax(1.0 - std::exp(-mean), mean / kPfCols + 0.5);
+    const double rounds = items * ((out_rows + 12u * rows_a_wave - 1u) / (12u * rows_a_wave)) / ctx->num_cus;
+    return 0.95 * std::ceil(rounds) <= rounds + 0.25 ? 12u : 4u;
+}
+
+template <bool PAIRED>
+hipError_t pf_launch(lev_ctx *ctx, const lev_moe_grouped_args &a, const _Float16 *ph, const _Float16 *pl, const uint32_t *pmax,
+                     const int32_t *glist, const lev_pf_item *items, const uint32_t *nitems, float *out) {
+    if ((PAIRED ? a.hidden : a.inter) <= 32u * kPfChain)
+        return pf_launch_as<PAIRED, 8, false>(ctx, a, ph, pl, pmax, glist, items, nitems, out);
+    if (pf_waves(ctx, a, PAIRED ? a.inter : a.hidden, PAIRED ? 16u : 32u) == 12u)
+        return pf_launch_as<PAIRED, 12, true>(ctx, a, ph, pl, pmax, glist, items, nitems, out);
+    return pf_launch_as<PAIRED, 4, true>(ctx, a, ph, pl, pmax, glist, items, nitems, out);
+}
+
 }  // namespace
 
 size_t lev_moe_prefill_scratch_bytes(const lev_moe_grouped_args &a) { return pf_layout_of(a).total; }
@@ -489,29 +552,15 @@ hipError_t lev_moe_prefill_launch(lev_ctx *ctx, const lev_moe_grouped_args &a, c
     float *dn = reinterpret_cast<float *>(s + L.dn);
     const uint32_t pairs = a.tokens * a.top_k;
     hipError_t e;
-    static bool configured = false;
-    if (!configured) {
-        for (const void *k : {reinterpret_cast<const void *>(&moe_pf_kernel<true>), reinterpret_cast<const void *>(&moe_pf_kernel<false>)}) {
-            e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)pf_lds_map::kBytes);
-            if (e != hipSuccess) return e;
-        }
-        configured = true;
-    }
     hipLaunchKernelGGL(moe_pf_group_kernel, dim3(1u + (a.tokens + 15u) / 16u), dim3(1024), (size_t)2 * a.experts * 4,
                        ctx->stream, ids, pairs, a.experts, a.top_k, glist, valid, items, nitems, ctx->d_flag, x, a.tokens,
                        a.hidden, xh, xl, xmax);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    const uint32_t slots = (uint32_t)((pf_max_items(a) + 7u) / 8u) * 8u;
-    const uint32_t tiles_gu = (a.inter + 127u) / 128u, tiles_dn = (a.hidden + 255u) / 256u;
-    hipLaunchKernelGGL((moe_pf_kernel<true>), dim3(slots * tiles_gu), dim3(kPfThreads), pf_lds_map::kBytes, ctx->stream, a,
-                       tiles_gu, xh, xl, xmax, glist, items, nitems, act);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
+    if ((e = pf_launch<true>(ctx, a, xh, xl, xmax, glist, items, nitems, act)) != hipSuccess) return e;
     // rows of act that belong to dropped pairs were never written: their planes are never read
     hipLaunchKernelGGL(moe_pf_planes_kernel, dim3((pairs + 3u) / 4u), dim3(256), 0, ctx->stream, act, pairs, a.inter, ah,
                        al, amax);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    hipLaunchKernelGGL((moe_pf_kernel<false>), dim3(slots * tiles_dn), dim3(kPfThreads), pf_lds_map::kBytes, ctx->stream, a,
-                       tiles_dn, ah, al, amax, glist, items, nitems, dn);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
+    if ((e = pf_launch<false>(ctx, a, ah, al, amax, glist, items, nitems, dn)) != hipSuccess) return e;
     return lev_moe_merge_launch(ctx, a, dn, weights, valid, y);
 }

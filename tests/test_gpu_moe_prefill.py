@@ -72,3 +72,39 @@ def test_moe_few_tokens_ragged_rows(ctx, hidden, inter, experts, top_k, tokens):
         assert O.max_rel_err(act[t], ref["act"]) < TOL
         y32, _ = O.moe_experts_f32(g, u, d, hidden, inter, ids[t], wts[t], x[t])
         assert O.max_rel_err(y[t], ref["y"]) < max(TOL, 1.5 * O.max_rel_err(y32, ref["y"]))
+
+
+@pytest.mark.parametrize("hidden,inter,experts,tokens", [
+    (1024, 512, 2, 100),          # 32 blocks a row: one chain
+    (1088, 512, 2, 100),          # 34: two parts and two blocks
+    (4096, 256, 2, 64),           # 128: eight parts, workgroups of four waves
+    (1088, 384, 128, 1200),       # workgroups of twelve waves; rows past the last whole workgroup
+    (256, 1088, 2, 260),          # down folded
+])
+def test_moe_grouped_product_folded_sums(ctx, hidden, inter, experts, tokens):
+    """The f32 sums of the grouped product against 64 bits, on positive weights and activations, where a chain's
+    partial sums grow evenly: n additions leave sqrt(n / 3) roundings u = 2^-24 / sqrt(3) of the whole (rms), 3.3 at
+    32 blocks and 6.5 at 128, parts of 16 blocks folded at most 2.0 (8 parts).  gelu is the identity here, so
+    act = g * u has sqrt(2) times that and some two roundings of its own: 5.1 u, held to 5.5; y adds its own row and
+    some two: 6.4 u, held to 7.  One chain of 128 blocks leaves 9.4 u in act."""
+    u = 2.0 ** -24 / 3 ** 0.5
+    wr, pool, offs, x = H.config5(hidden, inter, experts, tokens, seed=hidden + inter)
+    blocks = pool.reshape(-1, 18)
+    blocks[:, 1] &= 0x7F
+    blocks[:, 2:] |= 0x88
+    x = np.abs(x)
+    rng = np.random.default_rng(tokens)
+    ids = rng.permutation(np.arange(tokens) % experts).astype(np.int32)[:, None]
+    wts = np.ones((tokens, 1), np.float32)
+    y, act = run_experts(ctx, pool, offs, hidden, inter, experts, x, ids, wts)
+    g, up, d = (pool[offs["gate_off"]:], pool[offs["up_off"]:], pool[offs["down_off"]:])
+    off = {"act": [], "y": []}
+    for t in range(0, tokens, max(1, tokens // 24)):
+        ref = O.moe_experts_f64(g, up, d, hidden, inter, ids[t], wts[t], x[t])
+        for k, got in (("act", act[t]), ("y", y[t])):
+            r = np.asarray(ref[k], np.float64).ravel()
+            off[k].append((np.linalg.norm(got.astype(np.float64).ravel() - r) / np.linalg.norm(r)) ** 2)
+    act_off, y_off = (np.sqrt(np.mean(off[k])) / u for k in ("act", "y"))
+    print(f"act {act_off:.2f} u, y {y_off:.2f} u")
+    assert act_off < 5.5
+    assert y_off < 7
