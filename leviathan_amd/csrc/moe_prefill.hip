@@ -53,16 +53,17 @@ constexpr uint32_t kPfChain = 32;            // blocks of a row from which on it
 
 // ---------------------------------------------------------------------------
 // Activation planes of one row, by one wave.  The row is scaled by the power of two that brings its
-// maximum into [2^14, 2^15) (zero, denormal and non-finite maxima: no scaling) and split into fp16 high
-// and low halves; at the top of fp16's range the low half of every element down to 2^-17 of the
-// maximum is still a normal number.  Run r (eight values) of block b holds elements 8r + 0, 2, 1, 3, 4,
+// maximum into [2^14, 2^15) (2^126 at most, which makes multiples of 2^-23 of the subnormal numbers; a row
+// with a NaN or an infinity as it is: its results are not finite) and split into fp16 high and low halves;
+// at the top of fp16's range the low half of every element down to 2^-17 of the maximum is still a normal
+// number.  Run r (eight values) of block b holds elements 8r + 0, 2, 1, 3, 4,
 // 6, 5, 7: the weights of code bytes 8(r & 1) .. +7 (r < 2: low nibbles, else high ones) in the order in
 // which the masks of the matrix kernel deliver them.
 // ---------------------------------------------------------------------------
 struct pf_scale { float scale, unscale; };
 __device__ __forceinline__ pf_scale pf_row_scale(uint32_t max_bits) {
     uint32_t ex = (max_bits >> 23) & 0xFFu;                    // maximum in [2^(ex - 127), 2^(ex - 126))
-    if (ex == 0u || ex >= 254u) ex = 141u;                     // (no scaling)
+    if (ex == 255u) ex = 141u;                                 // (no scaling)
     ex = ex < 15u ? 15u : ex;                                  // keeps both powers of two normal numbers
     return pf_scale{__uint_as_float((268u - ex) << 23), __uint_as_float((ex - 14u) << 23)};   // 2^(141 - ex), 2^(ex - 141)
 }

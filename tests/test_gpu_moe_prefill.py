@@ -108,3 +108,36 @@ def test_moe_grouped_product_folded_sums(ctx, hidden, inter, experts, tokens):
     print(f"act {act_off:.2f} u, y {y_off:.2f} u")
     assert act_off < 5.5
     assert y_off < 7
+
+
+@pytest.mark.parametrize("x_exp,d_exp", [
+    (68, -24),      # act near 2^127.6: its own power of two scales it
+    (-63, 12),      # act near 2^-135, a subnormal number
+])
+def test_moe_grouped_product_range_of_act(ctx, x_exp, d_exp):
+    """Rows of act whose maximum is at either end of f32's range are operands like any other.  g = u = 7 d x[0] with
+    the gate's and the up matrix's only weights in column 0; every weight of down is 7 * 2^d_exp."""
+    hidden = inter = 320
+    experts, tokens = 2, 700
+    gu, dn = inter * hidden // 32 * 18, hidden * inter // 32 * 18
+    one = np.zeros((inter * hidden // 32, 18), np.uint8)
+    one[:, 2:] = 0x88                                                # weight zero
+    one[:, 0:2] = np.array([2.0 ** -7], np.float16).view(np.uint8)
+    one.reshape(inter, hidden // 32, 18)[:, 0, 2] = 0x8F             # element 0: 7
+    down = np.empty((hidden * inter // 32, 18), np.uint8)
+    down[:, 2:] = 0xFF
+    down[:, 0:2] = np.array([2.0 ** d_exp], np.float16).view(np.uint8)
+    pool = np.concatenate([np.tile(one.ravel(), 2 * experts), np.tile(down.ravel(), experts)])
+    offs = dict(gate_off=0, up_off=experts * gu, down_off=2 * experts * gu, gate_stride=gu, up_stride=gu, down_stride=dn)
+    x = np.zeros((tokens, hidden), np.float32)
+    x[:, 0] = np.ldexp(1.0 + np.arange(tokens) / 8192.0, x_exp)
+    ids = (np.arange(tokens) % experts).astype(np.int32)[:, None]
+    y, act = run_experts(ctx, pool, offs, hidden, inter, experts, x, ids, np.ones((tokens, 1), np.float32))
+    g = 7 * 2.0 ** -7 * x[:, :1].astype(np.float64)
+    want = (g if x_exp > 0 else 0.5 * g) * g
+    quantum = 2.0 ** -149
+    assert np.all(np.abs(act[:, 0] - want) <= 1e-6 * want + quantum)
+    # against the act that was stored, whose subnormal numbers have fewer bits
+    y_want = act[:, 0].astype(np.float64).sum(axis=1, keepdims=True) * 7 * 2.0 ** d_exp
+    assert np.all(np.isfinite(y)) and np.all(y > 0)
+    assert np.all(np.abs(y - y_want) <= 1e-6 * y_want)
