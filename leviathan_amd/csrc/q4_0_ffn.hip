@@ -126,6 +126,26 @@ q4_0_ffn_gate_up(ffn_args a) {
     }
 }
 
+struct span {
+    uintptr_t at;
+    size_t bytes;
+    template <typename T>
+    span(const T *p, size_t n) : at(reinterpret_cast<uintptr_t>(p)), bytes(p ? n : 0u) {}
+    bool meets(const span &o) const { return at < o.at + o.bytes && o.at < at + bytes; }
+};
+
+// Whether the first three stages may run at the same time: every workgroup reads all of x, the norm and its own rows
+// of the weights while others already write h, gu and act, which the operators one by one only do when all readers are
+// through.  act may be one of the halves of gu, whose value a lane replaces with its own.
+bool ffn_apart(const ffn_args &a, size_t gate_bytes, size_t up_bytes) {
+    const size_t nh = (size_t)a.hidden * 4u, ni = (size_t)a.inter * 4u;
+    const span in[] = {{a.x, nh}, {a.gain, nh}, {a.gate, gate_bytes}, {a.up, up_bytes}};
+    const span h(a.h, nh), gu(a.gu, 2u * ni), act(a.act, ni);
+    for (const span &i : in)
+        if (i.meets(h) || i.meets(gu) || i.meets(act)) return false;
+    return !h.meets(gu) && !h.meets(act) && (!act.meets(gu) || a.act == a.gu || a.act == a.gu + a.inter);
+}
+
 }  // namespace
 
 extern "C" int lev_hip_shared_expert_ffn_q4_0(lev_ctx *ctx, const float *d_x, const float *d_ffn_norm, const void *d_gate_w,
@@ -148,14 +168,15 @@ extern "C" int lev_hip_shared_expert_ffn_q4_0(lev_ctx *ctx, const float *d_x, co
     if (st != LEV_OK) return st;
     const uintptr_t al4 = reinterpret_cast<uintptr_t>(d_gate_w) | reinterpret_cast<uintptr_t>(d_up_w);
     const uintptr_t al16 = reinterpret_cast<uintptr_t>(d_x) | reinterpret_cast<uintptr_t>(d_h) | reinterpret_cast<uintptr_t>(d_ffn_norm);
+    ffn_args a = {static_cast<const uint8_t *>(d_gate_w), static_cast<const uint8_t *>(d_up_w), d_x, d_ffn_norm, d_h,
+                  d_gu, d_act, hidden, inter, 0u, eps};
     // A schedule installed for the gate/up GEMV keeps the operators apart, so that it is the one that runs.
-    const bool fused = hidden % 64u == 0u && hidden <= 4096u && (al4 & 3u) == 0u && (al16 & 15u) == 0u && d_x != d_h &&
-                       !lev_selected(ctx, LEV_OP_Q4_0_GEMV, hidden, inter, 1);
+    const bool fused = hidden % 64u == 0u && hidden <= 4096u && (al4 & 3u) == 0u && (al16 & 15u) == 0u &&
+                       ffn_apart(a, gate_bytes, up_bytes) && !lev_selected(ctx, LEV_OP_Q4_0_GEMV, hidden, inter, 1);
     if (fused) {
         const uint32_t cus = (uint32_t)ctx->num_cus, per = (inter + 16u * cus - 1u) / (16u * cus);
         const uint32_t rows = per == 1u ? (inter + cus - 1u) / cus : (inter + 16u * cus - 1u) / (16u * cus) * 16u;
-        const ffn_args a = {static_cast<const uint8_t *>(d_gate_w), static_cast<const uint8_t *>(d_up_w), d_x, d_ffn_norm, d_h,
-                            d_gu, d_act, hidden, inter, rows, eps};
+        a.rows_per_block = rows;
         const dim3 grid((inter + rows - 1u) / rows);
 #define LEV_FFN(NW) hipLaunchKernelGGL((q4_0_ffn_gate_up<NW>), grid, dim3(NW * LEV_WAVE), ffn_lds(NW), ctx->stream, a)
         if (hidden <= 2048u) LEV_FFN(8);

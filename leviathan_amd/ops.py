@@ -205,7 +205,8 @@ class Context:
         """The shared expert that runs beside the routed ones (Gemma4.swift:3742-3773):
         h = rmsnorm(x, ffn_norm); gu = [gate h | up h] (Q4_0 matvecs, up at float offset
         `inter` of the one buffer); act = gelu_up(gu); shared = rmsnorm(down act, post_norm).
-        `bufs` = (h, gu, act, shared) to reuse buffers (a recorded program needs fixed ones).
+        `bufs` = (h, gu, act, shared) to reuse buffers (a recorded program needs fixed ones); they may share
+        memory with each other and with x where the operators one after the other allow it.
         Returns (h, shared): h also feeds the routed experts."""
         if inter % 32 or hidden % 32 or (inter * 4) % 256:
             raise LevError(capi.BAD_DIMENSIONS,

@@ -38,3 +38,54 @@ def test_shared_ffn_shapes(hidden, inter, norms):
     ref = O.rmsnorm_f64(O.q4_0_matvec_f64(down, hidden, inter, act).astype(np.float32), pn, 1e-6)
     assert O.max_rel_err(shared.cpu().numpy(), ref) < 1e-4
     ctx.close()
+
+
+# name: offsets in floats, in one buffer, of x, h, gu, act and shared at hidden 2048, inter 1024
+OVERLAPS = {
+    "apart": (0, 2048, 4096, 6144, 7168),
+    "act over x": (0, 2048, 4096, 1024, 7168),
+    "act over h": (0, 2048, 4096, 2064, 7168),
+    "act over gu": (0, 2048, 4096, 4096, 7168),
+    "act over the up half": (0, 2048, 4096, 5120, 7168),
+    "gu over x": (0, 4096, 0, 6144, 7168),
+    "gu over a part of x": (0, 4096, 1984, 6144, 7168),
+    "h over x": (0, 0, 4096, 6144, 7168),
+    "h over a part of x": (0, 1024, 4096, 6144, 7168),
+    "shared over x and h": (0, 2048, 4096, 6144, 1024),
+}
+
+
+@pytest.mark.parametrize("name", OVERLAPS)
+def test_shared_ffn_buffers_that_overlap(name):
+    """Buffers that share memory, as far as the operators one after the other allow it, give what those give: the same
+    bits of `shared`, and of h where nothing is written over it."""
+    from leviathan_amd import ops
+    ctx = ops.Context(0)
+    hidden, inter = 2048, 1024
+    gate, up = (dev(O.synth_q4_0(s, inter * hidden // 32, 0.02)) for s in (1, 2))
+    down = dev(O.synth_q4_0(3, hidden * inter // 32, 0.02))
+    x0 = O.normal(hidden, 4)
+    fn, pn = (dev(O.normal(hidden, s, 1.0, 0.1)) for s in (5, 6))
+    sizes = (hidden, hidden, 2 * inter, inter, hidden)
+
+    def buffers():
+        pool = torch.full((9216,), float("nan"), device="cuda")
+        parts = [pool[o:o + n] for o, n in zip(OVERLAPS[name], sizes)]
+        parts[0].copy_(dev(x0))
+        return parts
+    x, h, gu, act, shared = buffers()
+    ctx.rmsnorm(x, hidden, 1, weight=fn, y=h)
+    want_h = h.clone()
+    ctx.q4_0_gemv(gate, h, hidden, inter, y=gu)
+    ctx.q4_0_gemv(up, h, hidden, inter, y=gu[inter:])
+    ctx.gelu_up(gu, inter, y=act)
+    ctx.q4_0_gemv(down, act, inter, hidden, y=shared)
+    ctx.rmsnorm(shared, hidden, 1, weight=pn, y=shared)
+    want = shared.clone()
+    for _ in range(4):
+        x, h, gu, act, shared = buffers()
+        ctx.shared_expert_ffn(x, fn, gate, up, down, pn, hidden, inter, bufs=(h, gu, act, shared))
+        assert torch.equal(shared, want)
+        if name not in ("act over h", "shared over x and h"):
+            assert torch.equal(h, want_h)
+    ctx.close()
