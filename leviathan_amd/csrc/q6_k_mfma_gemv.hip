@@ -1475,7 +1475,7 @@ namespace {
 // eight more for its latency (4096 x 12288: three slices of sixteen are 85 workgroups each and four rounds, four of
 // twelve are 64 and four shorter rounds).
 struct q6m_slices {
-    uint32_t slices, wpr, slots, blocks;
+    uint32_t slices, wpr, slots, blocks, rounds;
 };
 q6m_slices q6m_q8_one_grid(const lev_ctx *ctx, uint32_t cols, uint32_t rows, uint32_t waves) {
     const uint32_t SB = cols >> 8, ngroups = (rows + 15u) / 16u, cus = (uint32_t)ctx->num_cus;
@@ -1488,10 +1488,37 @@ q6m_slices q6m_q8_one_grid(const lev_ctx *ctx, uint32_t cols, uint32_t rows, uin
         uint32_t room = cus / sl;
         room = room < 1u ? 1u : room > lev_ctx::kSliceTickets ? lev_ctx::kSliceTickets : room;
         const uint32_t blocks = nrounds < room ? nrounds : room;
-        const uint32_t cost = (nrounds + blocks - 1u) / blocks * (wpr * slots + 8u);
-        if (cost < best_cost) best_cost = cost, best = q6m_slices{sl, wpr, slots, blocks};
+        const uint32_t rounds = (nrounds + blocks - 1u) / blocks, cost = rounds * (wpr * slots + 8u);
+        if (cost < best_cost) best_cost = cost, best = q6m_slices{sl, wpr, slots, blocks, rounds};
     }
     return best;
+}
+
+// Whether a row that does not fit a workgroup's waves is better left to the kernel that stages the activations of the
+// `held` columns its LDS has room for: from times of both over 2304 to 16384 columns, 1000 to 64000 rows and one to
+// sixteen columns (us, 624 shapes, by the columns a kernel is built for: 4, 8 and 16).  In slices a round takes some
+// time whatever it multiplies, and every slice but one is a value a row and column more that goes to memory and
+// back; staged, the weights are read again for every `held` columns.  4096 x 32000 by sixteen columns 46.3 us in slices,
+// 32.6 staged; 4352 x 16000 by eight 28.4 and 21.1; 5120 x 16000 by eight 25.8 and 22.0; 12288 x 4096 by sixteen 28.5 and
+// 54.6.  Left to the staging kernel where the estimates differ by 4 % and more: of the shapes measured the worst that
+// moves loses 2.6 %, the worst that stays would gain 8 %.
+bool q6m_q8_staged_is_faster(const lev_ctx *ctx, const q6m_slices &g, uint32_t cols, uint32_t rows, uint32_t ncol,
+                             uint32_t held) {
+    // a launch, a round of row groups, a wave (sliced) or a task of the wave (staged) in it, 10^6 values of the sums that
+    // the slices exchange (sliced) or of y (staged), 10^6 weights
+    struct cost { double start, round, part, mvalue, mweight; };
+    constexpr cost sliced_by[3] = {{5.5, 0.2, 0.034, 15.0, 0.104}, {6.6, 0.37, 0.078, 12.7, 0.066}, {6.4, 1.0, 0.095, 18.0, 0.03}};
+    constexpr cost staged_by[3] = {{7.7, -0.1, 1.07, 7.6, 0.071}, {7.0, 0.68, 1.38, 13.0, 0.058}, {5.9, 2.44, 2.14, 0.9, 0.065}};
+    auto kind = [](uint32_t n) { return n > 8u ? 2 : n > 4u ? 1 : 0; };
+    const cost &k = sliced_by[kind(ncol)], &t = staged_by[kind(ncol < held ? ncol : held)];
+    const uint32_t SB = cols >> 8, cus = (uint32_t)ctx->num_cus;
+    const uint32_t S = q6m_waves_per_group(ctx, cols, rows), slots = (uint32_t)kQWaves / S;
+    const uint32_t groups = ((rows + 15u) / 16u + slots - 1u) / slots;
+    const double rounds = (groups + cus - 1u) / cus, tasks = (SB + S - 1u) / S, passes = (ncol + held - 1u) / held;
+    const double mvalues = 1e-6 * ncol * rows, mweights = 1e-6 * cols * rows;
+    const double sliced = k.start + g.rounds * (k.round + k.part * g.wpr * g.slots) + k.mvalue * (g.slices - 1u) * mvalues + k.mweight * mweights;
+    const double staged = passes * (t.start + rounds * (t.round + t.part * tasks) + t.mweight * mweights) + t.mvalue * mvalues;
+    return staged < 0.96 * sliced;
 }
 
 // hipErrorOutOfMemory: the scratch cannot be had (a program is being recorded and the context's is still too small).
@@ -1523,6 +1550,8 @@ template <int NC>
 hipError_t q6m_q8_one_launch(lev_ctx *ctx, const uint8_t *w, const uint32_t *xq, const float *xs, float *y,
                              uint32_t cols, uint32_t rows, uint32_t ncol) {
     const q6m_slices g = q6m_q8_one_grid(ctx, cols, rows, (uint32_t)q6m_q8_one_waves(NC));
+    const uint32_t held = lev_q6_k_mfma_q8_cols(ctx, cols);
+    if (g.slices > 1u && held && q6m_q8_staged_is_faster(ctx, g, cols, rows, ncol, held)) return hipErrorNotSupported;
     if (g.slices > 1u) return q6m_q8_one_launch_grid<NC, true>(ctx, w, xq, xs, y, cols, rows, ncol, g);
     return q6m_q8_one_launch_grid<NC, false>(ctx, w, xq, xs, y, cols, rows, ncol, g);
 }

@@ -38,3 +38,11 @@ def test_q6_q8_sliced_rows(blocks, rows, ncol):
         ref = O.q6_k_matvec_q8_f64(ww, len(pick), cols, xq[c], d[c])
         assert np.allclose(outs[0][c][pick], ref, rtol=1e-4, atol=1e-4 * np.abs(ref).max() + 1e-6), (blocks, rows, ncol, c)
     ctx.close()
+
+
+@pytest.mark.parametrize("ncol", [4, 9, 16])
+@pytest.mark.parametrize("blocks,rows", [(10, 4096), (10, 12288), (17, 4096), (17, 16016), (18, 2064)])
+def test_q6_q8_sliced_or_staged(blocks, rows, ncol):
+    """Either side of the line from which wide rows are left to the kernel that stages the activations: by rows, by
+    columns, and by width where it no longer holds sixteen columns in one pass."""
+    test_q6_q8_sliced_rows(blocks, rows, ncol)
