@@ -859,7 +859,21 @@ q6_k_mfma_gemv_one(const uint8_t *__restrict__ w, const float *__restrict__ x, c
         while (step(Wa, Wc) && step(Wb, Wa) && step(Wc, Wb)) {
         }
     } else {
-        while (step(Wa, Wb) && step(Wb, Wa)) {
+        while (true) {
+            uint32_t next = rb + gridDim.x;
+            __builtin_amdgcn_sched_barrier(0);
+            issue(next < nrounds ? next : rb, Wb);
+            __builtin_amdgcn_sched_barrier(0);
+            finish(Wa);
+            if (next >= nrounds) break;
+            rb = next;
+            next = rb + gridDim.x;
+            __builtin_amdgcn_sched_barrier(0);
+            issue(next < nrounds ? next : rb, Wa);
+            __builtin_amdgcn_sched_barrier(0);
+            finish(Wb);
+            if (next >= nrounds) break;
+            rb = next;
         }
     }
     if (NC == 1 && partials) q6m_greedy_token(best, slots, partials, tickets, out_idx, out_margin);
