@@ -68,6 +68,15 @@ q4_0_mfma_gemv(const uint8_t *__restrict__ w, const float *__restrict__ x, float
     const uint8_t *const w_end = w + rows * row_bytes;
     const uint32_t ngroups = (nrows + 15u) >> 4;
     const uint32_t lrow = lane >> 2;                             // fetch order: lane = 4 * row + pair
+    // bytes of a row in front of the lane's pair, past the row's end its last one, once for all rounds (8192 x 8192 10.53
+    // us with the clamp in every round, 10.45 without; 20000 x 5120 12.99 and 12.84)
+    uint32_t at[TPW];
+#pragma unroll
+    for (int t = 0; t < TPW; ++t) {
+        const uint32_t T = t_first + t < ntask ? t_first + t : ntask - 1u, pair = 4u * T + (lane & 3u);
+        at[t] = (pair < npairs ? pair : npairs - 1u) * 36u;
+        if (!SINGLE) lev_pin(at[t]);
+    }
     auto issue = [&](uint32_t round_block, uint32_t (&D)[TPW][9]) {
         uint32_t rg = round_block * slots + (active ? slot : 0u);
         rg = rg < ngroups ? rg : ngroups - 1u;
@@ -80,7 +89,7 @@ q4_0_mfma_gemv(const uint8_t *__restrict__ w, const float *__restrict__ x, float
             if (ODD)
                 q4m_load_task_odd(rowp, 4u * T, npairs, w_end, D[t]);
             else
-                q4m_load_task_part(rowp, 4u * T, npairs, D[t]);
+                lev_q4_load_pair(rowp + at[t], D[t]);
         }
     };
     uint32_t Da[TPW][9];
