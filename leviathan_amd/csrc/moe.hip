@@ -18,6 +18,7 @@
 //      workgroup's tile of outputs; partial results meet in LDS and are merged
 //      IN SLOT ORDER in f32, as the reference's axpy chain does.
 #include "moe_grouped.hpp"
+#include "moe_split.hpp"
 #include "q4_0_mfma.hpp"
 
 namespace {
@@ -1449,18 +1450,7 @@ void launch_gate_up_as(lev_ctx *ctx, const moe_args &a, const float *x, const gu
 
 hipError_t launch_gate_up_mfma(lev_ctx *ctx, const moe_args &a, const float *x, const gu_route &rt,
                                float *act, uint32_t tokens, uint32_t per_cu) {
-    // A group is 16 rows.  `most` workgroups of one group fit a CU at once: while three rounds of them hold all rows, a
-    // workgroup takes one group, as small as the same number of workgroups a CU allows (3968 / 1472, top-6, one token:
-    // 18 rows a workgroup are two groups, the second of two rows); beyond, several whole groups with the next one's
-    // weights in flight.  per_cu: at least that many workgroups a CU (a schedule's field; built in: 2).
-    const uint64_t rows = (uint64_t)a.inter * a.top_k * tokens, cus = (uint64_t)ctx->num_cus;
-    const uint64_t most = a.hidden <= 2048u ? 4u : 2u;
-    uint64_t per = (rows + 16u * cus - 1) / (16u * cus);                          // groups a CU
-    if (per > most) per = (per + most - 1) / most * most;                         // whole rounds
-    if (per < per_cu) per = per_cu;
-    const uint64_t want = per <= 3u * most && (most == 2u || per <= most) ? (rows + per * cus - 1) / (per * cus)
-                                                                          : 16u * ((rows + 32u * cus - 1) / (32u * cus));
-    const uint32_t rows_per_block = want < a.inter ? (uint32_t)want : a.inter;
+    const uint32_t rows_per_block = moe_gate_up_rows(ctx->num_cus, a.hidden, a.inter, a.top_k * tokens, per_cu);
     const uint32_t chunks = (a.inter + rows_per_block - 1) / rows_per_block;
     const uint32_t route = rt.ids ? 0u : a.experts <= 128u ? 2u : 4u;      // callers keep experts <= kRouteInKernelMax
     const dim3 grid(chunks, a.top_k, tokens);
@@ -1554,7 +1544,7 @@ bool experts_fast(const moe_args &a, const float *x) {
 // fast path: callers test experts_fast() first.
 hipError_t run_experts(lev_ctx *ctx, const moe_args &a, const float *x, const gu_route &rt,
                        const int32_t *ids, const float *weights, float *y, float *act,
-                       uint32_t tokens, bool fast, uint32_t gu_per_cu = 2u, bool matrix_cores = true) {
+                       uint32_t tokens, bool fast, uint32_t gu_per_cu = kGateUpPerCu, bool matrix_cores = true) {
     hipError_t e;
     if (!fast) {
         hipLaunchKernelGGL(moe_gate_up_generic, dim3((a.inter + 3) / 4, a.top_k, tokens), dim3(256), 0,
@@ -1803,7 +1793,7 @@ int moe_layer_impl(lev_ctx *ctx, const lev_moe_experts *pools, const float *d_ro
     const lev_schedule *sel = tokens <= 4u ? lev_selected(ctx, LEV_OP_MOE_LAYER_Q4_0, a.hidden, a.inter, tokens)
                                            : nullptr;
     const uint32_t family = sel ? sel->family : 1u;
-    const uint32_t gu_per_cu = sel && sel->rows_in_flight ? sel->rows_in_flight : 2u;
+    const uint32_t gu_per_cu = sel && sel->rows_in_flight ? sel->rows_in_flight : kGateUpPerCu;
     const bool matrix_cores = !(sel && sel->persistent);   // schedule field `persistent` = 1: the vector-ALU expert kernels
     const bool few = !grouped && selects_itself(a, d_x, tokens);
     if (few && family == 2u) {
@@ -1848,7 +1838,7 @@ int moe_layer_impl(lev_ctx *ctx, const lev_moe_experts *pools, const float *d_ro
 // lowered layer the same way): who selects the experts (family 1: the gate/up
 // workgroups themselves, the built-in choice; 2: the last workgroup of the router
 // kernel to finish; 0: a top-k kernel of its own, one launch more) and how many
-// gate/up workgroups per CU the rows are cut into.  On MI355X the hand-over inside
+// gate/up workgroups per CU the rows are cut into (2: as the built-in rule has it, moe_gate_up_rows).  On MI355X the hand-over inside
 // the router kernel (a fence and an arrival counter over 16 workgroups) costs as
 // much as the launch it saves: 18.8 us a layer against 15.9 and 18.9.  Every candidate computes each row with the same lanes in the same order:
 // their outputs agree bit for bit.  (Shapes the streaming kernels cannot take run
@@ -1869,8 +1859,8 @@ uint32_t lev_moe_layer_candidates(const lev_ctx *ctx, uint32_t hidden, uint32_t 
     add(1u, 4u);
     add(2u, 2u);
     add(0u, 2u);
-    // the expert kernels on the vector ALU (f32 FMA chains) instead of the integer matrix cores, the
-    // built-in choice wherever rows are whole 256-value tasks: same routing, sums rounded differently
+    // the expert kernels on the vector ALU (f32 FMA chains) instead of the integer matrix cores, the built-in choice
+    // wherever rows are whole block pairs (gate_up_mfma_ok, down_mfma_ok): same routing, sums rounded differently
     if (n < capacity) out[n] = lev_schedule{LEV_OP_MOE_LAYER_Q4_0, 1u, 2u, 1u};
     ++n;
     return n;
