@@ -335,13 +335,7 @@ template <typename W, int T, int RW, int KW>
 hipError_t launch_as(lev_ctx *ctx, const uint8_t *w, const uint16_t *x, float *out, uint32_t in_dim, uint32_t rows,
                      uint32_t tokens, uint32_t tok_tiles, uint32_t splits) {
     constexpr size_t lds = (size_t)KW * x_bufs<W>(T, RW, KW) * T * kTile + RW * KW * W::kArea;
-    static bool configured = false;
-    if (!configured && lds > 48 * 1024) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_split_kernel<W, T, RW, KW>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-        configured = true;
-    }
+    if (hipError_t e = lev_allow_lds(ctx, reinterpret_cast<const void *>(&gemm_split_kernel<W, T, RW, KW>), lds); e != hipSuccess) return e;
     const uint32_t row_tiles = (rows + RW * 32u - 1u) / (RW * 32u);
     hipLaunchKernelGGL((gemm_split_kernel<W, T, RW, KW>), dim3((row_tiles * tok_tiles * splits + 7u) / 8u * 8u),
                        dim3(RW * KW * 64), lds, ctx->stream, w, x, out, in_dim, rows, tokens, row_tiles, tok_tiles, splits);

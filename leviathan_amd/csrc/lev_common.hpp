@@ -68,6 +68,10 @@ struct lev_ctx {
     // Device address, on this context's GPU, of the static scratch array of
     // lev_hip_moe_layer_q4_0_noalloc (looked up once at context creation).
     void *moe_static_scratch = nullptr;
+    // Kernels whose dynamic LDS limit has been raised on this context's device (lev_allow_lds).
+    static constexpr size_t kLargeLds = 160;
+    const void *large_lds[kLargeLds];
+    size_t large_lds_count = 0;
 };
 
 // Looks the static MoE scratch array up on the current device (moe.hip).
@@ -83,6 +87,23 @@ void *lev_scratch(lev_ctx *ctx, size_t bytes);
 // Zero-fills `bytes` (a multiple of 4) with a small kernel on the context's
 // stream (safe to record into a HIP graph, unlike a memset node).
 hipError_t lev_zero_async(lev_ctx *ctx, void *d_ptr, size_t bytes);
+
+// Lets `kernel` be launched with `bytes` of dynamic LDS.  The attribute belongs to the current device, which is the
+// context's, and that it is raised is remembered with the context (one thread uses a context at a time).  It is raised
+// to all the device has, so that two contexts on one device never lower it for each other.
+inline hipError_t lev_allow_lds(lev_ctx *ctx, const void *kernel, size_t bytes) {
+    if (bytes <= 48u * 1024u) return hipSuccess;
+    for (size_t i = 0; i < ctx->large_lds_count; ++i)
+        if (ctx->large_lds[i] == kernel) return hipSuccess;
+    hipFuncAttributes own;
+    hipError_t e = hipFuncGetAttributes(&own, kernel);
+    if (e != hipSuccess) return e;
+    constexpr size_t kAll = 160u * 1024u;
+    if (bytes + own.sharedSizeBytes > kAll) return hipErrorInvalidValue;
+    e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(kAll - own.sharedSizeBytes));
+    if (e == hipSuccess && ctx->large_lds_count < lev_ctx::kLargeLds) ctx->large_lds[ctx->large_lds_count++] = kernel;
+    return e;
+}
 
 #define LEV_REQUIRE_CTX(ctx)                         \
     do {                                             \

@@ -1420,11 +1420,7 @@ hipError_t launch_down(lev_ctx *ctx, const moe_args &a, const float *act, const 
     uint32_t tiles = (a.hidden + tile - 1) / tile;
     size_t lds = (size_t)kDnWaves * 16 * (a.inter / 64u + 1u) * sizeof(lev_f32x4) +
                  (size_t)a.top_k * (tile + 1u) * sizeof(float);
-    if (lds > 48 * 1024) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&moe_down_kernel<L>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-    }
+    if (hipError_t e = lev_allow_lds(ctx, reinterpret_cast<const void *>(&moe_down_kernel<L>), lds); e != hipSuccess) return e;
     hipLaunchKernelGGL((moe_down_kernel<L>), dim3(tiles, tokens), dim3(kDnThreads), lds, ctx->stream,
                        a, act, ids, weights, y, ctx->d_flag, steps);
     return hipGetLastError();
@@ -1678,9 +1674,7 @@ hipError_t run_topk(lev_ctx *ctx, float *scores, const double *partials, const f
     else if (experts <= 256u) LEV_TOPK(4);
     else if (experts <= 1024u) LEV_TOPK(16);
     else {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&moe_topk_kernel<64>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           (int)router_lds_bytes(64));
+        hipError_t e = lev_allow_lds(ctx, reinterpret_cast<const void *>(&moe_topk_kernel<64>), router_lds_bytes(64));
         if (e != hipSuccess) return e;
         LEV_TOPK(64);
     }

@@ -656,13 +656,7 @@ hipError_t g8_launch_as(lev_ctx *ctx, const lev_moe_grouped_args &a, const g8_ge
     uint64_t slot_of_wave, pos_of_wave;
     lev_wave_tables(q.wpr, &slot_of_wave, &pos_of_wave);
     constexpr size_t lds = g8_lds<NTILE, NW>();
-    static bool configured = false;   // per instantiation: raise the dynamic LDS limit once
-    if (!configured) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&moe_grouped_i8_kernel<NTILE, PAIRED, NW>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-        configured = true;
-    }
+    if (hipError_t e = lev_allow_lds(ctx, reinterpret_cast<const void *>(&moe_grouped_i8_kernel<NTILE, PAIRED, NW>), lds); e != hipSuccess) return e;
     hipLaunchKernelGGL((moe_grouped_i8_kernel<NTILE, PAIRED, NW>), dim3(grid), dim3(64u * q.wpr * q.slots), lds,
                        ctx->stream, a, src, items, starts, out, q.wpr, q.slots, q.rpi, slot_of_wave, pos_of_wave);
     return hipGetLastError();
@@ -744,13 +738,7 @@ hipError_t lev_moe_grouped_launch(lev_ctx *ctx, const lev_moe_grouped_args &a, c
     }();
     const uint32_t w1 = cut[0], w2 = cut[1], s0_gu = cut[2], w1_dn = cut[3], w2_dn = cut[4], s0_dn = cut[5];
     const size_t lds_group = (size_t)5 * a.experts * 4;
-    static size_t lds_group_set = 0;
-    if (lds_group > 48 * 1024 && lds_group > lds_group_set) {
-        e = hipFuncSetAttribute(reinterpret_cast<const void *>(&moe_group_kernel),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_group);
-        if (e != hipSuccess) return e;
-        lds_group_set = lds_group;
-    }
+    if ((e = lev_allow_lds(ctx, reinterpret_cast<const void *>(&moe_group_kernel), lds_group)) != hipSuccess) return e;
     hipLaunchKernelGGL(moe_group_kernel, dim3(1), dim3(1024), lds_group, ctx->stream, ids, pairs,
                        a.experts, a.top_k, valid, ctx->d_flag, items, starts, grid, q_gu.rpi, q_dn.rpi, w1, w2, w1_dn, w2_dn,
                        s0_gu, s0_dn);

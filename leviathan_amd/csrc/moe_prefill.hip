@@ -490,13 +490,9 @@ pf_layout pf_layout_of(const lev_moe_grouped_args &a) {
 template <bool PAIRED, uint32_t WAVES, bool FOLD>
 hipError_t pf_launch_as(lev_ctx *ctx, const lev_moe_grouped_args &a, const _Float16 *ph, const _Float16 *pl, const uint32_t *pmax,
                         const int32_t *glist, const lev_pf_item *items, const uint32_t *nitems, float *out) {
-    const void *kernel = reinterpret_cast<const void *>(&moe_pf_kernel<PAIRED, WAVES, FOLD>);
-    static bool configured = false;
-    if (!configured) {
-        hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)pf_lds_map<WAVES>::kBytes);
-        if (e != hipSuccess) return e;
-        configured = true;
-    }
+    if (hipError_t e = lev_allow_lds(ctx, reinterpret_cast<const void *>(&moe_pf_kernel<PAIRED, WAVES, FOLD>), pf_lds_map<WAVES>::kBytes);
+        e != hipSuccess)
+        return e;
     const uint32_t slots = (uint32_t)((pf_max_items(a) + 7u) / 8u) * 8u;
     const uint32_t rows = PAIRED ? a.inter : a.hidden, per_wg = WAVES * (PAIRED ? 16u : 32u), tiles = (rows + per_wg - 1u) / per_wg;
     hipLaunchKernelGGL((moe_pf_kernel<PAIRED, WAVES, FOLD>), dim3(slots * tiles), dim3(WAVES * 64u), pf_lds_map<WAVES>::kBytes,

@@ -256,11 +256,7 @@ hipError_t launch_pairs(lev_ctx *ctx, const uint8_t *w, const float *x, float *y
     uint32_t cap = (uint32_t)ctx->num_cus * lev_q4_gemv_wg_per_cu();
     if (blocks > cap) blocks = cap;
     size_t lds = (size_t)16 * (pairs + 1) * sizeof(lev_f32x4) + (size_t)2 * pairs * sizeof(float);
-    if (lds > 48 * 1024) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&q4_0_gemv_pairs<L, R, MULTI, NS>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-    }
+    if (hipError_t e = lev_allow_lds(ctx, reinterpret_cast<const void *>(&q4_0_gemv_pairs<L, R, MULTI, NS>), lds); e != hipSuccess) return e;
     hipLaunchKernelGGL((q4_0_gemv_pairs<L, R, MULTI, NS>), dim3(blocks), dim3(kThreads), lds, ctx->stream, w, x,
                        y, pairs, rows);
     return hipGetLastError();

@@ -207,11 +207,7 @@ hipError_t launch_grid(lev_ctx *ctx, const uint8_t *w, const float *x, float *y,
     constexpr size_t lds = q4m_gemv_lds(TPW);
     uint64_t slot_of_wave, pos_of_wave;
     lev_wave_tables(wpr, &slot_of_wave, &pos_of_wave);
-    if (lds > 48 * 1024) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&q4_0_mfma_gemv<TPW, SINGLE, ODD>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-    }
+    if (hipError_t e = lev_allow_lds(ctx, reinterpret_cast<const void *>(&q4_0_mfma_gemv<TPW, SINGLE, ODD>), lds); e != hipSuccess) return e;
     hipLaunchKernelGGL((q4_0_mfma_gemv<TPW, SINGLE, ODD>), dim3(blocks), dim3(slots * wpr * LEV_WAVE), lds, ctx->stream, w, x, y,
                        in_dim, rows, wpr, slots, slot_of_wave, pos_of_wave);
     return hipGetLastError();

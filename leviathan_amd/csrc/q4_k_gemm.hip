@@ -278,14 +278,8 @@ hipError_t lev_q4_k_gemm_launch(lev_ctx *ctx, const uint8_t *w, const uint16_t *
                                 uint32_t in_dim, uint32_t rows, uint32_t tokens) {
     const lev_gemm_split_plan plan = lev_gemm_split_choose(ctx, false, in_dim, rows, tokens, kSBN);
     if (plan.kw) return lev_gemm_split_launch(ctx, false, w, x, y, in_dim, rows, tokens, plan);
-    static bool attr_set = false;
     const size_t lds = (size_t)kXBufs * kXBuf + 2 * kBBuf;
-    if (!attr_set) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&q4_k_gemm_kernel),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-        attr_set = true;
-    }
+    if (hipError_t e = lev_allow_lds(ctx, reinterpret_cast<const void *>(&q4_k_gemm_kernel), lds); e != hipSuccess) return e;
     dim3 grid((rows + kSBN - 1) / kSBN, (tokens + kBM - 1) / kBM);
     hipLaunchKernelGGL(q4_k_gemm_kernel, grid, dim3(kSThreads), lds, ctx->stream, w, x, y, in_dim,
                        rows, tokens);

@@ -283,12 +283,7 @@ hipError_t launch_ncol(lev_ctx *ctx, const uint8_t *w, const float *x, const flo
     constexpr uint32_t rows_per_tile = kWaves * (LEV_WAVE / L);
     uint32_t blocks = (rows + rows_per_tile - 1) / rows_per_tile;
     size_t lds = (size_t)NC * 16 * (units + 1) * sizeof(lev_f32x4);
-    if (lds > 48 * 1024) {
-        hipError_t e = hipFuncSetAttribute(
-            reinterpret_cast<const void *>(&q4_k_gemv_ncol<NC, L, RESIDENT>),
-            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-    }
+    if (hipError_t e = lev_allow_lds(ctx, reinterpret_cast<const void *>(&q4_k_gemv_ncol<NC, L, RESIDENT>), lds); e != hipSuccess) return e;
     // persistent grid: exactly the workgroups that are resident at once (a grid
     // larger than that runs its surplus as a second, mostly idle round)
     int resident = 0;

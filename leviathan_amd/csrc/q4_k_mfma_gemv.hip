@@ -1064,13 +1064,7 @@ hipError_t launch_mfma_variant(lev_ctx *ctx, const uint8_t *w, const float *x, c
                        float *y, uint32_t cols, uint32_t rows, uint32_t ncol) {
     const uint32_t pb = q4k_mfma_lds_bytes(cols, NC, 2u) <= q4k_lds_limit(ctx) ? 2u : 1u;
     const size_t lds = q4k_mfma_lds_bytes(cols, NC, pb);
-    static size_t configured = 0;   // per instantiation: raise the dynamic LDS limit once per size
-    if (lds > 48 * 1024 && lds > configured) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&q4_k_mfma_gemv<NC, SHORT>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-        configured = lds;
-    }
+    if (hipError_t e = lev_allow_lds(ctx, reinterpret_cast<const void *>(&q4_k_mfma_gemv<NC, SHORT>), lds); e != hipSuccess) return e;
     uint32_t groups = (rows + 15u) / 16u;
     uint32_t blocks = groups < (uint32_t)ctx->num_cus ? groups : (uint32_t)ctx->num_cus;
     hipLaunchKernelGGL((q4_k_mfma_gemv<NC, SHORT>), dim3(blocks), dim3(kMThreads), lds, ctx->stream, w,
@@ -1182,13 +1176,7 @@ hipError_t launch_narrow_variant(lev_ctx *ctx, const uint8_t *w, const float *x,
                                  float *y, uint32_t cols, uint32_t rows, uint32_t ncol) {
     const uint32_t pb = q4k_narrow_lds_bytes(cols, NC, 2u) <= q4k_lds_limit(ctx) ? 2u : 1u;
     const size_t lds = q4k_narrow_lds_bytes(cols, NC, pb);
-    static size_t configured = 0;   // per instantiation: raise the dynamic LDS limit once per size
-    if (lds > 48 * 1024 && lds > configured) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&q4_k_mfma_gemv_narrow<NC, SHORT>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-        configured = lds;
-    }
+    if (hipError_t e = lev_allow_lds(ctx, reinterpret_cast<const void *>(&q4_k_mfma_gemv_narrow<NC, SHORT>), lds); e != hipSuccess) return e;
     const uint32_t groups = (rows + 15u) / 16u;
     const uint32_t blocks = groups < (uint32_t)ctx->num_cus ? groups : (uint32_t)ctx->num_cus;
     hipLaunchKernelGGL((q4_k_mfma_gemv_narrow<NC, SHORT>), dim3(blocks), dim3(kMThreads), lds, ctx->stream, w,

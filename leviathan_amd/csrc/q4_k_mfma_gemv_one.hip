@@ -382,15 +382,7 @@ hipError_t launch_one(lev_ctx *ctx, const uint8_t *w, const float *x, const floa
     uint64_t slot_of_wave, pos_of_wave;
     lev_wave_tables(wpr, &slot_of_wave, &pos_of_wave);
     constexpr size_t lds = q4k_one_lds(NC);
-    if (lds > 48u * 1024u) {
-        static bool configured = false;   // per instantiation: raise the dynamic LDS limit once
-        if (!configured) {
-            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&q4_k_mfma_gemv_one<NC, NORM>),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-            if (e != hipSuccess) return e;
-            configured = true;
-        }
-    }
+    if (hipError_t e = lev_allow_lds(ctx, reinterpret_cast<const void *>(&q4_k_mfma_gemv_one<NC, NORM>), lds); e != hipSuccess) return e;
     const uint32_t cus = (uint32_t)ctx->num_cus;
     const uint32_t blocks = nrounds < cus ? nrounds : cus;
     hipLaunchKernelGGL((q4_k_mfma_gemv_one<NC, NORM>), dim3(blocks), dim3(kOneThreads), lds, ctx->stream, w, x, gain,

@@ -262,14 +262,8 @@ hipError_t lev_q6_k_gemm_launch(lev_ctx *ctx, const uint8_t *w, const uint16_t *
                                 uint32_t in_dim, uint32_t rows, uint32_t tokens) {
     const lev_gemm_split_plan plan = lev_gemm_split_choose(ctx, true, in_dim, rows, tokens, kTR);
     if (plan.kw) return lev_gemm_split_launch(ctx, true, w, x, y, in_dim, rows, tokens, plan);
-    static bool attr_set = false;
     const size_t lds = (size_t)kRXBufs * kRXBuf + 2 * kRBBuf;   // 160 KB: one workgroup per CU
-    if (!attr_set) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&q6_k_gemm_kernel),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-        attr_set = true;
-    }
+    if (hipError_t e = lev_allow_lds(ctx, reinterpret_cast<const void *>(&q6_k_gemm_kernel), lds); e != hipSuccess) return e;
     // One workgroup per CU (160 KB of LDS).  When the row tiles alone nearly fill the chip, a workgroup
     // takes several token tiles of its rows in turn instead of leaving them to a later round of
     // workgroups: as many rounds of work, and only the last tile's stores are not covered

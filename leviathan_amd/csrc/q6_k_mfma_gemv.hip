@@ -1336,13 +1336,7 @@ hipError_t q6m_launch(lev_ctx *ctx, const uint8_t *w, const float *x, const floa
                       uint32_t *d_argmax, float *d_margin) {
     const uint32_t pb = q6m_lds_bytes(cols, NC, 2u) <= q6m_lds_limit(ctx) ? 2u : 1u;
     const size_t lds = q6m_lds_bytes(cols, NC, pb);
-    static size_t configured = 0;   // per instantiation: raise the dynamic LDS limit once per size
-    if (lds > 48 * 1024 && lds > configured) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&q6_k_mfma_gemv<NC>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-        configured = lds;
-    }
+    if (hipError_t e = lev_allow_lds(ctx, reinterpret_cast<const void *>(&q6_k_mfma_gemv<NC>), lds); e != hipSuccess) return e;
     const uint32_t S = waves ? waves : q6m_waves_per_group(ctx, cols, rows);
     const uint32_t slots = kQWaves / S, ngroups = (rows + 15u) / 16u;
     const uint32_t wgrounds = (ngroups + slots - 1u) / slots;
@@ -1364,13 +1358,7 @@ hipError_t q6m_one_launch_waves(lev_ctx *ctx, const uint8_t *w, const float *x, 
     uint64_t slot_of_wave, pos_of_wave;
     lev_wave_tables(wpr, &slot_of_wave, &pos_of_wave);
     constexpr size_t lds = q6m_one_lds(NC);
-    static bool configured = false;   // per instantiation: raise the dynamic LDS limit once
-    if (!configured) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&q6_k_mfma_gemv_one<NC, NORM, MAXW>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-        configured = true;
-    }
+    if (hipError_t e = lev_allow_lds(ctx, reinterpret_cast<const void *>(&q6_k_mfma_gemv_one<NC, NORM, MAXW>), lds); e != hipSuccess) return e;
     if (NC != 1) partials = nullptr;
     uint32_t blocks = nrounds < (uint32_t)ctx->num_cus ? nrounds : (uint32_t)ctx->num_cus;
     if (partials && blocks > lev_ctx::kArgmaxPartials) blocks = lev_ctx::kArgmaxPartials;
@@ -1457,13 +1445,7 @@ hipError_t q6m_q8_launch(lev_ctx *ctx, const uint8_t *w, const uint32_t *xq, con
                          uint32_t cols, uint32_t rows, uint32_t ncol, uint32_t waves) {
     const uint32_t pb = q6m_q8_lds_bytes(cols, NC, 2u) <= q6m_lds_limit(ctx) ? 2u : 1u;
     const size_t lds = q6m_q8_lds_bytes(cols, NC, pb);
-    static size_t configured = 0;   // per instantiation: raise the dynamic LDS limit once per size
-    if (lds > 48 * 1024 && lds > configured) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&q6_k_mfma_gemv_q8<NC, (NC > 8 ? 2 : 3)>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-        configured = lds;
-    }
+    if (hipError_t e = lev_allow_lds(ctx, reinterpret_cast<const void *>(&q6_k_mfma_gemv_q8<NC, (NC > 8 ? 2 : 3)>), lds); e != hipSuccess) return e;
     const uint32_t S = waves ? waves : q6m_waves_per_group(ctx, cols, rows);
     const uint32_t slots = kQWaves / S, ngroups = (rows + 15u) / 16u;
     const uint32_t wgrounds = (ngroups + slots - 1u) / slots;
@@ -1542,13 +1524,7 @@ hipError_t q6m_q8_one_launch_grid(lev_ctx *ctx, const uint8_t *w, const uint32_t
     uint64_t slot_of_wave, pos_of_wave;
     lev_wave_tables(g.wpr, &slot_of_wave, &pos_of_wave);
     constexpr size_t lds = q6m_q8_one_lds(NC, q6m_q8_one_waves(NC));
-    static bool configured = false;   // per instantiation: raise the dynamic LDS limit once
-    if (!configured) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&q6_k_mfma_gemv_q8_one<NC, SLICED>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-        configured = true;
-    }
+    if (hipError_t e = lev_allow_lds(ctx, reinterpret_cast<const void *>(&q6_k_mfma_gemv_q8_one<NC, SLICED>), lds); e != hipSuccess) return e;
     float *sums = nullptr;
     if (SLICED) {
         sums = static_cast<float *>(lev_scratch(ctx, (size_t)g.slices * ncol * rows * 4u));

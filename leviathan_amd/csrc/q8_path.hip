@@ -275,13 +275,7 @@ hipError_t launch_q8(lev_ctx *ctx, const uint8_t *w, const uint32_t *xq, const f
                      uint32_t in_dim, uint32_t rows, uint32_t ncol) {
     const uint32_t SB = in_dim >> 8;
     const size_t lds = (size_t)NC * SB * (kCodeStride + kPairStride);
-    static size_t configured = 0;
-    if (lds > 48 * 1024 && lds > configured) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&q4_k_gemv_q8_kernel<NC>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-        configured = lds;
-    }
+    if (hipError_t e = lev_allow_lds(ctx, reinterpret_cast<const void *>(&q4_k_gemv_q8_kernel<NC>), lds); e != hipSuccess) return e;
     int per_cu = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, q4_k_gemv_q8_kernel<NC>, kQThreads, lds) !=
             hipSuccess || per_cu < 1)
@@ -419,13 +413,7 @@ template <int NC>
 hipError_t launch_q6_q8(lev_ctx *ctx, const uint8_t *w, const uint32_t *xq, const float *xs, float *y,
                         uint32_t in_dim, uint32_t rows, uint32_t ncol, bool persistent) {
     const size_t lds = (size_t)NC * (in_dim >> 8) * kQ6Stride;
-    static size_t configured = 0;
-    if (lds > 48 * 1024 && lds > configured) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&q6_k_gemv_q8_kernel<NC>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-        configured = lds;
-    }
+    if (hipError_t e = lev_allow_lds(ctx, reinterpret_cast<const void *>(&q6_k_gemv_q8_kernel<NC>), lds); e != hipSuccess) return e;
     int per_cu = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, q6_k_gemv_q8_kernel<NC>, kQ6Threads, lds) !=
             hipSuccess || per_cu < 1)
@@ -944,13 +932,7 @@ template <int NCL, bool SHORT>
 hipError_t launch_q8m_variant(lev_ctx *ctx, const uint8_t *w, const uint8_t *xq, const float *xs, float *y,
                               uint32_t cols, uint32_t rows, uint32_t ncol, uint32_t blocks) {
     const size_t lds = q8m_lds_bytes(cols, NCL);
-    static size_t configured = 0;   // per instantiation: raise the dynamic LDS limit once per size
-    if (lds > 48 * 1024 && lds > configured) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&q4_k_q8_mfma<NCL, SHORT>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-        configured = lds;
-    }
+    if (hipError_t e = lev_allow_lds(ctx, reinterpret_cast<const void *>(&q4_k_q8_mfma<NCL, SHORT>), lds); e != hipSuccess) return e;
     uint32_t lognp = 0;
     while ((1u << lognp) < ncol) ++lognp;
     hipLaunchKernelGGL((q4_k_q8_mfma<NCL, SHORT>), dim3(blocks), dim3(kMThreads), lds, ctx->stream, w, xq,

@@ -131,3 +131,20 @@ def test_grouped_moe_offset_scan_writes_every_entry():
                 writes[experts] += 1
         assert np.all(writes == 1), experts
         assert np.array_equal(goff, np.concatenate([[0], np.cumsum(cnt)])), experts
+
+
+def test_no_kernel_state_is_kept_per_process():
+    """What belongs to a device (a kernel's LDS limit) is kept with the context: the sources hold no function-local
+    variable that outlives a call, and set kernel attributes in one place."""
+    csrc = os.path.join(ROOT, "leviathan_amd", "csrc")
+    kept, setters = [], []
+    for name in sorted(os.listdir(csrc)):
+        if not name.endswith((".hip", ".hpp")):
+            continue
+        for line in open(os.path.join(csrc, name)):
+            if re.match(r"\s+static (bool|size_t|int|u?int\d+_t|void|float|double)\b[^(]*[=;]", line) and "[] {" not in line:
+                kept.append((name, line.strip()))
+            if "hipFuncSetAttribute" in line:
+                setters.append(name)
+    assert not kept
+    assert setters == ["lev_common.hpp"]
