@@ -1724,15 +1724,17 @@ extern "C" int lev_hip_moe_experts_q4_0(lev_ctx *ctx, const lev_moe_experts *poo
     moe_args a;
     int st = check_pools(ctx, pools, top_k, tokens, &a);
     if (st != LEV_OK) return st;
-    const bool grouped = use_grouped(ctx, a, d_x, tokens, false) && (reinterpret_cast<uintptr_t>(d_act) & 15u) == 0u;
+    bool grouped = use_grouped(ctx, a, d_x, tokens, false) && (reinterpret_cast<uintptr_t>(d_act) & 15u) == 0u;
     float *act = d_act;
     moe_scratch s{nullptr, nullptr, nullptr};
-    if (!act || grouped) {
-        st = get_scratch(ctx, tokens, a.experts, top_k, a.inter, &s,
-                         grouped ? lev_moe_grouped_scratch_bytes(ctx, grouped_args(a, tokens)) : 0);
+    // without room for grouping (a program is being recorded and the context's scratch is still too small) pair by pair
+    if (grouped) grouped = get_scratch(ctx, tokens, a.experts, top_k, a.inter, &s,
+                                       lev_moe_grouped_scratch_bytes(ctx, grouped_args(a, tokens))) == LEV_OK;
+    if (!act && !grouped) {
+        st = get_scratch(ctx, tokens, a.experts, top_k, a.inter, &s);
         if (st != LEV_OK) return st;
-        if (!act) act = s.act;
     }
+    if (!act) act = s.act;
     if (grouped)
         return lev_hip_check(ctx,
                              lev_moe_grouped_launch(ctx, grouped_args(a, tokens), d_x, d_ids, d_weights,
@@ -1760,7 +1762,7 @@ int moe_layer_impl(lev_ctx *ctx, const lev_moe_experts *pools, const float *d_ro
     int st = check_pools(ctx, pools, top_k, tokens, &a);
     if (st != LEV_OK) return st;
     if (a.experts > 4096u) return lev_fail(ctx, LEV_ERR_BAD_DIMENSIONS, "moe_layer: %u experts", a.experts);
-    const bool grouped = !fixed && use_grouped(ctx, a, d_x, tokens, true);
+    bool grouped = !fixed && use_grouped(ctx, a, d_x, tokens, true);
     moe_scratch s;
     if (fixed) {
         if (tokens > LEV_NOALLOC_MOE_MAX_TOKENS)
@@ -1777,9 +1779,13 @@ int moe_layer_impl(lev_ctx *ctx, const lev_moe_experts *pools, const float *d_ro
         s.act = reinterpret_cast<float *>(static_cast<char *>(fixed) + s_bytes);
         s.grouped = nullptr;
     } else {
-        st = get_scratch(ctx, tokens, a.experts, top_k, a.inter, &s,
-                         grouped ? lev_moe_grouped_scratch_bytes(ctx, grouped_args(a, tokens)) : 0);
-        if (st != LEV_OK) return st;
+        // without room for grouping pair by pair, as in lev_hip_moe_experts_q4_0
+        if (grouped) grouped = get_scratch(ctx, tokens, a.experts, top_k, a.inter, &s,
+                                           lev_moe_grouped_scratch_bytes(ctx, grouped_args(a, tokens))) == LEV_OK;
+        if (!grouped) {
+            st = get_scratch(ctx, tokens, a.experts, top_k, a.inter, &s);
+            if (st != LEV_OK) return st;
+        }
     }
     const bool fast = experts_fast(a, d_x);
     gu_route rt{d_ids, nullptr, nullptr, nullptr, nullptr};

@@ -1,8 +1,9 @@
 """GPU parity of the grouped matrix product that serves prompts and large batches of the MoE layer, at the
-edges of its tiles: column tiles of 32 in items of 64 pairs, rows in tiles of 128 (gate/up) and 256 (down)
-cut into waves, K in steps of two blocks and weight groups of four.  FP64 chain at the reference's 1e-4."""
+edges of its tiles: column tiles of 32 in items of 64 pairs, workgroups of four, eight and twelve waves of 16
+(gate/up) and 32 (down) rows, K in steps of two blocks and weight groups of four.  FP64 chain at the reference's 1e-4."""
 import numpy as np
 import pytest
+import torch
 
 import oracle as O
 from tests import helpers as H
@@ -141,3 +142,60 @@ def test_moe_grouped_product_range_of_act(ctx, x_exp, d_exp):
     y_want = act[:, 0].astype(np.float64).sum(axis=1, keepdims=True) * 7 * 2.0 ** d_exp
     assert np.all(np.isfinite(y)) and np.all(y > 0)
     assert np.all(np.abs(y - y_want) <= 1e-6 * y_want)
+
+
+def test_moe_experts_with_their_own_act_record_on_a_fresh_context(ctx):
+    """A caller that brings `act` needs no scratch of the context's but for grouping: recorded on a context that has
+    none, where nothing may be allocated, the pairs are taken one by one."""
+    from leviathan_amd import capi, ops
+    import ctypes as C
+    hidden, inter, experts, tokens = 320, 192, 2, 700
+    wr, pool, offs, x = H.config5(hidden, inter, experts, tokens, seed=9)
+    rng = np.random.default_rng(9)
+    ids = (np.arange(tokens) % experts).astype(np.int32)[:, None]
+    wts = rng.random((tokens, 1)).astype(np.float32)
+    want_y, want_act = run_experts(ctx, pool, offs, hidden, inter, experts, x, ids, wts)      # grouped
+    fresh = ops.Context(0, own_stream=True)
+    pool_d, x_d, ids_d, wts_d = (torch.from_numpy(a).cuda() for a in (pool, x, ids, wts))
+    pools = ops.Context.moe_pools(pool_d, hidden, inter, experts, offs["gate_off"], offs["up_off"], offs["down_off"])
+    y, act = torch.empty(tokens, hidden, device="cuda"), torch.empty(tokens, 1, inter, device="cuda")
+    torch.cuda.synchronize()
+    fresh.program_begin()
+    st = fresh.lib.lev_hip_moe_experts_q4_0(fresh.ctx, C.byref(pools), *(C.c_void_p(t.data_ptr()) for t in (x_d, ids_d, wts_d, y, act)),
+                                            1, tokens)
+    program = fresh.program_end()
+    assert st == capi.OK
+    for _ in range(3):
+        y.fill_(float("nan")), act.fill_(float("nan"))
+        torch.cuda.synchronize()
+        program.run()
+        fresh.sync()
+        assert O.max_rel_err(act.cpu().numpy().ravel(), want_act.ravel()) < 1e-4
+        assert O.max_rel_err(y.cpu().numpy().ravel(), want_y.ravel()) < 1e-4
+    program.destroy()
+    fresh.close()
+
+
+@pytest.mark.parametrize("hidden,inter,counts", [
+    (64, 64, (1, 32)), (192, 320, (33, 31, 0)), (320, 192, (64, 65)), (4160, 128, (40, 24)), (4160, 64, (97, 7, 128)),
+])
+def test_moe_grouped_product_tiles_of_small_experts(ctx, hidden, inter, counts):
+    """The tiles of test_moe_grouped_product_tiles where experts are so small that pairs are only grouped when there are
+    thousands: one expert more takes as many as the rule asks for (65 MB of weights that grouping saves reading, ten
+    experts' worth counted in; lev_moe_grouped_usable), twelve of them checked."""
+    nbytes = 3 * hidden * inter * 18 // 32
+    counts = counts + (int(65e6 / nbytes) + 70,)
+    experts, tokens = len(counts), sum(counts)
+    assert (tokens - experts + 10) * nbytes >= 65e6 and tokens > 8 * experts
+    wr, pool, offs, x = H.config5(hidden, inter, experts, tokens, seed=hidden + inter)
+    rng = np.random.default_rng(tokens)
+    ids = rng.permutation(np.repeat(np.arange(experts), counts)).astype(np.int32)[:, None]
+    wts = rng.random((tokens, 1)).astype(np.float32)
+    y, act = run_experts(ctx, pool, offs, hidden, inter, experts, x, ids, wts)
+    g, u, d = (pool[offs["gate_off"]:], pool[offs["up_off"]:], pool[offs["down_off"]:])
+    filler = np.flatnonzero(ids[:, 0] == experts - 1)
+    for t in np.concatenate([np.flatnonzero(ids[:, 0] != experts - 1), filler[::max(1, len(filler) // 12)]]):
+        ref = O.moe_experts_f64(g, u, d, hidden, inter, ids[t], wts[t], x[t])
+        assert O.max_rel_err(act[t], ref["act"]) < TOL, t
+        y32, _ = O.moe_experts_f32(g, u, d, hidden, inter, ids[t], wts[t], x[t])
+        assert O.max_rel_err(y[t], ref["y"]) < max(TOL, 1.5 * O.max_rel_err(y32, ref["y"])), t
