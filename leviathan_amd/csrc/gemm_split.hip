@@ -176,19 +176,22 @@ struct weights_q6k {
     __device__ __forceinline__ uint32_t unit(int q) const { return 4u * lh + (uint32_t)q; }
 };
 
-// grid: row tiles * token tiles * S workgroups in one line, up to a multiple of eight.  Workgroups go to the XCDs in
+// grid: row tiles * token tiles * (zn slices from z0 on, of the `splits`) workgroups in one line, up to a multiple of
+// eight.  All slices of a launch write partial tiles of their own to `out`, one behind the other; add: the one slice
+// of the launch is added to what is there.  Workgroups go to the XCDs in
 // turn: each takes an eighth of the tiles, whose order has the token tiles of a row tile together (they read the same
 // weights).
 template <typename W, int T, int RW, int KW>
 __global__ void __launch_bounds__(RW *KW * 64, 2)
 gemm_split_kernel(const uint8_t *__restrict__ w, const uint16_t *__restrict__ x, float *__restrict__ out, uint32_t in_dim,
-                  uint32_t rows, uint32_t tokens, uint32_t row_tiles, uint32_t tok_tiles, uint32_t splits) {
+                  uint32_t rows, uint32_t tokens, uint32_t row_tiles, uint32_t tok_tiles, uint32_t splits, uint32_t z0,
+                  uint32_t zn, uint32_t add) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
     const uint32_t lr = lane & 31u, lh = lane >> 5, rw = wave % RW, kw = wave / RW;
     const uint32_t tile = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3), zr = tile / tok_tiles;
-    const uint32_t z = zr / row_tiles, rt = zr - z * row_tiles, tok0 = (tile - zr * tok_tiles) * (32u * T);
-    if (z >= splits) return;
+    const uint32_t zl = zr / row_tiles, z = z0 + zl, rt = zr - zl * row_tiles, tok0 = (tile - zr * tok_tiles) * (32u * T);
+    if (zl >= zn) return;
     const uint32_t row0 = (rt * RW + rw) * 32u, row = row0 + lr;
     const uint32_t nsb = in_dim >> 8, ns = KW * splits;
     const uint32_t sb0 = (z * KW + kw) * nsb / ns, sb1 = (z * KW + kw + 1u) * nsb / ns;
@@ -308,7 +311,22 @@ gemm_split_kernel(const uint8_t *__restrict__ w, const uint16_t *__restrict__ x,
                 for (int i = 0; i < 16; ++i) acc[t][i] += red[((((k - 1u) * RW + rw) * T + t) * 16 + i) * 64 + lane];
     }
     if (row >= rows) return;
-    float *const dst = out + (uint64_t)z * tokens * rows + row;
+    float *const dst = out + (uint64_t)zl * tokens * rows + row;
+    if (add) {
+#pragma unroll 1
+        for (int t = 0; t < T; ++t) {
+            const uint32_t first = tok0 + 32u * t + 4u * lh;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const uint32_t tok = first + 8u * (i / 4) + (i % 4);
+                float v = 0.f;
+#pragma unroll
+                for (int k = 0; k < T; ++k) v = k == t ? acc[k][i] : v;
+                if (tok < tokens) dst[(uint64_t)tok * rows] += v;
+            }
+        }
+        return;
+    }
 #pragma unroll
     for (int t = 0; t < T; ++t)
 #pragma unroll
@@ -333,35 +351,35 @@ gemm_split_sum_kernel(const float *__restrict__ part, float *__restrict__ y, uin
 
 template <typename W, int T, int RW, int KW>
 hipError_t launch_as(lev_ctx *ctx, const uint8_t *w, const uint16_t *x, float *out, uint32_t in_dim, uint32_t rows,
-                     uint32_t tokens, uint32_t tok_tiles, uint32_t splits) {
+                     uint32_t tokens, uint32_t tok_tiles, uint32_t splits, uint32_t z0, uint32_t zn, bool add) {
     constexpr size_t lds = (size_t)KW * x_bufs<W>(T, RW, KW) * T * kTile + RW * KW * W::kArea;
     if (hipError_t e = lev_allow_lds(ctx, reinterpret_cast<const void *>(&gemm_split_kernel<W, T, RW, KW>), lds); e != hipSuccess) return e;
     const uint32_t row_tiles = (rows + RW * 32u - 1u) / (RW * 32u);
-    hipLaunchKernelGGL((gemm_split_kernel<W, T, RW, KW>), dim3((row_tiles * tok_tiles * splits + 7u) / 8u * 8u),
-                       dim3(RW * KW * 64), lds, ctx->stream, w, x, out, in_dim, rows, tokens, row_tiles, tok_tiles, splits);
+    hipLaunchKernelGGL((gemm_split_kernel<W, T, RW, KW>), dim3((row_tiles * tok_tiles * zn + 7u) / 8u * 8u), dim3(RW * KW * 64),
+                       lds, ctx->stream, w, x, out, in_dim, rows, tokens, row_tiles, tok_tiles, splits, z0, zn, add ? 1u : 0u);
     return hipGetLastError();
 }
 
 template <typename W, int T>
 hipError_t launch_tiles(lev_ctx *ctx, const uint8_t *w, const uint16_t *x, float *y, uint32_t in_dim, uint32_t rows,
                         uint32_t tokens, uint32_t tok_tiles, const lev_gemm_split_plan &plan) {
-    if (plan.kw == 1u) return launch_as<W, T, 4, 1>(ctx, w, x, y, in_dim, rows, tokens, tok_tiles, 1u);
-    uint32_t splits = plan.splits;
-    float *part = y;
-    if (splits > 1u) {
-        part = static_cast<float *>(lev_scratch(ctx, (size_t)splits * tokens * rows * 4));
-        if (!part) {   // recording, and the scratch is still too small: a workgroup takes all of K
-            splits = 1u;
-            part = y;
-        }
+    if (plan.kw == 1u) return launch_as<W, T, 4, 1>(ctx, w, x, y, in_dim, rows, tokens, tok_tiles, 1u, 0u, 1u, false);
+    const uint32_t splits = plan.splits;
+    auto slices = [&](float *out, uint32_t z0, uint32_t zn, bool add) {
+        if constexpr (4u * (x_bufs<W>(T, 2, 4) * T * kTile + 2u * W::kArea) <= 160u * 1024u)
+            if (plan.kw == 4u) return launch_as<W, T, 2, 4>(ctx, w, x, out, in_dim, rows, tokens, tok_tiles, splits, z0, zn, add);
+        return launch_as<W, T, 4, 2>(ctx, w, x, out, in_dim, rows, tokens, tok_tiles, splits, z0, zn, add);
+    };
+    if (splits == 1u) return slices(y, 0u, 1u, false);
+    float *const part = static_cast<float *>(lev_scratch(ctx, (size_t)splits * tokens * rows * 4));
+    if (!part) {
+        // a program is being recorded and the scratch is still too small: a launch for every slice, each added to y where
+        // the others are, in the same order and so to the same bits
+        for (uint32_t z = 0; z < splits; ++z)
+            if (hipError_t e = slices(y, z, 1u, z != 0u); e != hipSuccess) return e;
+        return hipSuccess;
     }
-    hipError_t e;
-    if constexpr (4u * (x_bufs<W>(T, 2, 4) * T * kTile + 2u * W::kArea) <= 160u * 1024u)
-        e = plan.kw == 4u ? launch_as<W, T, 2, 4>(ctx, w, x, part, in_dim, rows, tokens, tok_tiles, splits)
-                          : launch_as<W, T, 4, 2>(ctx, w, x, part, in_dim, rows, tokens, tok_tiles, splits);
-    else
-        e = launch_as<W, T, 4, 2>(ctx, w, x, part, in_dim, rows, tokens, tok_tiles, splits);
-    if (e != hipSuccess || splits == 1u) return e;
+    if (hipError_t e = slices(part, 0u, splits, false); e != hipSuccess) return e;
     const uint64_t n = (uint64_t)tokens * rows;
     if (n % 4u == 0u && (reinterpret_cast<uintptr_t>(y) & 15u) == 0u)
         hipLaunchKernelGGL((gemm_split_sum_kernel<4>), dim3((uint32_t)((n / 4u + 255u) / 256u)), dim3(256), 0, ctx->stream,

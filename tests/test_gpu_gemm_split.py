@@ -57,3 +57,28 @@ def test_gemm_split_recorded_without_scratch(ctx):
         assert np.linalg.norm(got - eager) < 1e-5 * np.linalg.norm(eager)     # f32 sums in another order
     program.destroy()
     fresh.close()
+
+
+@pytest.mark.parametrize("kind,rows,cols,tokens", [("q4_k", 512, 4096, 40), ("q4_k", 129, 1792, 33), ("q4_k", 257, 12288, 70),
+                                                   ("q6_k", 512, 4096, 40), ("q6_k", 96, 8192, 129), ("q6_k", 33, 11008, 97)])
+def test_gemm_split_records_the_eager_bits(ctx, kind, rows, cols, tokens):
+    """Slices that workgroups share meet in scratch or, recorded where there is none, one launch after the other in y:
+    the same sums in the same order."""
+    from leviathan_amd import ops
+    w, x = (H.config4 if kind == "q4_k" else config4_q6)(rows, cols, tokens, seed=rows + tokens)
+    wd, xd = dev(w), dev(x)
+    eager = (gemm if kind == "q4_k" else gemm6)(ctx, w, x, rows, cols, tokens)
+    fresh = ops.Context(0, own_stream=True)
+    y = torch.empty(tokens, rows, device="cuda")
+    torch.cuda.synchronize()
+    fresh.program_begin()
+    (fresh.q4_k_gemm_prefill if kind == "q4_k" else fresh.q6_k_gemm_prefill)(wd, xd, cols, rows, tokens, y=y)
+    program = fresh.program_end()
+    for _ in range(3):
+        y.fill_(float("nan"))
+        torch.cuda.synchronize()
+        program.run()
+        fresh.sync()
+        assert np.array_equal(y.cpu().numpy().view(np.uint32), eager.reshape(tokens, rows).view(np.uint32))
+    program.destroy()
+    fresh.close()
