@@ -1104,9 +1104,11 @@ q6_k_mfma_gemv_q8(const uint8_t *__restrict__ w, const uint32_t *__restrict__ xq
 // its wave's superblock straight into registers, with the quarter activation scales of its
 // blocks beside them: nothing is staged in LDS but the turn-round of the weights and the
 // partial sums of a round.
-// SLICED: a row of more superblocks than the workgroup has waves is cut into gridDim.y slices of wpr,
+// kSliced: a row of more superblocks than the workgroup has waves is cut into gridDim.y slices of wpr,
 // a workgroup taking one for its row groups.  The slices' sums meet in scratch, and the last of the
 // workgroups that share a blockIdx.x to finish adds them up, in the order of the slices (lev_publish_wait).
+// kOneSlice: the launch is slice `slice` of such a row, added to what the slices before it left in y: the same
+// sums in the same order without scratch, a launch a slice.
 // Staged in LDS as a whole (q6_k_mfma_gemv_q8) such rows leave room for four columns at 12288, and the
 // weights are read again for every four: 4096 x 12288 by one, five and
 // sixteen columns 15.0, 27.5 and 53.8 us with it, 13.5, 15.6 and 28.5 here.
@@ -1119,13 +1121,17 @@ __host__ __device__ constexpr size_t q6m_q8_one_lds(uint32_t nc, uint32_t waves)
 // Waves of a workgroup: the operands of sixteen columns take the registers of sixteen waves.
 constexpr int q6m_q8_one_waves(int nc) { return nc > 8 ? 8 : kQWaves; }
 
+enum q6m_q8_mode { kWholeRow, kSliced, kOneSlice };
+
 // NC: columns held (4, 8 or 16; >= ncol).
-template <int NC, bool SLICED>
+template <int NC, q6m_q8_mode MODE>
 __global__ void __launch_bounds__(q6m_q8_one_waves(NC) * LEV_WAVE)
 q6_k_mfma_gemv_q8_one(const uint8_t *__restrict__ w, const uint32_t *__restrict__ xq, const float *__restrict__ xs,
                       float *__restrict__ y, uint32_t cols, uint32_t rows, uint32_t ncol, uint32_t wpr, uint32_t slots,
-                      uint64_t slot_of_wave, uint64_t pos_of_wave, float *__restrict__ sums, uint32_t *__restrict__ tickets) {
+                      uint64_t slot_of_wave, uint64_t pos_of_wave, uint32_t slice, float *__restrict__ sums,
+                      uint32_t *__restrict__ tickets) {
     constexpr int NCH = NC / 4, WAVES = q6m_q8_one_waves(NC);
+    constexpr bool SLICED = MODE == kSliced;
     constexpr uint32_t kPart = q6m_q8_one_part_bytes(NC, WAVES);
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
@@ -1133,7 +1139,7 @@ q6_k_mfma_gemv_q8_one(const uint8_t *__restrict__ w, const uint32_t *__restrict_
     const uint32_t slot = (uint32_t)(slot_of_wave >> (4u * wave)) & 15u;   // idle waves: slot >= slots
     const uint32_t SB = cols >> 8, nblk = cols >> 5;
     const uint32_t pos = (uint32_t)(pos_of_wave >> (4u * wave)) & 15u;
-    const uint32_t sbw = SLICED ? blockIdx.y * wpr + pos : pos;
+    const uint32_t sbw = MODE == kWholeRow ? pos : (SLICED ? blockIdx.y : slice) * wpr + pos;
     const uint32_t sb = sbw < SB ? sbw : SB - 1u;                          // the wave's superblock column
     const uint32_t r = lane & 15u, q = lane >> 4;
     const uint32_t hf = q >> 1, jb = q & 1u;
@@ -1243,8 +1249,10 @@ q6_k_mfma_gemv_q8_one(const uint8_t *__restrict__ w, const uint32_t *__restrict_
                     if (SLICED)
                         __hip_atomic_store(reinterpret_cast<float *>(yp + (uint64_t)(4 * ch) * rows * 4u), s, __ATOMIC_RELAXED,
                                            __HIP_MEMORY_SCOPE_AGENT);
-                    else
-                        *reinterpret_cast<__attribute__((address_space(1))) float *>(yp + (uint64_t)(4 * ch) * rows * 4u) = s;
+                    else {
+                        auto *const at = reinterpret_cast<__attribute__((address_space(1))) float *>(yp + (uint64_t)(4 * ch) * rows * 4u);
+                        *at = MODE == kOneSlice ? (slice ? *at : 0.f) + s : s;
+                    }
                 }
             }
         }
@@ -1517,21 +1525,16 @@ bool q6m_q8_staged_is_faster(const lev_ctx *ctx, const q6m_slices &g, uint32_t c
     return staged < 0.96 * sliced;
 }
 
-// hipErrorOutOfMemory: the scratch cannot be had (a program is being recorded and the context's is still too small).
-template <int NC, bool SLICED>
+template <int NC, q6m_q8_mode MODE>
 hipError_t q6m_q8_one_launch_grid(lev_ctx *ctx, const uint8_t *w, const uint32_t *xq, const float *xs, float *y,
-                                  uint32_t cols, uint32_t rows, uint32_t ncol, const q6m_slices &g) {
+                                  uint32_t cols, uint32_t rows, uint32_t ncol, const q6m_slices &g, uint32_t slice, float *sums) {
     uint64_t slot_of_wave, pos_of_wave;
     lev_wave_tables(g.wpr, &slot_of_wave, &pos_of_wave);
     constexpr size_t lds = q6m_q8_one_lds(NC, q6m_q8_one_waves(NC));
-    if (hipError_t e = lev_allow_lds(ctx, reinterpret_cast<const void *>(&q6_k_mfma_gemv_q8_one<NC, SLICED>), lds); e != hipSuccess) return e;
-    float *sums = nullptr;
-    if (SLICED) {
-        sums = static_cast<float *>(lev_scratch(ctx, (size_t)g.slices * ncol * rows * 4u));
-        if (!sums) return hipErrorOutOfMemory;
-    }
-    hipLaunchKernelGGL((q6_k_mfma_gemv_q8_one<NC, SLICED>), dim3(g.blocks, g.slices), dim3(g.slots * g.wpr * LEV_WAVE), lds,
-                       ctx->stream, w, xq, xs, y, cols, rows, ncol, g.wpr, g.slots, slot_of_wave, pos_of_wave, sums,
+    if (hipError_t e = lev_allow_lds(ctx, reinterpret_cast<const void *>(&q6_k_mfma_gemv_q8_one<NC, MODE>), lds); e != hipSuccess) return e;
+    hipLaunchKernelGGL((q6_k_mfma_gemv_q8_one<NC, MODE>), dim3(g.blocks, MODE == kSliced ? g.slices : 1u),
+                       dim3(g.slots * g.wpr * LEV_WAVE), lds, ctx->stream, w, xq, xs, y, cols, rows, ncol, g.wpr, g.slots,
+                       slot_of_wave, pos_of_wave, slice, sums,
                        reinterpret_cast<uint32_t *>(ctx->d_flag) + lev_ctx::kSliceTicketWord);
     return hipGetLastError();
 }
@@ -1540,10 +1543,15 @@ template <int NC>
 hipError_t q6m_q8_one_launch(lev_ctx *ctx, const uint8_t *w, const uint32_t *xq, const float *xs, float *y,
                              uint32_t cols, uint32_t rows, uint32_t ncol) {
     const q6m_slices g = q6m_q8_one_grid(ctx, cols, rows, (uint32_t)q6m_q8_one_waves(NC));
+    if (g.slices == 1u) return q6m_q8_one_launch_grid<NC, kWholeRow>(ctx, w, xq, xs, y, cols, rows, ncol, g, 0u, nullptr);
     const uint32_t held = lev_q6_k_mfma_q8_cols(ctx, cols);
-    if (g.slices > 1u && held && q6m_q8_staged_is_faster(ctx, g, cols, rows, ncol, held)) return hipErrorNotSupported;
-    if (g.slices > 1u) return q6m_q8_one_launch_grid<NC, true>(ctx, w, xq, xs, y, cols, rows, ncol, g);
-    return q6m_q8_one_launch_grid<NC, false>(ctx, w, xq, xs, y, cols, rows, ncol, g);
+    if (held && q6m_q8_staged_is_faster(ctx, g, cols, rows, ncol, held)) return hipErrorNotSupported;
+    float *const sums = static_cast<float *>(lev_scratch(ctx, (size_t)g.slices * ncol * rows * 4u));
+    if (sums) return q6m_q8_one_launch_grid<NC, kSliced>(ctx, w, xq, xs, y, cols, rows, ncol, g, 0u, sums);
+    // a program is being recorded and the context's scratch is still too small
+    for (uint32_t z = 0; z < g.slices; ++z)
+        if (hipError_t e = q6m_q8_one_launch_grid<NC, kOneSlice>(ctx, w, xq, xs, y, cols, rows, ncol, g, z, nullptr); e != hipSuccess) return e;
+    return hipSuccess;
 }
 
 // LEV_Q6K_ONE=0: the kernel that stages the activations everywhere, for comparison
@@ -1557,8 +1565,7 @@ bool q6m_q8_one_off() {
 }  // namespace
 
 // All columns (at most sixteen) in one pass over the weights, a wave per superblock column; w 2-byte, xq 16-byte, xs
-// 8-byte aligned.  hipErrorNotSupported: the shape is the staging kernel's (lev_q6_k_mfma_gemv_q8_launch);
-// hipErrorOutOfMemory: the scratch cannot be had.
+// 8-byte aligned.  hipErrorNotSupported: the shape is the staging kernel's (lev_q6_k_mfma_gemv_q8_launch).
 hipError_t lev_q6_k_mfma_gemv_q8_one_pass(lev_ctx *ctx, const uint8_t *w, const uint32_t *xq, const float *xs,
                                           float *y, uint32_t in_dim, uint32_t rows, uint32_t ncol) {
     if (q6m_q8_one_off()) return hipErrorNotSupported;

@@ -1153,7 +1153,7 @@ extern "C" int lev_hip_q6_k_gemv_q8(lev_ctx *ctx, const void *d_w, size_t w_byte
     const uint32_t mcols = lev_q6_k_mfma_q8_cols(ctx, in_dim);
     if (mcols && (!sel || sel->family == 1u)) {
         hipError_t one = lev_q6_k_mfma_gemv_q8_one_pass(ctx, w, xq, d_xs, d_y, in_dim, rows, ncol);
-        if (one != hipErrorNotSupported && one != hipErrorOutOfMemory) return lev_hip_check(ctx, one, "q6_k_gemv_q8 launch");
+        if (one != hipErrorNotSupported) return lev_hip_check(ctx, one, "q6_k_gemv_q8 launch");
         // the integer matrix-core kernel: up to mcols columns per pass over the weights
         for (uint32_t done = 0; done < ncol; done += mcols) {
             const uint32_t nc = ncol - done < mcols ? ncol - done : mcols;

@@ -46,3 +46,34 @@ def test_q6_q8_sliced_or_staged(blocks, rows, ncol):
     """Either side of the line from which wide rows are left to the kernel that stages the activations: by rows, by
     columns, and by width where it no longer holds sixteen columns in one pass."""
     test_q6_q8_sliced_rows(blocks, rows, ncol)
+
+
+@pytest.mark.parametrize("blocks,rows,ncol", [(17, 300, 1), (19, 2000, 4), (33, 48, 8), (9, 17, 9), (48, 1000, 16)])
+def test_q6_q8_sliced_rows_record_the_eager_bits(blocks, rows, ncol):
+    """Recorded on a context without scratch the slices are launched one after the other: the same sums in the same
+    order as where they meet in scratch."""
+    from leviathan_amd import ops
+    cols = 256 * blocks
+    w = dev(O.synth_q6_k(blocks + rows, rows * blocks))
+    x = O.normal(ncol * cols, 7 + ncol).reshape(ncol, cols)
+    q = [O.quantize_q8(v) for v in x]
+    xq = np.stack([a for a, *_ in q])
+    d = np.stack([b for _, b, *_ in q])
+    xs = dev(np.stack([d, d * xq.reshape(ncol, -1, 32).sum(2)], axis=2).astype(np.float32))
+    xq = dev(xq)
+    want, y = (torch.full((ncol, rows), float("nan"), device="cuda") for _ in range(2))
+    eager, fresh = ops.Context(0), ops.Context(0, own_stream=True)
+    eager.q6_k_gemv_q8(w, xq, xs, cols, rows, ncol, y=want)
+    torch.cuda.synchronize()
+    fresh.program_begin()
+    fresh.q6_k_gemv_q8(w, xq, xs, cols, rows, ncol, y=y)
+    program = fresh.program_end()
+    for _ in range(3):
+        y.fill_(float("nan"))
+        torch.cuda.synchronize()
+        program.run()
+        fresh.sync()
+        assert torch.equal(y.view(torch.int32), want.view(torch.int32))
+    program.destroy()
+    fresh.close()
+    eager.close()
