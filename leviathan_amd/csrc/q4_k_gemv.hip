@@ -354,6 +354,7 @@ hipError_t lev_q4_k_gemv_launch(lev_ctx *ctx, const uint8_t *w, const float *x, 
                                 uint32_t ncol) {
     const uint32_t units = in_dim / 64u;
     uint32_t done = 0;
+    bool no_scratch = false;
     // a schedule installed for this shape (lev_hip_forge_select) overrides the built-in choice
     const lev_schedule *sel = lev_selected(ctx, LEV_OP_Q4_K_GEMV, in_dim, rows, ncol);
     const bool mfma = (sel ? sel->family : q4k_builtin_family(ctx, in_dim, rows, ncol)) == 1u;
@@ -365,11 +366,24 @@ hipError_t lev_q4_k_gemv_launch(lev_ctx *ctx, const uint8_t *w, const float *x, 
         if (!lev_q4_k_mfma_planes(ctx, in_dim, rows, nc)) break;
         hipError_t e = lev_q4_k_mfma_gemv_launch(ctx, w, x + (uint64_t)done * in_dim, gain, eps,
                                                  y + (uint64_t)done * rows, in_dim, rows, nc);
-        if (e == hipErrorOutOfMemory) break;
+        if (e == hipErrorOutOfMemory) {
+            no_scratch = true;
+            break;
+        }
         if (e != hipSuccess) return e;
         done += nc;
     }
     const uint32_t mfma_cols = mfma ? lev_q4_k_mfma_cols(ctx, in_dim) : 0u;
+    // A program is being recorded and the context's scratch has no room for the planes of a row too wide to be staged by
+    // fours: by ones and twos, whose sums are exact as well, so that the recorded call gives the eager one's values.
+    const uint32_t narrow_cols = no_scratch && !mfma_cols ? lev_q4_k_mfma_narrow_cols(ctx, in_dim) : 0u;
+    while (narrow_cols && done < ncol) {
+        const uint32_t nc = ncol - done < narrow_cols ? ncol - done : narrow_cols;
+        hipError_t e = lev_q4_k_mfma_gemv_launch(ctx, w, x + (uint64_t)done * in_dim, gain, eps,
+                                                 y + (uint64_t)done * rows, in_dim, rows, nc);
+        if (e != hipSuccess) return e;
+        done += nc;
+    }
     while (mfma_cols && done < ncol) {
         uint32_t nc = ncol - done < mfma_cols ? ncol - done : mfma_cols;
         hipError_t e = lev_q4_k_mfma_gemv_launch(ctx, w, x + (uint64_t)done * in_dim, gain, eps,

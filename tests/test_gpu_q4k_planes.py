@@ -39,3 +39,31 @@ def test_q4k_sliced_rows(rows, ncol, blocks):
         again = ctx.q4_k_gemv_ncol(dw, dx, cols, rows, ncol, gain=dg).cpu().numpy()
         assert np.array_equal(again.view(np.uint32), got.view(np.uint32))
     ctx.close()
+
+
+@pytest.mark.parametrize("blocks,rows,ncol", [(17, 700, 5), (33, 300, 3), (47, 1000, 8), (64, 50, 6)])
+def test_q4_k_wide_columns_record_the_eager_values(blocks, rows, ncol):
+    """Recorded on a context without scratch, where the planes have no room, a row too wide to be staged by fours is
+    taken by ones and twos.  Both ways a sum is exact but for the order of f64 additions in front of its one rounding to
+    f32 (2^-53 against 2^-24: the same bits for all but one value in 10^8)."""
+    from leviathan_amd import ops
+    cols = 256 * blocks
+    w = dev(O.synth_q4_k(blocks + rows, rows * blocks, 0.01))
+    x = dev(O.normal(ncol * cols, 7 + ncol).reshape(ncol, cols))
+    gain = dev(O.normal(cols, 3, 1.0, 0.1))
+    want, y = (torch.full((ncol, rows), float("nan"), device="cuda") for _ in range(2))
+    eager, fresh = ops.Context(0), ops.Context(0, own_stream=True)
+    eager.q4_k_gemv_ncol(w, x, cols, rows, ncol, gain=gain, y=want)
+    torch.cuda.synchronize()
+    fresh.program_begin()
+    fresh.q4_k_gemv_ncol(w, x, cols, rows, ncol, gain=gain, y=y)
+    program = fresh.program_end()
+    for _ in range(3):
+        y.fill_(float("nan"))
+        torch.cuda.synchronize()
+        program.run()
+        fresh.sync()
+        assert torch.equal(y.view(torch.int32), want.view(torch.int32))
+    program.destroy()
+    fresh.close()
+    eager.close()
