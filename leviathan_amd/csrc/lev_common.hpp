@@ -210,9 +210,10 @@ __device__ __forceinline__ void lev_barrier_lds() {
     asm volatile("s_barrier" ::: "memory");
 }
 
-// 1/sqrt(a) of a positive f64: the hardware estimate and two Newton steps (error of a few f64 ulps), a
-// handful of dependent instructions where the square root and the division of the library take over a
-// hundred, all of them on the critical path of a one-workgroup kernel.
+// 1/sqrt(a) of a positive f64 that is rounded to f32 next: the hardware estimate and two Newton steps (error of a few
+// f64 units, so another f32 than the exact value's for one a in some 10^8), a handful of dependent instructions
+// where the square root and the division of the library take over a hundred, all of them on the critical path
+// of a one-workgroup kernel.
 __device__ __forceinline__ double lev_rsqrt_f64(double a) {
     const double est = __builtin_amdgcn_rsq(a);
     double r = est;

@@ -52,13 +52,13 @@ __device__ __forceinline__ int dpp_addi(int v) {
 
 // R: 16-byte pieces of the column a thread keeps in registers (the whole column); gains are requested with them,
 // so that a call is one trip to memory.  R = 0: any length, values beyond the first pass read again.
-// Measured, one column of 4096: 3.7 us with the gains behind the sum, f64 shuffles and the library's f64 root
-// and division, 2.9 with this.
+// Measured, one column of 4096: 3.2 us with the gains behind the sum and f64 shuffles, 2.7 with this (2.5 with an
+// estimate and Newton steps in place of the f64 root and divisions, which round the last bits otherwise).
 template <int R>
 __global__ void __launch_bounds__(kNQThreads)
 norm_quant_kernel(float *__restrict__ x, const float *__restrict__ add,
                   const float *__restrict__ gain, float eps, uint32_t *__restrict__ xq,
-                  float *__restrict__ xs, float *__restrict__ y_out, uint32_t n, double inv_n) {
+                  float *__restrict__ xs, float *__restrict__ y_out, uint32_t n) {
     __shared__ double s_part[kNQThreads / 64];
     const uint32_t col = blockIdx.x, t = threadIdx.x, nt = blockDim.x, lane = t & 63u;
     const uint32_t n4 = n >> 2;
@@ -111,7 +111,7 @@ norm_quant_kernel(float *__restrict__ x, const float *__restrict__ add,
             lev_barrier_lds();   // (the gains may still be on their way)
             double tot = 0.0;
             for (uint32_t k = 0; k < nt >> 6; ++k) tot += s_part[k];
-            inv = lev_rsqrt_f64(tot * inv_n + (double)eps);
+            inv = 1.0 / sqrt(tot / (double)n + (double)eps);   // as the oracle rounds it: codes hang on it
         }
     }
     // whole passes: every lane takes part in the group reductions
@@ -987,7 +987,7 @@ extern "C" int lev_hip_norm_quant_q8(lev_ctx *ctx, float *d_x, size_t x_count, c
     const uint32_t pieces = (n / 4u + 63u) / 64u, threads = 64u * (pieces < 16u ? pieces : 16u);
 #define LEV_NQ(R)                                                                                                 \
     hipLaunchKernelGGL((norm_quant_kernel<R>), dim3(ncol), dim3(threads), 0, ctx->stream, d_x, d_add, d_gain, eps, \
-                       reinterpret_cast<uint32_t *>(d_xq), d_xs, d_y, n, 1.0 / (double)n)
+                       reinterpret_cast<uint32_t *>(d_xq), d_xs, d_y, n)
     if (pieces <= 16u) LEV_NQ(1);
     else if (pieces <= 32u) LEV_NQ(2);
     else if (pieces <= 64u) LEV_NQ(4);
