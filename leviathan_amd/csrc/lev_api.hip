@@ -635,7 +635,12 @@ extern "C" int lev_hip_program_end(lev_ctx *ctx, lev_program **out) {
     p->graph = graph;
     (void)hipGraphGetNodes(graph, nullptr, &p->nodes);
     p->nodes += ctx->folded_nodes;   // counted as recorded: an operator each
-    hipError_t e = fuse_norm_chains(graph);
+    hipError_t e;
+    try {
+        e = fuse_norm_chains(graph);
+    } catch (const std::bad_alloc &) {   // (its lists of nodes; nothing leaves a C entry as an exception)
+        e = hipErrorOutOfMemory;
+    }
     if (e == hipSuccess) e = hipGraphInstantiate(&p->exec, graph, nullptr, nullptr, 0);
     if (e != hipSuccess) {
         (void)hipGraphDestroy(graph);
