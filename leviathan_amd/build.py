@@ -1,7 +1,8 @@
 """Builds ``libleviathan_hip.so`` (gfx950 only) from ``csrc/*.hip`` with hipcc, and with the host compiler
 ``_lev_ops.so``, the argument handling of ``ops.py``, from ``csrc/py_ops.cpp``.
 
-Run ``python -m leviathan_amd.build``.  hipcc cross-compiles without a GPU.
+Run ``python -m leviathan_amd.build``.  hipcc cross-compiles without a GPU.  Without torch or a host compiler
+the library alone is built.
 Objects are compiled in parallel and linked into ``leviathan_amd/lib``.
 """
 from __future__ import annotations
@@ -61,15 +62,24 @@ def _compile(src: str, force: bool, extra: list[str]) -> str:
     return obj
 
 
-def _build_ops(force: bool) -> None:
-    """The CPython extension. It names torch's libraries without a path: they are loaded when it is."""
+def _build_ops(force: bool) -> str:
+    """The CPython extension. It names torch's libraries without a path: they are loaded when it is.
+
+    Returns what it lacks where torch or a host compiler is missing, which only ``ops.py`` needs: the C library and
+    its callers do without.
+    """
     import sysconfig
-    from torch.utils import cpp_extension
+    try:
+        from torch.utils import cpp_extension
+    except ImportError:
+        return "torch"
     src = os.path.join(CSRC, "py_ops.cpp")
     if (not force and os.path.exists(OPS_PATH)
             and os.path.getmtime(OPS_PATH) >= max(os.path.getmtime(src), _headers_mtime())):
-        return
-    cxx = os.environ.get("CXX") or shutil.which("g++") or "g++"
+        return ""
+    cxx = shutil.which(os.environ.get("CXX") or "g++")
+    if not cxx:
+        return "a C++ compiler (g++, or the one CXX names)"
     tmp = OPS_PATH + ".tmp"
     cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-fvisibility=hidden",
            *(a for p in (*cpp_extension.include_paths(), sysconfig.get_paths()["include"]) for a in ("-isystem", p)),
@@ -79,6 +89,7 @@ def _build_ops(force: bool) -> None:
     if res.returncode != 0:
         raise RuntimeError(f"g++ failed for {src}:\n{res.stderr}")
     os.replace(tmp, OPS_PATH)
+    return ""
 
 
 def build(force: bool = True, jobs: int = 8, extra_flags: list[str] | None = None) -> str:
@@ -93,7 +104,9 @@ def build(force: bool = True, jobs: int = 8, extra_flags: list[str] | None = Non
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stderr}")
     os.replace(tmp, LIB_PATH)
-    _build_ops(force)
+    lacks = _build_ops(force)
+    if lacks:
+        sys.stderr.write(f"{os.path.basename(OPS_PATH)}, which leviathan_amd.ops loads, is not built: it needs {lacks}\n")
     return LIB_PATH
 
 

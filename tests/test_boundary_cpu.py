@@ -148,3 +148,19 @@ def test_no_kernel_state_is_kept_per_process():
                 setters.append(name)
     assert not kept
     assert setters == ["lev_common.hpp"]
+
+
+@pytest.mark.parametrize("missing", ["torch", "compiler"])
+def test_the_library_builds_without_what_only_python_callers_need(missing, monkeypatch, tmp_path):
+    """The extension behind ops.py takes torch's headers and a host compiler; without them it is left out and named."""
+    import sys
+    from leviathan_amd import build
+    monkeypatch.setattr(build, "OPS_PATH", str(tmp_path / "_lev_ops.so"))
+    if missing == "torch":
+        monkeypatch.setitem(sys.modules, "torch", None)
+        monkeypatch.setitem(sys.modules, "torch.utils", None)
+    else:
+        monkeypatch.setenv("CXX", str(tmp_path / "no-such-compiler"))
+    lacks = build._build_ops(True)
+    assert missing in lacks
+    assert not os.path.exists(build.OPS_PATH)
