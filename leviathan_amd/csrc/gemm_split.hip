@@ -77,6 +77,7 @@ struct weights_q4k {
 // the chip, 45 without the loads.  So the wave fetches in the order of memory, from the dword that a block
 // starts in: 14 pieces of 16 bytes a row (the last one ends with the block: bytes 196 .. 211), seven loads of
 // 1 KB, parks them in an area of its own and reads every dword it needs back, shifted by the row's two bytes.
+// (Of the dwords in which the matrix begins and ends two bytes may not be its own: read with the others, never used.)
 struct weights_q6k {
     static constexpr int kLoads = 7;
     static constexpr uint32_t kRow = 240u;   // 224 bytes of pieces + 16: the 32 rows start in different banks

@@ -265,12 +265,6 @@ int lev_check_matvec(lev_ctx *ctx, const char *op, uint32_t block_values, uint32
 
 namespace {
 
-// One workgroup of up to 16 waves per vector.  Sum of squares in f32 per lane, wave DPP sums, f64 across
-// waves; y = x * inv * w.  A call on one vector is latency and nothing else (11 KB at n = 2816), so the
-// vector and the gains are requested together, 16 bytes a lane, and x stays in registers between the two
-// passes: one memory round trip.  V = 16-byte pieces a lane holds; V = 0 takes any length and alignment,
-// a float at a time, and reads x twice.  Measured in a recorded chain of 56 operators with three of these a
-// layer: 276 us with 256 threads that read x twice and the library's f64 root and division, 189 with this.
 // What follows an RMSNorm in a recorded program: y += c[k] * x[k], in order (see fuse_norm_chains).
 struct norm_adds {
     static constexpr int kMost = 4;
@@ -279,6 +273,13 @@ struct norm_adds {
     int count;
 };
 
+// One workgroup of up to 16 waves per vector.  Sum of squares in f32 per lane, wave DPP sums, f64 across
+// waves; y = x * inv * w.  A call on one vector is latency and nothing else (11 KB at n = 2816), so the
+// vector and the gains are requested together, 16 bytes a lane, and x stays in registers between the two
+// passes: one memory round trip.  V = 16-byte pieces a lane holds; V = 0 takes any length and alignment,
+// a float at a time, and reads x twice.  Measured in a recorded chain of 56 operators with three of these a
+// layer: 276 us with 256 threads that read x twice and the library's 1 / sqrt in f64, 189 with this (the mean is
+// still an f64 division).
 template <int V, bool ADDS>
 __device__ __forceinline__ void rmsnorm_vector(const float *__restrict__ x, float *__restrict__ y, const float *__restrict__ w,
                                                uint32_t n, float eps, const norm_adds &adds) {

@@ -17,6 +17,11 @@
 // (X + 0x808080) ^ 0x808080 read as int8).  The integer sums are exact; a block's planes are
 // recombined and scaled by d in f32, so what is rounded is one number per block of 32 weights.
 //
+// Against 64-bit sums, on normal activations: 6e-8 to 8e-8 (2-norm) over rows of 480 to 8000 values, where the f32
+// chains of the vector-ALU kernels leave 2.0e-7 to 3.3e-7.  What the integers do not have is f32's range: a value far
+// below the largest of its 64 keeps multiples of 2^-31 of that maximum, which is all that a row has where the weight of
+// the maximum is zero, and below a maximum of 2^-93 the unit stays 2^-123.
+//
 // A wave stages the 256 activations of its own task by itself (one float4 per lane, a 1 KB area
 // of LDS nobody else touches): no workgroup barrier stands between the activations and the
 // products, and the A operands (16 registers a task) serve every row group the wave visits.

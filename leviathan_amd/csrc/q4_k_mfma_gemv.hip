@@ -40,6 +40,10 @@
 // Five to eight columns, or three and more of a row of more than sixteen superblocks: the planes are made
 // once per launch by a small kernel in front (q4k_planes_kernel, below) instead of by every workgroup.
 //
+// Against 64-bit sums, on normal activations: 5e-8 to 6e-8 (2-norm); the f32 chains of the vector-ALU kernel, which
+// three and more columns of rows wider than 8192 take without planes, leave 1.4e-7.  A value far below the largest of its
+// superblock keeps multiples of 2^-26 of that maximum.
+//
 // A NaN or infinity in a column of x makes every output of that column NaN.
 #include "lev_common.hpp"
 
