@@ -687,10 +687,11 @@ hipError_t lev_moe_merge_launch(lev_ctx *ctx, const lev_moe_grouped_args &a, con
 // 60: 15 tokens 50, 45; 3072 / 1408, top-6 of 256: 8 tokens 97, 89; 12 tokens 128, 134); with a selection in front 65 MB
 // (2816 / 704: 16 tokens 89, 109; 1408 / 320, top-4 of 64: 16 tokens 39, 31; 64 tokens 50, 57; 1024 / 576, top-2 of 32:
 // 32 tokens 34, 31; 64 tokens 36, 45).
-// Rows of whole 256-value tasks up to 2048 wide are grouped from five tokens on whatever that saves, as they were before
-// there was this line: from twelve tokens on the two are level there, below the line would be the better choice (us a
-// layer, grouped against pair by pair: 2048 / 768, top-8 of 128: 5 tokens 41, 26; 8 tokens 45, 33; 10 tokens 49, 39;
-// 12 tokens 53, 52; 15 tokens 58, 58; 1536 / 768, top-4 of 60: 5 tokens 31, 16; 15 tokens 40, 28).
+// Rows of whole 256-value tasks up to 2048 wide are grouped from five tokens on whatever that saves: from there up to
+// eight pairs per expert a token's bits do not depend on how many travel with it (up to four tokens and beyond
+// eight pairs other kernels run, and the last bits differ).  It is not for speed: the line above would choose better
+// below twelve tokens (us a layer, grouped against pair by pair: 2048 / 768, top-8 of 128: 5 tokens 41, 26; 8 tokens 45,
+// 33; 10 tokens 49, 39; 12 tokens 53, 52; 15 tokens 58, 58; 1536 / 768, top-4 of 60: 5 tokens 31, 16; 15 tokens 40, 28).
 bool lev_moe_grouped_usable(const lev_ctx *ctx, const lev_moe_grouped_args &a, bool selects) {
     if (!lev_moe_prefill_usable(a)) return false;
     if (a.hidden % 256u == 0u && a.inter % 256u == 0u && a.hidden <= 2048u && a.inter <= 2048u) return true;

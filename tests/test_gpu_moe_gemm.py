@@ -344,7 +344,7 @@ def test_moe_grouped_path_many_tokens(ctx, experts, tokens, again):
                 ids[t] = [3, 5 + t % 30, 4 if t % 10 else 36, 37 + t % 3]
         for t in range(tokens):
             assert len(set(ids[t].tolist())) == top_k
-    # which kernels a batch takes (integer matrix cores up to 5.5 pairs per expert on average)
+    # which kernels a batch takes (integer matrix cores up to 5.5 pairs per expert on average, eight from 32 experts on)
     assert (2 * tokens * top_k <= 11 * experts) == (2 * again * top_k <= 11 * experts)
     wts = rng.random((tokens, top_k)).astype(np.float32)
     y, act = run_experts(ctx, pool, offs, hidden, inter, experts, x, ids, wts)
@@ -363,7 +363,7 @@ def test_moe_non_finite_activation_stays_in_its_token(ctx, experts, tokens, top_
     """A NaN or an infinity in one token's activations makes every output of THAT token non-finite
     (as the reference's f32 dot products do: each of them contains the element) and leaves the
     other tokens' bits alone, on the per-pair kernels (2 tokens), the integer grouped kernels
-    (6 tokens over 16 experts) and the fp16 grouped kernels (12 tokens over 4 experts)."""
+    (6 tokens over 16 experts) and the grouped matrix product (12 tokens over 4 experts)."""
     hidden, inter = 256, 256
     wr, pool, offs, x = H.config5(hidden, inter, experts, tokens, seed=91 + tokens)
     rng = np.random.default_rng(91 + tokens)
@@ -385,7 +385,7 @@ def test_moe_non_finite_activation_stays_in_its_token(ctx, experts, tokens, top_
 def test_moe_block_scale_edge_cases(ctx, experts, tokens, top_k):
     """Block scales the synthetic pools do not draw: zero, negative, the smallest fp16 subnormal
     and a large one, sprinkled over every matrix, and activations spanning forty-six binades within a
-    row; the three schedules (per-pair, integer grouped, fp16 grouped) against the FP64 chain."""
+    row; the three schedules (per-pair, integer grouped, grouped product) against the FP64 chain."""
     hidden, inter = 256, 256
     wr, pool, offs, x = H.config5(hidden, inter, experts, tokens, seed=311 + tokens)
     pool = pool.copy()
@@ -524,9 +524,9 @@ def test_moe_layer_config5(ctx, tokens):
     # batch invariance (main.swift:9053-9056: a schedule gives the same bits whatever
     # else is in the batch).  Three schedules exist here: up to four tokens every
     # (token, slot) streams its expert alone; from five tokens pairs are grouped
-    # by expert on the matrix cores, by the integer kernels up to 5.5 pairs per
-    # expert on average (64 and 8 tokens over 128 experts both) and by the fp16
-    # kernels beyond.  Within a schedule a token's bits do not depend on the rest
+    # by expert on the matrix cores, by the integer kernels up to eight pairs per
+    # expert on average (64 and 8 tokens over 128 experts both) and by the grouped
+    # matrix product beyond.  Within a schedule a token's bits do not depend on the rest
     # of the batch; across schedules the same token agrees to the
     # summation-order noise.
     if tokens > 1:

@@ -115,7 +115,7 @@ def test_recorded_step_replays_bit_exact():
 @pytest.mark.parametrize("experts", [12, 16])
 def test_recorded_prefill_like_sequence_replays_bit_exact(experts):
     """f32 -> f16, the two prefill GEMMs (first use of the kernels happens while recording),
-    grouped MoE over 24 tokens (72 pairs: over 12 experts the fp16 grouped kernels, over 16 the
+    grouped MoE over 24 tokens (72 pairs: over 12 experts the grouped matrix product, over 16 the
     integer ones with their work items and start records), and a Q4_0 GEMV under a forge selection
     made before recording: three replays with changed inputs equal the eager results bit for bit."""
     from leviathan_amd import capi, ops
