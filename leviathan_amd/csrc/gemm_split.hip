@@ -413,6 +413,15 @@ hipError_t launch(lev_ctx *ctx, const uint8_t *w, const uint16_t *x, float *y, u
 //   KW = 1:           a round of up to two workgroups a CU; their steps take 1.6 times those of one alone;
 //   KW = 2, KW = 4:   a round of one a CU, and with S > 1 splits the kernel that adds and its reads and writes.
 // Lower token tiles are more workgroups that decode the same weights: what fills the chip where rows alone do not.
+// Beyond 1024 tokens the times of KW = 1 outgrow these, by 1.1 to 1.45, with the tokens that its tiles really hold
+// (those of 256 tokens stay within 0.87 to 1.1).  Over 216 shapes of 1025 to 8192 tokens the 256-token tiles were the
+// faster ones where nearly every token of them is one and the CUs are full: for Q6_K from 15/16 of the CUs (4096 x 4096 at
+// 4096 tokens 174.7 us against 187.2, 32000 x 4096 at 4096 tokens 1361 against 1449), unless the weights are more than
+// the 256 MB that the Infinity Cache holds (32000 rows of 12288 at 3072 tokens 4 % more); for Q4_K from 31/32 of them and
+// eight token tiles (12288 x 4096 at 4096 tokens 469 us against 505, at 2048 tokens 236 against 242), but not over short
+// rows (16384 rows of 1024 at 8192 tokens 2 % more), and where the estimates are within 1.1 (12288 x 4096 at 1500 tokens
+// 180 us against 193).  47 shapes of Q6_K and 23 of Q4_K are faster so, by some 4 % on average and none slower by more
+// than 0.4 %; Q4_K at 2048 tokens is between 2.7 % faster and 1.5 % slower, by the shape and the card's clock.
 // Tall matrices (768 row tiles and more) and rows of fewer than six superblocks are never cut along K, so that
 // there every kernel adds in the same order.
 lev_gemm_split_plan lev_gemm_split_choose(const lev_ctx *ctx, bool q6, uint32_t in_dim, uint32_t rows, uint32_t tokens,
@@ -423,6 +432,13 @@ lev_gemm_split_plan lev_gemm_split_choose(const lev_ctx *ctx, bool q6, uint32_t 
     const double big_rounds = std::ceil(big_wgs / cus), fill = big_wgs / (big_rounds * cus);
     lev_gemm_split_plan best{0u, 1u, 1u};
     double least = big_rounds * (q6 ? 5.7 + in_dim / 1024.0 * (19.2 + 3.5 * fill) : 6.1 + in_dim / 1024.0 * (9.8 + 3.8 * fill));
+    if (tokens > 1024u) {
+        const uint64_t tiled = (tokens + 255ull) / 256u * 256u;
+        if (tokens * 32ull >= tiled * 31u && (q6 ? fill >= 15.0 / 16.0 && (uint64_t)in_dim * rows <= 1u << 28
+                                                 : fill >= 31.0 / 32.0 && in_dim >= 2048u && tiled >= 2048u))
+            return best;
+        if (!q6) least /= 1.1;
+    }
     struct cost { double start, step, per_tile, full, sum, sum_mb; };
     const cost k1 = q6 ? cost{4.9, 0.383, 0.067, 0.60, 0, 0} : cost{4.0, 0.267, 0.076, 0.66, 0, 0};
     const cost k2 = q6 ? cost{4.3, 0.558, 0.145, 0.16, 3.1, 0.7} : cost{3.9, 0.363, 0.165, 0.08, 2.9, 0.75};

@@ -82,3 +82,27 @@ def test_gemm_split_records_the_eager_bits(ctx, kind, rows, cols, tokens):
         assert np.array_equal(y.cpu().numpy().view(np.uint32), eager.reshape(tokens, rows).view(np.uint32))
     program.destroy()
     fresh.close()
+
+
+@pytest.mark.parametrize("kind,rows,cols,tokens", [
+    ("q6_k", 32000, 1024, 1250),     # 250 row tiles: five token tiles of a workgroup one after the other, the last ragged
+    ("q6_k", 16384, 1280, 1510),     # 128 row tiles: two token tiles side by side, three in turn
+    ("q6_k", 6140, 1024, 1270),      # one round of 240 workgroups, the last row tile ragged
+    ("q4_k", 24570, 2048, 2290),     # nine rounds, ragged in rows and tokens
+    ("q4_k", 12288, 2048, 1985),     # eight token tiles, the last one ragged
+    ("q4_k", 12288, 2048, 1500),     # three rounds: the estimates within 1.1 of each other
+])
+def test_gemm_long_prompts_in_256_token_tiles(ctx, kind, rows, cols, tokens):
+    """Prompts above 1024 tokens whose 256-token tiles fill the chip: each tile is the product of its tokens alone, which
+    the 128-token kernel forms in the same order where it never cuts K (from 768 row tiles, below six superblocks), bit
+    for bit; sampled rows meet the gate."""
+    w, x = (H.config4 if kind == "q4_k" else config4_q6)(rows, cols, tokens, seed=rows + tokens)
+    run = gemm if kind == "q4_k" else gemm6
+    got = run(ctx, w, x, rows, cols, tokens)
+    whole = rows > 767 * 32 or cols < 6 * 256
+    for lo in (0, tokens // 512 * 256, tokens // 256 * 256) if whole else ():
+        hi = min(lo + 256, tokens)
+        part = run(ctx, w, x[lo:hi].copy(), rows, cols, hi - lo)
+        assert np.array_equal(part.view(np.uint32), got[lo:hi].view(np.uint32)), (lo, hi)
+    oracle = O.q4_k_gemm_f16_oracle if kind == "q4_k" else O.q6_k_gemm_f16_oracle
+    assert O.max_rel_err(got[:, 0::499], oracle(w, rows, cols, x.view(np.uint16), tokens, 0, 499)) < GEMM_TOL
