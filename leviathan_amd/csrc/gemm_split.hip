@@ -416,8 +416,8 @@ hipError_t launch(lev_ctx *ctx, const uint8_t *w, const uint16_t *x, float *y, u
 // Beyond 1024 tokens the times of KW = 1 outgrow these, by 1.1 to 1.45, with the tokens that its tiles really hold
 // (those of 256 tokens stay within 0.87 to 1.1).  Over 216 shapes of 1025 to 8192 tokens the 256-token tiles were the
 // faster ones where nearly every token of them is one and the CUs are full: for Q6_K from 15/16 of the CUs (4096 x 4096 at
-// 4096 tokens 174.7 us against 187.2, 32000 x 4096 at 4096 tokens 1361 against 1449), unless the weights are more than
-// the 256 MB that the Infinity Cache holds (32000 rows of 12288 at 3072 tokens 4 % more); for Q4_K from 31/32 of them and
+// 4096 tokens 174.7 us against 187.2, 32000 x 4096 at 4096 tokens 1361 against 1449), unless there are more than 2^28
+// weights (220 MB, about what the Infinity Cache holds: 32000 rows of 12288 at 3072 tokens 4 % more); for Q4_K from 31/32 of them and
 // eight token tiles (12288 x 4096 at 4096 tokens 469 us against 505, at 2048 tokens 236 against 242), but not over short
 // rows (16384 rows of 1024 at 8192 tokens 2 % more), and where the estimates are within 1.1 (12288 x 4096 at 1500 tokens
 // 180 us against 193).  47 shapes of Q6_K and 23 of Q4_K are faster so, by some 4 % on average and none slower by more
