@@ -239,11 +239,27 @@ __device__ __forceinline__ uint32_t lev_lds_offset(const void *lds) {
     return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const uint8_t *)lds;
 }
 
+// Loads from `bytes` bytes at a wave-uniform base by 32-bit offset.  A lane whose offset is kNothing gets zeros and asks
+// the memory for nothing.  `fixed` is a constant, `uniform` the same for all lanes; the sum is checked against
+// `bytes`, for which kNothing leaves room on both sides (bytes, fixed and uniform at most 2^30).
+struct lev_buffer {
+    static constexpr uint32_t kNothing = 0x80000000u;
+    __amdgpu_buffer_rsrc_t rsrc;
+    __device__ __forceinline__ lev_buffer(const void *base, uint32_t bytes)
+        : rsrc(__builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)bytes, 0x00020000)) {}
+    __device__ __forceinline__ lev_u32x4 load16(uint32_t offset, int fixed, uint32_t uniform = 0u) const {
+        return __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)offset + fixed, (int)uniform, 0);
+    }
+    __device__ __forceinline__ uint32_t load4(uint32_t offset, int fixed, uint32_t uniform = 0u) const {
+        return __builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)offset + fixed, (int)uniform, 0);
+    }
+};
+
 // ---- shared by the kernels in which a wave owns one column block of the matrix (a Q4_0 task,
 // a Q4_K or Q6_K superblock column) and `wpr` waves of a workgroup of 16 cover a row ----
 
 // Sum over lanes l, l ^ 16, l ^ 32, l ^ 48 (the four lane groups of a matrix-core row), in every
-// lane, in f64, by two row swaps per dword: no LDS.
+// lane, in f64 or f32, by two row swaps per dword: no LDS.
 __device__ __forceinline__ double lev_row_sum_f64(double v) {
     uint32_t lo = (uint32_t)__double2loint(v), hi = (uint32_t)__double2hiint(v);
     auto a0 = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
@@ -254,6 +270,35 @@ __device__ __forceinline__ double lev_row_sum_f64(double v) {
     a0 = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
     a1 = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
     return __hiloint2double((int)a1[0], (int)a0[0]) + __hiloint2double((int)a1[1], (int)a0[1]);
+}
+
+__device__ __forceinline__ float lev_row_sum_f32(float v) {
+    const uint32_t u = __float_as_uint(v);
+    const auto s0 = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    v = __uint_as_float(s0[0]) + __uint_as_float(s0[1]);
+    const uint32_t u2 = __float_as_uint(v);
+    const auto s1 = __builtin_amdgcn_permlane16_swap(u2, u2, false, false);
+    return __uint_as_float(s1[0]) + __uint_as_float(s1[1]);
+}
+
+// out[i] = what lane FIRST + i of the lane's row of 16 holds (DPP row_newbcast).
+template <int LANE>
+__device__ __forceinline__ float lev_row_bcast(uint32_t v) {
+    return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x150 + LANE, 0xF, 0xF, false));
+}
+template <int N, int FIRST = 0, int I = 0>
+__device__ __forceinline__ void lev_row_spread(uint32_t v, float (&out)[N]) {
+    if constexpr (I < N) {
+        out[I] = lev_row_bcast<FIRST + I>(v);
+        lev_row_spread<N, FIRST, I + 1>(v, out);
+    }
+}
+template <int N, int FIRST = 0, int I = 0>
+__device__ __forceinline__ void lev_row_spread(const lev_u32x4 v, lev_f32x4 (&out)[N]) {
+    if constexpr (I < N) {
+        out[I] = lev_f32x4{lev_row_bcast<FIRST + I>(v.x), lev_row_bcast<FIRST + I>(v.y), lev_row_bcast<FIRST + I>(v.z), lev_row_bcast<FIRST + I>(v.w)};
+        lev_row_spread<N, FIRST, I + 1>(v, out);
+    }
 }
 
 // Largest of an unsigned value over the 16 lanes of a row of the wave, in every lane of the row:

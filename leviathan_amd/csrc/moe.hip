@@ -1144,8 +1144,8 @@ moe_gate_up_mfma(moe_args a, const float *__restrict__ x, const int32_t *ids, co
         float vg = q4m_task_dot(W, op);
         q4m_turn_task(Du, W);
         float vu = q4m_task_dot(W, op);
-        vg = q4m_row_sum(vg);
-        vu = q4m_row_sum(vu);
+        vg = lev_row_sum_f32(vg);
+        vu = lev_row_sum_f32(vu);
         if (lane < 16u) {
             *reinterpret_cast<float *>(smem + pw) = vg;
             *reinterpret_cast<float *>(smem + pw + kUp) = vu;
@@ -1162,8 +1162,8 @@ moe_gate_up_mfma(moe_args a, const float *__restrict__ x, const int32_t *ids, co
                 g += pg[192];
                 u += pu[192];
             }
-            g = q4m_row_sum(g);
-            u = q4m_row_sum(u);
+            g = lev_row_sum_f32(g);
+            u = lev_row_sum_f32(u);
             if (q == 0u && i_here + r16 < i_end) arow[i_here + r16] = lev_gelu_up_value(g, u);
         }
         pw ^= kPart;                                              // the other half of `part` next round
@@ -1258,7 +1258,7 @@ moe_down_mfma(moe_args a, const float *__restrict__ act, const int32_t *__restri
             q4m_turn_task(D[k], W);
             val += q4m_task_dot(W, op[k]);
         }
-        val = q4m_row_sum(val);
+        val = lev_row_sum_f32(val);
         if (lane < 16u) partial[slot * 16u + lane] = val;
     }
     if (bad && lane == 0) atomicOr(flag, kFlagBadExpertId);

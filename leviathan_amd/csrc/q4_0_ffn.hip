@@ -89,9 +89,9 @@ q4_0_ffn_gate_up(ffn_args a) {
         const uint32_t next = i0 + 16u;
         issue(next < i_end ? next : i0, Gb, Ub);                  // unconditional (clamped)
         q4m_turn_task(Ga, W);
-        const float vg = q4m_row_sum(q4m_task_dot(W, op));
+        const float vg = lev_row_sum_f32(q4m_task_dot(W, op));
         q4m_turn_task(Ua, W);
-        const float vu = q4m_row_sum(q4m_task_dot(W, op));
+        const float vu = lev_row_sum_f32(q4m_task_dot(W, op));
         if (lane < 16u) {
             *reinterpret_cast<float *>(smem + pw) = vg;
             *reinterpret_cast<float *>(smem + pw + kFfnUp) = vu;
@@ -105,8 +105,8 @@ q4_0_ffn_gate_up(ffn_args a) {
                 g += pg[64 * k];
                 u += pu[64 * k];
             }
-            g = q4m_row_sum(g);
-            u = q4m_row_sum(u);
+            g = lev_row_sum_f32(g);
+            u = lev_row_sum_f32(u);
             const uint32_t row = i0 + r16;
             if (q == 0u && row < i_end) {
                 a.gu[row] = g;

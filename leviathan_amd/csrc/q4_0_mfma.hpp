@@ -191,15 +191,3 @@ __device__ __forceinline__ float q4m_task_dot(const uint32_t W[9], const q4m_ope
     const float fb = fmaf((float)(sb[2] + (sb[3] << 8)), 65536.0f, (float)(sb[0] + (sb[1] << 8)));
     return fmaf(da, fa, db * fb) * op.unscale;
 }
-
-// Sum over lanes l, l ^ 16, l ^ 32, l ^ 48 (the four lane groups of a row), in every lane,
-// by two row swaps: no LDS.
-__device__ __forceinline__ float q4m_row_sum(float v) {
-    const uint32_t u = __float_as_uint(v);
-    const auto s0 = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-    v = __uint_as_float(s0[0]) + __uint_as_float(s0[1]);
-    const uint32_t u2 = __float_as_uint(v);
-    const auto s1 = __builtin_amdgcn_permlane16_swap(u2, u2, false, false);
-    return __uint_as_float(s1[0]) + __uint_as_float(s1[1]);
-}
-

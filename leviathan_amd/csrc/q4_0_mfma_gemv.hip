@@ -161,7 +161,7 @@ q4_0_mfma_gemv(const uint8_t *__restrict__ w, const float *__restrict__ x, float
             }
             val += q4m_task_dot(W, op[kKept ? t : 0]);
         }
-        val = q4m_row_sum(val);
+        val = lev_row_sum_f32(val);
         if (lane < 16u) *reinterpret_cast<float *>(smem + pw) = val;
         lev_barrier_lds();
         if (wave < slots) {
@@ -169,7 +169,7 @@ q4_0_mfma_gemv(const uint8_t *__restrict__ w, const float *__restrict__ x, float
             const float p0 = pp[0], p1 = pp[64], p2 = pp[128], p3 = pp[192];   // four reads in flight together
             auto keep = [](float p, uint32_t k) { return __uint_as_float(__float_as_uint(p) & k); };
             float s = (keep(p0, k0) + keep(p1, k1)) + (keep(p2, k2) + keep(p3, k3));
-            s = q4m_row_sum(s);
+            s = lev_row_sum_f32(s);
             if (stores) *reinterpret_cast<__attribute__((address_space(1))) float *>(yp) = s;   // a global store, not a flat one
         }
         if (!SINGLE) {

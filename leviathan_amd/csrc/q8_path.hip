@@ -721,8 +721,8 @@ q4_k_q8_mfma(const uint8_t *__restrict__ w, const uint8_t *__restrict__ xq, cons
 }
 
 // ---------------------------------------------------------------------------
-// Up to four columns, rows of at most sixteen superblocks, in the shape of the f32 one-column
-// kernel (q4_k_mfma_gemv_one.hip): a wave owns ONE superblock column of the matrix.  Lane (r, g)
+// Up to eight columns of rows of at most sixteen superblocks, up to four of rows of at most twenty-four, in the shape of the
+// f32 one-column kernel (q4_k_mfma_gemv_one.hip): a wave owns TPW superblock columns of the matrix.  Lane (r, g)
 // multiplies chunk g (32 code bytes: low nibbles = sub-block 2g, high = 2g+1) of row r by four
 // v_mfma_i32_16x16x64_i8; A row 4g + c holds the 16 activation codes of column c (of a chunk of
 // four columns) that lane group g multiplies, zeros elsewhere, so the four accumulator registers
@@ -731,25 +731,45 @@ q4_k_q8_mfma(const uint8_t *__restrict__ w, const uint8_t *__restrict__ xq, cons
 // the scales and sums of its two blocks beside them: nothing is staged in LDS, no barrier stands
 // in front of the products.  The wave walks the row groups with the next group's weights in
 // flight; the partial sums of a row meet in LDS behind one barrier per round.
+// NC is the number of columns and not their multiple of four: a second chunk of one column costs a quarter of the scaling
+// that a full one does.
 // Weights: lane 4*row + c fetches dword c of the superblock's header and the 32 aligned bytes of
 // chunk c (a quad reads the row's 144 contiguous bytes); one lane permutation per dword hands them
 // to lane (row, c).
-// LDS: part [2][16 waves][16 rows][NC] f32.
+// LDS: part [2][waves][16 rows][NC] f32, and room for the masked reads behind a slot's last wave.
 // ---------------------------------------------------------------------------
-__host__ __device__ constexpr uint32_t q8m_one_part_bytes(uint32_t nc) { return 2u * kMWaves * 16u * 4u * nc; }
+__host__ __device__ constexpr uint32_t q8m_one_part_bytes(uint32_t nc, uint32_t waves) { return 3u * waves * 16u * 4u * nc; }
 
-// NC: columns staged (a multiple of 4, >= ncol; 4 is what is built).
-template <int NC>
-__global__ void __launch_bounds__(kMThreads)
+// One chunk of up to four columns of a task: v[i] += y of the lane's two sub-blocks.
+template <int N>
+__device__ __forceinline__ void q8m_one_chunk(const lev_i32x4 (&A)[4], const lev_i32x4 la, const lev_i32x4 lb, const lev_i32x4 ha,
+                                              const lev_i32x4 hb, const lev_f32x4 (&xs)[N], float sca, float scb, float mna,
+                                              float mnb, float (&v)[4]) {
+    lev_i32x4 d0 = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[0], la, lev_i32x4{0, 0, 0, 0}, 0, 0, 0);
+    lev_i32x4 d1 = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[2], ha, lev_i32x4{0, 0, 0, 0}, 0, 0, 0);
+    d0 = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[1], lb, d0, 0, 0, 0);
+    d1 = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[3], hb, d1, 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        // y += d*sc_j*dx_j*idot - dmin*m_j*s_j for the lane's two sub-blocks (xs: dx, s of the first, dx, s of the second)
+        float t = fmaf(sca, xs[i].x * (float)d0[i], -mna * xs[i].y);
+        t = fmaf(scb, xs[i].z * (float)d1[i], t);
+        v[i] += fmaf(-mnb, xs[i].w, t);
+    }
+}
+
+template <int NC, int TPW, int NW>
+__global__ void __launch_bounds__(NW * LEV_WAVE)
 q4_k_q8_mfma_one(const uint8_t *__restrict__ w, const uint8_t *__restrict__ xq, const float *__restrict__ xs,
-                 float *__restrict__ y, uint32_t cols, uint32_t rows, uint32_t ncol, uint32_t wpr, uint32_t slots,
+                 float *__restrict__ y, uint32_t cols, uint32_t rows, uint32_t wpr, uint32_t slots,
                  uint64_t slot_of_wave, uint64_t pos_of_wave) {
-    constexpr int NCH = NC / 4;
+    constexpr int NCH = (NC + 3) / 4, N0 = NC < 4 ? NC : 4, N1 = NC > 4 ? NC - 4 : 1;
+    static_assert(NCH <= 2 && (NCH == 1 || TPW == 1), "the operands stay in registers");
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
     const uint32_t slot = (uint32_t)(slot_of_wave >> (4u * wave)) & 15u;   // idle waves: slot >= slots
-    const uint32_t sb = (uint32_t)(pos_of_wave >> (4u * wave)) & 15u;      // the wave's superblock column
+    const uint32_t sb0 = ((uint32_t)(pos_of_wave >> (4u * wave)) & 15u) * TPW;   // the wave's superblock columns
     const uint32_t SB = cols >> 8, nblk = cols >> 5;
     const uint32_t r = lane & 15u, g = lane >> 4;
     const bool active = slot < slots;
@@ -760,11 +780,12 @@ q4_k_q8_mfma_one(const uint8_t *__restrict__ w, const uint8_t *__restrict__ xq, 
     const uint32_t ngroups = (rows + 15u) >> 4;
     const uint32_t nrounds = (ngroups + slots - 1u) / slots;     // rounds of `slots` row groups
     const uint32_t lrow = lane >> 2, lc = lane & 3u;             // fetch order: lane = 4 * row + chunk
-    auto issue = [&](uint32_t round_block, uint32_t (&D)[9]) {
+    auto issue = [&](uint32_t round_block, int t, uint32_t (&D)[9]) {
         uint32_t rg = round_block * slots + (active ? slot : 0u);
         rg = rg < ngroups ? rg : ngroups - 1u;
         uint32_t row = rg * 16u + lrow;
         row = row < rows ? row : rows - 1u;
+        const uint32_t sb = TPW == 1 || sb0 + t < SB ? sb0 + t : SB - 1u;
         const uint8_t *p = w + (uint64_t)row * row_bytes + (uint64_t)sb * 144u;
         D[0] = *reinterpret_cast<const uint32_t *>(p + 4u * lc);
         const lev_u32x4 a = *reinterpret_cast<const lev_u32x4 *>(p + 16u + 32u * lc);
@@ -772,54 +793,60 @@ q4_k_q8_mfma_one(const uint8_t *__restrict__ w, const uint8_t *__restrict__ xq, 
         D[1] = a.x; D[2] = a.y; D[3] = a.z; D[4] = a.w;
         D[5] = b.x; D[6] = b.y; D[7] = b.z; D[8] = b.w;
     };
-    uint32_t D[9];
+    uint32_t D[TPW][9];
     uint32_t rb = blockIdx.x;
-    issue(rb, D);
+#pragma unroll
+    for (int t = 0; t < TPW; ++t) issue(rb, t, D[t]);
     __builtin_amdgcn_sched_barrier(0);
 
     // the wave's activations: lane (r, g) feeds A row r = 4*gs + c, i.e. column 4*ch + r%4, the 16
     // codes 64g + 16h .. of the superblock (h = 0, 1: sub-block 2g; 2, 3: sub-block 2g+1), when
-    // gs == g, zeros otherwise (columns beyond ncol repeat the last one: their scales are zeroed)
-    lev_i32x4 A[NCH][4];
-    float dxa[NCH][4], dxb[NCH][4], sa[NCH][4], sbm[NCH][4];     // scale and sum of blocks 2g and 2g+1, column 4*ch + i
+    // gs == g, zeros otherwise.  The lanes that get zeros ask for nothing: their offset lies behind the buffer's end.
+    // (With an address for every lane, and the scales of a column a load of its own, the activations of eight columns were
+    // 10000 lookups of the L1 a workgroup where the weights of a round are 1300: 12288 x 4096 by eight 11.7 us, 10.2 with
+    // this; 8192 x 1024 8.2 and 6.0.)
+    const lev_buffer codes(xq, cols * NC), scales(xs, nblk * NC * 8u);
+    lev_i32x4 A[TPW][NCH][4];
+    lev_u32x4 xin[TPW];                                          // scale and sum of blocks 2g and 2g+1
 #pragma unroll
-    for (int ch = 0; ch < NCH; ++ch) {
-        const uint32_t ca = 4u * (uint32_t)ch + (r & 3u);
-        const uint8_t *xa = xq + (uint64_t)(ca < ncol ? ca : ncol - 1u) * cols + 256u * sb + 64u * g;
+    for (int t = 0; t < TPW; ++t) {
+        const uint32_t sb = sb0 + t;
+        const bool on = active && (TPW == 1 || sb < SB);
+        const bool feeds = on && (r >> 2) == g;
 #pragma unroll
-        for (int h = 0; h < 4; ++h) A[ch][h] = *reinterpret_cast<const lev_i32x4 *>(xa + 16 * h);
+        for (int ch = 0; ch < NCH; ++ch) {
+            const uint32_t ca = 4u * (uint32_t)ch + (r & 3u);
+            const uint32_t at = feeds && ca < (uint32_t)NC ? ca * cols + 256u * sb + 64u * g : lev_buffer::kNothing;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t ci = 4u * (uint32_t)ch + (uint32_t)i;
-            const lev_f32x4 t = *reinterpret_cast<const lev_f32x4 *>(
-                xs + ((uint64_t)(ci < ncol ? ci : ncol - 1u) * nblk + 8u * sb + 2u * g) * 2u);
-            const bool on = active && ci < ncol;
-            dxa[ch][i] = on ? t.x : 0.f;
-            sa[ch][i] = on ? t.y : 0.f;
-            dxb[ch][i] = on ? t.z : 0.f;
-            sbm[ch][i] = on ? t.w : 0.f;
+            for (int h = 0; h < 4; ++h) A[t][ch][h] = __builtin_bit_cast(lev_i32x4, codes.load16(at, 16 * h));
         }
+        // lane (r, g): column r's, handed to the lane group below
+        xin[t] = scales.load16(on && r < (uint32_t)NC ? r * nblk * 8u + (8u * sb + 2u * g) * 8u : lev_buffer::kNothing, 0);
     }
 
     // ---- everything the tail of a round needs, while the loads are on their way ----
     // byte offsets into the workgroup's LDS, not pointers
     uint32_t pw = ((wave * 16u + r) * NC + g) * 4u;              // lane (r, g): row r, column g (+ 4 per chunk)
-    uint32_t pr = ((((wave < slots ? wave : 0u) * wpr) * 16u + r) * NC + g) * 4u;
-    uint32_t orow = (rb * slots + wave) * 16u + r;
+    // wave s + slots * ch adds up chunk ch of slot s (two chunks: at least two waves share a row)
+    const uint32_t ss = NCH == 2 && wave >= slots ? wave - slots : wave, sch = NCH == 2 && wave >= slots ? 1u : 0u;
+    const bool adds = wave < slots * NCH;
+    const uint32_t ocol = 4u * sch + g;
+    uint32_t pr = ((((adds ? ss : 0u) * wpr) * 16u + r) * NC + (ocol < (uint32_t)NC ? ocol : (uint32_t)NC - 1u)) * 4u;
+    uint32_t orow = (rb * slots + ss) * 16u + r;
     const uint32_t orow_step = gridDim.x * slots * 16u;
-    const bool writer = wave < slots;
+    const bool writer = adds && ocol < (uint32_t)NC;
     uint32_t stores = writer && orow < rows ? 1u : 0u;
-    uint64_t yp = reinterpret_cast<uint64_t>(y + (uint64_t)g * rows + orow);
+    uint64_t yp = reinterpret_cast<uint64_t>(y + (uint64_t)ocol * rows + orow);
     lev_pin(pw);
     lev_pin(pr);
     lev_pin(stores);
     lev_pin(yp);
-    {
-        const bool feeds = active && (r >> 2) == g;
+    uint32_t flip = NW * 16u * 4u * NC;
+    lev_f32x4 xv0[TPW][N0], xv1[N1];                             // column i's, in every lane of the group
 #pragma unroll
-        for (int ch = 0; ch < NCH; ++ch)
-#pragma unroll
-            for (int h = 0; h < 4; ++h) A[ch][h] = feeds ? A[ch][h] : lev_i32x4{0, 0, 0, 0};
+    for (int t = 0; t < TPW; ++t) {
+        lev_row_spread<N0>(xin[t], xv0[t]);
+        if constexpr (NCH == 2) lev_row_spread<N1, 4>(xin[t], xv1);
     }
     __builtin_amdgcn_sched_barrier(0);
 
@@ -827,76 +854,69 @@ q4_k_q8_mfma_one(const uint8_t *__restrict__ w, const uint8_t *__restrict__ xq, 
     // in take the NEXT round's request at once (unconditional, clamped: a branch around the loads
     // would make the compiler wait for them before the current group is multiplied).
     auto round = [&](uint32_t next_block) {
-        // lane (r, g) <- lane 4r + g for the chunk, lanes 4r .. 4r + 3 for the header's four dwords
-        uint32_t hdr[4];
-        lev_u32x4 ca, cb;
+        float v0[4] = {0.f, 0.f, 0.f, 0.f}, v1[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int k = 0; k < 4; ++k) hdr[k] = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(16u * r + 4u * k), (int)D[0]);
-        const int src = (int)((4u * r + g) * 4u);
+        for (int t = 0; t < TPW; ++t) {
+            // lane (r, g) <- lane 4r + g for the chunk, lanes 4r .. 4r + 3 for the header's four dwords
+            uint32_t hdr[4];
+            lev_u32x4 ca, cb;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            ca[k] = (uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)D[1 + k]);
-            cb[k] = (uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)D[5 + k]);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        issue(next_block, D);
-        __builtin_amdgcn_sched_barrier(0);
-        // unpack_scale_min (lev-cpu/src/lib.rs:64-74), four sub-blocks a word; this lane wants sub-blocks
-        // 2g and 2g + 1: bytes 2 * (g % 2) and + 1 of word g / 2 (both words are formed and one is
-        // kept by a bit select: a conditional here becomes a branch)
-        const uint32_t S0 = hdr[1], S1 = hdr[2], S2 = hdr[3];
-        const uint32_t up = g >= 2u ? ~0u : 0u;
-        const uint32_t sc_hi = (S2 & 0x0F0F0F0Fu) | ((S0 >> 2) & 0x30303030u), sc_lo = S0 & 0x3F3F3F3Fu;
-        const uint32_t mn_hi = ((S2 >> 4) & 0x0F0F0F0Fu) | ((S1 >> 2) & 0x30303030u), mn_lo = S1 & 0x3F3F3F3Fu;
-        const uint32_t scw = (sc_hi & up) | (sc_lo & ~up);
-        const uint32_t mnw = (mn_hi & up) | (mn_lo & ~up);
-        const uint32_t sh = 16u * (g & 1u);
-        const float d = lev_f16_bits_to_f32(hdr[0] & 0xFFFFu);
-        const float dmin = lev_f16_bits_to_f32(hdr[0] >> 16);
-        const float sca = d * (float)__builtin_amdgcn_ubfe(scw, sh, 8u);
-        const float scb = d * (float)__builtin_amdgcn_ubfe(scw, sh + 8u, 8u);
-        const float mna = dmin * (float)__builtin_amdgcn_ubfe(mnw, sh, 8u);
-        const float mnb = dmin * (float)__builtin_amdgcn_ubfe(mnw, sh + 8u, 8u);
-        const lev_i32x4 la = __builtin_bit_cast(lev_i32x4, ca & 0x0F0F0F0Fu);
-        const lev_i32x4 lb = __builtin_bit_cast(lev_i32x4, cb & 0x0F0F0F0Fu);
-        const lev_i32x4 ha = __builtin_bit_cast(lev_i32x4, (ca >> 4) & 0x0F0F0F0Fu);
-        const lev_i32x4 hb = __builtin_bit_cast(lev_i32x4, (cb >> 4) & 0x0F0F0F0Fu);
+            for (int k = 0; k < 4; ++k) hdr[k] = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(16u * r + 4u * k), (int)D[t][0]);
+            const int src = (int)((4u * r + g) * 4u);
 #pragma unroll
-        for (int ch = 0; ch < NCH; ++ch) {
-            lev_i32x4 d0 = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[ch][0], la, lev_i32x4{0, 0, 0, 0}, 0, 0, 0);
-            lev_i32x4 d1 = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[ch][2], ha, lev_i32x4{0, 0, 0, 0}, 0, 0, 0);
-            d0 = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[ch][1], lb, d0, 0, 0, 0);
-            d1 = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[ch][3], hb, d1, 0, 0, 0);
-            float v[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                // y += d*sc_j*dx_j*idot - dmin*m_j*s_j for the lane's two sub-blocks
-                float t = fmaf(sca, dxa[ch][i] * (float)d0[i], -mna * sa[ch][i]);
-                t = fmaf(scb, dxb[ch][i] * (float)d1[i], t);
-                v[i] = fmaf(-mnb, sbm[ch][i], t);
+            for (int k = 0; k < 4; ++k) {
+                ca[k] = (uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)D[t][1 + k]);
+                cb[k] = (uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)D[t][5 + k]);
             }
-            // the four lane groups' shares of a row meet, lane group g keeping column 4*ch + g
-            *reinterpret_cast<float *>(smem + pw + 16 * ch) = lev_lanegroup_sums4(v);
+            __builtin_amdgcn_sched_barrier(0);
+            issue(next_block, t, D[t]);
+            __builtin_amdgcn_sched_barrier(0);
+            // unpack_scale_min (lev-cpu/src/lib.rs:64-74), four sub-blocks a word; this lane wants sub-blocks
+            // 2g and 2g + 1: bytes 2 * (g % 2) and + 1 of word g / 2 (both words are formed and one is
+            // kept by a bit select: a conditional here becomes a branch)
+            const uint32_t S0 = hdr[1], S1 = hdr[2], S2 = hdr[3];
+            const uint32_t up = g >= 2u ? ~0u : 0u;
+            const uint32_t sc_hi = (S2 & 0x0F0F0F0Fu) | ((S0 >> 2) & 0x30303030u), sc_lo = S0 & 0x3F3F3F3Fu;
+            const uint32_t mn_hi = ((S2 >> 4) & 0x0F0F0F0Fu) | ((S1 >> 2) & 0x30303030u), mn_lo = S1 & 0x3F3F3F3Fu;
+            const uint32_t scw = (sc_hi & up) | (sc_lo & ~up);
+            const uint32_t mnw = (mn_hi & up) | (mn_lo & ~up);
+            const uint32_t sh = 16u * (g & 1u);
+            const float d = lev_f16_bits_to_f32(hdr[0] & 0xFFFFu);
+            const float dmin = lev_f16_bits_to_f32(hdr[0] >> 16);
+            const float sca = d * (float)__builtin_amdgcn_ubfe(scw, sh, 8u);
+            const float scb = d * (float)__builtin_amdgcn_ubfe(scw, sh + 8u, 8u);
+            const float mna = dmin * (float)__builtin_amdgcn_ubfe(mnw, sh, 8u);
+            const float mnb = dmin * (float)__builtin_amdgcn_ubfe(mnw, sh + 8u, 8u);
+            const lev_i32x4 la = __builtin_bit_cast(lev_i32x4, ca & 0x0F0F0F0Fu);
+            const lev_i32x4 lb = __builtin_bit_cast(lev_i32x4, cb & 0x0F0F0F0Fu);
+            const lev_i32x4 ha = __builtin_bit_cast(lev_i32x4, (ca >> 4) & 0x0F0F0F0Fu);
+            const lev_i32x4 hb = __builtin_bit_cast(lev_i32x4, (cb >> 4) & 0x0F0F0F0Fu);
+            q8m_one_chunk<N0>(A[t][0], la, lb, ha, hb, xv0[t], sca, scb, mna, mnb, v0);
+            if constexpr (NCH == 2) q8m_one_chunk<N1>(A[t][1], la, lb, ha, hb, xv1, sca, scb, mna, mnb, v1);
         }
+        // the four lane groups' shares of a row meet, lane group g keeping column 4*ch + g
+        auto meet = [&](const float (&v)[4], int n, uint32_t at) {
+            const float s = n == 1 ? lev_row_sum_f32(v[0]) : lev_lanegroup_sums4(v);
+            if (n == 4 || g < (uint32_t)n) *reinterpret_cast<float *>(smem + at) = s;
+        };
+        meet(v0, N0, pw);
+        if constexpr (NCH == 2) meet(v1, N1, pw + 16u);
         lev_barrier_lds();
-        if (wave < slots) {
+        if (adds) {
             const float *pp = reinterpret_cast<const float *>(smem + pr);
+            // the slot's waves in order, four chains added at the end (sixteen reads in flight)
+            float s4[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int ch = 0; ch < NCH; ++ch) {
-                // the slot's waves in order, four chains added at the end (sixteen reads in flight)
-                float s4[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int k = 0; k < kMWaves; ++k) {
-                    const float pk = pp[k * 16 * NC + 4 * ch];
-                    s4[k & 3] += (uint32_t)k < wpr ? pk : 0.f;
-                }
-                const float s = (s4[0] + s4[1]) + (s4[2] + s4[3]);
-                if (stores && 4u * (uint32_t)ch + g < ncol)
-                    *reinterpret_cast<__attribute__((address_space(1))) float *>(yp + (uint64_t)(4 * ch) * rows * 4u) = s;
+            for (int k = 0; k < NW; ++k) {
+                const float pk = pp[k * 16 * NC];
+                s4[k & 3] += (uint32_t)k < wpr ? pk : 0.f;
             }
+            const float s = (s4[0] + s4[1]) + (s4[2] + s4[3]);
+            if (stores) *reinterpret_cast<__attribute__((address_space(1))) float *>(yp) = s;
         }
-        pw ^= kMWaves * 16u * 4u * NC;                          // the other half of `part` next round
-        pr ^= kMWaves * 16u * 4u * NC;
+        pw += flip;                                             // the other half of `part` next round
+        pr += flip;
+        flip = 0u - flip;
         orow += orow_step;
         yp += (uint64_t)orow_step * 4u;
         stores = writer && orow < rows ? 1u : 0u;
@@ -908,20 +928,54 @@ q4_k_q8_mfma_one(const uint8_t *__restrict__ w, const uint8_t *__restrict__ xq, 
         rb = next;
     }
 }
+// Whether the kernel above takes nc columns (as many as a launch still has).  us for it and for what took the shape
+// before, the kernel that stages every column (from four columns on) or the dot4 kernel: 12288 x 4096 by five 9.2 and 12.1,
+// by eight 10.2 and 12.4; 8192 x 1024 by eight 6.0 and 8.2; 2048 x 3072 by eight 5.4 and 6.6; 16384 x 6144 by one 14.4 and
+// 16.9, by three 14.8 and 24.0, by four 15.2 and 21.8.  Rows of more than twenty-four superblocks leave no wave without two
+// of them: 4096 x 8192 by one 8.1 and 7.4.  Fewer rows than one each for the CUs are latency with either kernel; the wide
+// ones of up to three columns stay where they were.
+bool q8m_one_takes(uint32_t in_dim, uint32_t rows, uint32_t nc) {
+    return in_dim <= 4096u ? nc <= 4u || (nc <= 8u && in_dim > 256u) : in_dim <= 6144u && nc <= 4u && (rows >= 256u || nc == 4u);
+}
 
-template <int NC>
+template <int NC, int TPW, int NW>
 hipError_t launch_q8m_one(lev_ctx *ctx, const uint8_t *w, const uint8_t *xq, const float *xs, float *y,
-                          uint32_t cols, uint32_t rows, uint32_t ncol) {
-    const uint32_t wpr = cols >> 8, slots = (uint32_t)kMWaves / wpr;
+                          uint32_t cols, uint32_t rows) {
+    const uint32_t wpr = ((cols >> 8) + TPW - 1u) / TPW, slots = (uint32_t)kMWaves / wpr;
     const uint32_t ngroups = (rows + 15u) / 16u;
     const uint32_t nrounds = (ngroups + slots - 1u) / slots;
     uint64_t slot_of_wave, pos_of_wave;
     lev_wave_tables(wpr, &slot_of_wave, &pos_of_wave);
     const uint32_t blocks = nrounds < (uint32_t)ctx->num_cus ? nrounds : (uint32_t)ctx->num_cus;
-    static_assert(q8m_one_part_bytes(NC) <= 48u * 1024u, "fits the default dynamic LDS limit");
-    hipLaunchKernelGGL((q4_k_q8_mfma_one<NC>), dim3(blocks), dim3(kMThreads), q8m_one_part_bytes(NC), ctx->stream, w,
-                       xq, xs, y, cols, rows, ncol, wpr, slots, slot_of_wave, pos_of_wave);
+    static_assert(q8m_one_part_bytes(NC, NW) <= 48u * 1024u, "fits the default dynamic LDS limit");
+    hipLaunchKernelGGL((q4_k_q8_mfma_one<NC, TPW, NW>), dim3(blocks), dim3(NW * LEV_WAVE), q8m_one_part_bytes(NC, NW), ctx->stream,
+                       w, xq, xs, y, cols, rows, wpr, slots, slot_of_wave, pos_of_wave);
     return hipGetLastError();
+}
+
+hipError_t launch_q8m_one(lev_ctx *ctx, const uint8_t *w, const uint8_t *xq, const float *xs, float *y, uint32_t cols,
+                          uint32_t rows, uint32_t nc) {
+#define LEV_ONE(NC, TPW, NW) \
+    case NC: return launch_q8m_one<NC, TPW, NW>(ctx, w, xq, xs, y, cols, rows)
+    if (cols <= 4096u) {
+        switch (nc) {
+            LEV_ONE(1, 1, 16);
+            LEV_ONE(2, 1, 16);
+            LEV_ONE(3, 1, 16);
+            LEV_ONE(4, 1, 16);
+            LEV_ONE(5, 1, 16);
+            LEV_ONE(6, 1, 16);
+            LEV_ONE(7, 1, 16);
+            default: return launch_q8m_one<8, 1, 16>(ctx, w, xq, xs, y, cols, rows);
+        }
+    }
+    switch (nc) {
+        LEV_ONE(1, 2, 12);
+        LEV_ONE(2, 2, 12);
+        LEV_ONE(3, 2, 12);
+        default: return launch_q8m_one<4, 2, 12>(ctx, w, xq, xs, y, cols, rows);
+    }
+#undef LEV_ONE
 }
 
 size_t q8m_lds_bytes(uint32_t cols, uint32_t ncl) {
@@ -1000,11 +1054,10 @@ extern "C" int lev_hip_norm_quant_q8(lev_ctx *ctx, float *d_x, size_t x_count, c
 // the dot4 kernel and, where its staging fits, the integer matrix-core kernel.
 uint32_t lev_q4_k_gemv_q8_candidates(const lev_ctx *ctx, uint32_t in_dim, uint32_t rows, uint32_t ncol,
                                      lev_schedule *out, uint32_t capacity) {
-    (void)rows;
     const bool has_mfma = q8m_cols(ctx, in_dim) != 0u;
-    // built-in: the matrix cores for every column count of rows up to 4096 wide (a wave per
-    // superblock column up to four columns), from kQ8MfmaMinCols columns for wider rows
-    const uint32_t first = has_mfma && (ncol >= kQ8MfmaMinCols || in_dim <= 4096u) ? 1u : 0u;
+    // built-in: the matrix cores for every column count of rows up to 4096 wide and, from 256 rows on, 6144
+    // (q8m_one_takes), from kQ8MfmaMinCols columns for wider rows
+    const uint32_t first = has_mfma && (ncol >= kQ8MfmaMinCols || q8m_one_takes(in_dim, rows, ncol)) ? 1u : 0u;
     uint32_t n = 0;
     if (n < capacity) out[n] = lev_schedule{LEV_OP_Q4_K_GEMV_Q8, first, 0u, 0u};
     ++n;
@@ -1041,14 +1094,11 @@ extern "C" int lev_hip_q4_k_gemv_q8(lev_ctx *ctx, const void *d_w, size_t w_byte
     // overrides it.
     const uint32_t mcols = q8m_cols(ctx, in_dim);
     const lev_schedule *sel = lev_selected(ctx, LEV_OP_Q4_K_GEMV_Q8, in_dim, rows, ncol);
-    const bool mfma = mcols != 0u && (sel ? sel->family == 1u : (ncol >= kQ8MfmaMinCols || in_dim <= 4096u));
-    // rows of at most sixteen superblocks: the matrix-core kernel with a wave per superblock column,
-    // for every column count (a schedule of family 0 still selects the dot4 kernel)
+    const bool mfma = mcols != 0u && (sel ? sel->family == 1u : (ncol >= kQ8MfmaMinCols || q8m_one_takes(in_dim, rows, ncol)));
     static const bool one_off = [] {
         const char *e = getenv("LEV_Q4K_Q8_ONE");   // LEV_Q4K_Q8_ONE=0: the kernels below, for comparison
         return e && e[0] == '0';
     }();
-    const bool mfma_one = !one_off && in_dim <= 4096u && mfma;
     uint32_t done = 0;
     while (done < ncol) {
         uint32_t nc = ncol - done;
@@ -1056,11 +1106,8 @@ extern "C" int lev_hip_q4_k_gemv_q8(lev_ctx *ctx, const void *d_w, size_t w_byte
         const float *xsc = d_xs + (uint64_t)done * (in_dim >> 5) * 2u;
         float *yc = d_y + (uint64_t)done * rows;
         hipError_t e;
-        if (mfma_one && nc <= 4u) {
-            // up to four columns (eight through it measured 11.9 us at 12288 x 4096, what the
-            // sixteen-column kernel below takes for eight as well)
-            if (nc > 4u) nc = 4u;
-            e = launch_q8m_one<4>(ctx, w, reinterpret_cast<const uint8_t *>(xqc), xsc, yc, in_dim, rows, nc);
+        if (mfma && !one_off && q8m_one_takes(in_dim, rows, nc)) {
+            e = launch_q8m_one(ctx, w, reinterpret_cast<const uint8_t *>(xqc), xsc, yc, in_dim, rows, nc);
         } else if (mfma) {
             if (nc > mcols) nc = mcols;
             const uint8_t *xb = reinterpret_cast<const uint8_t *>(xqc);

@@ -353,3 +353,18 @@ def test_q8_guards(ctx):
         with pytest.raises(LevError) as e:
             ctx.q4_k_gemv_q8(w, xq, xs, **kw)
         assert e.value.status == status, kw
+
+
+@pytest.mark.parametrize("ncol", range(1, 9))
+@pytest.mark.parametrize("rows,cols", [(16, 512), (33, 256), (4100, 1024), (18, 4096), (4099, 4096), (256, 4352), (301, 6144), (4113, 5120)])
+def test_q4_k_q8_a_kernel_per_column_count(ctx, rows, cols, ncol):
+    """Every column count has an instantiation of its own up to 4096 values (eight columns, beyond one superblock) and
+    6144 (four columns, from 256 rows on): row groups that end inside one, one round and several of the resident
+    grid, an odd number of superblocks of two a wave; against the f64 product over the same codes, and each
+    column the bits that it has by itself."""
+    w, x, gain = H.config3(rows, cols, ncol, seed=3 * rows + ncol)
+    got, xq, xs = q8_gemv(ctx, w, x, rows, cols, gain)
+    check_gemv(got, w, rows, cols, xq, xs)
+    if cols <= 4096 and ncol > 1 and (cols > 256 or ncol <= 4):
+        one, _, _ = q8_gemv(ctx, w, x[:1], rows, cols, gain)
+        assert (one[0].view("u4") == got[0].view("u4")).all()
