@@ -1111,7 +1111,7 @@ q6_k_mfma_gemv_q8(const uint8_t *__restrict__ w, const uint32_t *__restrict__ xq
 // sums in the same order without scratch, a launch a slice.
 // Staged in LDS as a whole (q6_k_mfma_gemv_q8) such rows leave room for four columns at 12288, and the
 // weights are read again for every four: 4096 x 12288 by one, five and
-// sixteen columns 15.0, 27.5 and 53.8 us with it, 13.5, 15.6 and 28.5 here.
+// sixteen columns 15.0, 27.5 and 53.8 us with it, 13.9, 15.8 and 27.7 here.
 // LDS: part [2][MAXW waves][16 rows][NC] f32 | per wave: the turn-round area.
 // ---------------------------------------------------------------------------
 __host__ __device__ constexpr uint32_t q6m_q8_one_part_bytes(uint32_t nc, uint32_t waves) { return 2u * waves * 16u * 4u * nc; }
@@ -1147,26 +1147,24 @@ q6_k_mfma_gemv_q8_one(const uint8_t *__restrict__ w, const uint32_t *__restrict_
 
     // the wave's activations first: lane (r, g) feeds A row r = 4*gs + c, i.e. column 4*ch + r%4,
     // the 16 codes of weight group 16*sb + 8*hf + 2*jb (+ 4*nb + lh), when gs == g, zeros
-    // otherwise (columns of the layout beyond ncol repeat the last one and are never stored)
+    // otherwise (columns of the layout beyond ncol are zeros and never stored).  A lane that gets zeros asks for
+    // nothing: with an address for every lane the activations took the L1 more lookups than the weights (32000 x 4096 by
+    // eight 26.8 us, 25.1 without; 1024 x 2048 by eight 8.1 and 6.6).
+    const lev_buffer codes(xq, cols * ncol), scales(xs, nblk * ncol * 8u);
+    const bool feeds = active && (r >> 2) == q;
     q6m_i4 A[NCH][2][2];
-    float dx[NCH][2][4];   // a quarter of the activation scale (the codes in the operand are 4*(q - 32)) of block nb, column 4*ch + i
-    const uint32_t blk0 = 8u * sb + 4u * hf + jb;   // 32-activation block of nb = 0; nb = 1: + 2
 #pragma unroll
     for (int ch = 0; ch < NCH; ++ch) {
         const uint32_t ca = 4u * (uint32_t)ch + (r & 3u);
-        const uint8_t *xa = reinterpret_cast<const uint8_t *>(xq) + (uint64_t)(ca < ncol ? ca : ncol - 1u) * cols +
-                            256u * sb + (8u * hf + 2u * jb) * 16u;
+        const uint32_t at = feeds && ca < ncol ? ca * cols + 256u * sb + (8u * hf + 2u * jb) * 16u : lev_buffer::kNothing;
 #pragma unroll
-        for (int nb = 0; nb < 2; ++nb) {
+        for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
-            for (int lh = 0; lh < 2; ++lh) A[ch][nb][lh] = *reinterpret_cast<const q6m_i4 *>(xa + (4 * nb + lh) * 16);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t ci = 4u * (uint32_t)ch + (uint32_t)i;
-                dx[ch][nb][i] = xs[((uint64_t)(ci < ncol ? ci : ncol - 1u) * nblk + blk0 + 2u * (uint32_t)nb) * 2u];
-            }
-        }
+            for (int lh = 0; lh < 2; ++lh) A[ch][nb][lh] = __builtin_bit_cast(q6m_i4, codes.load16(at, (4 * nb + lh) * 16));
     }
+    // column r's activation scales of the lane group's 32-activation blocks (nb = 0; nb = 1: two further on)
+    const uint32_t dat = active && r < ncol ? (r * nblk + 8u * sb + 4u * hf + jb) * 8u : lev_buffer::kNothing;
+    const uint32_t din[2] = {scales.load4(dat, 0), scales.load4(dat, 16)};
     // ... the first row group's weights right behind them
     const uint64_t row_bytes = (uint64_t)SB * 210u;
     const uint32_t ngroups = (rows + 15u) >> 4;
@@ -1195,16 +1193,13 @@ q6_k_mfma_gemv_q8_one(const uint8_t *__restrict__ w, const uint32_t *__restrict_
     lev_pin(pr);
     lev_pin(stores);
     lev_pin(yp);
-    const bool feeds = active && (r >> 2) == q;
+    float dx[2][NC];   // a quarter of the activation scale (the codes in the operand are 4*(q - 32)) of block nb, every column's
 #pragma unroll
-    for (int ch = 0; ch < NCH; ++ch)
+    for (int nb = 0; nb < 2; ++nb) {
+        lev_row_spread(din[nb], dx[nb]);
 #pragma unroll
-        for (int nb = 0; nb < 2; ++nb) {
-#pragma unroll
-            for (int lh = 0; lh < 2; ++lh) A[ch][nb][lh] = feeds ? A[ch][nb][lh] : q6m_i4{0, 0, 0, 0};
-#pragma unroll
-            for (int i = 0; i < 4; ++i) dx[ch][nb][i] *= active ? 0.25f : 0.f;
-        }
+        for (int i = 0; i < NC; ++i) dx[nb][i] *= 0.25f;
+    }
     const q6m_lane L6(smem + kPart, wave, lane, q6m_odd(sb, r, alt));
     __builtin_amdgcn_sched_barrier(0);
 
@@ -1226,7 +1221,7 @@ q6_k_mfma_gemv_q8_one(const uint8_t *__restrict__ w, const uint32_t *__restrict_
                 for (int i = 0; i < 4; ++i) {
                     int E = __mul24(D0[i], sc[nb][0]);
                     E += __mul24(D1[i], sc[nb][1]);
-                    v[i] = fmaf((float)E, dx[ch][nb][i], v[i]);
+                    v[i] = fmaf((float)E, dx[nb][4 * ch + i], v[i]);
                 }
             }
             // the four lane groups' shares of a row meet, lane group g keeping column 4*ch + g
