@@ -780,16 +780,17 @@ q4_k_q8_mfma_one(const uint8_t *__restrict__ w, const uint8_t *__restrict__ xq, 
     const uint32_t ngroups = (rows + 15u) >> 4;
     const uint32_t nrounds = (ngroups + slots - 1u) / slots;     // rounds of `slots` row groups
     const uint32_t lrow = lane >> 2, lc = lane & 3u;             // fetch order: lane = 4 * row + chunk
+    // (a row past the matrix's end, and every row of a round past the last one, asks for nothing: with the last round
+    // requested again 12288 x 4096 by eight takes 10.0 us, 9.6 without, 16384 x 6144 by four 15.3 and 14.6)
+    const uint32_t lane_at = lrow * (uint32_t)row_bytes;
     auto issue = [&](uint32_t round_block, int t, uint32_t (&D)[9]) {
-        uint32_t rg = round_block * slots + (active ? slot : 0u);
-        rg = rg < ngroups ? rg : ngroups - 1u;
-        uint32_t row = rg * 16u + lrow;
-        row = row < rows ? row : rows - 1u;
+        const uint32_t rg = round_block * slots + (active ? slot : 0u);
         const uint32_t sb = TPW == 1 || sb0 + t < SB ? sb0 + t : SB - 1u;
-        const uint8_t *p = w + (uint64_t)row * row_bytes + (uint64_t)sb * 144u;
-        D[0] = *reinterpret_cast<const uint32_t *>(p + 4u * lc);
-        const lev_u32x4 a = *reinterpret_cast<const lev_u32x4 *>(p + 16u + 32u * lc);
-        const lev_u32x4 b = *reinterpret_cast<const lev_u32x4 *>(p + 32u + 32u * lc);
+        const uint32_t left = rg < ngroups ? (rows - rg * 16u < 16u ? rows - rg * 16u : 16u) * (uint32_t)row_bytes - sb * 144u : 0u;
+        const lev_buffer group(w + (uint64_t)rg * 16u * row_bytes + sb * 144u, left);
+        D[0] = group.load4(lane_at + 4u * lc, 0);
+        const lev_u32x4 a = group.load16(lane_at + 32u * lc, 16);
+        const lev_u32x4 b = group.load16(lane_at + 32u * lc, 32);
         D[1] = a.x; D[2] = a.y; D[3] = a.z; D[4] = a.w;
         D[5] = b.x; D[6] = b.y; D[7] = b.z; D[8] = b.w;
     };
@@ -851,7 +852,7 @@ q4_k_q8_mfma_one(const uint8_t *__restrict__ w, const uint8_t *__restrict__ xq, 
     __builtin_amdgcn_sched_barrier(0);
 
     // A round: the fetched dwords go to the lanes that multiply them, and the registers they came
-    // in take the NEXT round's request at once (unconditional, clamped: a branch around the loads
+    // in take the NEXT round's request at once (unconditional: a branch around the loads
     // would make the compiler wait for them before the current group is multiplied).
     auto round = [&](uint32_t next_block) {
         float v0[4] = {0.f, 0.f, 0.f, 0.f}, v1[4] = {0.f, 0.f, 0.f, 0.f};
