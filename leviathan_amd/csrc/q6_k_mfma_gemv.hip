@@ -53,6 +53,7 @@
 #include "top2.hpp"
 
 #include <cstdlib>
+#include <type_traits>
 
 namespace {
 
@@ -1111,7 +1112,7 @@ q6_k_mfma_gemv_q8(const uint8_t *__restrict__ w, const uint32_t *__restrict__ xq
 // sums in the same order without scratch, a launch a slice.
 // Staged in LDS as a whole (q6_k_mfma_gemv_q8) such rows leave room for four columns at 12288, and the
 // weights are read again for every four: 4096 x 12288 by one, five and
-// sixteen columns 15.0, 27.5 and 53.8 us with it, 13.9, 15.8 and 27.7 here.
+// sixteen columns 15.0, 27.5 and 53.8 us with it, 13.9, 15.8 and 27.7 here (the first two run on q6_k_mfma_gemv_q8_wide).
 // LDS: part [2][MAXW waves][16 rows][NC] f32 | per wave: the turn-round area.
 // ---------------------------------------------------------------------------
 __host__ __device__ constexpr uint32_t q6m_q8_one_part_bytes(uint32_t nc, uint32_t waves) { return 2u * waves * 16u * 4u * nc; }
@@ -1296,6 +1297,181 @@ q6_k_mfma_gemv_q8_one(const uint8_t *__restrict__ w, const uint32_t *__restrict_
         for (uint32_t sl = 0; sl < gridDim.y; ++sl)
             sum += __hip_atomic_load(p + (uint64_t)sl * ncol * rows, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         y[(uint64_t)c * rows + row] = sum;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Int8 activations, rows of 17 to 64 superblocks, a whole row group a workgroup: a wave has TPW superblock columns, wpr
+// apart (an even number, so that all of them are even or all odd), and requests the weights of all of them in front of
+// the first product.  What the kernel above pays for cutting such a row into slices, a value a row, column and slice
+// through memory and the wait for the last slice, is gone, and a CU has 10 KB a wave on their way where it had 3.4.  The
+// activations of the wave's superblocks go through LDS of its own (codes as [task][column][256], quarter scales as
+// [task][block][column]): as operands in registers they would leave no room for the weights.
+// NC: columns held (4, 6 or 8; >= ncol), for which the LDS has to have room.
+// SINGLE: a workgroup a row group; otherwise the next round's weights are requested as a task's registers are free.
+// LDS: part [2][16 waves][16 rows][NC] f32 | per wave: the turn-round area, a zero strip, codes, scales.
+// ---------------------------------------------------------------------------
+constexpr uint32_t kWideZero = 16u;
+__host__ __device__ constexpr uint32_t q6m_wide_area(uint32_t nc, uint32_t tpw) { return kQAreaBytes + kWideZero + tpw * nc * (256u + 32u); }
+__host__ __device__ constexpr size_t q6m_wide_lds(uint32_t nc, uint32_t tpw) {
+    return (q6m_q8_one_part_bytes(nc, kQWaves) + 15u) / 16u * 16u + (size_t)kQWaves * ((q6m_wide_area(nc, tpw) + 15u) / 16u * 16u);
+}
+
+template <int NC, int TPW, bool SINGLE>
+__global__ void __launch_bounds__(kQThreads)
+q6_k_mfma_gemv_q8_wide(const uint8_t *__restrict__ w, const uint32_t *__restrict__ xq, const float *__restrict__ xs,
+                       float *__restrict__ y, uint32_t cols, uint32_t rows, uint32_t ncol, uint32_t wpr) {
+    constexpr int NCH = (NC + 3) / 4, N1 = NC > 4 ? NC - 4 : 1;
+    constexpr uint32_t kPart = q6m_q8_one_part_bytes(NC, kQWaves), kArea = (q6m_wide_area(NC, TPW) + 15u) / 16u * 16u;
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+    const uint32_t SB = cols >> 8, nblk = cols >> 5;
+    const uint32_t r = lane & 15u, q = lane >> 4, hf = q >> 1, jb = q & 1u;
+
+    // the activations first: lane l has 16 codes of column 4*ch + l / 16, and of each block of 32 a few lanes the scales
+    const lev_buffer codes(xq, cols * ncol), scales(xs, nblk * ncol * 8u);
+    lev_u32x4 xc[TPW][NCH];
+    uint32_t xd[TPW][NCH];
+#pragma unroll
+    for (int t = 0; t < TPW; ++t) {
+        const uint32_t sb = wave + (uint32_t)t * wpr;
+#pragma unroll
+        for (int ch = 0; ch < NCH; ++ch) {
+            const uint32_t n = ch ? N1 : 4u, cx = 4u * ch + q, cd = 4u * ch + lane % n, blk = lane / n;
+            xc[t][ch] = codes.load16(sb < SB && cx < ncol ? cx * cols + 256u * sb + 16u * r : lev_buffer::kNothing, 0);
+            xd[t][ch] = scales.load4(sb < SB && blk < 8u && cd < ncol ? (cd * nblk + 8u * sb + blk) * 8u : lev_buffer::kNothing, 0);
+        }
+    }
+    const uint64_t row_bytes = (uint64_t)SB * 210u;
+    const uint32_t nrounds = (rows + 15u) >> 4;
+    const uint32_t alt = q6m_alt(SB, rows), odd0 = q6m_odd(wave, q, alt);
+    const int32_t poff = q6m_piece_offset(lane, odd0);
+    q6m_regs W[TPW];
+    uint32_t rb = blockIdx.x;
+    auto issue = [&](uint32_t rg, int t) {
+        const uint32_t sb = wave + (uint32_t)t * wpr;             // past the row's end one of the wave's parity, times zero
+        q6m_issue(w, row_bytes, rg * 16u, rows, alt, sb < SB ? sb : wave < SB ? wave : wave & 1u, lane, poff, W[t]);
+    };
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int t = 0; t < TPW; ++t) issue(rb, t);
+    __builtin_amdgcn_sched_barrier(0);
+
+    uint8_t *const own = smem + kPart + wave * kArea, *const zero = own + kQAreaBytes, *const codes_at = zero + kWideZero;
+    uint8_t *const scales_at = codes_at + TPW * NC * 256;
+    uint32_t pw = ((wave * 16u + r) * NC + q) * 4u;              // lane (r, q): row r, column q (+ 4 a chunk)
+    // wave ch adds up chunk ch
+    const uint32_t ocol = 4u * wave + q;
+    uint32_t pr = (r * NC + (ocol < (uint32_t)NC ? ocol : 0u)) * 4u;
+    uint32_t orow = rb * 16u + r;
+    const bool writer = wave < (uint32_t)NCH && ocol < ncol;
+    uint32_t stores = writer && orow < rows ? 1u : 0u;
+    uint64_t yp = reinterpret_cast<uint64_t>(y + (uint64_t)ocol * rows + orow);
+    uint32_t flip = kPart / 2u;
+    lev_pin(pw);
+    lev_pin(pr);
+    lev_pin(stores);
+    lev_pin(yp);
+    const q6m_lane L6(smem + kPart, wave, lane, q6m_odd(wave, r, alt), kArea);
+    if (lane < kWideZero / 4u) reinterpret_cast<uint32_t *>(zero)[lane] = 0u;
+#pragma unroll
+    for (int t = 0; t < TPW; ++t)
+#pragma unroll
+        for (int ch = 0; ch < NCH; ++ch) {
+            const uint32_t n = ch ? N1 : 4u;
+            if (q < n) *reinterpret_cast<lev_u32x4 *>(codes_at + (t * NC + 4 * ch) * 256 + lane * 16u) = xc[t][ch];
+            if (lane < 8u * n) *reinterpret_cast<float *>(scales_at + (t * NC + 4 * ch) * 32 + lane * 4u) = 0.25f * __uint_as_float(xd[t][ch]);
+        }
+    // lane (r, q) feeds A row r = 4*gs + c, column 4*ch + r % 4, the 16 codes of weight group 8*hf + 2*jb (+ 4*nb + lh), when gs == q
+    const uint8_t *ap[NCH];
+    uint32_t a_task[NCH], a_nb[NCH], a_lh[NCH];
+#pragma unroll
+    for (int ch = 0; ch < NCH; ++ch) {
+        const bool feeds = (r >> 2) == q && (r & 3u) < (ch ? (uint32_t)N1 : 4u);
+        ap[ch] = feeds ? codes_at + (4u * ch + (r & 3u)) * 256u + (8u * hf + 2u * jb) * 16u : zero;
+        a_task[ch] = feeds ? NC * 256u : 0u, a_nb[ch] = feeds ? 64u : 0u, a_lh[ch] = feeds ? 16u : 0u;
+    }
+    const uint32_t blk0 = 4u * hf + jb;                          // the lane group's first block of 32; nb = 1: two further on
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+
+    auto round = [&](uint32_t next) {
+        float v[NCH][4];
+#pragma unroll
+        for (int t = 0; t < TPW; ++t) {
+            q6m_i4 B[2][2];
+            int sc[2][2];
+            uint32_t dbits;
+            L6.operands(W[t], B, sc, dbits);
+            __builtin_amdgcn_sched_barrier(0);
+            if (!SINGLE) issue(next, t);
+            __builtin_amdgcn_sched_barrier(0);
+            // (past the row's end the activations are zeros, the scale may be anything)
+            const float d = wave + (uint32_t)t * wpr < SB ? lev_f16_bits_to_f32(dbits) : 0.f;
+            auto chunk = [&](auto count, int ch) {
+                constexpr int N = decltype(count)::value;
+                float u[N];
+#pragma unroll
+                for (int nb = 0; nb < 2; ++nb) {
+                    const uint8_t *const an = ap[ch] + t * a_task[ch] + nb * a_nb[ch];
+                    const q6m_i4 A0 = *reinterpret_cast<const q6m_i4 *>(an), A1 = *reinterpret_cast<const q6m_i4 *>(an + a_lh[ch]);
+                    struct alignas(N == 4 ? 16 : N == 2 ? 8 : 4) { float s[N]; } dx;
+                    dx = *reinterpret_cast<const decltype(dx) *>(scales_at + (t * NC + 4 * ch) * 32 + (blk0 + 2u * nb) * N * 4u);
+                    const q6m_i4 D0 = __builtin_amdgcn_mfma_i32_16x16x64_i8(A0, B[nb][0], q6m_i4{0, 0, 0, 0}, 0, 0, 0);
+                    const q6m_i4 D1 = __builtin_amdgcn_mfma_i32_16x16x64_i8(A1, B[nb][1], q6m_i4{0, 0, 0, 0}, 0, 0, 0);
+                    // |D| <= 16*128*127 < 2^18, |sc| <= 2^7: the sum of the two halves fits 32 bits
+#pragma unroll
+                    for (int i = 0; i < N; ++i) {
+                        int E = __mul24(D0[i], sc[nb][0]);
+                        E += __mul24(D1[i], sc[nb][1]);
+                        u[i] = nb ? fmaf((float)E, dx.s[i], u[i]) : (float)E * dx.s[i];
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    if (i < N) v[ch][i] = t ? fmaf(d, u[i < N ? i : 0], v[ch][i]) : d * u[i < N ? i : 0];
+                    else v[ch][i] = 0.f;
+                }
+            };
+            chunk(std::integral_constant<int, 4>{}, 0);
+            if constexpr (NCH == 2) chunk(std::integral_constant<int, N1>{}, 1);
+        }
+        // the four lane groups' shares of a row meet, lane group g keeping column 4*ch + g
+#pragma unroll
+        for (int ch = 0; ch < NCH; ++ch) {
+            const float s = ch && N1 == 1 ? lev_row_sum_f32(v[ch][0]) : lev_lanegroup_sums4(v[ch]);
+            if (!ch || q < (uint32_t)N1) *reinterpret_cast<float *>(smem + pw + 16 * ch) = s;
+        }
+        lev_barrier_lds();
+        if (wave < (uint32_t)NCH) {
+            const float *pp = reinterpret_cast<const float *>(smem + pr);
+            // the waves in order, four chains added at the end (sixteen reads in flight)
+            float s4[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int k = 0; k < kQWaves; ++k) {
+                const float pk = pp[k * 16 * NC];
+                s4[k & 3] += (uint32_t)k < wpr ? pk : 0.f;
+            }
+            if (stores) *reinterpret_cast<__attribute__((address_space(1))) float *>(yp) = (s4[0] + s4[1]) + (s4[2] + s4[3]);
+        }
+        pw += flip;                                              // the other half of `part` next round
+        pr += flip;
+        flip = 0u - flip;
+        orow += gridDim.x * 16u;
+        yp += (uint64_t)gridDim.x * 64u;
+        stores = writer && orow < rows ? 1u : 0u;
+    };
+    if (SINGLE) {
+        round(0u);
+        return;
+    }
+    while (true) {
+        const uint32_t next = rb + gridDim.x;
+        round(next < nrounds ? next : rb);
+        if (next >= nrounds) break;
+        rb = next;
     }
 }
 
@@ -1498,8 +1674,8 @@ q6m_slices q6m_q8_one_grid(const lev_ctx *ctx, uint32_t cols, uint32_t rows, uin
 // sixteen columns (us, 624 shapes, by the columns a kernel is built for: 4, 8 and 16).  In slices a round takes some
 // time whatever it multiplies, and every slice but one is a value a row and column more that goes to memory and
 // back; staged, the weights are read again for every `held` columns.  4096 x 32000 by sixteen columns 46.3 us in slices,
-// 32.6 staged; 4352 x 16000 by eight 28.4 and 21.1; 5120 x 16000 by eight 25.8 and 22.0; 12288 x 4096 by sixteen 28.5 and
-// 54.6.  Left to the staging kernel where the estimates differ by 4 % and more: of the shapes measured the worst that
+// 32.6 staged; 12288 x 4096 by sixteen 28.5 and 54.6.  (Asked after q6m_q8_wide_launch, which takes rows of up to 32
+// superblocks by up to eight columns and some longer ones from both.)  Left to the staging kernel where the estimates differ by 4 % and more: of the shapes measured the worst that
 // moves loses 2.6 %, the worst that stays would gain 8 %.
 bool q6m_q8_staged_is_faster(const lev_ctx *ctx, const q6m_slices &g, uint32_t cols, uint32_t rows, uint32_t ncol,
                              uint32_t held) {
@@ -1534,9 +1710,52 @@ hipError_t q6m_q8_one_launch_grid(lev_ctx *ctx, const uint8_t *w, const uint32_t
     return hipGetLastError();
 }
 
+template <int NC, int TPW, bool SINGLE>
+hipError_t q6m_q8_wide_launch(lev_ctx *ctx, const uint8_t *w, const uint32_t *xq, const float *xs, float *y, uint32_t cols,
+                              uint32_t rows, uint32_t ncol, uint32_t blocks) {
+    const uint32_t wpr = (((cols >> 8) + TPW - 1u) / TPW + 1u) & ~1u;
+    constexpr size_t lds = q6m_wide_lds(NC, TPW);
+    static_assert(lds <= 160u * 1024u, "fits the LDS");
+    if (hipError_t e = lev_allow_lds(ctx, reinterpret_cast<const void *>(&q6_k_mfma_gemv_q8_wide<NC, TPW, SINGLE>), lds); e != hipSuccess) return e;
+    hipLaunchKernelGGL((q6_k_mfma_gemv_q8_wide<NC, TPW, SINGLE>), dim3(blocks), dim3(wpr * LEV_WAVE), lds, ctx->stream, w, xq, xs, y,
+                       cols, rows, ncol, wpr);
+    return hipGetLastError();
+}
+// Whole row groups a workgroup where that is faster than slices (hipErrorNotSupported: it is not, or does not fit).  us of
+// both, cold: rows of up to 32 superblocks at any number of rows (4096 x 4352 by one 6.3 and 8.2, 16000 x 6144 by eight
+// 20.8 and 25.1, 32000 x 8192 by four 39.8 and 45.7; of 90 shapes one loses, 6144 x 8192 by eight, 15.5 and 15.2); longer
+// ones where a workgroup a row group fills more than half of the CUs in one round (4096 x 12288 by one 11.5 and 14.0, by five
+// 12.5 and 15.8, 3072 x 16384 by four 13.4 and 14.2, but 2048 x 16384 12.4 and 11.7, 1024 x 12288 8.6 and 7.7).  A second
+// round of those has no registers for its weights beside the first one's (5120 x 12288 24.5 and 15.7).
+hipError_t q6m_q8_wide_launch(lev_ctx *ctx, const uint8_t *w, const uint32_t *xq, const float *xs, float *y, uint32_t cols,
+                              uint32_t rows, uint32_t ncol) {
+    const uint32_t groups = (rows + 15u) / 16u, cus = (uint32_t)ctx->num_cus, SB = cols >> 8;
+    if (SB <= 16u || ncol > 8u) return hipErrorNotSupported;
+#define LEV_WIDE(NC, TPW, SINGLE) return q6m_q8_wide_launch<NC, TPW, SINGLE>(ctx, w, xq, xs, y, cols, rows, ncol, SINGLE ? groups : cus)
+    if (SB <= 32u) {
+        if (groups <= cus) {
+            if (ncol <= 4u) LEV_WIDE(4, 2, true);
+            if (ncol <= 6u) LEV_WIDE(6, 2, true);
+            LEV_WIDE(8, 2, true);
+        }
+        if (ncol <= 4u) LEV_WIDE(4, 2, false);
+        if (ncol <= 6u) LEV_WIDE(6, 2, false);
+        LEV_WIDE(8, 2, false);
+    }
+    if (groups <= cus && 2u * groups > cus) {
+        if (SB <= 48u && ncol <= 4u) LEV_WIDE(4, 3, true);
+        if (SB <= 48u && ncol <= 6u) LEV_WIDE(6, 3, true);
+        if (SB <= 64u && ncol <= 4u) LEV_WIDE(4, 4, true);
+    }
+#undef LEV_WIDE
+    return hipErrorNotSupported;
+}
+
 template <int NC>
 hipError_t q6m_q8_one_launch(lev_ctx *ctx, const uint8_t *w, const uint32_t *xq, const float *xs, float *y,
                              uint32_t cols, uint32_t rows, uint32_t ncol) {
+    if constexpr (NC <= 8)
+        if (hipError_t e = q6m_q8_wide_launch(ctx, w, xq, xs, y, cols, rows, ncol); e != hipErrorNotSupported) return e;
     const q6m_slices g = q6m_q8_one_grid(ctx, cols, rows, (uint32_t)q6m_q8_one_waves(NC));
     if (g.slices == 1u) return q6m_q8_one_launch_grid<NC, kWholeRow>(ctx, w, xq, xs, y, cols, rows, ncol, g, 0u, nullptr);
     const uint32_t held = lev_q6_k_mfma_q8_cols(ctx, cols);

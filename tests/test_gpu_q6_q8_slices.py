@@ -77,3 +77,12 @@ def test_q6_q8_sliced_rows_record_the_eager_bits(blocks, rows, ncol):
     program.destroy()
     fresh.close()
     eager.close()
+
+
+@pytest.mark.parametrize("ncol", [1, 3, 4, 5, 6, 7, 8])
+@pytest.mark.parametrize("blocks,rows", [(17, 15), (18, 4096), (19, 4097), (31, 33), (32, 8200), (33, 2049), (41, 4095), (48, 2064),
+                                         (48, 2048), (49, 2056), (63, 4096), (64, 3000), (33, 4097)])
+def test_q6_q8_whole_row_groups(blocks, rows, ncol):
+    """Rows of which a wave takes two, three or four superblocks: an odd number of them, one short and one more than the
+    waves hold, row groups that end inside one, one round and several, and either side of the lines to the slices."""
+    test_q6_q8_sliced_rows(blocks, rows, ncol)
