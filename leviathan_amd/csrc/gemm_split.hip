@@ -14,9 +14,12 @@
 // CUs have work (lev_gemm_split_choose).  A wave that takes all of K adds the same products in the same
 // order as the 256-token kernels: bit for bit their results.
 //
-// What bounds it: a step of a wave is some 105 vector instructions of decode and 4 T MFMAs behind LDS reads and a
-// barrier, about twice what the vector unit alone takes; 6 us of a launch are its first weights and its stores.
-// 77 tokens, 4096 rows, 12288 columns of Q6_K: 27 us (218 in 256-token tiles on 32 CUs); 123 tokens, 1617 rows, 4096
+// What bounds it: a step of a wave is some 80 (Q4_K) or 105 (Q6_K) vector instructions of decode and 4 T MFMAs, two waves a
+// SIMD; and around the steps 2 to 5 us until the first weights are there, 2.5 for adding up the slices and storing, 5 for
+// the kernel that adds the workgroups' (in-kernel time stamps).  With the products of a step right behind its barrier all
+// waves waited for their first LDS reads together: 24 cases drawn over 1000 to 20000 rows and 19 to 740 tokens take 0.92 of
+// that, 2048 columns x 3000 rows of Q4_K at 700 tokens 21.2 us and 18.2.
+// 77 tokens, 4096 rows, 12288 columns of Q6_K: 25 us (218 in 256-token tiles on 32 CUs); 123 tokens, 1617 rows, 4096
 // columns of Q4_K: 13.7 us (49; 17 in tiles of 128 tokens alone).
 #include "prefill_decode.hpp"
 
@@ -24,158 +27,13 @@
 
 namespace {
 
-typedef lev_u32x4 u32x4_a4 __attribute__((aligned(4)));   // a vector on a dword boundary
-
 constexpr uint32_t kTile = 4096u;        // X step of 32 tokens: 32 rows of 128 bytes
-// X steps in LDS: the one in use and three on their way, or one where 160 KB hold no more
+// X steps in LDS: the one in use and three on their way, or one where 160 KB (for KW = 1, of which two workgroups share a
+// CU, 80 KB) hold no more or more is no faster (32000 x 4096 of Q6_K at 90 tokens 51 us with one on its way, 47 with three)
 template <typename W>
 constexpr uint32_t x_bufs(int t, int rw, int kw) {
-    return t >= 3 || kw * (4u * t * kTile + rw * W::kArea) > 160u * 1024u ? 2u : 4u;
+    return t >= (kw == 1 ? 4 : 3) || kw * (4u * t * kTile + rw * W::kArea) > 160u * 1024u ? 2u : 4u;
 }
-
-// The weights of a wave's 32 rows, a superblock column at a time: request() the column's bytes, touch() (the
-// wait for them), take() them as the current column, frag() its fragments; unit(): the 16-byte unit of the
-// step's X row that fragment q meets.  Rows past the end repeat the last row.
-struct weights_q4k {
-    static constexpr int kLoads = 5;
-    static constexpr uint32_t kArea = 0u;    // LDS bytes a wave
-    const uint8_t *row;
-    uint32_t lh;
-    lev_u32x4 nhdr, nqs[4], qs[4];
-    float d1[8], mm[8];
-    __device__ __forceinline__ void init(const uint8_t *w, uint32_t row0, uint32_t rows, uint32_t nsb, uint8_t *) {
-        const uint32_t lane = threadIdx.x & 63u, r = row0 + (lane & 31u);
-        lh = lane >> 5;
-        row = w + (uint64_t)(r < rows ? r : rows - 1u) * nsb * 144u;
-    }
-    __device__ __forceinline__ void request(uint32_t sb) {
-        const uint8_t *blk = row + (uint64_t)sb * 144u;
-        nhdr = *reinterpret_cast<const lev_u32x4 *>(blk);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) nqs[c] = *reinterpret_cast<const lev_u32x4 *>(blk + 16u + 32u * c + 16u * lh);
-    }
-    __device__ __forceinline__ void touch() {
-        asm volatile("" : "+v"(nhdr.x), "+v"(nhdr.y), "+v"(nhdr.z), "+v"(nhdr.w));
-#pragma unroll
-        for (int c = 0; c < 4; ++c) asm volatile("" : "+v"(nqs[c].x), "+v"(nqs[c].y), "+v"(nqs[c].z), "+v"(nqs[c].w));
-    }
-    __device__ __forceinline__ void take() {
-#pragma unroll
-        for (int c = 0; c < 4; ++c) qs[c] = nqs[c];
-        q4k_all_factors(nhdr, d1, mm);
-    }
-    __device__ __forceinline__ void half(int) {}
-    __device__ __forceinline__ f16x8 frag(int c, int q) const {
-        const bool hi = q >= 2;
-        return q4k_frag(q & 1 ? qs[c].z : qs[c].x, q & 1 ? qs[c].w : qs[c].y, hi, d1[2 * c + hi], mm[2 * c + hi]);
-    }
-    __device__ __forceinline__ uint32_t unit(int q) const { return 2u * lh + (q < 2 ? q : 2u + q); }
-};
-
-// Q6_K blocks are 210 bytes on 2-byte boundaries.  A lane that fetches its own row's 37 dwords costs the
-// address unit ten misaligned loads a column, 64 rows apart each: 84 us for 77 tokens x 4096 x 12288 on half of
-// the chip, 45 without the loads.  So the wave fetches in the order of memory, from the dword that a block
-// starts in: 14 pieces of 16 bytes a row (the last one ends with the block: bytes 196 .. 211), seven loads of
-// 1 KB, parks them in an area of its own and reads every dword it needs back, shifted by the row's two bytes.
-// (Of the dwords in which the matrix begins and ends two bytes may not be its own: read with the others, never used.)
-struct weights_q6k {
-    static constexpr int kLoads = 7;
-    static constexpr uint32_t kRow = 240u;   // 224 bytes of pieces + 16: the 32 rows start in different banks
-    static constexpr uint32_t kArea = 32u * kRow;
-    const uint8_t *base;
-    uint8_t *area;
-    uint32_t lh, lr, row_off[kLoads], nshift, shift, stride;
-    lev_u32x4 n[kLoads];
-    uint32_t ql[8], qh[8], sc[4];
-    float d;
-    static __device__ __forceinline__ uint32_t piece(int j) {   // (recomputed: cheaper than registers)
-        return (threadIdx.x & 63u) + 64u * j;
-    }
-    __device__ __forceinline__ void init(const uint8_t *w, uint32_t row0, uint32_t rows, uint32_t nsb, uint8_t *wave_area) {
-        const uint32_t lane = threadIdx.x & 63u;
-        lh = lane >> 5;
-        lr = lane & 31u;
-        area = wave_area;
-        stride = nsb * 210u;
-        base = w + (uint64_t)(row0 < rows ? row0 : rows - 1u) * stride;
-        const uint32_t most = row0 < rows ? rows - 1u - row0 : 0u;
-#pragma unroll
-        for (int j = 0; j < kLoads; ++j) {
-            const uint32_t r = piece(j) / 14u;
-            row_off[j] = (r < most ? r : most) * stride;
-        }
-        lr_off = (lr < most ? lr : most) * stride;
-    }
-    uint32_t lr_off;
-    __device__ __forceinline__ void request(uint32_t sb) {
-        const uint8_t *const b = base + (uint64_t)sb * 210u;
-        const uint32_t low = (uint32_t)(uintptr_t)b & 3u;
-#pragma unroll
-        for (int j = 0; j < kLoads; ++j) {
-            const uint32_t i = piece(j) % 14u;
-            n[j] = *reinterpret_cast<const u32x4_a4 *>((b - low) + (((low + row_off[j]) & ~3u) + (i < 13u ? 16u * i : 196u)));
-        }
-        nshift = ((low + lr_off) & 2u) * 8u;
-    }
-    __device__ __forceinline__ void touch() {
-#pragma unroll
-        for (int j = 0; j < kLoads; ++j) asm volatile("" : "+v"(n[j].x), "+v"(n[j].y), "+v"(n[j].z), "+v"(n[j].w));
-    }
-    __device__ __forceinline__ void take() {
-        // the area is this wave's own: LDS runs a wave's accesses in order
-#pragma unroll
-        for (int j = 0; j < kLoads; ++j) {
-            const uint32_t q = piece(j), r = q / 14u;
-            *reinterpret_cast<lev_u32x4 *>(area + r * kRow + (q - 14u * r) * 16u) = n[j];
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        shift = nshift;
-        const uint8_t *const mine = area + lr * kRow;
-        const lev_u32x4 s = *reinterpret_cast<const lev_u32x4 *>(mine + 192u);
-        const uint32_t last = *reinterpret_cast<const uint32_t *>(mine + 220u);   // bytes 208 .. 211 from the first dword
-        sc[0] = __builtin_amdgcn_alignbit(s.y, s.x, shift);
-        sc[1] = __builtin_amdgcn_alignbit(s.z, s.y, shift);
-        sc[2] = __builtin_amdgcn_alignbit(s.w, s.z, shift);
-        sc[3] = __builtin_amdgcn_alignbit(last, s.w, shift);
-        d = lev_f16_bits_to_f32((last >> shift) & 0xFFFFu);
-        half(0);
-    }
-    // the codes of half a column: 32 bytes of ql (the lane's half of 64), 32 of qh
-    __device__ __forceinline__ void half(int hf) {
-        const uint8_t *const mine = area + lr * kRow;
-        auto eight = [&](const uint8_t *p, uint32_t (&o)[8]) {
-            const lev_u32x4 a = *reinterpret_cast<const lev_u32x4 *>(p), b = *reinterpret_cast<const lev_u32x4 *>(p + 16);
-            const uint32_t c = *reinterpret_cast<const uint32_t *>(p + 32);
-            o[0] = __builtin_amdgcn_alignbit(a.y, a.x, shift);
-            o[1] = __builtin_amdgcn_alignbit(a.z, a.y, shift);
-            o[2] = __builtin_amdgcn_alignbit(a.w, a.z, shift);
-            o[3] = __builtin_amdgcn_alignbit(b.x, a.w, shift);
-            o[4] = __builtin_amdgcn_alignbit(b.y, b.x, shift);
-            o[5] = __builtin_amdgcn_alignbit(b.z, b.y, shift);
-            o[6] = __builtin_amdgcn_alignbit(b.w, b.z, shift);
-            o[7] = __builtin_amdgcn_alignbit(c, b.w, shift);
-        };
-        eight(mine + 64u * hf + 32u * lh, ql);
-        eight(mine + 128u + 32u * hf, qh);
-    }
-    __device__ __forceinline__ f16x8 frag(int c, int q) const {
-        const int hf = c >> 1, np = c & 1;
-        const float ds = d * (float)(int)__builtin_amdgcn_sbfe((int)sc[2 * hf + np], 8u * (2u * lh + (uint32_t)(q >> 1)), 8u);
-        const float nbm = -1056.0f * ds;
-        f16x8 f;
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const uint32_t a = ql[2 * q + i], h = qh[2 * q + i];
-            const uint32_t code = np ? (((a >> 4) & 0x0F0F0F0Fu) | ((h >> (2u * lh)) & 0x30303030u))
-                                     : ((a & 0x0F0F0F0Fu) | ((h << (4u - 2u * lh)) & 0x30303030u));
-            q6g_put4_mix(code, ds, nbm, f, 4 * i);
-        }
-        return f;
-    }
-    __device__ __forceinline__ uint32_t unit(int q) const { return 4u * lh + (uint32_t)q; }
-};
 
 // grid: row tiles * token tiles * (zn slices from z0 on, of the `splits`) workgroups in one line, up to a multiple of
 // eight.  All slices of a launch write partial tiles of their own to `out`, one behind the other; add: the one slice
@@ -230,66 +88,74 @@ gemm_split_kernel(const uint8_t *__restrict__ w, const uint16_t *__restrict__ x,
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[t][i] = 0.f;
 
-    wt.touch();
-    wt.take();
-    f16x8 a[2][T], b = wt.frag(0, 0);
-    for (uint32_t i = 0; i < most; ++i) {
+    // The products run two groups (of the four of a step) behind the barriers: groups 2 and 3 of a step are multiplied
+    // behind the next barrier, from fragments read in front of it, while the first fragments of the new step come in.
+    // Otherwise all waves wait for their LDS reads at the same time, behind every barrier.  The first step's are zeros.
+    const uint32_t mine = sb1 - sb0;
+    f16x8 a[4][T], b;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        b[i] = (_Float16)0.f;
+#pragma unroll
+        for (int t = 0; t < T; ++t) a[2][t][i] = a[3][t][i] = (_Float16)0.f;
+    }
+    wt.clear();
+    // products of a group and behind them, while they run, the X fragments of the group `read` (-1: none) and `next`,
+    // which makes the following B: one MFMA, then what can issue while it runs (a wave issues in order, and a second
+    // MFMA behind the first would hold it for 32 clocks)
+    auto phase = [&](const uint8_t *xb, int q, int read, auto next) {
+#pragma unroll
+        for (int t = 0; t < T; ++t) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[q][t], b, acc[t], 0, 0, 0);
+        if (read >= 0) {
+#pragma unroll
+            for (int t = 0; t < T; ++t)
+                a[read][t] = *reinterpret_cast<const f16x8 *>(xb + t * kTile + 16u * (wt.unit(read) ^ (lr & 7u)));
+        }
+        next();
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                    // MFMA
+            if (read >= 0) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);     // LDS read
+            __builtin_amdgcn_sched_group_barrier(0x002, (28 + T - 1) / T, 0);     // VALU
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    for (uint32_t i = 0; i < mine; ++i) {
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
             const uint32_t step = i * 4u + c;
             // This step's X has landed: newer are the X of the steps behind it and, behind a superblock's
-            // first step, the next superblock's weights, which are wanted by the fourth.
+            // first step, the next superblock's weights, which are wanted by the one after its fourth.
             static_assert(kBufs == 4u || kBufs == 2u, "the counts below");
-            if (c == 1 || (c == 2 && kBufs == 4u)) LEV_WAIT_VMCNT((kBufs - 2u) * kXLoads + W::kLoads);
+            if (c == 1 || (c >= 2 && kBufs == 4u)) LEV_WAIT_VMCNT((kBufs - 2u) * kXLoads + W::kLoads);
             else LEV_WAIT_VMCNT((kBufs - 2u) * kXLoads);
-            if (c == 3) wt.touch();   // the compiler's own wait for them goes here, where it is free
+            if (c == 0) wt.touch();   // the compiler's own wait for them goes here, behind ours for the X requested after them
             __builtin_amdgcn_sched_barrier(0);
             lev_barrier_lds();          // everybody's has, and everybody is done with the other buffer
             x_request(step + kBufs - 1u);
+            __builtin_amdgcn_sched_barrier(0);
+            const uint8_t *const xb = xmine + (step % kBufs) * (T * kTile);
+#pragma unroll
+            for (int t = 0; t < T; ++t) a[0][t] = *reinterpret_cast<const f16x8 *>(xb + t * kTile + 16u * (wt.unit(0) ^ (lr & 7u)));
+            phase(xb, 2, -1, [&] { b = wt.frag((c + 3) & 3, 3); });
+            phase(xb, 3, 1, [&] {
+                if (c == 0) wt.take();
+                if (c == 2) wt.half(1);
+                b = wt.frag(c, 0);
+            });
             if (c == 0) {
-                __builtin_amdgcn_sched_barrier(0);
                 const uint32_t sb = sb0 + i + 1u;
                 wt.request(sb < sb1 ? sb : sb1 - 1u);
                 __builtin_amdgcn_sched_barrier(0);
             }
-            const uint8_t *const xb = xmine + (step % kBufs) * (T * kTile);
-            auto a_read = [&](int q) {
-#pragma unroll
-                for (int t = 0; t < T; ++t)
-                    a[q & 1][t] = *reinterpret_cast<const f16x8 *>(xb + t * kTile + 16u * (wt.unit(q) ^ (lr & 7u)));
-            };
-            if (sb0 + i < sb1) {
-                a_read(0);
-                a_read(1);
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-#pragma unroll
-                    for (int t = 0; t < T; ++t) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[q & 1][t], b, acc[t], 0, 0, 0);
-                    // behind them, while they run: the X fragments of the product after the next and the next B
-                    if (q < 2) a_read(q + 2);
-                    if (q < 3) {
-                        b = wt.frag(c, q + 1);
-                    } else if (c < 3) {
-                        if (c == 1) wt.half(1);
-                        b = wt.frag(c + 1, 0);
-                    } else {
-                        wt.take();
-                        b = wt.frag(0, 0);
-                    }
-                    // one MFMA, then what can issue while it runs: a wave issues in order, and a second MFMA
-                    // behind the first would hold it for 32 clocks
-#pragma unroll
-                    for (int t = 0; t < T; ++t) {
-                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                    // MFMA
-                        if (q < 2) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);         // LDS read
-                        __builtin_amdgcn_sched_group_barrier(0x002, (28 + T - 1) / T, 0);     // VALU
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            }
+            phase(xb, 0, 2, [&] { b = wt.frag(c, 1); });
+            phase(xb, 1, 3, [&] { b = wt.frag(c, 2); });
         }
     }
+    phase(xmine, 2, -1, [&] { b = wt.frag(3, 3); });
+    phase(xmine, 3, -1, [] {});
+    // (the waves of a shorter slice: one superblock less)
+    for (uint32_t i = 4u * mine; i < 4u * most; ++i) asm volatile("s_barrier" ::: "memory");
     LEV_WAIT_VMCNT(0);   // the request past the end lands before the LDS is used again
 
     if (KW > 1) {
@@ -311,30 +177,20 @@ gemm_split_kernel(const uint8_t *__restrict__ w, const uint16_t *__restrict__ x,
 #pragma unroll
                 for (int i = 0; i < 16; ++i) acc[t][i] += red[((((k - 1u) * RW + rw) * T + t) * 16 + i) * 64 + lane];
     }
-    if (row >= rows) return;
-    float *const dst = out + (uint64_t)zl * tokens * rows + row;
-    if (add) {
-#pragma unroll 1
-        for (int t = 0; t < T; ++t) {
-            const uint32_t first = tok0 + 32u * t + 4u * lh;
+    // a tile's 32 tokens from `first` on; past the tokens' end and for rows past the last one nothing is stored
+    float *const dst = out + (uint64_t)zl * tokens * rows;
+    const uint32_t at = row < rows ? (4u * lh * rows + row) * 4u : lev_buffer::kNothing;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const uint32_t tok = first + 8u * (i / 4) + (i % 4);
-                float v = 0.f;
-#pragma unroll
-                for (int k = 0; k < T; ++k) v = k == t ? acc[k][i] : v;
-                if (tok < tokens) dst[(uint64_t)tok * rows] += v;
-            }
-        }
-        return;
-    }
-#pragma unroll
-    for (int t = 0; t < T; ++t)
+    for (int t = 0; t < T; ++t) {
+        const uint32_t first = tok0 + 32u * t, here = first < tokens ? (tokens - first < 32u ? tokens - first : 32u) : 0u;
+        const lev_buffer tile_out(dst + (uint64_t)(here ? first : 0u) * rows, here * rows * 4u);
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-            const uint32_t tok = tok0 + 32u * t + 8u * (i / 4) + 4u * lh + (i % 4);
-            if (tok < tokens) dst[(uint64_t)tok * rows] = acc[t][i];
+            const uint32_t tok = (uint32_t)(8 * (i / 4) + (i % 4)) * rows * 4u;
+            const float v = add ? acc[t][i] + __uint_as_float(tile_out.load4(at, 0, tok)) : acc[t][i];
+            tile_out.store4(__float_as_uint(v), at, 0, tok);
         }
+    }
 }
 
 // y[i] = sum over the splits, in order

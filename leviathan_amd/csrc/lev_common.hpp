@@ -239,8 +239,8 @@ __device__ __forceinline__ uint32_t lev_lds_offset(const void *lds) {
     return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const uint8_t *)lds;
 }
 
-// Loads from `bytes` bytes at a wave-uniform base by 32-bit offset.  A lane whose offset is kNothing gets zeros and asks
-// the memory for nothing.  `fixed` is a constant, `uniform` the same for all lanes; the sum is checked against
+// Loads from and stores to `bytes` bytes at a wave-uniform base by 32-bit offset.  A lane whose offset is kNothing, or
+// beyond the end, gets zeros and asks the memory for nothing; nothing of it is stored.  `fixed` is a constant, `uniform` the same for all lanes; the sum is checked against
 // `bytes`, for which kNothing leaves room on both sides (bytes, fixed and uniform at most 2^30).
 struct lev_buffer {
     static constexpr uint32_t kNothing = 0x80000000u;
@@ -252,6 +252,9 @@ struct lev_buffer {
     }
     __device__ __forceinline__ uint32_t load4(uint32_t offset, int fixed, uint32_t uniform = 0u) const {
         return __builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)offset + fixed, (int)uniform, 0);
+    }
+    __device__ __forceinline__ void store4(uint32_t v, uint32_t offset, int fixed, uint32_t uniform = 0u) const {
+        __builtin_amdgcn_raw_buffer_store_b32(v, rsrc, (int)offset + fixed, (int)uniform, 0);
     }
 };
 

@@ -210,15 +210,8 @@ q4_k_gemm_kernel(const uint8_t *__restrict__ w, const uint16_t *__restrict__ x,
                 const int rg = ph == 0 ? 1 : ph;   // the group read in this phase (none in phase 1)
                 // fragment ph of the NEXT chunk is decoded behind this phase's MFMAs
                 const lev_u32x4 w4 = qs[cn];
-                uint32_t c0 = (ph & 1) ? w4.z : w4.x, c1 = (ph & 1) ? w4.w : w4.y;
-                if (ph >= 2) {
-                    c0 >>= 4;
-                    c1 >>= 4;
-                }
-                c0 &= 0x0F0F0F0Fu;
-                c1 &= 0x0F0F0F0Fu;
-                asm("" : "+v"(c0));
-                asm("" : "+v"(c1));
+                const uint32_t c0 = (ph & 1) ? w4.z : w4.x, c1 = (ph & 1) ? w4.w : w4.y;
+                const uint32_t hmask = ph >= 2 ? 0x00F000F0u : 0x000F000Fu;
                 const float fd = d1[2 * cn + (ph >> 1)], fm = mm[2 * cn + (ph >> 1)];
                 f16x8 nf;
                 // Six slots of { one MFMA, a few other instructions }: a wave issues in
@@ -234,10 +227,9 @@ q4_k_gemm_kernel(const uint8_t *__restrict__ w, const uint16_t *__restrict__ x,
                     if (r != 2) {
                         const int s4 = 2 * m + r;
                         const uint32_t cw = s4 < 2 ? c0 : c1;
-                        const float e0 = (s4 & 1) ? (float)((cw >> 16) & 0xFFu) : (float)(cw & 0xFFu);
-                        const float e1 = (s4 & 1) ? (float)(cw >> 24) : (float)((cw >> 8) & 0xFFu);
-                        nf[2 * s4] = q4k_weight_f16(fd, e0, fm);
-                        nf[2 * s4 + 1] = q4k_weight_f16(fd, e1, fm);
+                        const f16x2 ev = __builtin_bit_cast(f16x2, cw & hmask), od = __builtin_bit_cast(f16x2, (cw >> 8) & hmask);
+                        nf[2 * s4] = q4k_weight_f16(fd, (s4 & 1) ? ev.y : ev.x, fm);
+                        nf[2 * s4 + 1] = q4k_weight_f16(fd, (s4 & 1) ? od.y : od.x, fm);
                     }
                     // wave 3 decoded wave 2's rows: it stores the same values to the same place,
                     // which keeps the stream free of branches (a branch makes the compiler wait
