@@ -262,49 +262,40 @@ hipError_t launch(lev_ctx *ctx, const uint8_t *w, const uint16_t *x, float *y, u
 }  // namespace
 
 // Which of the GEMMs takes a shape, in how many K slices and token tiles of which height: the least of what each would
-// take, from times measured over 1000 to 32000 rows, 1024 to 12288 columns and 17 to 1000 tokens (us; a step is 64 values
-// of K, t = 32-token tiles a wave; of 60 shapes the choice was within 0.2 % of the best on average, 5 % at worst).
-//   256-token tiles:  a round of workgroups (one per CU) 6.1 + in_dim / 1024 * (9.8 + 3.8 * share of the CUs it
-//                     fills), Q6_K 5.7 + in_dim / 1024 * (19.2 + 3.5 *): 46 to 60 us at 4096 columns of Q4_K;
-//   KW = 1:           a round of up to two workgroups a CU; their steps take 1.6 times those of one alone;
+// take, from times measured on every plan of 450 shapes a format drawn over 1000 to 32000 rows, 1024 to 12288 columns and
+// 17 to 1024 tokens (us; a step is 64 values of K, t = 32-token tiles a wave; the choice is within 1.2 % of the best on
+// average, 7.5 % in nineteen of twenty).
+//   256-token tiles:  a round of workgroups (one per CU), more as it fills the CUs, and X put into order in front;
+//   KW = 1:           a round of up to two workgroups a CU; their steps take 1.8 times those of one alone;
 //   KW = 2, KW = 4:   a round of one a CU, and with S > 1 splits the kernel that adds and its reads and writes.
 // Lower token tiles are more workgroups that decode the same weights: what fills the chip where rows alone do not.
-// Beyond 1024 tokens the times of KW = 1 outgrow these, by 1.1 to 1.45, with the tokens that its tiles really hold
-// (those of 256 tokens stay within 0.87 to 1.1).  Over 216 shapes of 1025 to 8192 tokens the 256-token tiles were the
-// faster ones where nearly every token of them is one and the CUs are full: for Q6_K from 15/16 of the CUs (4096 x 4096 at
-// 4096 tokens 174.7 us against 187.2, 32000 x 4096 at 4096 tokens 1361 against 1449), unless there are more than 2^28
-// weights (220 MB, about what the Infinity Cache holds: 32000 rows of 12288 at 3072 tokens 4 % more); for Q4_K from 31/32 of them and
-// eight token tiles (12288 x 4096 at 4096 tokens 469 us against 505, at 2048 tokens 236 against 242), but not over short
-// rows (16384 rows of 1024 at 8192 tokens 2 % more), and where the estimates are within 1.1 (12288 x 4096 at 1500 tokens
-// 180 us against 193).  47 shapes of Q6_K and 23 of Q4_K are faster so, by some 4 % on average and none slower by more
-// than 0.4 %; Q4_K at 2048 tokens is between 2.7 % faster and 1.5 % slower, by the shape and the card's clock.
+// Beyond 1024 tokens the times of these outgrow the estimates, by 1.1 in the middle and up to 1.4, those of the 256-token
+// tiles hardly do: 1.15 is allowed for that (120 shapes a format of up to 8192 tokens).
 // Tall matrices (768 row tiles and more) and rows of fewer than six superblocks are never cut along K, so that
 // there every kernel adds in the same order.
-lev_gemm_split_plan lev_gemm_split_choose(const lev_ctx *ctx, bool q6, uint32_t in_dim, uint32_t rows, uint32_t tokens,
-                                          uint32_t big_rows) {
-    const double cus = ctx->num_cus;
+lev_gemm_split_plan lev_gemm_split_choose(const lev_ctx *ctx, bool q6, uint32_t in_dim, uint32_t rows, uint32_t tokens) {
+    const double cus = ctx->num_cus, long_prompt = tokens > 1024u ? 1.15 : 1.0;
     const uint32_t nsb = in_dim / 256u, tiles = (tokens + 31u) / 32u;
-    const double big_wgs = (double)((rows + big_rows - 1u) / big_rows) * ((tokens + 255u) / 256u);
-    const double big_rounds = std::ceil(big_wgs / cus), fill = big_wgs / (big_rounds * cus);
-    lev_gemm_split_plan best{0u, 1u, 1u};
-    double least = big_rounds * (q6 ? 5.7 + in_dim / 1024.0 * (19.2 + 3.5 * fill) : 6.1 + in_dim / 1024.0 * (9.8 + 3.8 * fill));
-    if (tokens > 1024u) {
-        const uint64_t tiled = (tokens + 255ull) / 256u * 256u;
-        if (tokens * 32ull >= tiled * 31u && (q6 ? fill >= 15.0 / 16.0 && (uint64_t)in_dim * rows <= 1u << 28
-                                                 : fill >= 31.0 / 32.0 && in_dim >= 2048u && tiled >= 2048u))
-            return best;
-        if (!q6) least /= 1.1;
-    }
-    struct cost { double start, step, per_tile, full, sum, sum_mb; };
-    const cost k1 = q6 ? cost{4.9, 0.383, 0.067, 0.60, 0, 0} : cost{4.0, 0.267, 0.076, 0.66, 0, 0};
-    const cost k2 = q6 ? cost{4.3, 0.558, 0.145, 0.16, 3.1, 0.7} : cost{3.9, 0.363, 0.165, 0.08, 2.9, 0.75};
-    const cost k4 = q6 ? cost{4.1, 0.534, 0.248, 0.02, 4.8, 0.0} : cost{4.6, 0.206, 0.287, 0.05, 3.1, 0.56};
+    lev_gemm_split_plan best{};
+    double least = 1e300;
     auto offer = [&](double us, uint32_t kw, uint32_t splits, uint32_t t) {
         if (us < least) {
             least = us;
             best = lev_gemm_split_plan{kw, splits, t};
         }
     };
+    struct wide_cost { double start, k, fill, once, order; };
+    const wide_cost w3 = q6 ? wide_cost{5.3, 7.9, 4.25, 4.4, 1.15} : wide_cost{6.2, 5.15, 5.45, 3.75, 1.8};
+    const wide_cost w4 = q6 ? wide_cost{6.9, 8.1, 7.0, 4.3, 1.05} : wide_cost{7.7, 6.1, 7.4, 3.0, 1.35};
+    for (uint32_t rt = 3; rt <= 4u; ++rt) {
+        const wide_cost &k = rt == 3u ? w3 : w4;
+        const double n = (double)((rows + 32u * rt - 1u) / (32u * rt)) * ((tokens + 255u) / 256u), rounds = std::ceil(n / cus);
+        offer(rounds * (k.start + in_dim / 1024.0 * (k.k + k.fill * n / (rounds * cus))) + k.once + k.order * 1e-6 * tokens * in_dim, 0u, rt, 0u);
+    }
+    struct cost { double start, step, per_tile, full, once, sum, sum_mb; };
+    const cost k1 = q6 ? cost{0.66, 0.33, 0.089, 0.72, 2.9, 0, 0} : cost{0.0, 0.205, 0.085, 0.78, 3.0, 0, 0};
+    const cost k2 = q6 ? cost{2.1, 0.457, 0.111, 0.27, 3.2, 1.6, 1.08} : cost{0.17, 0.224, 0.125, 0.42, 4.4, 2.1, 1.14};
+    const cost k4 = q6 ? cost{2.56, 0.42, 0.165, 0.31, 2.06, 2.26, 0.93} : cost{0.83, 0.198, 0.193, 0.39, 3.6, 2.07, 1.47};
     for (uint32_t t = 1; t <= 4u && t <= tiles; ++t) {
         const double tok_tiles = (tiles + t - 1u) / t;
         // workgroups, whole eighths of them on an XCD each
@@ -312,7 +303,7 @@ lev_gemm_split_plan lev_gemm_split_choose(const lev_ctx *ctx, bool q6, uint32_t 
         {
             const double n = wgs_of(128u, 1u), whole = std::floor(n / (2.0 * cus)), rest = n - whole * 2.0 * cus;
             const double rounds = whole + (rest > 0.0 ? 1.0 : 0.0), pairs = whole + (rest > cus ? 1.0 : 0.0);
-            offer(rounds * k1.start + 4.0 * nsb * (k1.step + k1.per_tile * t) * (rounds + k1.full * pairs), 1u, 1u, t);
+            offer(long_prompt * (rounds * k1.start + 4.0 * nsb * (k1.step + k1.per_tile * t) * (rounds + k1.full * pairs) + k1.once), 1u, 1u, t);
         }
         if ((rows + 31u) / 32u >= 768u || nsb < 6u) continue;
         for (uint32_t kw = 2; kw <= 4u; kw += 2u) {
@@ -321,8 +312,8 @@ lev_gemm_split_plan lev_gemm_split_choose(const lev_ctx *ctx, bool q6, uint32_t 
             for (uint32_t s = 1; s <= 8u && s * kw <= nsb; ++s) {
                 const double n = wgs_of(kw == 2u ? 128u : 64u, s), rounds = std::ceil(n / cus), full = n / (rounds * cus);
                 const double steps = 4.0 * ((nsb + kw * s - 1u) / (kw * s));
-                offer(rounds * (k.start + steps * (k.step + k.per_tile * t) * (1.0 + k.full * full)) +
-                          (s > 1u ? k.sum + k.sum_mb * 1e-6 * (s + 1.0) * tokens * rows : 0.0), kw, s, t);
+                offer(long_prompt * (rounds * (k.start + steps * (k.step + k.per_tile * t) * (1.0 + k.full * full)) + k.once +
+                                     (s > 1u ? k.sum + k.sum_mb * 1e-6 * (s + 1.0) * tokens * rows : 0.0)), kw, s, t);
             }
         }
     }

@@ -1,0 +1,241 @@
+// Q4_K and Q6_K prefill GEMM for prompts whose 256-token tiles fill the chip:  Y[t][r] = sum_k X[t][k] W[r][k].
+//
+// Stands in for the cooperative-matrix "gemm blocked" kernels (lev-forge/src/coopmat.rs:236-425; caller
+// lev-model/src/gpu.rs:345-355; gate lev-cli/src/main.rs:1187-1279).  As there, W is dequantised to fp16 (f32 arithmetic,
+// then round-to-nearest-even) and X arrives as fp16; products accumulate in f32.  Both operands use the same 16-bit type
+// because one MFMA takes one input type; fp16 keeps X exactly as given.
+//
+// A workgroup owns 256 tokens x 32 RT rows (RT = 3 or 4), one workgroup a CU, eight waves, two a SIMD:
+//   * waves 0..3 multiply: 64 tokens x all rows each, 2 RT tiles of v_mfma_f32_32x32x16_f16, K step 64.  Their tokens are
+//     nobody else's, so X never goes through LDS: a small kernel in front puts X into the order in which the lanes of a
+//     fragment take it (1 KB of consecutive bytes a fragment), and a wave requests a fragment four or eight products ahead
+//     of its use, straight into registers;
+//   * waves 4..7 decode, one 32-row tile each (RT = 3: three of them): every weight is decoded once a workgroup, a step
+//     ahead, and handed over as B fragments in two LDS buffers of 4 RT KB, one barrier a step.
+// The multiplying waves run two groups of products behind the barriers: groups 2 and 3 of a step are multiplied behind the
+// next barrier, from fragments read in front of it, while the first fragments of the new step come in.
+//
+// Why this split.  A lone wave of a SIMD issues a vector instruction every six clocks, two waves one every three to five,
+// and an MFMA leaves the vector pipe half of its 32 clocks, so decode and products on different waves of a SIMD cover each
+// other.  What the LDS has to carry bounds the tile: with X in LDS as well (the kernels this one took the place of) it was
+// 124 KB a step of 96 x 256 x 64, 990 clocks beside 770 of MFMAs; 60 KB here.  512 tokens, 4096 columns, us under a
+// sustained load: 12288 rows of Q4_K 58.9 before and 55.6, of Q6_K 76.7 and 60.0, 32000 rows of Q6_K 175.8 and 143.4
+// (0.94 PFLOP/s).  Without the decode 44, without the X loads no less: what is left is the clock, which under these
+// products falls to 1.5 to 1.8 GHz (a loop of MFMAs alone takes 33 us for the first of these, the library's fp16 product 51).
+//
+// K order inside a 64-step is permuted consistently on both operands (unit_of of the formats' weights); the sums are formed
+// in the order in which a wave of gemm_split.hip that takes all of K forms them: the same bits.
+#include "prefill_decode.hpp"
+
+namespace {
+
+constexpr uint32_t kWideThreads = 512;      // four waves that multiply, four that decode
+constexpr uint32_t kFrag = 1024u;           // a fragment: 16 bytes a lane
+constexpr int kTM = 2;                      // 32-token tiles a wave
+
+// X as fragments: [32-token tile][chunk of 64][group q][lane][16 bytes].  A wave a chunk of a tile; tokens past the end
+// repeat the last.  512 x 4096: 2.6 us.
+template <typename W>
+__global__ void __launch_bounds__(256)
+gemm_x_fragments(const uint16_t *__restrict__ x, lev_u32x4 *__restrict__ out, uint32_t in_dim, uint32_t tokens) {
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, lr = lane & 31u;
+    const uint32_t chunk = blockIdx.x * 4u + wave, t = blockIdx.y * 32u + lr, nchunk = in_dim >> 6;
+    if (chunk >= nchunk) return;
+    const lev_u32x4 *src = reinterpret_cast<const lev_u32x4 *>(x + (uint64_t)(t < tokens ? t : tokens - 1u) * in_dim + 64u * chunk);
+    lev_u32x4 v[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] = src[W::unit_of(lane >> 5, q)];
+    lev_u32x4 *dst = out + ((uint64_t)blockIdx.y * nchunk + chunk) * 256u + lane;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) dst[64 * q] = v[q];
+}
+
+// grid: row tiles * token tiles in one line, up to a multiple of eight; the workgroups of an XCD take an eighth of the tiles,
+// in whose order the token tiles of a row tile are together (they read the same weights).
+// LDS: two buffers of B fragments [group][row tile], and what the format's weights take a decoding wave.
+template <typename W, int RT>
+__global__ void __launch_bounds__(kWideThreads, 2)
+gemm_wide_kernel(const uint8_t *__restrict__ w, const uint8_t *__restrict__ xf, float *__restrict__ y, uint32_t in_dim,
+                 uint32_t rows, uint32_t tokens, uint32_t row_tiles, uint32_t tok_tiles) {
+    constexpr int RING = RT == 4 ? 4 : 8;      // groups of X requested ahead, as many as the registers hold
+    constexpr uint32_t kBuf = RT * 4u * kFrag;
+    extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
+    const uint32_t lane = threadIdx.x & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const uint32_t lr = lane & 31u, lh = lane >> 5;
+    const uint32_t tile = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3), rt = tile / tok_tiles;
+    if (rt >= row_tiles) return;
+    const uint32_t row0 = rt * (32u * RT), tt0 = (tile - rt * tok_tiles) * (4u * kTM);
+    const uint32_t nsb = in_dim >> 8, nsteps = nsb * 4u;
+    if (wave >= 4u) {
+        const uint32_t f = wave - 4u;
+        if (f >= (uint32_t)RT) {
+            for (uint32_t ks = 0; ks < nsteps; ++ks) asm volatile("s_barrier" ::: "memory");   // nothing to decode
+            return;
+        }
+        W wt;
+        wt.init(w, row0 + 32u * f, rows, nsb, lds + 2u * kBuf + f * W::kArea);
+        wt.request(0);
+        wt.touch();
+        wt.take();
+        uint8_t *const dst = lds + f * kFrag + lane * 16u;
+        auto produce = [&](int c, uint32_t buf) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) *reinterpret_cast<f16x8 *>(dst + buf * kBuf + q * (RT * kFrag)) = wt.frag(c, q);
+        };
+        produce(0, 0u);
+        for (uint32_t i = 0; i < nsb; ++i) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                __builtin_amdgcn_s_waitcnt(0xC07F);
+                asm volatile("s_barrier" ::: "memory");
+                if (c == 0) wt.request(i + 1u < nsb ? i + 1u : nsb - 1u);
+                if (c == 1) wt.half(1);
+                if (c == 3) {
+                    wt.touch();
+                    wt.take();
+                }
+                produce((c + 1) & 3, (c + 1) & 1);
+            }
+        }
+        return;
+    }
+    const uint32_t ngroup = nsteps * 4u;
+    const uint32_t tile_bytes = ngroup * kFrag;
+    const uint32_t tt = tt0 + wave * kTM, last_tt = (tokens + 31u) / 32u - 1u;
+    const lev_buffer xb0(xf + (uint64_t)(tt < last_tt ? tt : last_tt) * tile_bytes, tile_bytes);
+    const lev_buffer xb1(xf + (uint64_t)(tt + 1u < last_tt ? tt + 1u : last_tt) * tile_bytes, tile_bytes);
+    lev_u32x4 xr[RING][kTM];
+    auto x_request = [&](uint32_t n, int slot) {
+        xr[slot][0] = xb0.load16(lane * 16u, 0, n * kFrag);
+        xr[slot][1] = xb1.load16(lane * 16u, 0, n * kFrag);
+    };
+#pragma unroll
+    for (int n = 0; n < RING; ++n) x_request(n, n);
+    f32x16 acc[RT][kTM];
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int m = 0; m < kTM; ++m)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[r][m][i] = 0.f;
+    f16x8 b[4][RT];
+    const uint8_t *const bb = lds + lane * 16u;
+    auto b_read = [&](int q, int r, uint32_t buf) { b[q][r] = *reinterpret_cast<const f16x8 *>(bb + buf * kBuf + (q * RT + r) * kFrag); };
+    // group q of step parity p: products, meanwhile group `rq` of buffer rbuf is read
+    auto phase = [&](int q, int p, uint32_t n, int rq, uint32_t rbuf) {
+        const int slot = (4 * p + q) % RING;
+#pragma unroll
+        for (int i = 0; i < RT * kTM; ++i) {
+            const int r = i % RT, m = i / RT;
+            acc[r][m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, xr[slot][m]), b[q][r], acc[r][m], 0, 0, 0);
+            if (rq >= 0 && i < RT) b_read(rq, i, rbuf);
+            if (i == RT * kTM - 1) x_request(n + RING, slot);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    auto meet = [&] {
+        __builtin_amdgcn_s_waitcnt(0xC07F);
+        asm volatile("s_barrier" ::: "memory");
+    };
+    meet();
+#pragma unroll
+    for (int r = 0; r < RT; ++r) b_read(0, r, 0u);
+#pragma unroll
+    for (int r = 0; r < RT; ++r) b_read(1, r, 0u);
+    __builtin_amdgcn_sched_barrier(0);
+    phase(0, 0, 0u, 2, 0u);
+    phase(1, 0, 1u, 3, 0u);
+    auto step = [&](auto parity, uint32_t ks) {
+        constexpr int p = decltype(parity)::value;
+        meet();
+#pragma unroll
+        for (int r = 0; r < RT; ++r) b_read(0, r, p);
+        __builtin_amdgcn_sched_barrier(0);
+        phase(2, 1 - p, ks * 4u - 2u, -1, 0u);
+        phase(3, 1 - p, ks * 4u - 1u, 1, p);
+        phase(0, p, ks * 4u, 2, p);
+        phase(1, p, ks * 4u + 1u, 3, p);
+    };
+    uint32_t ks = 1;
+    for (; ks + 1u < nsteps; ks += 2u) {
+        step(std::integral_constant<int, 1>{}, ks);
+        step(std::integral_constant<int, 0>{}, ks + 1u);
+    }
+    step(std::integral_constant<int, 1>{}, ks);
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    phase(2, 1, ks * 4u + 2u, -1, 0u);
+    phase(3, 1, ks * 4u + 3u, -1, 0u);
+    // past the tokens' end and for rows past the last one nothing is stored
+#pragma unroll
+    for (int m = 0; m < kTM; ++m) {
+        const uint32_t first = (tt + m) * 32u, here = first < tokens ? (tokens - first < 32u ? tokens - first : 32u) : 0u;
+        const lev_buffer out(y + (uint64_t)(here ? first : 0u) * rows, here * rows * 4u);
+#pragma unroll
+        for (int r = 0; r < RT; ++r) {
+            const uint32_t row = row0 + 32u * r + lr, at = row < rows ? (4u * lh * rows + row) * 4u : lev_buffer::kNothing;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) out.store4(__float_as_uint(acc[r][m][i]), at, 0, (uint32_t)(8 * (i / 4) + (i % 4)) * rows * 4u);
+        }
+    }
+}
+
+template <typename W, int RT>
+hipError_t launch_as(lev_ctx *ctx, const uint8_t *w, const uint8_t *xf, float *y, uint32_t in_dim, uint32_t rows, uint32_t tokens) {
+    constexpr size_t lds = 2u * RT * 4u * kFrag + RT * W::kArea;
+    if (hipError_t e = lev_allow_lds(ctx, reinterpret_cast<const void *>(&gemm_wide_kernel<W, RT>), lds); e != hipSuccess) return e;
+    const uint32_t row_tiles = (rows + 32u * RT - 1u) / (32u * RT), tok_tiles = (tokens + 128u * kTM - 1u) / (128u * kTM);
+    hipLaunchKernelGGL((gemm_wide_kernel<W, RT>), dim3((row_tiles * tok_tiles + 7u) / 8u * 8u), dim3(kWideThreads), lds, ctx->stream,
+                       w, xf, y, in_dim, rows, tokens, row_tiles, tok_tiles);
+    return hipGetLastError();
+}
+
+// plan.splits: row tiles a workgroup.  Without scratch for the fragments of X (a program is being recorded and the context's
+// is still too small) a wave of the kernel for short prompts takes all of K.
+template <typename W>
+hipError_t launch(lev_ctx *ctx, const uint8_t *w, const uint16_t *x, float *y, uint32_t in_dim, uint32_t rows, uint32_t tokens,
+                  const lev_gemm_split_plan &plan) {
+    const uint32_t tiles = (tokens + 31u) / 32u;
+    uint8_t *const xf = static_cast<uint8_t *>(lev_scratch(ctx, (size_t)tiles * 32u * in_dim * 2u));
+    if (!xf) return lev_gemm_split_launch(ctx, W::kQ6, w, x, y, in_dim, rows, tokens, lev_gemm_split_plan{1u, 1u, 4u});
+    hipLaunchKernelGGL((gemm_x_fragments<W>), dim3((in_dim / 64u + 3u) / 4u, tiles), dim3(256), 0, ctx->stream, x,
+                       reinterpret_cast<lev_u32x4 *>(xf), in_dim, tokens);
+    if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+    return plan.splits == 4u ? launch_as<W, 4>(ctx, w, xf, y, in_dim, rows, tokens) : launch_as<W, 3>(ctx, w, xf, y, in_dim, rows, tokens);
+}
+
+template <typename W>
+int prefill(lev_ctx *ctx, const char *op, uint32_t block_bytes, uintptr_t w_align, const void *d_w, size_t w_bytes, uint64_t w_off,
+            const uint16_t *d_x_f16, size_t x_count, float *d_y, size_t y_capacity, uint32_t in_dim, uint32_t rows, uint32_t tokens) {
+    if (tokens == 0 || tokens > (1u << 20)) return lev_fail(ctx, LEV_ERR_BAD_DIMENSIONS, "%s: %u tokens", op, tokens);
+    if (in_dim > (1u << 22))
+        return lev_fail(ctx, LEV_ERR_BAD_DIMENSIONS, "%s: in_dim %u above 4194304", op, in_dim);
+    lev_geom g;
+    int st = lev_check_matvec(ctx, op, 256, block_bytes, d_w, w_bytes, w_off, d_x_f16, x_count, (uint64_t)in_dim * tokens, d_y,
+                              y_capacity, (uint64_t)rows * tokens, in_dim, rows, &g);
+    if (st != LEV_OK) return st;
+    const uint8_t *w = static_cast<const uint8_t *>(d_w) + w_off;
+    if ((reinterpret_cast<uintptr_t>(w) & (w_align - 1u)) || (reinterpret_cast<uintptr_t>(d_x_f16) & 15u))
+        return lev_fail(ctx, LEV_ERR_BAD_DIMENSIONS, "%s: weights must be %u-byte and x 16-byte aligned", op, (unsigned)w_align);
+    const lev_gemm_split_plan plan = lev_gemm_split_choose(ctx, W::kQ6, in_dim, rows, tokens);
+    const hipError_t e = plan.kw ? lev_gemm_split_launch(ctx, W::kQ6, w, d_x_f16, d_y, in_dim, rows, tokens, plan)
+                                 : launch<W>(ctx, w, d_x_f16, d_y, in_dim, rows, tokens, plan);
+    return e == hipSuccess ? LEV_OK : lev_hip_check(ctx, e, W::kQ6 ? "q6_k_gemm_prefill launch" : "q4_k_gemm_prefill launch");
+}
+
+}  // namespace
+
+extern "C" int lev_hip_q4_k_gemm_prefill(lev_ctx *ctx, const void *d_w, size_t w_bytes, uint64_t w_off, const uint16_t *d_x_f16,
+                                         size_t x_count, float *d_y, size_t y_capacity, uint32_t in_dim, uint32_t rows,
+                                         uint32_t tokens) {
+    LEV_REQUIRE_CTX(ctx);
+    return prefill<weights_q4k>(ctx, "q4_k_gemm_prefill", 144, 16, d_w, w_bytes, w_off, d_x_f16, x_count, d_y, y_capacity, in_dim,
+                                rows, tokens);
+}
+
+extern "C" int lev_hip_q6_k_gemm_prefill(lev_ctx *ctx, const void *d_w, size_t w_bytes, uint64_t w_off, const uint16_t *d_x_f16,
+                                         size_t x_count, float *d_y, size_t y_capacity, uint32_t in_dim, uint32_t rows,
+                                         uint32_t tokens) {
+    LEV_REQUIRE_CTX(ctx);
+    return prefill<weights_q6k>(ctx, "q6_k_gemm_prefill", 210, 2, d_w, w_bytes, w_off, d_x_f16, x_count, d_y, y_capacity, in_dim,
+                                rows, tokens);
+}

@@ -83,6 +83,7 @@ typedef lev_u32x4 u32x4_a4 __attribute__((aligned(4)));   // a vector on a dword
 // wait for them), take() them as the current column, frag() its fragments; unit(): the 16-byte unit of the
 // step's X row that fragment q meets.  Rows past the end repeat the last row.
 struct weights_q4k {
+    static constexpr bool kQ6 = false;
     static constexpr int kLoads = 5;
     static constexpr uint32_t kArea = 0u;    // LDS bytes a wave
     const uint8_t *row;
@@ -132,6 +133,7 @@ struct weights_q4k {
 // 1 KB, parks them in an area of its own and reads every dword it needs back, shifted by the row's two bytes.
 // (Of the dwords in which the matrix begins and ends two bytes may not be its own: read with the others, never used.)
 struct weights_q6k {
+    static constexpr bool kQ6 = true;
     static constexpr int kLoads = 7;
     static constexpr uint32_t kRow = 240u;   // 224 bytes of pieces + 16: the 32 rows start in different banks
     static constexpr uint32_t kArea = 32u * kRow;
@@ -238,11 +240,10 @@ struct weights_q6k {
     __device__ __forceinline__ uint32_t unit(int q) const { return unit_of(lh, q); }
 };
 
-// The GEMM for short prompts and for shapes whose 256-token tiles leave the chip idle (gemm_split.hip):
-// kw = 0: the 256-token kernel takes the shape (`big_rows` rows a workgroup); else K slices a workgroup, and
-// workgroups that share a tile.
+// Which kernel takes a prefill GEMM (gemm_split.hip).  kw = 0: the one of 256-token tiles (gemm_wide.hip) with `splits` tiles
+// of 32 rows a workgroup; else the one for short prompts and small matrices: K slices a workgroup, workgroups that share a
+// tile, token tiles of 32 a wave.
 struct lev_gemm_split_plan { uint32_t kw, splits, t; };
-lev_gemm_split_plan lev_gemm_split_choose(const lev_ctx *ctx, bool q6, uint32_t in_dim, uint32_t rows, uint32_t tokens,
-                                          uint32_t big_rows);
+lev_gemm_split_plan lev_gemm_split_choose(const lev_ctx *ctx, bool q6, uint32_t in_dim, uint32_t rows, uint32_t tokens);
 hipError_t lev_gemm_split_launch(lev_ctx *ctx, bool q6, const uint8_t *w, const uint16_t *x, float *y, uint32_t in_dim,
                                  uint32_t rows, uint32_t tokens, const lev_gemm_split_plan &plan);

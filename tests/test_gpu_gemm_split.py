@@ -106,3 +106,36 @@ def test_gemm_long_prompts_in_256_token_tiles(ctx, kind, rows, cols, tokens):
         assert np.array_equal(part.view(np.uint32), got[lo:hi].view(np.uint32)), (lo, hi)
     oracle = O.q4_k_gemm_f16_oracle if kind == "q4_k" else O.q6_k_gemm_f16_oracle
     assert O.max_rel_err(got[:, 0::499], oracle(w, rows, cols, x.view(np.uint16), tokens, 0, 499)) < GEMM_TOL
+
+
+@pytest.mark.parametrize("kind,rows,cols,tokens", [
+    ("q4_k", 12200, 2048, 505),     # row tiles of 96, the last ragged; the second token tile ragged
+    ("q4_k", 24500, 4352, 241),     # an odd number of superblocks, one token tile; row tiles of 128
+    ("q6_k", 12200, 2048, 505),
+    ("q6_k", 31990, 2304, 500),     # row tiles of 128, two rounds
+    ("q6_k", 12288, 1792, 256),
+])
+def test_gemm_256_token_tiles(ctx, kind, rows, cols, tokens):
+    """Prompts whose 256-token tiles fill the chip: sampled rows meet the gate, and recorded on a context without room for
+    X in the order of the fragments the call forms the same sums in the same order."""
+    from leviathan_amd import ops
+    w, x = (H.config4 if kind == "q4_k" else config4_q6)(rows, cols, tokens, seed=rows + tokens)
+    got = (gemm if kind == "q4_k" else gemm6)(ctx, w, x, rows, cols, tokens)
+    oracle = O.q4_k_gemm_f16_oracle if kind == "q4_k" else O.q6_k_gemm_f16_oracle
+    assert O.max_rel_err(got[:, 0::331], oracle(w, rows, cols, x.view(np.uint16), tokens, 0, 331)) < GEMM_TOL
+    assert O.max_rel_err(got[:, rows - 1:], oracle(w, rows, cols, x.view(np.uint16), tokens, rows - 1, rows)) < GEMM_TOL
+    wd, xd = dev(w), dev(x)
+    fresh = ops.Context(0, own_stream=True)
+    y = torch.full((tokens, rows), float("nan"), device="cuda")
+    torch.cuda.synchronize()
+    fresh.program_begin()
+    (fresh.q4_k_gemm_prefill if kind == "q4_k" else fresh.q6_k_gemm_prefill)(wd, xd, cols, rows, tokens, y=y)
+    program = fresh.program_end()
+    for _ in range(3):
+        y.fill_(float("nan"))
+        torch.cuda.synchronize()
+        program.run()
+        fresh.sync()
+        assert np.array_equal(y.cpu().numpy().view(np.uint32), got.view(np.uint32))
+    program.destroy()
+    fresh.close()
