@@ -17,6 +17,8 @@
 //   3. down: wave s of a workgroup streams the rows of slot s for the
 //      workgroup's tile of outputs; partial results meet in LDS and are merged
 //      IN SLOT ORDER in f32, as the reference's axpy chain does.
+#include "moe_scores_few.hpp"
+#include "program_nodes.hpp"
 #include "moe_grouped.hpp"
 #include "moe_split.hpp"
 #include "q4_0_mfma.hpp"
@@ -31,39 +33,7 @@ constexpr uint32_t kScoresMfmaMinTokens = 16;   // from here the router scores r
 // router
 // ---------------------------------------------------------------------------
 
-// DPP lane exchange of a 64-bit value; lanes the control word does not write
-// keep their own value.
-template <int CTRL, int ROW_MASK = 0xF>
-__device__ __forceinline__ double dpp_move_f64(double v) {
-    int lo = __double2loint(v), hi = __double2hiint(v);
-    lo = __builtin_amdgcn_update_dpp(lo, lo, CTRL, ROW_MASK, 0xF, false);
-    hi = __builtin_amdgcn_update_dpp(hi, hi, CTRL, ROW_MASK, 0xF, false);
-    return __hiloint2double(hi, lo);
-}
-
-__device__ __forceinline__ double lane63_f64(double v) {
-    int lo = __builtin_amdgcn_readlane(__double2loint(v), 63);
-    int hi = __builtin_amdgcn_readlane(__double2hiint(v), 63);
-    return __hiloint2double(hi, lo);
-}
-
-// Sum / maximum over the 64 lanes, returned in every lane (wave-uniform).
-__device__ __forceinline__ double wave_sum_f64(double v) {
-    v += dpp_move_f64<0xB1>(v);
-    v += dpp_move_f64<0x4E>(v);
-    v += dpp_move_f64<0x141>(v);
-    v += dpp_move_f64<0x140>(v);
-    {   // row_bcast steps: lanes outside the mask must add nothing
-        int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x142, 0xA, 0xF, false);
-        int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x142, 0xA, 0xF, false);
-        v += __hiloint2double(hi, lo);
-        lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x143, 0xC, 0xF, false);
-        hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x143, 0xC, 0xF, false);
-        v += __hiloint2double(hi, lo);
-    }
-    return lane63_f64(v);
-}
-
+// Maximum over the 64 lanes, returned in every lane (wave-uniform).
 __device__ __forceinline__ float wave_max_f32(float v) {
 #define LEV_MAXSTEP(CTRL, MASK)                                                                   \
     v = fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(                           \
@@ -426,48 +396,12 @@ __device__ __forceinline__ float router_weight(const router_sel &r, const float 
     return wgt;
 }
 
-// Router scores of few tokens, f64 accumulation rounded to f32 once: a workgroup per expert and token, whose waves
-// share the row and meet in LDS.  A launch is one trip to memory, so a thread's four pieces of both operands are
-// requested together (rows of up to 4096 columns; longer ones repeat that).  The router comes from L2 for all tokens
-// but the first: at 2816 columns and 128 experts five tokens take 20 us with a row read once for four tokens by one
-// wave, 4.5 us this way.
+// grid (experts, tokens)
 __global__ void __launch_bounds__(256)
 moe_scores_few_kernel(const float *__restrict__ wr, const float *__restrict__ x, float *__restrict__ scores, uint32_t hidden,
                       uint32_t experts) {
     __shared__ double partial[4];
-    const uint32_t e = blockIdx.x, t = blockIdx.y, tid = threadIdx.x;
-    const float *row = wr + (uint64_t)e * hidden, *xv = x + (uint64_t)t * hidden;
-    double acc;
-    if ((hidden & 3u) == 0u && ((reinterpret_cast<uintptr_t>(wr) | reinterpret_cast<uintptr_t>(x)) & 15u) == 0u) {
-        const lev_f32x4 *r4 = reinterpret_cast<const lev_f32x4 *>(row), *x4 = reinterpret_cast<const lev_f32x4 *>(xv);
-        const uint32_t n4 = hidden >> 2;
-        double a0 = 0.0, a1 = 0.0;
-        for (uint32_t i0 = tid; i0 < n4; i0 += 1024u) {
-            lev_f32x4 a[4], b[4];
-#pragma unroll
-            for (uint32_t k = 0; k < 4u; ++k) {
-                const uint32_t i = i0 + 256u * k < n4 ? i0 + 256u * k : i0;
-                a[k] = r4[i];
-                b[k] = x4[i];
-            }
-#pragma unroll
-            for (uint32_t k = 0; k < 4u; ++k) {
-                if (i0 + 256u * k >= n4) b[k] = lev_f32x4{0.f, 0.f, 0.f, 0.f}, a[k] = b[k];
-                a0 = fma((double)a[k].x, (double)b[k].x, a0);
-                a1 = fma((double)a[k].y, (double)b[k].y, a1);
-                a0 = fma((double)a[k].z, (double)b[k].z, a0);
-                a1 = fma((double)a[k].w, (double)b[k].w, a1);
-            }
-        }
-        acc = a0 + a1;
-    } else {
-        acc = 0.0;
-        for (uint32_t i = tid; i < hidden; i += 256u) acc = fma((double)row[i], (double)xv[i], acc);
-    }
-    acc = wave_sum_f64(acc);
-    if ((tid & 63u) == 0u) partial[tid >> 6] = acc;
-    lev_barrier_lds();
-    if (tid == 0u) scores[(uint64_t)t * experts + e] = (float)(((partial[0] + partial[1]) + partial[2]) + partial[3]);
+    moe_score_few(wr, x, scores, hidden, experts, blockIdx.x, blockIdx.y, threadIdx.x, partial);
 }
 
 // Many tokens where the matrix-core kernel below does not apply (rows of no whole 16 columns, unaligned operands):
@@ -1910,4 +1844,55 @@ extern "C" int lev_hip_moe_layer_q4_0_noalloc(lev_ctx *ctx, const lev_moe_expert
         return lev_fail(ctx, LEV_ERR_DEVICE_UNAVAILABLE, "moe_layer_noalloc: the static scratch has no device address");
     return moe_layer_impl(ctx, pools, d_router_w, d_expert_scale, d_x, d_y, d_ids, d_weights, top_k,
                           tokens, ctx->moe_static_scratch, LEV_NOALLOC_MOE_SCRATCH_BYTES);
+}
+
+// ---------------------------------------------------------------------------
+// what recorded programs know of these kernels (program_nodes.hpp)
+// ---------------------------------------------------------------------------
+
+const void *lev_moe_scores_few() { return reinterpret_cast<const void *>(&moe_scores_few_kernel); }
+
+namespace {
+
+template <int NW>
+bool is_gate_up_of(const void *f) {
+    return f == reinterpret_cast<const void *>(&moe_gate_up_mfma<NW, true, 2>) || f == reinterpret_cast<const void *>(&moe_gate_up_mfma<NW, true, 4>) ||
+           f == reinterpret_cast<const void *>(&moe_gate_up_mfma<NW, false, 2>) || f == reinterpret_cast<const void *>(&moe_gate_up_mfma<NW, false, 4>);
+}
+bool is_gate_up(const void *f) { return is_gate_up_of<8>(f) || is_gate_up_of<12>(f) || is_gate_up_of<16>(f); }
+bool is_down(const void *f) {
+    return f == reinterpret_cast<const void *>(&moe_down_mfma<1>) || f == reinterpret_cast<const void *>(&moe_down_mfma<2>) ||
+           f == reinterpret_cast<const void *>(&moe_down_mfma<3>) || f == reinterpret_cast<const void *>(&moe_down_mfma<4>) ||
+           f == reinterpret_cast<const void *>(&moe_down_kernel<16>) || f == reinterpret_cast<const void *>(&moe_down_kernel<32>) ||
+           f == reinterpret_cast<const void *>(&moe_down_kernel<64>);
+}
+
+}  // namespace
+
+bool lev_moe_expert_node(const lev_ctx *ctx, const void *func, void **args, lev_footprint *touches) {
+    const bool gate_up = is_gate_up(func);
+    if (!gate_up && !is_down(func)) return false;
+    const moe_args &a = *static_cast<const moe_args *>(args[0]);
+    const size_t gu = (size_t)a.inter * (a.hidden / 32u) * 18u, dn = (size_t)a.hidden * (a.inter / 32u) * 18u, k = a.top_k;
+    auto ptr = [&](int i) { return *static_cast<const float *const *>(args[i]); };
+    lev_footprint &t = *touches;
+    t = lev_footprint{};
+    if (gate_up) {   // a, x, ids, scores, expert_scale, ids_out, weights_out, act, flag, rows_per_block
+        t.reads[0] = lev_span(ptr(1), 4u * (size_t)a.hidden);
+        t.reads[1] = lev_span(a.base + a.gate_off, a.gate_stride * (a.experts - 1u) + gu);
+        t.reads[2] = lev_span(a.base + a.up_off, a.up_stride * (a.experts - 1u) + gu);
+        t.reads[3] = lev_span(ptr(3), 4u * (size_t)a.experts);
+        t.reads[4] = lev_span(ptr(4), 4u * (size_t)a.experts);
+        t.writes[0] = lev_span(ptr(5), 4u * k);
+        t.writes[1] = lev_span(ptr(6), 4u * k);
+        t.writes[2] = lev_span(ptr(7), 4u * k * a.inter);
+    } else {         // a, act, ids, weights, y, flag, tile or steps
+        t.reads[0] = lev_span(ptr(1), 4u * k * a.inter);
+        t.reads[1] = lev_span(ptr(2), 4u * k);
+        t.reads[2] = lev_span(ptr(3), 4u * k);
+        t.reads[3] = lev_span(a.base + a.down_off, a.down_stride * (a.experts - 1u) + dn);
+        t.writes[0] = lev_span(ptr(4), 4u * (size_t)a.hidden);
+    }
+    t.writes[3] = lev_span(ctx->d_flag, 4u);
+    return true;
 }

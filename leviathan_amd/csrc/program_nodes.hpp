@@ -1,0 +1,55 @@
+// What the fusions of recorded programs (lev_api.hip) know of the kernels of other files: which function of a kernel node is
+// which, the memory that it touches, and the launches that stand for two of them.
+#pragma once
+
+#include "lev_common.hpp"
+
+struct lev_span {
+    uintptr_t at = 0;
+    size_t bytes = 0;
+    lev_span() = default;
+    template <typename T>
+    lev_span(const T *p, size_t n) : at(reinterpret_cast<uintptr_t>(p)), bytes(p ? n : 0u) {}
+    bool meets(const lev_span &o) const { return at < o.at + o.bytes && o.at < at + bytes; }
+};
+
+// The memory of one kernel.
+struct lev_footprint {
+    lev_span reads[8], writes[4];
+    // neither writes what the other touches: they may change places or run side by side
+    bool apart(const lev_footprint &o) const {
+        for (const lev_span &w : writes) {
+            for (const lev_span &r : o.reads)
+                if (w.meets(r)) return false;
+            for (const lev_span &v : o.writes)
+                if (w.meets(v)) return false;
+        }
+        for (const lev_span &w : o.writes)
+            for (const lev_span &r : reads)
+                if (w.meets(r)) return false;
+        return true;
+    }
+};
+
+struct lev_gemv_args {
+    const uint8_t *w;
+    const float *x;
+    float *y;
+    uint32_t in_dim, rows, wpr, slots;
+    uint64_t slot_of_wave, pos_of_wave;
+};
+struct lev_scores_args {
+    const float *wr, *x;
+    float *scores;
+    uint32_t hidden, experts;
+};
+struct lev_fused_launch {
+    void *func;
+    uint32_t blocks, threads, lds;
+};
+
+const void *lev_q4_0_gemv_one_round();     // q4_0_mfma_gemv<1, true, false>: the arguments of lev_gemv_args in order
+const void *lev_moe_scores_few();          // moe_scores_few_kernel: those of lev_scores_args
+lev_fused_launch lev_q4_0_gemv_and_scores(uint32_t gemv_blocks, uint32_t gemv_threads, uint32_t experts);
+// Whether `func` is one of the MoE layer's kernels at one token (gate/up, down), and what it touches.
+bool lev_moe_expert_node(const lev_ctx *ctx, const void *func, void **args, lev_footprint *touches);

@@ -7,6 +7,7 @@
 // 256-value column task of gate row group i and of up row group i, keeps the operands in registers and
 // meets the others in LDS; in front of it every workgroup normalises x for itself (a wave its own 256 values,
 // the sum of squares crosses the waves once), with its weights already on their way.
+#include "program_nodes.hpp"
 #include "q4_0_mfma.hpp"
 
 hipError_t lev_q4_0_gemv_launch(lev_ctx *ctx, const uint8_t *w, const float *x, float *y, uint32_t in_dim, uint32_t rows);
@@ -126,22 +127,14 @@ q4_0_ffn_gate_up(ffn_args a) {
     }
 }
 
-struct span {
-    uintptr_t at;
-    size_t bytes;
-    template <typename T>
-    span(const T *p, size_t n) : at(reinterpret_cast<uintptr_t>(p)), bytes(p ? n : 0u) {}
-    bool meets(const span &o) const { return at < o.at + o.bytes && o.at < at + bytes; }
-};
-
 // Whether the first three stages may run at the same time: every workgroup reads all of x, the norm and its own rows
 // of the weights while others already write h, gu and act, which the operators one by one only do when all readers are
 // through.  act may be one of the halves of gu, whose value a lane replaces with its own.
 bool ffn_apart(const ffn_args &a, size_t gate_bytes, size_t up_bytes) {
     const size_t nh = (size_t)a.hidden * 4u, ni = (size_t)a.inter * 4u;
-    const span in[] = {{a.x, nh}, {a.gain, nh}, {a.gate, gate_bytes}, {a.up, up_bytes}};
-    const span h(a.h, nh), gu(a.gu, 2u * ni), act(a.act, ni);
-    for (const span &i : in)
+    const lev_span in[] = {{a.x, nh}, {a.gain, nh}, {a.gate, gate_bytes}, {a.up, up_bytes}};
+    const lev_span h(a.h, nh), gu(a.gu, 2u * ni), act(a.act, ni);
+    for (const lev_span &i : in)
         if (i.meets(h) || i.meets(gu) || i.meets(act)) return false;
     return !h.meets(gu) && !h.meets(act) && (!act.meets(gu) || a.act == a.gu || a.act == a.gu + a.inter);
 }

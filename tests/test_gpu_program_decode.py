@@ -1,0 +1,86 @@
+"""GPU: a recorded decode step, the shared expert's FFN, the MoE layer on its normalised residual and the norm and residuals
+behind both, gives the bits of the operators called one by one on every replay, and replays as the launches that it is meant
+to: the scores of the router go into the launch of the shared expert's down projection, the shared expert's norm into the
+layer's, unless what the one writes the other touches."""
+import pytest
+import torch
+
+from tests.test_gpu_program_norm_adds import launches_of
+
+pytestmark = pytest.mark.gpu
+
+
+def q4_0(rows, n, g):
+    nb = rows * n // 32
+    w = torch.randint(0, 256, (nb, 18), dtype=torch.uint8, device="cuda", generator=g)
+    w[:, :2] = (torch.randn(nb, 1, device="cuda", generator=g) / (4.6 * n ** 0.5)).abs().half().view(torch.uint8)
+    return w.reshape(-1)
+
+
+@pytest.mark.parametrize("case,launches", [("plain", 5), ("two layers", 10), ("scores of the sum", 7), ("sum not added", 6), ("added twice", 6),
+                                           ("part of the sum", 8), ("result is the sum", 6), ("gain is the sum", 6)])
+@pytest.mark.parametrize("hidden,inter,shared,experts,top_k", [
+    (2816, 704, 2112, 128, 8), (1024, 256, 512, 32, 2), (4096, 1536, 4096, 256, 8), (1152, 320, 1344, 60, 4), (2048, 768, 1024, 128, 8), (1280, 576, 640, 256, 8)])
+def test_recorded_decode_step(hidden, inter, shared, experts, top_k, case, launches):
+    from leviathan_amd import ops
+    ctx = ops.Context(0, own_stream=True)
+    g = torch.Generator(device="cuda").manual_seed(hidden + experts)
+    normal = lambda *s: torch.randn(s, device="cuda", generator=g)
+    gu = inter * (hidden // 32) * 18 * experts
+    layers = []
+    for _ in range(2 if case == "two layers" else 1):
+        pool = torch.cat([q4_0(experts * inter, hidden, g), q4_0(experts * inter, hidden, g), q4_0(experts * hidden, inter, g)])
+        layers.append(dict(
+            pools=ops.Context.moe_pools(pool, hidden, inter, experts, 0, gu, 2 * gu), pool=pool, router=0.02 * normal(experts, hidden),
+            norm=1 + 0.1 * normal(hidden), gate=q4_0(shared, hidden, g), up=q4_0(shared, hidden, g), down=q4_0(hidden, shared, g),
+            post=1 + 0.1 * normal(hidden), post2=1 + 0.1 * normal(hidden),
+            bufs=tuple(torch.empty(n, device="cuda") for n in (hidden, 2 * shared, shared, hidden)), y=torch.empty(1, hidden, device="cuda"),
+            ids=torch.empty((1, top_k), dtype=torch.int32, device="cuda"), weights=torch.empty(1, top_k, device="cuda"),
+            out=torch.empty(hidden, device="cuda")))
+    x0 = normal(hidden)
+
+    def step():
+        x = x0
+        for m in layers:
+            h, s = ctx.shared_expert_ffn(x, m["norm"], m["gate"], m["up"], m["down"], m["post"], hidden, shared, bufs=m["bufs"])
+            ctx.moe_layer_q4_0(m["pools"], m["router"], (s if case == "scores of the sum" else h)[None], top_k, 1, y=m["y"], ids=m["ids"],
+                               weights=m["weights"])
+            out = s if case == "result is the sum" else m["out"]
+            ctx.rmsnorm(m["y"], hidden, 1, weight=s if case == "gain is the sum" else m["post2"], y=out)
+            if case == "part of the sum":
+                ctx.axpy(s[4:], out, 1.0, hidden - 4)
+            elif case not in ("sum not added", "result is the sum"):
+                ctx.axpy(s, out, 0.5 if case == "added twice" else 1.0, hidden)
+            if case == "added twice":
+                ctx.axpy(s, out, 0.25, hidden)
+            ctx.axpy(x, out, 1.0, hidden)
+            x = m["out"]
+
+    def results():
+        ctx.sync()
+        return [t.clone() for m in layers for t in (*m["bufs"], m["y"], m["ids"], m["weights"], m["out"])]
+
+    def wipe():
+        for m in layers:
+            for t in (*m["bufs"], m["y"], m["weights"], m["out"]):
+                t.fill_(float("nan"))
+            m["ids"].fill_(-1)
+        torch.cuda.synchronize()
+
+    wipe()
+    step()
+    want = results()
+    torch.cuda.synchronize()
+    ctx.program_begin()
+    step()
+    prog = ctx.program_end()
+    for _ in range(3):
+        wipe()
+        prog.run()
+        for a, b in zip(results(), want):
+            assert torch.equal(a.view(torch.int32), b.view(torch.int32))
+    # (the scores join the kernel of the matrix cores, which does not take every width of the down projection)
+    alone = 0 if shared % 256 == 0 or shared > 1280 or case == "scores of the sum" else len(layers)
+    assert launches_of(prog) == launches + alone
+    prog.destroy()
+    ctx.close()
