@@ -3,7 +3,7 @@
 //
 // Called operator by operator it is six launches of which four are the launch floor and little else: at
 // 2816 / 2112 18.7 us recorded, 29 us enqueued one by one.  Here three: everything up to act, the down GEMV, the
-// norm behind it (11.7 us recorded, 14 enqueued).  The first kernel has the shape of the MoE gate/up kernel: a wave owns one
+// norm behind it (9.3 us recorded, 9.5 enqueued; 9.5 and 9.65 with the only group's weights requested a second time).  The first kernel has the shape of the MoE gate/up kernel: a wave owns one
 // 256-value column task of gate row group i and of up row group i, keeps the operands in registers and
 // meets the others in LDS; in front of it every workgroup normalises x for itself (a wave its own 256 values,
 // the sum of squares crosses the waves once), with its weights already on their way.
@@ -26,8 +26,9 @@ struct ffn_args {
 constexpr uint32_t kFfnPart = 2u * 16u * 16u * 4u, kFfnUp = kFfnPart / 2u;
 constexpr size_t ffn_lds(int nw) { return 2u * kFfnPart + 64u + (size_t)nw * (kQ4mTaskArea + kQ4mZeroBytes); }
 
-// NW waves, one per column task (at most 16).  grid (row chunks).
-template <int NW>
+// NW waves, one per column task (at most 16).  SINGLE: a workgroup has one group of 16 rows, nothing to prefetch.
+// grid (row chunks).
+template <int NW, bool SINGLE>
 __global__ void __launch_bounds__(NW * LEV_WAVE, NW / 4)
 q4_0_ffn_gate_up(ffn_args a) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
@@ -88,7 +89,7 @@ q4_0_ffn_gate_up(ffn_args a) {
     while (true) {
         uint32_t Gb[9], Ub[9], W[9];
         const uint32_t next = i0 + 16u;
-        issue(next < i_end ? next : i0, Gb, Ub);                  // unconditional (clamped)
+        if (!SINGLE) issue(next < i_end ? next : i0, Gb, Ub);     // unconditional (clamped)
         q4m_turn_task(Ga, W);
         const float vg = lev_row_sum_f32(q4m_task_dot(W, op));
         q4m_turn_task(Ua, W);
@@ -115,7 +116,7 @@ q4_0_ffn_gate_up(ffn_args a) {
                 a.act[row] = lev_gelu_up_value(g, u);
             }
         }
-        if (next >= i_end) break;
+        if (SINGLE || next >= i_end) break;
         i0 = next;
         pw ^= kFfnPart;
         pr ^= kFfnPart;
@@ -171,10 +172,12 @@ extern "C" int lev_hip_shared_expert_ffn_q4_0(lev_ctx *ctx, const float *d_x, co
         const uint32_t rows = per == 1u ? (inter + cus - 1u) / cus : (inter + 16u * cus - 1u) / (16u * cus) * 16u;
         a.rows_per_block = rows;
         const dim3 grid((inter + rows - 1u) / rows);
-#define LEV_FFN(NW) hipLaunchKernelGGL((q4_0_ffn_gate_up<NW>), grid, dim3(NW * LEV_WAVE), ffn_lds(NW), ctx->stream, a)
-        if (hidden <= 2048u) LEV_FFN(8);
-        else if (hidden <= 3072u) LEV_FFN(12);
-        else LEV_FFN(16);
+#define LEV_FFN(NW)                                                                                                    \
+    if (rows <= 16u) hipLaunchKernelGGL((q4_0_ffn_gate_up<NW, true>), grid, dim3(NW * LEV_WAVE), ffn_lds(NW), ctx->stream, a); \
+    else hipLaunchKernelGGL((q4_0_ffn_gate_up<NW, false>), grid, dim3(NW * LEV_WAVE), ffn_lds(NW), ctx->stream, a)
+        if (hidden <= 2048u) { LEV_FFN(8); }
+        else if (hidden <= 3072u) { LEV_FFN(12); }
+        else { LEV_FFN(16); }
 #undef LEV_FFN
         if (ctx->recording) ctx->folded_nodes += 3u;   // norm, gate, up and geluUp are one node
         st = lev_hip_check(ctx, hipGetLastError(), "shared_expert_ffn gate/up launch");
