@@ -568,9 +568,9 @@ namespace {
 // cannot see through stays as it was recorded.  Recorded decode step of four layers at 2816: 135 us with
 // the operators at the end of a layer apart, 123 with this; seven kernels a layer.
 // Two more rules look through the shared expert and the MoE layer behind it, whose kernels otherwise run one after the other
-// although only the sum at the end needs both: the router's scores join the shared expert's down projection (move_scores) and
-// its norm the layer's (pair_norms).  Five kernels a layer: 115.5 us and 100.0 for the same four layers (weights of two such
-// states in turn), 1.05 to 1.21 times as fast over ten drawn ones.
+// although they share only the normalised input and the sum at the end (weave_shared_expert, pair_norms).  Four kernels a
+// layer, 115 us and 92 for the same four layers (weights of two such states in turn); five where the launches of the middle
+// do not fit the chip together, 100 us here.  1.04 to 1.42 times as fast over 26 drawn ones.
 struct node_view {
     const void *func;
     void **args;
@@ -594,6 +594,29 @@ bool only_next(hipGraphNode_t node, hipGraphNode_t *next) {
     if (hipGraphNodeGetDependentNodes(node, nullptr, &n) != hipSuccess || n != 1) return false;
     if (hipGraphNodeGetDependentNodes(node, next, &n) != hipSuccess || n != 1) return false;
     return hipGraphNodeGetDependencies(*next, nullptr, &m) == hipSuccess && m == 1;
+}
+
+// Another launch in the place of a node's own.  (Not a new node for the old one: the runtime walks the nodes in the order in
+// which they were added, and with the first of a graph replaced by a later one it deals one chain over two queues: the four
+// layers took 130 us instead of 93.)  `args` must not lie in the node.
+hipError_t become(hipGraphNode_t node, void *func, uint32_t blocks, uint32_t threads, uint32_t lds, void **args, uint32_t blocks_y = 1u) {
+    hipKernelNodeParams kp{};
+    kp.func = func;
+    kp.gridDim = dim3(blocks, blocks_y);
+    kp.blockDim = dim3(threads);
+    kp.sharedMemBytes = lds;
+    kp.kernelParams = args;
+    return hipGraphKernelNodeSetParams(node, &kp);
+}
+// What waits for `last` waits for `one` as well.
+hipError_t hand_on(hipGraph_t graph, hipGraphNode_t last, hipGraphNode_t one) {
+    size_t n = 0;
+    hipError_t e = hipGraphNodeGetDependentNodes(last, nullptr, &n);
+    if (e != hipSuccess || n == 0) return e;
+    std::vector<hipGraphNode_t> behind(n);
+    if ((e = hipGraphNodeGetDependentNodes(last, behind.data(), &n)) != hipSuccess) return e;
+    const std::vector<hipGraphNode_t> from(n, one);
+    return hipGraphAddDependencies(graph, from.data(), behind.data(), n);
 }
 
 hipError_t fuse_norm_chains(hipGraph_t graph) {
@@ -641,62 +664,14 @@ hipError_t fuse_norm_chains(hipGraph_t graph) {
             last = next;
         }
         if (chain.empty()) continue;
-        size_t nbefore = 0, nbehind = 0;
-        if (hipGraphNodeGetDependencies(first, nullptr, &nbefore) != hipSuccess ||
-            hipGraphNodeGetDependentNodes(last, nullptr, &nbehind) != hipSuccess)
-            continue;
-        std::vector<hipGraphNode_t> before(nbefore), behind(nbehind);
-        if ((nbefore && hipGraphNodeGetDependencies(first, before.data(), &nbefore) != hipSuccess) ||
-            (nbehind && hipGraphNodeGetDependentNodes(last, behind.data(), &nbehind) != hipSuccess))
-            continue;
         void *args[6] = {&x, &y, &w, &n, &eps, &adds};
-        hipKernelNodeParams kp{};
-        kp.func = fused[which];
-        kp.gridDim = norm.params.gridDim;
-        kp.blockDim = norm.params.blockDim;
-        kp.sharedMemBytes = 0;
-        kp.kernelParams = args;
-        hipGraphNode_t one;
-        hipError_t e = hipGraphAddKernelNode(&one, graph, before.data(), nbefore, &kp);
-        if (e != hipSuccess) return e;
-        if (nbehind) {
-            const std::vector<hipGraphNode_t> from(nbehind, one);
-            if ((e = hipGraphAddDependencies(graph, from.data(), behind.data(), nbehind)) != hipSuccess) return e;
-        }
+        hipError_t e = become(first, fused[which], 1u, norm.params.blockDim.x, 0u, args);
+        if (e == hipSuccess) e = hand_on(graph, last, first);
         for (hipGraphNode_t gone : chain)
-            if ((e = hipGraphDestroyNode(gone)) != hipSuccess) return e;
-        if ((e = hipGraphDestroyNode(first)) != hipSuccess) return e;
+            if (e == hipSuccess) e = hipGraphDestroyNode(gone);
+        if (e != hipSuccess) return e;
     }
     return hipSuccess;
-}
-
-// A node in the place of `first` .. `last`, which are not destroyed here.
-hipError_t put_node(hipGraph_t graph, hipGraphNode_t first, const hipKernelNodeParams &kp, hipGraphNode_t *one) {
-    size_t n = 0;
-    hipError_t e = hipGraphNodeGetDependencies(first, nullptr, &n);
-    if (e != hipSuccess) return e;
-    std::vector<hipGraphNode_t> before(n);
-    if (n && (e = hipGraphNodeGetDependencies(first, before.data(), &n)) != hipSuccess) return e;
-    return hipGraphAddKernelNode(one, graph, before.data(), n, &kp);
-}
-// What waits for `last` waits for `one` as well.
-hipError_t hand_on(hipGraph_t graph, hipGraphNode_t last, hipGraphNode_t one) {
-    size_t n = 0;
-    hipError_t e = hipGraphNodeGetDependentNodes(last, nullptr, &n);
-    if (e != hipSuccess || n == 0) return e;
-    std::vector<hipGraphNode_t> behind(n);
-    if ((e = hipGraphNodeGetDependentNodes(last, behind.data(), &n)) != hipSuccess) return e;
-    const std::vector<hipGraphNode_t> from(n, one);
-    return hipGraphAddDependencies(graph, from.data(), behind.data(), n);
-}
-hipKernelNodeParams params_of(void *func, uint32_t blocks, uint32_t threads, uint32_t lds, void **args) {
-    hipKernelNodeParams kp{};
-    kp.func = func;
-    kp.gridDim = dim3(blocks);
-    kp.blockDim = dim3(threads);
-    kp.sharedMemBytes = lds;
-    kp.kernelParams = args;
-    return kp;
 }
 
 const void *norm_of(int k) {
@@ -727,35 +702,64 @@ lev_footprint scores_touches(const node_view &v) {   // of one token
     return t;
 }
 
-// A GEMV of one round, a norm and the router scores of one token behind it: the scores go into the GEMV's launch where they
-// depend on neither (the shared expert's down projection and norm, then the MoE layer on the same normalised residual).
-hipError_t move_scores(hipGraph_t graph, const std::vector<hipGraphNode_t> &nodes) {
-    for (hipGraphNode_t first : nodes) {
-        node_view g, n, r;
-        hipGraphNode_t norm, scores;
-        if (!kernel_node(first, &g) || g.func != lev_q4_0_gemv_one_round() || !only_next(first, &norm) || !kernel_node(norm, &n) ||
-            norm_kind(n) < 0 || !only_next(norm, &scores) || !kernel_node(scores, &r) || r.func != lev_moe_scores_few() ||
-            r.params.gridDim.y != 1u)
+lev_gemv_args gemv_args_of(const node_view &v) {
+    return lev_gemv_args{arg_of<const uint8_t *>(v, 0), arg_of<const float *>(v, 1), arg_of<float *>(v, 2), arg_of<uint32_t>(v, 3),
+                         arg_of<uint32_t>(v, 4), arg_of<uint32_t>(v, 5), arg_of<uint32_t>(v, 6), arg_of<uint64_t>(v, 7),
+                         arg_of<uint64_t>(v, 8)};
+}
+lev_footprint gemv_touches(const lev_gemv_args &g) {
+    lev_footprint t;
+    t.reads[0] = lev_span(g.w, (size_t)g.rows * (g.in_dim / 32u) * 18u);
+    t.reads[1] = lev_span(g.x, 4u * (size_t)g.in_dim);
+    t.writes[0] = lev_span(g.y, 4u * (size_t)g.rows);
+    return t;
+}
+
+// The shared expert's FFN (gate/up, down, norm) and the scores and gate/up kernel of a MoE layer on the same h behind it, whose
+// kernels only share that h: the scores join the FFN's gate/up kernel, which normalises it, and the down projection the
+// layer's gate/up.  Where the layer's gate/up takes no GEMV along (more than one group of rows a workgroup, a down projection
+// of more columns than it has waves, too many workgroups) the scores join the down projection; where they are not those of h, too.
+hipError_t weave_shared_expert(hipGraph_t graph, const std::vector<hipGraphNode_t> &heads, const lev_ctx *ctx) {
+    for (hipGraphNode_t first : heads) {   // down projections
+        node_view g, n, r, u, f;
+        hipGraphNode_t norm, scores, gate_up, ffn, next;
+        if (!kernel_node(first, &g) || !only_next(first, &norm) || !kernel_node(norm, &n) || norm_kind(n) < 0 || !only_next(norm, &scores) ||
+            !kernel_node(scores, &r) || r.func != lev_moe_scores_few() || r.params.gridDim.y != 1u)
             continue;
-        lev_gemv_args ga{arg_of<const uint8_t *>(g, 0), arg_of<const float *>(g, 1), arg_of<float *>(g, 2), arg_of<uint32_t>(g, 3),
-                         arg_of<uint32_t>(g, 4), arg_of<uint32_t>(g, 5), arg_of<uint32_t>(g, 6), arg_of<uint64_t>(g, 7),
-                         arg_of<uint64_t>(g, 8)};
+        lev_gemv_args ga = gemv_args_of(g);
         lev_scores_args sa{arg_of<const float *>(r, 0), arg_of<const float *>(r, 1), arg_of<float *>(r, 2), arg_of<uint32_t>(r, 3),
                            arg_of<uint32_t>(r, 4)};
-        const lev_footprint st = scores_touches(r);
-        lev_footprint gt;
-        gt.reads[0] = lev_span(ga.w, (size_t)ga.rows * (ga.in_dim / 32u) * 18u);
-        gt.reads[1] = lev_span(ga.x, 4u * (size_t)ga.in_dim);
-        gt.writes[0] = lev_span(ga.y, 4u * (size_t)ga.rows);
-        if (!st.apart(gt) || !st.apart(norm_touches(n))) continue;
-        uint32_t blocks = g.params.gridDim.x;
-        const lev_fused_launch f = lev_q4_0_gemv_and_scores(blocks, g.params.blockDim.x, sa.experts);
-        void *args[3] = {&ga, &sa, &blocks};
-        hipGraphNode_t one;
-        hipError_t e = put_node(graph, first, params_of(f.func, f.blocks, f.threads, f.lds, args), &one);
-        if (e == hipSuccess) e = hipGraphAddDependencies(graph, &one, &norm, 1);
-        if (e == hipSuccess) e = hand_on(graph, scores, norm);
-        if (e == hipSuccess) e = hipGraphDestroyNode(first);
+        const lev_footprint gt = gemv_touches(ga), nt = norm_touches(n), st = scores_touches(r);
+        if (!st.apart(gt) || !st.apart(nt)) continue;
+        size_t ndeps = 0;
+        lev_ffn_node fn;
+        lev_footprint ut, wt = st;
+        wt.reads[1] = lev_span();          // (h, which the workgroups of the scores form for themselves)
+        lev_gate_up_gemv gu;
+        lev_gemv_args gg = ga;
+        hipError_t e;
+        if (hipGraphNodeGetDependencies(first, nullptr, &ndeps) == hipSuccess && ndeps == 1u &&
+            hipGraphNodeGetDependencies(first, &ffn, &ndeps) == hipSuccess && only_next(ffn, &next) && kernel_node(ffn, &f) &&
+            lev_ffn_gate_up_node(f.func, f.args, &fn) && sa.x == fn.args.h && sa.hidden == fn.args.hidden && wt.apart(fn.touches) &&
+            only_next(scores, &gate_up) && kernel_node(gate_up, &u) && u.params.gridDim.z == 1u &&
+            lev_moe_expert_node(ctx, u.func, u.args, &ut) && ut.apart(gt) && ut.apart(nt) &&
+            lev_moe_gate_up_and_gemv(ctx, u.func, u.args, &gg, &gu)) {
+            const uint32_t each = fn.with_scores.threads / 256u;
+            uint32_t blocks = f.params.gridDim.x;
+            void *with_scores[3] = {&fn.args, &sa, &blocks}, *with_gemv[13];
+            for (int k = 0; k < 9; ++k) with_gemv[k] = u.args[k];
+            with_gemv[9] = &gu.rows_per_block, with_gemv[10] = &gg, with_gemv[11] = &gu.extra, with_gemv[12] = &gu.gemv_blocks;
+            e = become(ffn, fn.with_scores.func, blocks + (sa.experts + each - 1u) / each, fn.with_scores.threads, fn.with_scores.lds, with_scores);
+            if (e == hipSuccess) e = become(first, gu.launch.func, gu.launch.blocks, gu.launch.threads, gu.launch.lds, with_gemv, gu.top_k);
+            if (e == hipSuccess) e = hand_on(graph, gate_up, norm);
+            if (e == hipSuccess) e = hipGraphDestroyNode(gate_up);
+        } else {
+            uint32_t blocks = g.params.gridDim.x;
+            const lev_fused_launch l = lev_q4_0_gemv_and_scores(blocks, g.params.blockDim.x, sa.experts);
+            void *args[3] = {&ga, &sa, &blocks};
+            e = become(first, l.func, l.blocks, l.threads, l.lds, args);
+            if (e == hipSuccess) e = hand_on(graph, scores, norm);
+        }
         if (e == hipSuccess) e = hipGraphDestroyNode(scores);
         if (e != hipSuccess) return e;
     }
@@ -802,10 +806,8 @@ hipError_t pair_norms(hipGraph_t graph, const std::vector<hipGraphNode_t> &nodes
         uint32_t len = arg_of<uint32_t>(s, 3);
         float eps = arg_of<float>(s, 4);
         void *args[7] = {&p, &y, &out, &wy, &len, &eps, &adds};
-        hipGraphNode_t one;
         size_t nbefore = 0;
-        hipError_t e = put_node(graph, last, params_of(pair_kernel[kind], 1u, s.params.blockDim.x, 0u, args), &one);
-        if (e == hipSuccess) e = hand_on(graph, last, one);
+        hipError_t e = become(last, pair_kernel[kind], 1u, s.params.blockDim.x, 0u, args);
         if (e == hipSuccess) e = hipGraphNodeGetDependencies(first, nullptr, &nbefore);
         if (e == hipSuccess && nbefore) {
             std::vector<hipGraphNode_t> before(nbefore);
@@ -814,7 +816,6 @@ hipError_t pair_norms(hipGraph_t graph, const std::vector<hipGraphNode_t> &nodes
             if (e == hipSuccess) e = hipGraphAddDependencies(graph, before.data(), to.data(), nbefore);
         }
         if (e == hipSuccess) e = hipGraphDestroyNode(first);
-        if (e == hipSuccess) e = hipGraphDestroyNode(last);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
@@ -833,7 +834,7 @@ hipError_t fuse_nodes(hipGraph_t graph, const lev_ctx *ctx) {
             node_view v;
             if (kernel_node(node, &v) && (rule == 0 ? v.func == lev_q4_0_gemv_one_round() : norm_kind(v) >= 0)) heads.push_back(node);
         }
-        e = rule == 0 ? move_scores(graph, heads) : pair_norms(graph, heads, ctx);
+        e = rule == 0 ? weave_shared_expert(graph, heads, ctx) : pair_norms(graph, heads, ctx);
     }
     return e;
 }

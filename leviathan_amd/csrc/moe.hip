@@ -21,7 +21,7 @@
 #include "program_nodes.hpp"
 #include "moe_grouped.hpp"
 #include "moe_split.hpp"
-#include "q4_0_mfma.hpp"
+#include "q4_0_mfma_gemv.hpp"
 
 namespace {
 
@@ -975,15 +975,13 @@ __host__ __device__ constexpr size_t mm_areas_bytes(uint32_t waves, uint32_t tpw
 // weights.  Otherwise the ids are read from `ids`.
 // LDS: part [2] | expert word | task areas | router area (ROUTE > 0)
 template <int NW, bool SINGLE, int ROUTE>
-__global__ void __launch_bounds__(NW * LEV_WAVE, SINGLE || NW < 16 ? NW / 2 : NW / 4)
-moe_gate_up_mfma(moe_args a, const float *__restrict__ x, const int32_t *ids, const float *__restrict__ scores,
-                 const float *__restrict__ expert_scale, int32_t *ids_out, float *weights_out,
-                 float *__restrict__ act, int *__restrict__ flag, uint32_t rows_per_block) {
-    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+__device__ __forceinline__ void gate_up_mfma(const moe_args &a, const float *__restrict__ x, const int32_t *ids,
+                                             const float *__restrict__ scores, const float *__restrict__ expert_scale,
+                                             int32_t *ids_out, float *weights_out, float *__restrict__ act, int *__restrict__ flag,
+                                             uint32_t rows_per_block, uint32_t chunk, uint32_t slot, uint32_t t, uint8_t *smem) {
     constexpr uint32_t kPart = gum_part_bytes(NW), kUp = kPart / 2u;
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
-    const uint32_t slot = blockIdx.y, t = blockIdx.z;
     const uint32_t npairs = a.hidden >> 6, ntask = (npairs + 3u) >> 2;
     const bool active = wave < ntask;
     const uint32_t T = active ? wave : ntask - 1u;
@@ -1004,7 +1002,7 @@ moe_gate_up_mfma(moe_args a, const float *__restrict__ x, const int32_t *ids, co
     void *rl = smem + 2u * kPart + 16u + mm_areas_bytes(NW, 1u);
     uint32_t e;
     bool ok = true;
-    const bool publisher = ROUTE > 0 && blockIdx.x == 0 && slot == 0;
+    const bool publisher = ROUTE > 0 && chunk == 0u && slot == 0u;
     if constexpr (ROUTE > 0) {
         // (all eight waves ranking a share of the keys each was measured as well: the layer takes 0.5 us
         // longer, the 16 waves of a CU then queue for its four vector pipelines)
@@ -1032,7 +1030,7 @@ moe_gate_up_mfma(moe_args a, const float *__restrict__ x, const int32_t *ids, co
     const uint64_t row_bytes = (uint64_t)(a.hidden >> 6) * 36u;
     const uint8_t *gbase = a.base + a.gate_off + e * a.gate_stride;
     const uint8_t *ubase = a.base + a.up_off + e * a.up_stride;
-    const uint32_t i_begin = blockIdx.x * rows_per_block;
+    const uint32_t i_begin = chunk * rows_per_block;
     const uint32_t i_end = min(i_begin + rows_per_block, a.inter);
     const uint32_t lrow = lane >> 2;                              // fetch order: lane = 4 * row + pair
     auto issue = [&](uint32_t i0, uint32_t (&Dg)[9], uint32_t (&Du)[9]) {
@@ -1122,6 +1120,39 @@ moe_gate_up_mfma(moe_args a, const float *__restrict__ x, const int32_t *ids, co
         if (next >= i_end) break;
         i0 = next;
     }
+}
+
+template <int NW, bool SINGLE, int ROUTE>
+__global__ void __launch_bounds__(NW * LEV_WAVE, SINGLE || NW < 16 ? NW / 2 : NW / 4)
+moe_gate_up_mfma(moe_args a, const float *__restrict__ x, const int32_t *ids, const float *__restrict__ scores,
+                 const float *__restrict__ expert_scale, int32_t *ids_out, float *weights_out,
+                 float *__restrict__ act, int *__restrict__ flag, uint32_t rows_per_block) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    gate_up_mfma<NW, SINGLE, ROUTE>(a, x, ids, scores, expert_scale, ids_out, weights_out, act, flag, rows_per_block, blockIdx.x,
+                                    blockIdx.y, blockIdx.z, smem);
+}
+
+// The same at one token beside a GEMV that does not depend on it (recorded programs: the shared expert's down projection,
+// which alone on the chip is the launch and little else).  grid (extra + chunks, top_k): the first `extra` workgroups of a
+// slot are the GEMV's, gemv_blocks in all.  Two workgroups of 12 or 16 waves a CU, four of 8: 80 and 64 registers (the latter
+// without the pins of q4m_gemv).
+template <int NW, int ROUTE>
+__global__ void __launch_bounds__(NW * LEV_WAVE, NW / 2)
+moe_gate_up_and_gemv(moe_args a, const float *__restrict__ x, const int32_t *ids, const float *__restrict__ scores,
+                     const float *__restrict__ expert_scale, int32_t *ids_out, float *weights_out, float *__restrict__ act,
+                     int *__restrict__ flag, uint32_t rows_per_block, lev_gemv_args g, uint32_t extra, uint32_t gemv_blocks) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    if (blockIdx.x >= extra) {
+        gate_up_mfma<NW, true, ROUTE>(a, x, ids, scores, expert_scale, ids_out, weights_out, act, flag, rows_per_block,
+                                      blockIdx.x - extra, blockIdx.y, 0u, smem);
+        return;
+    }
+    const uint32_t block = blockIdx.y * extra + blockIdx.x;
+    if (block >= gemv_blocks) return;
+    if (gemv_blocks * g.slots * 16u >= g.rows)
+        q4m_gemv<1, true, false>(g.w, g.x, g.y, g.in_dim, g.rows, g.wpr, g.slots, g.slot_of_wave, g.pos_of_wave, block, gemv_blocks, smem);
+    else
+        q4m_gemv<1, false, false, NW == 12>(g.w, g.x, g.y, g.in_dim, g.rows, g.wpr, g.slots, g.slot_of_wave, g.pos_of_wave, block, gemv_blocks, smem);
 }
 
 // grid (row tiles of `tile` <= 16 rows, tokens), 8 waves.  Wave s takes slots s, s + 8, ...: the
@@ -1895,4 +1926,52 @@ bool lev_moe_expert_node(const lev_ctx *ctx, const void *func, void **args, lev_
     }
     t.writes[3] = lev_span(ctx->d_flag, 4u);
     return true;
+}
+
+namespace {
+constexpr uint32_t kGemvRounds = 2u;
+template <int NW, int ROUTE>
+bool gate_up_and_gemv(const void *func, const lev_ctx *ctx, const moe_args &a, uint32_t rows_per_block, lev_gemv_args &g,
+                      lev_gate_up_gemv *out) {
+    if (func != reinterpret_cast<const void *>(&moe_gate_up_mfma<NW, true, ROUTE>) || g.wpr > (uint32_t)NW) return false;
+    g.slots = NW / g.wpr;
+    uint64_t slot_of_wave, pos_of_wave;
+    lev_wave_tables(g.wpr, &slot_of_wave, &pos_of_wave);
+    g.slot_of_wave = slot_of_wave, g.pos_of_wave = pos_of_wave;
+    const uint32_t groups = (g.rows + 15u) / 16u;
+    // Everything on the chip at once: of the splits that fit, the one whose largest workgroup reads the least (rows of the
+    // gate/up, at most the 16 of a group, and rounds of the GEMV).  With one round alone the four layers of 2816 / 704 and
+    // 2112 take 98.4 us and not 92.0, of three none gains.  Past the chip by more than an eighth the launch does not pay: 3328 /
+    // 1344 and 2176, 712 workgroups for 512 places, 141.5 us and 137.9 with five kernels a layer; 2560 / 1280 and 1344, 560
+    // of them, 52.3 and 57.2.
+    const uint32_t room = (NW <= 8 ? 4u : 2u) * (uint32_t)ctx->num_cus;
+    uint64_t best = ~0ull;
+    for (uint32_t rounds = 1u; rounds <= kGemvRounds; ++rounds) {
+        const uint32_t blocks = (groups + g.slots * rounds - 1u) / (g.slots * rounds), extra = (blocks + a.top_k - 1u) / a.top_k;
+        uint32_t rows = rows_per_block;
+        while (rows < 16u && rows < a.inter && ((a.inter + rows - 1u) / rows + extra) * a.top_k > room) ++rows;
+        const uint32_t chunks = (a.inter + rows - 1u) / rows;
+        if ((chunks + extra) * a.top_k > room + room / 8u) continue;
+        const uint64_t over = (chunks + extra) * a.top_k > room ? 1ull << 40 : 0ull;
+        const uint64_t most = std::max<uint64_t>(2ull * rows * a.hidden, 16ull * g.slots * rounds * g.in_dim) + over;
+        if (most >= best) continue;
+        best = most;
+        out->rows_per_block = rows, out->extra = extra, out->gemv_blocks = blocks;
+        out->launch.blocks = extra + chunks;
+    }
+    if (best == ~0ull) return false;
+    const size_t lds = 2u * gum_part_bytes(NW) + 16u + mm_areas_bytes(NW, 1u) + router_lds_bytes(ROUTE) + 8u, gemv = q4m_gemv_lds(1u);
+    out->launch = lev_fused_launch{reinterpret_cast<void *>(&moe_gate_up_and_gemv<NW, ROUTE>), out->launch.blocks, NW * LEV_WAVE,
+                                   (uint32_t)(lds > gemv ? lds : gemv)};
+    out->top_k = a.top_k;
+    return true;
+}
+}  // namespace
+
+bool lev_moe_gate_up_and_gemv(const lev_ctx *ctx, const void *func, void **args, lev_gemv_args *g, lev_gate_up_gemv *out) {
+    const moe_args &a = *static_cast<const moe_args *>(args[0]);
+    const uint32_t rows = *static_cast<const uint32_t *>(args[9]);
+    return gate_up_and_gemv<8, 2>(func, ctx, a, rows, *g, out) || gate_up_and_gemv<8, 4>(func, ctx, a, rows, *g, out) ||
+           gate_up_and_gemv<12, 2>(func, ctx, a, rows, *g, out) || gate_up_and_gemv<12, 4>(func, ctx, a, rows, *g, out) ||
+           gate_up_and_gemv<16, 2>(func, ctx, a, rows, *g, out) || gate_up_and_gemv<16, 4>(func, ctx, a, rows, *g, out);
 }

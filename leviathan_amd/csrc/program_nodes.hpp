@@ -53,3 +53,27 @@ const void *lev_moe_scores_few();          // moe_scores_few_kernel: those of le
 lev_fused_launch lev_q4_0_gemv_and_scores(uint32_t gemv_blocks, uint32_t gemv_threads, uint32_t experts);
 // Whether `func` is one of the MoE layer's kernels at one token (gate/up, down), and what it touches.
 bool lev_moe_expert_node(const lev_ctx *ctx, const void *func, void **args, lev_footprint *touches);
+
+struct lev_ffn_args {
+    const uint8_t *gate, *up;
+    const float *x, *gain;
+    float *h, *gu, *act;
+    uint32_t hidden, inter, rows_per_block;
+    float eps;
+};
+// The first kernel of the shared expert's FFN: its arguments, what it touches, and the launch (without its number of
+// workgroups) that computes the router's scores of h as well: arguments lev_ffn_args, lev_scores_args, its own workgroups.
+struct lev_ffn_node {
+    lev_ffn_args args;
+    lev_footprint touches;
+    lev_fused_launch with_scores;
+};
+bool lev_ffn_gate_up_node(const void *func, void **args, lev_ffn_node *out);
+
+// The launch of the MoE layer's gate/up kernel of one token with a GEMV of one round beside it: `args` of the former with
+// rows_per_block, then *g (its slots are those of the launch), extra, gemv_blocks; grid (launch.blocks, top_k).
+struct lev_gate_up_gemv {
+    lev_fused_launch launch;
+    uint32_t rows_per_block, extra, gemv_blocks, top_k;
+};
+bool lev_moe_gate_up_and_gemv(const lev_ctx *ctx, const void *func, void **args, lev_gemv_args *g, lev_gate_up_gemv *out);

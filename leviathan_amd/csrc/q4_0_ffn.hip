@@ -7,6 +7,7 @@
 // 256-value column task of gate row group i and of up row group i, keeps the operands in registers and
 // meets the others in LDS; in front of it every workgroup normalises x for itself (a wave its own 256 values,
 // the sum of squares crosses the waves once), with its weights already on their way.
+#include "moe_scores_few.hpp"
 #include "program_nodes.hpp"
 #include "q4_0_mfma.hpp"
 
@@ -14,24 +15,33 @@ hipError_t lev_q4_0_gemv_launch(lev_ctx *ctx, const uint8_t *w, const float *x, 
 
 namespace {
 
-struct ffn_args {
-    const uint8_t *gate, *up;
-    const float *x, *gain;
-    float *h, *gu, *act;
-    uint32_t hidden, inter, rows_per_block;
-    float eps;
-};
-
 // part of a round: [gate, up][wave][row] f32, two of them
 constexpr uint32_t kFfnPart = 2u * 16u * 16u * 4u, kFfnUp = kFfnPart / 2u;
 constexpr size_t ffn_lds(int nw) { return 2u * kFfnPart + 64u + (size_t)nw * (kQ4mTaskArea + kQ4mZeroBytes); }
 
+// The wave's 256 values of x, normalised as lev_hip_rmsnorm does it: squares in f32 per wave, f64 across the waves.
+template <int NW>
+__device__ __forceinline__ void ffn_normalise(const lev_ffn_args &a, lev_f32x4 &v, const lev_f32x4 &gain, bool live, float *s_ss,
+                                              uint32_t wave, uint32_t lane) {
+    v = q4m_mask_activations(v, live);
+    float ss = 0.f;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) ss = fmaf(v[c], v[c], ss);
+    ss = lev_wave_sum_broadcast(ss);
+    if (lane == 0u) s_ss[wave] = ss;
+    lev_barrier_lds();
+    double tot = 0.0;
+    for (int k = 0; k < NW; ++k) tot += (double)s_ss[k];
+    const float inv = (float)lev_rsqrt_f64(tot / (double)a.hidden + (double)a.eps);
+    v = v * inv;
+    if (a.gain) v = v * gain;
+    if (!live) v = lev_f32x4{0.f, 0.f, 0.f, 0.f};                 // (an infinite inv made NaNs of the zeros past the end)
+}
+
 // NW waves, one per column task (at most 16).  SINGLE: a workgroup has one group of 16 rows, nothing to prefetch.
 // grid (row chunks).
 template <int NW, bool SINGLE>
-__global__ void __launch_bounds__(NW * LEV_WAVE, NW / 4)
-q4_0_ffn_gate_up(ffn_args a) {
-    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+__device__ __forceinline__ void ffn_gate_up(const lev_ffn_args &a, uint8_t *smem) {
     float *const s_ss = reinterpret_cast<float *>(smem + 2u * kFfnPart);
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
@@ -60,20 +70,7 @@ q4_0_ffn_gate_up(ffn_args a) {
     issue(i0, Ga, Ua);
     __builtin_amdgcn_sched_barrier(0);
 
-    // rmsnorm as lev_hip_rmsnorm forms it: squares in f32 per wave, f64 across the waves
-    v = q4m_mask_activations(v, live && active);
-    float ss = 0.f;
-#pragma unroll
-    for (int c = 0; c < 4; ++c) ss = fmaf(v[c], v[c], ss);
-    ss = lev_wave_sum_broadcast(ss);
-    if (lane == 0u) s_ss[wave] = ss;
-    lev_barrier_lds();
-    double tot = 0.0;
-    for (int k = 0; k < NW; ++k) tot += (double)s_ss[k];
-    const float inv = (float)lev_rsqrt_f64(tot / (double)a.hidden + (double)a.eps);
-    v = v * inv;
-    if (a.gain) v = v * gain;
-    if (!live || !active) v = lev_f32x4{0.f, 0.f, 0.f, 0.f};      // (an infinite inv made NaNs of the zeros past the end)
+    ffn_normalise<NW>(a, v, gain, live && active, s_ss, wave, lane);
     if (blockIdx.x == 0u && active && live) reinterpret_cast<lev_f32x4 *>(a.h)[64u * T + lane] = v;
 
     uint8_t *area = smem + 2u * kFfnPart + 64u + (size_t)wave * (kQ4mTaskArea + kQ4mZeroBytes), *zero = area + kQ4mTaskArea;
@@ -128,10 +125,42 @@ q4_0_ffn_gate_up(ffn_args a) {
     }
 }
 
+template <int NW, bool SINGLE>
+__global__ void __launch_bounds__(NW * LEV_WAVE, NW / 4)
+q4_0_ffn_gate_up(lev_ffn_args a) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    ffn_gate_up<NW, SINGLE>(a, smem);
+}
+
+// The same and, by the workgroups from `gate_blocks` on, the router scores of h, which those normalise for themselves as
+// well: NW / 4 experts each (recorded programs).
+template <int NW, bool SINGLE>
+__global__ void __launch_bounds__(NW * LEV_WAVE, NW / 4)
+q4_0_ffn_gate_up_and_scores(lev_ffn_args a, lev_scores_args r, uint32_t gate_blocks) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    if (blockIdx.x < gate_blocks) {
+        ffn_gate_up<NW, SINGLE>(a, smem);
+        return;
+    }
+    float *const s_ss = reinterpret_cast<float *>(smem + 2u * kFfnPart), *const s_h = s_ss + 16;
+    const uint32_t lane = threadIdx.x & 63u, part = threadIdx.x >> 8;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const uint32_t n4 = a.hidden >> 2, ntask = (a.hidden + 255u) >> 8, T = wave < ntask ? wave : ntask - 1u;
+    bool live, unused;
+    lev_f32x4 v = q4m_load_activations(a.x, T, n4, live), gain = {1.f, 1.f, 1.f, 1.f};
+    if (a.gain) gain = q4m_load_activations(a.gain, T, n4, unused);
+    live = live && wave < ntask;
+    ffn_normalise<NW>(a, v, gain, live, s_ss, wave, lane);
+    if (live) reinterpret_cast<lev_f32x4 *>(s_h)[64u * T + lane] = v;
+    lev_barrier_lds();
+    moe_score_few(r.wr, s_h, r.scores, r.hidden, r.experts, (blockIdx.x - gate_blocks) * (NW / 4) + part, 0u, threadIdx.x & 255u,
+                  reinterpret_cast<double *>(smem) + 4u * part);
+}
+
 // Whether the first three stages may run at the same time: every workgroup reads all of x, the norm and its own rows
 // of the weights while others already write h, gu and act, which the operators one by one only do when all readers are
 // through.  act may be one of the halves of gu, whose value a lane replaces with its own.
-bool ffn_apart(const ffn_args &a, size_t gate_bytes, size_t up_bytes) {
+bool ffn_apart(const lev_ffn_args &a, size_t gate_bytes, size_t up_bytes) {
     const size_t nh = (size_t)a.hidden * 4u, ni = (size_t)a.inter * 4u;
     const lev_span in[] = {{a.x, nh}, {a.gain, nh}, {a.gate, gate_bytes}, {a.up, up_bytes}};
     const lev_span h(a.h, nh), gu(a.gu, 2u * ni), act(a.act, ni);
@@ -162,7 +191,7 @@ extern "C" int lev_hip_shared_expert_ffn_q4_0(lev_ctx *ctx, const float *d_x, co
     if (st != LEV_OK) return st;
     const uintptr_t al4 = reinterpret_cast<uintptr_t>(d_gate_w) | reinterpret_cast<uintptr_t>(d_up_w);
     const uintptr_t al16 = reinterpret_cast<uintptr_t>(d_x) | reinterpret_cast<uintptr_t>(d_h) | reinterpret_cast<uintptr_t>(d_ffn_norm);
-    ffn_args a = {static_cast<const uint8_t *>(d_gate_w), static_cast<const uint8_t *>(d_up_w), d_x, d_ffn_norm, d_h,
+    lev_ffn_args a = {static_cast<const uint8_t *>(d_gate_w), static_cast<const uint8_t *>(d_up_w), d_x, d_ffn_norm, d_h,
                   d_gu, d_act, hidden, inter, 0u, eps};
     // A schedule installed for the gate/up GEMV keeps the operators apart, so that it is the one that runs.
     const bool fused = hidden % 64u == 0u && hidden <= 4096u && (al4 & 3u) == 0u && (al16 & 15u) == 0u &&
@@ -196,4 +225,32 @@ extern "C" int lev_hip_shared_expert_ffn_q4_0(lev_ctx *ctx, const float *d_x, co
                            "shared_expert_ffn down launch");
     if (st == LEV_OK) st = lev_hip_rmsnorm(ctx, d_shared, d_shared, hidden, 1, d_post_norm, eps);
     return st;
+}
+
+// ---- what recorded programs know of the first kernel (program_nodes.hpp) ----
+namespace {
+template <int NW, bool SINGLE>
+bool with_scores(const void *func, lev_fused_launch *f) {
+    if (func != reinterpret_cast<const void *>(&q4_0_ffn_gate_up<NW, SINGLE>)) return false;
+    *f = lev_fused_launch{reinterpret_cast<void *>(&q4_0_ffn_gate_up_and_scores<NW, SINGLE>), 0u, NW * LEV_WAVE, (uint32_t)ffn_lds(NW)};
+    return true;
+}
+}  // namespace
+
+bool lev_ffn_gate_up_node(const void *func, void **args, lev_ffn_node *out) {
+    lev_fused_launch &f = out->with_scores;
+    if (!with_scores<8, true>(func, &f) && !with_scores<8, false>(func, &f) && !with_scores<12, true>(func, &f) &&
+        !with_scores<12, false>(func, &f) && !with_scores<16, true>(func, &f) && !with_scores<16, false>(func, &f))
+        return false;
+    const lev_ffn_args &a = out->args = *static_cast<const lev_ffn_args *>(args[0]);
+    const size_t nh = 4u * (size_t)a.hidden, ni = 4u * (size_t)a.inter, w = (size_t)a.inter * (a.hidden / 32u) * 18u;
+    out->touches = lev_footprint{};
+    out->touches.reads[0] = lev_span(a.x, nh);
+    out->touches.reads[1] = lev_span(a.gain, nh);
+    out->touches.reads[2] = lev_span(a.gate, w);
+    out->touches.reads[3] = lev_span(a.up, w);
+    out->touches.writes[0] = lev_span(a.h, nh);
+    out->touches.writes[1] = lev_span(a.gu, 2u * ni);
+    out->touches.writes[2] = lev_span(a.act, ni);
+    return true;
 }

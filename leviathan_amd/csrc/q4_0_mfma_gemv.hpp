@@ -16,7 +16,8 @@ __host__ __device__ constexpr size_t q4m_gemv_lds(uint32_t tpw) {
 // wave -> (slot, position in the slot): 4-bit entries of two 64-bit kernel arguments (lev_wave_tables).
 // SINGLE: the grid covers every round once: straight-line code, nothing to prefetch.
 // block, nblocks: the workgroup's place among those of the product.  Waves beyond the slots' only meet the barrier.
-template <int TPW, bool SINGLE, bool ODD>
+// PIN: addresses and masks of the sums held in registers over the rounds (64 of which do not hold them as well).
+template <int TPW, bool SINGLE, bool ODD, bool PIN = true>
 __device__ __forceinline__ void q4m_gemv(const uint8_t *__restrict__ w, const float *__restrict__ x, float *__restrict__ y,
                                          uint32_t in_dim, uint32_t rows, uint32_t wpr, uint32_t slots, uint64_t slot_of_wave,
                                          uint64_t pos_of_wave, uint32_t block_idx, uint32_t grid_dim, uint8_t *smem) {
@@ -96,14 +97,16 @@ __device__ __forceinline__ void q4m_gemv(const uint8_t *__restrict__ w, const fl
     const bool writer = wave < slots && q == 0u;
     uint32_t stores = writer && orow < nrows ? 1u : 0u;
     uint64_t yp = reinterpret_cast<uint64_t>(ODD ? y + 2u * (uint64_t)orow + parity : y + orow);   // (the pointer argument is read here, not behind the barrier)
-    lev_pin(pw);
-    lev_pin(pr);
-    lev_pin(k0);
-    lev_pin(k1);
-    lev_pin(k2);
-    lev_pin(k3);
-    lev_pin(stores);
-    lev_pin(yp);
+    if (PIN) {
+        lev_pin(pw);
+        lev_pin(pr);
+        lev_pin(k0);
+        lev_pin(k1);
+        lev_pin(k2);
+        lev_pin(k3);
+        lev_pin(stores);
+        lev_pin(yp);
+    }
 
     if (lane < kQ4mZeroBytes / 4u) reinterpret_cast<uint32_t *>(zero)[lane] = 0u;
     // more than two tasks' operands do not fit the registers: a product reads them again

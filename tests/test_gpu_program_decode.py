@@ -1,7 +1,7 @@
 """GPU: a recorded decode step, the shared expert's FFN, the MoE layer on its normalised residual and the norm and residuals
 behind both, gives the bits of the operators called one by one on every replay, and replays as the launches that it is meant
-to: the scores of the router go into the launch of the shared expert's down projection, the shared expert's norm into the
-layer's, unless what the one writes the other touches."""
+to: the scores of the router go into the launch of the shared expert's gate/up, its down projection into the layer's, its norm
+into the layer's, unless what the one writes the other touches."""
 import pytest
 import torch
 
@@ -17,10 +17,11 @@ def q4_0(rows, n, g):
     return w.reshape(-1)
 
 
-@pytest.mark.parametrize("case,launches", [("plain", 5), ("two layers", 10), ("scores of the sum", 7), ("sum not added", 6), ("added twice", 6),
-                                           ("part of the sum", 8), ("result is the sum", 6), ("gain is the sum", 6)])
+@pytest.mark.parametrize("case,launches", [("plain", 4), ("two layers", 8), ("scores of the sum", 7), ("sum not added", 5), ("added twice", 5),
+                                           ("part of the sum", 7), ("result is the sum", 5), ("gain is the sum", 5)])
 @pytest.mark.parametrize("hidden,inter,shared,experts,top_k", [
-    (2816, 704, 2112, 128, 8), (1024, 256, 512, 32, 2), (4096, 1536, 4096, 256, 8), (1152, 320, 1344, 60, 4), (2048, 768, 1024, 128, 8), (1280, 576, 640, 256, 8)])
+    (2816, 704, 2112, 128, 8), (1024, 256, 512, 32, 2), (4096, 1536, 4096, 256, 8), (1152, 320, 1344, 60, 4), (2048, 768, 1024, 128, 8), (1280, 576, 640, 256, 8),
+    (2432, 512, 1280, 60, 6), (3840, 896, 1344, 64, 8), (1024, 1984, 768, 32, 8), (3712, 320, 1408, 64, 4)])
 def test_recorded_decode_step(hidden, inter, shared, experts, top_k, case, launches):
     from leviathan_amd import ops
     ctx = ops.Context(0, own_stream=True)
@@ -79,8 +80,10 @@ def test_recorded_decode_step(hidden, inter, shared, experts, top_k, case, launc
         prog.run()
         for a, b in zip(results(), want):
             assert torch.equal(a.view(torch.int32), b.view(torch.int32))
-    # (the scores join the kernel of the matrix cores, which does not take every width of the down projection)
-    alone = 0 if shared % 256 == 0 or shared > 1280 or case == "scores of the sum" else len(layers)
-    assert launches_of(prog) == launches + alone
+    # (nothing joins the vector-ALU kernel that some widths of the down projection take)
+    alone = 0 if shared % 256 == 0 or shared > 1280 or case == "scores of the sum" else 2 * len(layers)
+    # (nor the layer's gate/up where the down projection's workgroups do not fit the chip beside its own)
+    crowded = len(layers) if hidden == 4096 and case != "scores of the sum" else 0
+    assert launches_of(prog) == launches + alone + crowded
     prog.destroy()
     ctx.close()
