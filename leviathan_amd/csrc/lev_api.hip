@@ -570,7 +570,7 @@ namespace {
 // Two more rules look through the shared expert and the MoE layer behind it, whose kernels otherwise run one after the other
 // although they share only the normalised input and the sum at the end (weave_shared_expert, pair_norms).  Four kernels a
 // layer, 115 us and 92 for the same four layers (weights of two such states in turn); five where the launches of the middle
-// do not fit the chip together, 100 us here.  1.04 to 1.42 times as fast over 26 drawn ones.
+// do not fit the chip together, 100 us here.  1.14 to 1.46 times as fast over 26 drawn ones.
 struct node_view {
     const void *func;
     void **args;

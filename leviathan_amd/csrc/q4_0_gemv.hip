@@ -264,14 +264,15 @@ hipError_t launch_pairs(lev_ctx *ctx, const uint8_t *w, const float *x, float *y
 
 }  // namespace
 
-bool lev_q4_0_mfma_gemv_usable(const uint8_t *w, const float *x, uint32_t in_dim);
+bool lev_q4_0_mfma_gemv_usable(const uint8_t *w, const float *x, uint32_t in_dim, bool narrow);
 hipError_t lev_q4_0_mfma_gemv_launch(lev_ctx *ctx, const uint8_t *w, const float *x, float *y, uint32_t in_dim,
                                      uint32_t rows, int persistent);
 void lev_q4_0_mfma_gemv_choice(const lev_ctx *ctx, uint32_t in_dim, uint32_t rows, uint32_t *persistent, bool *other);
 
-// Enqueue without argument checks (callers validated the geometry).
+// Enqueue without argument checks (callers validated the geometry).  narrow: rows that end inside one of their first five
+// tasks take the matrix cores as well (lev_q4_0_mfma_in_dim).
 hipError_t lev_q4_0_gemv_launch(lev_ctx *ctx, const uint8_t *w, const float *x, float *y,
-                                uint32_t in_dim, uint32_t rows) {
+                                uint32_t in_dim, uint32_t rows, bool narrow) {
     const uint32_t nb = in_dim / 32u;
     {
         // a schedule installed for this shape (lev_hip_forge_select) overrides the built-in choice
@@ -280,7 +281,7 @@ hipError_t lev_q4_0_gemv_launch(lev_ctx *ctx, const uint8_t *w, const float *x, 
             const char *e = getenv("LEV_Q4_MFMA");   // experiments: 0 = vector-ALU kernels, 1 = matrix-core kernel
             return e ? atoi(e) : -1;
         }();
-        const bool usable = lev_q4_0_mfma_gemv_usable(w, x, in_dim);
+        const bool usable = lev_q4_0_mfma_gemv_usable(w, x, in_dim, narrow);
         if (usable && (sel ? sel->family == 1u : env_mfma != 0))
             return lev_q4_0_mfma_gemv_launch(ctx, w, x, y, in_dim, rows, sel ? (int)sel->persistent : -1);
     }
@@ -368,6 +369,6 @@ extern "C" int lev_hip_q4_0_gemv(lev_ctx *ctx, const void *d_w, size_t w_bytes, 
                               d_y, y_capacity, out_rows, in_dim, out_rows, &g);
     if (st != LEV_OK) return st;
     const uint8_t *w = static_cast<const uint8_t *>(d_w) + w_off;
-    return lev_hip_check(ctx, lev_q4_0_gemv_launch(ctx, w, d_x, d_y, in_dim, out_rows),
+    return lev_hip_check(ctx, lev_q4_0_gemv_launch(ctx, w, d_x, d_y, in_dim, out_rows, false),
                          "q4_0_gemv launch");
 }

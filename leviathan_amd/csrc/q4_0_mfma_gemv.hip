@@ -98,8 +98,8 @@ hipError_t launch(lev_ctx *ctx, const uint8_t *w, const float *x, float *y, uint
 
 }  // namespace
 
-bool lev_q4_0_mfma_gemv_usable(const uint8_t *w, const float *x, uint32_t in_dim) {
-    return lev_q4_0_mfma_in_dim(in_dim) && (reinterpret_cast<uintptr_t>(w) & 3u) == 0u &&
+bool lev_q4_0_mfma_gemv_usable(const uint8_t *w, const float *x, uint32_t in_dim, bool narrow) {
+    return (lev_q4_0_mfma_in_dim(in_dim) || (narrow && in_dim != 0u && in_dim % 64u == 0u && in_dim <= 1280u)) && (reinterpret_cast<uintptr_t>(w) & 3u) == 0u &&
            (reinterpret_cast<uintptr_t>(x) & 15u) == 0u;
 }
 

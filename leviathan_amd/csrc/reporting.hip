@@ -8,7 +8,7 @@
 #include <cmath>
 
 hipError_t lev_q4_0_gemv_launch(lev_ctx *ctx, const uint8_t *w, const float *x, float *y,
-                                uint32_t in_dim, uint32_t rows);
+                                uint32_t in_dim, uint32_t rows, bool narrow);
 hipError_t lev_q6_k_gemv_launch(lev_ctx *ctx, const uint8_t *w, const float *x, float *y,
                                 uint32_t in_dim, uint32_t rows);
 
@@ -72,7 +72,7 @@ int matvec_reporting(bool q6, const uint8_t *blocks, size_t blocks_count, int64_
                       : lev_q4_0_gemv_launch(b.ctx, static_cast<const uint8_t *>(b.w),
                                              static_cast<const float *>(b.x),
                                              static_cast<float *>(b.y), (uint32_t)in_dim,
-                                             (uint32_t)out_dim);
+                                             (uint32_t)out_dim, false);
     if (e != hipSuccess) return LEV_ERR_COMMAND_FAILED;
     if ((st = lev_hip_sync(b.ctx)) != LEV_OK) return LEV_ERR_COMMAND_FAILED;
     if ((st = lev_hip_buf_download(b.ctx, y_out, b.y, (size_t)out_dim * 4)) != LEV_OK) return st;
