@@ -358,6 +358,28 @@ def test_moe_grouped_path_many_tokens(ctx, experts, tokens, again):
     assert np.array_equal(act2.view(np.uint32), act[:again].view(np.uint32))
 
 
+@pytest.mark.parametrize("experts,tokens,top_k", [(24, 40, 12), (24, 1100, 12), (20, 1030, 8), (9, 1025, 3)])
+def test_moe_grouped_product_places_every_pair(ctx, experts, tokens, top_k):
+    """The grouping of a prompt keeps a thread's first eight pairs in registers and parks the others: tokens past the 1024
+    threads, slots past the eighth.  A token's outputs against the same token in a batch of its own size class, bit for bit
+    (a pair's result does not depend on the batch), and sampled tokens against the FP64 chain."""
+    hidden, inter = 256, 256
+    wr, pool, offs, x = H.config5(hidden, inter, experts, tokens, seed=experts + top_k)
+    rng = np.random.default_rng(experts + top_k)
+    ids = np.stack([rng.permutation(experts)[:top_k] for _ in range(tokens)]).astype(np.int32)
+    wts = rng.random((tokens, top_k)).astype(np.float32)
+    y, act = run_experts(ctx, pool, offs, hidden, inter, experts, x, ids, wts)
+    back = tokens - 40
+    y2, act2 = run_experts(ctx, pool, offs, hidden, inter, experts, x[back:], ids[back:], wts[back:])
+    assert np.array_equal(y2.view(np.uint32), y[back:].view(np.uint32))
+    assert np.array_equal(act2.view(np.uint32), act[back:].view(np.uint32))
+    g, u, d = (pool[offs["gate_off"]:], pool[offs["up_off"]:], pool[offs["down_off"]:])
+    for t in sorted({0, 7, min(1023, tokens - 1), min(1024, tokens - 1), tokens - 1}):
+        ref = O.moe_experts_f64(g, u, d, hidden, inter, ids[t], wts[t], x[t])
+        assert O.max_rel_err(act[t], ref["act"]) < TOL
+        assert O.max_rel_err(y[t], ref["y"]) < TOL
+
+
 @pytest.mark.parametrize("experts,tokens,top_k", [(16, 2, 2), (16, 6, 2), (4, 12, 2)])
 def test_moe_non_finite_activation_stays_in_its_token(ctx, experts, tokens, top_k):
     """A NaN or an infinity in one token's activations makes every output of THAT token non-finite
