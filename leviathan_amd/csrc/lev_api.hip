@@ -266,13 +266,7 @@ int lev_check_matvec(lev_ctx *ctx, const char *op, uint32_t block_values, uint32
 
 namespace {
 
-// What follows an RMSNorm in a recorded program: y += c[k] * x[k], in order (see fuse_norm_chains).
-struct norm_adds {
-    static constexpr int kMost = 4;
-    const float *x[kMost];
-    float c[kMost];
-    int count;
-};
+using norm_adds = lev_norm_adds;
 
 // One workgroup of up to 16 waves per vector.  Sum of squares in f32 per lane, wave DPP sums, f64 across
 // waves; y = x * inv * w.  A call on one vector is latency and nothing else (11 KB at n = 2816), so the
@@ -567,10 +561,11 @@ namespace {
 // values; an addend that does not overlap the result.  The same values, rounded at the same places.  Anything this
 // cannot see through stays as it was recorded.  Recorded decode step of four layers at 2816: 135 us with
 // the operators at the end of a layer apart, 123 with this; seven kernels a layer.
-// Two more rules look through the shared expert and the MoE layer behind it, whose kernels otherwise run one after the other
-// although they share only the normalised input and the sum at the end (weave_shared_expert, pair_norms).  Four kernels a
-// layer, 115 us and 92 for the same four layers (weights of two such states in turn); five where the launches of the middle
-// do not fit the chip together, 100 us here.  1.14 to 1.46 times as fast over 26 drawn ones.
+// Three more rules look through the shared expert and the MoE layer behind it, whose kernels otherwise run one after the other
+// although they share only the normalised input and the sum at the end (weave_shared_expert, pair_norms), and through the
+// norm and residuals in front of an FFN (front_norms).  Four kernels a layer and three for the next, 115 us and 89 for the same
+// four layers (weights of two such states in turn; 92 with the norms apart, 100 where the launches of the middle do not fit the
+// chip together).  1.15 to 1.56 times as fast over 26 drawn ones.
 struct node_view {
     const void *func;
     void **args;
@@ -746,9 +741,11 @@ hipError_t weave_shared_expert(hipGraph_t graph, const std::vector<hipGraphNode_
             lev_moe_gate_up_and_gemv(ctx, u.func, u.args, &gg, &gu)) {
             const uint32_t each = fn.with_scores.threads / 256u;
             uint32_t blocks = f.params.gridDim.x;
-            void *with_scores[3] = {&fn.args, &sa, &blocks}, *with_gemv[13];
+            void *with_scores[3] = {&fn.args, &sa, &blocks}, *with_gemv[14];
             for (int k = 0; k < 9; ++k) with_gemv[k] = u.args[k];
             with_gemv[9] = &gu.rows_per_block, with_gemv[10] = &gg, with_gemv[11] = &gu.extra, with_gemv[12] = &gu.gemv_blocks;
+            lev_norm_tail none{};
+            with_gemv[13] = &none;
             e = become(ffn, fn.with_scores.func, blocks + (sa.experts + each - 1u) / each, fn.with_scores.threads, fn.with_scores.lds, with_scores);
             if (e == hipSuccess) e = become(first, gu.launch.func, gu.launch.blocks, gu.launch.threads, gu.launch.lds, with_gemv, gu.top_k);
             if (e == hipSuccess) e = hand_on(graph, gate_up, norm);
@@ -821,20 +818,100 @@ hipError_t pair_norms(hipGraph_t graph, const std::vector<hipGraphNode_t> &nodes
     return hipSuccess;
 }
 
+// The norm and adds in front of an FFN whose gate/up computes the scores too: every workgroup of it makes x for itself, with its
+// weights on their way (2432 / 512 and 1280 four layers 78.9 us and 76.3, 3712 / 320 and 1408 79.4 and 73.3; 19 programs of
+// several layers 0.92 to 1.01 of the time).  The
+// norm of the pair that goes in place (the shared expert's of the layer before) is stored by the launch behind, unless that
+// writes a new value there.
+hipError_t front_norms(hipGraph_t graph, const std::vector<hipGraphNode_t> &heads, const lev_ctx *ctx) {
+    for (hipGraphNode_t norm : heads) {
+        node_view n, f, u;
+        hipGraphNode_t ffn, behind;
+        lev_ffn_node fn;
+        lev_footprint ut;
+        if (!kernel_node(norm, &n) || !only_next(norm, &ffn) || !kernel_node(ffn, &f) || !lev_ffn_gate_up_node(f.func, f.args, &fn) ||
+            f.func != fn.with_scores.func || !only_next(ffn, &behind) || !kernel_node(behind, &u))
+            continue;
+        lev_norm_front front{};
+        uint32_t len;
+        front.own = -1;
+        if (n.func == reinterpret_cast<const void *>(&rmsnorm_adds_kernel<1>)) {
+            front.y = arg_of<const float *>(n, 0), front.out = arg_of<float *>(n, 1), front.wy = arg_of<const float *>(n, 2);
+            len = arg_of<uint32_t>(n, 3), front.eps = arg_of<float>(n, 4), front.adds = arg_of<norm_adds>(n, 5);
+        } else {
+            const norm_pair p = arg_of<norm_pair>(n, 0);
+            front.s = p.x, front.ws = p.wx, front.eps_s = p.eps, front.own = p.own;
+            front.y = arg_of<const float *>(n, 1), front.out = arg_of<float *>(n, 2), front.wy = arg_of<const float *>(n, 3);
+            len = arg_of<uint32_t>(n, 4), front.eps = arg_of<float>(n, 5), front.adds = arg_of<norm_adds>(n, 6);
+        }
+        lev_scores_args sa = arg_of<lev_scores_args>(f, 1);
+        uint32_t blocks = arg_of<uint32_t>(f, 2);
+        if (n.params.gridDim.x != 1u || front.out != fn.args.x || len != fn.args.hidden || front.adds.count > lev_norm_front::kMost) continue;
+        int per_cu = 0;   // (more registers: what was on the chip at once has to be so still)
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn.with_front.func, (int)fn.with_front.threads, fn.with_front.lds) != hipSuccess ||
+            (uint32_t)(per_cu * ctx->num_cus) < f.params.gridDim.x)
+            continue;
+        // what the norm reads, whose values no workgroup of the FFN's may change, and its result beside what those touch
+        const size_t bytes = 4u * (size_t)len;
+        lev_footprint rt, wt, ft = fn.touches;
+        rt.reads[0] = lev_span(front.y, bytes), rt.reads[1] = lev_span(front.wy, bytes), rt.reads[2] = lev_span(front.s, bytes),
+        rt.reads[3] = lev_span(front.ws, bytes);
+        for (int k = 0; k < front.adds.count; ++k)
+            if (k != front.own) rt.reads[4 + k] = lev_span(front.adds.x[k], bytes);
+        wt.writes[0] = lev_span(front.out, bytes);
+        ft.reads[0] = lev_span();                                          // (x, which is made)
+        ft.reads[4] = lev_span(sa.wr, 4u * (size_t)sa.experts * sa.hidden);
+        ft.writes[3] = lev_span(sa.scores, 4u * (size_t)sa.experts);
+        if (!rt.apart(ft) || !wt.apart(ft) || !wt.apart(rt)) continue;
+        if (front.s) {
+            const lev_norm_tail tail{const_cast<float *>(front.s), front.ws, len, front.eps_s};
+            if (!lev_moe_gate_up_and_gemv_is(u.func) || !lev_moe_expert_node(ctx, u.func, u.args, &ut)) continue;
+            lev_footprint tt;
+            tt.writes[0] = lev_span(front.s, bytes);
+            tt.reads[0] = lev_span(front.ws, bytes);
+            const lev_gemv_args g = arg_of<lev_gemv_args>(u, 10);
+            if (!(g.y == front.s && g.rows >= len)) {
+                if (!tt.apart(ut) || !tt.apart(gemv_touches(g))) continue;
+                const hipError_t e = lev_moe_gate_up_and_gemv_tail(behind, tail);
+                if (e == hipErrorNotSupported) continue;
+                if (e != hipSuccess) return e;
+            }
+        }
+        size_t nbefore = 0;
+        void *args[4] = {&fn.args, &sa, &blocks, &front};
+        hipError_t e = become(ffn, fn.with_front.func, f.params.gridDim.x, fn.with_front.threads, fn.with_front.lds, args);
+        if (e == hipSuccess) e = hipGraphNodeGetDependencies(norm, nullptr, &nbefore);
+        if (e == hipSuccess && nbefore) {
+            std::vector<hipGraphNode_t> before(nbefore);
+            const std::vector<hipGraphNode_t> to(nbefore, ffn);
+            e = hipGraphNodeGetDependencies(norm, before.data(), &nbefore);
+            if (e == hipSuccess) e = hipGraphAddDependencies(graph, before.data(), to.data(), nbefore);
+        }
+        if (e == hipSuccess) e = hipGraphDestroyNode(norm);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
 hipError_t fuse_nodes(hipGraph_t graph, const lev_ctx *ctx) {
     hipError_t e = fuse_norm_chains(graph);
-    for (int rule = 0; rule < 2 && e == hipSuccess; ++rule) {
+    for (int rule = 0; rule < 3 && e == hipSuccess; ++rule) {
         size_t count = 0;
         if (hipGraphGetNodes(graph, nullptr, &count) != hipSuccess || count == 0) return hipSuccess;
         std::vector<hipGraphNode_t> nodes(count);
         if (hipGraphGetNodes(graph, nodes.data(), &count) != hipSuccess) return hipSuccess;
-        // the heads of the pattern alone: a fusion destroys the nodes behind its head, which are never heads themselves
+        // the heads of the pattern alone: a fusion destroys nodes that are no heads, or the head itself
+        auto is_head = [&](const node_view &v) {
+            if (rule == 0) return v.func == lev_q4_0_gemv_one_round();
+            if (rule == 1) return norm_kind(v) >= 0;
+            return v.func == reinterpret_cast<const void *>(&rmsnorm_adds_kernel<1>) || v.func == reinterpret_cast<const void *>(&rmsnorm_pair_kernel<1>);
+        };
         std::vector<hipGraphNode_t> heads;
         for (hipGraphNode_t node : nodes) {
             node_view v;
-            if (kernel_node(node, &v) && (rule == 0 ? v.func == lev_q4_0_gemv_one_round() : norm_kind(v) >= 0)) heads.push_back(node);
+            if (kernel_node(node, &v) && is_head(v)) heads.push_back(node);
         }
-        e = rule == 0 ? weave_shared_expert(graph, heads, ctx) : pair_norms(graph, heads, ctx);
+        e = rule == 0 ? weave_shared_expert(graph, heads, ctx) : rule == 1 ? pair_norms(graph, heads, ctx) : front_norms(graph, heads, ctx);
     }
     return e;
 }

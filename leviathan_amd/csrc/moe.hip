@@ -1134,13 +1134,14 @@ moe_gate_up_mfma(moe_args a, const float *__restrict__ x, const int32_t *ids, co
 
 // The same at one token beside a GEMV that does not depend on it (recorded programs: the shared expert's down projection,
 // which alone on the chip is the launch and little else).  grid (extra + chunks, top_k): the first `extra` workgroups of a
-// slot are the GEMV's, gemv_blocks in all.  Two workgroups of 12 or 16 waves a CU, four of 8: 80 and 64 registers (the latter
+// slot are the GEMV's, gemv_blocks in all, and one the tail's (the norm of the layer before, if it has one to store).  Two workgroups of 12 or 16 waves a CU, four of 8: 80 and 64 registers (the latter
 // without the pins of q4m_gemv).
 template <int NW, int ROUTE>
 __global__ void __launch_bounds__(NW * LEV_WAVE, NW / 2)
 moe_gate_up_and_gemv(moe_args a, const float *__restrict__ x, const int32_t *ids, const float *__restrict__ scores,
                      const float *__restrict__ expert_scale, int32_t *ids_out, float *weights_out, float *__restrict__ act,
-                     int *__restrict__ flag, uint32_t rows_per_block, lev_gemv_args g, uint32_t extra, uint32_t gemv_blocks) {
+                     int *__restrict__ flag, uint32_t rows_per_block, lev_gemv_args g, uint32_t extra, uint32_t gemv_blocks,
+                     lev_norm_tail tail) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     if (blockIdx.x >= extra) {
         gate_up_mfma<NW, true, ROUTE>(a, x, ids, scores, expert_scale, ids_out, weights_out, act, flag, rows_per_block,
@@ -1148,7 +1149,27 @@ moe_gate_up_and_gemv(moe_args a, const float *__restrict__ x, const int32_t *ids
         return;
     }
     const uint32_t block = blockIdx.y * extra + blockIdx.x;
-    if (block >= gemv_blocks) return;
+    if (block > gemv_blocks || (block == gemv_blocks && !tail.s)) return;
+    if (block == gemv_blocks) {
+        // as rmsnorm_pair_kernel: a piece of four values a lane (n <= NW * 256)
+        float *const part = reinterpret_cast<float *>(smem);
+        const uint32_t i = threadIdx.x, n4 = tail.n >> 2;
+        lev_f32x4 *const s4 = reinterpret_cast<lev_f32x4 *>(tail.s);
+        lev_f32x4 v = i < n4 ? s4[i] : lev_f32x4{0.f, 0.f, 0.f, 0.f}, w = {1.f, 1.f, 1.f, 1.f};
+        if (tail.ws) w = reinterpret_cast<const lev_f32x4 *>(tail.ws)[i < n4 ? i : 0u];
+        float ss = 0.f;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) ss = fmaf(v[c], v[c], ss);
+        ss = lev_wave_sum_broadcast(ss);
+        if ((i & 63u) == 0u) part[i >> 6] = ss;
+        lev_barrier_lds();
+        double tot = 0.0;
+        for (int k = 0; k < NW; ++k) tot += (double)part[k];
+        v = v * (float)lev_rsqrt_f64(tot / (double)tail.n + (double)tail.eps);
+        if (tail.ws) v = v * w;
+        if (i < n4) s4[i] = v;
+        return;
+    }
     if (gemv_blocks * g.slots * 16u >= g.rows)
         q4m_gemv<1, true, false>(g.w, g.x, g.y, g.in_dim, g.rows, g.wpr, g.slots, g.slot_of_wave, g.pos_of_wave, block, gemv_blocks, smem);
     else
@@ -1898,10 +1919,16 @@ bool is_down(const void *f) {
            f == reinterpret_cast<const void *>(&moe_down_kernel<64>);
 }
 
+template <int NW>
+bool is_gate_up_and_gemv_of(const void *f) {
+    return f == reinterpret_cast<const void *>(&moe_gate_up_and_gemv<NW, 2>) || f == reinterpret_cast<const void *>(&moe_gate_up_and_gemv<NW, 4>);
+}
+bool is_gate_up_and_gemv(const void *f) { return is_gate_up_and_gemv_of<8>(f) || is_gate_up_and_gemv_of<12>(f) || is_gate_up_and_gemv_of<16>(f); }
+
 }  // namespace
 
 bool lev_moe_expert_node(const lev_ctx *ctx, const void *func, void **args, lev_footprint *touches) {
-    const bool gate_up = is_gate_up(func);
+    const bool gate_up = is_gate_up(func) || is_gate_up_and_gemv(func);   // (of the latter, the layer's part)
     if (!gate_up && !is_down(func)) return false;
     const moe_args &a = *static_cast<const moe_args *>(args[0]);
     const size_t gu = (size_t)a.inter * (a.hidden / 32u) * 18u, dn = (size_t)a.hidden * (a.inter / 32u) * 18u, k = a.top_k;
@@ -1974,4 +2001,27 @@ bool lev_moe_gate_up_and_gemv(const lev_ctx *ctx, const void *func, void **args,
     return gate_up_and_gemv<8, 2>(func, ctx, a, rows, *g, out) || gate_up_and_gemv<8, 4>(func, ctx, a, rows, *g, out) ||
            gate_up_and_gemv<12, 2>(func, ctx, a, rows, *g, out) || gate_up_and_gemv<12, 4>(func, ctx, a, rows, *g, out) ||
            gate_up_and_gemv<16, 2>(func, ctx, a, rows, *g, out) || gate_up_and_gemv<16, 4>(func, ctx, a, rows, *g, out);
+}
+
+bool lev_moe_gate_up_and_gemv_is(const void *func) { return is_gate_up_and_gemv(func); }
+
+hipError_t lev_moe_gate_up_and_gemv_tail(hipGraphNode_t node, const lev_norm_tail &tail) {
+    hipKernelNodeParams now;
+    hipError_t e = hipGraphKernelNodeGetParams(node, &now);
+    if (e != hipSuccess) return e;
+    if (!is_gate_up_and_gemv(now.func) || tail.n > now.blockDim.x * 4u) return hipErrorNotSupported;
+    // copies: the node's own arguments are gone when it gets new ones
+    moe_args a = *static_cast<moe_args *>(now.kernelParams[0]);
+    void *p[8];
+    for (int k = 0; k < 8; ++k) p[k] = *static_cast<void **>(now.kernelParams[k + 1]);
+    uint32_t rows = *static_cast<uint32_t *>(now.kernelParams[9]), extra = *static_cast<uint32_t *>(now.kernelParams[11]),
+             blocks = *static_cast<uint32_t *>(now.kernelParams[12]);
+    lev_gemv_args g = *static_cast<lev_gemv_args *>(now.kernelParams[10]);
+    lev_norm_tail t = tail;
+    hipKernelNodeParams kp = now;
+    if (extra * now.gridDim.y == blocks) ++extra, ++kp.gridDim.x;
+    void *args[14] = {&a, &p[0], &p[1], &p[2], &p[3], &p[4], &p[5], &p[6], &p[7], &rows, &g, &extra, &blocks, &t};
+    kp.kernelParams = args;
+    kp.extra = nullptr;
+    return hipGraphKernelNodeSetParams(node, &kp);
 }

@@ -54,6 +54,31 @@ lev_fused_launch lev_q4_0_gemv_and_scores(uint32_t gemv_blocks, uint32_t gemv_th
 // Whether `func` is one of the MoE layer's kernels at one token (gate/up, down), and what it touches.
 bool lev_moe_expert_node(const lev_ctx *ctx, const void *func, void **args, lev_footprint *touches);
 
+// What follows an RMSNorm in a recorded program: y += c[k] * x[k], in order.
+struct lev_norm_adds {
+    static constexpr int kMost = 4;
+    const float *x[kMost];
+    float c[kMost];
+    int count;
+};
+// The norm and adds (two at most) that make the input of an FFN: out = rmsnorm(y) * wy + adds, where adds number `own` is
+// rmsnorm(s) * ws unless s is null.
+struct lev_norm_front {
+    static constexpr int kMost = 2;
+    const float *y, *wy, *s, *ws;
+    float *out;
+    lev_norm_adds adds;
+    float eps, eps_s;
+    int own;
+};
+// s = rmsnorm(s) * ws, of n values
+struct lev_norm_tail {
+    float *s;
+    const float *ws;
+    uint32_t n;
+    float eps;
+};
+
 struct lev_ffn_args {
     const uint8_t *gate, *up;
     const float *x, *gain;
@@ -61,19 +86,23 @@ struct lev_ffn_args {
     uint32_t hidden, inter, rows_per_block;
     float eps;
 };
-// The first kernel of the shared expert's FFN: its arguments, what it touches, and the launch (without its number of
-// workgroups) that computes the router's scores of h as well: arguments lev_ffn_args, lev_scores_args, its own workgroups.
+// The first kernel of the shared expert's FFN: its arguments, what it touches, and the launches (without their number of
+// workgroups) that compute the router's scores of h as well: arguments lev_ffn_args, lev_scores_args, its own workgroups;
+// with_front: lev_norm_front behind them, in whose place x is.
 struct lev_ffn_node {
     lev_ffn_args args;
     lev_footprint touches;
-    lev_fused_launch with_scores;
+    lev_fused_launch with_scores, with_front;
 };
 bool lev_ffn_gate_up_node(const void *func, void **args, lev_ffn_node *out);
 
 // The launch of the MoE layer's gate/up kernel of one token with a GEMV of one round beside it: `args` of the former with
-// rows_per_block, then *g (its slots are those of the launch), extra, gemv_blocks; grid (launch.blocks, top_k).
+// rows_per_block, then *g (its slots are those of the launch), extra, gemv_blocks, a lev_norm_tail; grid (launch.blocks, top_k).
 struct lev_gate_up_gemv {
     lev_fused_launch launch;
     uint32_t rows_per_block, extra, gemv_blocks, top_k;
 };
 bool lev_moe_gate_up_and_gemv(const lev_ctx *ctx, const void *func, void **args, lev_gemv_args *g, lev_gate_up_gemv *out);
+bool lev_moe_gate_up_and_gemv_is(const void *func);
+// Gives such a launch its tail, which one more workgroup (of a slot) does.
+hipError_t lev_moe_gate_up_and_gemv_tail(hipGraphNode_t node, const lev_norm_tail &tail);

@@ -17,7 +17,8 @@ namespace {
 
 // part of a round: [gate, up][wave][row] f32, two of them
 constexpr uint32_t kFfnPart = 2u * 16u * 16u * 4u, kFfnUp = kFfnPart / 2u;
-constexpr size_t ffn_lds(int nw) { return 2u * kFfnPart + 64u + (size_t)nw * (kQ4mTaskArea + kQ4mZeroBytes); }
+constexpr uint32_t kFfnSums = 3u * 64u;   // three sums of squares of sixteen waves
+constexpr size_t ffn_lds(int nw) { return 2u * kFfnPart + kFfnSums + (size_t)nw * (kQ4mTaskArea + kQ4mZeroBytes); }
 
 // The wave's 256 values of x, normalised as lev_hip_rmsnorm does it: squares in f32 per wave, f64 across the waves.
 template <int NW>
@@ -38,10 +39,61 @@ __device__ __forceinline__ void ffn_normalise(const lev_ffn_args &a, lev_f32x4 &
     if (!live) v = lev_f32x4{0.f, 0.f, 0.f, 0.f};                 // (an infinite inv made NaNs of the zeros past the end)
 }
 
+// x itself where a norm and adds make it: as rmsnorm_adds_kernel and rmsnorm_pair_kernel do, a lane the same four values.
+// The first workgroup stores it.
+struct ffn_front {
+    lev_f32x4 b, gb, a, ga, ad[lev_norm_front::kMost];
+    bool live;
+    __device__ __forceinline__ void request(const lev_norm_front &f, uint32_t T, uint32_t n4) {
+        bool unused;
+        b = q4m_load_activations(f.y, T, n4, live);
+        if (f.wy) gb = q4m_load_activations(f.wy, T, n4, unused);
+        if (f.s) a = q4m_load_activations(f.s, T, n4, unused);
+        if (f.s && f.ws) ga = q4m_load_activations(f.ws, T, n4, unused);
+#pragma unroll
+        for (int m = 0; m < lev_norm_front::kMost; ++m)
+            if (m < f.adds.count && m != f.own) ad[m] = q4m_load_activations(f.adds.x[m], T, n4, unused);
+    }
+    template <int NW>
+    __device__ __forceinline__ lev_f32x4 value(const lev_norm_front &f, uint32_t n, bool active, float *sums, uint32_t wave, uint32_t lane) {
+        b = q4m_mask_activations(b, live && active);
+        float sb = 0.f, sa = 0.f;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) sb = fmaf(b[c], b[c], sb);
+        if (f.s) {
+            a = q4m_mask_activations(a, live && active);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) sa = fmaf(a[c], a[c], sa);
+            sa = lev_wave_sum_broadcast(sa);
+        }
+        sb = lev_wave_sum_broadcast(sb);
+        if (lane == 0u) sums[wave] = sb, sums[16u + wave] = sa;
+        lev_barrier_lds();
+        double tb = 0.0, ta = 0.0;
+        for (int k = 0; k < NW; ++k) tb += (double)sums[k];
+        const float ib = (float)lev_rsqrt_f64(tb / (double)n + (double)f.eps);
+        lev_f32x4 o = b * ib, x = {0.f, 0.f, 0.f, 0.f};
+        if (f.wy) o = o * gb;
+        if (f.s) {
+            for (int k = 0; k < NW; ++k) ta += (double)sums[16 + k];
+            x = a * (float)lev_rsqrt_f64(ta / (double)n + (double)f.eps_s);
+            if (f.ws) x = x * ga;
+        }
+#pragma unroll
+        for (int m = 0; m < lev_norm_front::kMost; ++m) {
+            if (m >= f.adds.count) break;
+            const lev_f32x4 v = m == f.own ? x : ad[m];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) o[c] = fmaf(f.adds.c[m], v[c], o[c]);
+        }
+        return o;
+    }
+};
+
 // NW waves, one per column task (at most 16).  SINGLE: a workgroup has one group of 16 rows, nothing to prefetch.
 // grid (row chunks).
-template <int NW, bool SINGLE>
-__device__ __forceinline__ void ffn_gate_up(const lev_ffn_args &a, uint8_t *smem) {
+template <int NW, bool SINGLE, bool FRONT = false>
+__device__ __forceinline__ void ffn_gate_up(const lev_ffn_args &a, uint8_t *smem, const lev_norm_front &front = lev_norm_front{}) {
     float *const s_ss = reinterpret_cast<float *>(smem + 2u * kFfnPart);
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
@@ -49,8 +101,14 @@ __device__ __forceinline__ void ffn_gate_up(const lev_ffn_args &a, uint8_t *smem
     const bool active = wave < ntask;
     const uint32_t T = active ? wave : ntask - 1u;
     bool live;
-    lev_f32x4 v = q4m_load_activations(a.x, T, n4, live);
-    lev_f32x4 gain = {1.f, 1.f, 1.f, 1.f};
+    lev_f32x4 v, gain = {1.f, 1.f, 1.f, 1.f};
+    ffn_front before;
+    if (FRONT) {
+        before.request(front, T, n4);
+        live = before.live;
+    } else {
+        v = q4m_load_activations(a.x, T, n4, live);
+    }
     if (a.gain) {
         bool unused;
         gain = q4m_load_activations(a.gain, T, n4, unused);
@@ -70,10 +128,14 @@ __device__ __forceinline__ void ffn_gate_up(const lev_ffn_args &a, uint8_t *smem
     issue(i0, Ga, Ua);
     __builtin_amdgcn_sched_barrier(0);
 
+    if (FRONT) {
+        v = before.value<NW>(front, a.hidden, active, s_ss + 16, wave, lane);
+        if (blockIdx.x == 0u && active && live) reinterpret_cast<lev_f32x4 *>(front.out)[64u * T + lane] = v;
+    }
     ffn_normalise<NW>(a, v, gain, live && active, s_ss, wave, lane);
     if (blockIdx.x == 0u && active && live) reinterpret_cast<lev_f32x4 *>(a.h)[64u * T + lane] = v;
 
-    uint8_t *area = smem + 2u * kFfnPart + 64u + (size_t)wave * (kQ4mTaskArea + kQ4mZeroBytes), *zero = area + kQ4mTaskArea;
+    uint8_t *area = smem + 2u * kFfnPart + kFfnSums + (size_t)wave * (kQ4mTaskArea + kQ4mZeroBytes), *zero = area + kQ4mTaskArea;
     if (lane < kQ4mZeroBytes / 4u) reinterpret_cast<uint32_t *>(zero)[lane] = 0u;
     q4m_operand op;
     q4m_stage_task(v, area, zero, active, op);
@@ -133,28 +195,49 @@ q4_0_ffn_gate_up(lev_ffn_args a) {
 }
 
 // The same and, by the workgroups from `gate_blocks` on, the router scores of h, which those normalise for themselves as
-// well: NW / 4 experts each (recorded programs).
-template <int NW, bool SINGLE>
-__global__ void __launch_bounds__(NW * LEV_WAVE, NW / 4)
-q4_0_ffn_gate_up_and_scores(lev_ffn_args a, lev_scores_args r, uint32_t gate_blocks) {
-    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+// well: NW / 4 experts each (recorded programs).  FRONT: every workgroup makes x for itself, from the norm and adds in front
+// of the FFN, which as a launch of their own take 2.7 us and a gap.
+template <int NW, bool SINGLE, bool FRONT>
+__device__ __forceinline__ void ffn_gate_up_and_scores(const lev_ffn_args &a, const lev_scores_args &r, uint32_t gate_blocks, uint8_t *smem,
+                                                       const lev_norm_front &front) {
     if (blockIdx.x < gate_blocks) {
-        ffn_gate_up<NW, SINGLE>(a, smem);
+        ffn_gate_up<NW, SINGLE, FRONT>(a, smem, front);
         return;
     }
-    float *const s_ss = reinterpret_cast<float *>(smem + 2u * kFfnPart), *const s_h = s_ss + 16;
+    float *const s_ss = reinterpret_cast<float *>(smem + 2u * kFfnPart), *const s_h = s_ss + kFfnSums / 4u;
     const uint32_t lane = threadIdx.x & 63u, part = threadIdx.x >> 8;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const uint32_t n4 = a.hidden >> 2, ntask = (a.hidden + 255u) >> 8, T = wave < ntask ? wave : ntask - 1u;
     bool live, unused;
-    lev_f32x4 v = q4m_load_activations(a.x, T, n4, live), gain = {1.f, 1.f, 1.f, 1.f};
+    lev_f32x4 v, gain = {1.f, 1.f, 1.f, 1.f};
+    ffn_front before;
+    if (FRONT) {
+        before.request(front, T, n4);
+        live = before.live;
+    } else {
+        v = q4m_load_activations(a.x, T, n4, live);
+    }
     if (a.gain) gain = q4m_load_activations(a.gain, T, n4, unused);
+    if (FRONT) v = before.value<NW>(front, a.hidden, wave < ntask, s_ss + 16, wave, lane);
     live = live && wave < ntask;
     ffn_normalise<NW>(a, v, gain, live, s_ss, wave, lane);
     if (live) reinterpret_cast<lev_f32x4 *>(s_h)[64u * T + lane] = v;
     lev_barrier_lds();
     moe_score_few(r.wr, s_h, r.scores, r.hidden, r.experts, (blockIdx.x - gate_blocks) * (NW / 4) + part, 0u, threadIdx.x & 255u,
                   reinterpret_cast<double *>(smem) + 4u * part);
+}
+
+template <int NW, bool SINGLE>
+__global__ void __launch_bounds__(NW * LEV_WAVE, NW / 4)
+q4_0_ffn_gate_up_and_scores(lev_ffn_args a, lev_scores_args r, uint32_t gate_blocks) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    ffn_gate_up_and_scores<NW, SINGLE, false>(a, r, gate_blocks, smem, lev_norm_front{});
+}
+template <int NW, bool SINGLE>
+__global__ void __launch_bounds__(NW * LEV_WAVE, NW / 4)
+q4_0_ffn_norm_gate_up_and_scores(lev_ffn_args a, lev_scores_args r, uint32_t gate_blocks, lev_norm_front front) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    ffn_gate_up_and_scores<NW, SINGLE, true>(a, r, gate_blocks, smem, front);
 }
 
 // Whether the first three stages may run at the same time: every workgroup reads all of x, the norm and its own rows
@@ -232,18 +315,21 @@ extern "C" int lev_hip_shared_expert_ffn_q4_0(lev_ctx *ctx, const float *d_x, co
 
 // ---- what recorded programs know of the first kernel (program_nodes.hpp) ----
 namespace {
+// (the FFN's own kernel or the one with scores)
 template <int NW, bool SINGLE>
-bool with_scores(const void *func, lev_fused_launch *f) {
-    if (func != reinterpret_cast<const void *>(&q4_0_ffn_gate_up<NW, SINGLE>)) return false;
-    *f = lev_fused_launch{reinterpret_cast<void *>(&q4_0_ffn_gate_up_and_scores<NW, SINGLE>), 0u, NW * LEV_WAVE, (uint32_t)ffn_lds(NW)};
+bool with_scores(const void *func, lev_ffn_node *n) {
+    void *const both = reinterpret_cast<void *>(&q4_0_ffn_gate_up_and_scores<NW, SINGLE>);
+    if (func != reinterpret_cast<const void *>(&q4_0_ffn_gate_up<NW, SINGLE>) && func != both) return false;
+    n->with_scores = lev_fused_launch{both, 0u, NW * LEV_WAVE, (uint32_t)ffn_lds(NW)};
+    n->with_front = n->with_scores;
+    n->with_front.func = reinterpret_cast<void *>(&q4_0_ffn_norm_gate_up_and_scores<NW, SINGLE>);
     return true;
 }
 }  // namespace
 
 bool lev_ffn_gate_up_node(const void *func, void **args, lev_ffn_node *out) {
-    lev_fused_launch &f = out->with_scores;
-    if (!with_scores<8, true>(func, &f) && !with_scores<8, false>(func, &f) && !with_scores<12, true>(func, &f) &&
-        !with_scores<12, false>(func, &f) && !with_scores<16, true>(func, &f) && !with_scores<16, false>(func, &f))
+    if (!with_scores<8, true>(func, out) && !with_scores<8, false>(func, out) && !with_scores<12, true>(func, out) &&
+        !with_scores<12, false>(func, out) && !with_scores<16, true>(func, out) && !with_scores<16, false>(func, out))
         return false;
     const lev_ffn_args &a = out->args = *static_cast<const lev_ffn_args *>(args[0]);
     const size_t nh = 4u * (size_t)a.hidden, ni = 4u * (size_t)a.inter, w = (size_t)a.inter * (a.hidden / 32u) * 18u;

@@ -1,7 +1,7 @@
 """GPU: a recorded decode step, the shared expert's FFN, the MoE layer on its normalised residual and the norm and residuals
 behind both, gives the bits of the operators called one by one on every replay, and replays as the launches that it is meant
 to: the scores of the router go into the launch of the shared expert's gate/up, its down projection into the layer's, its norm
-into the layer's, unless what the one writes the other touches."""
+into the layer's, that norm and the residuals into the next layer's gate/up, unless what the one writes the other touches."""
 import pytest
 import torch
 
@@ -17,7 +17,7 @@ def q4_0(rows, n, g):
     return w.reshape(-1)
 
 
-@pytest.mark.parametrize("case,launches", [("plain", 4), ("two layers", 8), ("scores of the sum", 7), ("sum not added", 5), ("added twice", 5),
+@pytest.mark.parametrize("case,launches", [("plain", 4), ("two layers", 7), ("two layers on the same buffers", 7), ("norm in front", 4), ("scores of the sum", 7), ("sum not added", 5), ("added twice", 5),
                                            ("part of the sum", 7), ("result is the sum", 5), ("gain is the sum", 5)])
 @pytest.mark.parametrize("hidden,inter,shared,experts,top_k", [
     (2816, 704, 2112, 128, 8), (1024, 256, 512, 32, 2), (4096, 1536, 4096, 256, 8), (1152, 320, 1344, 60, 4), (2048, 768, 1024, 128, 8), (1280, 576, 640, 256, 8),
@@ -30,7 +30,7 @@ def test_recorded_decode_step(hidden, inter, shared, experts, top_k, case, launc
     normal = lambda *s: torch.randn(s, device="cuda", generator=g)
     gu = inter * (hidden // 32) * 18 * experts
     layers = []
-    for _ in range(2 if case == "two layers" else 1):
+    for _ in range(2 if "two" in case else 1):
         pool = torch.cat([q4_0(experts * inter, hidden, g), q4_0(experts * inter, hidden, g), q4_0(experts * hidden, inter, g)])
         layers.append(dict(
             pools=ops.Context.moe_pools(pool, hidden, inter, experts, 0, gu, 2 * gu), pool=pool, router=0.02 * normal(experts, hidden),
@@ -39,10 +39,15 @@ def test_recorded_decode_step(hidden, inter, shared, experts, top_k, case, launc
             bufs=tuple(torch.empty(n, device="cuda") for n in (hidden, 2 * shared, shared, hidden)), y=torch.empty(1, hidden, device="cuda"),
             ids=torch.empty((1, top_k), dtype=torch.int32, device="cuda"), weights=torch.empty(1, top_k, device="cuda"),
             out=torch.empty(hidden, device="cuda")))
-    x0 = normal(hidden)
+    if case == "two layers on the same buffers":
+        layers[1]["bufs"], layers[1]["y"] = layers[0]["bufs"], layers[0]["y"]
+    x0, before = normal(hidden), normal(2, hidden)
 
     def step():
         x = x0
+        if case == "norm in front":
+            ctx.rmsnorm(before[0], hidden, 1, weight=layers[0]["post"], y=x)
+            ctx.axpy(before[1], x, 1.0, hidden)
         for m in layers:
             h, s = ctx.shared_expert_ffn(x, m["norm"], m["gate"], m["up"], m["down"], m["post"], hidden, shared, bufs=m["bufs"])
             ctx.moe_layer_q4_0(m["pools"], m["router"], (s if case == "scores of the sum" else h)[None], top_k, 1, y=m["y"], ids=m["ids"],
@@ -60,7 +65,7 @@ def test_recorded_decode_step(hidden, inter, shared, experts, top_k, case, launc
 
     def results():
         ctx.sync()
-        return [t.clone() for m in layers for t in (*m["bufs"], m["y"], m["ids"], m["weights"], m["out"])]
+        return [x0.clone()] + [t.clone() for m in layers for t in (*m["bufs"], m["y"], m["ids"], m["weights"], m["out"])]
 
     def wipe():
         for m in layers:
@@ -82,7 +87,7 @@ def test_recorded_decode_step(hidden, inter, shared, experts, top_k, case, launc
         for a, b in zip(results(), want):
             assert torch.equal(a.view(torch.int32), b.view(torch.int32))
     # (the layer's gate/up takes nothing along where the down projection's workgroups do not fit the chip beside its own)
-    crowded = len(layers) if hidden == 4096 and case != "scores of the sum" else 0
+    crowded = 2 * len(layers) - 1 + (case == "norm in front") if hidden == 4096 and case != "scores of the sum" else 0
     assert launches_of(prog) == launches + crowded
     prog.destroy()
     ctx.close()
