@@ -37,8 +37,9 @@
 // activations take 64 KB of LDS).  The waves of a workgroup share 16 weight rows,
 // one superblock column each; their partial sums meet in LDS.
 //
-// Five to eight columns, or three and more of a row of more than sixteen superblocks: the planes are made
-// once per launch by a small kernel in front (q4k_planes_kernel, below) instead of by every workgroup.
+// Five to eight columns of a matrix of many rows, or three and more of a row of more than sixteen superblocks: the planes are made
+// once per launch by a small kernel in front (q4k_planes_kernel, below) instead of by every workgroup.  Fewer superblocks, most
+// other shapes: a wave makes the planes of the superblock column that it multiplies (OWN, q4k_own_takes).
 //
 // Against 64-bit sums, on normal activations: 5e-8 to 6e-8 (2-norm); the f32 chains of the vector-ALU kernel, which
 // three and more columns of rows wider than 8192 take without planes, leave 1.4e-7.  A value far below the largest of its
@@ -271,7 +272,11 @@ q4k_planes_kernel(const float *__restrict__ x, const float *__restrict__ gain, f
 // sixteen superblocks, so a wave has one superblock column and keeps its A operands in registers; LDS
 // holds the partial sums only.  Rows that are not cut have kernels without the slices' arithmetic: with
 // it 12288 x 4096 takes 16.6 us by five columns and 16.7 by eight, without 15.5 and 16.0.
-template <int NC, bool SHORT, bool PLANES = false, bool SLICED = false>
+// OWN: rows of at most sixteen superblocks: a wave multiplies one superblock column and makes the digits of that one alone, two
+// columns a pass, so no barrier stands between the digits and the products, the operands are kept in registers for
+// all row groups and the mins are taken as with PLANES.  12288 x 4096 by four columns 10.6 us a call with the digits of all
+// superblocks made by all waves, 9.4 like this; by six 15.4 with the planes made in front, 13.4.  The same integers, the same bits.
+template <int NC, bool SHORT, bool PLANES = false, bool SLICED = false, bool OWN = false>
 __global__ void __launch_bounds__(kMThreads)
 q4_k_mfma_gemv(const uint8_t *__restrict__ w, const float *__restrict__ x,
                const float *__restrict__ gain, float eps, float *__restrict__ y, uint32_t cols,
@@ -282,8 +287,8 @@ q4_k_mfma_gemv(const uint8_t *__restrict__ w, const float *__restrict__ x,
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const uint32_t SB = cols >> 8, subs = PLANES ? 0u : cols >> 5;
     uint8_t *dig = smem;
-    double *sxd = reinterpret_cast<double *>(smem + L::dig_bytes(subs));
-    double *part = sxd + (size_t)subs * NL;
+    double *sxd = reinterpret_cast<double *>(smem + (OWN ? 512u * subs : L::dig_bytes(subs)));
+    double *part = sxd + (OWN ? 0u : (size_t)subs * NL);
     double *psb = part + (size_t)pb * kMWaves * 16u * NL;
     double *s_inv = psb + (size_t)SB * NL;
     uint32_t *s_bad = reinterpret_cast<uint32_t *>(s_inv + NL);
@@ -298,7 +303,9 @@ q4_k_mfma_gemv(const uint8_t *__restrict__ w, const float *__restrict__ x,
     const uint32_t slices = SLICED ? gridDim.y : 1u, per_slice = SLICED ? (SB + slices - 1u) / slices : SB;
     const uint32_t sb0 = SLICED ? blockIdx.y * per_slice : 0u;            // the slice's superblocks
     const uint32_t nsb = SLICED && SB - sb0 < per_slice ? SB - sb0 : per_slice;
-    const uint32_t tpr = PLANES ? 1u : (SB + kMWaves - 1u) / kMWaves;    // tasks per row group and wave
+    constexpr bool REG = PLANES || OWN;      // A operands in registers
+    static_assert(!OWN || (!PLANES && NC % 2 == 0), "a wave's lanes take two columns of its superblock at a time");
+    const uint32_t tpr = REG ? 1u : (SB + kMWaves - 1u) / kMWaves;    // tasks per row group and wave
     const uint32_t ntasks = ((ngroups - blockIdx.x + gridDim.x - 1u) / gridDim.x) * tpr;
     // A cursor walks the wave's tasks in order: row group rg (stride gridDim.x),
     // within it superblock wave + 16*t for t < tpr.  A task past the end (or
@@ -357,22 +364,31 @@ q4_k_mfma_gemv(const uint8_t *__restrict__ w, const float *__restrict__ x,
         constexpr int CH = 4;                                   // slots per thread: NC*cols/8 <= 4096
         constexpr uint32_t kLogNC = NC == 8 ? 3u : NC == 4 ? 2u : NC == 2 ? 1u : 0u;
         const uint32_t total_slots = (cols >> 3) * NC;
-        auto slot_of = [&](uint32_t q, uint32_t &c, uint32_t &k8) {
+        auto slot_of = [&](int i, uint32_t &c, uint32_t &k8) {
+            if (OWN) {   // two columns of the wave's superblock a pass
+                c = 2u * (uint32_t)i + (lane >> 5);
+                k8 = (wave << 5) | (lane & 31u);
+                return wave < SB && c < ncol;
+            }
+            const uint32_t q = tid + (uint32_t)i * kMThreads;
             c = (q >> 5) & (NC - 1u);
             k8 = ((q >> (5u + kLogNC)) << 5) | (q & 31u);
             return q < total_slots && c < ncol;
         };
+        auto past = [&](int i) { return OWN ? 2 * i >= NC : (uint32_t)i * kMThreads >= total_slots; };   // workgroup-uniform
         lev_f32x4 va[CH], vb[CH];
         {
             lev_f32x4 ga[CH], gb[CH];
     #pragma unroll
             for (int i = 0; i < CH; ++i) {
-                if ((uint32_t)i * kMThreads >= total_slots) break;   // workgroup-uniform
+                if (past(i)) break;
                 uint32_t c, k8;
-                if (!slot_of(tid + (uint32_t)i * kMThreads, c, k8)) c = 0u, k8 = 0u;
+                if (!slot_of(i, c, k8)) c = 0u, k8 = 0u;
                 const lev_f32x4 *xp = reinterpret_cast<const lev_f32x4 *>(x + (uint64_t)c * cols) + 2u * k8;
                 va[i] = xp[0];
                 vb[i] = xp[1];
+                if (OWN && i != 0) continue;   // (one superblock: one set of gains)
+                if (OWN) k8 = wave < SB ? (wave << 5) | (lane & 31u) : 0u;   // (also where the first pass has no column)
                 const lev_f32x4 *gp = reinterpret_cast<const lev_f32x4 *>(gain ? gain : x) + 2u * k8;
                 ga[i] = gp[0];
                 gb[i] = gp[1];
@@ -383,9 +399,9 @@ q4_k_mfma_gemv(const uint8_t *__restrict__ w, const float *__restrict__ x,
             if (gain) {
     #pragma unroll
                 for (int i = 0; i < CH; ++i) {
-                    if ((uint32_t)i * kMThreads >= total_slots) break;
+                    if (past(i)) break;
                     uint32_t c, k8;
-                    const bool real = slot_of(tid + (uint32_t)i * kMThreads, c, k8);
+                    const bool real = slot_of(i, c, k8);
                     const lev_f32x4 a = va[i], b = vb[i];
                     double ss = (double)a.x * (double)a.x;
                     ss = fma((double)a.y, (double)a.y, ss); ss = fma((double)a.z, (double)a.z, ss);
@@ -421,23 +437,23 @@ q4_k_mfma_gemv(const uint8_t *__restrict__ w, const float *__restrict__ x,
                 lev_barrier_lds();   // the sums (in the digit area) are dead from here
     #pragma unroll
                 for (int i = 0; i < CH; ++i) {
-                    if ((uint32_t)i * kMThreads >= total_slots) break;
+                    if (past(i)) break;
                     uint32_t c, k8;
-                    const bool real = slot_of(tid + (uint32_t)i * kMThreads, c, k8);
+                    const bool real = slot_of(i, c, k8);
                     const double inv = s_inv[real ? c : 0u];
     #pragma unroll
                     for (int k = 0; k < 4; ++k) {
-                        va[i][k] = (float)((double)va[i][k] * inv) * ga[i][k];
-                        vb[i][k] = (float)((double)vb[i][k] * inv) * gb[i][k];
+                        va[i][k] = (float)((double)va[i][k] * inv) * ga[OWN ? 0 : i][k];
+                        vb[i][k] = (float)((double)vb[i][k] * inv) * gb[OWN ? 0 : i][k];
                     }
                 }
             }
         }
     #pragma unroll
         for (int i = 0; i < CH; ++i) {
-            if ((uint32_t)i * kMThreads >= total_slots) break;
+            if (past(i)) break;
             uint32_t c, k8;
-            const bool real = slot_of(tid + (uint32_t)i * kMThreads, c, k8);
+            const bool real = slot_of(i, c, k8);
             const lev_f32x4 a = va[i], b = vb[i];
             const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
             // largest magnitude of the superblock as an integer: NaN and infinity sort above every number
@@ -481,23 +497,45 @@ q4_k_mfma_gemv(const uint8_t *__restrict__ w, const float *__restrict__ x,
                 dw[2][h] = __builtin_amdgcn_perm(t3, t1, 0x05040100u);
                 dw[3][h] = __builtin_amdgcn_perm(t3, t1, 0x07060302u);
             }
-            sum += __builtin_amdgcn_update_dpp(0, sum, 0xB1, 0xF, 0xF, true);   // 32 values of at most 2^25
-            sum += __builtin_amdgcn_update_dpp(0, sum, 0x4E, 0xF, 0xF, true);
+            if constexpr (!OWN) {
+                sum += __builtin_amdgcn_update_dpp(0, sum, 0xB1, 0xF, 0xF, true);   // 32 values of at most 2^25
+                sum += __builtin_amdgcn_update_dpp(0, sum, 0x4E, 0xF, 0xF, true);
+            }
             if (real) {
                 const uint32_t j = k8 >> 2, kg = k8 & 3u;       // sub-block, k-group
                 // 16-byte unit u = 8*kg + (A row)/2 of the sub-block's 512 bytes, stored at q4k_unit(u, kg, j)
-                uint8_t *blk = dig + ((size_t)j * NX + (c >> 2)) * 512u;
+                uint8_t *blk = dig + (OWN ? (size_t)j : (size_t)j * NX + (c >> 2)) * 512u;
                 const uint32_t u = 8u * kg + 2u * (c & 3u);
                 *reinterpret_cast<lev_u4 *>(blk + q4k_unit(u, kg, j)) = lev_u4{dw[3][0], dw[3][1], dw[2][0], dw[2][1]};
                 *reinterpret_cast<lev_u4 *>(blk + q4k_unit(u + 1u, kg, j)) = lev_u4{dw[1][0], dw[1][1], dw[0][0], dw[0][1]};
-                if (kg == 3u) sxd[((j >> 3) * NL + c) * 8u + (j & 7u)] = (double)sum;
+                if (!OWN && kg == 3u) sxd[((j >> 3) * NL + c) * 8u + (j & 7u)] = (double)sum;
                 if ((k8 & 31u) == 31u) psb[(j >> 3) * NL + c] = __hiloint2double((int)((ex + 872u) << 20), 0);   // 2^(ex-151)
+            }
+            if constexpr (OWN) {
+                if ((i & 1) == 0 && 2 * i + 2 < NC) continue;
+                // Four columns' digits are there (or the last ones'): into registers, the next four take their place.  LDS
+                // runs a wave's accesses in order, the fences only keep the compiler from moving them.
+                const int q = i >> 1;
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                const uint32_t sbw = wave < SB ? wave : SB - 1u;
+                const uint8_t *ablk = dig + (size_t)sbw * 8u * 512u;
+                const uint32_t aoff = q4k_unit(8u * g + (r >> 1), g, 0u) + 8u * (r & 1u);
+#pragma unroll
+                for (int jp = 0; jp < 4; ++jp) {
+                    const lev_u2 lo = *reinterpret_cast<const lev_u2 *>(ablk + 1024u * jp + aoff),
+                                 hi = *reinterpret_cast<const lev_u2 *>(ablk + 1024u * jp + 512u + (aoff ^ 32u));
+                    Areg[jp][q] = lev_i4{(int)lo.x, (int)lo.y, (int)hi.x, (int)hi.y};
+                }
+                pwreg[q] = wave < SB ? psb[sbw * NL + 4u * (uint32_t)q + g] : 0.0;
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
             }
         }
         // columns of the layout beyond ncol hold no data: the lanes that read them
         // only feed outputs that are never stored
-        lev_barrier_lds();
-
+        if constexpr (!OWN) lev_barrier_lds();
     }
     // ---- stream the weights ----
     uint32_t *count = reinterpret_cast<uint32_t *>(reinterpret_cast<uint64_t>(x) + q4k_count_at(SB, NX));
@@ -528,7 +566,7 @@ q4_k_mfma_gemv(const uint8_t *__restrict__ w, const float *__restrict__ x,
             E[q][0] = E[q][1] = E[q][2] = E[q][3] = 0;
             acc2[q] = 0.0;
             M[q] = lev_i4{0, 0, 0, 0};
-            if constexpr (PLANES) {
+            if constexpr (REG) {
                 pw[q] = pwreg[q];
             } else {
                 const uint32_t m = sb * NL + 4u * q + g;
@@ -555,7 +593,7 @@ q4_k_mfma_gemv(const uint8_t *__restrict__ w, const float *__restrict__ x,
 #pragma unroll
             for (int q = 0; q < NX; ++q) {
                 long A;
-                if constexpr (PLANES) {
+                if constexpr (REG) {
                     const lev_i4 a4 = Areg[j >> 1][q];
                     A = __builtin_bit_cast(long, (j & 1) ? lev_u2{(uint32_t)a4.z, (uint32_t)a4.w} : lev_u2{(uint32_t)a4.x, (uint32_t)a4.y});
                 } else {
@@ -568,9 +606,9 @@ q4_k_mfma_gemv(const uint8_t *__restrict__ w, const float *__restrict__ x,
                     E[q][p] += __mul24(D[p], sc);
                     asm("" : "+v"(E[q][p]));   // one multiply-add per plane: keeps the sums from being regrouped
                 }
-                if constexpr (!PLANES) acc2[q] = fma(mnd, SX[q][j >> 1][j & 1], acc2[q]);
+                if constexpr (!REG) acc2[q] = fma(mnd, SX[q][j >> 1][j & 1], acc2[q]);
             }
-            if constexpr (PLANES) {
+            if constexpr (REG) {
                 if (j & 1) {
                     // the mins of sub-blocks j - 1 and j in every B byte of their halves of a 64-deep product:
                     // the sum over the pair of m * (sum of the sub-block's digits), per plane (below 2^21 over
@@ -594,7 +632,7 @@ q4_k_mfma_gemv(const uint8_t *__restrict__ w, const float *__restrict__ x,
             const double hi = fma((double)E[q][0], 256.0, (double)E[q][1]);
             const double lo = fma((double)E[q][2], 256.0, (double)E[q][3]);
             const double dot = fma(hi, 65536.0, lo);
-            if constexpr (PLANES) {
+            if constexpr (REG) {
                 const double mhi = fma((double)M[q][0], 256.0, (double)M[q][1]);
                 const double mlo = fma((double)M[q][2], 256.0, (double)M[q][3]);
                 acc2[q] = fma(mhi, 65536.0, mlo);
@@ -1063,15 +1101,17 @@ size_t q4k_lds_limit(const lev_ctx *ctx) {
                                                                             : ctx->props.sharedMemPerBlock;
 }
 
-template <int NC, bool SHORT>
+template <int NC, bool SHORT, bool OWN = false>
 hipError_t launch_mfma_variant(lev_ctx *ctx, const uint8_t *w, const float *x, const float *gain, float eps,
                        float *y, uint32_t cols, uint32_t rows, uint32_t ncol) {
-    const uint32_t pb = q4k_mfma_lds_bytes(cols, NC, 2u) <= q4k_lds_limit(ctx) ? 2u : 1u;
-    const size_t lds = q4k_mfma_lds_bytes(cols, NC, pb);
-    if (hipError_t e = lev_allow_lds(ctx, reinterpret_cast<const void *>(&q4_k_mfma_gemv<NC, SHORT>), lds); e != hipSuccess) return e;
+    constexpr uint32_t NL = NC > 4 ? 8u : 4u;
+    const uint32_t pb = OWN || q4k_mfma_lds_bytes(cols, NC, 2u) <= q4k_lds_limit(ctx) ? 2u : 1u;
+    const size_t lds = OWN ? (cols >> 5) * 512u + pb * kMWaves * 16u * NL * 8u + (cols >> 8) * NL * 8u + NL * 12u   // 97 KB at most
+                           : q4k_mfma_lds_bytes(cols, NC, pb);
+    if (hipError_t e = lev_allow_lds(ctx, reinterpret_cast<const void *>(&q4_k_mfma_gemv<NC, SHORT, false, false, OWN>), lds); e != hipSuccess) return e;
     uint32_t groups = (rows + 15u) / 16u;
     uint32_t blocks = groups < (uint32_t)ctx->num_cus ? groups : (uint32_t)ctx->num_cus;
-    hipLaunchKernelGGL((q4_k_mfma_gemv<NC, SHORT>), dim3(blocks), dim3(kMThreads), lds, ctx->stream, w,
+    hipLaunchKernelGGL((q4_k_mfma_gemv<NC, SHORT, false, false, OWN>), dim3(blocks), dim3(kMThreads), lds, ctx->stream, w,
                        x, gain, eps, y, cols, rows, ncol, pb, 1.0 / (double)cols);
     return hipGetLastError();
 }
@@ -1085,6 +1125,28 @@ hipError_t launch_mfma(lev_ctx *ctx, const uint8_t *w, const float *x, const flo
     const uint32_t most = ((groups + blocks - 1u) / blocks) * tpr;   // tasks of the busiest wave
     if (most <= 3u) return launch_mfma_variant<NC, true>(ctx, w, x, gain, eps, y, cols, rows, ncol);
     return launch_mfma_variant<NC, false>(ctx, w, x, gain, eps, y, cols, rows, ncol);
+}
+
+template <int NC>
+hipError_t launch_own(lev_ctx *ctx, const uint8_t *w, const float *x, const float *gain, float eps, float *y, uint32_t cols,
+                      uint32_t rows, uint32_t ncol) {
+    if constexpr (NC <= 4)
+        if ((rows + 15u) / 16u > 3u * (uint32_t)ctx->num_cus) return launch_mfma_variant<NC, false, true>(ctx, w, x, gain, eps, y, cols, rows, ncol);
+    return launch_mfma_variant<NC, true, true>(ctx, w, x, gain, eps, y, cols, rows, ncol);
+}
+
+// Whether the waves make the digits of their own superblock column each (us, recorded, for what took the shape before and for
+// this).  Two columns: always (12288 x 4096 10.3, 9.9; 1491 x 2048 5.5, 5.1).  Three and four: rows of more than eight superblocks (12288
+// x 4096 11.6, 10.4; 1200 x 2304 7.0, 6.2); of fewer, half of the waves have none to make and all sixteen make them faster
+// together (6000 x 2048 7.06, 7.12, 3677 x 1024 5.6, 5.9).  Five and more, which had the planes made in front: three rounds of
+// row groups at most, more have no registers for their weights beside two sets of operands (32768 x 4096 by six 28.5, 38.6); by
+// five and six always (12288 x 4096 15.4, 13.4; 500 x 2560 8.5, 7.7), by seven and eight up to eight superblocks and from
+// two rounds on (12288 x 4096 15.8, 14.8; 1491 x 2048 9.06, 8.77; but 3000 x 3584 9.6, 10.0).
+bool q4k_own_takes(const lev_ctx *ctx, uint32_t cols, uint32_t rows, uint32_t ncol) {
+    const uint32_t groups = (rows + 15u) / 16u, cus = (uint32_t)ctx->num_cus;
+    if (cols > 256u * kMWaves || ncol < 2u || ncol > 8u) return false;
+    if (ncol <= 4u) return ncol == 2u || cols > 2048u;
+    return groups <= 3u * cus && (ncol <= 6u || cols <= 2048u || groups > cus);
 }
 
 constexpr uint32_t kMaxMerged = 4096u;   // row groups a workgroup can merge: a flag each in the LDS of the partial sums
@@ -1138,8 +1200,7 @@ uint32_t q4k_planes_min_cols() {
     return v;
 }
 
-// Rows of at most sixteen superblocks: from five columns on (four: staged by every workgroup 10.6 us, with the
-// planes in front 11.4, 12288 x 4096).  Wider ones: as soon as the kernel that stages for itself needs a second
+// Rows of at most sixteen superblocks: from five columns on, where q4k_own_takes leaves them.  Wider ones: as soon as the kernel that stages for itself needs a second
 // launch (4352 x 16000, four columns: 19.4 us with it, 21.4 with the planes in front).
 bool q4k_planes_serves(const lev_ctx *ctx, uint32_t cols, uint32_t rows, uint32_t ncol) {
     const uint32_t from = q4k_planes_min_cols();
@@ -1250,6 +1311,13 @@ hipError_t lev_q4_k_mfma_gemv_launch(lev_ctx *ctx, const uint8_t *w, const float
     if (ncol <= lev_q4_k_mfma_narrow_cols(ctx, in_dim) && (ncol == 1u || lev_q4_k_mfma_cols(ctx, in_dim) < ncol)) {
         if (ncol > 1) return launch_narrow<2>(ctx, w, x, gain, eps, y, in_dim, rows, ncol);
         return launch_narrow<1>(ctx, w, x, gain, eps, y, in_dim, rows, ncol);
+    }
+    static const bool planes_named = getenv("LEV_Q4K_PLANES") != nullptr;   // (then its line holds)
+    if (q4k_own_takes(ctx, in_dim, rows, ncol) && !(planes_named && q4k_planes_serves(ctx, in_dim, rows, ncol))) {
+        if (ncol > 6u) return launch_own<8>(ctx, w, x, gain, eps, y, in_dim, rows, ncol);
+        if (ncol > 4u) return launch_own<6>(ctx, w, x, gain, eps, y, in_dim, rows, ncol);
+        if (ncol > 2u) return launch_own<4>(ctx, w, x, gain, eps, y, in_dim, rows, ncol);
+        return launch_own<2>(ctx, w, x, gain, eps, y, in_dim, rows, ncol);
     }
     if (q4k_planes_serves(ctx, in_dim, rows, ncol)) {
         const hipError_t e = launch_planes(ctx, w, x, gain, eps, y, in_dim, rows, ncol);

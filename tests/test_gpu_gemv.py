@@ -696,6 +696,27 @@ def test_q4_k_one_column_kernel_shapes(ctx, rows, cols):
     assert np.isnan(q4k_gemv(ctx, w, xb, rows, cols, 1, gain)).all()
 
 
+@pytest.mark.parametrize("rows,cols", [(37, 256), (16, 2048), (37, 2304), (4100, 3584), (4096, 4096), (12305, 2304), (12288, 768)])
+def test_q4_k_digits_of_a_wave_s_own_superblock(ctx, rows, cols):
+    """Two to eight columns of at most sixteen superblocks, at the edges of which kernel makes the digits: fewer waves with
+    work than the workgroup has, an odd column, rows of a part of a group, one to four rounds.  Column c has the same bits
+    whatever the number of columns, and is the oracle's dot product; a NaN stays in its column."""
+    w, x, gain = H.config3(rows, cols, 8, seed=rows % 89 + cols // 256)
+    for g in (gain, None):
+        got = q4k_gemv(ctx, w, x, rows, cols, 8, g)
+        xn = H.rmsnorm_rows(x, g) if g is not None else x
+        for c in (0, 3, 4, 7):
+            assert O.max_rel_err(got[c], O.q4_k_matvec_f64(w, rows, cols, xn[c])) < TOL, c
+        for n in range(2, 8):
+            assert np.array_equal(bits(q4k_gemv(ctx, w, x[:n], rows, cols, n, g)), bits(got[:n])), n
+    for n, c in ((2, 1), (3, 2), (5, 4), (6, 0)):
+        xb = x[:n].copy()
+        xb[c, cols - 3] = np.nan
+        hit, keep = q4k_gemv(ctx, w, xb, rows, cols, n), [k for k in range(n) if k != c]
+        assert np.isnan(hit[c]).all()
+        assert np.array_equal(bits(hit[keep]), bits(got[:n][keep])), n
+
+
 @pytest.mark.parametrize("rows,cols,ncol", [(50, 4096, 8), (33, 3840, 5), (100, 2048, 7), (11205, 512, 6), (16, 768, 8),
                                             (4099, 4096, 8), (1, 256, 5)])
 def test_q4_k_five_to_eight_columns_planes_made_once(ctx, rows, cols, ncol):
