@@ -263,11 +263,13 @@ hipError_t launch(lev_ctx *ctx, const uint8_t *w, const uint16_t *x, float *y, u
 
 // Which of the GEMMs takes a shape, in how many K slices and token tiles of which height: the least of what each would
 // take, from times measured on every plan of 450 shapes a format drawn over 1000 to 32000 rows, 1024 to 12288 columns and
-// 17 to 1024 tokens (us; a step is 64 values of K, t = 32-token tiles a wave; the choice is within 1.2 % of the best on
-// average, 7.5 % in nineteen of twenty).
+// 17 to 1024 tokens (us; a step is 64 values of K, t = 32-token tiles a wave; the choice is within 1.0 % of the best on
+// average, 7 % in nineteen of twenty, and 0.7 % on 120 others a format).
 //   256-token tiles:  a round of workgroups (one per CU), more as it fills the CUs, and X put into order in front;
-//   KW = 1:           a round of up to two workgroups a CU; their steps take 1.8 times those of one alone;
-//   KW = 2, KW = 4:   a round of one a CU, and with S > 1 splits the kernel that adds and its reads and writes.
+//   KW = 1:           a round of up to two workgroups a CU; their steps take 1.8 times those of one alone, a tenth of the
+//                     difference less where hardly any CU has two (3072 x 16536 of Q6_K at 330 tokens 57.7 us, with KW = 2 61.6);
+//   KW = 2, KW = 4:   a round of one a CU, and with S > 1 splits the kernel that adds and its reads and writes; of estimates
+//                     that are alike KW = 4 in splits is the better one in 56 of 71 shapes, by 3 %: 0.95 of its own.
 // Lower token tiles are more workgroups that decode the same weights: what fills the chip where rows alone do not.
 // Beyond 1024 tokens the times of these outgrow the estimates, by 1.1 in the middle and up to 1.4, those of the 256-token
 // tiles hardly do: 1.15 is allowed for that (120 shapes a format of up to 8192 tokens).
@@ -302,7 +304,7 @@ lev_gemm_split_plan lev_gemm_split_choose(const lev_ctx *ctx, bool q6, uint32_t 
         auto wgs_of = [&](uint32_t rows_wg, uint32_t splits) { return 8.0 * std::ceil((rows + rows_wg - 1u) / rows_wg * tok_tiles * splits / 8.0); };
         {
             const double n = wgs_of(128u, 1u), whole = std::floor(n / (2.0 * cus)), rest = n - whole * 2.0 * cus;
-            const double rounds = whole + (rest > 0.0 ? 1.0 : 0.0), pairs = whole + (rest > cus ? 1.0 : 0.0);
+            const double rounds = whole + (rest > 0.0 ? 1.0 : 0.0), pairs = whole + (rest > cus ? 0.9 + 0.1 * (rest - cus) / cus : 0.0);
             offer(long_prompt * (rounds * k1.start + 4.0 * nsb * (k1.step + k1.per_tile * t) * (rounds + k1.full * pairs) + k1.once), 1u, 1u, t);
         }
         if ((rows + 31u) / 32u >= 768u || nsb < 6u) continue;
@@ -312,7 +314,7 @@ lev_gemm_split_plan lev_gemm_split_choose(const lev_ctx *ctx, bool q6, uint32_t 
             for (uint32_t s = 1; s <= 8u && s * kw <= nsb; ++s) {
                 const double n = wgs_of(kw == 2u ? 128u : 64u, s), rounds = std::ceil(n / cus), full = n / (rounds * cus);
                 const double steps = 4.0 * ((nsb + kw * s - 1u) / (kw * s));
-                offer(long_prompt * (rounds * (k.start + steps * (k.step + k.per_tile * t) * (1.0 + k.full * full)) + k.once +
+                offer((kw == 4u && s > 1u ? 0.95 : 1.0) * long_prompt * (rounds * (k.start + steps * (k.step + k.per_tile * t) * (1.0 + k.full * full)) + k.once +
                                      (s > 1u ? k.sum + k.sum_mb * 1e-6 * (s + 1.0) * tokens * rows : 0.0)), kw, s, t);
             }
         }
