@@ -869,6 +869,7 @@ hipError_t front_norms(hipGraph_t graph, const std::vector<hipGraphNode_t> &head
             lev_footprint tt;
             tt.writes[0] = lev_span(front.s, bytes);
             tt.reads[0] = lev_span(front.ws, bytes);
+            if (!tt.apart(ft)) continue;                                   // (the FFN, which would read s as it was before this norm)
             const lev_gemv_args g = arg_of<lev_gemv_args>(u, 10);
             if (!(g.y == front.s && g.rows >= len)) {
                 if (!tt.apart(ut) || !tt.apart(gemv_touches(g))) continue;

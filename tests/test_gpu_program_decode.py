@@ -91,3 +91,73 @@ def test_recorded_decode_step(hidden, inter, shared, experts, top_k, case, launc
     assert launches_of(prog) == launches + crowded
     prog.destroy()
     ctx.close()
+
+
+@pytest.mark.parametrize("what,buffers,launches", [("norm", "own", 8), ("norm", "shared", 8), ("router", "own", 8), ("router", "shared", 11),
+                                                   ("post", "own", 7), ("post", "shared", 7)])
+def test_next_layer_reads_the_shared_sum(what, launches, buffers):
+    """A layer's `shared` as a weight of the next layer's FFN: what that reads is the normalised sum, so the norm stays in
+    front of it, whether the sum is needed behind it (buffers of its own) or the next down projection writes a new one (over the
+    router, in one case, so that the second layer's kernels stay as they are).  As the weight of that layer's post norm the sum is
+    read behind all of this, and the norm goes along."""
+    from leviathan_amd import ops
+    ctx = ops.Context(0, own_stream=True)
+    hidden, inter, shared, experts, top_k = 2816, 704, 512, 32, 4
+    g = torch.Generator(device="cuda").manual_seed(7)
+    normal = lambda *s: torch.randn(s, device="cuda", generator=g)
+    gu = inter * (hidden // 32) * 18 * experts
+    layers = []
+    for _ in range(2):
+        pool = torch.cat([q4_0(experts * inter, hidden, g), q4_0(experts * inter, hidden, g), q4_0(experts * hidden, inter, g)])
+        layers.append(dict(
+            pools=ops.Context.moe_pools(pool, hidden, inter, experts, 0, gu, 2 * gu), pool=pool, router=0.02 * normal(experts, hidden),
+            norm=1 + 0.1 * normal(hidden), gate=q4_0(shared, hidden, g), up=q4_0(shared, hidden, g), down=q4_0(hidden, shared, g),
+            post=1 + 0.1 * normal(hidden), post2=1 + 0.1 * normal(hidden),
+            bufs=[torch.empty(n, device="cuda") for n in (hidden, 2 * shared, shared, hidden)], y=torch.empty(1, hidden, device="cuda"),
+            ids=torch.empty((1, top_k), dtype=torch.int32, device="cuda"), weights=torch.empty(1, top_k, device="cuda"),
+            out=torch.empty(hidden, device="cuda")))
+    first, second = layers
+    if what == "router":                                  # (of its first expert)
+        first["bufs"][3] = second["router"][0]
+    else:
+        second[what] = first["bufs"][3]
+    if buffers == "shared":
+        second["bufs"][3] = first["bufs"][3]
+    x0 = normal(hidden)
+
+    def step():
+        x = x0
+        for m in layers:
+            h, s = ctx.shared_expert_ffn(x, m["norm"], m["gate"], m["up"], m["down"], m["post"], hidden, shared, bufs=tuple(m["bufs"]))
+            ctx.moe_layer_q4_0(m["pools"], m["router"], h[None], top_k, 1, y=m["y"], ids=m["ids"], weights=m["weights"])
+            ctx.rmsnorm(m["y"], hidden, 1, weight=m["post2"], y=m["out"])
+            ctx.axpy(s, m["out"], 1.0, hidden)
+            ctx.axpy(x, m["out"], 1.0, hidden)
+            x = m["out"]
+
+    def results():
+        ctx.sync()
+        return [t.clone() for m in layers for t in (*m["bufs"], m["y"], m["ids"], m["weights"], m["out"])]
+
+    def wipe():
+        for m in layers:
+            for t in (*m["bufs"], m["y"], m["weights"], m["out"]):
+                t.fill_(float("nan"))
+            m["ids"].fill_(-1)
+        torch.cuda.synchronize()
+
+    wipe()
+    step()
+    want = results()
+    torch.cuda.synchronize()
+    ctx.program_begin()
+    step()
+    prog = ctx.program_end()
+    for _ in range(3):
+        wipe()
+        prog.run()
+        for a, b in zip(results(), want):
+            assert torch.equal(a.view(torch.int32), b.view(torch.int32))
+    assert launches_of(prog) == launches
+    prog.destroy()
+    ctx.close()
