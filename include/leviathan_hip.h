@@ -265,7 +265,8 @@ int lev_hip_axpy(lev_ctx *ctx, const float *d_x, float *d_y, float c, uint32_t n
  * (h hidden floats, gu 2*inter, act inter, shared hidden); either norm weight may be NULL.  Gate and up are
  * [inter, hidden], down [hidden, inter], Q4_0, each from the start of its buffer.  Buffers may share memory wherever
  * the operators one after the other allow it (act over x, h or gu, say): such a call takes them one after the other,
- * six launches instead of three, unless act is just a half of gu. */
+ * six launches instead of three, unless act is just a half of gu.  With inter below 1280 and no multiple of 256 the
+ * down projection adds in another order than lev_hip_q4_0_gemv called for it: more exact, not the same bits. */
 int lev_hip_shared_expert_ffn_q4_0(lev_ctx *ctx, const float *d_x, const float *d_ffn_norm, const void *d_gate_w,
                                    size_t gate_bytes, const void *d_up_w, size_t up_bytes, const void *d_down_w,
                                    size_t down_bytes, const float *d_post_norm, float eps, float *d_h, float *d_gu,

@@ -304,21 +304,21 @@ __device__ __forceinline__ void lev_row_spread(const lev_u32x4 v, lev_f32x4 (&ou
     }
 }
 
-// Largest of an unsigned value over the 16 lanes of a row of the wave, in every lane of the row:
-// quad swaps, then the two row mirrors (DPP: no LDS, no other unit).  Magnitudes of floats
+// Largest of an unsigned value over the 8 lanes of a half row of the wave, or the 16 of a row, in every lane of it:
+// quad swaps, then the row mirrors (DPP: no LDS, no other unit).  Magnitudes of floats
 // compare as their bit patterns do; NaN and infinity sort above every number.
+template <int CTRL>
+__device__ __forceinline__ uint32_t lev_dpp_max_u32(uint32_t v) {
+    const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, 0xF, 0xF, false);
+    return o > v ? o : v;
+}
+__device__ __forceinline__ uint32_t lev_row8_max_u32(uint32_t v) {
+    v = lev_dpp_max_u32<0xB1>(v);    // quad_perm [1,0,3,2]
+    v = lev_dpp_max_u32<0x4E>(v);    // quad_perm [2,3,0,1]
+    return lev_dpp_max_u32<0x141>(v);   // row_half_mirror
+}
 __device__ __forceinline__ uint32_t lev_row16_max_u32(uint32_t v) {
-#define LEV_ROW16_MAX_STEP(CTRL)                                                                        \
-    {                                                                                                   \
-        const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, 0xF, 0xF, false); \
-        v = o > v ? o : v;                                                                              \
-    }
-    LEV_ROW16_MAX_STEP(0xB1)    // quad_perm [1,0,3,2]
-    LEV_ROW16_MAX_STEP(0x4E)    // quad_perm [2,3,0,1]
-    LEV_ROW16_MAX_STEP(0x141)   // row_half_mirror
-    LEV_ROW16_MAX_STEP(0x140)   // row_mirror
-#undef LEV_ROW16_MAX_STEP
-    return v;
+    return lev_dpp_max_u32<0x140>(lev_row8_max_u32(v));   // row_mirror
 }
 
 // The same over all 64 lanes: the four rows' maxima meet by two row swaps.

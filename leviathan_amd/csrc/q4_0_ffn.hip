@@ -306,7 +306,8 @@ extern "C" int lev_hip_shared_expert_ffn_q4_0(lev_ctx *ctx, const float *d_x, co
     if (st == LEV_OK)
         // narrow rows of the down projection on the matrix cores too: as a launch the two kernels are alike (3968 x 1216 12.1 us
         // a call and 10.5, others 0 to 6 %), but the MoE layer's gate/up takes this one along in recorded programs, 94 us and 72
-        // for four layers of 1664 / 320 and 1216; the error against 64 bits is less than half (rms 1.9e-7 and 7.4e-8)
+        // for four layers of 1664 / 320 and 1216; the error against 64 bits is less than half (rms 1.9e-7 and 7.4e-8), beside
+        // outliers a hundredth (q4_0_mfma.hpp)
         st = lev_hip_check(ctx, lev_q4_0_gemv_launch(ctx, static_cast<const uint8_t *>(d_down_w), d_act, d_shared, inter, hidden, true),
                            "shared_expert_ffn down launch");
     if (st == LEV_OK) st = lev_hip_rmsnorm(ctx, d_shared, d_shared, hidden, 1, d_post_norm, eps);

@@ -11,16 +11,19 @@
 // register p of lane (r, g) is the plane-p sum of that lane's own codes: nothing is exchanged
 // between lanes until a row's four lane groups add their finished pair sums.
 //
-// Activations: per pair of blocks (64 values) x becomes integers X = rint(x * 2^(156 - ex)),
-// |X| <= 2^30, ex the biased exponent of the pair's largest magnitude: every value within 2^-6 of
+// Activations: per block (32 values) x becomes integers X = rint(x * 2^(156 - ex)),
+// |X| <= 2^30, ex the biased exponent of the block's largest magnitude: every value within 2^-6 of
 // that maximum is represented exactly.  X is cut into four balanced base-256 digits (the bytes of
 // (X + 0x808080) ^ 0x808080 read as int8).  The integer sums are exact; a block's planes are
 // recombined and scaled by d in f32, so what is rounded is one number per block of 32 weights.
 //
 // Against 64-bit sums, on normal activations: 6e-8 to 8e-8 (2-norm) over rows of 480 to 8000 values, where the f32
 // chains of the vector-ALU kernels leave 2.0e-7 to 3.3e-7.  What the integers do not have is f32's range: a value far
-// below the largest of its 64 keeps multiples of 2^-31 of that maximum, which is all that a row has where the weight of
-// the maximum is zero, and below a maximum of 2^-93 the unit stays 2^-123.
+// below the largest of its block keeps multiples of 2^-31 of that maximum.  Where the block has a scale the maximum costs the
+// chains more, which add n * x and take 8 * x off in the end: an outlier of 2^13 in every other block that meets the code of
+// zero leaves 3.2e-4 with them (1216 values) and 3e-6 here.  Where the scale is zero the block adds nothing in either, which
+// is why the power of two is a block's and not a pair's: with one for 64 values the pair's other block was 5e-6 off beside
+// 2^13 and lost beside 2^31.  Below a maximum of 2^-93 the unit stays 2^-123.
 //
 // A wave stages the 256 activations of its own task by itself (one float4 per lane, a 1 KB area
 // of LDS nobody else touches): no workgroup barrier stands between the activations and the
@@ -48,18 +51,22 @@ __host__ inline bool lev_q4_0_mfma_in_dim(uint32_t in_dim) {
 constexpr uint32_t kQ4mTaskArea = 1024u;   // LDS bytes of one staged task: [pair 4][plane 4][half 4][16 B]
 constexpr uint32_t kQ4mZeroBytes = 16u;    // what the lanes outside a row's own lane group read as their A operand
 
-// A operands of one task (four halves: block A low / high nibbles, block B low / high) and the
-// power of two that undoes the scaling of the lane's own pair (and the 16 of the codes).
+// The powers of two that undo the scaling of the two blocks of the lane's own pair (and the 16 of the codes), but for 2^8: a
+// block's sum with its power is finite as long as the activations are.
+struct q4m_unscale {
+    float a, b;
+};
+// A operands of one task (four halves: block A low / high nibbles, block B low / high).
 struct q4m_operand {
     lev_i32x4 a[4];
-    float unscale;
+    q4m_unscale unscale;
 };
 
 // Stages the task whose activations are v (lane i holds elements 4i..4i+3 of the task's 256)
 // into `area` (kQ4mTaskArea bytes, this wave's own); returns the lane's `unscale`.  live == false: the
-// task lies beyond the row (it adds nothing).  A NaN or an infinity among the 64 activations of a pair
-// makes the pair's factor NaN, and with it every row's sum.
-__device__ __forceinline__ float q4m_stage_planes(const lev_f32x4 v, uint8_t *area, bool live) {
+// task lies beyond the row (it adds nothing).  A NaN or an infinity among the 32 activations of a block
+// makes the block's factor NaN, and with it every row's sum.
+__device__ __forceinline__ q4m_unscale q4m_stage_planes(const lev_f32x4 v, uint8_t *area, bool live) {
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t r = lane & 15u, g = lane >> 4;
     uint32_t mb = 0u;
@@ -68,12 +75,11 @@ __device__ __forceinline__ float q4m_stage_planes(const lev_f32x4 v, uint8_t *ar
         const uint32_t bits = __float_as_uint(v[k]) & 0x7FFFFFFFu;
         mb = bits > mb ? bits : mb;
     }
-    mb = lev_row16_max_u32(mb);   // the 16 lanes of a pair hold the pair's maximum
+    mb = lev_row8_max_u32(mb);    // the 8 lanes of a block hold the block's maximum
     uint32_t ex = mb >> 23;                                    // |x| < 2^(ex - 126)
     const bool bad = ex == 255u;
     ex = ex < 34u ? 34u : (ex > 254u ? 254u : ex);             // keeps both powers of two normal numbers
     const float scale = __uint_as_float((283u - ex) << 23);    // 2^(156 - ex): |x * scale| < 2^30
-    const float unscale = !live ? 0.f : bad ? __builtin_nanf("") : __uint_as_float((ex - 33u) << 23);   // 2^(ex - 160)
     uint32_t Y[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) Y[k] = ((uint32_t)(int)rintf(v[k] * scale) + 0x00808080u) ^ 0x00808080u;
@@ -96,7 +102,9 @@ __device__ __forceinline__ float q4m_stage_planes(const lev_f32x4 v, uint8_t *ar
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    return unscale;
+    // 2^(ex - 168), from 2^-134 on, of the lane's block; the pair's two from lanes 0 and 8 of its 16
+    const uint32_t own = __float_as_uint(!live ? 0.f : bad ? __builtin_nanf("") : __uint_as_float((ex - 33u) << 23) * 0x1p-8f);
+    return q4m_unscale{lev_row_bcast<0>(own), lev_row_bcast<8>(own)};
 }
 
 // The lane's A operands of a staged task.  `zero` points at kQ4mZeroBytes of zeros: what a lane outside the
@@ -189,5 +197,5 @@ __device__ __forceinline__ float q4m_task_dot(const uint32_t W[9], const q4m_ope
     // |plane sum| <= 32 * 128 * 128 = 2^19: two planes recombine in 32 bits, the halves in f32
     const float fa = fmaf((float)(sa[2] + (sa[3] << 8)), 65536.0f, (float)(sa[0] + (sa[1] << 8)));
     const float fb = fmaf((float)(sb[2] + (sb[3] << 8)), 65536.0f, (float)(sb[0] + (sb[1] << 8)));
-    return fmaf(da, fa, db * fb) * op.unscale;
+    return fmaf(da, fa * op.unscale.a, db * (fb * op.unscale.b)) * 256.0f;
 }

@@ -112,7 +112,7 @@ __device__ __forceinline__ void q4m_gemv(const uint8_t *__restrict__ w, const fl
     // more than two tasks' operands do not fit the registers: a product reads them again
     constexpr bool kKept = TPW <= 2;
     q4m_operand op[kKept ? TPW : 1];
-    float unscale[TPW];
+    q4m_unscale unscale[TPW];
 #pragma unroll
     for (int t = 0; t < TPW; ++t) {
         const bool live = active && t_first + t < ntask;
