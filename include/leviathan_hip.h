@@ -228,7 +228,11 @@ int lev_hip_swiglu_quant_q8(lev_ctx *ctx, const float *d_gate, const float *d_up
  * q4k gemm blocked, lev-forge/src/coopmat.rs:236-323) ----
  * x is fp16 [tokens][in_dim], y is f32 [tokens][rows]; W is dequantised to
  * fp16 tiles in LDS and multiplied on the matrix cores, f32 accumulate.
- * in_dim at most 4194304, tokens at most 1048576 (LEV_ERR_BAD_DIMENSIONS beyond). */
+ * in_dim at most 4194304, tokens at most 1048576 (LEV_ERR_BAD_DIMENSIONS beyond).
+ * Long prompts put x into the matrix cores' order first, into scratch of x's size, short ones may keep partial sums
+ * there (up to eight times y): the context's scratch, which grows with the largest call (a wait for the stream and an
+ * allocation) and is given back with the context.  Without memory for it, or while a program is being recorded that
+ * found less, kernels that need none serve the call, to the same bits. */
 int lev_hip_q4_k_gemm_prefill(lev_ctx *ctx, const void *d_w, size_t w_bytes, uint64_t w_off,
                               const uint16_t *d_x_f16, size_t x_count, float *d_y,
                               size_t y_capacity, uint32_t in_dim, uint32_t rows,

@@ -23,8 +23,11 @@ int lev_fail(lev_ctx *ctx, int status, const char *fmt, ...) {
     return status;
 }
 
+// The runtime keeps a failed call's error until it is fetched, and what fetches it is the check behind the next launch: an
+// error that is reported or answered in another way is taken out here, so that it is not the next call's as well.
 int lev_hip_check(lev_ctx *ctx, hipError_t err, const char *what) {
     if (err == hipSuccess) return LEV_OK;
+    (void)hipGetLastError();
     return lev_fail(ctx, LEV_ERR_COMMAND_FAILED, "%s: %s", what, hipGetErrorString(err));
 }
 
@@ -38,7 +41,7 @@ void *lev_scratch(lev_ctx *ctx, size_t bytes) {
             // a recorded program may hold this address: keep the memory alive
             ctx->retired_scratch.push_back(ctx->scratch);
         } else {
-            if (hipStreamSynchronize(ctx->stream) != hipSuccess) return nullptr;
+            if (hipStreamSynchronize(ctx->stream) != hipSuccess) return nullptr;   // (an error that stays: the stream's)
             (void)hipFree(ctx->scratch);
         }
         ctx->scratch = nullptr;
@@ -46,7 +49,10 @@ void *lev_scratch(lev_ctx *ctx, size_t bytes) {
     }
     size_t want = (bytes + 0xFFFFFu) & ~(size_t)0xFFFFFu;
     void *p = nullptr;
-    if (hipMalloc(&p, want) != hipSuccess) return nullptr;
+    if (hipMalloc(&p, want) != hipSuccess) {
+        (void)hipGetLastError();   // (most callers do without)
+        return nullptr;
+    }
     ctx->scratch = p;
     ctx->scratch_bytes = want;
     return p;
@@ -153,6 +159,7 @@ extern "C" int lev_hip_ctx_destroy(lev_ctx *ctx) {
     if (ctx->d_flag) (void)hipFree(ctx->d_flag);
     if (ctx->h_flag) (void)hipHostFree(ctx->h_flag);
     if (ctx->owns_stream && ctx->stream) (void)hipStreamDestroy(ctx->stream);
+    (void)hipGetLastError();   // (also what ended ctx_create)
     delete ctx;
     return LEV_OK;
 }
@@ -197,9 +204,10 @@ extern "C" int lev_hip_buf_alloc(lev_ctx *ctx, size_t bytes, void **d_out) {
         return lev_fail(ctx, LEV_ERR_EXCEEDS_MAX_BUFFER_LENGTH, "buf_alloc %zu bytes > device %zu",
                         bytes, (size_t)ctx->props.totalGlobalMem);
     hipError_t e = hipMalloc(d_out, bytes);
+    const int st = lev_hip_check(ctx, e, "hipMalloc");
     if (e == hipErrorOutOfMemory)
         return lev_fail(ctx, LEV_ERR_EXCEEDS_WORKING_SET, "buf_alloc %zu bytes: out of memory", bytes);
-    return lev_hip_check(ctx, e, "hipMalloc");
+    return st;
 }
 
 extern "C" int lev_hip_buf_free(lev_ctx *ctx, void *d_ptr) {
@@ -960,6 +968,7 @@ extern "C" int lev_hip_program_end(lev_ctx *ctx, lev_program **out) {
     } catch (const std::bad_alloc &) {   // (its lists of nodes; nothing leaves a C entry as an exception)
         e = hipErrorOutOfMemory;
     }
+    if (e == hipSuccess) (void)hipGetLastError();   // (of a question to the graph that had no answer: the nodes stayed as they were)
     if (e == hipSuccess) e = hipGraphInstantiate(&p->exec, graph, nullptr, nullptr, 0);
     if (e != hipSuccess) {
         (void)hipGraphDestroy(graph);

@@ -1,7 +1,7 @@
 """The C++ host mirror of the Swift operator surface (leviathan_amd/host).
 
 CPU: the parity program compiles against the in-tree headers and libraries and
-lists its cases without touching a device.  GPU: every case passes.
+lists its cases without touching a device; the library against a HIP runtime whose allocations fail.  GPU: every case passes.
 """
 import os
 import subprocess
@@ -18,7 +18,7 @@ CASES = ["q4_backend_2x32", "q4_backend_minus_16", "q4_backend_guards", "q6_back
 
 
 def _built():
-    if not os.path.exists(BIN):
+    if not all(os.path.exists(os.path.join(os.path.dirname(BIN), b)) for b in ("host_parity", "hip_errors")):
         import oracle  # noqa: F401  (builds liblev_oracle.so if missing)
         from leviathan_amd import build as hip_build
         hip_build.build()
@@ -40,3 +40,10 @@ def test_host_mirror_parity_on_gpu():
     assert out.returncode == 0, out.stdout[-2000:]
     for name in CASES:
         assert f"ok {name}" in out.stdout
+
+
+def test_errors_of_hip_calls():
+    """A call that was served in another way, or refused, does not make the next one fail."""
+    _built()
+    out = subprocess.run([os.path.join(os.path.dirname(BIN), "hip_errors")], capture_output=True, text=True, timeout=60)
+    assert out.returncode == 0, out.stdout
