@@ -372,44 +372,34 @@ rmsnorm_adds_kernel(const float *__restrict__ x, float *__restrict__ y, const fl
 }
 
 // Two norms of one length in one launch: x = rmsnorm(x) * wx in place, then what rmsnorm_adds_kernel does with y, of whose
-// addends number `own` is that x (see pair_norms).  One memory round trip for both.
+// addends number `own` is that x (see pair_norms).  One memory round trip for both.  A piece of four values a lane: the length is
+// the width of a MoE layer whose kernels pair_norms knows, 4096 at most.
 struct norm_pair {
     float *x;
     const float *wx;
     float eps;
     int own;
 };
-template <int V>
 __global__ void __launch_bounds__(1024)
 rmsnorm_pair_kernel(norm_pair p, const float *__restrict__ y, float *__restrict__ out, const float *__restrict__ wy, uint32_t n, float eps,
                     norm_adds adds) {
     __shared__ float part[2][16];
-    const uint32_t t = threadIdx.x, nt = blockDim.x, n4 = n >> 2;
+    const uint32_t t = threadIdx.x, nt = blockDim.x, n4 = n >> 2, i = t < n4 ? t : 0u;
     auto vec = [](const float *q) { return reinterpret_cast<const lev_f32x4 *>(q); };
-    lev_f32x4 a[V], b[V], ga[V], gb[V], ad[norm_adds::kMost][V];
+    lev_f32x4 ga, gb, ad[norm_adds::kMost];
+    const lev_f32x4 a = t < n4 ? vec(p.x)[t] : lev_f32x4{0.f, 0.f, 0.f, 0.f};
+    const lev_f32x4 b = t < n4 ? vec(y)[t] : lev_f32x4{0.f, 0.f, 0.f, 0.f};
+    if (p.wx) ga = vec(p.wx)[i];
+    if (wy) gb = vec(wy)[i];
+#pragma unroll
+    for (int m = 0; m < norm_adds::kMost; ++m)
+        if (m < adds.count && m != p.own) ad[m] = vec(adds.x[m])[i];
     float sa = 0.f, sb = 0.f;
 #pragma unroll
-    for (int k = 0; k < V; ++k) {
-        const uint32_t i = t + nt * k;
-        a[k] = i < n4 ? vec(p.x)[i] : lev_f32x4{0.f, 0.f, 0.f, 0.f};
-        b[k] = i < n4 ? vec(y)[i] : lev_f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int c = 0; c < 4; ++c) {
+        sa = fmaf(a[c], a[c], sa);
+        sb = fmaf(b[c], b[c], sb);
     }
-#pragma unroll
-    for (int k = 0; k < V; ++k) {
-        const uint32_t i = t + nt * k < n4 ? t + nt * k : 0u;
-        if (p.wx) ga[k] = vec(p.wx)[i];
-        if (wy) gb[k] = vec(wy)[i];
-#pragma unroll
-        for (int m = 0; m < norm_adds::kMost; ++m)
-            if (m < adds.count && m != p.own) ad[m][k] = vec(adds.x[m])[i];
-    }
-#pragma unroll
-    for (int k = 0; k < V; ++k)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            sa = fmaf(a[k][c], a[k][c], sa);
-            sb = fmaf(b[k][c], b[k][c], sb);
-        }
     sa = lev_wave_sum_broadcast(sa);
     sb = lev_wave_sum_broadcast(sb);
     if ((t & 63u) == 0u) part[0][t >> 6] = sa, part[1][t >> 6] = sb;
@@ -417,23 +407,19 @@ rmsnorm_pair_kernel(norm_pair p, const float *__restrict__ y, float *__restrict_
     double ta = 0.0, tb = 0.0;
     for (uint32_t k = 0; k < nt >> 6; ++k) ta += (double)part[0][k], tb += (double)part[1][k];
     const float ia = (float)lev_rsqrt_f64(ta / (double)n + (double)p.eps), ib = (float)lev_rsqrt_f64(tb / (double)n + (double)eps);
+    lev_f32x4 x = a * ia, o = b * ib;
+    if (p.wx) x = x * ga;
+    if (wy) o = o * gb;
 #pragma unroll
-    for (int k = 0; k < V; ++k) {
-        const uint32_t i = t + nt * k;
-        lev_f32x4 x = a[k] * ia, o = b[k] * ib;
-        if (p.wx) x = x * ga[k];
-        if (wy) o = o * gb[k];
+    for (int m = 0; m < norm_adds::kMost; ++m) {
+        if (m >= adds.count) break;
+        const lev_f32x4 v = m == p.own ? x : ad[m];
 #pragma unroll
-        for (int m = 0; m < norm_adds::kMost; ++m) {
-            if (m >= adds.count) break;
-            const lev_f32x4 v = m == p.own ? x : ad[m][k];
-#pragma unroll
-            for (int c = 0; c < 4; ++c) o[c] = fmaf(adds.c[m], v[c], o[c]);
-        }
-        if (i < n4) {
-            reinterpret_cast<lev_f32x4 *>(p.x)[i] = x;
-            reinterpret_cast<lev_f32x4 *>(out)[i] = o;
-        }
+        for (int c = 0; c < 4; ++c) o[c] = fmaf(adds.c[m], v[c], o[c]);
+    }
+    if (t < n4) {
+        reinterpret_cast<lev_f32x4 *>(p.x)[t] = x;
+        reinterpret_cast<lev_f32x4 *>(out)[t] = o;
     }
 }
 
@@ -773,30 +759,26 @@ hipError_t weave_shared_expert(hipGraph_t graph, const std::vector<hipGraphNode_
 
 // A norm in place, kernels of the MoE layer of one token, and a norm of the same length that adds the first one's result:
 // the first norm goes into the second one's launch where the layer does not touch what it does (the shared expert's norm and
-// the layer's).
+// the layer's; of 4096 values at most, as the layer).
 hipError_t pair_norms(hipGraph_t graph, const std::vector<hipGraphNode_t> &nodes, const lev_ctx *ctx) {
-    void *const adds_kernel[3] = {reinterpret_cast<void *>(&rmsnorm_adds_kernel<1>), reinterpret_cast<void *>(&rmsnorm_adds_kernel<2>),
-                                  reinterpret_cast<void *>(&rmsnorm_adds_kernel<4>)};
-    void *const pair_kernel[3] = {reinterpret_cast<void *>(&rmsnorm_pair_kernel<1>), reinterpret_cast<void *>(&rmsnorm_pair_kernel<2>),
-                                  reinterpret_cast<void *>(&rmsnorm_pair_kernel<4>)};
+    const void *const adds_kernel = reinterpret_cast<const void *>(&rmsnorm_adds_kernel<1>);
     for (hipGraphNode_t first : nodes) {
         node_view n, s;
         hipGraphNode_t behind, last;
-        int kind;
-        if (!kernel_node(first, &n) || (kind = norm_kind(n)) < 0 || arg_of<const float *>(n, 0) != arg_of<float *>(n, 1) ||
+        if (!kernel_node(first, &n) || norm_kind(n) != 0 || arg_of<const float *>(n, 0) != arg_of<float *>(n, 1) ||
             !only_next(first, &behind))
             continue;
         const lev_footprint nt = norm_touches(n);
         bool fits = true;
         last = behind;
-        for (int layer = 0; layer < 3 && kernel_node(last, &s) && s.func != adds_kernel[kind]; ++layer) {   // scores, gate/up, down
+        for (int layer = 0; layer < 3 && kernel_node(last, &s) && s.func != adds_kernel; ++layer) {   // scores, gate/up, down
             lev_footprint t;
             if (s.func == lev_moe_scores_few() && s.params.gridDim.y == 1u) t = scores_touches(s);
             else if (!lev_moe_expert_node(ctx, s.func, s.args, &t)) fits = false;
             fits = fits && nt.apart(t) && only_next(last, &last);
             if (!fits) break;
         }
-        if (!fits || last == behind || !kernel_node(last, &s) || s.func != adds_kernel[kind] || s.params.gridDim.x != 1u ||
+        if (!fits || last == behind || !kernel_node(last, &s) || s.func != adds_kernel || s.params.gridDim.x != 1u ||
             arg_of<uint32_t>(s, 3) != arg_of<uint32_t>(n, 3) || !nt.apart(norm_touches(s)))
             continue;
         norm_adds adds = arg_of<norm_adds>(s, 5);
@@ -812,7 +794,7 @@ hipError_t pair_norms(hipGraph_t graph, const std::vector<hipGraphNode_t> &nodes
         float eps = arg_of<float>(s, 4);
         void *args[7] = {&p, &y, &out, &wy, &len, &eps, &adds};
         size_t nbefore = 0;
-        hipError_t e = become(last, pair_kernel[kind], 1u, s.params.blockDim.x, 0u, args);
+        hipError_t e = become(last, reinterpret_cast<void *>(&rmsnorm_pair_kernel), 1u, s.params.blockDim.x, 0u, args);
         if (e == hipSuccess) e = hipGraphNodeGetDependencies(first, nullptr, &nbefore);
         if (e == hipSuccess && nbefore) {
             std::vector<hipGraphNode_t> before(nbefore);
@@ -912,8 +894,8 @@ hipError_t fuse_nodes(hipGraph_t graph, const lev_ctx *ctx) {
         // the heads of the pattern alone: a fusion destroys nodes that are no heads, or the head itself
         auto is_head = [&](const node_view &v) {
             if (rule == 0) return v.func == lev_q4_0_gemv_one_round();
-            if (rule == 1) return norm_kind(v) >= 0;
-            return v.func == reinterpret_cast<const void *>(&rmsnorm_adds_kernel<1>) || v.func == reinterpret_cast<const void *>(&rmsnorm_pair_kernel<1>);
+            if (rule == 1) return norm_kind(v) == 0;
+            return v.func == reinterpret_cast<const void *>(&rmsnorm_adds_kernel<1>) || v.func == reinterpret_cast<const void *>(&rmsnorm_pair_kernel);
         };
         std::vector<hipGraphNode_t> heads;
         for (hipGraphNode_t node : nodes) {
