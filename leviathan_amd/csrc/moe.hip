@@ -1094,8 +1094,8 @@ __device__ __forceinline__ void gate_up_mfma(const moe_args &a, const float *__r
                 g += pg[192];
                 u += pu[192];
             }
-            g = lev_row_sum_f32(g);
-            u = lev_row_sum_f32(u);
+            g = 0.5f * lev_row_sum_f32(g);
+            u = 0.5f * lev_row_sum_f32(u);
             if (q == 0u && i_here + r16 < i_end) arow[i_here + r16] = lev_gelu_up_value(g, u);
         }
         pw ^= kPart;                                              // the other half of `part` next round
@@ -1134,7 +1134,7 @@ moe_gate_up_mfma(moe_args a, const float *__restrict__ x, const int32_t *ids, co
 
 // The same at one token beside a GEMV that does not depend on it (recorded programs: the shared expert's down projection,
 // which alone on the chip is the launch and little else).  grid (extra + chunks, top_k): the first `extra` workgroups of a
-// slot are the GEMV's, gemv_blocks in all, and one the tail's (the norm of the layer before, if it has one to store).  Two workgroups of 12 or 16 waves a CU, four of 8: 80 and 64 registers (the latter
+// slot are the GEMV's, gemv_blocks in all, and one the tail's (the norm of the layer before, if it has one to store).  Two workgroups of 12 or 16 waves a CU, four of 8: 69 and 64 registers (the latter
 // without the pins of q4m_gemv).
 template <int NW, int ROUTE>
 __global__ void __launch_bounds__(NW * LEV_WAVE, NW / 2)
@@ -1242,9 +1242,10 @@ moe_down_mfma(moe_args a, const float *__restrict__ act, const int32_t *__restri
         for (int k = 0; k < TPW; ++k) {
             uint32_t W[9];
             q4m_turn_task(D[k], W);
-            val += q4m_task_dot(W, op[k]);
+            const float dot = q4m_task_dot(W, op[k]);
+            val = k ? val + dot : dot;
         }
-        val = lev_row_sum_f32(val);
+        val = 0.5f * lev_row_sum_f32(val);
         if (lane < 16u) partial[slot * 16u + lane] = val;
     }
     if (bad && lane == 0) atomicOr(flag, kFlagBadExpertId);

@@ -3,7 +3,8 @@
 //
 // Called operator by operator it is six launches of which four are the launch floor and little else: at
 // 2816 / 2112 18.7 us recorded, 29 us enqueued one by one.  Here three: everything up to act, the down GEMV, the
-// norm behind it (9.3 us recorded, 9.5 enqueued; 9.5 and 9.65 with the only group's weights requested a second time).  The first kernel has the shape of the MoE gate/up kernel: a wave owns one
+// norm behind it (9.1 us recorded; enqueued 9.2 to 9.9, the host's pace; recorded 0.15 more with the only group's weights
+// requested a second time).  The first kernel has the shape of the MoE gate/up kernel: a wave owns one
 // 256-value column task of gate row group i and of up row group i, keeps the operands in registers and
 // meets the others in LDS; in front of it every workgroup normalises x for itself (a wave its own 256 values,
 // the sum of squares crosses the waves once), with its weights already on their way.
@@ -166,8 +167,8 @@ __device__ __forceinline__ void ffn_gate_up(const lev_ffn_args &a, uint8_t *smem
                 g += pg[64 * k];
                 u += pu[64 * k];
             }
-            g = lev_row_sum_f32(g);
-            u = lev_row_sum_f32(u);
+            g = 0.5f * lev_row_sum_f32(g);
+            u = 0.5f * lev_row_sum_f32(u);
             const uint32_t row = i0 + r16;
             if (q == 0u && row < i_end) {
                 a.gu[row] = g;

@@ -51,8 +51,8 @@ __host__ inline bool lev_q4_0_mfma_in_dim(uint32_t in_dim) {
 constexpr uint32_t kQ4mTaskArea = 1024u;   // LDS bytes of one staged task: [pair 4][plane 4][half 4][16 B]
 constexpr uint32_t kQ4mZeroBytes = 16u;    // what the lanes outside a row's own lane group read as their A operand
 
-// The powers of two that undo the scaling of the two blocks of the lane's own pair (and the 16 of the codes), but for 2^8: a
-// block's sum with its power is finite as long as the activations are.
+// Twice the powers of two that undo the scaling of the two blocks of the lane's own pair (and the 16 of the codes): times a
+// scale d of the weights, subnormal ones included, they are exact.
 struct q4m_unscale {
     float a, b;
 };
@@ -102,8 +102,8 @@ __device__ __forceinline__ q4m_unscale q4m_stage_planes(const lev_f32x4 v, uint8
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    // 2^(ex - 168), from 2^-134 on, of the lane's block; the pair's two from lanes 0 and 8 of its 16
-    const uint32_t own = __float_as_uint(!live ? 0.f : bad ? __builtin_nanf("") : __uint_as_float((ex - 33u) << 23) * 0x1p-8f);
+    // 2^(ex - 159) of the lane's block; the pair's two from lanes 0 and 8 of its 16
+    const uint32_t own = !live ? 0u : bad ? 0x7FC00000u : (ex - 32u) << 23;
     return q4m_unscale{lev_row_bcast<0>(own), lev_row_bcast<8>(own)};
 }
 
@@ -174,11 +174,12 @@ __device__ __forceinline__ void q4m_turn_task(const uint32_t D[9], uint32_t W[9]
     for (int k = 0; k < 9; ++k) W[k] = (uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)D[k]);
 }
 
-// Contribution of the lane's pair (W: its 36 bytes, already turned) to its row's dot product.
+// Twice the contribution of the lane's pair (W: its 36 bytes, already turned) to its row's dot product, which is halved where
+// the row's sum ends.
 __device__ __forceinline__ float q4m_task_dot(const uint32_t W[9], const q4m_operand &op) {
     typedef uint32_t u4 __attribute__((ext_vector_type(4)));
-    const float da = lev_f16_bits_to_f32(W[0] & 0xFFFFu);
-    const float db = lev_f16_bits_to_f32(W[4] >> 16);
+    const float da = fmaf(lev_f16_bits_to_f32(W[0] & 0xFFFFu), op.unscale.a, 0.f);   // (converts and multiplies in one)
+    const float db = fmaf(lev_f16_bits_to_f32(W[4] >> 16), op.unscale.b, 0.f);
     u4 qa, qb;
     qa.x = __builtin_amdgcn_alignbit(W[1], W[0], 16);
     qa.y = __builtin_amdgcn_alignbit(W[2], W[1], 16);
@@ -197,5 +198,5 @@ __device__ __forceinline__ float q4m_task_dot(const uint32_t W[9], const q4m_ope
     // |plane sum| <= 32 * 128 * 128 = 2^19: two planes recombine in 32 bits, the halves in f32
     const float fa = fmaf((float)(sa[2] + (sa[3] << 8)), 65536.0f, (float)(sa[0] + (sa[1] << 8)));
     const float fb = fmaf((float)(sb[2] + (sb[3] << 8)), 65536.0f, (float)(sb[0] + (sb[1] << 8)));
-    return fmaf(da, fa * op.unscale.a, db * (fb * op.unscale.b)) * 256.0f;
+    return fmaf(da, fa, db * fb);
 }

@@ -122,6 +122,22 @@ __device__ __forceinline__ void q4m_gemv(const uint8_t *__restrict__ w, const fl
             op[t].unscale = unscale[t];
         }
     }
+    // ODD: without the scale of the neighbour's block, A of the first pair of an odd row, B of the last of an even one (as
+    // requested: lanes and tasks past the row's end repeat its last pair).  Kept as masks over the rounds: seen through, they
+    // become selects between the conversion of a scale and its product, which are one instruction otherwise (30092 x 3168
+    // 11.00 us and 10.86; one round alone is 0.1 of 6.9 us faster without the registers).
+    uint32_t own_a[TPW], own_b[TPW];
+    if (ODD) {
+#pragma unroll
+        for (int t = 0; t < TPW; ++t) {
+            const uint32_t T = t_first + t < ntask ? t_first + t : ntask - 1u;
+            const uint32_t pair = 4u * T + q < npairs ? 4u * T + q : npairs - 1u;
+            own_a[t] = parity && pair == 0u ? 0xFFFF0000u : ~0u;
+            own_b[t] = !parity && pair + 1u == npairs ? 0x0000FFFFu : ~0u;
+            if (!SINGLE) lev_pin(own_a[t]);
+            if (!SINGLE) lev_pin(own_b[t]);
+        }
+    }
     // the operands are read back before the wait for the weights, not behind it
     __builtin_amdgcn_sched_barrier(0);
 
@@ -133,18 +149,15 @@ __device__ __forceinline__ void q4m_gemv(const uint8_t *__restrict__ w, const fl
             uint32_t W[9];
             q4m_turn_task(D[t], W);
             if (ODD) {
-                // the scale of the neighbour's block: A of the first pair of an odd row, B of the last of an even one
-                // (as requested: lanes and tasks past the row's end repeat its last pair)
-                const uint32_t T = t_first + t < ntask ? t_first + t : ntask - 1u;
-                const uint32_t pair = 4u * T + q < npairs ? 4u * T + q : npairs - 1u;
-                W[0] &= parity && pair == 0u ? 0xFFFF0000u : ~0u;
-                W[4] &= !parity && pair + 1u == npairs ? 0x0000FFFFu : ~0u;
+                W[0] &= own_a[t];
+                W[4] &= own_b[t];
             }
             if (!kKept) {
                 q4m_read_operands(area + t * kQ4mTaskArea, zero, active && t_first + t < ntask, op[0]);
                 op[0].unscale = unscale[t];
             }
-            val += q4m_task_dot(W, op[kKept ? t : 0]);
+            const float dot = q4m_task_dot(W, op[kKept ? t : 0]);
+            val = t ? val + dot : dot;
         }
         val = lev_row_sum_f32(val);
         if (lane < 16u) *reinterpret_cast<float *>(smem + pw) = val;
@@ -154,7 +167,7 @@ __device__ __forceinline__ void q4m_gemv(const uint8_t *__restrict__ w, const fl
             const float p0 = pp[0], p1 = pp[64], p2 = pp[128], p3 = pp[192];   // four reads in flight together
             auto keep = [](float p, uint32_t k) { return __uint_as_float(__float_as_uint(p) & k); };
             float s = (keep(p0, k0) + keep(p1, k1)) + (keep(p2, k2) + keep(p3, k3));
-            s = lev_row_sum_f32(s);
+            s = 0.5f * lev_row_sum_f32(s);
             if (stores) *reinterpret_cast<__attribute__((address_space(1))) float *>(yp) = s;   // a global store, not a flat one
         }
         if (!SINGLE) {
