@@ -230,7 +230,7 @@ hipError_t launch_tiles(lev_ctx *ctx, const uint8_t *w, const uint16_t *x, float
     if (splits == 1u) return slices(y, 0u, 1u, false);
     float *const part = static_cast<float *>(lev_scratch(ctx, (size_t)splits * tokens * rows * 4));
     if (!part) {
-        // a program is being recorded and the scratch is still too small: a launch for every slice, each added to y where
+        // no memory, or a program is being recorded and the scratch is still too small: a launch for every slice, each added to y where
         // the others are, in the same order and so to the same bits
         for (uint32_t z = 0; z < splits; ++z)
             if (hipError_t e = slices(y, z, 1u, z != 0u); e != hipSuccess) return e;

@@ -189,8 +189,8 @@ hipError_t launch_as(lev_ctx *ctx, const uint8_t *w, const uint8_t *xf, float *y
     return hipGetLastError();
 }
 
-// plan.splits: row tiles a workgroup.  Without scratch for the fragments of X (a program is being recorded and the context's
-// is still too small) a wave of the kernel for short prompts takes all of K.
+// plan.splits: row tiles a workgroup.  Without scratch for the fragments of X (no memory, or a program is being recorded and the
+// context's is still too small) a wave of the kernel for short prompts takes all of K.
 template <typename W>
 hipError_t launch(lev_ctx *ctx, const uint8_t *w, const uint16_t *x, float *y, uint32_t in_dim, uint32_t rows, uint32_t tokens,
                   const lev_gemm_split_plan &plan) {

@@ -1174,7 +1174,7 @@ q4k_grid q4k_planes_grid(const lev_ctx *ctx, uint32_t cols, uint32_t rows) {
 }
 
 // The planes once per launch (q4k_planes_kernel), then the products.  Returns hipErrorOutOfMemory when the scratch
-// cannot be had (a program is being recorded and the context's scratch is still too small): the caller then takes
+// cannot be had (no memory, or a program is being recorded and the context's scratch is still too small): the caller then takes
 // the kernels that stage for themselves.
 template <int NC, bool SHORT>
 hipError_t launch_planes_variant(lev_ctx *ctx, const uint8_t *w, const uint8_t *scratch, float *y, uint32_t cols,

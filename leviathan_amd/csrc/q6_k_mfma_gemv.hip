@@ -1762,7 +1762,7 @@ hipError_t q6m_q8_one_launch(lev_ctx *ctx, const uint8_t *w, const uint32_t *xq,
     if (held && q6m_q8_staged_is_faster(ctx, g, cols, rows, ncol, held)) return hipErrorNotSupported;
     float *const sums = static_cast<float *>(lev_scratch(ctx, (size_t)g.slices * ncol * rows * 4u));
     if (sums) return q6m_q8_one_launch_grid<NC, kSliced>(ctx, w, xq, xs, y, cols, rows, ncol, g, 0u, sums);
-    // a program is being recorded and the context's scratch is still too small
+    // no memory, or a program is being recorded and the context's scratch is still too small
     for (uint32_t z = 0; z < g.slices; ++z)
         if (hipError_t e = q6m_q8_one_launch_grid<NC, kOneSlice>(ctx, w, xq, xs, y, cols, rows, ncol, g, z, nullptr); e != hipSuccess) return e;
     return hipSuccess;
