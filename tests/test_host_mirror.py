@@ -17,14 +17,14 @@ CASES = ["q4_backend_2x32", "q4_backend_minus_16", "q4_backend_guards", "q6_back
          "runner_moe_hand_computed", "runner_gguf_file", "forge_matvec", "forge_moe_layer"]
 
 
-def _built():
-    if not all(os.path.exists(os.path.join(os.path.dirname(BIN), b)) for b in ("host_parity", "hip_errors")):
+def _built(path=BIN):
+    if not os.path.exists(path):
         import oracle  # noqa: F401  (builds liblev_oracle.so if missing)
         from leviathan_amd import build as hip_build
         hip_build.build()
         subprocess.run(["make", "-C", os.path.join(ROOT, "tests", "host")], check=True,
                        stdout=subprocess.DEVNULL)
-    return BIN
+    return path
 
 
 def test_host_mirror_compiles_and_lists_cases():
@@ -44,6 +44,5 @@ def test_host_mirror_parity_on_gpu():
 
 def test_errors_of_hip_calls():
     """A call that was served in another way, or refused, does not make the next one fail."""
-    _built()
-    out = subprocess.run([os.path.join(os.path.dirname(BIN), "hip_errors")], capture_output=True, text=True, timeout=60)
+    out = subprocess.run([_built(os.path.join(os.path.dirname(BIN), "hip_errors"))], capture_output=True, text=True, timeout=60)
     assert out.returncode == 0, out.stdout
