@@ -22,19 +22,22 @@
 // 3.2; against 64-bit sums the layer's outputs are off by 2.2e-7 (2-norm) at 2816 / 704 and 2.3e-7 at
 // 4096 / 448 where one chain left 3.0e-7 and 3.5e-7 and the kernels that these sizes took before 2.4e-7.
 //
-// Measured: hidden 2816, intermediate 704, top-8 of 128 experts, 1000 tokens: the layer 408 us (402 with one
-// chain a row; 4420 with a workgroup per token and slot, which these sizes took before); 2048 / 768, 1000
-// tokens: 324 us (317; 627 with twelve columns a pass over the weights); 4096 / 448, top-4 of 32, 300 tokens:
-// 111 us (131).
+// What bounds it: instructions.  A unit, 32 x 32 outputs and a block, is 4 v_mfma_f32_32x32x16_f16 (130 clocks of the matrix
+// pipe), 16 multiply-adds by d, 4 fragment reads, and per row 18 instructions of decode shared by the item's column tiles: some
+// 45 in all, and a SIMD's two to four waves issue one per 4.4 to 5 clocks, whatever its kind; over the whole chip the products
+// alone run at 1.45 GHz (92 ns a unit and SIMD, 117 with the rest).  So the loop is written for their number (three buffers
+// of activations, weights read 8 bytes a lane, two codes decoded by three instructions) and for what the others cover: fragments and
+// weights of the next step are read and decoded behind this step's products, requests are issued one behind a product, and
+// a workgroup's start is three dependent trips to memory (nine thousand clocks of a down product's 42 thousand before).
 //
-// What bounds it: per 32 x 32 outputs and block, 4 v_mfma_f32_32x32x16_f16 (128 clocks of the matrix
-// pipe) against 16 multiply-adds by d (some 70 clocks of vector issue) and, shared by a wave's two
-// token tiles, 24 instructions of decode per row tile; the two kinds overlap between the two waves of a
-// SIMD (eight 16x16x32 MFMAs and 32 multiply-adds of four waves: 900 clocks together, 600 and 640
-// alone; four 32x32x16 and the same multiply-adds: 760; hence the larger instruction).
+// Measured (us, the two products, before -> now; 2816 / 704, top-8 of 128 experts): 1000 tokens 231 + 117 -> 208 + 108; 300 tokens
+// 114 + 62 -> 110 + 59; 2048 / 768, 1000 tokens 167 + 89 -> 156 + 82; 1024 / 256, top-4 of 32, 300 tokens 23 + 9.9 -> 18.6 + 8.7;
+// 4096 / 1536, top-6 of 64, 500 tokens 277 + 149 -> 232 + 139; 4096 / 832, top-4 of 128, 420 tokens 205 + 93 -> 186 + 89.
+// Tried and not kept: 64 rows a wave (half the fragment reads: no faster, the registers of two folded tiles spill), items of 96
+// (203 + 113), deeper requests, wave priorities.
 #include "moe_prefill.hpp"
+#include "moe_prefill_plan.hpp"
 
-#include <cmath>
 #include <type_traits>
 
 namespace {
@@ -43,13 +46,10 @@ typedef _Float16 p_h8 __attribute__((ext_vector_type(8)));
 typedef float p_f16v __attribute__((ext_vector_type(16)));
 
 constexpr int kFlagBadExpertId = 1;          // same bit as the other expert kernels
-constexpr uint32_t kPfCols = 64;             // columns (pairs) of an item: two 32-column tiles
 constexpr uint32_t kPfStep = 64;             // activations per K-step: two blocks, 128 bytes a row and plane
-constexpr uint32_t kPfWRow = 80;             // a weight row's group of four blocks (72 bytes) in LDS: five pieces of 16 bytes
 constexpr int kPfFetch = 3;                  // direct loads per group: 160 pieces, 64 a load (the third: half a wave)
-constexpr uint32_t kPfWArea = 32 * kPfWRow;  // 32 rows a wave
+constexpr uint32_t kPfWRow = 80;             // a weight row's group of four blocks (72 bytes) in LDS: five pieces of 16 bytes
 constexpr uint32_t kPfFold = 8;              // steps (16 blocks) of a part of a folded sum
-constexpr uint32_t kPfChain = 32;            // blocks of a row from which on its sums are folded: more
 
 // ---------------------------------------------------------------------------
 // Activation planes of one row, by one wave.  The row is scaled by the power of two that brings its
@@ -111,7 +111,7 @@ moe_pf_planes_kernel(const float *__restrict__ src, uint32_t rows, uint32_t len,
 // Workgroup 0: pairs by expert.  A pair is dropped (and flagged) when its id is out of range or
 // repeats another slot's of the same token, as MoEModelBinding.offsets requires
 // (MoEModelBinding.swift:174-214); valid[p]: pair p takes part.  glist: the pairs in expert order;
-// items: runs of at most kPfCols of them, those of more than 32 pairs (two column tiles, twice the
+// items: runs of at most `cols` of them (64 or 32), those of more than 32 pairs (two column tiles, twice the
 // work) first.  Workgroups 1..: the planes of x, a wave per token.
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(1024)
@@ -119,7 +119,7 @@ moe_pf_group_kernel(const int32_t *__restrict__ ids, uint32_t pairs, uint32_t ex
                     int32_t *__restrict__ glist, uint8_t *__restrict__ valid, int32_t *__restrict__ ranks,
                     lev_pf_item *__restrict__ items, uint32_t *__restrict__ nitems, int *__restrict__ flag, const float *__restrict__ x,
                     uint32_t tokens, uint32_t hidden, _Float16 *__restrict__ xh, _Float16 *__restrict__ xl,
-                    uint32_t *__restrict__ xmax) {
+                    uint32_t *__restrict__ xmax, uint32_t cols) {
     extern __shared__ int32_t s_cnt[];           // [experts] counts | cursors
     const uint32_t tid = threadIdx.x;
     if (blockIdx.x != 0u) {
@@ -188,8 +188,8 @@ moe_pf_group_kernel(const int32_t *__restrict__ ids, uint32_t pairs, uint32_t ex
     for (uint32_t k = 0; k < 4u; ++k) {
         const uint32_t e = 4u * tid + k;
         c4[k] = e < experts ? s_cnt[e] : 0;
-        const uint32_t full = (uint32_t)c4[k] / kPfCols, rem = (uint32_t)c4[k] % kPfCols;
-        local += (uint64_t)c4[k] | (uint64_t)(full + (rem > 32u)) << 21 | (uint64_t)(rem > 0u && rem <= 32u) << 42;
+        const uint32_t full = (uint32_t)c4[k] / cols, rem = (uint32_t)c4[k] % cols;
+        local += (uint64_t)c4[k] | (uint64_t)((cols > 32u ? full : 0u) + (rem > 32u)) << 21 | (uint64_t)((cols > 32u ? 0u : full) + (rem > 0u && rem <= 32u)) << 42;
     }
     uint64_t incl = local;
 #pragma unroll
@@ -213,8 +213,8 @@ moe_pf_group_kernel(const int32_t *__restrict__ ids, uint32_t pairs, uint32_t ex
     for (uint32_t k = 0; k < 4u; ++k) {
         const uint32_t e = 4u * tid + k;
         if (e < experts) s_cur[e] = run;
-        for (int32_t j = 0; j < c4[k]; j += (int32_t)kPfCols) {
-            const int32_t left = c4[k] - j, count = left < (int32_t)kPfCols ? left : (int32_t)kPfCols;
+        for (int32_t j = 0; j < c4[k]; j += (int32_t)cols) {
+            const int32_t left = c4[k] - j, count = left < (int32_t)cols ? left : (int32_t)cols;
             items[count > 32 ? big++ : small++] = lev_pf_item{(int32_t)e, run + j, count, 0};
         }
         run += c4[k];
@@ -244,37 +244,49 @@ moe_pf_group_kernel(const int32_t *__restrict__ ids, uint32_t pairs, uint32_t ex
 // The grouped product.  A wave of a PAIRED (gate/up) workgroup owns 16 rows of the gate matrix and the
 // same 16 rows of the up matrix, so that g and u of an output meet in one lane; down: 32 rows.  The
 // activation step (64 values of every column, both planes) is shared by the workgroup in LDS, two
-// buffers, brought by direct global -> LDS loads; the weights of a wave are its own: 72 bytes of each
+// or three buffers, brought by direct global -> LDS loads; the weights of a wave are its own: 72 bytes of each
 // row fetched 16 bytes a lane with consecutive lanes on consecutive bytes, one group of four blocks
 // ahead, parked as they lie in memory and decoded by the lane that multiplies them.
-// One chain a row (FOLD false): eight waves, 71 KB of LDS and 128 registers, two workgroups per CU whose
-// waits cover each other.  Folded, the parts already added take 32 registers more, three waves a SIMD:
-// one workgroup of twelve waves a CU, or three of four (pf_waves).
+// One chain a row (FOLD false): eight waves, two buffers, 72 KB of LDS and 128 registers, two workgroups per CU whose
+// waits cover each other.  Folded, the parts already added take up to 32 registers more: pf_estimate chooses among four forms.
 // ---------------------------------------------------------------------------
-template <uint32_t WAVES>
+template <uint32_t WAVES, uint32_t TMAX, uint32_t NBUF>
 struct pf_lds_map {
-    static constexpr uint32_t kABuf = 2u * 8u * 1024u;        // two planes x eight regions of eight columns
-    static constexpr uint32_t kW = 2u * kABuf;
-    static constexpr uint32_t kWBuf = WAVES * kPfWArea;
+    static constexpr uint32_t kPlane = TMAX * 4096u;          // four regions of eight columns a column tile
+    static constexpr uint32_t kABuf = 2u * kPlane;
+    static constexpr uint32_t kW = NBUF * kABuf;
+    static constexpr uint32_t kWArea = 32u * kPfWRow;         // 32 rows a wave
+    static constexpr uint32_t kWBuf = WAVES * kWArea;
     static constexpr uint32_t kBytes = kW + 2u * kWBuf;
 };
 
-// the four code bytes of one dword -> half a B operand (fp16 integers n - 8): bytes (0, 2), (1, 3) of
-// the nibble that `shift` (0 or 4) selects
-__device__ __forceinline__ void pf_decode(uint32_t codes, uint32_t mask, uint32_t magic, uint32_t out[2]) {
-    typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-    const f16x2 bias = {(_Float16)1032.0f, (_Float16)1032.0f};
-    // 0x6400 | n is the fp16 number 1024 + n
-    out[0] = __builtin_bit_cast(uint32_t, (f16x2)(__builtin_bit_cast(f16x2, (codes & mask) | magic) - bias));
-    out[1] = __builtin_bit_cast(uint32_t, (f16x2)(__builtin_bit_cast(f16x2, ((codes >> 8) & mask) | magic) - bias));
+// lev_load_lds16 for the lanes of a mask, of a wave that has all its lanes: without a branch, which would end the region in
+// which products and requests are ordered.
+__device__ __forceinline__ void pf_load_lds16_of(const void *src, uint32_t dst, uint32_t lanes_lo, uint32_t lanes_hi) {
+    asm volatile("s_mov_b32 m0, %1\n\ts_mov_b32 exec_lo, %2\n\ts_mov_b32 exec_hi, %3\n\tglobal_load_lds_dwordx4 %0, off\n\ts_mov_b64 exec, -1"
+                 ::"v"(src), "s"(dst), "s"(lanes_lo), "s"(lanes_hi) : "memory");
+}
+constexpr __host__ __device__ uint32_t pf_min(uint32_t a, uint32_t b) { return a < b ? a : b; }
+
+// A block's 16 codes of a lane, two dwords (code bytes 8g .. 8g + 7) -> the operands of both halves, fp16 integers n - 8.
+// 0x6400 | n is the fp16 number 1024 + n, 0x6400 | 16 n is 1024 + 16 n: a subtraction and a multiply-add, both exact.
+struct pf_consts {
+    uint32_t low = 0x000F000Fu, high = 0x00F000F0u, magic = 0x64006400u;
+    lev_f16x2 m1032 = {(_Float16)-1032.0f, (_Float16)-1032.0f}, sixteenth = {(_Float16)0.0625f, (_Float16)0.0625f}, m72 = {(_Float16)-72.0f, (_Float16)-72.0f};
+    // (in registers: (v & mask) | magic is one instruction)
+    __device__ __forceinline__ pf_consts() { asm("" : "+v"(low), "+v"(high), "+v"(magic)); }
+};
+__device__ __forceinline__ void pf_decode(uint32_t c, const pf_consts &k, uint32_t &low, uint32_t &high) {
+    low = __builtin_bit_cast(uint32_t, (lev_f16x2)(__builtin_bit_cast(lev_f16x2, (c & k.low) | k.magic) + k.m1032));
+    high = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(lev_f16x2, (c & k.high) | k.magic), k.sixteenth, k.m72));
 }
 
-template <bool PAIRED, uint32_t WAVES, bool FOLD, int T>
+template <bool PAIRED, uint32_t WAVES, uint32_t TMAX, uint32_t OCC, uint32_t NBUF, bool FOLD, uint32_t T>
 __device__ __forceinline__ void pf_tile(const lev_moe_grouped_args &a, const lev_pf_item it, uint32_t rt,
                                         const _Float16 *__restrict__ ph, const _Float16 *__restrict__ pl,
                                         const uint32_t *__restrict__ pmax, const int32_t *__restrict__ glist,
                                         float *__restrict__ out, uint8_t *lds, int32_t *s_pair, float *s_us) {
-    typedef pf_lds_map<WAVES> L;
+    typedef pf_lds_map<WAVES, TMAX, NBUF> L;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
     const uint32_t lr = lane & 31u, g = lane >> 5;
     const uint32_t in_len = PAIRED ? a.hidden : a.inter, out_rows = PAIRED ? a.inter : a.hidden;
@@ -283,8 +295,8 @@ __device__ __forceinline__ void pf_tile(const lev_moe_grouped_args &a, const lev
 
     // ---- weights: rows 0..15 of a PAIRED wave's 32 are gate rows, 16..31 the same rows of the up matrix (rows come in
     // whole waves: both row counts are multiples of 64).  Piece q of a group is piece q % 5 of row q / 5: the row's
-    // bytes 0, 16, 32, 48 and 56 .. + 15 at 16 bytes a piece, so the fourth block's codes lie at 64, not 56; the last
-    // group of a row may hold two blocks (36 bytes): then its third piece is bytes 20 .. 35, the second block's codes ----
+    // bytes 0, 16, 32, 48 and 56 .. + 15 at 16 bytes a piece, so its last 8 bytes lie at 72, not 64; the last
+    // group of a row may hold two blocks (36 bytes): then its third piece is bytes 20 .. 35 ----
     const uint32_t row0 = (rt * WAVES + wave) * (PAIRED ? 16u : 32u);
     const bool live = row0 < out_rows;   // a wave past the last row only brings activations
     const uint32_t lds0 = lev_lds_offset(lds);
@@ -300,147 +312,246 @@ __device__ __forceinline__ void pf_tile(const lev_moe_grouped_args &a, const lev
         wsrc[j] = a.base + mat + (uint64_t)row * row_bytes;
     }
     const uint32_t ngrp = (nblk + 3u) >> 2;
-    auto w_request = [&](uint32_t grp) {
+    auto w_request = [&](uint32_t grp, uint32_t j) {
         const uint32_t gc = grp < ngrp ? grp : ngrp - 1u, left = row_bytes - gc * 72u, last = (left < 72u ? left : 72u) - 16u;
-        const uint32_t dst = lds0 + L::kW + (grp & 1u) * L::kWBuf + wave * kPfWArea;
-#pragma unroll
-        for (int j = 0; j < kPfFetch; ++j) {
-            const uint32_t at = (wpos >> (8 * j)) & 0xFFu;
-            if (j < 2 || lane < 32u) lev_load_lds16(wsrc[j] + (gc * 72u + (at < last ? at : last)), dst + j * 1024u);
-        }
+        const uint32_t dst = lds0 + L::kW + (grp & 1u) * L::kWBuf + wave * L::kWArea;
+        const uint32_t at = (wpos >> (8 * j)) & 0xFFu;
+        const uint8_t *const src = wsrc[j] + (gc * 72u + (at < last ? at : last));
+        if (j == 2u) pf_load_lds16_of(src, dst + 2048u, ~0u, 0u);
+        else lev_load_lds16(src, dst + j * 1024u);
     };
-    w_request(0);
 
-    // ---- columns ----
-    if (tid < kPfCols) {
-        const int32_t p = glist[it.first + (int32_t)(tid < count ? tid : count - 1u)];
-        s_pair[tid] = p;
-        s_us[tid] = pf_row_scale(pmax[PAIRED ? (uint32_t)p / a.top_k : (uint32_t)p]).unscale;
-    }
-    __syncthreads();
-
-    // ---- activations: load k of a step (T of them a wave) is plane k & 1 of region k / 2; a region is eight
+    // ---- activations: load k of a step is plane k & 1 of region k / 2; a region is eight
     // columns x eight runs of eight values.  Slot 8 * (run ^ region parity) + ((column & 7) ^ run) of a
     // region: a load's 64 lanes fetch 8 rows x 128 contiguous bytes, and the lanes of a fragment read (32
     // columns, one run each half) hit every bank equally ----
+    // A wave that has fewer than the others brings one lane's piece of the last load once more (the same bytes to the same
+    // place): every wave has as many requests in flight, which the waits count.
     constexpr uint32_t kALoads = (8u * T + WAVES - 1u) / WAVES;
+    constexpr bool kAll = 8u * T == WAVES * kALoads;
     const _Float16 *asrc[kALoads];
 #pragma unroll
     for (uint32_t j = 0; j < kALoads; ++j) {
-        const uint32_t k = wave * kALoads + j < 8u * T ? wave * kALoads + j : 8u * T - 1u, region = k >> 1, run = (lane >> 3) ^ (region & 1u);
-        const uint32_t p = (uint32_t)s_pair[region * 8u + ((lane & 7u) ^ run)];
+        const uint32_t k = pf_min(wave * kALoads + j, 8u * T - 1u), region = k >> 1, run = (lane >> 3) ^ (region & 1u);
+        const uint32_t col = region * 8u + ((lane & 7u) ^ run), p = (uint32_t)glist[it.first + (int32_t)(col < count ? col : count - 1u)];
         asrc[j] = (k & 1u ? pl : ph) + (uint64_t)(PAIRED ? p / a.top_k : p) * in_len + run * 8u;
     }
-    auto a_request = [&](uint32_t step) {
-        const uint32_t s = step < nsteps ? step : nsteps - 1u;   // past the end: any valid step, never read
-        const uint32_t dst = lds0 + (step & 1u) * L::kABuf;
+    int32_t own_pair = 0;     // a column's pair and scale, wanted at the end
+    uint32_t own_max = 0u;
+    if (tid < 32u * T) {
+        own_pair = glist[it.first + (int32_t)(tid < count ? tid : count - 1u)];
+        own_max = pmax[PAIRED ? (uint32_t)own_pair / a.top_k : (uint32_t)own_pair];
+    }
+    // (up to two steps past the end of a row, which lie in front of something else of the scratch: read, never used)
+    auto a_request = [&](uint32_t buf, uint32_t j) {
+        const uint32_t n = wave * kALoads + j, k = pf_min(n, 8u * T - 1u), dst = lds0 + buf + (k & 1u) * L::kPlane + (k >> 1) * 1024u;
+        if (kAll) {
+            lev_load_lds16(asrc[j], dst);
+        } else {
+            const uint32_t all = (uint32_t)__builtin_amdgcn_readfirstlane(n < 8u * T ? -1 : 0);
+            pf_load_lds16_of(asrc[j], dst, all | 1u, all);
+        }
+        asrc[j] += kPfStep;
+    };
 #pragma unroll
-        for (uint32_t j = 0; j < kALoads; ++j) {
-            const uint32_t k = wave * kALoads + j;
-            if (kALoads * WAVES == 8u * T || k < 8u * T) lev_load_lds16(asrc[j] + s * kPfStep, dst + (k & 1u) * 8192u + (k >> 1) * 1024u);
+    for (uint32_t j = 0; j < kALoads; ++j) a_request(0u, j);
+#pragma unroll
+    for (uint32_t j = 0; j < kPfFetch; ++j) w_request(0u, j);
+    if (NBUF == 3u) {
+#pragma unroll
+        for (uint32_t j = 0; j < kALoads; ++j) a_request(L::kABuf, j);
+    }
+
+    // The buffers of this step's activations, of the next's and of the one's to be requested.  Three: at the start of a step
+    // the next step's have landed, every wave's, and a wave reads its first fragments of a step behind the products of
+    // the step before, not behind the barrier.  Two: this step's have landed, the next's are requested.
+    uint32_t buf0 = 0u, buf1 = L::kABuf, buf2 = (NBUF - 1u) * L::kABuf;
+    auto bring = [&](uint32_t step, auto kind) {
+        // (newer than the activations waited for: the next group's weights, requested in the first step of a group)
+        if (decltype(kind)::value == 1u) LEV_WAIT_VMCNT(kPfFetch);
+        else LEV_WAIT_VMCNT(0);
+        lev_barrier_lds();   // and everybody is done with the step before
+    };
+    // A step's requests, one behind a product each: issued together behind the barrier, by all waves, they waited in the issue
+    // for 300 to 570 of a step's 2300 clocks.
+    auto requests = [&](uint32_t step, auto kind, uint32_t b, uint32_t slot) {   // slot: of the 4 T products of a block
+        if (b == 0u) {
+#pragma unroll
+            for (uint32_t j = 0; j < kALoads; ++j)
+                if (slot == j * (4u * T / kALoads)) a_request(buf2, j);
+        } else if (decltype(kind)::value != 1u) {
+#pragma unroll
+            for (uint32_t j = 0; j < kPfFetch; ++j)
+                if (slot == j * (4u * T / 3u)) w_request((step >> 1) + 1u, j);
         }
     };
-    a_request(0);
+    auto turn = [&]() {
+        const uint32_t b = buf0;
+        if (NBUF == 3u) buf0 = buf1, buf1 = buf2, buf2 = b;
+        else buf0 = buf2, buf2 = b;
+    };
+    const std::integral_constant<uint32_t, 0> first;    // of a group's steps
+    const std::integral_constant<uint32_t, 1> second;
+    const std::integral_constant<uint32_t, 2> only;     // of a group of two blocks
+    LEV_WAIT_VMCNT(0);
+    asm volatile("" : "+v"(own_pair), "+v"(own_max)::"memory");   // (not waited for in front of the requests)
+    if (tid < 32u * T) {
+        s_pair[tid] = own_pair;
+        s_us[tid] = pf_row_scale(own_max).unscale;
+    }
+    lev_barrier_lds();
+    if (!live) {
+        auto pass = [&](uint32_t step, auto kind) {
+            bring(step, kind);
+#pragma unroll
+            for (uint32_t i = 0; i < 8u * T; ++i) requests(step, kind, i / (4u * T), i % (4u * T));
+            turn();
+        };
+        for (uint32_t step = 0; step + 1u < nsteps; step += 2u) pass(step, first), pass(step + 1u, second);
+        if (nsteps & 1u) pass(nsteps - 1u, only);
+        LEV_WAIT_VMCNT(0);
+        return;
+    }
 
     float y[T][16], whole[T][16];   // FOLD: the part under way, and the parts before it
 #pragma unroll
-    for (int t = 0; t < T; ++t)
+    for (uint32_t t = 0; t < T; ++t)
 #pragma unroll
         for (int i = 0; i < 16; ++i) y[t][i] = whole[t][i] = 0.f;
     auto fold = [&]() {
 #pragma unroll
-        for (int t = 0; t < T; ++t)
+        for (uint32_t t = 0; t < T; ++t)
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
                 whole[t][i] += y[t][i];
                 y[t][i] = 0.f;
             }
     };
-    uint32_t k_mask = 0x000F000Fu, k_magic = 0x64006400u;
-    asm("" : "+v"(k_mask), "+v"(k_magic));   // in registers: (v & mask) | magic is one instruction
-    const uint8_t *const wmine = lds + L::kW + wave * kPfWArea + lr * kPfWRow;
+    const pf_consts kc;
+    const uint8_t *const wmine = lds + L::kW + wave * L::kWArea + lr * kPfWRow;
     const uint32_t areg = (lr >> 3) * 1024u, apar = (lr >> 3) & 1u, acol = lr & 7u;
-    uint32_t aoff[4];   // this lane's fragment of half s of block b of a step: aoff[2b + s], + 4096 per column tile, + 8192 for the low plane
+    uint32_t aoff[4];   // this lane's fragment of half s of block b of a step: aoff[2b + s], + 4096 per column tile, + kPlane for the low plane
 #pragma unroll
     for (uint32_t k = 0; k < 4u; ++k) {
         const uint32_t run = 2u * k + g;
         aoff[k] = areg + ((run ^ apar) * 8u + (acol ^ run)) * 16u;
     }
 
-    auto step_of = [&](uint32_t step, auto odd) {
-        constexpr uint32_t st = decltype(odd)::value;   // second step of a group
-        // This step's activations have landed: they are the newest loads but for the next group's
-        // weights, which are requested behind them in the first step of a group.
-        if (st == 1u) LEV_WAIT_VMCNT(kPfFetch);
-        else LEV_WAIT_VMCNT(0);
-        lev_barrier_lds();   // everybody's have, and everybody is done with the other buffer
-        a_request(step + 1u);
-        if (st == 0u) w_request((step >> 1) + 1u);
-        if (!live) return;
-        const uint8_t *const ab = lds + (step & 1u) * L::kABuf;
-        const uint8_t *const wb = wmine + ((step >> 1) & 1u) * L::kWBuf + st * 36u;
-        // codes and scales of the step's two blocks: code bytes 8g .. 8g + 7 of the first start two bytes
-        // behind a dword boundary, those of the second on one
-        const uint32_t *const wq = reinterpret_cast<const uint32_t *>(wb + 8u * g);
-        const uint32_t at = st == 1u ? 28u : step + 1u == nsteps ? 32u : 20u;   // (see the pieces above)
-        const uint32_t *const wo = reinterpret_cast<const uint32_t *>(wb + at + 8u * g);
-        const uint32_t q0 = wq[0], q1 = wq[1], q2 = wq[2], q5 = wo[0], q6 = wo[1];
-        const _Float16 dh[2] = {*reinterpret_cast<const _Float16 *>(wb), *reinterpret_cast<const _Float16 *>(wb + 18)};
-        p_h8 A[2][2][2];   // [unit parity][plane][half of the block]
-        auto a_read = [&](uint32_t u) {
-            const uint32_t b = u / T, t = u % T;
-#pragma unroll
-            for (uint32_t s = 0; s < 2u; ++s) {
-                const uint8_t *q = ab + aoff[2u * b + s] + t * 4096u;
-                A[u & 1u][0][s] = *reinterpret_cast<const p_h8 *>(q);
-                A[u & 1u][1][s] = *reinterpret_cast<const p_h8 *>(q + 8192u);
-            }
-        };
-        a_read(0);
-        p_h8 B0, B1;
-        float d = 0.f;
-#pragma unroll
-        for (uint32_t u = 0; u < 2u * T; ++u) {   // unit: one block x one column tile
-            const uint32_t b = u / T, t = u % T;
-            if (t == 0u) {
-                const uint32_t c0 = b ? q5 : __builtin_amdgcn_alignbit(q1, q0, 16), c1 = b ? q6 : __builtin_amdgcn_alignbit(q2, q1, 16);
-                d = (float)dh[b];
-                asm("" : "+v"(d));   // converted once: the mixed-precision multiply-add takes longer than the f32 one
-                uint32_t w[8];
-                pf_decode(c0, k_mask, k_magic, w);
-                pf_decode(c1, k_mask, k_magic, w + 2);
-                pf_decode(c0 >> 4, k_mask, k_magic, w + 4);
-                pf_decode(c1 >> 4, k_mask, k_magic, w + 6);
-                B0 = __builtin_bit_cast(p_h8, lev_u32x4{w[0], w[1], w[2], w[3]});
-                B1 = __builtin_bit_cast(p_h8, lev_u32x4{w[4], w[5], w[6], w[7]});
-            }
-            // the next unit's fragments are requested ahead of this unit's products
-            if (u + 1u < 2u * T) a_read(u + 1u);
-            __builtin_amdgcn_sched_barrier(0);
-            const p_h8(&F)[2][2] = A[u & 1u];
-            p_f16v acc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(F[0][0], B0, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(F[0][1], B1, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(F[1][0], B0, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(F[1][1], B1, acc, 0, 0, 0);
-#pragma unroll
-            for (int i = 0; i < 16; ++i) y[t][i] = fmaf(d, acc[i], y[t][i]);
-        }
+    // Codes and scale of a block, 8 aligned bytes a read: at this row stride 4.2 clocks of the LDS, where one dword or half
+    // word takes 8.1 and two dwords at once 16.  They are decoded behind the products of the block before.  Code bytes 8g .. 8g + 7 of a step's first block start two
+    // bytes behind a dword boundary, those of its second on one.
+    lev_u32x2 w[3];
+    auto w_read = [&](const uint8_t *q, uint32_t st, uint32_t b, bool part) {
+        auto at = [&](uint32_t byte) { return *reinterpret_cast<const lev_u32x2 *>(q + byte); };
+        if (b == 0u) w[0] = at(32u * st + 8u * g), w[1] = at(32u * st + 8u * g + 8u), w[2] = at(32u * st);
+        else if (st == 1u) w[0] = at(56u + 16u * g), w[2] = at(48u);   // (the last 8 bytes lie at 72)
+        else if (part) w[0] = at(32u + 8u * g), w[2] = at(16u);
+        else w[0] = at(16u + 8u * g), w[1] = at(24u + 8u * g), w[2] = at(16u);
     };
-    for (uint32_t step = 0; step < nsteps; step += 2u) {
-        step_of(step, std::integral_constant<uint32_t, 0>());
-        if (step + 1u < nsteps) step_of(step + 1u, std::integral_constant<uint32_t, 1>());
+    uint32_t code[2];   // the next block's code dwords, its scale, its operands
+    float dn;
+    uint32_t bn[8];
+    auto w_take = [&](uint32_t st, uint32_t b, bool part) {
+        uint32_t dw;
+        if (b == 0u) {
+            code[0] = st ? __builtin_amdgcn_alignbit(w[1].x, w[0].y, 16) : __builtin_amdgcn_alignbit(w[0].y, w[0].x, 16);
+            code[1] = st ? __builtin_amdgcn_alignbit(w[1].y, w[1].x, 16) : __builtin_amdgcn_alignbit(w[1].x, w[0].y, 16);
+            dw = st ? w[2].y : w[2].x;
+        } else {
+            code[0] = st || part ? w[0].x : w[0].y;
+            code[1] = st || part ? w[0].y : w[1].x;
+            dw = (st ? w[2].y : w[2].x) >> 16;
+        }
+        dn = lev_f16_bits_to_f32(dw & 0xFFFFu);
+        asm("" : "+v"(dn));   // converted once: the mixed-precision multiply-add takes longer than the f32 one
+    };
+    auto quarter = [&](uint32_t k) { pf_decode(k & 1u ? code[k >> 1] >> 8 : code[k >> 1], kc, bn[k], bn[4u + k]); };
+    p_h8 A[4];   // high plane's halves of the block, low plane's
+    auto a_read = [&](uint32_t buf, uint32_t u, uint32_t k) {
+        A[k] = *reinterpret_cast<const p_h8 *>(lds + buf + aoff[2u * (u / T) + (k & 1u)] + (u % T) * 4096u + (k >> 1) * L::kPlane);
+    };
+    w_read(wmine, 0, 0, false);
+    if (NBUF == 3u) {
+#pragma unroll
+        for (uint32_t k = 0; k < 4u; ++k) a_read(0u, 0u, k);
+    }
+    w_take(0, 0, false);
+#pragma unroll
+    for (uint32_t k = 0; k < 4u; ++k) quarter(k);
+
+    // a unit's product is added behind the products of the next one (four waves a SIMD: at once, they have no registers for two)
+    constexpr bool kLate = OCC < 4u;
+    p_f16v pend = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    float pend_d = 0.f;
+    auto step_of = [&](uint32_t step, auto kind) {
+        constexpr uint32_t st = decltype(kind)::value & 1u;
+        constexpr bool part = decltype(kind)::value == 2u;
+        bring(step, kind);
+        if (NBUF == 2u) {
+#pragma unroll
+            for (uint32_t k = 0; k < 4u; ++k) a_read(buf0, 0u, k);
+        }
+        const uint8_t *const wb = wmine + ((step >> 1) & 1u) * L::kWBuf, *const wnext = wmine + (((step + 1u) >> 1) & 1u) * L::kWBuf;
+#pragma unroll
+        for (uint32_t b = 0; b < 2u; ++b) {
+            const float d = dn;
+            const p_h8 B[2] = {__builtin_bit_cast(p_h8, lev_u32x4{bn[0], bn[1], bn[2], bn[3]}), __builtin_bit_cast(p_h8, lev_u32x4{bn[4], bn[5], bn[6], bn[7]})};
+            if (b == 0u) {
+                w_read(wb, st, 1u, part);
+            } else {
+                if (st == 1u) {
+                    LEV_WAIT_VMCNT(kALoads);   // the next group's weights have landed
+                    asm volatile("" ::: "memory");
+                }
+                w_read(wnext, st ^ 1u, 0u, false);
+            }
+#pragma unroll
+            for (uint32_t t = 0; t < T; ++t) {   // unit: one block x one column tile
+                const uint32_t u = b * T + t, pt = t ? t - 1u : T - 1u;
+                p_f16v acc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+                if (t == T - 1u) w_take(b == 0u ? st : st ^ 1u, b ^ 1u, b == 0u && part);
+#pragma unroll
+                for (uint32_t k = 0; k < 4u; ++k) {
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[k], B[k & 1u], acc, 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);   // (else it comes behind the additions, and they wait for the product before)
+                    // the next unit's fragment takes the place of this one
+                    if (u + 1u < 2u * T) a_read(buf0, u + 1u, k);
+                    else if (NBUF == 3u) a_read(buf1, 0u, k);
+                    // the product before this one, while the matrix cores have this one
+#pragma unroll
+                    for (uint32_t i = 4u * k; kLate && i < 4u * k + 4u; ++i) y[pt][i] = fmaf(pend_d, pend[i], y[pt][i]);
+                    if (t == T - 1u) quarter(k);
+                    requests(step, kind, b, 4u * t + k);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                if (kLate) {
+                    pend = acc;
+                    pend_d = d;
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) y[t][i] = fmaf(d, acc[i], y[t][i]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+        }
+        turn();
+    };
+    for (uint32_t step = 0; step + 1u < nsteps; step += 2u) {
+        step_of(step, first);
+        step_of(step + 1u, second);
         if (FOLD && (step & (kPfFold - 2u)) == kPfFold - 2u) fold();
     }
+    if (nsteps & 1u) step_of(nsteps - 1u, only);
+#pragma unroll
+    for (int i = 0; kLate && i < 16; ++i) y[T - 1u][i] = fmaf(pend_d, pend[i], y[T - 1u][i]);
     if (FOLD) fold();
     float(&sum)[T][16] = FOLD ? whole : y;
 
-    LEV_WAIT_VMCNT(0);   // the request past the end lands before the LDS is given back
-    if (!live) return;
+    LEV_WAIT_VMCNT(0);   // the requests past the end land before the LDS is given back
     // lane (lr, g), register i of a tile: weight row lr, column 8 (i / 4) + 4 g + i % 4
     const uint32_t row = row0 + (PAIRED ? lr & 15u : lr);
 #pragma unroll
-    for (int t = 0; t < T; ++t)
+    for (uint32_t t = 0; t < T; ++t)
 #pragma unroll
         for (int i = 0; i < 16; i += PAIRED ? 2 : 1) {
             uint32_t col = 32u * t + 8u * (i / 4) + 4u * g + (i % 4);
@@ -461,19 +572,20 @@ __device__ __forceinline__ void pf_tile(const lev_moe_grouped_args &a, const lev
 
 // grid: 8 * ceil(items / 8) * row tiles, in one line.  Workgroups go to the XCDs in turn, so item 8j + c
 // sits on XCD c with all its row tiles, which read the same activations through one L2.
-template <bool PAIRED, uint32_t WAVES, bool FOLD>
-__global__ void __launch_bounds__(WAVES * 64, FOLD ? 3 : 4)
+template <bool PAIRED, uint32_t WAVES, uint32_t TMAX, uint32_t OCC, uint32_t NBUF, bool FOLD>
+__global__ void __launch_bounds__(WAVES * 64, OCC)
 moe_pf_kernel(lev_moe_grouped_args a, uint32_t row_tiles, const _Float16 *__restrict__ ph,
               const _Float16 *__restrict__ pl, const uint32_t *__restrict__ pmax, const int32_t *__restrict__ glist,
               const lev_pf_item *__restrict__ items, const uint32_t *__restrict__ nitems, float *__restrict__ out) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
-    __shared__ int32_t s_pair[kPfCols];
-    __shared__ float s_us[kPfCols];
+    __shared__ int32_t s_pair[32u * TMAX];
+    __shared__ float s_us[32u * TMAX];
     const uint32_t j = blockIdx.x >> 3, at = (j / row_tiles) * 8u + (blockIdx.x & 7u), rt = j % row_tiles;
+    const lev_pf_item it = items[at];   // (there is room for the whole grid's)
     if (at >= *nitems) return;
-    const lev_pf_item it = items[at];
-    if (it.count > 32) pf_tile<PAIRED, WAVES, FOLD, 2>(a, it, rt, ph, pl, pmax, glist, out, smem, s_pair, s_us);
-    else pf_tile<PAIRED, WAVES, FOLD, 1>(a, it, rt, ph, pl, pmax, glist, out, smem, s_pair, s_us);
+    if constexpr (TMAX >= 2u)
+        if (it.count > 32) return pf_tile<PAIRED, WAVES, TMAX, OCC, NBUF, FOLD, 2>(a, it, rt, ph, pl, pmax, glist, out, smem, s_pair, s_us);
+    pf_tile<PAIRED, WAVES, TMAX, OCC, NBUF, FOLD, 1>(a, it, rt, ph, pl, pmax, glist, out, smem, s_pair, s_us);
 }
 
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
@@ -481,9 +593,9 @@ size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 struct pf_layout {
     size_t glist, valid, items, nitems, xh, xl, xmax, ah, al, amax, dn, total;
 };
-size_t pf_max_items(const lev_moe_grouped_args &a) {
+size_t pf_max_items(const lev_moe_grouped_args &a, uint32_t cols) {
     const size_t pairs = (size_t)a.tokens * a.top_k;
-    return pairs / kPfCols + (a.experts < pairs ? a.experts : pairs);
+    return (pairs / cols + (a.experts < pairs ? a.experts : pairs) + 7u) & ~(size_t)7;   // whole turns of the XCDs
 }
 pf_layout pf_layout_of(const lev_moe_grouped_args &a) {
     const size_t pairs = (size_t)a.tokens * a.top_k;
@@ -491,7 +603,7 @@ pf_layout pf_layout_of(const lev_moe_grouped_args &a) {
     size_t o = 0;
     L.glist = o; o += align256(pairs * 4);
     L.valid = o; o += align256(pairs);
-    L.items = o; o += align256(pf_max_items(a) * sizeof(lev_pf_item));
+    L.items = o; o += align256(pf_max_items(a, 32u) * sizeof(lev_pf_item));
     L.nitems = o; o += 256;
     L.xh = o; o += align256((size_t)a.tokens * a.hidden * 2);
     L.xl = o; o += align256((size_t)a.tokens * a.hidden * 2);
@@ -504,40 +616,30 @@ pf_layout pf_layout_of(const lev_moe_grouped_args &a) {
     return L;
 }
 
-template <bool PAIRED, uint32_t WAVES, bool FOLD>
-hipError_t pf_launch_as(lev_ctx *ctx, const lev_moe_grouped_args &a, const _Float16 *ph, const _Float16 *pl, const uint32_t *pmax,
+template <bool PAIRED, uint32_t WAVES, uint32_t TMAX, uint32_t OCC, uint32_t NBUF, bool FOLD>
+hipError_t pf_launch_as(lev_ctx *ctx, const lev_moe_grouped_args &a, uint32_t cols, const _Float16 *ph, const _Float16 *pl, const uint32_t *pmax,
                         const int32_t *glist, const lev_pf_item *items, const uint32_t *nitems, float *out) {
-    if (hipError_t e = lev_allow_lds(ctx, reinterpret_cast<const void *>(&moe_pf_kernel<PAIRED, WAVES, FOLD>), pf_lds_map<WAVES>::kBytes);
+    constexpr size_t lds = pf_lds_map<WAVES, TMAX, NBUF>::kBytes;
+    if (hipError_t e = lev_allow_lds(ctx, reinterpret_cast<const void *>(&moe_pf_kernel<PAIRED, WAVES, TMAX, OCC, NBUF, FOLD>), lds);
         e != hipSuccess)
         return e;
-    const uint32_t slots = (uint32_t)((pf_max_items(a) + 7u) / 8u) * 8u;
+    const uint32_t slots = (uint32_t)pf_max_items(a, cols);
     const uint32_t rows = PAIRED ? a.inter : a.hidden, per_wg = WAVES * (PAIRED ? 16u : 32u), tiles = (rows + per_wg - 1u) / per_wg;
-    hipLaunchKernelGGL((moe_pf_kernel<PAIRED, WAVES, FOLD>), dim3(slots * tiles), dim3(WAVES * 64u), pf_lds_map<WAVES>::kBytes,
+    hipLaunchKernelGGL((moe_pf_kernel<PAIRED, WAVES, TMAX, OCC, NBUF, FOLD>), dim3(slots * tiles), dim3(WAVES * 64u), lds,
                        ctx->stream, a, tiles, ph, pl, pmax, glist, items, nitems, out);
     return hipGetLastError();
 }
 
-// Waves of a folded workgroup.  Three of four waves share a CU where one of twelve has it to itself: they read the
-// activations three times, and their last round is finer.  So twelve where whole rounds of them come near the
-// work there is (us a layer with twelve, with four: 2816 / 704, top-8 of 128: 1000 tokens, 2.9 rounds, 393, 409; 300
-// tokens, 2 rounds, 209, 217; 2048 / 768, 1000 tokens, 310, 330; 1536 / 1088, top-4 of 60, 600 tokens, 1.5 rounds, 155,
-// 147; 2304 / 1280, top-2 of 32, 1000 tokens, 1.3 rounds, 184, 167; 4096 / 448, top-4 of 32, 300 tokens, 0.4 rounds, 149,
-// 105).  Items: one an expert that has pairs, and half an item more where they are many.
-uint32_t pf_waves(const lev_ctx *ctx, const lev_moe_grouped_args &a, uint32_t out_rows, uint32_t rows_a_wave) {
-    const double mean = (double)a.tokens * a.top_k / a.experts;
-    const double items = a.experts * std::fmax(1.0 - std::exp(-mean), mean / kPfCols + 0.5);
-    const double rounds = items * ((out_rows + 12u * rows_a_wave - 1u) / (12u * rows_a_wave)) / ctx->num_cus;
-    return 0.95 * std::ceil(rounds) <= rounds + 0.25 ? 12u : 4u;
-}
-
 template <bool PAIRED>
-hipError_t pf_launch(lev_ctx *ctx, const lev_moe_grouped_args &a, const _Float16 *ph, const _Float16 *pl, const uint32_t *pmax,
-                     const int32_t *glist, const lev_pf_item *items, const uint32_t *nitems, float *out) {
-    if ((PAIRED ? a.hidden : a.inter) <= 32u * kPfChain)
-        return pf_launch_as<PAIRED, 8, false>(ctx, a, ph, pl, pmax, glist, items, nitems, out);
-    if (pf_waves(ctx, a, PAIRED ? a.inter : a.hidden, PAIRED ? 16u : 32u) == 12u)
-        return pf_launch_as<PAIRED, 12, true>(ctx, a, ph, pl, pmax, glist, items, nitems, out);
-    return pf_launch_as<PAIRED, 4, true>(ctx, a, ph, pl, pmax, glist, items, nitems, out);
+hipError_t pf_launch(lev_ctx *ctx, const lev_moe_grouped_args &a, const pf_plan &plan, const _Float16 *ph, const _Float16 *pl,
+                     const uint32_t *pmax, const int32_t *glist, const lev_pf_item *items, const uint32_t *nitems, float *out) {
+    switch (PAIRED ? plan.gate_up : plan.down) {
+        case kChain: return pf_launch_as<PAIRED, 8, 2, 4, 2, false>(ctx, a, plan.cols, ph, pl, pmax, glist, items, nitems, out);
+        case kTwelve: return pf_launch_as<PAIRED, 12, 2, 3, 3, true>(ctx, a, plan.cols, ph, pl, pmax, glist, items, nitems, out);
+        case kEight: return pf_launch_as<PAIRED, 8, 2, 2, 3, true>(ctx, a, plan.cols, ph, pl, pmax, glist, items, nitems, out);
+        case kFour: return pf_launch_as<PAIRED, 4, 2, 2, 3, true>(ctx, a, plan.cols, ph, pl, pmax, glist, items, nitems, out);
+        default: return pf_launch_as<PAIRED, 8, 1, 4, 3, true>(ctx, a, plan.cols, ph, pl, pmax, glist, items, nitems, out);
+    }
 }
 
 }  // namespace
@@ -565,16 +667,17 @@ hipError_t lev_moe_prefill_launch(lev_ctx *ctx, const lev_moe_grouped_args &a, c
     uint32_t *xmax = reinterpret_cast<uint32_t *>(s + L.xmax), *amax = reinterpret_cast<uint32_t *>(s + L.amax);
     float *dn = reinterpret_cast<float *>(s + L.dn);
     const uint32_t pairs = a.tokens * a.top_k;
+    const pf_plan plan = pf_plan_of(pf_shape{(uint32_t)ctx->num_cus, a.hidden, a.inter, a.experts, a.top_k, a.tokens});
     hipError_t e;
     hipLaunchKernelGGL(moe_pf_group_kernel, dim3(1u + (a.tokens + 15u) / 16u), dim3(1024), (size_t)2 * a.experts * 4,
                        ctx->stream, ids, pairs, a.experts, a.top_k, glist, valid, reinterpret_cast<int32_t *>(dn), items, nitems, ctx->d_flag, x,
-                       a.tokens, a.hidden, xh, xl, xmax);   // (the ranks are in the place of dn, which comes much later)
+                       a.tokens, a.hidden, xh, xl, xmax, plan.cols);   // (the ranks are in the place of dn, which comes much later)
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    if ((e = pf_launch<true>(ctx, a, xh, xl, xmax, glist, items, nitems, act)) != hipSuccess) return e;
+    if ((e = pf_launch<true>(ctx, a, plan, xh, xl, xmax, glist, items, nitems, act)) != hipSuccess) return e;
     // rows of act that belong to dropped pairs were never written: their planes are never read
     hipLaunchKernelGGL(moe_pf_planes_kernel, dim3((pairs + 3u) / 4u), dim3(256), 0, ctx->stream, act, pairs, a.inter, ah,
                        al, amax);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    if ((e = pf_launch<false>(ctx, a, ah, al, amax, glist, items, nitems, dn)) != hipSuccess) return e;
+    if ((e = pf_launch<false>(ctx, a, plan, ah, al, amax, glist, items, nitems, dn)) != hipSuccess) return e;
     return lev_moe_merge_launch(ctx, a, dn, weights, valid, y);
 }

@@ -199,3 +199,36 @@ def test_moe_grouped_product_tiles_of_small_experts(ctx, hidden, inter, counts):
         assert O.max_rel_err(act[t], ref["act"]) < TOL, t
         y32, _ = O.moe_experts_f32(g, u, d, hidden, inter, ids[t], wts[t], x[t])
         assert O.max_rel_err(y[t], ref["y"]) < max(TOL, 1.5 * O.max_rel_err(y32, ref["y"])), t
+
+
+# hidden, inter, experts, tokens, (pairs an item, form of gate/up, form of down) on 256 CUs: test_moe_rules.py holds the forms
+FORMS = [
+    (1024, 1088, 64, 832, (64, 0, 3)),
+    (1088, 1088, 64, 832, (64, 1, 1)),        # 17 steps a row: a last group of two blocks; waves past the last row
+    (1280, 640, 32, 7200, (64, 2, 0)),        # experts of four items
+    (1088, 2176, 40, 560, (64, 1, 3)),
+    (1088, 512, 16, 800, (64, 3, 0)),
+    (1088, 1088, 32, 640, (32, 4, 4)),
+    (2304, 1280, 32, 2000, (64, 2, 2)),
+]
+
+
+@pytest.mark.parametrize("hidden,inter,experts,tokens,forms", FORMS)
+def test_moe_grouped_product_forms(ctx, hidden, inter, experts, tokens, forms):
+    """Every form of the product, with lists at the edges of column tiles and items: one pair, and one more and less than
+    32 and 64.  Tokens of those lists and some others are checked."""
+    edges = [1, 31, 32, 33, 63, 64, 65]
+    wr, pool, offs, x = H.config5(hidden, inter, experts, tokens, seed=hidden + inter)
+    rng = np.random.default_rng(tokens)
+    rest = rng.multinomial(tokens - sum(edges), [1 / (experts - len(edges))] * (experts - len(edges)))
+    ids = rng.permutation(np.repeat(np.arange(experts), edges + rest.tolist())).astype(np.int32)[:, None]
+    wts = rng.random((tokens, 1)).astype(np.float32)
+    y, act = run_experts(ctx, pool, offs, hidden, inter, experts, x, ids, wts)
+    assert np.isfinite(y).all() and np.isfinite(act).all()
+    g, u, d = (pool[offs["gate_off"]:], pool[offs["up_off"]:], pool[offs["down_off"]:])
+    checked = np.concatenate([np.flatnonzero(ids[:, 0] == e)[[0, -1]] for e in range(experts)])
+    for t in checked:
+        ref = O.moe_experts_f64(g, u, d, hidden, inter, ids[t], wts[t], x[t])
+        assert O.max_rel_err(act[t], ref["act"]) < TOL, t
+        y32, _ = O.moe_experts_f32(g, u, d, hidden, inter, ids[t], wts[t], x[t])
+        assert O.max_rel_err(y[t], ref["y"]) < max(TOL, 1.5 * O.max_rel_err(y32, ref["y"])), t

@@ -1,4 +1,5 @@
 """CPU: the arithmetic by which the few-token expert kernels are cut into workgroups."""
+import itertools
 import os
 import shutil
 import subprocess
@@ -47,3 +48,38 @@ def test_gate_up_rows_cover_every_shape(rows_of):
     for (cus, h, i, pairs, f), rows in zip(cases, rows_of(cases)):
         assert 1 <= rows <= i
         assert f != 2 or rows <= 16 or rows % 16 == 0 or rows == i
+
+
+PLAN_PROGRAM = """
+#include "moe_prefill_plan.hpp"
+#include <cstdio>
+int main() {
+    unsigned cus, hidden, inter, experts, top_k, tokens;
+    while (std::scanf("%u %u %u %u %u %u", &cus, &hidden, &inter, &experts, &top_k, &tokens) == 6) {
+        const pf_plan p = pf_plan_of(pf_shape{cus, hidden, inter, experts, top_k, tokens});
+        std::printf("%u %u %u\\n", p.cols, (unsigned)p.gate_up, (unsigned)p.down);
+    }
+}
+"""
+
+
+def test_prompt_product_forms(tmp_path):
+    """Every form of the grouped product is reached by a shape of tests/test_gpu_moe_prefill.py, the narrow one (4) only where
+    items are cut to 32 pairs, the folded ones (1 to 4) exactly where a row has more than 32 blocks."""
+    from tests.test_gpu_moe_prefill import FORMS
+    cxx = os.environ.get("CXX") or shutil.which("g++")
+    if not cxx:
+        pytest.skip("no C++ compiler")
+    (tmp_path / "plan.cpp").write_text(PLAN_PROGRAM)
+    subprocess.run([cxx, "-std=c++17", "-Wall", "-Werror", f"-I{CSRC}", str(tmp_path / "plan.cpp"), "-o", str(tmp_path / "plan")], check=True)
+    cases = [(256, h, i, e, 1, t) for h, i, e, t, _ in FORMS]
+    cases += list(itertools.product((64, 256), (64, 1024, 1088, 4160), (64, 704, 1088), (1, 32, 128, 4096), (1, 8), (1, 300, 1000, 20000)))
+    text = "\n".join(" ".join(map(str, c)) for c in cases)
+    out = subprocess.run([str(tmp_path / "plan")], input=text, check=True, capture_output=True, text=True).stdout.split()
+    plans = [tuple(map(int, out[k:k + 3])) for k in range(0, len(out), 3)]
+    assert len(plans) == len(cases)
+    assert [p for p in plans[:len(FORMS)]] == [f[4] for f in FORMS]
+    assert {p[1] for p in plans[:len(FORMS)]} == {0, 1, 2, 3, 4} == {p[2] for p in plans[:len(FORMS)]}
+    for (cus, hidden, inter, *_), (cols, gate_up, down) in zip(cases, plans):
+        assert cols == (32 if 4 in (gate_up, down) else 64)
+        assert (gate_up == 0) == (hidden <= 1024) and (down == 0) == (inter <= 1024)
