@@ -15,12 +15,12 @@
 // order as the 256-token kernels: bit for bit their results.
 //
 // What bounds it: a step of a wave is some 80 (Q4_K) or 105 (Q6_K) vector instructions of decode and 4 T MFMAs, two waves a
-// SIMD; and around the steps 2 to 5 us until the first weights are there, 2.5 for adding up the slices and storing, 5 for
+// SIMD; and around the steps 2 to 5 us until the first weights are there, 1.5 for adding up the slices and storing, 5 for
 // the kernel that adds the workgroups' (in-kernel time stamps).  With the products of a step right behind its barrier all
 // waves waited for their first LDS reads together: 24 cases drawn over 1000 to 20000 rows and 19 to 740 tokens take 0.92 of
 // that, 2048 columns x 3000 rows of Q4_K at 700 tokens 21.2 us and 18.2.
-// 77 tokens, 4096 rows, 12288 columns of Q6_K: 25 us (218 in 256-token tiles on 32 CUs); 123 tokens, 1617 rows, 4096
-// columns of Q4_K: 13.7 us (49; 17 in tiles of 128 tokens alone).
+// 77 tokens, 4096 rows, 12288 columns of Q6_K: 23.8 us (24.4 with the sums of a row tile by one wave;
+// 218 in 256-token tiles on 32 CUs); 123 tokens, 1617 rows, 4096 columns of Q4_K: 11.2 us (11.9; 17 in tiles of 128 tokens alone).
 #include "prefill_decode.hpp"
 
 #include <cmath>
@@ -60,25 +60,27 @@ gemm_split_kernel(const uint8_t *__restrict__ w, const uint16_t *__restrict__ x,
         const uint32_t n = (z * KW + k + 1u) * nsb / ns - (z * KW + k) * nsb / ns;
         most = n > most ? n : most;
     }
-    // X: load j brings the 128 bytes of eight tokens; 16-byte unit c of token t lies at c ^ (t & 7)
+    // X: load j brings the 128 bytes of eight tokens; 16-byte unit c of token t lies at c ^ (t / 2 & 7): the LDS serves sixteen
+    // lanes of a fragment's read at once, 256 bytes, from sixteen different places (at c ^ (t & 7) tokens t and t + 8 met, and
+    // a read took 8 clocks for 4: 390 of the 2500 of a step of T = 3)
     constexpr uint32_t kBufs = x_bufs<W>(T, RW, KW);
     constexpr int kXLoads = 4 * T / RW;
     const uint8_t *xsrc[kXLoads];
 #pragma unroll
     for (int j = 0; j < kXLoads; ++j) {
         const uint32_t tl = 8u * (rw + RW * j) + (lane >> 3), t = tok0 + tl < tokens ? tok0 + tl : tokens - 1u;
-        xsrc[j] = reinterpret_cast<const uint8_t *>(x) + ((uint64_t)t * in_dim * 2u + 16u * ((lane & 7u) ^ (tl & 7u)));
+        xsrc[j] = reinterpret_cast<const uint8_t *>(x) + ((uint64_t)t * in_dim * 2u + 16u * ((lane & 7u) ^ (tl >> 1 & 7u)));
     }
     const uint32_t xlds = lev_lds_offset(lds) + kw * (kBufs * T * kTile) + rw * 1024u, steps = (sb1 - sb0) * 4u;
-    auto x_request = [&](uint32_t step) {
+    auto x_request = [&](uint32_t step, int from, int to) {   // loads from .. to - 1 of a step
         const uint32_t s = sb0 * 4u + (step < steps ? step : steps - 1u);   // past the end: any valid step, never read
 #pragma unroll
-        for (int j = 0; j < kXLoads; ++j) lev_load_lds16(xsrc[j] + (uint64_t)s * 128u, xlds + (step % kBufs) * (T * kTile) + j * (RW * 1024u));
+        for (int j = from; j < to; ++j) lev_load_lds16(xsrc[j] + (uint64_t)s * 128u, xlds + (step % kBufs) * (T * kTile) + j * (RW * 1024u));
     };
     const uint8_t *const xmine = lds + kw * (kBufs * T * kTile) + lr * 128u;
 
 #pragma unroll
-    for (uint32_t s = 0; s + 1u < kBufs; ++s) x_request(s);
+    for (uint32_t s = 0; s + 1u < kBufs; ++s) x_request(s, 0, kXLoads);
     W wt;
     wt.init(w, row0, rows, nsb, lds + KW * (kBufs * T * kTile) + wave * W::kArea);
     wt.request(sb0);
@@ -109,7 +111,7 @@ gemm_split_kernel(const uint8_t *__restrict__ w, const uint16_t *__restrict__ x,
         if (read >= 0) {
 #pragma unroll
             for (int t = 0; t < T; ++t)
-                a[read][t] = *reinterpret_cast<const f16x8 *>(xb + t * kTile + 16u * (wt.unit(read) ^ (lr & 7u)));
+                a[read][t] = *reinterpret_cast<const f16x8 *>(xb + t * kTile + 16u * (wt.unit(read) ^ (lr >> 1 & 7u)));
         }
         next();
 #pragma unroll
@@ -132,24 +134,42 @@ gemm_split_kernel(const uint8_t *__restrict__ w, const uint16_t *__restrict__ x,
             if (c == 0) wt.touch();   // the compiler's own wait for them goes here, behind ours for the X requested after them
             __builtin_amdgcn_sched_barrier(0);
             lev_barrier_lds();          // everybody's has, and everybody is done with the other buffer
-            x_request(step + kBufs - 1u);
-            __builtin_amdgcn_sched_barrier(0);
+            // Together, by all waves, right behind the barrier they wait in the issue for 400 to 800 clocks of a step's 3000. So
+            // they go out behind the step's products (in front of the weights' request) where the data is not wanted for another two
+            // steps and products are few (64 tokens x 12288 x 4096 of Q4_K 16.1 -> 15.4 us); else the data comes too
+            // late for that (500 x 2500 x 5120 of Q4_K 24.4 -> 25.8, 350 x 9000 x 1280 of Q6_K 17.4 -> 18.0).
+            constexpr bool kLater = kBufs == 4u && T <= 2;
+            constexpr int kHalf = (kXLoads + 1) / 2, kOf4[5] = {0, (kXLoads + 3) / 4, kHalf, kHalf + (kXLoads - kHalf + 1) / 2, kXLoads};
+            auto x_part = [&](int p) {
+                if (!kLater) return;
+                if (c != 0) x_request(step + kBufs - 1u, kOf4[p], kOf4[p + 1]);
+                else if (p < 2) x_request(step + kBufs - 1u, p ? kHalf : 0, p ? kXLoads : kHalf);
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            if (!kLater) {
+                x_request(step + kBufs - 1u, 0, kXLoads);
+                __builtin_amdgcn_sched_barrier(0);
+            }
             const uint8_t *const xb = xmine + (step % kBufs) * (T * kTile);
 #pragma unroll
-            for (int t = 0; t < T; ++t) a[0][t] = *reinterpret_cast<const f16x8 *>(xb + t * kTile + 16u * (wt.unit(0) ^ (lr & 7u)));
+            for (int t = 0; t < T; ++t) a[0][t] = *reinterpret_cast<const f16x8 *>(xb + t * kTile + 16u * (wt.unit(0) ^ (lr >> 1 & 7u)));
             phase(xb, 2, -1, [&] { b = wt.frag((c + 3) & 3, 3); });
+            x_part(0);
             phase(xb, 3, 1, [&] {
                 if (c == 0) wt.take();
                 if (c == 2) wt.half(1);
                 b = wt.frag(c, 0);
             });
+            x_part(1);
             if (c == 0) {
                 const uint32_t sb = sb0 + i + 1u;
                 wt.request(sb < sb1 ? sb : sb1 - 1u);
                 __builtin_amdgcn_sched_barrier(0);
             }
             phase(xb, 0, 2, [&] { b = wt.frag(c, 1); });
+            x_part(2);
             phase(xb, 1, 3, [&] { b = wt.frag(c, 2); });
+            x_part(3);
         }
     }
     phase(xmine, 2, -1, [&] { b = wt.frag(3, 3); });
@@ -158,38 +178,48 @@ gemm_split_kernel(const uint8_t *__restrict__ w, const uint16_t *__restrict__ x,
     for (uint32_t i = 4u * mine; i < 4u * most; ++i) asm volatile("s_barrier" ::: "memory");
     LEV_WAIT_VMCNT(0);   // the request past the end lands before the LDS is used again
 
-    if (KW > 1) {
-        // partial tiles of slices 1.. -> LDS, added to the first slice's in slice order
-        float *const red = reinterpret_cast<float *>(lds);
-        lev_barrier_lds();
-        if (kw != 0u) {
-#pragma unroll
-            for (int t = 0; t < T; ++t)
-#pragma unroll
-                for (int i = 0; i < 16; ++i) red[((((kw - 1u) * RW + rw) * T + t) * 16 + i) * 64 + lane] = acc[t][i];
-        }
-        lev_barrier_lds();
-        if (kw != 0u) return;
-#pragma unroll
-        for (uint32_t k = 1; k < KW; ++k)
-#pragma unroll
-            for (int t = 0; t < T; ++t)
-#pragma unroll
-                for (int i = 0; i < 16; ++i) acc[t][i] += red[((((k - 1u) * RW + rw) * T + t) * 16 + i) * 64 + lane];
-    }
     // a tile's 32 tokens from `first` on; past the tokens' end and for rows past the last one nothing is stored
     float *const dst = out + (uint64_t)zl * tokens * rows;
     const uint32_t at = row < rows ? (4u * lh * rows + row) * 4u : lev_buffer::kNothing;
-#pragma unroll
-    for (int t = 0; t < T; ++t) {
+    auto store = [&](int t, int i, float v) {
         const uint32_t first = tok0 + 32u * t, here = first < tokens ? (tokens - first < 32u ? tokens - first : 32u) : 0u;
         const lev_buffer tile_out(dst + (uint64_t)(here ? first : 0u) * rows, here * rows * 4u);
+        const uint32_t tok = (uint32_t)(8 * (i / 4) + (i % 4)) * rows * 4u;
+        if (add) v += __uint_as_float(tile_out.load4(at, 0, tok));
+        tile_out.store4(__float_as_uint(v), at, 0, tok);
+    };
+    // A wave adds up and stores one KW-th of its rows' outputs, registers i of part i / (16 / KW): it leaves the others'
+    // parts in LDS and adds theirs to its own in slice order.  (By the waves of the first slice alone: 9 of 50 thousand
+    // clocks at 77 tokens x 4096 x 12288.)
+    constexpr int kPart = 16 / KW;
+    float *const red = reinterpret_cast<float *>(lds);
+    auto left = [&](uint32_t part, uint32_t from, int t, int i) -> float & {   // what slice `from` leaves for the wave of `part`
+        return red[(((part * (KW - 1u) + (from < part ? from : from - 1u)) * RW + rw) * (T * kPart) + t * kPart + i % kPart) * 64 + lane];
+    };
+    if (KW > 1) {
+        lev_barrier_lds();
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const uint32_t tok = (uint32_t)(8 * (i / 4) + (i % 4)) * rows * 4u;
-            const float v = add ? acc[t][i] + __uint_as_float(tile_out.load4(at, 0, tok)) : acc[t][i];
-            tile_out.store4(__float_as_uint(v), at, 0, tok);
+        for (uint32_t p = 0; p < KW; ++p) {
+            if (p == kw) continue;
+#pragma unroll
+            for (int t = 0; t < T; ++t)
+#pragma unroll
+                for (int i = p * kPart; i < (int)(p + 1u) * kPart; ++i) left(p, kw, t, i) = acc[t][i];
         }
+        lev_barrier_lds();
+    }
+#pragma unroll
+    for (uint32_t p = 0; p < KW; ++p) {
+        if (p != kw) continue;
+#pragma unroll
+        for (int t = 0; t < T; ++t)
+#pragma unroll
+            for (int i = p * kPart; i < (int)(p + 1u) * kPart; ++i) {
+                float v = p == 0u ? acc[t][i] : left(p, 0u, t, i);
+#pragma unroll
+                for (uint32_t k = 1; k < KW; ++k) v += k == p ? acc[t][i] : left(p, k, t, i);
+                store(t, i, v);
+            }
     }
 }
 
