@@ -10,18 +10,22 @@
 //     nobody else's, so X never goes through LDS: a small kernel in front puts X into the order in which the lanes of a
 //     fragment take it (1 KB of consecutive bytes a fragment), and a wave requests a fragment four or eight products ahead
 //     of its use, straight into registers;
-//   * waves 4..7 decode, one 32-row tile each (RT = 3: three of them): every weight is decoded once a workgroup, a step
-//     ahead, and handed over as B fragments in two LDS buffers of 4 RT KB, one barrier a step.
-// The multiplying waves run two groups of products behind the barriers: groups 2 and 3 of a step are multiplied behind the
-// next barrier, from fragments read in front of it, while the first fragments of the new step come in.
+//   * waves 4..7 decode, one 32-row tile each (RT = 3: three of them): every weight is decoded once a workgroup, a span of two
+//     steps (half a superblock) ahead, and handed over as B fragments in two LDS buffers of 8 RT KB, one barrier a span.
+// The multiplying waves run two groups of products behind the barriers: the last two groups of a span are multiplied behind the
+// next barrier, from fragments read in front of it, while the first fragments of the new span come in.
 //
 // Why this split.  A lone wave of a SIMD issues a vector instruction every six clocks, two waves one every three to five,
 // and an MFMA leaves the vector pipe half of its 32 clocks, so decode and products on different waves of a SIMD cover each
-// other.  What the LDS has to carry bounds the tile: with X in LDS as well (the kernels this one took the place of) it was
-// 124 KB a step of 96 x 256 x 64, 990 clocks beside 770 of MFMAs; 60 KB here.  512 tokens, 4096 columns, us under a
-// sustained load: 12288 rows of Q4_K 58.9 before and 55.6, of Q6_K 76.7 and 60.0, 32000 rows of Q6_K 175.8 and 143.4
-// (0.94 PFLOP/s).  Without the decode 44, without the X loads no less: what is left is the clock, which under these
-// products falls to 1.5 to 1.8 GHz (a loop of MFMAs alone takes 33 us for the first of these, the library's fp16 product 51).
+// other.  What the LDS has to carry bounds the tile: with X in LDS as well it was
+// 124 KB a step of 96 x 256 x 64, 990 clocks beside 770 of MFMAs; 60 KB here.  A span is two steps because a superblock's
+// steps take the decoding waves unequal times (new weights and factors, then none): at a barrier a step both sides waited
+// for 350 to 520 of a step's 1260 clocks.  And the compiler must not move a superblock's requests and factors in among
+// its fragments: with the order kept a step takes 980 clocks where it took 1260.
+// 512 tokens, 4096 columns, us under a sustained load: 12288 rows of Q4_K 57.2 before and 55.0, of Q6_K 61.2 and 58.4, 32000 rows of
+// Q6_K 139 and 131; 9456 x 9472 of Q4_K 100.6 and 96.2.  What bounds it is power: of the 22 % fewer clocks the first of these keeps 4,
+// since the clock under these products falls from 1.73 to 1.47 GHz (a loop of MFMAs alone on random operands runs at 1.45 and
+// takes 35 us for it; the library's fp16 product 51).  The Q6_K one, 1200 clocks at 1.64 GHz, waits for its decoding waves.
 //
 // K order inside a 64-step is permuted consistently on both operands (unit_of of the formats' weights); the sums are formed
 // in the order in which a wave of gemm_split.hip that takes all of K forms them: the same bits.
@@ -58,48 +62,57 @@ __global__ void __launch_bounds__(kWideThreads, 2)
 gemm_wide_kernel(const uint8_t *__restrict__ w, const uint8_t *__restrict__ xf, float *__restrict__ y, uint32_t in_dim,
                  uint32_t rows, uint32_t tokens, uint32_t row_tiles, uint32_t tok_tiles) {
     constexpr int RING = RT == 4 ? 4 : 8;      // groups of X requested ahead, as many as the registers hold
-    constexpr uint32_t kBuf = RT * 4u * kFrag;
+    constexpr uint32_t kBuf = RT * 8u * kFrag;
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
     const uint32_t lane = threadIdx.x & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const uint32_t lr = lane & 31u, lh = lane >> 5;
     const uint32_t tile = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3), rt = tile / tok_tiles;
     if (rt >= row_tiles) return;
     const uint32_t row0 = rt * (32u * RT), tt0 = (tile - rt * tok_tiles) * (4u * kTM);
-    const uint32_t nsb = in_dim >> 8, nsteps = nsb * 4u;
+    const uint32_t nsb = in_dim >> 8, nspans = nsb * 2u;
     if (wave >= 4u) {
         const uint32_t f = wave - 4u;
         if (f >= (uint32_t)RT) {
-            for (uint32_t ks = 0; ks < nsteps; ++ks) asm volatile("s_barrier" ::: "memory");   // nothing to decode
+            for (uint32_t k = 0; k < nspans; ++k) asm volatile("s_barrier" ::: "memory");   // nothing to decode
             return;
         }
         W wt;
         wt.init(w, row0 + 32u * f, rows, nsb, lds + 2u * kBuf + f * W::kArea);
-        wt.request(0);
-        wt.touch();
-        wt.take();
         uint8_t *const dst = lds + f * kFrag + lane * 16u;
-        auto produce = [&](int c, uint32_t buf) {
+        auto produce = [&](uint32_t hf) {   // the span of half a superblock
 #pragma unroll
-            for (int q = 0; q < 4; ++q) *reinterpret_cast<f16x8 *>(dst + buf * kBuf + q * (RT * kFrag)) = wt.frag(c, q);
+            for (uint32_t g = 0; g < 8u; ++g)
+                *reinterpret_cast<f16x8 *>(dst + hf * kBuf + g * (RT * kFrag)) = wt.frag(2 * hf + (g >> 2), g & 3u);
         };
-        produce(0, 0u);
+        auto next = [&](uint32_t sb) {   // the superblock whose bytes are here, and the request of the one behind it
+            __builtin_amdgcn_sched_barrier(0);
+            wt.touch();
+            __builtin_amdgcn_sched_barrier(0);
+            wt.take();
+            __builtin_amdgcn_sched_barrier(0);
+            wt.request(sb < nsb ? sb : nsb - 1u);
+            __builtin_amdgcn_sched_barrier(0);
+            produce(0u);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto meet = [&] {
+            __builtin_amdgcn_s_waitcnt(0xC07F);
+            asm volatile("s_barrier" ::: "memory");
+        };
+        wt.request(0);
+        next(1u);
         for (uint32_t i = 0; i < nsb; ++i) {
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                __builtin_amdgcn_s_waitcnt(0xC07F);
-                asm volatile("s_barrier" ::: "memory");
-                if (c == 0) wt.request(i + 1u < nsb ? i + 1u : nsb - 1u);
-                if (c == 1) wt.half(1);
-                if (c == 3) {
-                    wt.touch();
-                    wt.take();
-                }
-                produce((c + 1) & 3, (c + 1) & 1);
-            }
+            meet();
+            __builtin_amdgcn_sched_barrier(0);
+            wt.half(1);
+            produce(1u);
+            __builtin_amdgcn_sched_barrier(0);
+            meet();
+            next(i + 2u);
         }
         return;
     }
-    const uint32_t ngroup = nsteps * 4u;
+    const uint32_t ngroup = nsb * 16u;
     const uint32_t tile_bytes = ngroup * kFrag;
     const uint32_t tt = tt0 + wave * kTM, last_tt = (tokens + 31u) / 32u - 1u;
     const lev_buffer xb0(xf + (uint64_t)(tt < last_tt ? tt : last_tt) * tile_bytes, tile_bytes);
@@ -120,16 +133,16 @@ gemm_wide_kernel(const uint8_t *__restrict__ w, const uint8_t *__restrict__ xf, 
             for (int i = 0; i < 16; ++i) acc[r][m][i] = 0.f;
     f16x8 b[4][RT];
     const uint8_t *const bb = lds + lane * 16u;
-    auto b_read = [&](int q, int r, uint32_t buf) { b[q][r] = *reinterpret_cast<const f16x8 *>(bb + buf * kBuf + (q * RT + r) * kFrag); };
-    // group q of step parity p: products, meanwhile group `rq` of buffer rbuf is read
-    auto phase = [&](int q, int p, uint32_t n, int rq, uint32_t rbuf) {
-        const int slot = (4 * p + q) % RING;
+    auto b_read = [&](int g, int r, uint32_t buf) { b[g & 3][r] = *reinterpret_cast<const f16x8 *>(bb + buf * kBuf + (g * RT + r) * kFrag); };
+    // products of group g of a span whose first group is n0, meanwhile group `rg` of buffer rbuf is read
+    auto phase = [&](int g, uint32_t n0, int rg, uint32_t rbuf) {
+        const int slot = g % RING;
 #pragma unroll
         for (int i = 0; i < RT * kTM; ++i) {
             const int r = i % RT, m = i / RT;
-            acc[r][m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, xr[slot][m]), b[q][r], acc[r][m], 0, 0, 0);
-            if (rq >= 0 && i < RT) b_read(rq, i, rbuf);
-            if (i == RT * kTM - 1) x_request(n + RING, slot);
+            acc[r][m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, xr[slot][m]), b[g & 3][r], acc[r][m], 0, 0, 0);
+            if (rg >= 0 && i < RT) b_read(rg, i, rbuf);
+            if (i == RT * kTM - 1) x_request(n0 + g + RING, slot);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
@@ -143,28 +156,28 @@ gemm_wide_kernel(const uint8_t *__restrict__ w, const uint8_t *__restrict__ xf, 
 #pragma unroll
     for (int r = 0; r < RT; ++r) b_read(1, r, 0u);
     __builtin_amdgcn_sched_barrier(0);
-    phase(0, 0, 0u, 2, 0u);
-    phase(1, 0, 1u, 3, 0u);
-    auto step = [&](auto parity, uint32_t ks) {
-        constexpr int p = decltype(parity)::value;
+#pragma unroll
+    for (int g = 0; g < 6; ++g) phase(g, 0u, g + 2, 0u);
+    auto span = [&](auto parity, uint32_t k) {
+        constexpr uint32_t p = decltype(parity)::value;
         meet();
 #pragma unroll
         for (int r = 0; r < RT; ++r) b_read(0, r, p);
         __builtin_amdgcn_sched_barrier(0);
-        phase(2, 1 - p, ks * 4u - 2u, -1, 0u);
-        phase(3, 1 - p, ks * 4u - 1u, 1, p);
-        phase(0, p, ks * 4u, 2, p);
-        phase(1, p, ks * 4u + 1u, 3, p);
+        phase(6, k * 8u - 8u, -1, 0u);
+        phase(7, k * 8u - 8u, 1, p);
+#pragma unroll
+        for (int g = 0; g < 6; ++g) phase(g, k * 8u, g + 2, p);
     };
-    uint32_t ks = 1;
-    for (; ks + 1u < nsteps; ks += 2u) {
-        step(std::integral_constant<int, 1>{}, ks);
-        step(std::integral_constant<int, 0>{}, ks + 1u);
+    uint32_t k = 1;
+    for (; k + 1u < nspans; k += 2u) {
+        span(std::integral_constant<uint32_t, 1>{}, k);
+        span(std::integral_constant<uint32_t, 0>{}, k + 1u);
     }
-    step(std::integral_constant<int, 1>{}, ks);
+    span(std::integral_constant<uint32_t, 1>{}, k);
     __builtin_amdgcn_s_waitcnt(0xC07F);
-    phase(2, 1, ks * 4u + 2u, -1, 0u);
-    phase(3, 1, ks * 4u + 3u, -1, 0u);
+    phase(6, k * 8u, -1, 0u);
+    phase(7, k * 8u, -1, 0u);
     // past the tokens' end and for rows past the last one nothing is stored
 #pragma unroll
     for (int m = 0; m < kTM; ++m) {
@@ -181,7 +194,7 @@ gemm_wide_kernel(const uint8_t *__restrict__ w, const uint8_t *__restrict__ xf, 
 
 template <typename W, int RT>
 hipError_t launch_as(lev_ctx *ctx, const uint8_t *w, const uint8_t *xf, float *y, uint32_t in_dim, uint32_t rows, uint32_t tokens) {
-    constexpr size_t lds = 2u * RT * 4u * kFrag + RT * W::kArea;
+    constexpr size_t lds = 2u * RT * 8u * kFrag + RT * W::kArea;
     if (hipError_t e = lev_allow_lds(ctx, reinterpret_cast<const void *>(&gemm_wide_kernel<W, RT>), lds); e != hipSuccess) return e;
     const uint32_t row_tiles = (rows + 32u * RT - 1u) / (32u * RT), tok_tiles = (tokens + 128u * kTM - 1u) / (128u * kTM);
     hipLaunchKernelGGL((gemm_wide_kernel<W, RT>), dim3((row_tiles * tok_tiles + 7u) / 8u * 8u), dim3(kWideThreads), lds, ctx->stream,

@@ -9,22 +9,23 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-// Of the 8 sub-blocks of a superblock: d*sc, times the power of two that q4k_frag wants (2^24 for the sub-blocks of the low
-// nibbles, 2^20 for those of the high ones), and dmin*m (lev-cpu/src/lib.rs:64-74, 117-124).
-__device__ __forceinline__ void q4k_all_factors(const lev_u32x4 hdr, float d1[8], float mm[8]) {
+// Of sub-blocks 4 HALF .. 4 HALF + 3 of a superblock: d*sc, times the power of two that q4k_frag wants (2^24 for the sub-blocks
+// of the low nibbles, 2^20 for those of the high ones), and dmin*m (lev-cpu/src/lib.rs:64-74, 117-124).
+template <int HALF>
+__device__ __forceinline__ void q4k_factors(const lev_u32x4 hdr, float d1[8], float mm[8]) {
     const float d = lev_f16_bits_to_f32(hdr.x & 0xFFFFu) * 0x1p20f, d16 = d * 16.f;
     const float dmin = lev_f16_bits_to_f32(hdr.x >> 16);
     const uint32_t s03 = hdr.y, s47 = hdr.z, s811 = hdr.w;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         uint32_t sc = (s03 >> (8 * j)) & 63u, mn = (s47 >> (8 * j)) & 63u;
-        d1[j] = (j & 1 ? d : d16) * (float)sc;
-        mm[j] = dmin * (float)mn;
-        uint32_t a = (s811 >> (8 * j)) & 0xFFu;
-        uint32_t sc2 = (a & 0x0Fu) | (((s03 >> (8 * j + 6)) & 3u) << 4);
-        uint32_t mn2 = (a >> 4) | (((s47 >> (8 * j + 6)) & 3u) << 4);
-        d1[4 + j] = (j & 1 ? d : d16) * (float)sc2;
-        mm[4 + j] = dmin * (float)mn2;
+        if (HALF) {
+            const uint32_t a = (s811 >> (8 * j)) & 0xFFu;
+            sc = (a & 0x0Fu) | (((s03 >> (8 * j + 6)) & 3u) << 4);
+            mn = (a >> 4) | (((s47 >> (8 * j + 6)) & 3u) << 4);
+        }
+        d1[4 * HALF + j] = (j & 1 ? d : d16) * (float)sc;
+        mm[4 * HALF + j] = dmin * (float)mn;
     }
 }
 
@@ -88,7 +89,7 @@ struct weights_q4k {
     static constexpr uint32_t kArea = 0u;    // LDS bytes a wave
     const uint8_t *row;
     uint32_t lh;
-    lev_u32x4 nhdr, nqs[4], qs[4];
+    lev_u32x4 nhdr, hdr, nqs[4], qs[4];
     float d1[8], mm[8];
     __device__ __forceinline__ void init(const uint8_t *w, uint32_t row0, uint32_t rows, uint32_t nsb, uint8_t *) {
         const uint32_t lane = threadIdx.x & 63u, r = row0 + (lane & 31u);
@@ -109,12 +110,18 @@ struct weights_q4k {
     __device__ __forceinline__ void take() {
 #pragma unroll
         for (int c = 0; c < 4; ++c) qs[c] = nqs[c];
-        q4k_all_factors(nhdr, d1, mm);
+        hdr = nhdr;
+        half(0);
     }
-    __device__ __forceinline__ void half(int) {}
+    // the factors of half a column
+    __device__ __forceinline__ void half(int hf) {
+        if (hf) q4k_factors<1>(hdr, d1, mm);
+        else q4k_factors<0>(hdr, d1, mm);
+    }
     __device__ __forceinline__ void clear() {   // fragments of zeros
 #pragma unroll
         for (int c = 0; c < 4; ++c) qs[c] = lev_u32x4{0u, 0u, 0u, 0u};
+        hdr = lev_u32x4{0u, 0u, 0u, 0u};
 #pragma unroll
         for (int j = 0; j < 8; ++j) d1[j] = mm[j] = 0.f;
     }
