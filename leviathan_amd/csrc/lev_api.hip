@@ -281,8 +281,7 @@ using norm_adds = lev_norm_adds;
 // vector and the gains are requested together, 16 bytes a lane, and x stays in registers between the two
 // passes: one memory round trip.  V = 16-byte pieces a lane holds; V = 0 takes any length and alignment,
 // a float at a time, and reads x twice.  Measured in a recorded chain of 56 operators with three of these a
-// layer: 276 us with 256 threads that read x twice and the library's 1 / sqrt in f64, 189 with this (the mean is
-// still an f64 division).
+// layer: 276 us with 256 threads that read x twice and the library's 1 / sqrt in f64, 189 with this.
 template <int V, bool ADDS>
 __device__ __forceinline__ void rmsnorm_vector(const float *__restrict__ x, float *__restrict__ y, const float *__restrict__ w,
                                                uint32_t n, float eps, const norm_adds &adds) {
@@ -293,6 +292,7 @@ __device__ __forceinline__ void rmsnorm_vector(const float *__restrict__ x, floa
     const lev_f32x4 *x4 = reinterpret_cast<const lev_f32x4 *>(xv), *w4 = reinterpret_cast<const lev_f32x4 *>(w);
     constexpr int R = V ? V : 1;
     lev_f32x4 v[R], g[R], ad[norm_adds::kMost][R];
+    double per = 1.0 / (double)n;
     float ss = 0.f;
     if (V) {
 #pragma unroll
@@ -318,6 +318,7 @@ __device__ __forceinline__ void rmsnorm_vector(const float *__restrict__ x, floa
                 }
             }
         }
+        lev_pin(per);
 #pragma unroll
         for (int k = 0; k < R; ++k)
 #pragma unroll
@@ -331,9 +332,7 @@ __device__ __forceinline__ void rmsnorm_vector(const float *__restrict__ x, floa
     ss = lev_wave_sum_broadcast(ss);
     if ((t & 63u) == 0u) part[t >> 6] = ss;
     lev_barrier_lds();   // (the gains may still be on their way)
-    double tot = 0.0;
-    for (uint32_t k = 0; k < nt >> 6; ++k) tot += (double)part[k];
-    const float inv = (float)lev_rsqrt_f64(tot / (double)n + (double)eps);
+    const float inv = lev_norm_scale(part, nt >> 6, per, eps);
     if (V) {
 #pragma unroll
         for (int k = 0; k < R; ++k) {
@@ -394,6 +393,8 @@ rmsnorm_pair_kernel(norm_pair p, const float *__restrict__ y, float *__restrict_
 #pragma unroll
     for (int m = 0; m < norm_adds::kMost; ++m)
         if (m < adds.count && m != p.own) ad[m] = vec(adds.x[m])[i];
+    double per = 1.0 / (double)n;
+    lev_pin(per);
     float sa = 0.f, sb = 0.f;
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
@@ -404,9 +405,7 @@ rmsnorm_pair_kernel(norm_pair p, const float *__restrict__ y, float *__restrict_
     sb = lev_wave_sum_broadcast(sb);
     if ((t & 63u) == 0u) part[0][t >> 6] = sa, part[1][t >> 6] = sb;
     lev_barrier_lds();   // (gains and addends may still be on their way)
-    double ta = 0.0, tb = 0.0;
-    for (uint32_t k = 0; k < nt >> 6; ++k) ta += (double)part[0][k], tb += (double)part[1][k];
-    const float ia = (float)lev_rsqrt_f64(ta / (double)n + (double)p.eps), ib = (float)lev_rsqrt_f64(tb / (double)n + (double)eps);
+    const float ia = lev_norm_scale(part[0], nt >> 6, per, p.eps), ib = lev_norm_scale(part[1], nt >> 6, per, eps);
     lev_f32x4 x = a * ia, o = b * ib;
     if (p.wx) x = x * ga;
     if (wy) o = o * gb;

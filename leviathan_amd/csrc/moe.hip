@@ -1157,15 +1157,15 @@ moe_gate_up_and_gemv(moe_args a, const float *__restrict__ x, const int32_t *ids
         lev_f32x4 *const s4 = reinterpret_cast<lev_f32x4 *>(tail.s);
         lev_f32x4 v = i < n4 ? s4[i] : lev_f32x4{0.f, 0.f, 0.f, 0.f}, w = {1.f, 1.f, 1.f, 1.f};
         if (tail.ws) w = reinterpret_cast<const lev_f32x4 *>(tail.ws)[i < n4 ? i : 0u];
+        double per = 1.0 / (double)tail.n;
+        lev_pin(per);
         float ss = 0.f;
 #pragma unroll
         for (int c = 0; c < 4; ++c) ss = fmaf(v[c], v[c], ss);
         ss = lev_wave_sum_broadcast(ss);
         if ((i & 63u) == 0u) part[i >> 6] = ss;
         lev_barrier_lds();
-        double tot = 0.0;
-        for (int k = 0; k < NW; ++k) tot += (double)part[k];
-        v = v * (float)lev_rsqrt_f64(tot / (double)tail.n + (double)tail.eps);
+        v = v * lev_norm_scale(part, NW, per, tail.eps);
         if (tail.ws) v = v * w;
         if (i < n4) s4[i] = v;
         return;

@@ -24,7 +24,7 @@ constexpr size_t ffn_lds(int nw) { return 2u * kFfnPart + kFfnSums + (size_t)nw 
 // The wave's 256 values of x, normalised as lev_hip_rmsnorm does it: squares in f32 per wave, f64 across the waves.
 template <int NW>
 __device__ __forceinline__ void ffn_normalise(const lev_ffn_args &a, lev_f32x4 &v, const lev_f32x4 &gain, bool live, float *s_ss,
-                                              uint32_t wave, uint32_t lane) {
+                                              double per, uint32_t wave, uint32_t lane) {
     v = q4m_mask_activations(v, live);
     float ss = 0.f;
 #pragma unroll
@@ -32,10 +32,7 @@ __device__ __forceinline__ void ffn_normalise(const lev_ffn_args &a, lev_f32x4 &
     ss = lev_wave_sum_broadcast(ss);
     if (lane == 0u) s_ss[wave] = ss;
     lev_barrier_lds();
-    double tot = 0.0;
-    for (int k = 0; k < NW; ++k) tot += (double)s_ss[k];
-    const float inv = (float)lev_rsqrt_f64(tot / (double)a.hidden + (double)a.eps);
-    v = v * inv;
+    v = v * lev_norm_scale(s_ss, NW, per, a.eps);
     if (a.gain) v = v * gain;
     if (!live) v = lev_f32x4{0.f, 0.f, 0.f, 0.f};                 // (an infinite inv made NaNs of the zeros past the end)
 }
@@ -56,7 +53,7 @@ struct ffn_front {
             if (m < f.adds.count && m != f.own) ad[m] = q4m_load_activations(f.adds.x[m], T, n4, unused);
     }
     template <int NW>
-    __device__ __forceinline__ lev_f32x4 value(const lev_norm_front &f, uint32_t n, bool active, float *sums, uint32_t wave, uint32_t lane) {
+    __device__ __forceinline__ lev_f32x4 value(const lev_norm_front &f, double per, bool active, float *sums, uint32_t wave, uint32_t lane) {
         b = q4m_mask_activations(b, live && active);
         float sb = 0.f, sa = 0.f;
 #pragma unroll
@@ -70,14 +67,10 @@ struct ffn_front {
         sb = lev_wave_sum_broadcast(sb);
         if (lane == 0u) sums[wave] = sb, sums[16u + wave] = sa;
         lev_barrier_lds();
-        double tb = 0.0, ta = 0.0;
-        for (int k = 0; k < NW; ++k) tb += (double)sums[k];
-        const float ib = (float)lev_rsqrt_f64(tb / (double)n + (double)f.eps);
-        lev_f32x4 o = b * ib, x = {0.f, 0.f, 0.f, 0.f};
+        lev_f32x4 o = b * lev_norm_scale(sums, NW, per, f.eps), x = {0.f, 0.f, 0.f, 0.f};
         if (f.wy) o = o * gb;
         if (f.s) {
-            for (int k = 0; k < NW; ++k) ta += (double)sums[16 + k];
-            x = a * (float)lev_rsqrt_f64(ta / (double)n + (double)f.eps_s);
+            x = a * lev_norm_scale(sums + 16, NW, per, f.eps_s);
             if (f.ws) x = x * ga;
         }
 #pragma unroll
@@ -127,13 +120,15 @@ __device__ __forceinline__ void ffn_gate_up(const lev_ffn_args &a, uint8_t *smem
     uint32_t Ga[9], Ua[9];
     uint32_t i0 = i_begin;
     issue(i0, Ga, Ua);
+    double per = 1.0 / (double)a.hidden;
+    lev_pin(per);
     __builtin_amdgcn_sched_barrier(0);
 
     if (FRONT) {
-        v = before.value<NW>(front, a.hidden, active, s_ss + 16, wave, lane);
+        v = before.value<NW>(front, per, active, s_ss + 16, wave, lane);
         if (blockIdx.x == 0u && active && live) reinterpret_cast<lev_f32x4 *>(front.out)[64u * T + lane] = v;
     }
-    ffn_normalise<NW>(a, v, gain, live && active, s_ss, wave, lane);
+    ffn_normalise<NW>(a, v, gain, live && active, s_ss, per, wave, lane);
     if (blockIdx.x == 0u && active && live) reinterpret_cast<lev_f32x4 *>(a.h)[64u * T + lane] = v;
 
     uint8_t *area = smem + 2u * kFfnPart + kFfnSums + (size_t)wave * (kQ4mTaskArea + kQ4mZeroBytes), *zero = area + kQ4mTaskArea;
@@ -219,9 +214,11 @@ __device__ __forceinline__ void ffn_gate_up_and_scores(const lev_ffn_args &a, co
         v = q4m_load_activations(a.x, T, n4, live);
     }
     if (a.gain) gain = q4m_load_activations(a.gain, T, n4, unused);
-    if (FRONT) v = before.value<NW>(front, a.hidden, wave < ntask, s_ss + 16, wave, lane);
+    double per = 1.0 / (double)a.hidden;
+    lev_pin(per);
+    if (FRONT) v = before.value<NW>(front, per, wave < ntask, s_ss + 16, wave, lane);
     live = live && wave < ntask;
-    ffn_normalise<NW>(a, v, gain, live, s_ss, wave, lane);
+    ffn_normalise<NW>(a, v, gain, live, s_ss, per, wave, lane);
     if (live) reinterpret_cast<lev_f32x4 *>(s_h)[64u * T + lane] = v;
     lev_barrier_lds();
     moe_score_few(r.wr, s_h, r.scores, r.hidden, r.experts, (blockIdx.x - gate_blocks) * (NW / 4) + part, 0u, threadIdx.x & 255u,
