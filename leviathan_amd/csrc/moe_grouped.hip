@@ -44,12 +44,14 @@ moe_group_kernel(const int32_t *__restrict__ ids, uint32_t pairs, uint32_t exper
                  uint8_t *__restrict__ valid, int *__restrict__ flag, lev_grp_item *items,
                  lev_grp_start *__restrict__ starts, uint32_t grid, uint32_t rpi_gu, uint32_t rpi_dn, uint32_t w1_gu,
                  uint32_t w2_gu, uint32_t w1_dn, uint32_t w2_dn, uint32_t s0_gu, uint32_t s0_dn) {
-    // [experts] counts | cursors | first pair | first item of more than four pairs | first other item
+    // [experts] counts | cursors | first pair | first item of more than four pairs | first other item; [items] expert * 16 + count
     extern __shared__ int32_t s_cnt[];
     int32_t *s_cur = s_cnt + experts, *s_first = s_cur + experts, *s_big = s_first + experts, *s_small = s_big + experts;
+    int32_t *s_item = s_small + experts;
     const uint32_t tid = threadIdx.x;
+    // (barriers that leave stores on their way: the workgroup exchanges nothing but LDS)
     for (uint32_t e = tid; e < experts; e += 1024u) s_cnt[e] = 0;
-    __syncthreads();
+    lev_barrier_lds();
     bool bad_seen = false;
     int32_t e_own = -1;                          // the thread's first pair, kept for the placement: its expert, or -1
     for (uint32_t p = tid; p < pairs; p += 1024u) {
@@ -72,19 +74,20 @@ moe_group_kernel(const int32_t *__restrict__ ids, uint32_t pairs, uint32_t exper
         bad_seen = bad_seen || !ok;
     }
     if (bad_seen) atomicOr(flag, kFlagBadExpertId);
-    __syncthreads();
-    // exclusive scan of the counts (experts <= 4096): thread i takes experts 4i..4i+3, the waves scan
-    // their threads' sums by shuffles and meet in LDS.  One scan carries three counts of at most
+    lev_barrier_lds();
+    // exclusive scan of the counts (experts <= 4096: up to four a thread, side by side).  One scan carries three counts of at most
     // 2^20 each in 21-bit fields: pairs, items of more than four pairs, other items.
     __shared__ uint64_t s_wave[16];
     uint32_t n_big = 0u, n_all = 0u;            // items of more than four pairs, all items
     {
+        const uint32_t per_thread = (experts + 1023u) >> 10;
         int32_t c4[4], big4[4], small4[4];
         constexpr int32_t ip = kG8NT, ish = ip == 8 ? 3 : 2;
         uint64_t local = 0;
 #pragma unroll
         for (uint32_t k = 0; k < 4u; ++k) {
-            const uint32_t e = 4u * tid + k;
+            if (k >= per_thread) break;
+            const uint32_t e = per_thread * tid + k;
             c4[k] = e < experts ? s_cnt[e] : 0;
             // work items of the integer matrix-core kernels: runs of at most kG8NT pairs of one expert
             const int32_t full = c4[k] >> ish, rem = c4[k] - (full << ish);
@@ -92,26 +95,14 @@ moe_group_kernel(const int32_t *__restrict__ ids, uint32_t pairs, uint32_t exper
             small4[k] = (ip > 4 ? 0 : full) + (rem > 0 && rem <= 4 ? 1 : 0);
             local += (uint64_t)c4[k] | (uint64_t)big4[k] << 21 | (uint64_t)small4[k] << 42;
         }
-        uint64_t incl = local;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const uint64_t o = __shfl_up(incl, off);
-            if ((int)(tid & 63u) >= off) incl += o;
-        }
-        if ((tid & 63u) == 63u) s_wave[tid >> 6] = incl;
-        __syncthreads();
-        uint64_t before = incl - local, all = 0;
-#pragma unroll
-        for (uint32_t w = 0; w < 16u; ++w) {
-            const uint64_t v = s_wave[w];
-            before += w < (tid >> 6) ? v : 0u;
-            all += v;
-        }
+        uint64_t before, all;
+        lev_scan_1024(local, s_wave, before, all);
         int32_t run = (int32_t)(before & 0x1FFFFFu);
         const int32_t first_pair = run;
 #pragma unroll
         for (uint32_t k = 0; k < 4u; ++k) {
-            const uint32_t e = 4u * tid + k;
+            if (k >= per_thread) break;
+            const uint32_t e = per_thread * tid + k;
             if (e < experts) s_cur[e] = run;
             run += c4[k];
         }
@@ -125,7 +116,8 @@ moe_group_kernel(const int32_t *__restrict__ ids, uint32_t pairs, uint32_t exper
         int32_t prun = first_pair;
 #pragma unroll
         for (uint32_t k = 0; k < 4u; ++k) {
-            const uint32_t e = 4u * tid + k;
+            if (k >= per_thread) break;
+            const uint32_t e = per_thread * tid + k;
             if (e < experts) {
                 s_first[e] = prun;
                 s_big[e] = brun;
@@ -134,7 +126,9 @@ moe_group_kernel(const int32_t *__restrict__ ids, uint32_t pairs, uint32_t exper
             const int32_t n = big4[k] + small4[k];
             for (int32_t j = 0; j < n; ++j) {
                 const int32_t left = c4[k] - j * ip, count = left < ip ? left : ip;
-                lev_grp_item *it = items + (count > 4 ? brun++ : srun++);
+                const int32_t at = count > 4 ? brun++ : srun++;
+                s_item[at] = (int32_t)e * 16 + count;
+                lev_grp_item *it = items + at;
                 it->expert = (int32_t)e;
                 it->count = count;
                 it->first = prun + j * ip;
@@ -142,7 +136,7 @@ moe_group_kernel(const int32_t *__restrict__ ids, uint32_t pairs, uint32_t exper
             prun += c4[k];
         }
     }
-    __syncthreads();
+    lev_barrier_lds();   // (the items' headers are still on their way to memory: what is read of them below is in LDS as well)
     const uint32_t sid = 1023u - tid;   // (the high threads: the low ones place the first 1024 pairs below)
     if (sid < 2u * grid) {
         // Where the workgroups of the two expert kernels start.  A round of an item of more than
@@ -168,9 +162,9 @@ moe_group_kernel(const int32_t *__restrict__ ids, uint32_t pairs, uint32_t exper
         st.first_round = rounds_before(per * L + rest * L / grid);
         st.end_round = rounds_before(per * (L + 1u) + rest * (L + 1u) / grid);
         st.item = st.first_round / rpi;
-        const lev_grp_item *it = items + (st.item < n_all ? st.item : 0u);   // (written before the barrier)
-        st.expert = it->expert;
-        st.count = it->count;
+        const int32_t header = n_all ? s_item[st.item < n_all ? st.item : 0u] : 0;
+        st.expert = header >> 4;
+        st.count = header & 15;
         st.pad[0] = st.pad[1] = st.pad[2] = 0u;
         starts[sid] = st;
     }
@@ -626,6 +620,11 @@ grouped_layout layout_of(const lev_moe_grouped_args &a) {
     return L;
 }
 
+// LDS of the grouping kernel: what it keeps of every expert and of every item (see layout_of).
+size_t group_lds(const lev_moe_grouped_args &a) {
+    return (size_t)5 * a.experts * 4 + ((size_t)a.tokens * a.top_k / 8 + a.experts + 1) * 4;
+}
+
 // Where the integer matrix-core kernels serve: rows of up to 4096 values, one 256-value task per wave, and
 // at most eight pairs per expert on average -- they multiply four tokens at a time and are
 // the faster ones while most experts hold no more than four or eight pairs; the grouped matrix product
@@ -641,7 +640,7 @@ bool g8_usable(const lev_ctx *ctx, const lev_moe_grouped_args &a) {
     const size_t limit = ctx->props.sharedMemPerBlockOptin > ctx->props.sharedMemPerBlock
                              ? ctx->props.sharedMemPerBlockOptin
                              : ctx->props.sharedMemPerBlock;
-    const size_t lds_group = (size_t)5 * a.experts * 4;
+    const size_t lds_group = group_lds(a);
     const bool fits = g8_lds<2, kG8WavesWide>() <= limit && g8_lds<2, kG8WavesMax>() <= limit && g8_lds<kG8TilesDown, kG8WavesMax>() <= limit &&
                       lds_group <= limit;
     // (us a layer, these kernels against the grouped product: 2048 / 768, top-8 of 128: 64 tokens 101, 145; 128 tokens
@@ -759,7 +758,7 @@ hipError_t lev_moe_grouped_launch(lev_ctx *ctx, const lev_moe_grouped_args &a, c
         return c;
     }();
     const uint32_t w1 = cut[0], w2 = cut[1], s0_gu = cut[2], w1_dn = cut[3], w2_dn = cut[4], s0_dn = cut[5];
-    const size_t lds_group = (size_t)5 * a.experts * 4;
+    const size_t lds_group = group_lds(a);
     if ((e = lev_allow_lds(ctx, reinterpret_cast<const void *>(&moe_group_kernel), lds_group)) != hipSuccess) return e;
     hipLaunchKernelGGL(moe_group_kernel, dim3(1), dim3(1024), lds_group, ctx->stream, ids, pairs,
                        a.experts, a.top_k, valid, ctx->d_flag, items, starts, grid, q_gu.rpi, q_dn.rpi, w1, w2, w1_dn, w2_dn,

@@ -120,7 +120,7 @@ moe_pf_group_kernel(const int32_t *__restrict__ ids, uint32_t pairs, uint32_t ex
                     lev_pf_item *__restrict__ items, uint32_t *__restrict__ nitems, int *__restrict__ flag, const float *__restrict__ x,
                     uint32_t tokens, uint32_t hidden, _Float16 *__restrict__ xh, _Float16 *__restrict__ xl,
                     uint32_t *__restrict__ xmax, uint32_t cols) {
-    extern __shared__ int32_t s_cnt[];           // [experts] counts | cursors
+    extern __shared__ int32_t s_cnt[];           // [experts] counts | cursors | a count of dropped pairs, never read
     const uint32_t tid = threadIdx.x;
     if (blockIdx.x != 0u) {
         const uint32_t t = (blockIdx.x - 1u) * 16u + (tid >> 6);
@@ -131,11 +131,10 @@ moe_pf_group_kernel(const int32_t *__restrict__ ids, uint32_t pairs, uint32_t ex
     int32_t *s_cur = s_cnt + experts;
     __shared__ uint64_t s_wave[16];
     for (uint32_t e = tid; e < experts; e += 1024u) s_cnt[e] = 0;
-    __syncthreads();
+    lev_barrier_lds();
     bool bad_seen = false;
     // A thread takes a token, eight of its ids a wait.  The count's atomic gives the pair's place among its expert's: kept in
-    // registers for a thread's first eight pairs, in `ranks` (-1: dropped) for others.  With the ids and `valid` read back and a
-    // second round of atomics 1000 tokens, top-8 of 128, took 18.5 us here, now 14.4.
+    // registers for a thread's first eight pairs, in `ranks` (-1: dropped) for others.
     const uint32_t tokens_all = pairs / top_k;
     int32_t first_id[8], first_rank[8];
 #pragma unroll
@@ -149,25 +148,43 @@ moe_pf_group_kernel(const int32_t *__restrict__ ids, uint32_t pairs, uint32_t ex
             for (uint32_t u = 0; u < 8u; ++u) own[u] = row[k0 + u < top_k ? k0 + u : k0];
 #pragma unroll
             for (uint32_t u = 0; u < 8u; ++u) ok[u] = own[u] >= 0 && (uint32_t)own[u] < experts;
+#pragma unroll
+            for (uint32_t u = 0; u < 8u; ++u)
+#pragma unroll
+                for (uint32_t v = 0; v < u; ++v)
+                    if (k0 + u < top_k && own[u] == own[v]) ok[u] = ok[v] = false;
             for (uint32_t j0 = 0; j0 < top_k; j0 += 8u) {
+                if (j0 == k0) continue;
                 int32_t other[8];
 #pragma unroll
-                for (uint32_t v = 0; v < 8u; ++v) other[v] = j0 == k0 ? own[v] : row[j0 + v < top_k ? j0 + v : j0];
+                for (uint32_t v = 0; v < 8u; ++v) other[v] = row[j0 + v < top_k ? j0 + v : j0];
 #pragma unroll
                 for (uint32_t u = 0; u < 8u; ++u)
 #pragma unroll
                     for (uint32_t v = 0; v < 8u; ++v)
-                        if (j0 + v < top_k && j0 + v != k0 + u && other[v] == own[u]) ok[u] = false;
+                        if (j0 + v < top_k && other[v] == own[u]) ok[u] = false;
             }
 #pragma unroll
             for (uint32_t u = 0; u < 8u; ++u) {
-                if (k0 + u >= top_k) continue;
-                valid[(uint64_t)t * top_k + k0 + u] = ok[u] ? 1 : 0;
-                bad_seen = bad_seen || !ok[u];
+                ok[u] = ok[u] && k0 + u < top_k;
+                bad_seen = bad_seen || (!ok[u] && k0 + u < top_k);
             }
+            // (without a branch around each, eight atomics are in flight together: a dropped pair counts in a word of its own)
             int32_t rank[8];
 #pragma unroll
-            for (uint32_t u = 0; u < 8u; ++u) rank[u] = k0 + u < top_k && ok[u] ? atomicAdd(&s_cnt[own[u]], 1) : -1;
+            for (uint32_t u = 0; u < 8u; ++u) rank[u] = atomicAdd(&s_cnt[ok[u] ? (uint32_t)own[u] : 2u * experts], 1);
+            if (top_k == 8u) {
+                uint64_t eight = 0;
+#pragma unroll
+                for (uint32_t u = 0; u < 8u; ++u) eight |= (uint64_t)(ok[u] ? 1 : 0) << (8u * u);
+                reinterpret_cast<uint64_t *>(valid)[t] = eight;
+            } else {
+#pragma unroll
+                for (uint32_t u = 0; u < 8u; ++u)
+                    if (k0 + u < top_k) valid[(uint64_t)t * top_k + k0 + u] = ok[u] ? 1 : 0;
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < 8u; ++u) rank[u] = ok[u] ? rank[u] : -1;
             if (t == tid && k0 == 0u) {
 #pragma unroll
                 for (uint32_t u = 0; u < 8u; ++u) first_id[u] = own[u], first_rank[u] = rank[u];
@@ -179,39 +196,30 @@ moe_pf_group_kernel(const int32_t *__restrict__ ids, uint32_t pairs, uint32_t ex
         }
     }
     if (bad_seen) atomicOr(flag, kFlagBadExpertId);
-    __syncthreads();
-    // exclusive scan over the experts (at most 4096: four a thread) of three counts in 21-bit fields:
+    lev_barrier_lds();
+    // exclusive scan over the experts (at most 4096: up to four a thread, side by side) of three counts in 21-bit fields:
     // pairs, items of more than 32 pairs, other items
-    uint64_t local = 0;
+    const uint32_t per_thread = (experts + 1023u) >> 10;
+    uint64_t local = 0, before, all;
     int32_t c4[4];
 #pragma unroll
     for (uint32_t k = 0; k < 4u; ++k) {
-        const uint32_t e = 4u * tid + k;
+        if (k >= per_thread) break;
+        const uint32_t e = per_thread * tid + k;
         c4[k] = e < experts ? s_cnt[e] : 0;
         const uint32_t full = (uint32_t)c4[k] / cols, rem = (uint32_t)c4[k] % cols;
-        local += (uint64_t)c4[k] | (uint64_t)((cols > 32u ? full : 0u) + (rem > 32u)) << 21 | (uint64_t)((cols > 32u ? 0u : full) + (rem > 0u && rem <= 32u)) << 42;
+        local += (uint64_t)c4[k] | (uint64_t)((cols > 32u ? full : 0u) + (rem > 32u)) << 21 |
+                 (uint64_t)((cols > 32u ? 0u : full) + (rem > 0u && rem <= 32u)) << 42;
     }
-    uint64_t incl = local;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const uint64_t o = __shfl_up(incl, off);
-        if ((int)(tid & 63u) >= off) incl += o;
-    }
-    if ((tid & 63u) == 63u) s_wave[tid >> 6] = incl;
-    __syncthreads();
-    uint64_t before = incl - local, all = 0;
-#pragma unroll
-    for (uint32_t w = 0; w < 16u; ++w) {
-        before += w < (tid >> 6) ? s_wave[w] : 0u;
-        all += s_wave[w];
-    }
+    lev_scan_1024(local, s_wave, before, all);
     const uint32_t nbig = (uint32_t)(all >> 21) & 0x1FFFFFu;
     if (tid == 0) *nitems = nbig + (uint32_t)(all >> 42);
     int32_t run = (int32_t)(before & 0x1FFFFFu);
     uint32_t big = (uint32_t)(before >> 21) & 0x1FFFFFu, small = nbig + (uint32_t)(before >> 42);
 #pragma unroll
     for (uint32_t k = 0; k < 4u; ++k) {
-        const uint32_t e = 4u * tid + k;
+        if (k >= per_thread) break;
+        const uint32_t e = per_thread * tid + k;
         if (e < experts) s_cur[e] = run;
         for (int32_t j = 0; j < c4[k]; j += (int32_t)cols) {
             const int32_t left = c4[k] - j, count = left < (int32_t)cols ? left : (int32_t)cols;
@@ -219,7 +227,7 @@ moe_pf_group_kernel(const int32_t *__restrict__ ids, uint32_t pairs, uint32_t ex
         }
         run += c4[k];
     }
-    __syncthreads();
+    lev_barrier_lds();
     // The order of an expert's pairs depends on the atomics; no result does: every pair is computed
     // by itself and owns its outputs.
 #pragma unroll
@@ -669,7 +677,7 @@ hipError_t lev_moe_prefill_launch(lev_ctx *ctx, const lev_moe_grouped_args &a, c
     const uint32_t pairs = a.tokens * a.top_k;
     const pf_plan plan = pf_plan_of(pf_shape{(uint32_t)ctx->num_cus, a.hidden, a.inter, a.experts, a.top_k, a.tokens});
     hipError_t e;
-    hipLaunchKernelGGL(moe_pf_group_kernel, dim3(1u + (a.tokens + 15u) / 16u), dim3(1024), (size_t)2 * a.experts * 4,
+    hipLaunchKernelGGL(moe_pf_group_kernel, dim3(1u + (a.tokens + 15u) / 16u), dim3(1024), (size_t)2 * a.experts * 4 + 4,
                        ctx->stream, ids, pairs, a.experts, a.top_k, glist, valid, reinterpret_cast<int32_t *>(dn), items, nitems, ctx->d_flag, x,
                        a.tokens, a.hidden, xh, xl, xmax, plan.cols);   // (the ranks are in the place of dn, which comes much later)
     if ((e = hipGetLastError()) != hipSuccess) return e;

@@ -232,3 +232,35 @@ def test_moe_grouped_product_forms(ctx, hidden, inter, experts, tokens, forms):
         assert O.max_rel_err(act[t], ref["act"]) < TOL, t
         y32, _ = O.moe_experts_f32(g, u, d, hidden, inter, ids[t], wts[t], x[t])
         assert O.max_rel_err(y[t], ref["y"]) < max(TOL, 1.5 * O.max_rel_err(y32, ref["y"])), t
+
+
+@pytest.mark.parametrize("top_k,tokens,experts", [(8, 70, 24), (12, 40, 24), (3, 1100, 40), (8, 1030, 1100), (8, 1200, 1100)])
+def test_moe_prompt_grouping_drops_bad_pairs(ctx, top_k, tokens, experts):
+    """Pairs whose id is out of range or repeats another slot of their token are dropped and reported, in the first eight
+    slots of a token and behind them, for the first 1024 tokens and for others, with one expert a thread of the grouping
+    and with more (1030 tokens of 1100 experts: the integer kernels); every other pair counts."""
+    from leviathan_amd import capi, ops
+    from leviathan_amd.ops import LevError
+    hidden, inter = 256, 256
+    wr, pool, offs, x = H.config5(hidden, inter, experts, tokens, seed=top_k)
+    rng = np.random.default_rng(top_k + tokens)
+    ids = np.stack([rng.permutation(min(experts, 60))[:top_k] for _ in range(tokens)]).astype(np.int32)
+    wts = rng.random((tokens, top_k)).astype(np.float32)
+    bad = {1: (0, experts), 5: (top_k - 1, -1), tokens - 1: (top_k - 1, ids[tokens - 1, 0]), tokens - 2: (1, ids[tokens - 2, 2])}
+    for t, (slot, value) in bad.items():
+        ids[t, slot] = value
+    pool_d = torch.from_numpy(pool).cuda()
+    pools = ops.Context.moe_pools(pool_d, hidden, inter, experts, offs["gate_off"], offs["up_off"], offs["down_off"])
+    x_d, ids_d, wts_d = (torch.from_numpy(a).cuda() for a in (x, ids, wts))
+    y = ctx.moe_experts_q4_0(pools, x_d, ids_d, wts_d, top_k, tokens)
+    with pytest.raises(LevError) as e:
+        ctx.sync()
+    assert e.value.status == capi.BAD_DIMENSIONS
+    y = y.cpu().numpy()
+    g, u, d = (pool[offs["gate_off"]:], pool[offs["up_off"]:], pool[offs["down_off"]:])
+    for t in sorted(set(bad) | set(range(0, tokens, max(1, tokens // 12)))):
+        keep = [k for k in range(top_k) if 0 <= ids[t, k] < experts and np.count_nonzero(ids[t] == ids[t, k]) == 1]
+        assert (len(keep) == top_k) == (t not in bad)
+        ref = O.moe_experts_f64(g, u, d, hidden, inter, ids[t, keep], wts[t, keep], x[t])
+        y32, _ = O.moe_experts_f32(g, u, d, hidden, inter, ids[t, keep], wts[t, keep], x[t])
+        assert O.max_rel_err(y[t], ref["y"]) < max(TOL, 1.5 * O.max_rel_err(y32, ref["y"])), t
