@@ -291,22 +291,33 @@ __device__ router_sel router_select_regs(const float (&sc)[J], void *lds, uint32
 // The same selection run by ONE wave with no exchange at all, for kernels in which a single
 // wave ranks the scores while the others of the workgroup do something else: the wave holds all
 // scores (lane l keeps experts j*64 + l) and extracts minima of the integer keys round by round
-// (see router_select_regs).  all == false: returns the expert of `slot` after slot + 1 rounds.
-// all == true: lists the top_k winners and their probabilities in sel_id / sel_p (LDS, the layout
-// of router_select_regs) and returns the expert of `slot`.
-// Returns kRouteNotFinite when a score is not finite, kRouteNeedsBlock when the integer keys do
+// (see router_select_regs).  kRouteNotFinite when a score is not finite, kRouteNeedsBlock when the integer keys do
 // not order the probabilities (exp saturating or running into denormals): the caller then runs
 // the workgroup-wide selection.
+// What bounds it: one wave alone issues an instruction per 5.5 to 7 clocks, so its count of them.  A
+// round is 36 (the DPP steps with the neutral value in the lanes that get none, which makes an
+// instruction of a move and a minimum; the winner taken out by a mask made of scalar registers); 60
+// with moves, a compare of the lane and branches around stores of the list.
 constexpr uint32_t kRouteNotFinite = 0xFFFFFFFFu, kRouteNeedsBlock = 0xFFFFFFFEu;
 
+// Maximum and minimum over a wave, for the lane 63 of it; T: int32_t or uint32_t.
+template <int CTRL, int ROWS, class T, class F>
+__device__ __forceinline__ T route_dpp(T v, T neutral, F pick) {
+    return pick(v, (T)__builtin_amdgcn_update_dpp((int)neutral, (int)v, CTRL, ROWS, 0xF, false));
+}
+template <class T, class F>
+__device__ __forceinline__ T route_wave(T v, T neutral, F pick) {
+    v = route_dpp<0xB1, 0xF>(v, neutral, pick);    // quad_perm [1,0,3,2]
+    v = route_dpp<0x4E, 0xF>(v, neutral, pick);    // quad_perm [2,3,0,1]
+    v = route_dpp<0x141, 0xF>(v, neutral, pick);   // row_half_mirror
+    v = route_dpp<0x140, 0xF>(v, neutral, pick);   // row_mirror
+    v = route_dpp<0x142, 0xA>(v, neutral, pick);   // row_bcast:15 into rows 1 and 3
+    v = route_dpp<0x143, 0xC>(v, neutral, pick);   // row_bcast:31 into rows 2 and 3: lane 63 holds the result
+    return (T)__builtin_amdgcn_readlane((int)v, 63);
+}
+
 template <int J>
-__device__ uint32_t router_select_wave(const float (&sc)[J], void *lds, uint32_t experts, uint32_t top_k,
-                                       uint32_t slot, bool all) {
-    constexpr uint32_t padded = 64u * J;
-    uint64_t *table = static_cast<uint64_t *>(lds);
-    double *sel_p = reinterpret_cast<double *>(table + padded);
-    uint32_t *rank = reinterpret_cast<uint32_t *>(sel_p + 64);
-    uint32_t *sel_id = rank + padded;
+__device__ __forceinline__ uint32_t router_wave_keys(const float (&sc)[J], uint32_t experts, float (&d)[J], uint32_t (&dk)[J]) {
     const uint32_t lane = threadIdx.x & 63u;
     float mx = -INFINITY;
     bool finite = true;
@@ -315,75 +326,98 @@ __device__ uint32_t router_select_wave(const float (&sc)[J], void *lds, uint32_t
         finite = finite && isfinite(sc[j]);
         mx = fmaxf(mx, sc[j]);
     }
-    mx = wave_max_f32(mx);
     if (__any(!finite)) return kRouteNotFinite;
-    uint32_t dk[J];
+    // floats as integers of the same order (either zero serves as the largest: the differences are the same)
+    auto ordered = [](int32_t b) { return b ^ (int32_t)((uint32_t)(b >> 31) >> 1); };
+    mx = __int_as_float(ordered(route_wave<int32_t>(ordered(__float_as_int(mx)), INT32_MIN, [](int32_t a, int32_t b) { return a > b ? a : b; })));
     bool plain = true;
 #pragma unroll
     for (int j = 0; j < J; ++j) {
         const bool valid = lane + 64u * j < experts;
-        const float d = sc[j] - mx;
-        plain = plain && (!valid || d == 0.f || (d <= -1e-6f && d >= -690.f));
-        dk[j] = valid ? __float_as_uint(d) & 0x7FFFFFFFu : 0xFFFFFFFFu;
+        d[j] = sc[j] - mx;                                        // subtraction in f32, as the reference
+        plain = plain && (!valid || d[j] == 0.f || (d[j] <= -1e-6f && d[j] >= -690.f));
+        dk[j] = valid ? __float_as_uint(d[j]) & 0x7FFFFFFFu : 0xFFFFFFFFu;
     }
-    if (__any(!plain)) return kRouteNeedsBlock;
+    return __any(!plain) ? kRouteNeedsBlock : 0u;
+}
+
+// Takes the best of the keys out: its expert.
+template <int J>
+__device__ __forceinline__ uint32_t router_wave_round(uint32_t (&dk)[J]) {
+    uint32_t m = dk[0];
+#pragma unroll
+    for (int j = 1; j < J; ++j) m = dk[j] < m ? dk[j] : m;
+    const uint32_t best = route_wave<uint32_t>(m, 0xFFFFFFFFu, [](uint32_t a, uint32_t b) { return a < b ? a : b; });
+    // ascending j, lowest lane: the lowest index among equals
+    unsigned long long hit = __ballot(dk[0] == best);
+    uint32_t wj = 0;
+#pragma unroll
+    for (int j = 1; j < J; ++j) {
+        const unsigned long long h = __ballot(dk[j] == best);
+        wj = hit ? wj : 64u * j;
+        hit = hit ? hit : h;
+    }
+    const uint32_t wl = (uint32_t)__builtin_ctzll(hit);
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+        const unsigned long long out = wj == 64u * j ? 1ull << wl : 0ull;
+        asm("v_cndmask_b32 %0, %0, -1, %1" : "+v"(dk[j]) : "s"(out));
+    }
+    return wl + wj;
+}
+
+// The expert of `slot`, or one of the two words above.
+template <int J>
+__device__ __forceinline__ uint32_t router_select_wave(const float (&sc)[J], uint32_t experts, uint32_t slot) {
+    float d[J];
+    uint32_t dk[J];
+    uint32_t found = router_wave_keys<J>(sc, experts, d, dk);
+    if (found != 0u) return found;
+    do found = router_wave_round<J>(dk);
+    while (slot-- != 0u);
+    return found;
+}
+
+// All of a token's, a lane a slot, with the renormalised weights (router_weight), in two halves.
+template <int J>
+struct router_wave_list {
+    uint32_t dk[J];
     double p[J];
-    if (all) {
+    __device__ __forceinline__ void probabilities(const float (&sc)[J], uint32_t experts) {
+        const uint32_t lane = threadIdx.x & 63u;
+        float d[J];
+        if (router_wave_keys<J>(sc, experts, d, dk) != 0u) return;   // (wave 0 has found the same)
         double sum = 0.0;
 #pragma unroll
         for (int j = 0; j < J; ++j) {
-            const bool valid = lane + 64u * j < experts;
-            p[j] = valid ? exp((double)(sc[j] - mx)) : 0.0;   // subtraction in f32, exp in f64
+            p[j] = lane + 64u * j < experts ? exp((double)d[j]) : 0.0;
             sum += p[j];
         }
         sum = wave_sum_f64(sum);
 #pragma unroll
         for (int j = 0; j < J; ++j) p[j] = lane + 64u * j < experts ? p[j] / sum : 0.0;
     }
-    const uint32_t rounds = all ? top_k : slot + 1u;
-    uint32_t mine = 0xFFFFFFFFu;
-    for (uint32_t rnd = 0; rnd < rounds; ++rnd) {
-        uint32_t m = dk[0];
+    // the lane's slot: its expert and, of a finite sum, its weight without the expert's scale
+    __device__ __forceinline__ void select(uint32_t top_k, int32_t &id, float &weight) {
+        const uint32_t lane = threadIdx.x & 63u;
+        double prob_sum = 0.0, mine = 0.0;
+        for (uint32_t rnd = 0; rnd < top_k; ++rnd) {
+            const uint32_t e = router_wave_round<J>(dk), wl = e & 63u;
+            double pw = 0.0;
 #pragma unroll
-        for (int j = 1; j < J; ++j) m = dk[j] < m ? dk[j] : m;
-#define LEV_MOE_MINSTEP(CTRL, ROWS)                                                                \
-        {                                                                                          \
-            const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp((int)m, (int)m, CTRL, ROWS, 0xF, false); \
-            m = o < m ? o : m;                                                                     \
-        }
-        LEV_MOE_MINSTEP(0xB1, 0xF)
-        LEV_MOE_MINSTEP(0x4E, 0xF)
-        LEV_MOE_MINSTEP(0x141, 0xF)
-        LEV_MOE_MINSTEP(0x140, 0xF)
-        LEV_MOE_MINSTEP(0x142, 0xA)
-        LEV_MOE_MINSTEP(0x143, 0xC)
-#undef LEV_MOE_MINSTEP
-        const uint32_t best = (uint32_t)__builtin_amdgcn_readlane((int)m, 63);
-        uint32_t wl = 0, wj = 0;
-        bool seen = false;
-#pragma unroll
-        for (int j = 0; j < J; ++j) {   // ascending j, lowest lane: the lowest index among equals
-            const unsigned long long hit = __ballot(dk[j] == best);
-            if (!seen && hit != 0ull) {
-                wl = (uint32_t)__builtin_ctzll(hit);
-                wj = (uint32_t)j;
-                seen = true;
+            for (int j = 0; j < J; ++j) {
+                const double c = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(p[j]), wl), __builtin_amdgcn_readlane(__double2loint(p[j]), wl));
+                pw = e >> 6 == (uint32_t)j ? c : pw;
+            }
+            prob_sum += pw;                                       // over the slots in order
+            if (lane == rnd) {
+                id = (int32_t)e;
+                mine = pw;
             }
         }
-        const uint32_t found = wl + 64u * wj;
-        if (rnd == slot) mine = found;
-#pragma unroll
-        for (int j = 0; j < J; ++j) {
-            const bool here = lane == wl && wj == (uint32_t)j;
-            if (all && here) {
-                sel_id[rnd] = found;
-                sel_p[rnd] = p[j];
-            }
-            dk[j] = here ? 0xFFFFFFFFu : dk[j];
-        }
+        weight = (float)(mine / prob_sum);
     }
-    return mine;
-}
+};
 
 // Renormalised weight of selection slot k (Gemma4.swift:3808-3810): the sum
 // runs over the slots in order, in f64.
@@ -971,8 +1005,16 @@ __host__ __device__ constexpr size_t mm_areas_bytes(uint32_t waves, uint32_t tpw
 // ROUTE > 0 (experts <= 64*ROUTE): the expert comes from this token's router scores, ranked by
 // wave 0 alone while the other waves' activation requests are on their way (every workgroup of a
 // token repeats the selection, which costs less than a kernel boundary; one wave ranking costs an
-// eighth of the vector instructions of eight); the first workgroup of a token publishes ids and
-// weights.  Otherwise the ids are read from `ids`.
+// eighth of the vector instructions of eight); the last wave of the first workgroup of a token lists
+// ids and weights: probabilities before the expert is known, rounds while the weights of its task are on
+// their way.  Otherwise the ids are read from `ids`.
+// Time stamps at 2048 / 768, top-8 of 128, us after the first wave's start, for slots 0 and 7: scores 0.5 and 0.6,
+// expert 0.9 and 1.9, weights 1.8 and 3.2, end 3.8 and 4.6.  From the expert on it is the stream of the weights (7 TB/s);
+// with loads of contiguous 16 bytes they arrive no sooner.  So what is in front of the expert counts: rounds of 36
+// instructions (60: 0.1 for 0.15 a round) ahead of the other waves' staging, and nothing of the list, which wave 0 made
+// there before (2 us; its workgroup was the last of all).  One layer of 2816 / 704 13.15 -> 12.5 us, eight of 2048 / 768
+// 101.9 -> 99.9, four decoded layers 80.2 -> 79.2.  The other waves' staging in front of the barrier as well: 12.2, 100.5,
+// 79.6, but 16.3 -> 18.9 at 4096 / 448, top-4 of 256, three tokens.
 // LDS: part [2] | expert word | task areas | router area (ROUTE > 0)
 template <int NW, bool SINGLE, int ROUTE>
 __device__ __forceinline__ void gate_up_mfma(const moe_args &a, const float *__restrict__ x, const int32_t *ids,
@@ -990,8 +1032,9 @@ __device__ __forceinline__ void gate_up_mfma(const moe_args &a, const float *__r
     // request order = return order: the scores (the expert, and with it every weight address,
     // hangs on them) first, the activations behind them
     float sc[ROUTE > 0 ? ROUTE : 1];
+    const bool publisher = ROUTE > 0 && chunk == 0u && slot == 0u && wave == NW - 1u;
     if constexpr (ROUTE > 0) {
-        if (wave == 0u) router_load_scores<ROUTE>(scores + (uint64_t)t * a.experts, a.experts, sc);
+        if (wave == 0u || publisher) router_load_scores<ROUTE>(scores + (uint64_t)t * a.experts, a.experts, sc);
     }
     bool v_live;
     lev_f32x4 v = q4m_load_activations(xt, T, a.hidden >> 2, v_live);
@@ -1000,22 +1043,27 @@ __device__ __forceinline__ void gate_up_mfma(const moe_args &a, const float *__r
     uint8_t *area = smem + 2u * kPart + 16u + (size_t)wave * (kQ4mTaskArea + kQ4mZeroBytes);
     uint8_t *zero = area + kQ4mTaskArea;
     void *rl = smem + 2u * kPart + 16u + mm_areas_bytes(NW, 1u);
+    router_wave_list<(ROUTE > 0 ? ROUTE : 1)> list;
     uint32_t e;
-    bool ok = true;
-    const bool publisher = ROUTE > 0 && chunk == 0u && slot == 0u;
+    bool ok = true, listed = false;
     if constexpr (ROUTE > 0) {
         // (all eight waves ranking a share of the keys each was measured as well: the layer takes 0.5 us
         // longer, the 16 waves of a CU then queue for its four vector pipelines)
         if (wave == 0u) {
-            const uint32_t got = router_select_wave<ROUTE>(sc, rl, a.experts, a.top_k, slot, publisher);
+            __builtin_amdgcn_s_setprio(3);   // the others' staging can wait, the expert is waited for
+            const uint32_t got = router_select_wave<ROUTE>(sc, a.experts, slot);
             if (lane == 0u) s_e[0] = got;
+            __builtin_amdgcn_s_setprio(0);
+        } else if (publisher) {
+            list.probabilities(sc, a.experts);
         }
         lev_barrier_lds();
         e = s_e[0];
         if (e == kRouteNeedsBlock) {   // workgroup-uniform and rare: the workgroup ranks the probabilities together
             const router_sel r = router_select_block<ROUTE>(scores + (uint64_t)t * a.experts, rl, a.experts,
-                                                            a.top_k, publisher);
+                                                            a.top_k, chunk == 0u && slot == 0u);
             e = r.ok ? r.sel_id[slot] : kRouteNotFinite;
+            listed = true;
         }
         ok = e != kRouteNotFinite;
         if (!ok) e = slot;
@@ -1045,20 +1093,36 @@ __device__ __forceinline__ void gate_up_mfma(const moe_args &a, const float *__r
     issue(i0, Ga, Ua);
 
     // ---- while the weights are on their way ----
+    int32_t my_id = 0;                                            // the publisher's lane k: slot k
+    float my_weight = 0.f, my_scale = 1.f;
     if constexpr (ROUTE > 0) {
         if (publisher) {
-            constexpr uint32_t padded = 64u * ROUTE;
-            uint64_t *table = static_cast<uint64_t *>(rl);
-            double *sel_p = reinterpret_cast<double *>(table + padded);
-            uint32_t *sel_id = reinterpret_cast<uint32_t *>(sel_p + 64) + padded;
-            const router_sel r{sel_p, sel_id, ok, 0xFFFFFFFFu};
-            if (!ok && tid == 0) atomicOr(flag, kFlagNonFiniteScore);
-            if (tid < a.top_k) {
-                ids_out[(uint64_t)t * a.top_k + tid] = ok ? (int32_t)sel_id[tid] : (int32_t)tid;
-                weights_out[(uint64_t)t * a.top_k + tid] = ok ? router_weight(r, expert_scale, a.top_k, tid) : 0.f;
+            __builtin_amdgcn_s_setprio(3);
+            if (!ok && lane == 0u) atomicOr(flag, kFlagNonFiniteScore);
+            my_id = (int32_t)lane;
+            if (listed && ok) {
+                constexpr uint32_t padded = 64u * ROUTE;
+                double *sel_p = reinterpret_cast<double *>(static_cast<uint64_t *>(rl) + padded);
+                uint32_t *sel_id = reinterpret_cast<uint32_t *>(sel_p + 64) + padded;
+                if (lane < a.top_k) {
+                    my_id = (int32_t)sel_id[lane];
+                    my_weight = router_weight(router_sel{sel_p, sel_id, ok, 0xFFFFFFFFu}, nullptr, a.top_k, lane);
+                }
+            } else if (ok) {
+                list.select(a.top_k, my_id, my_weight);
             }
+            if (ok && expert_scale && lane < a.top_k) my_scale = expert_scale[my_id];
+            __builtin_amdgcn_s_setprio(0);
         }
     }
+    auto publish = [&] {   // behind the products: the scale need not be there for them
+        if constexpr (ROUTE > 0) {
+            if (publisher && lane < a.top_k) {
+                ids_out[(uint64_t)t * a.top_k + lane] = my_id;
+                weights_out[(uint64_t)t * a.top_k + lane] = expert_scale ? my_weight * my_scale : my_weight;
+            }
+        }
+    };
     const uint32_t r16 = lane & 15u, q = lane >> 4;
     uint32_t pw = (wave * 16u + lane) * 4u;                       // byte offsets into `part`: gate, then up at + 512
     uint32_t pr = (q * 16u + r16) * 4u;                           // wave 0: lane (r, q) adds waves q, q + 4, ..
@@ -1103,6 +1167,7 @@ __device__ __forceinline__ void gate_up_mfma(const moe_args &a, const float *__r
     };
     if (SINGLE) {
         finish(i0, Ga, Ua);
+        publish();
         return;
     }
     // unconditional (clamped) prefetch: a branch around the loads would make the compiler wait
@@ -1120,6 +1185,7 @@ __device__ __forceinline__ void gate_up_mfma(const moe_args &a, const float *__r
         if (next >= i_end) break;
         i0 = next;
     }
+    publish();
 }
 
 template <int NW, bool SINGLE, int ROUTE>

@@ -52,3 +52,31 @@ def test_moe_layer_routed_by_the_gate_up_kernel(ctx, hidden, inter, experts, top
         ref = O.moe_experts_f64(g, u, d, hidden, inter, ids[t], wts[t], x[t])
         y32, _ = O.moe_experts_f32(g, u, d, hidden, inter, ids[t], wts[t], x[t])
         assert O.max_rel_err(y[t], ref["y"]) < max(TOL, 1.5 * O.max_rel_err(y32, ref["y"])), t
+
+
+@pytest.mark.parametrize("hidden,inter,experts,top_k,tokens", [
+    (64, 64, 64, 64, 1), (64, 64, 65, 65 - 1, 2),                   # every slot of a wave; fewer tasks than waves
+    (2048, 64, 128, 1, 1), (4096, 1024, 256, 8, 1), (2816, 2048, 129, 6, 3),   # 8, 16 and 12 waves, one row group and more
+])
+def test_moe_layer_lists_ids_and_weights_as_the_router(ctx, hidden, inter, experts, top_k, tokens):
+    """The list that the gate/up kernel makes is the stand-alone router's, bit for bit: equal scores (lower index first) and
+    an expert's scale."""
+    from leviathan_amd import ops
+    rng = np.random.default_rng(hidden + experts)
+    wr = np.zeros((experts, hidden), np.float32)
+    wr[:, 1] = rng.integers(-6, 7, experts) * 0.25                  # many ties, one-hot activations: the scores themselves
+    x = np.zeros((tokens, hidden), np.float32)
+    x[:, 1] = np.linspace(1.0, 0.5, tokens)
+    scale = dev(rng.random(experts).astype(np.float32) + 0.5)
+    pool = rng.integers(0, 256, experts * 3 * inter * hidden // 32 * 18, dtype=np.uint8)
+    pool.reshape(-1, 18)[:, 1] = 0x20                               # fp16 scales of ordinary size
+    step = experts * inter * hidden // 32 * 18
+    pools = ops.Context.moe_pools(dev(pool), hidden, inter, experts, 0, step, 2 * step)
+    for s in (None, scale):
+        _, ids, wts = ctx.moe_layer_q4_0(pools, dev(wr), dev(x), top_k, tokens, expert_scale=s)
+        rids, rwts = ctx.moe_route_topk(dev(wr), dev(x), hidden, experts, top_k, tokens, expert_scale=s)
+        ctx.sync()
+        assert np.array_equal(ids.cpu().numpy(), rids.cpu().numpy())
+        assert np.array_equal(wts.cpu().numpy(), rwts.cpu().numpy())
+    order = np.lexsort((np.arange(experts), -wr[:, 1]))[:top_k]
+    assert ids.cpu().numpy()[0].tolist() == order.tolist()
