@@ -293,10 +293,11 @@ __device__ __forceinline__ float lev_row_sum_f32(float v) {
     return __uint_as_float(s1[0]) + __uint_as_float(s1[1]);
 }
 
-// out[i] = what lane FIRST + i of the lane's row of 16 holds (DPP row_newbcast).
+// out[i] = what lane FIRST + i of the lane's row of 16 holds (DPP row_newbcast).  (Every lane has a source; bound_ctrl says so:
+// without it the register is cleared first.)
 template <int LANE>
 __device__ __forceinline__ float lev_row_bcast(uint32_t v) {
-    return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x150 + LANE, 0xF, 0xF, false));
+    return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x150 + LANE, 0xF, 0xF, true));
 }
 template <int N, int FIRST = 0, int I = 0>
 __device__ __forceinline__ void lev_row_spread(uint32_t v, float (&out)[N]) {
@@ -315,10 +316,11 @@ __device__ __forceinline__ void lev_row_spread(const lev_u32x4 v, lev_f32x4 (&ou
 
 // Largest of an unsigned value over the 8 lanes of a half row of the wave, or the 16 of a row, in every lane of it:
 // quad swaps, then the row mirrors (DPP: no LDS, no other unit).  Magnitudes of floats
-// compare as their bit patterns do; NaN and infinity sort above every number.
+// compare as their bit patterns do; NaN and infinity sort above every number.  A step is one instruction: the 0 for lanes
+// without a source (there are none) changes no maximum.
 template <int CTRL>
 __device__ __forceinline__ uint32_t lev_dpp_max_u32(uint32_t v) {
-    const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, 0xF, 0xF, false);
+    const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, true);
     return o > v ? o : v;
 }
 __device__ __forceinline__ uint32_t lev_row8_max_u32(uint32_t v) {

@@ -1246,6 +1246,10 @@ moe_gate_up_and_gemv(moe_args a, const float *__restrict__ x, const int32_t *ids
 // whole reduction (TPW tasks, inter <= 256*TPW) of the tile's rows against the slot's activations,
 // which it stages for itself; the per-slot results meet in LDS and are merged IN SLOT ORDER in
 // f32, as the reference's axpy chain does.
+// What bounds it is the issue of instructions, two waves a SIMD: time stamps at 2048 / 768, top-8, us after the first wave's
+// start, waves 0-3 and 4-7: ids 0.8 and 1.3, requests out 1.2 and 1.8, operands 1.9 and 2.7, products 2.7 and 3.4, end
+// 3.8; the weights are never waited for.  So the activations are requested before the ids are there, and a step of a
+// maximum over lanes is one instruction: eight layers 99.9 -> 99.0 us, four decoded ones 80.4 -> 79.2.
 // LDS: partial [top_k][16] f32 | w_slot [64] f32 | task areas
 template <int TPW>
 __global__ void __launch_bounds__(kMmThreads)
@@ -1283,13 +1287,11 @@ moe_down_mfma(moe_args a, const float *__restrict__ act, const int32_t *__restri
             const uint32_t T = (uint32_t)k < ntask ? (uint32_t)k : ntask - 1u;
             v[k] = q4m_load_activations(av, T, a.inter >> 2, v_live[k]);
         }
+        __builtin_amdgcn_sched_barrier(0);
         uint32_t e;
-        if (!expert_ids_verdict(ids_mine, a.top_k, slot, a.experts, &e)) {
-            bad = true;
-            if (lane < 16u) partial[slot * 16u + lane] = 0.f;
-            continue;
-        }
-        e = (uint32_t)__builtin_amdgcn_readfirstlane((int)e);
+        const bool good = expert_ids_verdict(ids_mine, a.top_k, slot, a.experts, &e);
+        bad = bad || !good;
+        e = good ? (uint32_t)__builtin_amdgcn_readfirstlane((int)e) : 0u;   // (no branch: it would hold the activations back)
         const uint8_t *rowp = a.base + a.down_off + e * a.down_stride + (uint64_t)lr * row_bytes;
         uint32_t D[TPW][9];
 #pragma unroll
@@ -1312,7 +1314,7 @@ moe_down_mfma(moe_args a, const float *__restrict__ act, const int32_t *__restri
             val = k ? val + dot : dot;
         }
         val = 0.5f * lev_row_sum_f32(val);
-        if (lane < 16u) partial[slot * 16u + lane] = val;
+        if (lane < 16u) partial[slot * 16u + lane] = good ? val : 0.f;
     }
     if (bad && lane == 0) atomicOr(flag, kFlagBadExpertId);
     if (wave == 0u && lane < a.top_k) w_slot[lane] = w_mine;

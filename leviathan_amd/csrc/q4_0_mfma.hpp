@@ -82,7 +82,7 @@ __device__ __forceinline__ q4m_unscale q4m_stage_planes(const lev_f32x4 v, uint8
     const float scale = __uint_as_float((283u - ex) << 23);    // 2^(156 - ex): |x * scale| < 2^30
     uint32_t Y[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) Y[k] = ((uint32_t)(int)rintf(v[k] * scale) + 0x00808080u) ^ 0x00808080u;
+    for (int k = 0; k < 4; ++k) Y[k] = (uint32_t)(int)rintf(v[k] * scale) + 0x00808080u;
     // 4x4 byte transpose: digit p of the lane's four values in one dword
     const uint32_t t0 = __builtin_amdgcn_perm(Y[1], Y[0], 0x05010400u);
     const uint32_t t1 = __builtin_amdgcn_perm(Y[1], Y[0], 0x07030602u);
@@ -93,6 +93,7 @@ __device__ __forceinline__ q4m_unscale q4m_stage_planes(const lev_f32x4 v, uint8
     dw[1] = __builtin_amdgcn_perm(t2, t0, 0x07060302u);
     dw[2] = __builtin_amdgcn_perm(t3, t1, 0x05040100u);
     dw[3] = __builtin_amdgcn_perm(t3, t1, 0x07060302u);
+    for (int p = 0; p < 3; ++p) dw[p] ^= 0x80808080u;
     // lane i: pair i / 16, half (i % 16) / 4, k-slots 4 * (i % 4) .. + 3
     uint8_t *at = area + g * 256u + (r >> 2) * 16u + (r & 3u) * 4u;
 #pragma unroll
