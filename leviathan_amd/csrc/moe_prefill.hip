@@ -559,6 +559,8 @@ __device__ __forceinline__ void pf_tile(const lev_moe_grouped_args &a, const lev
                 if (kLate) {
                     pend = acc;
                     pend_d = d;
+                    // the part before this step is whole only now, whatever T: the same bits wherever a pair lies in its item
+                    if (FOLD && st == 0u && u == 0u && step != 0u && (step & (kPfFold - 1u)) == 0u) fold();
                 } else {
 #pragma unroll
                     for (int i = 0; i < 16; ++i) y[t][i] = fmaf(d, acc[i], y[t][i]);
@@ -571,7 +573,7 @@ __device__ __forceinline__ void pf_tile(const lev_moe_grouped_args &a, const lev
     for (uint32_t step = 0; step + 1u < nsteps; step += 2u) {
         step_of(step, first);
         step_of(step + 1u, second);
-        if (FOLD && (step & (kPfFold - 2u)) == kPfFold - 2u) fold();
+        if (FOLD && !kLate && (step & (kPfFold - 2u)) == kPfFold - 2u) fold();
     }
     if (nsteps & 1u) step_of(nsteps - 1u, only);
 #pragma unroll

@@ -234,6 +234,22 @@ def test_moe_grouped_product_forms(ctx, hidden, inter, experts, tokens, forms):
         assert O.max_rel_err(y[t], ref["y"]) < max(TOL, 1.5 * O.max_rel_err(y32, ref["y"])), t
 
 
+@pytest.mark.parametrize("hidden,inter,experts,tokens", [f[:4] for f in FORMS])
+def test_moe_grouped_product_gives_a_pair_the_same_bits_anywhere(ctx, hidden, inter, experts, tokens):
+    """The order of an expert's pairs is that of atomics, so where a pair lies (its item, its column tile, the tiles of its
+    item) must not show in a bit: equal activations have equal outputs in all of an expert's lists of 1 to 65 pairs and more."""
+    edges = [1, 31, 32, 33, 63, 64, 65]
+    wr, pool, offs, x = H.config5(hidden, inter, experts, tokens, seed=hidden + inter)
+    rng = np.random.default_rng(tokens)
+    rest = rng.multinomial(tokens - sum(edges), [1 / (experts - len(edges))] * (experts - len(edges)))
+    ids = rng.permutation(np.repeat(np.arange(experts), edges + rest.tolist())).astype(np.int32)[:, None]
+    x[:] = x[0]
+    y, act = run_experts(ctx, pool, offs, hidden, inter, experts, x, ids, np.full((tokens, 1), 0.75, np.float32))
+    for e in range(experts):
+        mine = np.flatnonzero(ids[:, 0] == e)
+        assert (act[mine] == act[mine[0]]).all() and (y[mine] == y[mine[0]]).all(), e
+
+
 @pytest.mark.parametrize("top_k,tokens,experts", [(8, 70, 24), (12, 40, 24), (3, 1100, 40), (8, 1030, 1100), (8, 1200, 1100)])
 def test_moe_prompt_grouping_drops_bad_pairs(ctx, top_k, tokens, experts):
     """Pairs whose id is out of range or repeats another slot of their token are dropped and reported, in the first eight
