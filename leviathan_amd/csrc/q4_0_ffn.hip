@@ -3,9 +3,9 @@
 //
 // Called operator by operator it is six launches of which four are the launch floor and little else: at
 // 2816 / 2112 18.7 us recorded, 29 us enqueued one by one.  Here three: everything up to act, the down GEMV, the
-// norm behind it (9.1 us recorded; enqueued 9.2 to 9.9, the host's pace; recorded 0.15 more with the only group's weights
-// requested a second time).  The first kernel has the shape of the MoE gate/up kernel: a wave owns one
-// 256-value column task of gate row group i and of up row group i, keeps the operands in registers and
+// norm behind it (8.8 us recorded, 9.3 before the scale of the norms by DPP; enqueued 9.0 to 10.4, the host's pace; recorded
+// 0.15 more with the only group's weights requested a second time).  The first kernel has the shape of the MoE gate/up
+// kernel: a wave owns one 256-value column task of gate row group i and of up row group i, keeps the operands in registers and
 // meets the others in LDS; in front of it every workgroup normalises x for itself (a wave its own 256 values,
 // the sum of squares crosses the waves once), with its weights already on their way.
 #include "moe_scores_few.hpp"
