@@ -181,10 +181,8 @@ moe_pf_group_kernel(const int32_t *__restrict__ ids, uint32_t pairs, uint32_t ex
                 ok[u] = ok[u] && k0 + u < top_k;
                 bad_seen = bad_seen || (!ok[u] && k0 + u < top_k);
             }
-            // (without a branch around each, eight atomics are in flight together: a dropped pair counts in a word of its own)
             int32_t rank[8];
-#pragma unroll
-            for (uint32_t u = 0; u < 8u; ++u) rank[u] = atomicAdd(&s_cnt[ok[u] ? (uint32_t)own[u] : 2u * experts], 1);
+            pf_rank_pairs(own, ok, k0, top_k, experts, [&](uint32_t word) { return atomicAdd(&s_cnt[word], 1); }, rank);
             if (top_k == 8u) {
                 uint64_t eight = 0;
 #pragma unroll
@@ -195,8 +193,6 @@ moe_pf_group_kernel(const int32_t *__restrict__ ids, uint32_t pairs, uint32_t ex
                 for (uint32_t u = 0; u < 8u; ++u)
                     if (k0 + u < top_k) valid[(uint64_t)t * top_k + k0 + u] = ok[u] ? 1 : 0;
             }
-#pragma unroll
-            for (uint32_t u = 0; u < 8u; ++u) rank[u] = ok[u] ? rank[u] : -1;
             if (t == tid && k0 == 0u) {
 #pragma unroll
                 for (uint32_t u = 0; u < 8u; ++u) first_id[u] = own[u], first_rank[u] = rank[u];

@@ -83,3 +83,48 @@ def test_prompt_product_forms(tmp_path):
     for (cus, hidden, inter, *_), (cols, gate_up, down) in zip(cases, plans):
         assert cols == (32 if 4 in (gate_up, down) else 64)
         assert (gate_up == 0) == (hidden <= 1024) and (down == 0) == (inter <= 1024)
+
+
+RANK_PROGRAM = """
+#include "moe_prefill_plan.hpp"
+#include <cstdio>
+int main() {
+    unsigned experts, top_k, k0;
+    int own[8], good[8];
+    while (std::scanf("%u %u %u", &experts, &top_k, &k0) == 3) {
+        bool ok[8];
+        for (int u = 0; u < 8; ++u) {
+            if (std::scanf("%d %d", own + u, good + u) != 2) return 1;
+            ok[u] = good[u] != 0;
+        }
+        int rank[8], adds = 0;
+        pf_rank_pairs(own, ok, k0, top_k, experts, [&](uint32_t word) { std::printf("%u ", word); return 100 + adds++; }, rank);
+        std::printf("|");
+        for (int r : rank) std::printf(" %d", r);
+        std::printf("\\n");
+    }
+}
+"""
+
+
+def test_prompt_grouping_adds_once_a_pair(tmp_path):
+    """A slot past top_k adds to no word of the counts (lanes that add to one word take the LDS a turn each); a pair adds to its
+    expert's word, a dropped one to the word behind the lists, and gets no rank."""
+    cxx = os.environ.get("CXX") or shutil.which("g++")
+    if not cxx:
+        pytest.skip("no C++ compiler")
+    (tmp_path / "rank.cpp").write_text(RANK_PROGRAM)
+    subprocess.run([cxx, "-std=c++17", "-Wall", "-Werror", f"-I{CSRC}", str(tmp_path / "rank.cpp"),
+                    "-o", str(tmp_path / "rank")], check=True)
+    cases = [(60, top_k, k0, dropped) for top_k in range(1, 20) for k0 in range(0, top_k, 8) for dropped in ((), (0,), (1, 6))]
+    lines = []
+    for experts, top_k, k0, dropped in cases:
+        ok = [k0 + u < top_k and u not in dropped for u in range(8)]
+        lines.append(f"{experts} {top_k} {k0} " + " ".join(f"{7 * u if good else -5} {int(good)}" for u, good in enumerate(ok)))
+    out = subprocess.run([str(tmp_path / "rank")], input="\n".join(lines), check=True, capture_output=True, text=True).stdout.splitlines()
+    assert len(out) == len(cases)
+    for (experts, top_k, k0, dropped), line in zip(cases, out):
+        words, ranks = (list(map(int, part.split())) for part in line.split("|"))
+        pairs = min(8, top_k - k0)
+        assert words == [2 * experts if u in dropped else 7 * u for u in range(pairs)], (top_k, k0)
+        assert ranks == [100 + u if u < pairs and u not in dropped else -1 for u in range(8)], (top_k, k0)
