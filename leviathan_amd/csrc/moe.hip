@@ -1115,7 +1115,9 @@ __device__ __forceinline__ void gate_up_mfma(const moe_args &a, const float *__r
             __builtin_amdgcn_s_setprio(0);
         }
     }
-    auto publish = [&] {   // behind the products: the scale need not be there for them
+    // One row group: behind its products, the scale need not be there for them.  Several: in front of the first one's (the list's
+    // registers through all groups made the kernels of 12 waves, 80 registers each, spill ten).
+    auto publish = [&] {
         if constexpr (ROUTE > 0) {
             if (publisher && lane < a.top_k) {
                 ids_out[(uint64_t)t * a.top_k + lane] = my_id;
@@ -1132,6 +1134,7 @@ __device__ __forceinline__ void gate_up_mfma(const moe_args &a, const float *__r
     if (lane < kQ4mZeroBytes / 4u) reinterpret_cast<uint32_t *>(zero)[lane] = 0u;
     q4m_operand op;
     q4m_stage_task(q4m_mask_activations(v, v_live), area, zero, active, op);
+    if (!SINGLE) publish();
     __builtin_amdgcn_sched_barrier(0);
 
     auto finish = [&](uint32_t i_here, const uint32_t (&Dg)[9], const uint32_t (&Du)[9]) {
@@ -1185,7 +1188,6 @@ __device__ __forceinline__ void gate_up_mfma(const moe_args &a, const float *__r
         if (next >= i_end) break;
         i0 = next;
     }
-    publish();
 }
 
 template <int NW, bool SINGLE, int ROUTE>
