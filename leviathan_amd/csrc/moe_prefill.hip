@@ -32,7 +32,7 @@
 //
 // Measured (us, the two products, before -> now; 2816 / 704, top-8 of 128 experts): 1000 tokens 231 + 117 -> 208 + 108; 300 tokens
 // 114 + 62 -> 110 + 59; 2048 / 768, 1000 tokens 167 + 89 -> 156 + 82; 1024 / 256, top-4 of 32, 300 tokens 23 + 9.9 -> 18.6 + 8.7;
-// 4096 / 1536, top-6 of 64, 500 tokens 277 + 149 -> 232 + 139; 4096 / 832, top-4 of 128, 420 tokens 205 + 93 -> 186 + 89.
+// 4096 / 1536, top-6 of 64, 500 tokens 277 + 149 -> 224 + 133; 4096 / 832, top-4 of 128, 420 tokens 205 + 93 -> 186 + 89.
 // Tried and not kept: 64 rows a wave (half the fragment reads: no faster, the registers of two folded tiles spill), items of 96
 // (203 + 113), deeper requests, wave priorities.
 #include "moe_prefill.hpp"
@@ -298,13 +298,18 @@ constexpr __host__ __device__ uint32_t pf_min(uint32_t a, uint32_t b) { return a
 
 // A block's 16 codes of a lane, two dwords (code bytes 8g .. 8g + 7) -> the operands of both halves, fp16 integers n - 8.
 // 0x6400 | n is the fp16 number 1024 + n, 0x6400 | 16 n is 1024 + 16 n: a subtraction and a multiply-add, both exact.
+template <bool SCALAR>
 struct pf_consts {
     uint32_t low = 0x000F000Fu, high = 0x00F000F0u, magic = 0x64006400u;
     lev_f16x2 m1032 = {(_Float16)-1032.0f, (_Float16)-1032.0f}, sixteenth = {(_Float16)0.0625f, (_Float16)0.0625f}, m72 = {(_Float16)-72.0f, (_Float16)-72.0f};
-    // (in registers: (v & mask) | magic is one instruction)
-    __device__ __forceinline__ pf_consts() { asm("" : "+v"(low), "+v"(high), "+v"(magic)); }
+    // (in registers: (v & mask) | magic is one instruction, of which one operand may be a scalar register's)
+    __device__ __forceinline__ pf_consts() {
+        if constexpr (SCALAR) asm("" : "+s"(low), "+s"(high), "+v"(magic));
+        else asm("" : "+v"(low), "+v"(high), "+v"(magic));
+    }
 };
-__device__ __forceinline__ void pf_decode(uint32_t c, const pf_consts &k, uint32_t &low, uint32_t &high) {
+template <bool SCALAR>
+__device__ __forceinline__ void pf_decode(uint32_t c, const pf_consts<SCALAR> &k, uint32_t &low, uint32_t &high) {
     low = __builtin_bit_cast(uint32_t, (lev_f16x2)(__builtin_bit_cast(lev_f16x2, (c & k.low) | k.magic) + k.m1032));
     high = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(lev_f16x2, (c & k.high) | k.magic), k.sixteenth, k.m72));
 }
@@ -455,7 +460,10 @@ __device__ __forceinline__ void pf_tile(const lev_moe_grouped_args &a, const lev
                 y[t][i] = 0.f;
             }
     };
-    const pf_consts kc;
+    // Twelve waves have 168 registers each, which this and the lane's number made again at the end keep to: with five spilled, a
+    // folded sum among them, the down product of 4096 / 1536 (500 tokens, top-6 of 64) took 149 us for 133.  Other forms have the masks
+    // in vector registers (the down product of eight waves at 2304 / 1280 45.9 us, with scalar ones 46.7).
+    const pf_consts<FOLD && OCC == 3u> kc;
     const uint8_t *const wmine = lds + L::kW + wave * L::kWArea + lr * kPfWRow;
     const uint32_t areg = (lr >> 3) * 1024u, apar = (lr >> 3) & 1u, acol = lr & 7u;
     uint32_t aoff[4];   // this lane's fragment of half s of block b of a step: aoff[2b + s], + 4096 per column tile, + kPlane for the low plane
@@ -578,19 +586,20 @@ __device__ __forceinline__ void pf_tile(const lev_moe_grouped_args &a, const lev
     float(&sum)[T][16] = FOLD ? whole : y;
 
     LEV_WAIT_VMCNT(0);   // the requests past the end land before the LDS is given back
-    // lane (lr, g), register i of a tile: weight row lr, column 8 (i / 4) + 4 g + i % 4
-    const uint32_t row = row0 + (PAIRED ? lr & 15u : lr);
+    // lane (r, h), register i of a tile: weight row r, column 8 (i / 4) + 4 h + i % 4
+    const uint32_t me = FOLD && OCC == 3u ? __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)) : lane, r = me & 31u, h = me >> 5;
+    const uint32_t row = row0 + (PAIRED ? r & 15u : r);
 #pragma unroll
     for (uint32_t t = 0; t < T; ++t)
 #pragma unroll
         for (int i = 0; i < 16; i += PAIRED ? 2 : 1) {
-            uint32_t col = 32u * t + 8u * (i / 4) + 4u * g + (i % 4);
+            uint32_t col = 32u * t + 8u * (i / 4) + 4u * h + (i % 4);
             float v = sum[t][i];
             if (PAIRED) {
                 // lanes 0..15 of a half hold gate rows, 16..31 the same up rows: two columns trade halves, so
                 // that every lane has a gate and its up value, of column i in lanes 0..15, of i + 1 in 16..31
                 const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(sum[t][i + 1]), false, false);
-                col += lr >> 4;
+                col += r >> 4;
                 const float us = s_us[col];
                 v = lev_gelu_up_value(__uint_as_float(sw[0]) * us, __uint_as_float(sw[1]) * us);
             } else {

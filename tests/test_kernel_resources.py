@@ -39,7 +39,7 @@ def kernels():
     return found
 
 
-@pytest.mark.parametrize("pattern", ["moe_gate_up_mfma"])
+@pytest.mark.parametrize("pattern", ["moe_gate_up_mfma", "moe_pf_kernel"])
 def test_kernels_keep_their_registers(pattern):
     """The time of these kernels is what a wave issues and waits for: nothing of them goes through scratch memory."""
     mine = {name: k for name, k in kernels().items() if pattern in name}
