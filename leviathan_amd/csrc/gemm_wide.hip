@@ -108,7 +108,7 @@ gemm_wide_kernel(const uint8_t *__restrict__ w, const uint8_t *__restrict__ xf, 
             produce(1u);
             __builtin_amdgcn_sched_barrier(0);
             meet();
-            next(i + 2u);
+            if (i + 1u < nsb) next(i + 2u);
         }
         return;
     }
