@@ -53,11 +53,14 @@ def _headers_mtime() -> float:
 
 def _compile(src: str, force: bool, extra: list[str]) -> str:
     obj = os.path.join(OBJ_DIR, os.path.basename(src)[:-4] + ".o")
-    if (not force and os.path.exists(obj)
-            and os.path.getmtime(obj) >= max(os.path.getmtime(src), _headers_mtime())):
-        return obj
     preload = [] if os.path.basename(src) in NO_PRELOAD else PRELOAD_FLAGS
     cmd = [hipcc(), *HIPCC_FLAGS, *preload, *extra, "-c", src, "-o", obj]
+    made_by = obj + ".cmd"                   # an object made by another command is not up to date
+    if (not force and os.path.exists(obj) and os.path.exists(made_by) and open(made_by).read() == "\n".join(cmd)
+            and os.path.getmtime(obj) >= max(os.path.getmtime(src), _headers_mtime())):
+        return obj
+    if os.path.exists(made_by):
+        os.remove(made_by)
     res = subprocess.run(cmd, capture_output=True, text=True)
     noise = "is not a recognized feature for this target"
     err = "\n".join(l for l in res.stderr.splitlines() if noise not in l and l.strip())
@@ -65,6 +68,8 @@ def _compile(src: str, force: bool, extra: list[str]) -> str:
         raise RuntimeError(f"hipcc failed for {src}:\n{err}")
     if err:
         sys.stderr.write(err + "\n")
+    with open(made_by, "w") as f:
+        f.write("\n".join(cmd))
     return obj
 
 
