@@ -28,8 +28,11 @@ HIPCC_FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
 # The first 16 dwords of plain kernel arguments arrive in registers with the wave: a trip to memory less in front of the first
-# requests (Q4_K x 4 columns 8.87 -> 8.73 us, the int8 FFN of five columns 31.7 -> 30.7, 64 tokens through an MoE layer
-# 96.9 -> 95.6).  Not for the Q6_K head's long stream, which takes 105.3 us with it and 104.3 without.
+# requests.  us without and with it: the Q4_0 GEMV of 4096 x 4096 on cold weights 3.85 and 3.63; among other calls RMSNorm and Q4_K by
+# four columns (12288 x 4096) 9.1 and 8.8, the int8 FFN of five columns (4096 / 12288) 31.8 and 31.0, 64 tokens through an MoE layer
+# (2048 / 768) 95.5 and 94.0.  Recorded kernels of few us on weights that the caches hold lose up to 2 %: that GEMV 3.21 and 3.27,
+# Q4_K by two columns (4096 x 4096) 5.55 and 5.63, the int8 FFN of one column (1024 / 2048) 14.77 and 14.96.
+# Not for the Q6_K head's long stream, which takes 105.3 us with it and 104.3 without.
 PRELOAD_FLAGS = ["-mllvm", "-amdgpu-kernarg-preload-count=16"]
 NO_PRELOAD = {"q6_k_mfma_gemv.hip"}
 

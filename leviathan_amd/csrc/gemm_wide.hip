@@ -23,9 +23,13 @@
 // for 350 to 520 of a step's 1260 clocks.  And the compiler must not move a superblock's requests and factors in among
 // its fragments: with the order kept a step takes 980 clocks where it took 1260.
 // 512 tokens, 4096 columns, us under a sustained load: 12288 rows of Q4_K 57.2 before and 55.0, of Q6_K 61.2 and 58.4, 32000 rows of
-// Q6_K 139 and 131; 9456 x 9472 of Q4_K 100.6 and 96.2.  What bounds it is power: of the 22 % fewer clocks the first of these keeps 4,
-// since the clock under these products falls from 1.73 to 1.47 GHz (a loop of MFMAs alone on random operands runs at 1.45 and
-// takes 35 us for it; the library's fp16 product 51).  The Q6_K one, 1200 clocks at 1.64 GHz, waits for its decoding waves.
+// Q6_K 139 and 131; 9456 x 9472 of Q4_K 100.6 and 96.2.  Of the 22 % fewer clocks a step the first of these keeps 4: the
+// clock under these products falls with them, from 1.73 to 1.5 GHz (a loop of MFMAs alone on random operands runs at 1.45 and
+// takes 35 us for it; the library's fp16 product 51).
+// What bounds it (time stamps; 256 workgroups, one round of 45 to 50 us, 71 to 76 thousand clocks of Q4_K at 1.55 GHz): the 64 steps, 1000
+// clocks each for 770 of MFMAs, nine tenths of it; the first span is there after 4.0 to 4.8 thousand clocks (2.0 to 3.3 thousand until the first
+// weights, one to decode them), the stores take 2.3 to 6.5 thousand, and nothing covers either.  Q6_K: 83 thousand clocks, steps
+// of 1160, which wait for the decoding waves, the first span after 5.2 thousand.
 //
 // K order inside a 64-step is permuted consistently on both operands (unit_of of the formats' weights); the sums are formed
 // in the order in which a wave of gemm_split.hip that takes all of K forms them: the same bits.

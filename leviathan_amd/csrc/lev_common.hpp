@@ -210,9 +210,10 @@ __device__ __forceinline__ void lev_barrier_lds() {
     asm volatile("s_barrier" ::: "memory");
 }
 
-// 1/sqrt(a) of a positive f64 that is rounded to f32 next: the hardware estimate (relative error e below 2^-24) and one step of
-// third order, which leaves 5/16 e^3 and the rounding of f64: four dependent instructions, where the square root and
-// the division of the library take over a hundred, all of them on the critical path of a one-workgroup kernel.
+// 1/sqrt(a) of a positive f64 that is rounded to f32 next: the hardware estimate (v_rsq_f64, documented to 2^29 units in the
+// last place: relative error e of at most 2^-23) and one step of third order.  With h = 1 - a est^2, 2 e in size, the
+// series ends before 5/16 h^3 = 5/2 e^3, below 2^-67, and the rounding of f64 is what is left: four dependent instructions, where
+// the square root and the division of the library take over a hundred, all on the critical path of a one-workgroup kernel.
 __device__ __forceinline__ double lev_rsqrt_f64(double a) {
     const double est = __builtin_amdgcn_rsq(a);
     const double h = fma(-a * est, est, 1.0);

@@ -1012,9 +1012,9 @@ __host__ __device__ constexpr size_t mm_areas_bytes(uint32_t waves, uint32_t tpw
 // expert 0.9 and 1.9, weights 1.8 and 3.2, end 3.8 and 4.6.  From the expert on it is the stream of the weights (7 TB/s);
 // with loads of contiguous 16 bytes they arrive no sooner.  So what is in front of the expert counts: rounds of 36
 // instructions (60: 0.1 for 0.15 a round) ahead of the other waves' staging, and nothing of the list, which wave 0 made
-// there before (2 us; its workgroup was the last of all).  One layer of 2816 / 704 13.15 -> 12.5 us, eight of 2048 / 768
-// 101.9 -> 99.9, four decoded layers 80.2 -> 79.2.  The other waves' staging in front of the barrier as well: 12.2, 100.5,
-// 79.6, but 16.3 -> 18.9 at 4096 / 448, top-4 of 256, three tokens.
+// there before (2 us; its workgroup was the last of all).  One layer of 2816 / 704 13.15 -> 12.5 us; recorded, eight of 2048 / 768
+// 101.9 -> 99.9 (called one by one on cold weights 113.6 -> 110.9), four decoded layers 80.2 -> 79.2.  The other waves' staging
+// in front of the barrier as well: 12.2, 100.5, 79.6, but 16.3 -> 18.9 at 4096 / 448, top-4 of 256, three tokens.
 // LDS: part [2] | expert word | task areas | router area (ROUTE > 0)
 template <int NW, bool SINGLE, int ROUTE>
 __device__ __forceinline__ void gate_up_mfma(const moe_args &a, const float *__restrict__ x, const int32_t *ids,
@@ -1251,7 +1251,8 @@ moe_gate_up_and_gemv(moe_args a, const float *__restrict__ x, const int32_t *ids
 // What bounds it is the issue of instructions, two waves a SIMD: time stamps at 2048 / 768, top-8, us after the first wave's
 // start, waves 0-3 and 4-7: ids 0.8 and 1.3, requests out 1.2 and 1.8, operands 1.9 and 2.7, products 2.7 and 3.4, end
 // 3.8; the weights are never waited for.  So the activations are requested before the ids are there, and a step of a
-// maximum over lanes is one instruction: eight layers 99.9 -> 99.0 us, four decoded ones 80.4 -> 79.2.
+// maximum over lanes is one instruction: recorded, eight layers 99.9 -> 99.0 us (called one by one on cold weights 111.2 -> 110.4),
+// four decoded ones 80.4 -> 79.2.
 // LDS: partial [top_k][16] f32 | w_slot [64] f32 | task areas
 template <int TPW>
 __global__ void __launch_bounds__(kMmThreads)

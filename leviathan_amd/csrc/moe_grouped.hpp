@@ -40,7 +40,8 @@ hipError_t lev_moe_merge_launch(lev_ctx *ctx, const lev_moe_grouped_args &a, con
                                 const uint8_t *valid, float *y);
 
 // Exclusive scan over a workgroup of 1024 threads, of sums that do not meet beyond 64 bits (fields of counts): what the threads
-// in front of this one hold, and what all hold.  s_wave: 16 entries in LDS; two barriers.  The steps within a wave are DPP
+// in front of this one hold, and what all hold.  s_wave: 16 entries in LDS.  One barrier, between their stores and their reads: the
+// caller needs another one before it writes s_wave again.  The steps within a wave are DPP
 // moves: with lane permutations through the LDS they were most of what the grouping kernels' scan took.
 __device__ __forceinline__ void lev_scan_1024(uint64_t own, uint64_t *s_wave, uint64_t &before, uint64_t &all) {
     uint32_t lo = (uint32_t)own, hi = (uint32_t)(own >> 32);

@@ -238,8 +238,9 @@ moe_pf_group_kernel(const int32_t *__restrict__ ids, uint32_t pairs, uint32_t ex
     lev_barrier_lds();
     // The order of an expert's pairs depends on the atomics; no result does: every pair is computed
     // by itself and owns its outputs.  A long list is put together in LDS where it fits (64 lanes that store to 64 places of memory
-    // take the address unit 64 clocks) and stored as it lies there: 8000 pairs 12.6 us before, 10.2 with this and the wide loads;
-    // 1200 pairs 6.1 and, stored in place, 5.8.
+    // take the address unit 64 clocks) and stored as it lies there.  us stored in place and so, top-8 of 128 experts: 2000 pairs 5.1
+    // and 5.2, 4160 7.2 and 6.4, 8000 9.5 and 7.4, 16000 24.2 and 19.0; top-2 of 32 4200 13.0 and 12.7, top-1 4200 19.6 and 20.0.
+    // (Longer lists gain too, 28000 46.2 and 35.5: not taken, with 4096 experts' counts that is nine tenths of a CU's LDS.)
     const bool in_lds = pf_list_in_lds(pairs);
     int32_t *const s_list = s_cnt + 2u * experts + 1u;
     auto place = [&](int32_t e, int32_t rank, uint32_t pair) {
